@@ -30,7 +30,13 @@
 //    with the most tiles (low key blocks) start first, and each (batch, kv head)'s key blocks share an XCD (Q / dO
 //    reuse in L2);
 //  * block-sparse: each workgroup walks only the 32-row query tiles its key block meets in the layout (a host-built
-//    column LUT) and masks at the layout's block granularity (16/32/64/128) — cost scales with the layout density.
+//    column plan) and masks by the 32 bits that the plan holds per tile (2 x 16 rows, 16 x 16 keys) — cost scales with the
+//    layout density. List, masks and the per-key bias reach the loop through scalar loads and registers: a vector load in
+//    there waits for everything in flight ahead of it, the dQ atomics of waves 0..3 and the tiles of waves 4..7 included;
+//  * a sweep that is much longer than the others (the global columns of BigBird), or too few of them to fill the chip
+//    (short sequences of grouped-query models), is cut into parts that leave fp32 dK / dV in a workspace; a second launch
+//    adds them up in a fixed order. B2 H8 S16384, BigBird of 64-key blocks with padding: 1641 -> 506 us, now bound by the
+//    dQ atomics (below); B3 Hq16 Hk4 S1000 causal (48 workgroups uncut): 313 -> 103 us.
 // Measured (tools/bench_flash_bwd.py, profiles/flash_bwd_bench_r2_final.jsonl): B8 H32 S4096 D128 causal 4.2-4.3 ms
 // (round-2 start: 4.58). SQ PMC of the round-2 start: ~29 % MFMA busy, ~9 VALU per MFMA -- the VALU issue slots, not
 // the matrix pipe, are what the trims above (packed converts, pre-scaled row constants, uniform mask skip) buy back.
@@ -47,8 +53,6 @@
 // 4.3 ms; +10 SGPR spills and the split bookkeeping slowed every shape).
 #include "ds_hip.h"
 
-#include <cstdlib>
-
 namespace {
 
 constexpr int D = 128;
@@ -59,7 +63,7 @@ constexpr int K_BYTES = KB * 256;      // resident K image
 constexpr int DS_BYTES = KB * 64;      // dS^T image [KB keys][32 q] bf16
 constexpr int NBUF = 3;                // Q / dO / lse / delta tiles in flight: two ahead of the one in use
 template <int NW>
-constexpr int lds_bytes() { return K_BYTES + NBUF * 2 * TILE + 2 * DS_BYTES + NBUF * 64 * 4 + 2 * 8; }
+constexpr int lds_bytes() { return K_BYTES + NBUF * 2 * TILE + 2 * DS_BYTES + NBUF * 64 * 4; }
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
@@ -137,12 +141,18 @@ struct BwdArgs {
   int64_t qsb, qsh, qss, ksb, ksh, kss, vsb, vsh, vss, osb, osh, oss, dksb, dksh, dkss, dvsb, dvsh, dvss;
   float c;      // softmax scale * log2(e)
   float scale;
-  // block-sparse column LUT: qtiles [Hk, nkb, maxt] = (query head within the kv group << 16 | 32-row query tile)
-  // for every tile key block kb meets, nqt [Hk, nkb] = list lengths; layout [LH, nb, nb] uint8 at granularity blk
+  // block-sparse column plan, each for lut_heads (1 or Hk) kv heads: qtiles [nkb, maxt] = (query head within the kv group
+  // << 16 | 32-row query tile) for every tile key block kb meets, qmasks [nkb, maxt] (bit 16 r + k: its rows 16r.. see keys
+  // 16k.. of the block), work [nwork, 4] = (key block or -1, first entry of its list, entries, part slot or -1), merges
+  // [nmerge, 4] = (key block or -1, first slot, slots, 0)
   const int* qtiles;
-  const int* nqt;
-  const uint8_t* layout;
-  int maxt, lay_heads, nb, blk;
+  const int* qmasks;
+  const int* work;
+  const int* merges;
+  int maxt, lut_heads, nwork, nmerge;
+  // parts: dense sweeps are cut into nsplit of them (part p of key block kb: slot kb * nsplit + p)
+  int nsplit, nslots;
+  f32x4* part;  // [B * Hk, nslots, 32, 512]
   // additive score biases of the block-sparse path (see flash_fwd.hip SparseLut), any may be null
   const float *kbias, *abias, *rpe;
   int64_t kb_stride, ab_stride, rpe_hs, rpe_rs;
@@ -150,8 +160,11 @@ struct BwdArgs {
   // strides and key multipliers (ab_km / rpe_km) are 0, so the kernel loads unconditionally (a uniform branch around
   // these loads runs into a hipcc ROCm 7.2 code generation error)
   int bias_flags, kb_km, ab_km, rpe_km;
-  int dbg;  // experiment switches (DS_FLASH_BWD_DBG): 1 no atomics, 2 no dQ phase, 4 no dK/dV products, 8 no S/dP
 };
+
+// read-only and wave-uniform: scalar loads, whatever the kernel writes or clobbers in between
+typedef __attribute__((address_space(4))) const int const_int;
+__device__ __forceinline__ const_int* uniform_ints(const int* p) { return (const_int*)(uintptr_t)p; }
 
 // NW waves per workgroup, each owning KPW = 256 / NW keys (NC = KPW / 32 column tiles of the S / dP accumulators).
 // NW = 4: one wave per SIMD with the whole 512-register file (dK^T/dV^T of 64 keys = 256 accumulator registers),
@@ -167,8 +180,19 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
   const int S = a.S;
   const int nkb = (S + KB - 1) / KB;
   const int logical = xcd_remap(blockIdx.x, gridDim.x);
-  const int bh = logical / nkb, kb = logical % nkb;  // causal: low key blocks (most tiles) first within a head
+  const int per_bh = SPARSE ? a.nwork : nkb * a.nsplit;
+  const int bh = logical / per_bh, wi = logical % per_bh;
   const int b = bh / a.Hk, hk = bh % a.Hk, rep = a.Hq / a.Hk;
+  int kb = wi / a.nsplit, it0 = 0, slot = -1;  // causal: low key blocks (most tiles) first within a head
+  int n_it = 0;
+  if constexpr (SPARSE) {
+    const_int* wk = uniform_ints(a.work) + ((int64_t)(a.lut_heads == 1 ? 0 : hk) * a.nwork + wi) * 4;
+    kb = wk[0];
+    it0 = wk[1];
+    n_it = wk[2];
+    slot = wk[3];
+    if (kb < 0) return;  // (heads with fewer parts than the others)
+  }
   const int k0 = kb * KB;
   const int ntq = (S + QT - 1) / QT;
 
@@ -176,7 +200,6 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
   char* QD = smem + K_BYTES;                      // [NBUF][Q tile | dO tile]
   char* DSimg = QD + NBUF * 2 * TILE;             // [2][KB][32] bf16
   float* LD = reinterpret_cast<float*>(DSimg + 2 * DS_BYTES);  // [NBUF][lse (32) | delta (32)]
-  uint8_t* FL = reinterpret_cast<uint8_t*>(LD + NBUF * 64);       // [2][8 slabs]: slab met the tile
 
   const bf16* Kp = a.k + b * a.ksb + hk * a.ksh;
   const bf16* Vp = a.v + b * a.vsb + hk * a.vsh;
@@ -184,21 +207,28 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
   // ------------------------------------------------------------------ iteration space: (query head, query tile)
   const int t0 = CAUSAL ? k0 / QT : 0;
   const int per_head_dense = ntq - t0;
-  int n_it = rep * per_head_dense;
-  const int* lut = nullptr;
+  const_int* lut = nullptr;
+  const_int* lutm = nullptr;
   if constexpr (SPARSE) {
-    lut = a.qtiles + ((int64_t)hk * nkb + kb) * a.maxt;
-    n_it = a.nqt[hk * nkb + kb];
+    const int64_t at = ((int64_t)(a.lut_heads == 1 ? 0 : hk) * nkb + kb) * a.maxt + it0;
+    lut = uniform_ints(a.qtiles) + at;
+    lutm = uniform_ints(a.qmasks) + at;
+    it0 = 0;
+  } else {
+    const int all = rep * per_head_dense, part = wi % a.nsplit;
+    it0 = (int)((int64_t)all * part / a.nsplit);
+    n_it = (int)((int64_t)all * (part + 1) / a.nsplit) - it0;
+    if (a.nsplit > 1) slot = wi;
   }
-  // it -> (query head, query tile); the sparse LUT lists (head-in-group << 16 | tile) per (kv head, key block)
+  // it -> (query head, query tile); the sparse list holds (head-in-group << 16 | tile) per (kv head, key block)
   auto tile_at = [&](int it, int& hq, int& qt) {
     if constexpr (SPARSE) {
       const int code = lut[it];
       hq = hk * rep + (code >> 16);
       qt = code & 0xffff;
     } else {
-      hq = hk * rep + it / per_head_dense;
-      qt = t0 + it % per_head_dense;
+      hq = hk * rep + (it0 + it) / per_head_dense;
+      qt = t0 + (it0 + it) % per_head_dense;
     }
   };
 
@@ -313,12 +343,22 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) dk[c][dt][r] = dv[c][dt][r] = 0.f;
 
+  float kbv[NC];  // BIASED: the per-key bias of this lane's keys, in units of log2
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+    kbv[c] = BIASED == 0 ? 0.f : a.kbias[(int64_t)b * a.kb_stride + (int64_t)min(kw0 + 32 * c + l32, S - 1) * a.kb_km] *
+                                     1.4426950408889634f;
+
   // K image / V rows landed before the DMA starts: consuming the V fragments here makes hipcc's own waitcnt pass
   // retire them now instead of waiting vmcnt(0) (= draining the DMA) at their first use inside the tile loop
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) asm volatile("" : : "v"(vf[c][kk]));
+  if constexpr (BIASED != 0) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(kbv[c]));
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   if (n_it > 0) stage(0, 0);
   if (n_it > 1) stage(1, 1);
@@ -340,6 +380,7 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
     char* DSc = DSimg + cur * DS_BYTES;
 
     // ---------------- which of this wave's 32-key slabs meet the tile? keep[c] bit r: accumulator row r unmasked
+    const unsigned tmask = SPARSE ? (unsigned)lutm[it] : 0xffffffffu;
     bool act[NC];
     unsigned keep[NC];
 #pragma unroll
@@ -347,19 +388,11 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
       const int ks = kw0 + 32 * c, mykey = ks + l32;
       act[c] = ks < S && (!CAUSAL || ks <= q0 + QT - 1);
       keep[c] = mykey < S ? 0xffffu : 0u;
-      if constexpr (SPARSE) {
-        const int lh = a.lay_heads == 1 ? 0 : hq;
-        const int kbl = min(mykey, S - 1) / a.blk;
-        const uint8_t* lay = a.layout + (int64_t)lh * a.nb * a.nb;
-        const int r0 = q0 / a.blk;
-        const unsigned a0 = lay[(int64_t)r0 * a.nb + kbl] ? 0xffffu : 0u;
-        if (a.blk < QT) {  // 16-row blocks: registers 0..7 are rows 0..15 of the tile, 8..15 rows 16..31
-          const unsigned a1 = lay[(int64_t)min(r0 + 1, a.nb - 1) * a.nb + kbl] ? 0xffffu : 0u;
-          keep[c] &= (a0 & 0x00ffu) | (a1 & 0xff00u);
-        } else {
-          keep[c] &= a0;
-        }
-        act[c] = act[c] && __any(keep[c] != 0);
+      if constexpr (SPARSE) {  // registers 0..7 are rows 0..15 of the tile, 8..15 rows 16..31
+        const unsigned mine = tmask >> ((ks - k0) / 16);
+        act[c] = act[c] && (mine & 0x00030003u) != 0;
+        const unsigned lane_bits = mine >> (l32 >> 4);
+        keep[c] &= ((lane_bits & 1u) ? 0x00ffu : 0u) | ((lane_bits & 0x10000u) ? 0xff00u : 0u);
       }
       if (q0 + QT > S) {  // padded query rows of the last tile
 #pragma unroll
@@ -375,7 +408,7 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
     // one 32-key slab at a time (bounds the live S / dP accumulators to 32 registers)
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      if (!act[c] || (a.dbg & 8)) continue;
+      if (!act[c]) continue;
       // ---------------- S' = Q.K^T - LSE/scale and dP' = dO.V^T - delta (query rows in registers, key on the
       // lane); the row constants are the accumulators' initial values
       f32x16_t s, dp;
@@ -429,12 +462,11 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
         // BIASED == 1: per-key bias only (BERT padding masks); 2: all three terms.
         const int mykey = min(kw0 + 32 * c + l32, S - 1);
         const float l2e = 1.4426950408889634f;
-        const float kb = a.kbias[(int64_t)b * a.kb_stride + (int64_t)mykey * a.kb_km] * l2e;
         const float* abp = a.abias + (int64_t)mykey * a.ab_km;
         const float* rpp = a.rpe + (int64_t)hq * a.rpe_hs + (int64_t)mykey * a.rpe_km;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          float bv = kb;
+          float bv = kbv[c];
           if constexpr (BIASED == 2) {
             const int qr = min(q0 + crow(r, h), S - 1);
             bv = fmaf(abp[(int64_t)qr * a.ab_stride] + rpp[(int64_t)qr * a.rpe_rs], l2e, bv);
@@ -487,7 +519,7 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
       // pinned with sched_barrier (ALU may cross, MFMA / LDS may not; a full barrier hits a hipcc ROCm 7.2 codegen
       // error): left to itself the scheduler reused one operand quad and waited lgkmcnt(0) in front of every MFMA
       // (LDS latency fully exposed; SQ_VALU_MFMA_BUSY_CYCLES put the kernel at ~29 % MFMA utilisation).
-      if (!(a.dbg & 4)) {
+      {
         auto opnd = [&](int i) {
           const int dt = i >> 2, s2 = (i >> 1) & 1;
           const char* base = Qt + ((i & 1) ? 0 : TILE) + 4096 * s2;  // Ot = Qt + TILE (integer select)
@@ -509,21 +541,12 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
         }
       }
     }
-    // the dQ product walks only the slabs that met this tile
-    if (lane == 0) {
-#pragma unroll
-      for (int c = 0; c < NC; ++c) FL[cur * 8 + NC * w + c] = act[c] ? 1 : 0;
-    }
-
     barrier_keep_newest(it + 2 < n_it);
 
     // ---------------- dQ[q0:q0+32, 32wq:32wq+32] += dS . K over the slabs that met the tile (waves 0..3; waves
     // 4..7 run ahead into the next tile, so the SIMDs stay busy). Measured against an even 8-wave split on
     // 16x16x32 MFMAs: this form is 5% faster end to end (fewer transposed reads per MFMA).
-    if (w < 4 && !(a.dbg & 2)) {
-      const uint64_t fl = *reinterpret_cast<const uint64_t*>(FL + cur * 8);
-      const uint32_t flo = __builtin_amdgcn_readfirstlane((uint32_t)fl),
-                     fhi = __builtin_amdgcn_readfirstlane((uint32_t)(fl >> 32));
+    if (w < 4) {
       f32x16_t dq;
 #pragma unroll
       for (int r = 0; r < 16; ++r) dq[r] = 0.f;
@@ -537,7 +560,7 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
       if constexpr (SPARSE) {
 #pragma unroll 1
         for (int slab = 0; slab < 8; ++slab) {
-          if (!(((slab < 4 ? flo : fhi) >> (8 * (slab & 3))) & 0xff)) continue;
+          if (!((tmask >> (2 * slab)) & 0x00030003u)) continue;
           const bf16x8_t a0 = ld_a(2 * slab), b0 = ld_b(2 * slab), a1 = ld_a(2 * slab + 1), b1 = ld_b(2 * slab + 1);
           dq = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b0, dq, 0, 0, 0);
           dq = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, dq, 0, 0, 0);
@@ -548,8 +571,6 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
         int kmax = min(KB, S - k0);
         if (CAUSAL) kmax = min(kmax, q0 + QT - k0);
         nks = (kmax + 15) >> 4;
-        (void)flo;
-        (void)fhi;
         if (nks == KB / 16) {  // every key block but the diagonal one: straight-line, scheduled by hipcc
 #pragma unroll
           for (int s2 = 0; s2 < KB / 16; ++s2)
@@ -560,7 +581,7 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
             dq = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld_a(s2), ld_b(s2), dq, 0, 0, 0);
         }
       }
-      if (nks > 0 && !(a.dbg & 1)) {
+      if (nks > 0) {
         // lane part of the 16 destination rows, laundered so that hipcc forms each address next to its atomic
         // instead of keeping 16 64-bit addresses live across the loop (they spilled). One register of a 32x32
         // accumulator = two 128-B row segments, the full-rate atomic shape.
@@ -581,6 +602,24 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
   }
 
   // ------------------------------------------------------------------ epilogue: dK = scale * dK^T^T, dV
+  if (slot >= 0) {  // a part of the sweep: the accumulators as they are, 16 bytes per thread and piece
+    static_assert(NC == 1 && NTHR == 512, "the parts' layout");
+    f32x4* po = a.part + ((int64_t)bh * a.nslots + slot) * (32 * NTHR) + tid;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        f32x4 k4, v4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          k4[i] = dk[0][dt][4 * g + i];
+          v4[i] = dv[0][dt][4 * g + i];
+        }
+        po[(4 * dt + g) * NTHR] = k4;
+        po[(16 + 4 * dt + g) * NTHR] = v4;
+      }
+    return;
+  }
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     const int mykey = kw0 + 32 * c + l32;
@@ -601,6 +640,40 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
         *reinterpret_cast<bf16x4*>(dkp + d0) = k4;
         *reinterpret_cast<bf16x4*>(dvp + d0) = v4;
       }
+  }
+}
+
+// dK and dV of key blocks whose sweep was cut: the parts' accumulators added up, a block per 32 columns of one of the two (the
+// thread layout is the main kernel's).
+__global__ void __launch_bounds__(512) flash_bwd_merge_kernel(BwdArgs a) {
+  const int bh = blockIdx.y, b = bh / a.Hk, hk = bh % a.Hk, mi = blockIdx.x / 8, dt = blockIdx.x & 3, isv = (blockIdx.x >> 2) & 1;
+  int kb = mi, slot0 = mi * a.nsplit, n = a.nsplit;
+  if (a.merges != nullptr) {
+    const int* me = a.merges + ((int64_t)(a.lut_heads == 1 ? 0 : hk) * a.nmerge + mi) * 4;
+    kb = me[0];
+    slot0 = me[1];
+    n = me[2];
+    if (kb < 0) return;
+  }
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, key = kb * KB + 32 * (tid >> 6) + (lane & 31);
+  const f32x4* src = a.part + ((int64_t)bh * a.nslots + slot0) * (32 * 512) + (16 * isv + 4 * dt) * 512 + tid;
+  f32x4 acc[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) acc[g] = src[g * 512];
+  for (int p = 1; p < n; ++p) {
+    src += 32 * 512;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) acc[g] += src[g * 512];
+  }
+  if (key >= a.S) return;
+  bf16* dst = isv ? a.dv + b * a.dvsb + hk * a.dvsh + (int64_t)key * a.dvss : a.dk + b * a.dksb + hk * a.dksh + (int64_t)key * a.dkss;
+  const float f = isv ? 1.f : a.scale;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    bf16x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = (bf16)(acc[g][i] * f);
+    *reinterpret_cast<bf16x4*>(dst + 32 * dt + 8 * g + 4 * h) = r;
   }
 }
 
@@ -666,9 +739,14 @@ int launch_main(const BwdArgs& a, hipStream_t st) {
     attr = true;
   }
   const int nkb = (a.S + KB - 1) / KB;
-  const int grid = a.B * a.Hk * nkb;
+  const int grid = a.B * a.Hk * (SP ? a.nwork : nkb * a.nsplit);
   hipLaunchKernelGGL((flash_bwd_kernel<NW, C, SP, BI>), dim3(grid), dim3(NW * 64), lds_bytes<NW>(), st, a);
   DS_CHECK_LAUNCH();
+  const int nmerge = SP ? a.nmerge : (a.nsplit > 1 ? nkb : 0);
+  if (nmerge > 0) {
+    hipLaunchKernelGGL(flash_bwd_merge_kernel, dim3(nmerge * 8, a.B * a.Hk), dim3(512), 0, st, a);
+    DS_CHECK_LAUNCH();
+  }
   return 0;
 }
 
@@ -685,19 +763,34 @@ int launch_mode(const BwdArgs& a, int mode, hipStream_t st) {
 // Strides are (batch, head, seq) in elements, unit last stride everywhere, all bf16 rows 16-B aligned.
 // q/o/dout/dq [B,Hq,S,128], k/v/dk/dv [B,Hk,S,128], lse [B,Hq,S] natural-log (flash_fwd's), workspace:
 // delta [2*B*Hq*S] fp32 (the pre kernel's -delta and -LSE/scale rows) and dqacc [B*Hq*S*128] fp32.
-// mode: 0 full, 1 causal (top-left), 2 block-sparse (LUT below).
+// mode: 0 full, 1 causal (top-left), 2 block-sparse (plan: see BwdArgs). part: the workspace of the parts,
+// B * Hk * slots * 256 KB, slots = ds_flash_bwd_split(..) * key blocks of 256 for the dense modes (none if it is 1) or nslots.
+
+// Parts per key block of a dense sweep. A workgroup takes a CU for itself, so anything below 256 of them idles the rest;
+// parts shorter than 4 tiles would spend their time on the K image and the accumulators. Measured, us, causal, for parts
+// that make at most 1 / 128 / 256 / 512 / 1024 workgroups: B3 Hq16 Hk4 S1000 313 / 179 / 103 / 110 / 145, B1 Hq32 Hk8 S2048
+// 605 / 333 / 208 / 190 / 264, B1 Hq8 Hk2 S4096 1144 / 322 / 195 / 196 / 253; B1 H16 S512 (32 workgroups) with parts of at
+// least 16 / 8 / 4 tiles 55 / 45 / 39.
+extern "C" int ds_flash_bwd_split(int B, int Hq, int Hk, int S) {
+  const int nkb = (S + KB - 1) / KB, tiles = Hq / Hk * ((S + QT - 1) / QT);
+  const int fill = 256 / max(B * Hk * nkb, 1), most = tiles / 4;
+  return max(1, min(fill, most));
+}
+
 extern "C" int ds_flash_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout,
                             const float* lse, float* delta, float* dqacc, void* dq, void* dk, void* dv, int B, int Hq,
                             int Hk, int S, const int64_t* qs, const int64_t* ks, const int64_t* vs, const int64_t* os,
                             const int64_t* dos, const int64_t* dqs, const int64_t* dks, const int64_t* dvs,
-                            float scale, int mode, const int* qtiles, const int* nqt, const uint8_t* layout, int maxt,
-                            int lay_heads, int nb, int blk, int bias_flags, const float* kbias, int64_t kb_stride,
-                            const float* abias, int64_t ab_stride, const float* rpe, int64_t rpe_hs, int64_t rpe_rs,
-                            hipStream_t st) {
+                            float scale, int mode, const int* qtiles, const int* qmasks, const int* work, const int* merges,
+                            int maxt, int lut_heads, int nwork, int nmerge, int nslots, float* part, int bias_flags,
+                            const float* kbias, int64_t kb_stride, const float* abias, int64_t ab_stride, const float* rpe,
+                            int64_t rpe_hs, int64_t rpe_rs, hipStream_t st) {
   if (Hk <= 0 || Hq % Hk != 0 || S <= 0 || B <= 0) return (int)hipErrorInvalidValue;
-  if (mode == 2 && (qtiles == nullptr || nqt == nullptr || layout == nullptr || (lay_heads != 1 && lay_heads != Hq) ||
-                    (blk != 16 && blk != 32 && blk != 64 && blk != 128) || nb * blk < S))
+  if (mode == 2 && (qtiles == nullptr || qmasks == nullptr || work == nullptr || (lut_heads != 1 && lut_heads != Hk) ||
+                    nwork <= 0 || (nmerge > 0 && (merges == nullptr || nslots <= 0))))
     return (int)hipErrorInvalidValue;
+  const int nsplit = mode == 2 ? 1 : ds_flash_bwd_split(B, Hq, Hk, S);
+  if ((nsplit > 1 || (mode == 2 && nmerge > 0)) && part == nullptr) return (int)hipErrorInvalidValue;
   const int64_t rows = (int64_t)B * Hq * S;
   const int pgrid = (int)((rows + 15) / 16);
   hipLaunchKernelGGL(flash_bwd_pre_kernel, dim3(pgrid), dim3(256), 0, st, (const bf16*)o, (const bf16*)dout, lse,
@@ -715,8 +808,11 @@ extern "C" int ds_flash_bwd(const void* q, const void* k, const void* v, const v
   a.dvsb = dvs[0]; a.dvsh = dvs[1]; a.dvss = dvs[2];
   a.c = scale * 1.4426950408889634f;
   a.scale = scale;
-  { const char* e = getenv("DS_FLASH_BWD_DBG"); a.dbg = e ? atoi(e) : 0; }
-  a.qtiles = qtiles; a.nqt = nqt; a.layout = layout; a.maxt = maxt; a.lay_heads = lay_heads; a.nb = nb; a.blk = blk;
+  a.qtiles = qtiles; a.qmasks = qmasks; a.work = work; a.merges = mode == 2 ? merges : nullptr;
+  a.maxt = maxt; a.lut_heads = lut_heads; a.nwork = nwork; a.nmerge = nmerge;
+  a.nsplit = nsplit;
+  a.nslots = mode == 2 ? nslots : nsplit * ((S + KB - 1) / KB);
+  a.part = reinterpret_cast<f32x4*>(part);
   // biases: block-sparse path only; with any bias present every pointer must be valid (see BwdArgs::bias_flags)
   if (bias_flags && (mode != 2 || !kbias || !abias || !rpe)) return (int)hipErrorInvalidValue;
   a.kbias = kbias; a.abias = abias; a.rpe = rpe;

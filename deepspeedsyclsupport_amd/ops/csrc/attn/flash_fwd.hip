@@ -18,9 +18,15 @@
 //  * causal: fully-masked tiles are skipped per wave, heavy query blocks are launched first, and the block->tile map
 //    keeps every (batch, head) on one XCD so its K/V stay in that XCD's L2.
 //  * block-sparse variant (SPARSE=true, reference `ops/sparse_attention` SDD/softmax/DSD Triton kernels): each
-//    workgroup walks only the 64-key tiles listed for its (layout head, 128-row query block) in a host-built LUT, and
-//    masks inside a tile at the layout's block granularity (16/32/64/128) with a per-lane 64-bit allow mask built
-//    from the block layout — compute and K/V traffic scale with the layout's density, not with S^2.
+//    workgroup walks only the 64-key tiles listed for its (layout head, 128-row query block) in a host-built plan, and
+//    masks inside a tile by the 32 bits that the plan holds per tile (16 rows x 16 keys each) — compute and K/V traffic
+//    scale with the layout's density, not with S^2. Lists much longer than the average (the global rows of BigBird) are
+//    cut into parts that leave unnormalised rows in a workspace; a second launch merges them.
+//    What the sparse loop must not do is load from global memory: hipcc waits for its own loads with vmcnt(0), which
+//    drains the tile transfer that was just issued, so that every tile paid a full trip to memory. The list and the
+//    masks come through scalar loads (address space 4), the per-key bias by LDS-DMA with its tile.
+//    B2 H8 S16384, BigBird of 64-key blocks with padding: 1572 -> 113 us (1150 tiles per head; uncut, one workgroup
+//    walks the 256 of the global rows at 6 us each while the rest of the chip has long been idle).
 // Outputs O (any [B,H,S,D] strides, e.g. written straight into the [B,S,H,D] layout the o_proj GEMM wants) and the
 // natural-log LSE [B,H,S] in fp32 that the backward pass consumes.
 #include "ds_hip.h"
@@ -35,6 +41,7 @@ constexpr int BN = 64;             // keys per tile
 constexpr int NTHR = 256;
 constexpr int TILE_BYTES = BN * D * 2;     // 16 KB
 constexpr int LDS_BYTES = 4 * TILE_BYTES + 4 * 32 * 4;  // K0 K1 V0 V1 + per-wave row scratch
+constexpr int LDS_SPARSE = LDS_BYTES + 2 * BN * 4;      // + the per-key bias of two tiles
 
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -72,6 +79,16 @@ __device__ __forceinline__ void glds16_s(const char* base, uint32_t voff, const 
                : "memory");
 }
 
+__device__ __forceinline__ void glds4(const void* g, const char* lds_base) {  // 4 bytes per lane
+  const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_char*)lds_base);
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, off\n\t"
+               "s_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "v"(g), "s"(dst)
+               : "memory");
+}
+
 // byte offset of 16-B chunk `ch` (0..15) of row `row` in a [64][128 x bf16] tile: 256-B rows, chunk index XORed with
 // a bijection of row mod 16 so both the row reads (32 consecutive rows, one chunk) and the 4-row transposed reads
 // touch distinct banks.
@@ -94,14 +111,17 @@ __device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
   return r;
 }
 
-// block-sparse LUT: tiles [lay_heads, nqb, max_tiles] (ascending 64-key tile ids), ntiles [lay_heads, nqb],
-// layout [lay_heads, nb, nb] (uint8, block granularity blk)
+// block-sparse plan: tiles, masks [lay_heads, nqb, max_tiles] (64-key tile ids; bit 4 r + k of a mask: rows 16r.. of the
+// query block see keys 16k.. of the tile), work [lay_heads, nwork, 4] = (query block or -1, first entry of its list, number of
+// entries, part slot or -1) longest first, merges [lay_heads, nmerge, 4] = (query block or -1, first slot, slots, 0)
 struct SparseLut {
   const int* tiles;
-  const int* ntiles;
-  const int* qorder;  // [lay_heads, nqb] query blocks by descending tile count
-  const uint8_t* layout;
-  int max_tiles, lay_heads, nb, blk;
+  const int* masks;
+  const int* work;
+  const int* merges;
+  float* part_o;           // [B * Hq, nslots, 128, 128] unnormalised rows of the parts
+  float* part_ml;          // [B * Hq, nslots, 2, 128] their maxima (raw score units) and sums
+  int max_tiles, lay_heads, nwork, nmerge, nslots;
   // additive biases on the scaled scores (reference `ops/sparse_attention/softmax.py:37-70`: key-padding mask,
   // attention mask and relative position embedding are applied inside the sparse softmax); any may be null
   const float* kbias;      // [B, Skv] per-key (key_padding_mask in additive form), row stride kb_stride
@@ -109,8 +129,12 @@ struct SparseLut {
   const float* rpe;        // [H or 1, S, Skv] per head, head stride rpe_hs (0 = shared), row stride rpe_rs
   int64_t kb_stride, ab_stride, rpe_hs, rpe_rs;
 };
+// read-only and wave-uniform: scalar loads, whatever the kernel writes or clobbers in between
+typedef __attribute__((address_space(4))) const int const_int;
+__device__ __forceinline__ const_int* uniform_ints(const int* p) { return (const_int*)(uintptr_t)p; }
 
-template <bool CAUSAL, bool SPARSE>
+// ROWB: biases per query row and key (the loop without them keeps its registers)
+template <bool CAUSAL, bool SPARSE, bool ROWB = false>
 __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
     const bf16* __restrict__ Q, const bf16* __restrict__ K, const bf16* __restrict__ V, bf16* __restrict__ O,
     float* __restrict__ LSE, int B, int Hq, int Hk, int S, int Skv, int64_t qsb, int64_t qsh, int64_t qss,
@@ -127,11 +151,20 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
   // within a head the heaviest query blocks go first (causal: the longest rows; sparse: the LUT's order by tile
   // count, so global-attention rows do not start last). Measured: query-block-major heavy-first order loses more
   // to L2 misses than it gains in tail length (tools/bench_sparse_attn.py).
-  const int bh = logical / nqb;
-  const int qbi = logical % nqb;
+  const int per_bh = SPARSE ? lut.nwork : nqb;
+  const int bh = logical / per_bh;
+  const int qbi = logical % per_bh;
   const int b = bh / Hq, hq = bh % Hq, hk = hq / (Hq / Hk);
   const int lh = SPARSE ? (lut.lay_heads == 1 ? 0 : hq) : 0;
-  const int qb = SPARSE ? lut.qorder[lh * nqb + qbi] : (CAUSAL ? nqb - 1 - qbi : qbi);  // heaviest first
+  int qb = CAUSAL ? nqb - 1 - qbi : qbi, first = 0, count = 0, slot = -1;  // heaviest first
+  if constexpr (SPARSE) {
+    const_int* wk = uniform_ints(lut.work) + ((int64_t)lh * lut.nwork + qbi) * 4;
+    qb = wk[0];
+    first = wk[1];
+    count = wk[2];
+    slot = wk[3];
+    if (qb < 0) return;  // (heads with fewer parts than the others)
+  }
   const int q0 = qb * BM, q0w = q0 + wid * 32;
 
   const bf16* Qp = Q + b * qsb + hq * qsh;
@@ -149,14 +182,18 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
 
   int nt = (Skv + BN - 1) / BN;
   if (CAUSAL) nt = min(nt, (q0 + BM + BN - 1) / BN);
-  const int* tlist = nullptr;
+  const_int* tlist = nullptr;
+  const_int* mlist = nullptr;
+  const float* kbp = nullptr;
   if constexpr (SPARSE) {
-    nt = lut.ntiles[lh * nqb + qb];
-    tlist = lut.tiles + ((int64_t)lh * nqb + qb) * lut.max_tiles;
+    nt = count;
+    tlist = uniform_ints(lut.tiles) + ((int64_t)lh * nqb + qb) * lut.max_tiles + first;
+    mlist = uniform_ints(lut.masks) + ((int64_t)lh * nqb + qb) * lut.max_tiles + first;
+    if (lut.kbias != nullptr) kbp = lut.kbias + (int64_t)b * lut.kb_stride;
   }
   auto tile_of = [&](int j) { return SPARSE ? tlist[j] : j; };
 
-  // LDS: [K0][K1][V0][V1][scratch]
+  // LDS: [K0][K1][V0][V1][scratch][SPARSE: bias0 bias1]
   float* scratch = reinterpret_cast<float*>(smem + 4 * TILE_BYTES) + wid * 32;
   const lds_char* s3 = (const lds_char*)smem;  // 32-bit LDS addressing: per-lane base + compile-time displacement
 
@@ -173,6 +210,9 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
   const uint32_t kdma = (uint32_t)((drow * kss + dch * 8) * 2);
   const uint32_t vdma = (uint32_t)((drow * vss + dch * 8) * 2);
   auto dma_tile = [&](int tile, int buf) {
+    if constexpr (SPARSE) {
+      if (kbp != nullptr && wid == 0) glds4(kbp + tile * BN + lane, smem + LDS_BYTES + buf * BN * 4);
+    }
     if (tile * BN + BN <= Skv) {
       const char* kb = reinterpret_cast<const char*>(Kp + (int64_t)tile * BN * kss);
       const char* vb = reinterpret_cast<const char*>(Vp + (int64_t)tile * BN * vss);
@@ -235,7 +275,9 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
     constexpr int cur = decltype(cur_c)::value;
     if (j + 1 < nt) dma_tile(tile_of(j + 1), cur ^ 1);
     const int k0 = tile_of(j) * BN;
-    const bool active = !CAUSAL || k0 <= q0w + 31;
+    // SPARSE: this wave's 8 bits of the tile's mask
+    const unsigned seen = SPARSE ? ((unsigned)mlist[j] >> (8 * __builtin_amdgcn_readfirstlane(wid))) & 0xffu : 0xffu;
+    const bool active = (!CAUSAL || k0 <= q0w + 31) && seen != 0;
     if (active) {
       // ---------------- S^T = K . Q^T  (two 32-key halves), K fragments read three MFMAs ahead: left to itself
       // hipcc issued each ds_read right before its MFMA and waited lgkmcnt(0) in between, so every MFMA paid a
@@ -276,59 +318,47 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
       };
       bf16x8_t v0f = ldv(0), v1f = ldv(1);
       // ---------------- additive biases (key padding / attention mask / relative position), in raw score units
-      // (bias / scale), then the block-sparse mask at the layout's granularity (this lane's query row vs the 64 keys)
+      // (bias / scale), then the block-sparse mask: 16 x 16 per bit, eight registers of a lane share one
       if constexpr (SPARSE) {
-        if (lut.kbias != nullptr || lut.abias != nullptr || lut.rpe != nullptr) {
+        if (kbp != nullptr) {
           const float inv_scale = 1.f / scale;
-          const int qr = min(qrow_lane, S - 1);
-          const float* kbp = lut.kbias ? lut.kbias + (int64_t)b * lut.kb_stride : nullptr;
-          const float* abp = lut.abias ? lut.abias + (int64_t)qr * lut.ab_stride : nullptr;
-          const float* rpp = lut.rpe ? lut.rpe + (int64_t)hq * lut.rpe_hs + (int64_t)qr * lut.rpe_rs : nullptr;
+          const float* kbl = reinterpret_cast<const float*>(smem + LDS_BYTES + cur * BN * 4);
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {  // four consecutive keys: registers 4g .. 4g+3
+              const f32x4 bv = *reinterpret_cast<const f32x4*>(kbl + t * 32 + 8 * g + 4 * h);
+#pragma unroll
+              for (int i = 0; i < 4; ++i) s[t][4 * g + i] = fmaf(bv[i], inv_scale, s[t][4 * g + i]);
+            }
+        }
+        if constexpr (ROWB) {
+          const float inv_scale = 1.f / scale;
+          const float* abp = lut.abias ? lut.abias + (int64_t)qrow_lane * lut.ab_stride : nullptr;
+          const float* rpp = lut.rpe ? lut.rpe + (int64_t)hq * lut.rpe_hs + (int64_t)qrow_lane * lut.rpe_rs : nullptr;
 #pragma unroll
           for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-              const int key = k0 + t * 32 + 8 * g + 4 * h;  // four consecutive keys: registers 4g .. 4g+3
-              if (key + 3 < Skv) {
-                f32x4 bsum = {0.f, 0.f, 0.f, 0.f};
-                if (kbp) bsum += *reinterpret_cast<const f32x4*>(kbp + key);
-                if (abp) bsum += *reinterpret_cast<const f32x4*>(abp + key);
-                if (rpp) bsum += *reinterpret_cast<const f32x4*>(rpp + key);
+              const int key = k0 + t * 32 + 8 * g + 4 * h;
+              f32x4 bsum = {0.f, 0.f, 0.f, 0.f};
+              if (abp) bsum += *reinterpret_cast<const f32x4*>(abp + key);
+              if (rpp) bsum += *reinterpret_cast<const f32x4*>(rpp + key);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) s[t][4 * g + i] = fmaf(bsum[i], inv_scale, s[t][4 * g + i]);
-              } else {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                  if (key + i >= Skv) continue;
-                  float bv = 0.f;
-                  if (kbp) bv += kbp[key + i];
-                  if (abp) bv += abp[key + i];
-                  if (rpp) bv += rpp[key + i];
-                  s[t][4 * g + i] = fmaf(bv, inv_scale, s[t][4 * g + i]);
-                }
-              }
+              for (int i = 0; i < 4; ++i) s[t][4 * g + i] = fmaf(bsum[i], inv_scale, s[t][4 * g + i]);
             }
         }
-        const int qr = min(qrow_lane, S - 1);
-        const uint8_t* lrow = lut.layout + ((int64_t)lh * lut.nb + qr / lut.blk) * lut.nb;
-        uint64_t allow = 0;
-        for (int kb = k0 / lut.blk; kb < lut.nb && kb * lut.blk < k0 + BN; ++kb) {
-          if (!lrow[kb]) continue;
-          const int lo = max(kb * lut.blk - k0, 0), hi = min((kb + 1) * lut.blk - k0, BN);
-          allow |= (hi - lo >= 64 ? ~0ull : ((1ull << (hi - lo)) - 1)) << lo;
-        }
-        if (allow != ~0ull) {
+        if (seen != 0xffu) {
+          const unsigned mine = seen >> (4 * (l32 >> 4));
 #pragma unroll
           for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const int rel = t * 32 + (r & 3) + 8 * (r >> 2) + 4 * h;
-              if (!((allow >> rel) & 1ull)) s[t][r] = -INFINITY;
-            }
+            for (int r = 0; r < 16; ++r)
+              if (!((mine >> (2 * t + (r >> 3))) & 1u)) s[t][r] = -INFINITY;
         }
       }
       // ---------------- masking (causal diagonal / ragged key tail)
-      const bool need_mask = (CAUSAL && k0 + BN - 1 > q0w) || (k0 + BN > Skv);
+      const bool need_mask = !SPARSE && ((CAUSAL && k0 + BN - 1 > q0w) || (k0 + BN > Skv));
       if (need_mask) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -414,6 +444,22 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
 
   // ------------------------------------------------------------------ epilogue: O / l, LSE
   const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  if constexpr (SPARSE) {
+    if (slot >= 0) {  // a part of the list: rows as they are, maximum and sum
+      const int64_t at = (int64_t)bh * lut.nslots + slot;
+      float* po = lut.part_o + at * BM * D;
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+          po[(wid * 32 + (r & 3) + 8 * (r >> 2) + 4 * h) * D + dt * 32 + l32] = o[dt][r];
+      if (lane < 32) {
+        lut.part_ml[at * 2 * BM + wid * 32 + l32] = m_run;
+        lut.part_ml[at * 2 * BM + BM + wid * 32 + l32] = l_tot;
+      }
+      return;
+    }
+  }
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (lane < 32) scratch[lane] = inv;
   __builtin_amdgcn_wave_barrier();
@@ -441,24 +487,70 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
   }
 }
 
-template <bool C, bool SP>
+// Rows of query blocks whose list was cut: O = sum_p e^(m_p - m) O_p / sum_p e^(m_p - m) l_p. 8 threads per row, 16 columns
+// each; a block takes 32 rows of one query block.
+__global__ void __launch_bounds__(256) flash_merge_kernel(bf16* __restrict__ O, float* __restrict__ LSE, SparseLut lut, int Hq,
+                                                          int S, int64_t osb, int64_t osh, int64_t oss, float c) {
+  const int bh = blockIdx.y, b = bh / Hq, hq = bh % Hq, lh = lut.lay_heads == 1 ? 0 : hq;
+  const int* me = lut.merges + ((int64_t)lh * lut.nmerge + blockIdx.x / 4) * 4;
+  const int qb = me[0], slot0 = me[1], n = me[2];
+  if (qb < 0) return;
+  const int row = (blockIdx.x & 3) * 32 + (threadIdx.x >> 3), col = (threadIdx.x & 7) * 16, q = qb * BM + row;
+  const int64_t at = (int64_t)bh * lut.nslots + slot0;
+  float m = -INFINITY;
+  for (int p = 0; p < n; ++p) m = fmaxf(m, lut.part_ml[(at + p) * 2 * BM + row]);
+  float l = 0.f, acc[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  for (int p = 0; p < n; ++p) {
+    const float mp = lut.part_ml[(at + p) * 2 * BM + row];
+    const float f = mp == -INFINITY ? 0.f : fast_exp2((mp - m) * c);
+    l = fmaf(f, lut.part_ml[(at + p) * 2 * BM + BM + row], l);
+    const f32x4* src = reinterpret_cast<const f32x4*>(lut.part_o + ((at + p) * BM + row) * D + col);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const f32x4 v = src[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[4 * i + e] = fmaf(f, v[e], acc[4 * i + e]);
+    }
+  }
+  if (q >= S) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  bf16* dst = O + b * osb + hq * osh + (int64_t)q * oss + col;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = acc[8 * i + e] * inv;
+    Vec8<bf16>::store(dst + 8 * i, v);
+  }
+  if (LSE != nullptr && (threadIdx.x & 7) == 0)
+    LSE[((int64_t)b * Hq + hq) * S + q] = l > 0.f ? (m * c + __log2f(l)) * 0.69314718055994531f : INFINITY;
+}
+
+template <bool C, bool SP, bool RB = false>
 int launch(const bf16* q, const bf16* k, const bf16* v, bf16* o, float* lse, int B, int Hq, int Hk, int S, int Skv,
            const int64_t* qs, const int64_t* ks, const int64_t* vs, const int64_t* os, float scale, hipStream_t st,
-           SparseLut lut = SparseLut{nullptr, nullptr, nullptr, nullptr, 0, 1, 0, 1, nullptr, nullptr, nullptr, 0, 0,
-                                     0, 0}) {
+           const SparseLut& lut = SparseLut{}) {
+  constexpr int LDS = SP ? LDS_SPARSE : LDS_BYTES;
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_fwd_kernel<C, SP>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_fwd_kernel<C, SP, RB>),
+                        hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     attr = true;
   }
   const int nqb = (S + BM - 1) / BM;
-  const int grid = nqb * B * Hq;
+  const int grid = (SP ? lut.nwork : nqb) * B * Hq;
   const float c = scale * 1.4426950408889634f;
-  hipLaunchKernelGGL((flash_fwd_kernel<C, SP>), dim3(grid), dim3(NTHR), LDS_BYTES, st, q, k, v, o, lse, B, Hq, Hk, S,
+  hipLaunchKernelGGL((flash_fwd_kernel<C, SP, RB>), dim3(grid), dim3(NTHR), LDS, st, q, k, v, o, lse, B, Hq, Hk, S,
                      Skv, qs[0], qs[1], qs[2], ks[0], ks[1], ks[2], vs[0], vs[1], vs[2], os[0], os[1], os[2], c, scale,
                      lut);
   DS_CHECK_LAUNCH();
+  if (SP && lut.nmerge > 0) {
+    hipLaunchKernelGGL(flash_merge_kernel, dim3(lut.nmerge * 4, B * Hq), dim3(256), 0, st, o, lse, lut, Hq, S, os[0], os[1],
+                       os[2], c);
+    DS_CHECK_LAUNCH();
+  }
   return 0;
 }
 
@@ -479,23 +571,24 @@ extern "C" int ds_flash_fwd(const void* q, const void* k, const void* v, void* o
 }
 
 // Block-sparse forward: same tensors as ds_flash_fwd (non-causal; causality, if wanted, is part of the layout) plus
-// the LUT described at SparseLut. lay_heads is 1 (shared layout) or Hq. Requires S == Skv.
+// the plan described at SparseLut. lay_heads is 1 (shared layout) or Hq. Requires S == Skv, a multiple of 128. The merges'
+// slots need part_o (B Hq nslots 128 128 floats) and part_ml (B Hq nslots 2 128).
 extern "C" int ds_flash_fwd_sparse(const void* q, const void* k, const void* v, void* o, float* lse, int B, int Hq,
                                    int Hk, int S, const int64_t* qs, const int64_t* ks, const int64_t* vs,
-                                   const int64_t* os, float scale, const int* tiles, const int* ntiles,
-                                   const int* qorder, const uint8_t* layout, int max_tiles, int lay_heads, int nb,
-                                   int blk, const float* kbias, int64_t kb_stride, const float* abias,
-                                   int64_t ab_stride, const float* rpe, int64_t rpe_hs, int64_t rpe_rs,
+                                   const int64_t* os, float scale, const int* tiles, const int* masks, const int* work,
+                                   const int* merges, int max_tiles, int lay_heads, int nwork, int nmerge, int nslots,
+                                   float* part_o, float* part_ml, const float* kbias, int64_t kb_stride,
+                                   const float* abias, int64_t ab_stride, const float* rpe, int64_t rpe_hs, int64_t rpe_rs,
                                    hipStream_t st) {
-  if (Hk <= 0 || Hq % Hk != 0 || S <= 0 || blk <= 0 || nb * blk < S || max_tiles < 0 ||
-      (lay_heads != 1 && lay_heads != Hq) || tiles == nullptr || ntiles == nullptr || qorder == nullptr ||
-      layout == nullptr)
+  if (Hk <= 0 || Hq % Hk != 0 || S <= 0 || S % BM || max_tiles < 0 || nwork <= 0 || (lay_heads != 1 && lay_heads != Hq) ||
+      tiles == nullptr || masks == nullptr || work == nullptr || (nmerge > 0 && (merges == nullptr || nslots <= 0 || part_o == nullptr ||
+                                                                                 part_ml == nullptr)))
     return (int)hipErrorInvalidValue;
-  // bias rows are read four keys at a time
+  // rows of the attention bias and the relative positions are read four keys at a time
   auto al = [](const float* p, int64_t st) { return p == nullptr || (((uintptr_t)p % 16) == 0 && st % 4 == 0); };
   if (!al(kbias, kb_stride) || !al(abias, ab_stride) || !al(rpe, rpe_rs) || rpe_hs % 4) return (int)hipErrorInvalidValue;
-  return launch<false, true>((const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)o, lse, B, Hq, Hk, S, S, qs, ks,
-                             vs, os, scale, st,
-                             SparseLut{tiles, ntiles, qorder, layout, max_tiles, lay_heads, nb, blk, kbias, abias,
-                                       rpe, kb_stride, ab_stride, rpe_hs, rpe_rs});
+  const SparseLut lut{tiles, masks, work, merges, part_o, part_ml, max_tiles, lay_heads, nwork, nmerge, nslots,
+                      kbias, abias, rpe, kb_stride, ab_stride, rpe_hs, rpe_rs};
+  auto run = abias != nullptr || rpe != nullptr ? launch<false, true, true> : launch<false, true>;
+  return run((const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)o, lse, B, Hq, Hk, S, S, qs, ks, vs, os, scale, st, lut);
 }

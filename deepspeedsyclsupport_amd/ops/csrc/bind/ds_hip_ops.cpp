@@ -51,13 +51,14 @@ int ds_flash_fwd(const void*, const void*, const void*, void*, float*, int, int,
                  const int64_t*, const int64_t*, const int64_t*, float, int, hipStream_t);
 int ds_flash_fwd_sparse(const void*, const void*, const void*, void*, float*, int, int, int, int, const int64_t*,
                         const int64_t*, const int64_t*, const int64_t*, float, const int*, const int*, const int*,
-                        const uint8_t*, int, int, int, int, const float*, int64_t, const float*, int64_t, const float*,
-                        int64_t, int64_t, hipStream_t);
+                        const int*, int, int, int, int, int, float*, float*, const float*, int64_t, const float*, int64_t,
+                        const float*, int64_t, int64_t, hipStream_t);
+int ds_flash_bwd_split(int, int, int, int);
 int ds_flash_bwd(const void*, const void*, const void*, const void*, const void*, const float*, float*, float*, void*,
                  void*, void*, int, int, int, int, const int64_t*, const int64_t*, const int64_t*, const int64_t*,
                  const int64_t*, const int64_t*, const int64_t*, const int64_t*, float, int, const int*, const int*,
-                 const uint8_t*, int, int, int, int, int, const float*, int64_t, const float*, int64_t, const float*,
-                 int64_t, int64_t, hipStream_t);
+                 const int*, const int*, int, int, int, int, int, float*, int, const float*, int64_t, const float*, int64_t,
+                 const float*, int64_t, int64_t, hipStream_t);
 int ds_transpose16(const void*, void*, int, int, int, int64_t, hipStream_t);
 int ds_xent_fwd(const void*, const int64_t*, float*, float*, int64_t, int, int64_t, int, float, int, hipStream_t);
 int ds_xent_bwd(const void*, const int64_t*, const float*, const float*, float, void*, int64_t, int, int64_t, int64_t,
@@ -567,9 +568,45 @@ AttnBias attn_bias(const OptT& kbias, const OptT& abias, const OptT& rpe, int64_
   return r;
 }
 
-std::vector<Tensor> flash_fwd_sparse(Tensor q, Tensor k, Tensor v, double scale, Tensor tiles, Tensor ntiles,
-                                     Tensor qorder, Tensor layout, int64_t blk, bool want_lse, OptT kbias,
-                                     OptT abias, OptT rpe) {
+// The plan of a block-sparse pass (`ops/sparse_attention/block_sparse.py`): tensors [heads or 1, blocks, T] of tiles and masks,
+// [.., n, 4] of work and merges. `contents`: read them back and check every index (a plan that was checked when it was built
+// needs that no more).
+struct SparsePlan {
+  const int *tiles, *masks, *work, *merges;
+  int T, heads, nwork, nmerge, nslots;
+};
+
+SparsePlan sparse_plan(const OptT& tiles, const OptT& masks, const OptT& work, const OptT& merges, int64_t nslots, int64_t H,
+                       int64_t blocks, int64_t ntile, int64_t nhead, bool contents) {
+  for (const OptT* t : {&tiles, &masks, &work, &merges}) {
+    TORCH_CHECK(t->has_value(), "block-sparse plan missing");
+    need(**t, "plan");
+    TORCH_CHECK((*t)->scalar_type() == at::kInt && (*t)->dim() == 3, "block-sparse plan: int32 tensors of three dimensions");
+  }
+  const int64_t LH = tiles->size(0), T = tiles->size(2);
+  TORCH_CHECK((LH == 1 || LH == H) && tiles->size(1) == blocks && masks->sizes() == tiles->sizes(), "block-sparse plan: tiles");
+  TORCH_CHECK(work->size(0) == LH && work->size(1) > 0 && work->size(2) == 4 && merges->size(0) == LH && merges->size(2) == 4,
+              "block-sparse plan: lists");
+  if (contents) {
+    const Tensor code = tiles->cpu(), wk = work->cpu(), mg = merges->cpu();
+    auto in = [](const Tensor& t, int64_t lo, int64_t hi) {  // lo <= t < hi
+      return t.numel() == 0 || (t.min().item<int>() >= lo && t.max().item<int>() < hi);
+    };
+    TORCH_CHECK(in(code.bitwise_and(0xffff), 0, ntile) && in(torch::bitwise_right_shift(code, 16), 0, nhead),
+                "block-sparse plan: tile out of range");
+    TORCH_CHECK(in(wk.select(2, 0), -1, blocks) && in(wk.select(2, 1), 0, T + 1) && in(wk.select(2, 2), 0, T + 1) &&
+                    in(wk.select(2, 1) + wk.select(2, 2), 0, T + 1) && in(wk.select(2, 3), -1, nslots) &&
+                    in(mg.select(2, 0), -1, blocks) && in(mg.select(2, 1), 0, nslots) &&
+                    in(mg.select(2, 1) + mg.select(2, 2), 0, nslots + 1),
+                "block-sparse plan: entry out of range");
+  }
+  return {tiles->data_ptr<int>(), masks->data_ptr<int>(), work->data_ptr<int>(), merges->data_ptr<int>(), (int)T, (int)LH,
+          (int)work->size(1), (int)merges->size(1), (int)nslots};
+}
+
+std::vector<Tensor> flash_fwd_sparse(Tensor q, Tensor k, Tensor v, double scale, Tensor tiles, Tensor masks, Tensor work,
+                                     Tensor merges, int64_t nslots, bool want_lse, OptT kbias, OptT abias, OptT rpe,
+                                     bool check_plan) {
   TORCH_CHECK(q.is_cuda() && k.is_cuda() && v.is_cuda(), "flash_fwd_sparse: device tensors expected");
   TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4, "flash_fwd_sparse: 4-D [B,H,S,D] tensors expected");
   TORCH_CHECK(q.scalar_type() == at::kBFloat16 && k.scalar_type() == at::kBFloat16 && v.scalar_type() == at::kBFloat16,
@@ -581,20 +618,13 @@ std::vector<Tensor> flash_fwd_sparse(Tensor q, Tensor k, Tensor v, double scale,
   TORCH_CHECK(Hq % Hk == 0, "flash_fwd_sparse: Hq must be a multiple of Hk");
   for (const Tensor* t : {&q, &k, &v})
     for (int d = 0; d < 3; ++d) TORCH_CHECK(t->stride(d) % 8 == 0, "flash_fwd_sparse: strides must be multiples of 8");
-  need(tiles, "tiles"); need(ntiles, "ntiles"); need(layout, "layout"); need(qorder, "qorder");
-  TORCH_CHECK(tiles.scalar_type() == at::kInt && ntiles.scalar_type() == at::kInt && layout.scalar_type() == at::kByte,
-              "flash_fwd_sparse: int32 tiles/ntiles, uint8 layout");
-  const int64_t LH = layout.size(0), nb = layout.size(1), nqb = (S + 127) / 128;
-  TORCH_CHECK(layout.dim() == 3 && layout.size(2) == nb && nb * blk >= S, "flash_fwd_sparse: layout [LH, nb, nb]");
-  TORCH_CHECK((LH == 1 || LH == Hq) && tiles.dim() == 3 && tiles.size(0) == LH && tiles.size(1) == nqb &&
-                  ntiles.numel() == LH * nqb && qorder.numel() == LH * nqb && qorder.scalar_type() == at::kInt,
-              "flash_fwd_sparse: LUT shape");
-  TORCH_CHECK(qorder.min().item<int>() >= 0 && qorder.max().item<int>() < nqb, "flash_fwd_sparse: qorder range");
-  // every listed tile must lie inside the key range (the kernel trusts the LUT for its K/V addresses)
-  if (tiles.numel() > 0)
-    TORCH_CHECK(tiles.min().item<int>() >= 0 && tiles.max().item<int>() < (S + 63) / 64 &&
-                    ntiles.max().item<int>() <= tiles.size(2) && ntiles.min().item<int>() >= 0,
-                "flash_fwd_sparse: LUT entries out of range");
+  TORCH_CHECK(S % 128 == 0, "flash_fwd_sparse: sequence length");
+  const SparsePlan pl = sparse_plan(tiles, masks, work, merges, nslots, Hq, S / 128, S / 64, 1, check_plan);
+  Tensor parts, ml;
+  if (pl.nmerge > 0) {
+    parts = torch::empty({B * Hq * nslots, 128, 128}, q.options().dtype(at::kFloat));
+    ml = torch::empty({B * Hq * nslots, 2, 128}, q.options().dtype(at::kFloat));
+  }
   auto o = torch::empty({B, S, Hq, 128}, q.options()).transpose(1, 2);
   Tensor lse;
   if (want_lse) lse = torch::empty({B, Hq, S}, q.options().dtype(at::kFloat));
@@ -603,9 +633,9 @@ std::vector<Tensor> flash_fwd_sparse(Tensor q, Tensor k, Tensor v, double scale,
                 vs[3] = {v.stride(0), v.stride(1), v.stride(2)}, os[3] = {o.stride(0), o.stride(1), o.stride(2)};
   check(ds_flash_fwd_sparse(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                             want_lse ? lse.data_ptr<float>() : nullptr, (int)B, (int)Hq, (int)Hk, (int)S, qs, ks, vs,
-                            os, (float)scale, tiles.data_ptr<int>(), ntiles.data_ptr<int>(), qorder.data_ptr<int>(),
-                            layout.data_ptr<uint8_t>(), (int)tiles.size(2), (int)LH, (int)nb, (int)blk, ab.kb, ab.kbs,
-                            ab.ab, ab.abs_, ab.rp, ab.rhs, ab.rrs, stream()),
+                            os, (float)scale, pl.tiles, pl.masks, pl.work, pl.merges, pl.T, pl.heads, pl.nwork, pl.nmerge, pl.nslots,
+                            parts.defined() ? parts.data_ptr<float>() : nullptr, ml.defined() ? ml.data_ptr<float>() : nullptr,
+                            ab.kb, ab.kbs, ab.ab, ab.abs_, ab.rp, ab.rhs, ab.rrs, stream()),
         "flash_fwd_sparse");
   return {o, lse};
 }
@@ -615,8 +645,8 @@ std::vector<Tensor> flash_fwd_sparse(Tensor q, Tensor k, Tensor v, double scale,
 // [Hk, nkb, T] of (head-in-group << 16 | 32-row tile), nqt int32 [Hk, nkb], layout uint8 [LH, nb, nb], granularity
 // blk). Returns dq, dk, dv laid out [B,S,H,128] in memory (viewed [B,H,S,128]) like flash_fwd's output.
 std::vector<Tensor> flash_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, Tensor dout, double scale,
-                              int64_t mode, OptT qtiles, OptT nqt, OptT layout, int64_t blk, OptT kbias, OptT abias,
-                              OptT rpe) {
+                              int64_t mode, OptT qtiles, OptT qmasks, OptT work, OptT merges, int64_t nslots, OptT kbias,
+                              OptT abias, OptT rpe, bool check_plan) {
   for (const Tensor* t : {&q, &k, &v, &o, &dout}) {
     TORCH_CHECK(t->is_cuda() && t->dim() == 4 && t->scalar_type() == at::kBFloat16, "flash_bwd: 4-D bf16 device tensors");
     TORCH_CHECK(t->size(3) == 128 && t->stride(3) == 1, "flash_bwd: head dim 128 with unit last stride");
@@ -630,29 +660,19 @@ std::vector<Tensor> flash_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse
   TORCH_CHECK(lse.is_cuda() && lse.scalar_type() == at::kFloat && lse.is_contiguous() && lse.numel() == B * Hq * S,
               "flash_bwd: lse [B,Hq,S] fp32 contiguous");
   TORCH_CHECK(mode >= 0 && mode <= 2, "flash_bwd: mode");
-  const int* qt = nullptr; const int* nq = nullptr; const uint8_t* lay = nullptr;
-  int maxt = 0, LH = 1, nb = 0;
+  SparsePlan pl{};
+  pl.heads = 1;
+  const int64_t nkb = (S + 255) / 256;
   if (mode == 2) {
-    TORCH_CHECK(qtiles.has_value() && nqt.has_value() && layout.has_value(), "flash_bwd: sparse LUT required");
-    need(*qtiles, "qtiles"); need(*nqt, "nqt"); need(*layout, "layout");
-    TORCH_CHECK(qtiles->scalar_type() == at::kInt && nqt->scalar_type() == at::kInt &&
-                    layout->scalar_type() == at::kByte, "flash_bwd: int32 qtiles/nqt, uint8 layout");
-    const int64_t nkb = (S + 255) / 256;
-    LH = (int)layout->size(0); nb = (int)layout->size(1);
-    TORCH_CHECK(layout->dim() == 3 && layout->size(2) == nb && nb * blk >= S && (LH == 1 || LH == Hq),
-                "flash_bwd: layout [LH, nb, nb]");
-    TORCH_CHECK(qtiles->dim() == 3 && qtiles->size(0) == Hk && qtiles->size(1) == nkb && nqt->numel() == Hk * nkb,
-                "flash_bwd: LUT shape");
-    maxt = (int)qtiles->size(2);
-    if (nqt->numel() > 0) TORCH_CHECK(nqt->max().item<int>() <= maxt && nqt->min().item<int>() >= 0, "flash_bwd: nqt");
-    if (qtiles->numel() > 0) {  // the kernel trusts the LUT for its Q / dO addresses
-      const int ntq = (int)((S + 31) / 32), rep = (int)(Hq / Hk);
-      auto codes = qtiles->masked_fill(qtiles->lt(0), 0);
-      TORCH_CHECK((codes.bitwise_and(0xffff)).max().item<int>() < ntq && torch::bitwise_right_shift(codes, 16).max().item<int>() < rep,
-                  "flash_bwd: LUT entries out of range");
-    }
-    qt = qtiles->data_ptr<int>(); nq = nqt->data_ptr<int>(); lay = layout->data_ptr<uint8_t>();
+    TORCH_CHECK(S % 128 == 0, "flash_bwd: block-sparse sequence length");
+    pl = sparse_plan(qtiles, qmasks, work, merges, nslots, Hk, nkb, S / 32, Hq / Hk, check_plan);
   }
+  const int64_t slots = mode == 2 ? (pl.nmerge > 0 ? nslots : 0) : [&] {
+    const int n = ds_flash_bwd_split((int)B, (int)Hq, (int)Hk, (int)S);
+    return n > 1 ? n * nkb : (int64_t)0;
+  }();
+  Tensor parts;
+  if (slots) parts = torch::empty({B * Hk * slots, 65536}, q.options().dtype(at::kFloat));
   const AttnBias ab = attn_bias(kbias, abias, rpe, B, Hq, S);
   TORCH_CHECK(mode == 2 || (!ab.kb && !ab.ab && !ab.rp), "flash_bwd: score biases need the block-sparse mode");
   // the kernel loads all three bias terms unconditionally: absent ones read one zero float
@@ -669,9 +689,10 @@ std::vector<Tensor> flash_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse
   st3(q, qs); st3(k, ks); st3(v, vs); st3(o, os); st3(dout, gs); st3(dq, dqs); st3(dk, dks); st3(dv, dvs);
   check(ds_flash_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dout.data_ptr(), lse.data_ptr<float>(),
                      delta.data_ptr<float>(), dqacc.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-                     (int)B, (int)Hq, (int)Hk, (int)S, qs, ks, vs, os, gs, dqs, dks, dvs, (float)scale, (int)mode, qt,
-                     nq, lay, maxt, LH, nb, (int)blk, flags, zp(ab.kb), ab.kbs, zp(ab.ab), ab.abs_, zp(ab.rp), ab.rhs,
-                     ab.rrs, stream()),
+                     (int)B, (int)Hq, (int)Hk, (int)S, qs, ks, vs, os, gs, dqs, dks, dvs, (float)scale, (int)mode, pl.tiles,
+                     pl.masks, pl.work, pl.merges, pl.T, pl.heads, pl.nwork, pl.nmerge, pl.nslots,
+                     slots ? parts.data_ptr<float>() : nullptr, flags, zp(ab.kb), ab.kbs, zp(ab.ab), ab.abs_, zp(ab.rp),
+                     ab.rhs, ab.rrs, stream()),
         "flash_bwd");
   return {dq, dk, dv};
 }
@@ -720,12 +741,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("transpose16", &transpose16, py::arg("x"), py::arg("pad_to") = 0);
   m.def("flash_fwd", &flash_fwd);
   m.def("flash_fwd_sparse", &flash_fwd_sparse, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("scale"),
-        py::arg("tiles"), py::arg("ntiles"), py::arg("qorder"), py::arg("layout"), py::arg("blk"), py::arg("want_lse"),
-        py::arg("kbias") = py::none(), py::arg("abias") = py::none(), py::arg("rpe") = py::none());
+        py::arg("tiles"), py::arg("masks"), py::arg("work"), py::arg("merges"), py::arg("nslots"), py::arg("want_lse"),
+        py::arg("kbias") = py::none(), py::arg("abias") = py::none(), py::arg("rpe") = py::none(), py::arg("check_plan") = true);
   m.def("flash_bwd", &flash_bwd, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("o"), py::arg("lse"),
-        py::arg("dout"), py::arg("scale"), py::arg("mode"), py::arg("qtiles") = py::none(), py::arg("nqt") = py::none(),
-        py::arg("layout") = py::none(), py::arg("blk") = 0, py::arg("kbias") = py::none(),
-        py::arg("abias") = py::none(), py::arg("rpe") = py::none());
+        py::arg("dout"), py::arg("scale"), py::arg("mode"), py::arg("qtiles") = py::none(), py::arg("qmasks") = py::none(),
+        py::arg("work") = py::none(), py::arg("merges") = py::none(), py::arg("nslots") = 0, py::arg("kbias") = py::none(),
+        py::arg("abias") = py::none(), py::arg("rpe") = py::none(), py::arg("check_plan") = true);
   m.def("xent_fwd", &xent_fwd);
   m.def("xent_bwd", &xent_bwd);
 }

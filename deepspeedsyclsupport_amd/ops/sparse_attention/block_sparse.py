@@ -3,14 +3,20 @@
 
 Forward: `csrc/attn/flash_fwd.hip` in its SPARSE instantiation — every workgroup (one 128-row query block of one
 head) visits only the 64-key tiles its layout rows touch, listed in a LUT built here once per (layout, sequence
-length), and masks inside a tile at the layout's block granularity. Work and K/V traffic therefore scale with the
+length), and masks inside a tile by 16 x 16 pieces. Work and K/V traffic therefore scale with the
 layout density. Head dims below 128 are zero-padded to 128 (zeros change neither QK^T nor the kept part of PV).
 
 Backward: `csrc/attn/flash_bwd.hip` in its SPARSE instantiation (reference: the transposed DSD/SDD products of
 `matmul.py:605` and the sparse softmax backward `softmax.py:213`) — every workgroup (256 keys of one head) visits
-only the 32-row query tiles its key block meets in the layout (a column LUT built here) and masks at the layout's
-block granularity, recomputing P from the forward's LSE. No [L, L] tensor is ever built; work scales with density.
+only the 32-row query tiles its key block meets in the layout (a column LUT built here) and masks likewise,
+recomputing P from the forward's LSE. No [L, L] tensor is ever built; work scales with density.
+
+`SparsePlan` holds what both passes read: the lists, their masks, and how the lists are shared out over workgroups (a row or
+column that is much longer than the others is cut into parts).
 """
+from collections import namedtuple
+
+import numpy as np
 import torch
 
 from ..native import hip_ops
@@ -18,19 +24,23 @@ from ..native import hip_ops
 _LUTS = {}
 
 
+def _bits(layout):
+    return layout.detach().cpu().contiguous().numpy() != 0
+
+
 def _lut_key(layout, blk, L, device):
-    import hashlib
-    digest = hashlib.sha1(layout.detach().to("cpu", torch.uint8).contiguous().numpy().tobytes()).hexdigest()
-    return (digest, tuple(layout.shape), blk, L, str(device))
+    """The layout's contents (one bit per block) and what else a LUT depends on."""
+    bits = layout if isinstance(layout, np.ndarray) else _bits(layout)
+    return (np.packbits(bits).tobytes(), bits.shape, blk, L, str(device))
 
 
-def build_lut(layout, blk, L, device):
+def build_lut(layout, blk, L, device, key=None):
     """layout [H, nb, nb] (0/1) -> (tiles int32 [LH, nqb, T], ntiles int32 [LH, nqb], layout uint8 [LH, nb, nb],
     qorder int32 [LH, nqb] = query blocks by descending tile count, the kernel's launch order).
 
     LH = 1 when every head shares one layout. Tile t of query block qb is listed when any key of 64-key tile t is
     allowed for any of the 128 query rows of qb; the tile lists are ascending."""
-    key = _lut_key(layout, blk, L, device)
+    key = key or _lut_key(layout, blk, L, device)
     hit = _LUTS.get(key)
     if hit is not None:
         return hit
@@ -58,10 +68,10 @@ def build_lut(layout, blk, L, device):
 _BWD_LUTS = {}
 
 
-def build_bwd_lut(layout, blk, L, H, device):
+def build_bwd_lut(layout, blk, L, H, device, key=None):
     """Column LUT of the sparse backward: (qtiles int32 [H, nkb, T] = 32-row query tiles met by each 256-key block,
     ascending, nqt int32 [H, nkb], layout uint8 [LH, nb, nb] at granularity blk' = min(blk, 128), blk')."""
-    key = _lut_key(layout, blk, L, device) + (H,)
+    key = (key or _lut_key(layout, blk, L, device)) + (H,)
     hit = _BWD_LUTS.get(key)
     if hit is not None:
         return hit
@@ -93,6 +103,106 @@ def build_bwd_lut(layout, blk, L, H, device):
     return out
 
 
+# Workgroups that the chip holds at once (two of the forward's per CU, one of the backward's) and the shortest part worth cutting:
+# a part costs its operands' first load and a pass of its accumulators through memory, 64 KB in the forward, 256 KB in the
+# backward. Measured, us, BigBird of 64-key blocks, forward with parts of at least 4 / 8 / 16 / 32 tiles, backward with 8 / 16 /
+# 32 / 64: B2 H8 L16384 126 / 113 / 119 / 110 and 520 / 506 / 513 / 506; B1 H8 L4096 31 / 28 / 36 / 56 and 102 / 98 / 100 / 162;
+# B1 H4 L2048 23 / 21 / 32 / 52 and 47 / 72 / 89 / 154. A share of half a chip cuts layouts that fill it by themselves (Fixed,
+# L8192: forward 90 -> 107).
+_FWD_SHARE, _BWD_SHARE = (512, 8), (256, 8)
+
+PlanSide = namedtuple("PlanSide", "tiles masks work merges nslots")
+
+
+def _share_out(counts, copies, slots, least):
+    """counts [LH, n] list lengths; `copies` workgroups sets run side by side -> (work [LH, W, 4], merges [LH, M, 4], nslots):
+    lists far longer than an equal share of all the work are cut evenly. Entries as in the kernels; -1 pads."""
+    limit = max(least, -(-int(counts.sum()) * copies // slots))
+    work, merges, nslots = [], [], 0
+    for row in counts.tolist():
+        entries, joins, used = [], [], 0
+        for i, n in enumerate(row):
+            parts = 1 if n <= limit * 3 // 2 else -(-n // limit)
+            for p in range(parts):
+                a = n * p // parts
+                entries.append((i, a, n * (p + 1) // parts - a, used + p if parts > 1 else -1))
+            if parts > 1:
+                joins.append((i, used, parts, 0))
+                used += parts
+        work.append(sorted(entries, key=lambda e: -e[2]))   # longest first
+        merges.append(joins)
+        nslots = max(nslots, used)
+
+    def pad(lists):
+        width = max(len(x) for x in lists)
+        flat = [e for x in lists for e in x + [(-1, 0, 0, -1 if lists is work else 0)] * (width - len(x))]
+        return torch.tensor(flat, dtype=torch.int32).reshape(len(lists), width, 4)
+
+    return pad(work), pad(merges), nslots
+
+
+def _tile_masks(bits, blk, L, rows, cols):
+    """Layout [LH, nb, nb] (bool) -> int32 [LH, tiles down, tiles across] for tiles of rows x cols pieces of 16 x 16 tokens (8 x 4
+    or 2 x 16): bit r * cols + k is piece (r, k). Across, the last tile may reach past L: nothing is seen there."""
+    f, n = blk // 16, L // 16
+    seen = bits.repeat(f, 2)[:, :, :n]
+    seen = np.pad(seen, ((0, 0), (0, 0), (0, -n % 16)))
+    row = np.packbits(seen, axis=-1, bitorder="little")              # [LH, nb, pieces / 8]
+    if cols == 4:
+        row = np.stack([row & 15, row >> 4], -1).reshape(row.shape[0], row.shape[1], -1)[:, :, :n // 4]
+    else:
+        row = row.view("<u2")
+    row = row.astype(np.uint32).repeat(f, 1)[:, :n].reshape(row.shape[0], n // rows, rows, -1)
+    mask = row[:, :, 0].copy()
+    for r in range(1, rows):
+        mask |= row[:, :, r] << np.uint32(cols * r)
+    return torch.from_numpy(mask.view(np.int32))
+
+
+class SparsePlan:
+    """What the kernels read for one layout, sequence length and batch x heads; each side is made when it is first needed."""
+
+    def __init__(self, bits, blk, L, B, H, device):
+        self.layout, self.blk, self.L, self.B, self.H, self.device = torch.from_numpy(bits), blk, L, B, H, device
+        self.key, self.sides = _lut_key(bits, blk, L, "cpu"), {}
+
+    def _side(self, tiles, masks, counts, share):
+        LH = tiles.shape[0]
+        work, merges, nslots = _share_out(counts, self.B * self.H if LH == 1 else self.B, *share)
+        parts = (tiles, masks.gather(2, tiles.long()), work, merges)
+        flat = torch.cat([t.reshape(-1) for t in parts]).to(self.device)   # one copy to the device
+        return PlanSide(*(t.view(p.shape) for t, p in zip(flat.split([p.numel() for p in parts]), parts)), nslots)
+
+    def forward(self):
+        if "fwd" not in self.sides:
+            tiles, counts, lay, _ = build_lut(self.layout, self.blk, self.L, "cpu", self.key)
+            masks = _tile_masks(self.layout[:lay.shape[0]].numpy(), self.blk, self.L, 8, 4)
+            self.sides["fwd"] = self._side(tiles, masks, counts, _FWD_SHARE)
+        return self.sides["fwd"]
+
+    def backward(self):
+        if "bwd" not in self.sides:
+            LH = build_lut(self.layout, self.blk, self.L, "cpu", self.key)[2].shape[0]
+            codes, counts, _, _ = build_bwd_lut(self.layout, self.blk, self.L, LH, "cpu", self.key)
+            masks = _tile_masks(self.layout[:LH].numpy(), self.blk, self.L, 2, 16).transpose(1, 2)   # listed by key block
+            self.sides["bwd"] = self._side(codes, masks, counts, _BWD_SHARE)
+        return self.sides["bwd"]
+
+
+_PLANS = {}
+
+
+def sparse_plan(layout, blk, L, B, H, device):
+    bits = _bits(layout)
+    key = _lut_key(bits, blk, L, device) + (B, H)
+    plan = _PLANS.get(key)
+    if plan is None:
+        if len(_PLANS) > 64:
+            _PLANS.clear()
+        plan = _PLANS[key] = SparsePlan(bits, blk, L, B, H, device)
+    return plan
+
+
 def token_bias(layout, blk, L, H, dtype, device):
     """Additive [1, H, L, L] bias: 0 where the layout allows, -inf elsewhere. Reference semantics for tests and
     host fallbacks only — the kernels never build it."""
@@ -111,22 +221,22 @@ class BlockSparseAttnFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, layout, blk, scale, kbias, abias, rpe):
         B, H, L, D = q.shape
-        tiles, ntiles, lay_u8, qorder = build_lut(layout, blk, L, q.device)
+        plan = sparse_plan(layout, blk, L, B, H, q.device)
         if D < 128:
             pad = (0, 128 - D)
             qp, kp, vp = (torch.nn.functional.pad(t, pad) for t in (q, k, v))
         else:
             qp, kp, vp = q, k, v
         need_grad = any(t.requires_grad for t in (q, k, v))
-        o, lse = hip_ops().flash_fwd_sparse(qp, kp, vp, float(scale), tiles, ntiles, qorder, lay_u8, int(blk),
-                                              need_grad, kbias, abias, rpe)
+        o, lse = hip_ops().flash_fwd_sparse(qp, kp, vp, float(scale), *plan.forward(), need_grad, kbias, abias, rpe,
+                                            check_plan=False)
         o_full = o
         if D < 128:
             o = o[..., :D]
         if need_grad:
             ctx.save_for_backward(q, k, v, o_full, lse, *[t for t in (kbias, abias, rpe) if t is not None])
             ctx.has_bias = (kbias is not None, abias is not None, rpe is not None)
-            ctx.layout, ctx.blk, ctx.scale = layout, blk, float(scale)
+            ctx.plan, ctx.scale = plan, float(scale)
         return o
 
     @staticmethod
@@ -135,13 +245,13 @@ class BlockSparseAttnFn(torch.autograd.Function):
         it = iter(bias)
         kbias, abias, rpe = (next(it) if has else None for has in ctx.has_bias)
         B, H, L, D = q.shape
-        qtiles, nqt, lay_u8, blk = build_bwd_lut(ctx.layout, ctx.blk, L, H, q.device)
         if D < 128:
             pad = (0, 128 - D)
             q, k, v, do = (torch.nn.functional.pad(t, pad) for t in (q, k, v, do))
         elif do.stride(-1) != 1 or any(s % 8 for s in do.stride()[:3]):
             do = do.contiguous()
-        dq, dk, dv = hip_ops().flash_bwd(q, k, v, o, lse, do, ctx.scale, 2, qtiles, nqt, lay_u8, blk, kbias, abias, rpe)
+        dq, dk, dv = hip_ops().flash_bwd(q, k, v, o, lse, do, ctx.scale, 2, *ctx.plan.backward(), kbias, abias, rpe,
+                                         check_plan=False)
         if D < 128:
             dq, dk, dv = dq[..., :D], dk[..., :D], dv[..., :D]
         return dq, dk, dv, None, None, None, None, None, None

@@ -1,0 +1,95 @@
+"""How block-sparse lists are shared out over workgroups: the plan against the layout, and cut lists against dense attention."""
+import pytest
+import torch
+
+from deepspeedsyclsupport_amd.ops.sparse_attention import block_sparse as bs
+from deepspeedsyclsupport_amd.ops.sparse_attention.sparsity_config import BigBirdSparsityConfig, FixedSparsityConfig
+
+
+def _layout(kind, H, blk, L, seed=0):
+    n = L // blk
+    g = torch.Generator().manual_seed(seed)
+    lay = (torch.rand(H, n, n, generator=g) < 0.15).long()
+    lay[:, torch.arange(n), torch.arange(n)] = 1
+    lay[:, 0] = 1       # a global row and a global column
+    lay[:, :, 0] = 1
+    if kind == "shared":
+        lay = lay[:1].expand(H, -1, -1).contiguous()
+    elif kind == "empty":
+        lay[:, n // 2:] = 0
+        lay[:, :, n // 3:2 * n // 3] = 0
+    return lay
+
+
+def _covered(side, high, wide, L, head):
+    """Times that each 16 x 16 piece is visited, from the lists; blocks are `high` x `wide` tokens (tiles along the other axis)."""
+    seen, slots = torch.zeros(L // 16, -(-L // 256) * 16, dtype=torch.long), {}
+    for blk, first, n, slot in side.work[head].tolist():
+        if blk < 0:
+            continue
+        slots.setdefault(blk, []).append(slot)
+        for j in range(first, first + n):
+            t, m = side.tiles[head, blk, j].item(), side.masks[head, blk, j].item()
+            r0, c0, rows, cols = (blk * 8, t * 4, 8, 4) if (high, wide) == (128, 64) else (t * 2, blk * 16, 2, 16)
+            for r in range(rows):
+                for k in range(cols):
+                    seen[r0 + r, c0 + k] += (m >> (r * cols + k)) & 1
+    return seen[:, :L // 16], slots
+
+
+@pytest.mark.parametrize("kind", ["shared", "heads", "empty"])
+@pytest.mark.parametrize("blk,L", [(16, 256), (32, 640), (64, 1152), (128, 1280), (256, 1280)])
+def test_plan_visits_the_layout_once(kind, blk, L, monkeypatch):
+    monkeypatch.setattr(bs, "_FWD_SHARE", (1 << 20, 2))
+    monkeypatch.setattr(bs, "_BWD_SHARE", (1 << 20, 3))
+    bs._PLANS.clear()
+    H = 2
+    lay = _layout(kind, H, blk, L)
+    plan = bs.sparse_plan(lay, blk, L, 1, H, "cpu")
+    want = (lay != 0).repeat_interleave(blk // 16, 1).repeat_interleave(blk // 16, 2)[:, :L // 16, :L // 16].long()
+    for side, high, wide, blocks in ((plan.forward(), 128, 64, L // 128), (plan.backward(), 32, 256, -(-L // 256))):
+        for head in range(side.work.shape[0]):
+            seen, slots = _covered(side, high, wide, L, head)
+            assert torch.equal(seen, want[head])
+            assert sorted(slots) == list(range(blocks))          # blocks without a tile are written too
+            merged = {b: list(range(s, s + n)) for b, s, n, _ in side.merges[head].tolist() if b >= 0}
+            for b, got in slots.items():
+                assert got == [-1] if b not in merged else sorted(got) == merged[b]
+            used = [s for got in merged.values() for s in got]
+            assert len(set(used)) == len(used) and all(0 <= s < side.nslots for s in used)
+    bs._PLANS.clear()
+    if kind != "empty":
+        assert plan.forward().nslots > 0 or L <= 256
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,blk,L,kind,bias", [(128, 64, 1152, "shared", False), (64, 32, 1024, "heads", True),
+                                               (128, 16, 512, "empty", False), (128, 128, 1408, "shared", True)])
+def test_cut_lists_match_dense_attention(D, blk, L, kind, bias, monkeypatch):
+    """Lists cut after two (three) tiles, so that nearly every block is merged; rows without a key come out as zero."""
+    monkeypatch.setattr(bs, "_FWD_SHARE", (1 << 20, 2))
+    monkeypatch.setattr(bs, "_BWD_SHARE", (1 << 20, 3))
+    bs._PLANS.clear()
+    torch.manual_seed(3)
+    B, H = 2, 2
+    lay = _layout(kind, H, blk, L)
+    q, k, v, do = (torch.randn(B, H, L, D, device="cuda").bfloat16() for _ in range(4))
+    kpm = None
+    if bias:
+        kpm = torch.zeros(B, L, device="cuda")
+        kpm[:, L - L // 4:] = -10000.0
+    ins = [t.clone().requires_grad_(True) for t in (q, k, v)]
+    o = bs.block_sparse_attention(*ins, lay, blk, key_padding_mask=kpm)
+    got = [o, *torch.autograd.grad(o, ins, do)]
+    assert bs.sparse_plan(lay, blk, L, B, H, q.device).forward().nslots > 0
+    bs._PLANS.clear()
+    ref_in = [t.float().requires_grad_(True) for t in (q, k, v)]
+    s = ref_in[0] @ ref_in[1].transpose(-1, -2) * D**-0.5 + (0 if kpm is None else kpm[:, None, None, :])
+    ok = (lay != 0).repeat_interleave(blk, 1).repeat_interleave(blk, 2)[:, :L, :L].cuda()
+    p = torch.softmax(s.masked_fill(~ok, float("-inf")), -1)
+    ref = torch.where(ok.any(-1)[None, :, :, None], torch.nan_to_num(p), 0.0) @ ref_in[2]
+    want = [ref, *torch.autograd.grad(ref, ref_in, do.float())]
+    for name, a, b in zip(("o", "dq", "dk", "dv"), got, want):
+        # bf16 operands, weights and results: 2^-8 each, a few of them in a row
+        err = (a.float() - torch.nan_to_num(b)).norm() / b.nan_to_num().norm()
+        assert err < 0.015, (name, err.item())

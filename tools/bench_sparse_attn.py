@@ -33,10 +33,10 @@ def main():
                           ("fixed64", FixedSparsityConfig(num_heads=H, block=64, num_local_blocks=4))):
             layout = cfg.make_layout(L)
             q, k, v = (torch.randn(B, H, L, D, device="cuda").bfloat16() for _ in range(3))
-            tiles, ntiles, lay, qorder = bs.build_lut(layout, cfg.block, L, q.device)
+            ntiles = bs.build_lut(layout, cfg.block, L, q.device)[1]
             density = ntiles.float().mean().item() / (L // 64)
-            t_sparse = timeit(lambda: hip_ops().flash_fwd_sparse(q, k, v, D**-0.5, tiles, ntiles, qorder, lay,
-                                                                 cfg.block, False))
+            plan = bs.sparse_plan(layout, cfg.block, L, B, H, q.device).forward()
+            t_sparse = timeit(lambda: hip_ops().flash_fwd_sparse(q, k, v, D**-0.5, *plan, False, check_plan=False))
             t_dense = timeit(lambda: hip_ops().flash_fwd(q, k, v, False, D**-0.5, False))
             bias = bs.token_bias(layout, cfg.block, L, H, torch.bfloat16, q.device)
             t_sdpa = timeit(lambda: torch.nn.functional.scaled_dot_product_attention(q, k, v, attn_mask=bias))
