@@ -1,6 +1,6 @@
-// Ragged paged flash attention for inference prefill / prompt chunks (SplitFuse): entry points. The kernel is in
-// paged_prefill_core.h.
-#include "paged_prefill_core.h"
+// Ragged paged flash attention for inference prefill / prompt chunks (SplitFuse): entry points. The kernels are in
+// paged_flash.h (heads of 128) and paged_prefill_core.h (other widths and page sizes).
+#include "paged_flash.h"
 
 // q / o [T, Hq, D] bf16 (contiguous), caches [blocks, Hk, BS, D] bf16, D in {64, 80, 96, 128, 256}, block_table
 // [nseq, max_blocks] int32, start [nseq], cu_q [nseq + 1], work [nwork, 2] (sequence, 128-row query block) int32,
@@ -14,6 +14,7 @@ extern "C" int ds_paged_prefill(const void* q, const void* kc, const void* vc, v
   PagedArgs a{(const bf16*)q, (const bf16*)kc, (const bf16*)vc, (bf16*)o, block_table, start, cu_q, work, alibi,
               Hq, Hk, BS, max_blocks, window, scale * 1.4426950408889634f, 1.f / scale, D, D, 0, nullptr, nullptr, 0, 0, 0, 0, 0, nullptr, (int64_t)Hq * D,
               (int64_t)Hq * D, nullptr, 0, 0.f, 0.f};
+  if (paged_flash_fits(a)) return launch_flash<PLAIN>(a, nwork, st);
   switch (D) {
     case 64: return launch<64, 64, PLAIN>(a, nwork, st);
     case 80: return launch<80, 80, PLAIN>(a, nwork, st);
@@ -42,6 +43,7 @@ extern "C" int ds_paged_prefill_ext(const void* q, const void* kc, const void* v
               Hq, Hk, BS, max_blocks, window, cap ? 1.f : scale * LOG2E, 1.f / scale, dk, dv, chunk,
               sink, nullptr, 0, 0, 0, 0, 0, nullptr, ldo, (int64_t)Hq * dk, (const bf16*)gate, ldg,
               cap ? scale / softcap * 2.f * LOG2E : 0.f, cap ? softcap * LOG2E : 0.f};
+  if (paged_flash_fits(a)) return launch_flash<EXT_>(a, nwork, st);
 #define DS_ROW(K)                                              \
   {                                                            \
     if (dv <= 32) return launch<K, 32, EXT_>(a, nwork, st);    \

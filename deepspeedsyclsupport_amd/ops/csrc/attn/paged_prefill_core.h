@@ -10,7 +10,7 @@
 //    values are read straight from the paged cache [blocks, Hk, BS, D] through the block table — the new tokens'
 //    K/V were appended by the fused QKV epilogue first, so a chunk sees its whole cached prefix plus itself;
 //  * a host-built work list names (sequence, 128-row query block) pairs, so ragged lengths cost no padding beyond one
-//    block; every q head of a work item sits on one XCD (xcd_remap) so the GQA group's K/V tiles are shared in L2;
+//    block; workgroups go head by head (xcd_remap), so that an XCD's L2 serves few heads' K/V tiles;
 //  * per query row the position is start + i: causal masking against absolute positions, ALiBi bias
 //    slope_h * (key - pos) folded into the score before the online softmax, sliding window key > pos - window; tiles
 //    entirely outside [pos - window, pos] are never loaded;
@@ -22,7 +22,7 @@
 //    arguments. It keeps the softmax weights to 16 mantissa bits through the P.V product (two bf16 operands, high + low);
 //  * a third (LATENT) reads keys and values that were expanded from cached latents: rows laid end to end, a sequence's from
 //    kv_offs on, [keys of all heads | values of all heads] per row, with the last key columns (one rotated part for all
-//    heads) in the latent's own row. Its workgroups go head by head, so an XCD's L2 serves one head's keys;
+//    heads) in the latent's own row;
 //  * EXT and LATENT take a softmax sink per head: exp(sink) joins the denominator; EXT a gate per token and head: the output
 //    times its sigmoid;
 //  * the head dim is a template parameter: D / 16 MFMA steps for the scores, ceil(D / 32) output column tiles (D = 80
@@ -98,9 +98,9 @@ __global__ void __launch_bounds__(NTHR, (Cfg<DK, DV>::OCC)) paged_prefill_kernel
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, h = lane >> 5, l32 = lane & 31;
   const int logical = xcd_remap(blockIdx.x, gridDim.x);
   const int per_head = gridDim.x / a.Hq;
-  // (LATENT: the longest rows of a head first, they are the last of the work list)
-  const int w = LAT ? per_head - 1 - logical % per_head : logical / a.Hq;
-  const int hq = LAT ? logical / per_head : logical % a.Hq, hk = hq / (a.Hq / a.Hk);
+  // head by head, the longest rows of a head first (they are the last of the work list): row by row, an XCD got all heads of a
+  // run of neighbouring query blocks, the last XCD 15 / 8 of the mean work
+  const int w = per_head - 1 - logical % per_head, hq = logical / per_head, hk = hq / (a.Hq / a.Hk);
   const int seq = a.work[2 * w], qb = a.work[2 * w + 1];
   const int t0 = a.cu_q[seq], n = a.cu_q[seq + 1] - t0, start = a.start[seq], Skv = start + n;
   const int q0 = qb * BM, q0w = q0 + wid * 32;

@@ -81,3 +81,50 @@ def test_uniform_tables_are_cached():
     assert a[0] is b[0] and a[1] is b[1]
     assert a[0].tolist() == [0, 300, 600, 900]
     assert a[1].tolist() == [[s, q] for s in range(3) for q in range(3)]
+
+
+@pytest.mark.parametrize("BS", [16, 32, 128])
+@pytest.mark.parametrize("form", ["plain", "alibi", "window", "chunk", "cap", "cap_high", "sink_gate"])
+def test_pages_of_two_powers_match_other_pages(form, BS):
+    """Heads of 128 over pages of 16, 32, .. tokens take their own kernel; pages of 24 take the one for any width. Lengths at the
+    edges of tiles, query blocks and pages; an output that is columns of a wider matrix."""
+    from deepspeedsyclsupport_amd.inference.model_implementations.transformer import RaggedMeta, alibi_slopes
+    from deepspeedsyclsupport_amd.ops import hybrid_ops
+    from deepspeedsyclsupport_amd.ops.native import hip_ops
+    lens, starts, Hq, Hk, D = [1, 64, 128, 129, 15, 200], [17, 0, 64, 1, 240, 500], 4, 2, 128
+    g = torch.Generator(device="cuda").manual_seed(7)
+    T, L = sum(lens), [s + n for s, n in zip(starts, lens)]
+    q = torch.randn(T, Hq, D, device="cuda", generator=g).bfloat16() * 2
+    keys, vals = ([torch.randn(n, Hk, D, device="cuda", generator=g).bfloat16() for n in L] for _ in range(2))
+    gate = torch.randn(T, Hq, device="cuda", generator=g).bfloat16()
+    sink = torch.randn(Hq, device="cuda", generator=g)
+
+    def run(size):
+        blocks, used = [], 0
+        for n in L:
+            blocks.append([used + i for i in range(-(-n // size))][::-1])
+            used += -(-n // size)
+        # rows that no token has written hold anything: they must not reach the result
+        kc, vc = (torch.full((used, Hk, size, D), float("nan"), device="cuda").bfloat16() for _ in range(2))
+        for b, k, v in zip(blocks, keys, vals):
+            for j, blk in enumerate(b):
+                part = slice(j * size, (j + 1) * size)
+                kc[blk, :, :k[part].shape[0]] = k[part].transpose(0, 1)
+                vc[blk, :, :v[part].shape[0]] = v[part].transpose(0, 1)
+        m = RaggedMeta.build(starts, lens, blocks, 0, size, torch.device("cuda"))
+        if form in ("plain", "alibi", "window"):
+            return hip_ops().paged_prefill(q, kc, vc, m.block_tables, m.start_pos, m.cu_q, m.work,
+                                           alibi_slopes(Hq).cuda() if form == "alibi" else None, 70 if form == "window" else 0,
+                                           D**-0.5).view(T, Hq * D)
+        how = {"chunk": dict(chunk=100), "cap": dict(softcap=20.0), "cap_high": dict(softcap=60.0, window=90),
+               "sink_gate": dict(sink=sink, gate=gate)}[form]
+        wide = torch.zeros(T, Hq * D + 64, device="cuda", dtype=torch.bfloat16)
+        hybrid_ops.ragged_attention(q, kc, vc, m, D**-0.5, out=wide[:, 64:], **how)
+        assert not wide[:, :64].any()
+        return wide[:, 64:]
+
+    a, b = run(BS).float(), run(24).float()
+    assert torch.isfinite(a).all()
+    # results and (plain forms) weights are bf16: a few units of 2^-9 of the rows' size
+    assert ((a - b).norm() / b.norm()).item() < 6e-3
+    torch.testing.assert_close(a, b, rtol=2e-2, atol=2e-2)
