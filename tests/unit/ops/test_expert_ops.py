@@ -148,6 +148,33 @@ def test_experts_any_rows(path, monkeypatch):
 
 
 # ------------------------------------------------------------------------------------------------ rotary attention
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["silu_glu", "relu2", None])
+@pytest.mark.parametrize("N,K", [(32, 64), (96, 192), (160, 128), (288, 320)])
+def test_big_tiles_at_their_edges(N, K, act):
+    """256 x 256 tiles: experts whose rows end a tile, a wave's half or 32 rows of it early, late or not at all, one without
+    rows; columns that fill no tile; odd and even numbers of steps."""
+    from deepspeedsyclsupport_amd.ops.expert_ops import ACTS, expert_ops, operand_order
+    counts = [256, 0, 1, 257, 31, 33, 128, 129, 255, 513, 160, 32]
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    E, n = len(counts), sum(counts)
+    assert n >= 128 * E
+    parts = 2 if act == "silu_glu" else 1
+    w = (torch.randn(E, parts * N, K, device="cuda", generator=g) * K**-0.5).bfloat16()
+    x = torch.randn(n, K, device="cuda", generator=g).bfloat16()
+    experts = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(n, generator=torch.Generator().manual_seed(1))]
+    order = torch.argsort(experts, stable=True).int().cuda()
+    offs = torch.tensor([0, *counts]).cumsum(0).int().cuda()
+    y = expert_ops().expert_gemm(x, operand_order(w), experts.int().cuda(), offs, order, 1, ACTS[act] if act else 0, True, True)
+    z = torch.stack([x[i].float() @ w[e].float().t() for i, e in enumerate(experts.tolist())])
+    if act == "silu_glu":
+        z = torch.nn.functional.silu(z[:, :N]) * z[:, N:]
+    elif act:
+        z = torch.relu(z)**2
+    torch.testing.assert_close(y.float(), z, rtol=2e-2, atol=1e-2)   # sums in fp32, one rounding to bf16
+    assert ((y.float() - z).norm() / z.norm()).item() < 3e-3
+
+
 @pytest.mark.parametrize("device", [pytest.param("cpu"), pytest.param("cuda", marks=GPU)])
 def test_rope_table(device):
     """Angles of far positions, fp32 to the last digits."""
