@@ -286,7 +286,7 @@ class ProjectionLayer(nn.Module):
         self.tp = tp_size
         self.quant = {}
         # bf16 weights ALSO held in the shuffled decode layout (name -> Bf16Weight), next to the row-major parameters:
-        # decode steps of SH_MIN_ROWS..16 token rows stream these, everything else uses the parameters
+        # decode-sized batches stream these, everything else uses the parameters
         self.sh = {}
         # split (aliased) projections: name -> list of weights / biases applied side by side (hybrid engine shares
         # the training module's separate q/k/v and gate/up tensors instead of fusing copies)
@@ -303,12 +303,14 @@ class ProjectionLayer(nn.Module):
             getattr(self, name).data = torch.empty(0, dtype=getattr(self, name).dtype,
                                                    device=getattr(self, name).device)
 
-    SH_MIN_ROWS = 2  # measured on Llama-2-7B: the row-major stream wins at 1 token row, the shuffled one from 2 up
+    # token rows from which the shuffled copies serve a decode step: the four products of a 4096-wide, 14336-deep Llama layer
+    # take 81 us at one row, the row-major streams 86
+    SH_MIN_ROWS = 1
 
     def add_decode_layout(self):
         """Keep a second copy of the four projection weights in MFMA operand order (`ops/bf16_gemv.py`): twice the
-        weight memory — 288 GB of HBM is sized for it — for up to 1.2x on batched decode steps (2 - 16 token rows). No-op
-        for quantised, split or non-bf16 weights."""
+        weight memory — 288 GB of HBM is sized for it — for decode-sized batches. No-op for quantised, split or non-bf16
+        weights."""
         from ...ops.bf16_gemv import Bf16Weight
         if self.quant or self.split_w or self.spec.num_experts:
             return False
@@ -564,24 +566,42 @@ class DSInferenceLayer(ProjectionLayer):
         return down, res2
 
     # ------------------------------------------------------------------------------ weight-only decode fast path
-    def _streams(self, h):
-        """{projection name: weight-stream object} serving this input through the un-finalized decode GEMVs, or None:
-        the quantised / shuffled-only weights, or the extra shuffled copies for SH_MIN_ROWS..16 token rows."""
+    def _decode_weights(self, h):
+        """{projection name: `Bf16Weight`} when this input's layer runs as products over the shuffled bf16 weights (the extra
+        copies, or the only ones), else None."""
         spec = self.spec
         if (not self.quant and not self.sh) or self.split_w or spec.norm != "rms" or spec.parallel_residual \
-                or spec.num_experts or self.tp != 1:
+                or spec.num_experts or self.tp != 1 or not torch.is_tensor(h):
             return None
+        from ...ops.bf16_gemv import Bf16Weight, decode_rows_ok
+        ws = self.sh or {n: w.i8 for n, w in self.quant.items()}
+        return ws if decode_rows_ok(h) and all(isinstance(ws.get(n), Bf16Weight) for n in self.projection_names()) else None
+
+    def _forward_decode(self, h, residual, meta, cache, rope, alibi, ws):
+        """Four products, each with what stands around it: the norms are part of the products that read them, residuals,
+        biases and the activation of those that make them (`csrc/gemv/skinny_bf16_sh.hip`)."""
+        from ...ops.transformer.functional import ACT_CODES
+        spec = self.spec
+        x = h if residual is None else h + residual
+        qkv = ws["qkv_w"].raw(x, self.qkv_b).finish(norm=(self.ln1_w, spec.norm_eps))
+        x = ws["o_w"].raw(self._attend(qkv, meta, cache, rope, alibi), self.o_b).finish(residual=x)
+        mid = ws["fc1_w"].raw(x, self.fc1_b).finish(norm=(self.ln2_w, spec.norm_eps), act=ACT_CODES[spec.act],
+                                                    gated=spec.gated_mlp)
+        return ws["fc2_w"].raw(mid, self.fc2_b).finish(residual=x), None
+
+    def _streams(self, h):
+        """{projection name: weight-stream object} serving this input through the un-finalized int8 / int4 decode GEMVs, or
+        None."""
+        spec = self.spec
+        if not self.quant or self.split_w or spec.norm != "rms" or spec.parallel_residual or spec.num_experts \
+                or self.tp != 1:
+            return None
+        from ...ops.bf16_gemv import Bf16Weight
         from ...ops.int8_gemv import PendingAcc, raw_ok
-        names = ("qkv_w", "o_w", "fc1_w", "fc2_w")
-        if self.quant:
-            if not all(self.quant.get(n) is not None and self.quant[n].i8 is not None for n in names):
-                return None
-            q = {n: self.quant[n].i8 for n in names}
-            return q if isinstance(h, PendingAcc) or raw_ok(h) else None
-        if isinstance(h, PendingAcc):
-            return self.sh
-        rows = h.numel() // h.shape[-1]
-        return self.sh if raw_ok(h) and rows >= self.SH_MIN_ROWS else None
+        q = {n: self.quant[n].i8 if n in self.quant else None for n in self.projection_names()}
+        if any(w is None or isinstance(w, Bf16Weight) for w in q.values()):
+            return None
+        return q if isinstance(h, PendingAcc) or raw_ok(h) else None
 
     def _quant_skinny_ok(self, h):
         return self._streams(h) is not None
@@ -616,6 +636,9 @@ class DSInferenceLayer(ProjectionLayer):
         if self._quant_skinny_ok(h):
             return self._forward_quant_skinny(h, residual, meta, cache, rope, alibi)
         h = materialize(h)
+        ws = self._decode_weights(h)
+        if ws is not None:
+            return self._forward_decode(h, residual, meta, cache, rope, alibi, ws)
         if self._skinny_ok(h):
             return self._forward_skinny(h, residual, meta, cache, rope, alibi)
         if self.spec.parallel_residual:
@@ -888,6 +911,22 @@ class DSInferenceModel(nn.Module):
     def _logits(self, h):
         return self._gather_vocab(F.linear(h, self.lm_head, self.lm_head_b))
 
+    def _decode_logits(self, h, residual):
+        """Logits of decode-sized rows with the residual and the final RMSNorm part of the LM head's product, or None."""
+        spec = self.spec
+        if not (h.is_cuda and h.dtype == torch.bfloat16 and spec.final_norm and spec.norm == "rms"):
+            return None
+        from ...ops.bf16_gemv import decode_rows_ok
+        sh = getattr(self, "lm_head_sh", None)
+        if sh is not None and decode_rows_ok(h):
+            x = h if residual is None else h + residual
+            return self._gather_vocab(sh.raw(x, self.lm_head_b).finish(norm=(self.norm_w, spec.norm_eps)))
+        if not _skinny_rows_ok(h.shape[0], spec.hidden_size):
+            return None
+        from ...ops.native import hip_ops
+        return self._gather_vocab(hip_ops().skinny_gemm(h, self.lm_head, self.lm_head_b, None, 1, False, 0, residual, self.norm_w,
+                                                        spec.norm_eps, None))
+
     def _gather_vocab(self, logits):
         if self.tp_size > 1:
             parts = [torch.empty_like(logits) for _ in range(self.tp_size)]
@@ -903,24 +942,13 @@ class DSInferenceModel(nn.Module):
         rope = (self.rope_cos, self.rope_sin)
         for layer in self.layers:
             h, residual = layer(h, residual, meta, self.cache, rope, self.alibi)
-        sh = getattr(self, "lm_head_sh", None)
-        if sh is not None and not all_logits and hasattr(h, "finalize_rms") and len(h.lead) == 2 and h.lead[1] == 1 \
-                and self.spec.final_norm and self.spec.norm == "rms":
-            # decode step over the shuffled copies: the last block's sums go through the fused residual + final
-            # RMSNorm finalize, then the LM head streams in operand order like every other projection
-            normed, _ = h.finalize_rms(residual, self.norm_w, self.spec.norm_eps)
-            return self._gather_vocab(sh.linear(normed[:, -1], self.lm_head_b))
         h = materialize(h)
         if not all_logits:
             h = h[:, -1].contiguous()
             residual = residual[:, -1].contiguous() if residual is not None else None
-            if (h.is_cuda and h.dtype == torch.bfloat16 and self.spec.final_norm and self.spec.norm == "rms"
-                    and _skinny_rows_ok(h.shape[0], self.spec.hidden_size)):
-                # final RMSNorm (+ residual) fused into the LM-head GEMV
-                from ...ops.native import hip_ops
-                logits = hip_ops().skinny_gemm(h, self.lm_head, self.lm_head_b, None, 1, False, 0, residual,
-                                               self.norm_w, self.spec.norm_eps, None)
-                return self._gather_vocab(logits)
+            logits = self._decode_logits(h, residual)
+            if logits is not None:
+                return logits
         x = h if residual is None else h + residual
         if self.spec.final_norm:
             if self.spec.norm == "rms":
@@ -944,12 +972,9 @@ class DSInferenceModel(nn.Module):
             return h.new_empty((0, self.spec.vocab_size))
         h = h[0].index_select(0, meta.last_idx)
         residual = residual[0].index_select(0, meta.last_idx) if residual is not None else None
-        if (h.is_cuda and h.dtype == torch.bfloat16 and self.spec.final_norm and self.spec.norm == "rms"
-                and _skinny_rows_ok(h.shape[0], self.spec.hidden_size)):
-            from ...ops.native import hip_ops
-            logits = hip_ops().skinny_gemm(h, self.lm_head, self.lm_head_b, None, 1, False, 0, residual, self.norm_w,
-                                           self.spec.norm_eps, None)
-            return self._gather_vocab(logits)
+        logits = self._decode_logits(h, residual)
+        if logits is not None:
+            return logits
         x = h if residual is None else h + residual
         if self.spec.final_norm:
             if self.spec.norm == "rms":

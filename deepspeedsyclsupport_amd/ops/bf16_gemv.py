@@ -9,15 +9,27 @@ streams (`ops/int8_gemv.py`) — the matrix is re-laid ONCE:
 
     wsh[nb, kq, h, lane, :] = w[16 nb + (lane % 16), 64 kq + 16 (lane // 16) + 8 h : +8]      (2 KB per 16 x 64 tile)
 
-and every 16-byte-per-lane load reads 1 KB contiguous. With more than 16 token rows (prefill) the library GEMM runs
-on a row-major matrix: the copy kept next to the shuffled one when `keep_row_major` (twice the weight memory, sized
-for 288 GB of HBM), else a temporary un-shuffled right before the GEMM.
+and every 16-byte-per-lane load reads 1 KB contiguous. A product owns all of K, so the norm of its input, bias, residual and
+activation are part of it (`DecodeProduct.finish`): one launch each. With more than `MAX_DECODE_ROWS` token rows (prefill) the
+library GEMM runs on a row-major matrix: the copy kept next to the shuffled one when `keep_row_major` (twice the weight
+memory, sized for 288 GB of HBM), else a temporary un-shuffled right before the GEMM.
 """
 import torch
 import torch.nn.functional as F
 
-from .int8_gemv import MAX_DECODE_ROWS, PendingAcc, raw_ok  # noqa: F401
+from . import reference
 from .native import hip_ops
+
+# Rows up to which a decoder layer's products take the stream. Every workgroup reads all of x, so the library's blocking wins
+# from there on: layer of a 4096-wide, 14336-deep Llama, 40 rows 125 us against 143 + 17 for its norms and activation, 64 rows
+# 163 against 131 + 17.
+MAX_DECODE_ROWS = 48
+
+
+def decode_rows_ok(x, bias=None):
+    """Whether x [.., K] is a decode-sized bf16 batch on the GPU."""
+    return x.is_cuda and x.dtype == torch.bfloat16 and 0 < x.numel() // x.shape[-1] <= MAX_DECODE_ROWS and \
+        (bias is None or bias.dtype == torch.bfloat16)
 
 
 def preshuffle16(w):
@@ -64,15 +76,45 @@ class Bf16Weight:
         return w if dtype in (None, w.dtype) else w.to(dtype)
 
     def raw(self, x, bias=None):
-        """Decode GEMV without its finalize pass (see `PendingAcc`); `raw_ok(x, bias)` must hold."""
-        K = x.shape[-1]
-        acc = hip_ops().skinny_b16_raw(x.reshape(-1, K).contiguous(), self.wsh, self.shape[0])
-        return PendingAcc(acc, x.shape[:-1], self.shape[0], bias)
+        """x . w^T + bias, launched by `DecodeProduct.finish`; `decode_rows_ok(x, bias)` must hold."""
+        return DecodeProduct(self, x, bias)
 
     def linear(self, x, bias=None):
-        K = x.shape[-1]
-        M = x.numel() // K
-        if raw_ok(x, bias):
-            return hip_ops().skinny_b16_sh(x.reshape(M, K).contiguous(), self.wsh, bias, self.shape[0]).view(
-                *x.shape[:-1], self.shape[0])
+        if decode_rows_ok(x, bias):
+            return self.raw(x, bias).finish()
         return F.linear(x, self.materialize(x.dtype), bias)
+
+
+class DecodeProduct:
+    """A decode-sized product that waits for what is fused into it."""
+
+    def __init__(self, weight, x, bias=None):
+        self.weight, self.x, self.bias = weight, x, bias
+
+    def finish(self, norm=None, residual=None, act=None, gated=False):
+        """act(rms_norm(x) . w^T + bias) + residual in one launch: `norm` (weight, eps) of the input, `act` an activation code,
+        `gated`: w is [gate | up] (N % 32 == 0) and the result act(gate) up."""
+        x, N = self.x, self.weight.shape[0]
+        norm_w, eps = norm or (None, 0.0)
+        cols = N // 2 if gated else N
+        r = None if residual is None else residual.reshape(-1, cols).contiguous()
+        y = hip_ops().decode_gemm(x.reshape(-1, x.shape[-1]).contiguous(), self.weight.wsh, N, self.bias, norm_w, eps, r, gated,
+                                  -1 if act is None else act)
+        return y.view(*x.shape[:-1], cols)
+
+    def finalize(self):
+        return self.finish()
+
+    def finalize_rms(self, residual, weight, eps):
+        """-> (RMSNorm(product + residual) * weight, product + residual)"""
+        from .transformer.functional import rms_norm
+        y = self.finish(residual=residual)
+        return rms_norm(y, weight, eps), y
+
+    def finalize_gated(self, act_code):
+        """-> act(gate) * up of a fused [gate | up] projection"""
+        if self.weight.shape[0] % 32 == 0:
+            return self.finish(act=act_code, gated=True)
+        bias = None if self.bias is None else self.bias.float()  # halves that are no whole blocks: unfused, in fp32 as well
+        gate, up = F.linear(self.x.float(), self.weight.materialize(torch.float32), bias).chunk(2, -1)
+        return (reference.ACTS[act_code](gate) * up).to(self.x.dtype)

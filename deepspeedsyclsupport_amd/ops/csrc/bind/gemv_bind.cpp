@@ -1,19 +1,15 @@
-// Module of the bf16 decode products (up to 16 token rows) of the hybrid decoders, with activation epilogues.
+// Module of the bf16 decode products (up to 64 token rows) of the hybrid decoders, with activation epilogues.
 #include "bind_util.h"
-
-#include <map>
-#include <utility>
 
 extern "C" {
 int ds_skinny_gemm(const void*, const void*, const void*, const void*, const void*, const void*, void*, void*, int, int,
                    int, int, int, int, float, hipStream_t);
-int ds_skinny_b16_mfma_ok(int, int);
-int ds_skinny_b16_mfma(const void*, const void*, const void*, void*, float*, int, int, int, hipStream_t);
-int ds_skinny_finalize_gated(float*, const void*, void*, int, int, int, int, float, hipStream_t);
+int ds_decode_gemm_ok(int, int);
+int ds_decode_gemm(const void*, const void*, const void*, const void*, float, const void*, void*, int, int, int, int, int, float,
+                   hipStream_t);
 int ds_skinny_mfma_ok(int, int, int);
 int ds_skinny_mfma(const void*, const void*, const void*, const void*, const void*, const void*, void*, void*, int, int,
                    int, int, int, int, float, hipStream_t);
-int ds_skinny_finalize_act(float*, void*, int, int, int, int, hipStream_t);
 }
 
 namespace {
@@ -44,33 +40,31 @@ Tensor decode_linear(Tensor x, Tensor w, std::optional<double> glu_limit, std::o
   return y;
 }
 
-// The same over a weight in the shuffled decode layout (ops/bf16_gemv.py: preshuffle16), w [N, K], K % 64 == 0
+// The same for M <= 64 over a weight in the shuffled decode layout (ops/bf16_gemv.py: preshuffle16), w [N, K], K % 64 == 0;
+// with a limit: N % 32 == 0
 Tensor decode_linear_sh(Tensor x, Tensor wsh, int64_t N, std::optional<double> glu_limit, std::optional<int64_t> act) {
   need(x, "x"); need(wsh, "wsh");
   const int64_t K = x.size(-1), M = x.numel() / K, NB = (N + 15) / 16;
   const bool glu = glu_limit.has_value();
   TORCH_CHECK(x.scalar_type() == at::kBFloat16 && wsh.scalar_type() == at::kBFloat16 && wsh.numel() == NB * 16 * K &&
-              ds_skinny_b16_mfma_ok((int)M, (int)K), "decode_linear_sh: up to 16 bf16 rows, K % 64 == 0");
+              ds_decode_gemm_ok((int)M, (int)K), "decode_linear_sh: up to 64 bf16 rows, K % 64 == 0");
   TORCH_CHECK(NB * K < ((int64_t)1 << 40) && N < ((int64_t)1 << 31) / 16, "decode_linear_sh: matrix too large");
   TORCH_CHECK(!(glu && act.has_value()), "decode_linear_sh: one epilogue");
-  TORCH_CHECK(!glu || N % 2 == 0, "decode_linear_sh: [gate | up] rows");
-  // fp32 split-K sums, zero between calls (the kernels leave it so); one per device and stream, grown on demand
-  static std::map<std::pair<int, hipStream_t>, Tensor> workspaces;
-  Tensor& ws = workspaces[{x.get_device(), stream()}];
-  const int64_t NP = (NB + 3) / 4 * 64;  // row length of the sums
-  if (!ws.defined() || ws.numel() < 16 * NP) ws = torch::zeros({16 * NP}, x.options().dtype(at::kFloat));
+  TORCH_CHECK(!glu || N % 32 == 0, "decode_linear_sh: [gate | up] of whole blocks of 16 rows");
   auto sizes = x.sizes().vec();
   sizes.back() = glu ? N / 2 : N;
   auto y = torch::empty(sizes, x.options());
-  check(ds_skinny_b16_mfma(x.data_ptr(), wsh.data_ptr(), nullptr, glu || act.has_value() ? nullptr : y.data_ptr(),
-                           ws.data_ptr<float>(), (int)M, (int)N, (int)K, stream()), "decode_linear_sh");
-  if (act.has_value())
-    check(ds_skinny_finalize_act(ws.data_ptr<float>(), y.data_ptr(), (int)M, (int)N, (int)NP, (int)*act, stream()),
-          "decode_linear_sh (activation)");
-  if (glu)
-    check(ds_skinny_finalize_gated(ws.data_ptr<float>(), nullptr, y.data_ptr(), (int)M, (int)N, (int)NP, CLAMPED_GLU,
-                                   (float)*glu_limit, stream()), "decode_linear_sh (gated)");
+  const int code = glu ? CLAMPED_GLU : act.has_value() ? UNARY + (int)*act : -1;
+  check(ds_decode_gemm(x.data_ptr(), wsh.data_ptr(), nullptr, nullptr, 0.f, nullptr, y.data_ptr(), (int)M, (int)N, (int)K, glu, code,
+                       glu ? (float)*glu_limit : 0.f, stream()), "decode_linear_sh");
   return y;
+}
+// Whether decode_linear_sh takes a product and is the faster one. Every workgroup reads all of x: over deep contractions the
+// library's blocking wins from 17 rows on ([4096, 14336], us: 24 rows 30 here, 29 there; 40 rows 41 and 33), over short ones
+// the stream up to its 48 ([2048, 5632], 40 rows: 18 and 20; [4096, 4096] 15 and 20).
+bool decode_linear_sh_ok(int64_t M, int64_t N, int64_t K, bool glu) {
+  return M <= 48 && K < ((int64_t)1 << 31) && ds_decode_gemm_ok((int)M, (int)K) && (M <= 16 || K <= 8192) &&
+         (!glu || N % 32 == 0);
 }
 }  // namespace
 
@@ -78,6 +72,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_linear", &decode_linear, py::arg("x"), py::arg("w"), py::arg("glu_limit") = py::none(),
         py::arg("act") = py::none());
   m.def("decode_linear_ok", &decode_linear_ok);
+  m.def("decode_linear_sh_ok", &decode_linear_sh_ok);
   m.def("decode_linear_sh", &decode_linear_sh, py::arg("x"), py::arg("wsh"), py::arg("N"),
         py::arg("glu_limit") = py::none(), py::arg("act") = py::none());
 }

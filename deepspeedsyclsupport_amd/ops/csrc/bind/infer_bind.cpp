@@ -32,8 +32,9 @@ int ds_skinny_i8_mfma(const void*, const int8_t*, const float*, const void*, voi
                       hipStream_t);
 int64_t ds_skinny_i8_mfma_ws_floats(int);
 void ds_skinny_i8_tune(int, int, int);
-int ds_skinny_b16_mfma_ok(int, int);
-int ds_skinny_b16_mfma(const void*, const void*, const void*, void*, float*, int, int, int, hipStream_t);
+int ds_decode_gemm_ok(int, int);
+int ds_decode_gemm(const void*, const void*, const void*, const void*, float, const void*, void*, int, int, int, int, int, float,
+                   hipStream_t);
 int ds_unshuffle_sh16(const void*, void*, int, int, hipStream_t);
 void ds_skinny_b16_tune(int, int);
 int ds_dequant_sh(const int8_t*, const float*, void*, int, int, int, hipStream_t);
@@ -45,7 +46,7 @@ int64_t ds_skinny_i4_mfma_ws_floats(int);
 void ds_skinny_i4_tune(int, int, int);
 int ds_dequant_sh4(const int8_t*, const float*, void*, int, int, int, hipStream_t);
 int ds_skinny_finalize_rms(float*, const void*, const void*, const void*, void*, void*, int, int, int, float, hipStream_t);
-int ds_skinny_finalize_gated(float*, const void*, void*, int, int, int, int, float, hipStream_t);
+int ds_skinny_finalize_gated(float*, const void*, void*, int, int, int, int, hipStream_t);
 int ds_skinny_finalize_plain(float*, const void*, void*, int, int, int, hipStream_t);
 int ds_quantize(const void*, int8_t*, float*, float*, int64_t, int, int, int, int, unsigned, int, hipStream_t);
 int ds_dequantize(const int8_t*, const float*, const float*, void*, int64_t, int, int, int, int, hipStream_t);
@@ -405,40 +406,39 @@ Tensor skinny_q_raw(Tensor x, Tensor wq, Tensor ws_s, int64_t N, int64_t gs, int
   return ws.acc.narrow(0, 0, 16 * NP).view({16, NP});
 }
 
-// bf16 MFMA stream over the pre-shuffled weight (ops/bf16_gemv.py: preshuffle16): x [M, K] bf16 (M <= 16),
-// wsh bf16 [ceil(N/16), K/64, 2, 64, 8] -> y [M, N] bf16; `raw`: the un-finalized fp32 workspace view [16, NP] instead
-// (same contract as skinny_q_raw).
-Tensor skinny_b16_impl(Tensor x, Tensor wsh, OptT bias, int64_t N, bool raw) {
+const void* opt_bf16(const OptT& t, int64_t numel, const char* what) {
+  if (!t.has_value() || !t->defined()) return nullptr;
+  need(*t, what);
+  TORCH_CHECK(t->scalar_type() == at::kBFloat16 && t->numel() == numel, what, ": bf16 with ", numel, " elements");
+  return t->data_ptr();
+}
+
+// bf16 product over the pre-shuffled weight (ops/bf16_gemv.py: preshuffle16): x [M, K] bf16 (M <= 64), wsh bf16 [ceil(N/16), K/64,
+// 2, 64, 8] -> y [M, N] bf16. norm_w [K]: x is RMS-normed first. bias [N]; res [M, N] is added at the end. gated: w is a
+// fused [gate | up] weight, the result act(gate) up [M, N / 2] (limit: of the clamped activation); else act: an activation
+// code of the result, or -1.
+Tensor decode_gemm(Tensor x, Tensor wsh, int64_t N, OptT bias, OptT norm_w, double eps, OptT res, bool gated, int64_t act,
+                   double limit) {
   need(x, "x"); need(wsh, "wsh");
   TORCH_CHECK(x.scalar_type() == at::kBFloat16 && x.dim() == 2 && wsh.scalar_type() == at::kBFloat16,
-              "skinny_b16: bf16 x [M, K] and bf16 shuffled weight");
+              "decode_gemm: bf16 x [M, K] and bf16 shuffled weight");
   const int64_t M = x.size(0), K = x.size(1), NB = (N + 15) / 16;
-  TORCH_CHECK(ds_skinny_b16_mfma_ok((int)M, (int)K) != 0, "skinny_b16: unsupported shape (M ", M, ", K ", K, ")");
-  TORCH_CHECK(wsh.numel() == NB * 16 * K && wsh.is_contiguous(), "skinny_b16: shuffled weight size");
-  TORCH_CHECK(NB * K < ((int64_t)1 << 40) && N < ((int64_t)1 << 31) / 16, "skinny_b16: matrix too large");
-  TORCH_CHECK(reinterpret_cast<uintptr_t>(wsh.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
-              "skinny_b16: 16-B aligned x / weight");
-  const void* bp = nullptr;
-  if (!raw && bias.has_value() && bias->defined()) {
-    need(*bias, "bias");
-    TORCH_CHECK(bias->numel() == N && bias->scalar_type() == at::kBFloat16, "skinny_b16: bias bf16 [N]");
-    bp = bias->data_ptr();
-  }
-  auto& ws = i8_workspace(x, N);
-  if (raw) {
-    check(ds_skinny_b16_mfma(x.data_ptr(), wsh.data_ptr(), nullptr, nullptr, ws.acc.data_ptr<float>(), (int)M, (int)N,
-                             (int)K, stream()), "skinny_b16 (raw)");
-    const int64_t NP = ds_skinny_i8_mfma_ws_floats((int)N) / 16;
-    return ws.acc.narrow(0, 0, 16 * NP).view({16, NP});
-  }
-  auto y = torch::empty({M, N}, x.options());
-  check(ds_skinny_b16_mfma(x.data_ptr(), wsh.data_ptr(), bp, y.data_ptr(), ws.acc.data_ptr<float>(), (int)M, (int)N,
-                           (int)K, stream()), "skinny_b16");
+  TORCH_CHECK(ds_decode_gemm_ok((int)M, (int)K) != 0, "decode_gemm: unsupported shape (M ", M, ", K ", K, ")");
+  TORCH_CHECK(wsh.numel() == NB * 16 * K, "decode_gemm: shuffled weight size");
+  TORCH_CHECK(NB * K < ((int64_t)1 << 40) && N < ((int64_t)1 << 31) / 16, "decode_gemm: matrix too large");
+  TORCH_CHECK(!gated || N % 32 == 0, "decode_gemm: [gate | up] of whole blocks of 16 rows");
+  const int64_t cols = gated ? N / 2 : N;
+  const void* bp = opt_bf16(bias, N, "bias");
+  const void* np = opt_bf16(norm_w, K, "norm weight");
+  const void* rp = opt_bf16(res, M * cols, "residual");
+  for (const void* p : {(const void*)wsh.data_ptr(), (const void*)x.data_ptr(), np})
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(p) % 16 == 0, "decode_gemm: 16-B aligned x / weights");
+  auto y = torch::empty({M, cols}, x.options());
+  check(ds_decode_gemm(x.data_ptr(), wsh.data_ptr(), bp, np, (float)eps, rp, y.data_ptr(), (int)M, (int)N, (int)K, gated,
+                       gated || act < 0 ? (int)act : (int)act + 16, (float)limit, stream()), "decode_gemm");
   return y;
 }
-Tensor skinny_b16_sh(Tensor x, Tensor wsh, OptT bias, int64_t N) { return skinny_b16_impl(x, wsh, bias, N, false); }
-Tensor skinny_b16_raw(Tensor x, Tensor wsh, int64_t N) { return skinny_b16_impl(x, wsh, c10::nullopt, N, true); }
-bool skinny_b16_ok(int64_t M, int64_t K) { return ds_skinny_b16_mfma_ok((int)M, (int)K) != 0; }
+bool decode_gemm_ok(int64_t M, int64_t K) { return ds_decode_gemm_ok((int)M, (int)K) != 0; }
 
 // pre-shuffled bf16 -> row-major bf16 [N, K]
 Tensor unshuffle_sh16(Tensor wsh, int64_t N) {
@@ -451,12 +451,6 @@ Tensor unshuffle_sh16(Tensor wsh, int64_t N) {
   return w;
 }
 
-const void* opt_bf16(const OptT& t, int64_t numel, const char* what) {
-  if (!t.has_value() || !t->defined()) return nullptr;
-  need(*t, what);
-  TORCH_CHECK(t->scalar_type() == at::kBFloat16 && t->numel() == numel, what, ": bf16 with ", numel, " elements");
-  return t->data_ptr();
-}
 void check_acc(const Tensor& acc, int64_t M, int64_t N) {
   TORCH_CHECK(acc.is_cuda() && acc.scalar_type() == at::kFloat && acc.dim() == 2 && acc.size(0) == 16 &&
                   acc.is_contiguous() && acc.size(1) >= N && M >= 1 && M <= 16, "skinny_finalize: fp32 workspace view [16, NP]");
@@ -482,7 +476,7 @@ Tensor skinny_finalize_gated(Tensor acc, int64_t M, int64_t N, OptT bias, int64_
   const void* bp = opt_bf16(bias, N, "bias");
   auto out = torch::empty({M, N / 2}, acc.options().dtype(at::kBFloat16));
   check(ds_skinny_finalize_gated(acc.data_ptr<float>(), bp, out.data_ptr(), (int)M, (int)N, (int)acc.size(1), (int)act,
-                                 0.f, stream()), "skinny_finalize_gated");
+                                 stream()), "skinny_finalize_gated");
   return out;
 }
 
@@ -560,9 +554,10 @@ void register_inference_ops(pybind11::module& m) {
         py::arg("p"), py::arg("wpc"), py::arg("rounds") = 0);
   m.def("dequant_sh4", &dequant_sh4);
   m.def("skinny_q_raw", &skinny_q_raw);
-  m.def("skinny_b16_ok", &skinny_b16_ok);
-  m.def("skinny_b16_sh", &skinny_b16_sh, py::arg("x"), py::arg("wsh"), py::arg("bias"), py::arg("N"));
-  m.def("skinny_b16_raw", &skinny_b16_raw);
+  m.def("decode_gemm_ok", &decode_gemm_ok);
+  m.def("decode_gemm", &decode_gemm, py::arg("x"), py::arg("wsh"), py::arg("N"), py::arg("bias") = py::none(),
+        py::arg("norm_w") = py::none(), py::arg("eps") = 0.0, py::arg("res") = py::none(), py::arg("gated") = false,
+        py::arg("act") = -1, py::arg("limit") = 0.0);
   m.def("unshuffle_sh16", &unshuffle_sh16);
   m.def("skinny_b16_tune", [](int64_t cfg, int64_t wpc) { ds_skinny_b16_tune((int)cfg, (int)wpc); }, py::arg("cfg"),
         py::arg("wpc") = 0);

@@ -1,143 +1,244 @@
-// bf16 skinny GEMM for decode over a PRE-SHUFFLED weight: y[M, N] = X[M, K] . W[N, K]^T (+ bias), M <= 16.
+// bf16 products of decode-sized batches over a PRE-SHUFFLED weight: y[M, N] = X[M, K] . W[N, K]^T, M <= 48, with what stands
+// around them in a decoder layer: the RMS norm of X, bias, residual, gated or plain activation.
 //
 // Reference counterpart (behaviour): the bf16 / fp16 decode GEMMs of `transformer_inference` (`qkv_gemm`,
 // `vector_matmul`, `mlp_gemm`; `csrc/transformer/inference/csrc/pt_binding.cpp`), which call the vendor GEMM on the
 // row-major weight.
 //
-// MI355X design: a decode GEMM is a weight stream and the HBM stream only runs at full rate when every load
-// instruction covers long contiguous segments. Read from a row-major matrix, the MFMA operand layout is 16 rows x
-// 64 B per instruction, which measured 4.4 - 5.0 TB/s loads-only (`profiles/int8_load_patterns_r2.jsonl`), and the
-// row-major bf16 kernels of this directory run at 3 - 4.2 TB/s end to end. Inference weights are constants, so —
-// exactly like the int8 / int4 streams — the matrix is re-laid ONCE into operand order:
+// A decode GEMM is a weight stream, and the HBM stream only runs at full rate when every load instruction covers
+// long contiguous segments. Inference weights are constants, so the matrix is re-laid ONCE into operand order:
 //   Wsh[nb][kq][h][lane][8] = W[16 nb + (lane & 15)][64 kq + 16 (lane >> 4) + 8 h + 0..7]    (2 KB per 16 x 64 tile)
-// so each 16-byte-per-lane load reads 1 KB contiguous and IS the B operand of one v_mfma_f32_16x16x32_bf16 (X is
-// loaded with the same k permutation). The kernel is the int8 stream (skinny_int8.hip) minus the dequantisation:
-// a wave owns FB row blocks and walks a contiguous range of the (block group, k quarter) sequence with P quarters
-// in flight in registers; ranges may start / end inside a block group (split-K without a fixed factor); partial
-// sums go to the fp32 workspace shared with the int8 / int4 streams by f32 atomics, and the same finalize kernels
-// (skinny_finalize.hip: plain, + residual + RMSNorm, gated activation) convert and re-zero it.
-// Prefill (more than 16 token rows) un-shuffles into a row-major temporary for the library GEMM (`ds_unshuffle_sh16`),
+// so each 16-byte-per-lane load reads 1 KB contiguous and IS the A operand of one v_mfma_f32_16x16x32_bf16 (X is
+// loaded with the same k permutation).
+//  * a workgroup owns RB blocks of 16 weight rows over all of K and up to 48 token rows: its eight waves take alternating steps
+//    of 64 columns, straight into registers, and their sums meet in LDS once. No split over workgroups, so no fp32 sums in
+//    memory, no atomics and no second kernel: sums stay in one fixed order and the result leaves as bf16;
+//  * the norm costs no pass: y = rs (X w) . W^T with rs the row's 1 / rms, and every workgroup sees all of X anyway. It
+//    multiplies X by the norm's weight on the way to the matrix cores, adds up the squares beside, and scales the sums;
+//  * a gated pair (gate block i, up block i + N / 32) sits in one workgroup: act(gate) up leaves, half of N;
+//  * X is read once per workgroup (from L2), which is what bounds wide batches; RB trades that against workgroups enough.
+// Bound by the weights' read (6.5 TB/s here). Measured, us (the same products as split streams with fp32 atomics and a finalize
+// pass; the floor): 12 rows x [4096, 4096] 9 (14; 5), [4096, 14336] 23 (25; 18), gated [28672, 4096] 38 (45; 36), with the
+// norm 39, [32000, 4096] 42 (51; 40), [2048, 2048] 5.6 (7.6; 1.3). 24 and 40 rows (library GEMM): gated [28672, 4096] with the
+// norm 42 and 50 (52 and 52 without the norm and activation), [4096, 4096] 11 and 15 (20 and 20).
+// Prefill (more rows) un-shuffles into a row-major temporary for the library GEMM (`ds_unshuffle_sh16`),
 // or uses the row-major copy the caller kept.
 #include "ds_hip.h"
-
-#include <algorithm>
-
-extern "C" int ds_skinny_finalize_plain(float* ws, const void* bias, void* y, int M, int N, int NP, hipStream_t st);
 
 namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+constexpr int WAVES = 8;
 
-struct B16Args {
-  const bf16* x;
-  const bf16* w;  // shuffled
-  float* acc;     // [16, NP] fp32 workspace, zero between calls
-  int M, N, K, NB, KQ, NBG;
-  int NP;         // workspace row length: NBG * FB * 16
-  int64_t total;  // NBG * KQ
+struct ShArgs {
+  const bf16* x;       // [M, K]
+  const bf16* w;       // shuffled
+  const bf16* bias;    // [N] or null
+  const bf16* norm_w;  // [K] (NORM)
+  const bf16* res;     // [M, N] or null: added at the end
+  bf16* y;             // [M, N], gated [M, N / 2]
+  int M, N, K;
+  float eps;
+  int act;             // gated: activation code; else code + DS_ACT_UNARY, or -1
+  float limit;         // of the clamped gated activation
 };
 
-template <int FB>
-struct B16Stage {
-  bf16x8_t w0[FB], w1[FB];
-  bf16x8_t x0, x1;
-};
-
-template <int FB, int P>
-__global__ void __launch_bounds__(256) skinny_b16_mfma_kernel(B16Args a) {
-  const int lane = threadIdx.x & 63;
-  // wave-uniform bookkeeping lives in SGPRs (readfirstlane): scalar branches keep the vmcnt counts static
-  const int gw = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)), nw = gridDim.x * 4;
-  const int lo = (int)(a.total * gw / nw), hi = (int)(a.total * (gw + 1) / nw);
-  if (lo >= hi) return;
-  const int r = lane & 15, g = lane >> 4;
-
-  // issue cursor: wave-uniform offsets advanced per quarter; block offsets recomputed only when entering a group
-  int ibg = 0, ikq = 0;
-  bool hold = false;
-  int64_t iw = 0, ix = 0, fw[FB];
-  const int64_t xlane = (int64_t)min(r, a.M - 1) * a.K + 16 * g;  // token rows >= M re-read row M - 1
-  auto enter = [&](int bgv, int kqv) {
-    if (bgv >= a.NBG) {  // past the end of the range: keep re-loading the last quarter (static vmcnt)
-      bgv = a.NBG - 1;
-      kqv = a.KQ - 1;
-      hold = true;
-    }
-    ibg = bgv;
-    ikq = kqv;
-#pragma unroll
-    for (int f = 0; f < FB; ++f) fw[f] = (int64_t)min(bgv * FB + f, a.NB - 1) * a.KQ * 1024;  // (elements)
-    iw = (int64_t)kqv * 1024;
-    ix = (int64_t)kqv * 64;
-  };
-  auto advance = [&]() {
-    if (hold) return;
-    if (++ikq == a.KQ) {
-      enter(ibg + 1, 0);
-      return;
-    }
-    iw += 1024;
-    ix += 64;
-  };
-  auto load = [&](B16Stage<FB>& st) {
-#pragma unroll
-    for (int f = 0; f < FB; ++f) {
-      const bf16* p = a.w + fw[f] + iw + lane * 8;
-      st.w0[f] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(p));
-      st.w1[f] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(p + 512));
-    }
-    const bf16* xp = a.x + xlane + ix;
-    st.x0 = *reinterpret_cast<const bf16x8_t*>(xp);
-    st.x1 = *reinterpret_cast<const bf16x8_t*>(xp + 8);
-  };
-
-  const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
-  f32x4 acc[FB];
-#pragma unroll
-  for (int f = 0; f < FB; ++f) acc[f] = zero4;
-
-  int bg = lo / a.KQ, kq = lo - bg * a.KQ;
-  enter(bg, kq);
-  B16Stage<FB> st[P];
-#pragma unroll
-  for (int p = 0; p < P; ++p) {  // same issue order as the steady state
-    load(st[p]);
-    advance();
-    __builtin_amdgcn_sched_barrier(0);
+__device__ __forceinline__ float act_any(int a, float x) {
+  switch (a) {
+    case 0: return x / (1.f + __expf(-x));  // silu
+    case 1: return 0.5f * x * (1.f + tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x)));
+    case 2: return 0.5f * x * (1.f + erff(x * 0.7071067811865476f));
+    case 3: return fmaxf(x, 0.f);
+    default: return x;
   }
-  // partial sums of block group `grp` -> fp32 workspace (padded to whole groups; features >= N are never read)
-  auto spill = [&](int grp) {
-#pragma unroll
-    for (int f = 0; f < FB; ++f) {
-      const int n = (grp * FB + f) * 16 + r;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (4 * g + i < a.M) unsafeAtomicAdd(a.acc + (int64_t)(4 * g + i) * a.NP + n, acc[f][i]);
-      acc[f] = zero4;
-    }
+}
+
+template <int V>
+struct Int {
+  static constexpr int value = V;
+};
+
+template <int MT, int RB, bool NORM, bool GATED>
+__global__ void __launch_bounds__(WAVES * 64, (MT <= 2 ? 4 : 2)) decode_gemm_kernel(ShArgs a) {
+  static_assert(!GATED || RB % 2 == 0, "pairs");
+  constexpr int T = MT * RB, HALF = WAVES / 2;
+  constexpr int U = T == 1 ? 2 : 1;  // steps loaded together
+  __shared__ f32x4 red[HALF][T][64];
+  __shared__ float ssq[WAVES][MT][16], scale[MT * 16];
+  const int lane = threadIdx.x & 63, l16 = lane & 15, q4 = lane >> 4;
+  const int wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int K = a.K, KQ = K / 64, NB = (a.N + 15) / 16, HB = a.N / 32;
+  // block i of this workgroup
+  auto block_of = [&](int i) {
+    if (!GATED) return (int)blockIdx.x * RB + i;
+    return (int)blockIdx.x * (RB / 2) + i % (RB / 2) + (i < RB / 2 ? 0 : HB);
   };
-  // Straight-line steady state: every reload follows the compute that frees its registers; steps past the range end
-  // re-load the last quarter and skip the (wave-uniform) MFMA block.
-  for (int base = lo; base < hi; base += P) {
+  const bf16* wp[RB];
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-      const bool live = base + p < hi;
-      if (live) {
+  for (int i = 0; i < RB; ++i) {
+    const int last = GATED ? (i < RB / 2 ? HB : 2 * HB) - 1 : NB - 1;
+    wp[i] = a.w + (int64_t)min(block_of(i), last) * KQ * 1024 + lane * 8;
+  }
+  const bf16* xp[MT];
 #pragma unroll
-        for (int f = 0; f < FB; ++f) {
-          acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(st[p].x0, st[p].w0[f], acc[f], 0, 0, 0);
-          acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(st[p].x1, st[p].w1[f], acc[f], 0, 0, 0);
-        }
-        if (kq == a.KQ - 1) spill(bg);
+  for (int m = 0; m < MT; ++m) xp[m] = a.x + (int64_t)min(16 * m + l16, a.M - 1) * K + 16 * q4;
+  const bf16* np = NORM ? a.norm_w + 16 * q4 : nullptr;
+
+  f32x4 acc[RB][MT];
+  float ss[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    ss[m] = 0.f;
+#pragma unroll
+    for (int i = 0; i < RB; ++i) acc[i][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  struct Steps {
+    bf16x8_t w[U][2][RB], x[U][2][MT], norm[U][2];
+  };
+  // U steps, WAVES apart: all their loads (past the end the last step again, which counts for nothing) before the products
+  // of the steps at hand: without the barrier the compiler sinks them and a wave has a load or two in flight
+  auto load = [&](Steps& f, int s0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+          f.w[u][h][i] = __builtin_nontemporal_load(
+              reinterpret_cast<const bf16x8_t*>(wp[i] + (int64_t)min(s0 + WAVES * u, KQ - 1) * 1024 + 512 * h));
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int k = min(s0 + WAVES * u, KQ - 1) * 64 + 8 * h;
+        if constexpr (NORM) f.norm[u][h] = *reinterpret_cast<const bf16x8_t*>(np + k);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) f.x[u][h][m] = *reinterpret_cast<const bf16x8_t*>(xp[m] + k);
       }
-      if (++kq == a.KQ) { kq = 0; ++bg; }
-      __builtin_amdgcn_sched_barrier(0);
-      load(st[p]);
-      advance();
-      __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto products = [&](Steps& f, int s0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (u && s0 + WAVES * u >= KQ) break;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          if constexpr (NORM) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const float v = (float)f.x[u][h][m][j];
+              ss[m] = fmaf(v, v, ss[m]);
+              f.x[u][h][m][j] = (bf16)(v * (float)f.norm[u][h][j]);
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < RB; ++i)
+            acc[i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[u][h][i], f.x[u][h][m], acc[i][m], 0, 0, 0);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr int STRIDE = WAVES * U;
+  int s = wid;
+  if (s < KQ) {
+    Steps f0;
+    if constexpr (RB <= 2) {  // the next steps' loads run while these are multiplied
+      Steps f1;
+      load(f0, s);
+      for (;;) {
+        load(f1, s + STRIDE);
+        products(f0, s);
+        if ((s += STRIDE) >= KQ) break;
+        load(f0, s + STRIDE);
+        products(f1, s);
+        if ((s += STRIDE) >= KQ) break;
+      }
+    } else {  // four blocks a step: the workgroups beside this one cover its waits, a second set of registers costs more of them
+      for (; s < KQ; s += STRIDE) {
+        load(f0, s);
+        products(f0, s);
+      }
     }
   }
-  if ((hi % a.KQ) != 0) spill((hi - 1) / a.KQ);  // the range ends inside a group
+
+  // ---- the waves' sums meet: the upper half's through LDS, then all four halves' sums
+  if (wid >= HALF) {
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) red[wid - HALF][i * MT + m][lane] = acc[i][m];
+  }
+  if constexpr (NORM) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      float v = ss[m];
+      v += __shfl_xor(v, 16, 64);
+      v += __shfl_xor(v, 32, 64);
+      if (lane < 16) ssq[wid][m][l16] = v;
+    }
+  }
+  __syncthreads();
+  if (wid < HALF) {
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) red[wid][i * MT + m][lane] += acc[i][m];
+  }
+  if constexpr (NORM) {
+    if (threadIdx.x < MT * 16) {
+      float v = 0.f;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) v += ssq[w][threadIdx.x / 16][threadIdx.x % 16];
+      scale[threadIdx.x] = rsqrtf(v / K + a.eps);
+    }
+  }
+  __syncthreads();
+  // ---- lane: token row l16 of tile m, weight rows 4 q4 .. + 3 of a block
+  const int cols = GATED ? a.N / 2 : a.N;
+  for (int j = wid; j < (GATED ? T / 2 : T); j += WAVES) {
+    const int i = j / MT, m = j % MT, row = 16 * m + l16, n = block_of(i) * 16 + 4 * q4;
+    auto total = [&](int t) {
+      f32x4 v = red[0][t][lane];
+#pragma unroll
+      for (int w = 1; w < HALF; ++w) v += red[w][t][lane];
+      if constexpr (NORM) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] *= scale[row];
+      }
+      return v;
+    };
+    f32x4 v = total(j), u = GATED ? total(j + T / 2) : v;
+    if (row >= a.M) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int c = n + e;
+      if (c >= cols) continue;
+      float r = v[e] + (a.bias ? (float)a.bias[c] : 0.f);
+      if constexpr (GATED) {
+        const float g = r, up = u[e] + (a.bias ? (float)a.bias[cols + c] : 0.f);
+        r = a.act == DS_ACT_CLAMPED_GLU ? clamped_glu_f(g, up, a.limit) : act_any(a.act, g) * up;
+      } else if (a.act >= 0) {
+        r = act_any(a.act - DS_ACT_UNARY, r);
+      }
+      if (a.res) r += (float)a.res[(int64_t)row * cols + c];
+      v[e] = r;
+    }
+    bf16* yr = a.y + (int64_t)row * cols + n;
+    if (cols % 4 == 0) {
+      if (n < cols) {
+        bf16x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (bf16)v[e];
+        *reinterpret_cast<bf16x4*>(yr) = o;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < cols) yr[e] = (bf16)v[e];
+    }
+  }
 }
 
 // Pre-shuffled bf16 -> row-major bf16 [N, K]. One thread per 16-byte lane chunk (8 weights of one row).
@@ -155,16 +256,31 @@ __global__ void __launch_bounds__(256) unshuffle_sh16_kernel(const bf16* __restr
   *reinterpret_cast<bf16x8*>(W + row * KQ * 64 + kq * 64 + 16 * (lane >> 4) + 8 * h) = v;
 }
 
-int g_b16_cfg = 0, g_b16_wpc = 0;
+int g_blocks = 0;
+
+template <int MT, int RB>
+int launch(const ShArgs& a, bool gated, hipStream_t st) {
+  const int blocks = gated ? a.N / 16 : (a.N + 15) / 16;
+  const dim3 grid((blocks + RB - 1) / RB), threads(WAVES * 64);
+  if (gated) {
+    if constexpr (RB > 1) {
+      if (a.norm_w) hipLaunchKernelGGL((decode_gemm_kernel<MT, RB, true, true>), grid, threads, 0, st, a);
+      else hipLaunchKernelGGL((decode_gemm_kernel<MT, RB, false, true>), grid, threads, 0, st, a);
+    }
+  } else if constexpr (MT > 1 || RB < 4) {
+    if (a.norm_w) hipLaunchKernelGGL((decode_gemm_kernel<MT, RB, true, false>), grid, threads, 0, st, a);
+    else hipLaunchKernelGGL((decode_gemm_kernel<MT, RB, false, false>), grid, threads, 0, st, a);
+  }
+  DS_CHECK_LAUNCH();
+  return 0;
+}
 
 }  // namespace
 
-extern "C" void ds_skinny_b16_tune(int cfg, int wpc) {
-  g_b16_cfg = cfg;
-  g_b16_wpc = wpc;
-}
+// Forces blocks per workgroup (1, 2, 4, where the product has such a kernel; 0: by the rule below).
+extern "C" void ds_skinny_b16_tune(int cfg, int) { g_blocks = cfg; }
 
-extern "C" int ds_skinny_b16_mfma_ok(int M, int K) { return M >= 1 && M <= 16 && K % 64 == 0; }
+extern "C" int ds_decode_gemm_ok(int M, int K) { return M >= 1 && M <= 48 && K >= 64 && K % 64 == 0; }
 
 extern "C" int ds_unshuffle_sh16(const void* Wsh, void* W, int N, int K, hipStream_t st) {
   if (N <= 0 || K % 64) return (int)hipErrorInvalidValue;
@@ -176,39 +292,34 @@ extern "C" int ds_unshuffle_sh16(const void* Wsh, void* W, int N, int K, hipStre
   return 0;
 }
 
-// X [M, K] bf16 (M <= 16), Wsh in the shuffled layout above (N padded to a multiple of 16), bias bf16 [N] or null
-// -> Y [M, N] bf16 (Y == null: leave the sums in the workspace, row length ws_floats / 16, un-finalized). The
-// workspace is the int8 stream's: fp32 [16 x N padded to whole groups of 4 row blocks], zero between calls.
-extern "C" int ds_skinny_b16_mfma(const void* X, const void* Wsh, const void* bias, void* Y, float* ws, int M, int N,
-                                  int K, hipStream_t st) {
-  if (!ds_skinny_b16_mfma_ok(M, K) || N <= 0) return (int)hipErrorInvalidValue;
-  B16Args a;
-  a.x = (const bf16*)X;
-  a.w = (const bf16*)Wsh;
-  a.acc = ws;
-  a.M = M;
-  a.N = N;
-  a.K = K;
-  a.NB = (N + 15) / 16;
-  a.KQ = K / 64;
-  auto go = [&](auto kern, int P, int FB, int wpc) {
-    // one resident round of waves (wpc per CU, from the VGPR budget), each with the same number of quarters
-    const int nbg = (a.NB + FB - 1) / FB;
-    a.NBG = nbg;
-    a.NP = ((a.NB + 3) / 4) * 64;  // the shared workspace row length (whole groups of 4 row blocks)
-    a.total = (int64_t)nbg * a.KQ;
-    const int64_t waves = std::max<int64_t>(1, std::min<int64_t>(a.total / (2 * P), 256 * wpc));
-    hipLaunchKernelGGL(kern, dim3((int)((waves + 3) / 4)), dim3(256), 0, st, a);
-  };
-  int cfg = g_b16_cfg ? g_b16_cfg : 1;
-  const int wpc = g_b16_wpc;
-  switch (cfg) {
-    case 2: go(skinny_b16_mfma_kernel<4, 2>, 2, 4, wpc ? wpc : 8); break;
-    case 3: go(skinny_b16_mfma_kernel<2, 3>, 3, 2, wpc ? wpc : 12); break;
-    case 4: go(skinny_b16_mfma_kernel<4, 1>, 1, 4, wpc ? wpc : 12); break;
-    default: go(skinny_b16_mfma_kernel<2, 2>, 2, 2, wpc ? wpc : 8);
+// X [M, K] bf16 (M <= 48, K % 64 == 0), Wsh in the shuffled layout above (N padded to a multiple of 16). norm_w [K] or null: X
+// is RMS-normed by it first. bias [N], res [M, N] or null. gated: N / 2 columns act(gate) up (N % 32 == 0); else act: a
+// code + DS_ACT_UNARY, or -1.
+extern "C" int ds_decode_gemm(const void* X, const void* Wsh, const void* bias, const void* norm_w, float eps, const void* res,
+                              void* Y, int M, int N, int K, int gated, int act, float limit, hipStream_t st) {
+  if (!ds_decode_gemm_ok(M, K) || N <= 0 || (gated && N % 32)) return (int)hipErrorInvalidValue;
+  const ShArgs a{(const bf16*)X, (const bf16*)Wsh, (const bf16*)bias, (const bf16*)norm_w, (const bf16*)res, (bf16*)Y, M, N, K,
+                 eps, act, limit};
+  // Blocks of 16 weight rows per workgroup. One, until the blocks fill the chip's 256 CUs one and a half times (12 rows, us with
+  // one / two: [3072, 2048] 5.7 / 6.8, [4096, 14336] 23 / 30; [6144, 4096] 15 / 11). Then two, and with more than 16 token rows
+  // four from 1024 blocks on (24 rows x [32000, 4096] 48 with two, 46 with four; 12 rows 42 and 45). Gated pairs take four
+  // from 512 on ([11264, 2048] 13.0 with two, 11.0 with four; [28672, 4096] 41 and 38).
+  const int mt = (M + 15) / 16, blocks = gated ? N / 16 : (N + 15) / 16;
+  int rb = blocks < 384 ? 1 : 2;
+  if (gated ? blocks >= 512 : mt > 1 && blocks >= 1024) rb = 4;
+  if (g_blocks) rb = g_blocks >= 4 ? 4 : g_blocks == 3 ? 2 : g_blocks;
+  if (gated && rb < 2) rb = 2;
+  if (!gated && mt == 1 && rb == 4) rb = 2;
+#define GO(MT)                                  \
+  switch (rb) {                                 \
+    case 1: return launch<MT, 1>(a, gated, st); \
+    case 2: return launch<MT, 2>(a, gated, st); \
+    default: return launch<MT, 4>(a, gated, st); \
   }
-  DS_CHECK_LAUNCH();
-  if (Y == nullptr) return 0;  // sums stay in the workspace for a fused consumer (skinny_finalize.hip)
-  return ds_skinny_finalize_plain(ws, bias, Y, M, N, a.NP, st);
+  switch (mt) {
+    case 1: GO(1)
+    case 2: GO(2)
+    default: GO(3)
+  }
+#undef GO
 }

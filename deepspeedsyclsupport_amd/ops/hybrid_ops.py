@@ -91,11 +91,11 @@ def linear(x, w, sh=None, act=None):
     rows up), else the library product. act "gelu": the exact gelu of it (the stream's epilogue, else a pass of its own)."""
     rows = x.numel() // x.shape[-1]
     code = None if act is None else ACTS[act]
-    if sh is not None and x.is_cuda and x.is_contiguous() and 2 <= rows <= DECODE_ROWS:
-        return gemv_ops().decode_linear_sh(x, sh.wsh, sh.shape[0], act=code)
-    if x.is_cuda and x.is_contiguous() and x.dtype == torch.bfloat16 and 0 < rows <= DECODE_ROWS and \
-            gemv_ops().decode_linear_ok(rows, x.shape[-1]):
-        return gemv_ops().decode_linear(x, w, act=code)
+    if x.is_cuda and x.is_contiguous():
+        if sh is not None and rows >= 2 and gemv_ops().decode_linear_sh_ok(rows, *sh.shape, False):
+            return gemv_ops().decode_linear_sh(x, sh.wsh, sh.shape[0], act=code)
+        if x.dtype == torch.bfloat16 and 0 < rows <= DECODE_ROWS and gemv_ops().decode_linear_ok(rows, x.shape[-1]):
+            return gemv_ops().decode_linear(x, w, act=code)
     y = F.linear(x, w)
     return y if act is None else mixer_ops.gelu(y)
 
@@ -103,9 +103,9 @@ def linear(x, w, sh=None, act=None):
 def glu_linear(x, w, sh, limit):
     """Clamped gated activation of x . [gate | up]^T: the epilogue of the weight stream for decode-sized bf16 batches."""
     rows = x.numel() // x.shape[-1]
-    if x.is_cuda and x.dtype == torch.bfloat16 and 0 < rows <= DECODE_ROWS:
-        if sh is not None and rows >= 2:
+    if x.is_cuda and x.dtype == torch.bfloat16:
+        if sh is not None and rows >= 2 and gemv_ops().decode_linear_sh_ok(rows, *sh.shape, True):
             return gemv_ops().decode_linear_sh(x, sh.wsh, sh.shape[0], limit)
-        if gemv_ops().decode_linear_ok(rows, x.shape[-1]):
+        if 0 < rows <= DECODE_ROWS and gemv_ops().decode_linear_ok(rows, x.shape[-1]):
             return gemv_ops().decode_linear(x, w, limit)
     return clamped_glu(F.linear(x, w), limit)

@@ -66,7 +66,6 @@ EXTENSIONS = {
             "gemv/skinny_gemm.hip",
             "gemv/skinny_mfma.hip",
             "gemv/skinny_bf16_sh.hip",
-            "gemv/skinny_finalize.hip",
         ],
         "bindings": ["bind/gemv_bind.cpp"],
     },

@@ -88,3 +88,31 @@ def test_bf16_sh_fused_consumers_and_graph():
         torch.cuda.synchronize()
         torch.testing.assert_close(out.float(), bw.linear(x).float(), rtol=1e-2, atol=1e-2)
         torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 48])
+@pytest.mark.parametrize("N,K", [(50, 64), (6145, 576), (64, 8256), (16416, 128)])
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("norm", [False, True])
+def test_bf16_sh_products_with_what_stands_around_them_gpu(M, N, K, gated, norm):
+    """Edges of the tiles of rows, columns and steps, one to four blocks per workgroup, against fp64. A sum of K products is off
+    by at most K 2^-24 of their magnitudes' sum, the stored result by 2^-9 of itself; the activation multiplies the first by at most
+    1.2 times the other half's size."""
+    torch.manual_seed(M + N)
+    N = N // 32 * 32 + (0 if N % 32 == 0 else 32) if gated else N
+    x, w = torch.randn(M, K, device="cuda").bfloat16(), (torch.randn(N, K, device="cuda") * 0.1).bfloat16()
+    b, nw = torch.randn(N, device="cuda").bfloat16(), torch.randn(K, device="cuda").bfloat16()
+    res = torch.randn(M, N // 2 if gated else N, device="cuda").bfloat16()
+    xd = (x.float() * nw.float()).bfloat16().double() if norm else x.double()
+    rs = torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-5) if norm else 1.0
+    ref = rs * (xd @ w.double().t()) + b.double()
+    err = K * 2.0**-24 * (rs * (xd.abs() @ w.double().abs().t()) + b.double().abs())
+    if gated:
+        (g, u), (eg, eu) = ref.chunk(2, -1), err.chunk(2, -1)
+        ref, err = torch.nn.functional.silu(g) * u, 1.2 * (eg * u.abs() + eu * (g.abs() + 1))
+    ref = ref + res.double()
+    y = Bf16Weight(w).raw(x, b).finish(norm=(nw, 1e-5) if norm else None, residual=res, act=0 if gated else None, gated=gated)
+    assert y.shape == ref.shape
+    # (the activation's own exp is good to a few 2^-24, its error stays below that of the stored result)
+    assert ((y.double() - ref).abs() <= 2.0**-8 * ref.abs() + 2 * err + 2.0**-20 * (1 + ref.abs().max())).all()
