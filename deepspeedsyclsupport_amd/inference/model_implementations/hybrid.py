@@ -1160,7 +1160,7 @@ class DSHybridModel(DSInferenceModel):
         if meta.last_idx.numel() == 0:
             return tokens.new_empty((0, spec.vocab_size), dtype=self.dtype)
         y, r, gate = pending
-        return self._logits(r.finish(self, x, y, meta.last_idx.to(torch.int32), gate))
+        return self._logits(r.finish(self, x, y, meta.last_rows, gate))
 
     def _logits(self, h):
         return self._gather_vocab(ops.linear(h, self.lm_head, getattr(self, "lm_head_sh", None)))

@@ -171,7 +171,9 @@ class RaggedMeta:
     seq_ids: torch.Tensor            # [T] sequence of every token
     cu_q: torch.Tensor               # [S + 1] token offsets
     work: torch.Tensor               # [W, 2] (sequence, 128-row query block) for the prefill sequences
-    last_idx: torch.Tensor           # rows whose logits are wanted: [S] each sequence's last token, or a list given
+    last_idx: torch.Tensor           # int64 rows whose logits are wanted: [S] each sequence's last token, or a list given
+    last_rows: torch.Tensor          # the same as int32
+    all_rows: bool                   # those are all rows in their order
     n_decode: int                    # sequences [0, n_decode) are single-token decodes
     cu_host: List[int]
     start_host: List[int]
@@ -185,6 +187,7 @@ class RaggedMeta:
     n_short: int = 0                 # sequences [0, n_short) are decodes or short portions
     kv_offs: Optional[torch.Tensor] = None   # [S - n_short + 1] offsets of the other sequences' contexts laid end to end
     kv_total: int = 0                # ... and their end
+    ids: Optional[torch.Tensor] = None       # the new tokens, where `build` was given them
     seen: Dict[int, tuple] = field(default_factory=dict)   # `contexts` by window
 
     SHORT_TOKENS = 64    # portions up to this long count as short
@@ -212,9 +215,9 @@ class RaggedMeta:
         return self.seen[window]
 
     @staticmethod
-    def build(starts, n_new, block_lists, n_decode, block_size, device, slots=None, logit_rows=None):
+    def build(starts, n_new, block_lists, n_decode, block_size, device, slots=None, logit_rows=None, ids=None):
         """`slots`: state slots of the sequences; `logit_rows`: rows (of the concatenated tokens) whose logits are
-        wanted instead of every sequence's last."""
+        wanted instead of every sequence's last; `ids`: int64 tokens on the host that go along."""
         S = len(starts)
         cu = list(accumulate(n_new, initial=0))
         T = cu[-1]
@@ -262,14 +265,21 @@ class RaggedMeta:
         part(chunk_seqs)
         part(chunks)
         part(kv)
-        buf = torch.frombuffer(flat, dtype=torch.int32)
-        if device is not None and torch.device(device).type == "cuda":
-            buf = buf.pin_memory().to(device, non_blocking=True)
+        # ... behind the 64-bit ones: one copy, from pinned memory, so that no step waits for the steps before it
+        wide = torch.tensor(last, dtype=torch.int64)
+        wide = wide if ids is None else torch.cat([wide, ids])
+        cuda, n = device is not None and torch.device(device).type == "cuda", 2 * len(wide)
+        buf = torch.empty(n + len(flat), dtype=torch.int32, pin_memory=cuda)
+        buf[:n].view(torch.int64).copy_(wide)
+        buf[n:].copy_(torch.frombuffer(flat, dtype=torch.int32))
+        if cuda:
+            buf = buf.to(device, non_blocking=True)
+        wide, buf = buf[:n].view(torch.int64), buf[n:]
         views = [buf[a:b] for a, b in zip([0] + sizes, sizes)]
         pos_t, sid_t, st_t, len_t, cu_t, work_t, last_t, bt_t, slot_t, short_t, long_t, chunk_t, kv_t = views
         return RaggedMeta(block_tables=bt_t.view(S, width), start_pos=st_t, seq_lens=len_t, pos_ids=pos_t,
-                          seq_ids=sid_t, cu_q=cu_t, work=work_t.view(-1, 2), last_idx=last_t.long(),
-                          n_decode=n_decode, cu_host=cu, start_host=list(starts), max_len=width * block_size,
+                          seq_ids=sid_t, cu_q=cu_t, work=work_t.view(-1, 2), last_idx=wide[:len(last)], last_rows=last_t,
+                          all_rows=len(last) == T and last == list(range(T)), ids=None if ids is None else wide[len(last):], n_decode=n_decode, cu_host=cu, start_host=list(starts), max_len=width * block_size,
                           block_size=block_size, slots=slot_t, seq_list=short_t, chunk_seqs=long_t.view(-1, 2),
                           chunk_work=chunk_t.view(-1, 2), n_short=n_short, kv_offs=kv_t, kv_total=kv[-1])
 
@@ -781,23 +791,22 @@ def _ragged_attention(q, kc, vc, meta, scale, alibi, window):
     """q [T, Hq, D] -> [T, Hq, D] over the paged cache (new tokens already appended)."""
     T, Hq, D = q.shape
     nd, S = meta.n_decode, len(meta.start_host)
-    fast = q.is_cuda and q.dtype == torch.bfloat16 and kc.dtype == torch.bfloat16
+    fast = q.is_cuda and q.dtype == torch.bfloat16 and kc.dtype == torch.bfloat16 and D in PAGED_HEAD_DIMS
     from ...ops.native import hip_ops
-    if fast and D in PAGED_HEAD_DIMS and nd < S:
+    if fast and nd == S:
+        return hip_ops().paged_decode(q.contiguous(), kc, vc, meta.block_tables, meta.seq_lens, meta.max_len, scale, alibi,
+                                      window)
+    if fast:
         out = hip_ops().paged_prefill(q.contiguous(), kc, vc, meta.block_tables, meta.start_pos, meta.cu_q, meta.work,
                                       alibi, window, scale)
-    else:
-        out = torch.empty_like(q)
-        for i in range(nd, S):
-            a, b = meta.cu_host[i], meta.cu_host[i + 1]
-            out[a:b] = _seq_cached_attention(q[a:b], kc, vc, meta, i, scale, alibi, window)
-    if nd:
-        if fast and D in PAGED_HEAD_DIMS:
-            out[:nd] = hip_ops().paged_decode(q[:nd].contiguous(), kc, vc, meta.block_tables[:nd], meta.seq_lens[:nd],
-                                              meta.max_len, scale, alibi, window)
-        else:
-            for i in range(nd):
-                out[i:i + 1] = _seq_cached_attention(q[i:i + 1], kc, vc, meta, i, scale, alibi, window)
+        if nd:
+            hip_ops().paged_decode(q[:nd].contiguous(), kc, vc, meta.block_tables[:nd], meta.seq_lens[:nd], meta.max_len, scale,
+                                   alibi, window, out[:nd])
+        return out
+    out = torch.empty_like(q)
+    for i in range(S):
+        a, b = meta.cu_host[i], meta.cu_host[i + 1]
+        out[a:b] = _seq_cached_attention(q[a:b], kc, vc, meta, i, scale, alibi, window)
     return out
 
 
@@ -970,8 +979,10 @@ class DSInferenceModel(nn.Module):
         h = materialize(h)
         if meta.last_idx.numel() == 0:
             return h.new_empty((0, self.spec.vocab_size))
-        h = h[0].index_select(0, meta.last_idx)
-        residual = residual[0].index_select(0, meta.last_idx) if residual is not None else None
+        h, residual = h[0], residual[0] if residual is not None else None
+        if not meta.all_rows:
+            h = h.index_select(0, meta.last_idx)
+            residual = residual.index_select(0, meta.last_idx) if residual is not None else None
         logits = self._decode_logits(h, residual)
         if logits is not None:
             return logits

@@ -44,7 +44,8 @@ class InferenceEngineV2:
         model.allocate_cache(num_blocks, bs, num_slots)
         self._state_manager = DSStateManager(sm, num_blocks, bs, num_slots)
         self._state_manager.attach_cache(getattr(model, "cache", None))
-        self._device = model.device if model.device is not None else torch.device("cpu")
+        self._device = torch.device(model.device if model.device is not None else "cpu")
+        self._stream = None  # of the last step
         self._batch = RaggedBatchWrapper(sm, bs, self._device)
 
     def _state_slots(self, sm, slot_bytes):
@@ -77,7 +78,8 @@ class InferenceEngineV2:
     def put(self, batch_uids: Iterable[int], batch_tokens: Iterable[torch.Tensor], do_checks=True,
             logit_positions=None) -> torch.Tensor:
         """One step. Returns one row of logits per sequence (its last new token), in the order given; with
-        `logit_positions` (per sequence, places among its new tokens) the rows of those places, in that order."""
+        `logit_positions` (per sequence, places among its new tokens) the rows of those places, in that order. Nothing waits for
+        the device: a step is prepared while the one before it runs. On another stream than that one it starts behind it."""
         uids = list(batch_uids)
         toks = [t.reshape(-1) for t in batch_tokens]
         if do_checks:
@@ -90,6 +92,7 @@ class InferenceEngineV2:
                 if int(lo) < 0 or int(hi) >= self._model.spec.vocab_size:
                     raise ValueError(f"token ids {int(lo)} to {int(hi)} outside the vocabulary of "
                                      f"{self._model.spec.vocab_size}")
+        self._follow_last_step()
         batch = self._batch
         batch.clear()
         seqs = []
@@ -99,12 +102,22 @@ class InferenceEngineV2:
             seq.pre_forward(t.numel())
             batch.insert_sequence(seq, t, do_checks=False)
             seqs.append(seq)
-        batch.finalize(logit_positions=logit_positions)
+        batch.finalize(logit_positions=[(t.numel() - 1, ) for t in toks] if logit_positions is None else logit_positions)
         logits = self._model.forward_ragged(batch.input_ids(), batch.meta)
-        out = batch.restore_order(logits) if logit_positions is None else logits
         for s in seqs:
             s.post_forward()
-        return out
+        return logits
+
+    def _follow_last_step(self):
+        """Cache and state blocks pass from step to step, also from a flushed sequence to a new one."""
+        if self._device.type != "cuda":
+            return
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("put() plans its batch on the host: it cannot be captured in a graph")
+        stream = torch.cuda.current_stream(self._device)
+        if self._stream is not None and self._stream != stream:
+            stream.wait_stream(self._stream)
+        self._stream = stream
 
     # ------------------------------------------------------------------------------------------ scheduling
     def _kv_requirements(self, seq, max_tokens, max_blocks):
@@ -143,8 +156,8 @@ class InferenceEngineV2:
                 seq = PlaceholderSequenceDescriptor(self._state_manager.block_size)
             if seq.seen_tokens + n > sm.max_context:
                 return SchedulingResult.SequenceTokenLimitExceeded
-            got, blocks = self._kv_requirements(seq, n, free)
-            if got != n:
+            blocks = seq.blocks_needed(n)
+            if n > 0 and blocks > free:
                 return SchedulingResult.KVCacheLimitExceeded
             free -= blocks
             total += n

@@ -77,16 +77,22 @@ class RaggedBatchWrapper:
                 at += n[i]
             rows = [first[i] + int(p) for i, want in enumerate(logit_positions) for p in want]
         slots = [s.slot for s in seqs] if seqs[0].slot is not None else None
-        self.meta = RaggedMeta.build([s.seen_tokens for s in seqs], [n[i] for i in self.order],
-                                     [s.blocks for s in seqs], sum(is_decode), bs, self._device, slots, rows)
         ids = torch.cat([self._toks[i] for i in self.order])
-        if self._device is not None:
+        packed = ids.dtype == torch.int64 and not ids.is_cuda
+        self.meta = RaggedMeta.build([s.seen_tokens for s in seqs], [n[i] for i in self.order],
+                                     [s.blocks for s in seqs], sum(is_decode), bs, self._device, slots, rows,
+                                     ids if packed else None)
+        if packed:
+            ids = self.meta.ids
+        elif self._device is not None:
             ids = ids.to(self._device, non_blocking=True)
         self._ids = ids
         self._is_finalized = True
 
     def restore_order(self, rows: torch.Tensor) -> torch.Tensor:
         """Per-sequence rows in kernel order -> rows in insertion order."""
+        if self.order == list(range(len(self.order))):
+            return rows
         inv = [0] * len(self.order)
         for j, i in enumerate(self.order):
             inv[i] = j

@@ -72,7 +72,7 @@ void need(const Tensor& t, const char* n) {
 
 // q [B, Hq, D] bf16; caches [NB, Hk, BS, D] bf16; block_table [B, max_blocks] int32; seq_lens [B] int32
 Tensor paged_decode(Tensor q, Tensor kc, Tensor vc, Tensor block_table, Tensor seq_lens, int64_t max_len, double scale,
-                    OptT alibi, int64_t window) {
+                    OptT alibi, int64_t window, OptT into) {
   need(q, "q"); need(kc, "k_cache"); need(vc, "v_cache"); need(block_table, "block_table"); need(seq_lens, "seq_lens");
   TORCH_CHECK(q.scalar_type() == at::kBFloat16 && kc.scalar_type() == at::kBFloat16, "bf16 q/cache");
   TORCH_CHECK(block_table.scalar_type() == at::kInt && seq_lens.scalar_type() == at::kInt, "int32 tables");
@@ -83,7 +83,11 @@ Tensor paged_decode(Tensor q, Tensor kc, Tensor vc, Tensor block_table, Tensor s
   TORCH_CHECK((int64_t)max_blocks * BS >= max_len, "block table too small for max_len");
   const int64_t span = window > 0 && window < max_len ? window : max_len;  // keys in sight
   const int splits = ds_paged_decode_splits(B, Hk, (int)span);
-  auto out = torch::empty_like(q);
+  if (into.has_value()) {
+    need(*into, "out");
+    TORCH_CHECK(into->sizes() == q.sizes() && into->scalar_type() == at::kBFloat16, "paged_decode: out like q");
+  }
+  auto out = into.has_value() ? *into : torch::empty_like(q);
   auto fo = q.options().dtype(at::kFloat);
   Tensor pacc, pml;
   if (splits > 1) {
@@ -571,7 +575,8 @@ void register_inference_ops(pybind11::module& m) {
         py::arg("kc"), py::arg("vc"), py::arg("block_table"), py::arg("start_pos"), py::arg("n_new"), py::arg("Hq"),
         py::arg("Hk"), py::arg("rot"), py::arg("interleaved"), py::arg("want_kv"), py::arg("seq_ids") = py::none(), py::arg("acc_rows") = 0,
         py::arg("acc_bias") = py::none());
-  m.def("paged_decode", &paged_decode);
+  m.def("paged_decode", &paged_decode, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_table"),
+        py::arg("seq_lens"), py::arg("max_len"), py::arg("scale"), py::arg("alibi"), py::arg("window"), py::arg("out") = py::none());
   m.def("kv_append", &kv_append);
   m.def("quantize", &quantize);
   m.def("dequantize", &dequantize);

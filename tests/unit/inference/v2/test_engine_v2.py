@@ -139,3 +139,35 @@ def test_serialize_and_rebuild_from_ds_checkpoint(tmp_path):
     eng.serialize(str(tmp_path))
     eng2 = build_engine_from_ds_checkpoint(str(tmp_path), eng._config, device=torch.device("cpu"))
     assert _drive(eng2, prompts, 4) == ref
+
+
+@pytest.mark.parametrize("int32", [False, True])
+def test_rows_come_back_in_the_order_given(int32):
+    """Steps that mix prompts, portions and decodes (the kernels take decodes first), and steps of decodes alone."""
+    m = _model()
+    mixed, alone = _engine(m), _engine(m)
+    g = torch.Generator().manual_seed(4)
+    steps = [([3, 1], (7, 2)), ([5, 1, 3], (9, 1, 1)), ([1, 5, 3], (1, 1, 1)), ([3, 7, 5], (4, 70, 1))]
+    for uids, lens in steps:
+        toks = [torch.randint(0, 128, (n, ), generator=g, dtype=torch.int32 if int32 else torch.int64) for n in lens]
+        rows = mixed.put(uids, toks)
+        assert rows.shape[0] == len(uids)
+        for u, t, row in zip(uids, toks, rows):
+            assert torch.allclose(row, alone.put([u], [t])[0], atol=1e-5), (u, lens)
+
+
+@pytest.mark.gpu
+def test_steps_on_alternating_streams_gpu():
+    """No step waits on the host for the one before it: a step on another stream has to wait on the device."""
+    m = _model(H=256)
+    eng = [_engine(m, dtype=torch.bfloat16, device=torch.device("cuda"), blocks=128, bs=16) for _ in range(2)]
+    g = torch.Generator().manual_seed(5)
+    streams, rows = [torch.cuda.Stream() for _ in range(2)], []
+    for i in range(12):
+        toks = [torch.randint(0, 128, (60 if i == 0 else 1, ), generator=g) for _ in range(4)]
+        want = eng[0].put(range(4), toks).clone()
+        with torch.cuda.stream(streams[i % 2]):
+            rows.append((eng[1].put(range(4), toks), want))
+    torch.cuda.synchronize()
+    for got, want in rows:
+        assert torch.equal(got, want)
