@@ -8,16 +8,23 @@
 //
 // Tensors are [Z, S, H, D] with arbitrary (z, s, h) strides (Z = B*N for Evoformer, B for BERT); bias1 is indexed
 // [z, key] (per-key mask bias), bias2 is [Z / b2_div, H, S, S] (pair bias shared by b2_div consecutive z).
-//  * forward: one workgroup = 4 waves x 32 query rows of one (z, h); 64-key K/V tiles double-buffered in LDS (rows
-//    padded to 2D + 16 bytes: conflict-free b128 row reads without a swizzle); S^T = K.Q^T on
-//    v_mfma_f32_32x32x16 so each lane owns one query row's scores, biases added in natural units, online softmax,
-//    P reused as the A operand of O += P.V (V by the hardware transposed read); dropout multiplies P by
-//    keep / (1 - p) after the normaliser (Philox-4x32 keyed by (z, h, query, key), regenerated in the backward);
-//  * backward: three atomic-free passes (dQ query-outer; dK/dV key-outer; the shared pair-bias gradient summed over
-//    the z that share it in registers), P recomputed from the saved LSE in each — see the backward section.
+//  * forward: one workgroup = 4 waves x 32 query rows of one (z, h); 64-key K/V tiles in LDS (rows padded to 2D + 16 bytes:
+//    conflict-free b128 row reads without a swizzle); S^T = K.Q^T on v_mfma_f32_32x32x16 so each lane owns one query row's scores, biases added in natural units (a mask of the type's lowest
+//    value must not become -inf), online softmax, P reused as the A operand of O += P.V (V by the hardware transposed
+//    read); dropout multiplies P by keep / (1 - p) after the normaliser (Philox-4x32 keyed by (z, h, query, key),
+//    regenerated in the backward);
+//  * backward: passes without atomics on the big tensors (dQ query-outer; dK/dV key-outer; the shared pair-bias gradient summed
+//    over the z that share it in registers), P recomputed from the saved LSE in each — see the backward section.
+// All passes are bound by the vector instructions around the exponentials (about ten a score) and by latency: tiles are small and
+// few, so each has ONE buffer in LDS and nothing is held in registers for the next one: three workgroups share a CU and cover each
+// other's loads (held ahead: 52 us for 40 in the forward; a fourth workgroup, by spilling: 63). Keys past the end are -inf in
+// the tile's per-key biases, which costs a score nothing. Measured at [256, 256, 4, 32] with both biases, us, before (two
+// buffers, two workgroups a CU, a mask per score) and now: forward 64 and 40, dQ and dK/dV 158 and 97, dB2 234 and 47;
+// [100, 133, 8, 32], whose rows start anywhere: 29, 66 and 33.
 #include "ds_hip.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -84,8 +91,9 @@ struct SmallArgs {
   float pdrop;     // 0 = no dropout
   uint32_t thresh; // keep if philox >= thresh
   uint64_t seed;
-  int vec_bias;    // bias rows in whole 16-B chunks (Sk % 8 == 0, 16-B aligned rows): one load per 8 keys
-  int nsplit;      // dB2 pass: the b2_div sharing z are split over this many workgroups (atomics when > 1)
+  int64_t b2_last; // elements of bias2 - 8 (at least 0): where its last whole chunk begins
+  int nsplit;      // dB2 pass: the b2_div sharing z are split over this many workgroups
+  float* part;     // ... whose sums go here [nsplit, Z / b2_div, H, S, S] when they are several
   int Sk;          // keys (the forward may attend to a context of another length; the backward needs Sk == S)
 };
 
@@ -100,30 +108,29 @@ __device__ __forceinline__ void add4(const fp16* p, float (&f)[4]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) f[i] += (float)v[i];
 }
-__device__ __forceinline__ void store4(bf16* p, const float (&f)[4]) {
-  bf16x4 v;
+// 16-B chunks (8 keys) of rows of bias2, at any alignment, CPR a row: chunk tid + i NTHR of the rows row0.. and keys key0.. of the
+// matrix at `mat`. What lies past the end of a row belongs to keys that -inf masks; past the end of the tensor nothing is read: the
+// last whole chunk there is, shifted (a path of its own: the shifts would cost every tile an eighth of its instructions).
+template <int CPR, typename T>
+__device__ __forceinline__ void bias_chunks(const SmallArgs<T>& a, int64_t mat, int row0, int key0, int tid, u32x4_t (&out)[4]) {
+  typedef unsigned __int128 u128;
+  constexpr int ROWS = 4 * NTHR / CPR;
+  auto at = [&](int i) {
+    const int c = tid + i * NTHR;
+    return mat + (int64_t)min(row0 + c / CPR, a.S - 1) * a.Sk + key0 + c % CPR * 8;
+  };
+  if (mat + (int64_t)min(row0 + ROWS - 1, a.S - 1) * a.Sk + key0 + CPR * 8 <= a.b2_last + 8) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = (bf16)f[i];
-  *reinterpret_cast<bf16x4*>(p) = v;
-}
-__device__ __forceinline__ void store4(fp16* p, const float (&f)[4]) {
-  fp16x4 v;
+    for (int i = 0; i < 4; ++i) __builtin_memcpy(&out[i], a.b2 + at(i), 16);
+  } else {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = (fp16)f[i];
-  *reinterpret_cast<fp16x4*>(p) = v;
-}
-
-// 16 B (8 keys) of a bias row starting at key kb; never reads past key S-1 (vec: S % 8 == 0 and 16-B rows)
-template <typename T>
-__device__ __forceinline__ u32x4_t bias_chunk(const T* row, int kb, int S, int vec) {
-  if (vec) {
-    if (kb < S) return *reinterpret_cast<const u32x4_t*>(row + kb);
-    return u32x4_t{0u, 0u, 0u, 0u};
+    for (int i = 0; i < 4; ++i) {
+      const int64_t off = at(i), from = min(off, a.b2_last);
+      u128 v;
+      __builtin_memcpy(&v, a.b2 + from, 16);
+      out[i] = __builtin_bit_cast(u32x4_t, v >> 16 * (int)min(off - from, (int64_t)7));
+    }
   }
-  typename MF<T>::V8 v;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = kb + i < S ? row[kb + i] : (T)0.f;
-  return __builtin_bit_cast(u32x4_t, v);
 }
 
 __device__ __forceinline__ void st16_as_2x8(char* p, u32x4_t v) {  // 8-B aligned LDS destination
@@ -138,67 +145,55 @@ struct Tiles {
   static constexpr int CPR = D / 8, PER = CPR * BN / NTHR;
 };
 
-// One 64-key tile for the query-row kernels (forward, dQ, dB2): K and V rows, bias1 of the 64 keys and the
-// workgroup's [128 q][64 key] bias2 block, staged global -> registers -> LDS (two-phase so the loads of tile j+1
-// are in flight while tile j computes). bias2 rows are 136 B apart: the 8-B reads of 32 different rows by one wave
-// land on 64 distinct banks.
-template <typename T, int D>
+// One 64-key tile for the query-row kernels (forward, dQ): K and V rows, per-key biases of the 64 keys (fp32, -inf past the
+// end) and the workgroup's [128 q][64 key] bias2 block, staged global -> registers -> LDS. bias2 rows are 136 B apart: the 8-B reads of 32 different rows by one wave
+// land on 64 distinct banks. PAIR: with the bias2 block.
+template <typename T, int D, bool PAIR>
 struct KeyTile {
   static constexpr int PER = Tiles<T, D>::PER, CPR = Tiles<T, D>::CPR;
   static constexpr int B2RS = 2 * BN + 8;
-  static constexpr int OFF_V = TILE<D>(), OFF_B2 = 2 * TILE<D>(), OFF_B1 = OFF_B2 + BM * B2RS;
-  static constexpr int BYTES = OFF_B1 + 2 * BN;
-  u32x4_t rk[PER], rv[PER], rb2[4], rb1;
-  // b2blk: the [S, S] bias2 matrix of this (z-group, head) or null; qrow0: first query row of the workgroup
+  static constexpr int OFF_V = TILE<D>(), OFF_B1 = 2 * TILE<D>(), OFF_B2 = OFF_B1 + 4 * BN;
+  static constexpr int BYTES = OFF_B2 + (PAIR ? BM * B2RS : 0);
+  u32x4_t rk[PER], rv[PER], rb2[4];
+  float rb1;
+  // b2mat: where the [S, Sk] bias2 matrix of this (z-group, head) begins; qrow0: first query row of the workgroup
   __device__ __forceinline__ void load(const SmallArgs<T>& a, const T* Kp, const T* Vp, const T* b1p,
-                                       const T* b2blk, int qrow0, int k0, int tid, bool kv = true) {
-    if (kv) {
+                                       int64_t b2mat, int qrow0, int k0, int tid) {
 #pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int c = tid + i * NTHR, row = c / CPR, ch = c % CPR;
-        const int key = min(k0 + row, a.Sk - 1);
-        rk[i] = *reinterpret_cast<const u32x4_t*>(Kp + (int64_t)key * a.ks + ch * 8);
-        rv[i] = *reinterpret_cast<const u32x4_t*>(Vp + (int64_t)key * a.vs + ch * 8);
-      }
+    for (int i = 0; i < PER; ++i) {
+      const int c = tid + i * NTHR, row = c / CPR, ch = c % CPR;
+      const int key = min(k0 + row, a.Sk - 1);
+      rk[i] = *reinterpret_cast<const u32x4_t*>(Kp + (int64_t)key * a.ks + ch * 8);
+      rv[i] = *reinterpret_cast<const u32x4_t*>(Vp + (int64_t)key * a.vs + ch * 8);
     }
-    if (b2blk) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = tid + i * NTHR, row = c >> 3, ch = c & 7;
-        const int q = min(qrow0 + row, a.S - 1);
-        rb2[i] = bias_chunk(b2blk + (int64_t)q * a.Sk, k0 + ch * 8, a.Sk, a.vec_bias);
-      }
-    }
-    if (b1p && tid < BN / 8) rb1 = bias_chunk(b1p, k0 + tid * 8, a.Sk, a.vec_bias);
+    if constexpr (PAIR) bias_chunks<8>(a, b2mat, qrow0, k0, tid, rb2);
+    if (tid < BN) rb1 = k0 + tid >= a.Sk ? -INFINITY : b1p ? (float)b1p[k0 + tid] : 0.f;
   }
-  __device__ __forceinline__ void store(char* buf, int tid, bool hb1, bool hb2, bool kv = true) {
-    if (kv) {
+  __device__ __forceinline__ void store(char* buf, int tid) {
 #pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int c = tid + i * NTHR, row = c / CPR, ch = c % CPR;
-        *reinterpret_cast<u32x4_t*>(buf + row * RS<D>() + ch * 16) = rk[i];
-        *reinterpret_cast<u32x4_t*>(buf + OFF_V + row * RS<D>() + ch * 16) = rv[i];
-      }
+    for (int i = 0; i < PER; ++i) {
+      const int c = tid + i * NTHR, row = c / CPR, ch = c % CPR;
+      *reinterpret_cast<u32x4_t*>(buf + row * RS<D>() + ch * 16) = rk[i];
+      *reinterpret_cast<u32x4_t*>(buf + OFF_V + row * RS<D>() + ch * 16) = rv[i];
     }
-    if (hb2) {
+    if constexpr (PAIR) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int c = tid + i * NTHR, row = c >> 3, ch = c & 7;
         st16_as_2x8(buf + OFF_B2 + row * B2RS + ch * 16, rb2[i]);
       }
     }
-    if (hb1 && tid < BN / 8) *reinterpret_cast<u32x4_t*>(buf + OFF_B1 + tid * 16) = rb1;
+    if (tid < BN) reinterpret_cast<float*>(buf + OFF_B1)[tid] = rb1;
   }
 };
 
-// bias1 + bias2 of the 4 keys kr..kr+3 of the tile (kr % 4 == 0) for LDS bias2 row `brow`; keys >= S give -inf
-template <typename T, int D>
-__device__ __forceinline__ void tile_bias4(const char* buf, const char* b2buf, bool hb1, bool hb2, int brow, int kr,
-                                           int key0, int S, float (&bb)[4]) {
+// per-key bias + bias2 of the 4 keys kr + 4 h .. + 3 of the tile, kr a constant: `b1row` and `b2row` are where key 4 h stands
+template <typename T, bool PAIR>
+__device__ __forceinline__ void tile_bias4(const char* b1row, const char* b2row, int kr, float (&bb)[4]) {
+  const f32x4 b1 = *reinterpret_cast<const f32x4*>(b1row + kr * 4);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) bb[i] = key0 + i < S ? 0.f : -INFINITY;
-  if (hb1) add4(reinterpret_cast<const T*>(buf + KeyTile<T, D>::OFF_B1 + kr * 2), bb);
-  if (hb2) add4(reinterpret_cast<const T*>(b2buf + KeyTile<T, D>::OFF_B2 + brow * KeyTile<T, D>::B2RS + kr * 2), bb);
+  for (int i = 0; i < 4; ++i) bb[i] = b1[i];
+  if constexpr (PAIR) add4(reinterpret_cast<const T*>(b2row + kr * 2), bb);
 }
 
 // transposed 4+4-row read of a row-major 16-bit image into an MFMA operand (k slots = rows rb+{0..3}, rb+8+{0..3})
@@ -216,11 +211,11 @@ __device__ __forceinline__ V8 tr_read(const char* img, int rs, int rb, int ch0, 
 }
 
 // ================================================================================================== forward
-template <typename T, int D>
+template <typename T, int D, bool DROP, bool PAIR>
 __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
   typedef typename MF<T>::V8 V8;
-  typedef KeyTile<T, D> KT;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+  typedef KeyTile<T, D, PAIR> KT;
+  __shared__ __attribute__((aligned(16))) char smem[KT::BYTES + 4 * 32 * 4];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, h = lane >> 5, l32 = lane & 31;
   const int nqb = (a.S + BM - 1) / BM;
   const int qb = blockIdx.x % nqb, hd = (blockIdx.x / nqb) % a.H, z = blockIdx.x / (nqb * a.H);
@@ -229,8 +224,7 @@ __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
   const T* Kp = a.k + z * a.kz + hd * a.kh;
   const T* Vp = a.v + z * a.vz + hd * a.vh;
   const T* b1p = a.b1 ? a.b1 + z * a.b1_zs : nullptr;
-  const T* b2blk = a.b2 ? a.b2 + ((int64_t)(z / a.b2_div) * a.H + hd) * a.S * a.Sk : nullptr;
-  const bool hb1 = b1p != nullptr, hb2 = b2blk != nullptr;
+  const int64_t b2mat = ((int64_t)(z / a.b2_div) * a.H + hd) * a.S * a.Sk;
   const uint64_t drow = ((uint64_t)z * a.H + hd) * (uint64_t)a.S + (uint64_t)qrow;
 
   V8 qf[D / 16];
@@ -239,7 +233,7 @@ __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
 #pragma unroll
     for (int kk = 0; kk < D / 16; ++kk) qf[kk] = *reinterpret_cast<const V8*>(qr + 16 * kk);
   }
-  float* scratch = reinterpret_cast<float*>(smem + 2 * KT::BYTES) + wid * 32;
+  float* scratch = reinterpret_cast<float*>(smem + KT::BYTES) + wid * 32;
   KT stg;
 
   f32x16_t o[D / 32];
@@ -250,17 +244,18 @@ __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
   float m_run = -INFINITY, l_run = 0.f;
   const int nt = (a.Sk + BN - 1) / BN;
   const float LOG2E = 1.4426950408889634f;
-  const float inv_keep = a.pdrop > 0.f ? 1.f / (1.f - a.pdrop) : 1.f;
+  const float inv_keep = DROP ? 1.f / (1.f - a.pdrop) : 1.f;
   const int gch = (lane >> 1) & 1, colhalf = (lane >> 4) & 1;
 
-  stg.load(a, Kp, Vp, b1p, b2blk, qb * BM, 0, tid);
-  stg.store(smem, tid, hb1, hb2);
+  stg.load(a, Kp, Vp, b1p, b2mat, qb * BM, 0, tid);
+  stg.store(smem, tid);
   __syncthreads();
   for (int j = 0; j < nt; ++j) {
-    const int cur = j & 1, k0 = j * BN;
-    if (j + 1 < nt) stg.load(a, Kp, Vp, b1p, b2blk, qb * BM, k0 + BN, tid);
-    const char* buf = smem + cur * KT::BYTES;
+    const int k0 = j * BN;
+    const char* buf = smem;
     const char* Vt = buf + KT::OFF_V;
+    const char* b1row = buf + KT::OFF_B1 + 16 * h;
+    const char* b2row = buf + KT::OFF_B2 + (wid * 32 + l32) * KT::B2RS + 8 * h;
     f32x16_t s[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -272,14 +267,13 @@ __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
         s[t] = MF<T>::mma(av, qf[kk], s[t]);
       }
     }
-    // natural-unit logits: scale * q.k + bias1[key] + bias2[q, key]; keys past S masked
+    // natural-unit logits: scale * q.k + bias1[key] + bias2[q, key]
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int kr = t * 32 + 8 * g + 4 * h;
         float bb[4];
-        tile_bias4<T, D>(buf, buf, hb1, hb2, wid * 32 + l32, kr, k0 + kr, a.Sk, bb);
+        tile_bias4<T, PAIR>(b1row, b2row, t * 32 + 8 * g, bb);
 #pragma unroll
         for (int i = 0; i < 4; ++i) s[t][4 * g + i] = s[t][4 * g + i] * a.scale + bb[i];
       }
@@ -290,18 +284,19 @@ __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
     const float m_new = fmaxf(m_run, mx);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * LOG2E);
-    float psum = 0.f;
+    f32x4 psum{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const float p = __builtin_amdgcn_exp2f((s[t][r] - m_use) * LOG2E);
         s[t][r] = p;
-        psum += p;
+        psum[r & 3] += p;
       }
-    l_run = l_run * alpha + psum;
+    l_run = l_run * alpha + ((psum[0] + psum[1]) + (psum[2] + psum[3]));
+    asm volatile("" : "+v"(l_run));  // (summed here, not kept as 32 terms through the rest)
     m_run = m_new;
-    if (a.pdrop > 0.f) {  // dropout after the normaliser: O accumulates P * keep / (1 - p)
+    if constexpr (DROP) {  // dropout after the normaliser: O accumulates P * keep / (1 - p)
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -344,8 +339,12 @@ __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
         for (int ss = 0; ss < 2; ++ss)
           o[dt] = MF<T>::mma(pa[t][ss], tr_read<V8>(Vt, RS<D>(), t * 32 + 16 * ss + 4 * h, ch0, lane), o[dt]);
     }
-    if (j + 1 < nt) stg.store(smem + (cur ^ 1) * KT::BYTES, tid, hb1, hb2);
     __syncthreads();
+    if (j + 1 < nt) {
+      stg.load(a, Kp, Vp, b1p, b2mat, qb * BM, k0 + BN, tid);
+      stg.store(smem, tid);
+      __syncthreads();
+    }
   }
   const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
@@ -385,11 +384,11 @@ __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
 //     registers.
 
 // ---------------------------------------------------------------- pass 1: dQ, delta (and unshared dB2)
-template <typename T, int D>
-__global__ void __launch_bounds__(NTHR, D == 32 ? 2 : 1) small_bwd_dq_kernel(SmallArgs<T> a) {
+template <typename T, int D, bool DROP, bool PAIR>
+__global__ void __launch_bounds__(NTHR, 2) small_bwd_dq_kernel(SmallArgs<T> a) {
   typedef typename MF<T>::V8 V8;
-  typedef KeyTile<T, D> KT;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+  typedef KeyTile<T, D, PAIR> KT;
+  __shared__ __attribute__((aligned(16))) char smem[KT::BYTES];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, h = lane >> 5, l32 = lane & 31;
   const int nqb = (a.S + BM - 1) / BM;
   const int qb = blockIdx.x % nqb, hd = (blockIdx.x / nqb) % a.H, z = blockIdx.x / (nqb * a.H);
@@ -400,8 +399,6 @@ __global__ void __launch_bounds__(NTHR, D == 32 ? 2 : 1) small_bwd_dq_kernel(Sma
   const T* Vp = a.v + z * a.vz + hd * a.vh;
   const T* b1p = a.b1 ? a.b1 + z * a.b1_zs : nullptr;
   const int64_t b2mat = ((int64_t)(z / a.b2_div) * a.H + hd) * a.S * a.S;
-  const T* b2blk = a.b2 ? a.b2 + b2mat : nullptr;
-  const bool hb1 = b1p != nullptr, hb2 = b2blk != nullptr;
   float* db2p = (a.db2 && a.b2_div == 1) ? a.db2 + b2mat + (int64_t)qc * a.S : nullptr;
   const uint64_t drow = ((uint64_t)z * a.H + hd) * (uint64_t)a.S + (uint64_t)qrow;
 
@@ -423,9 +420,9 @@ __global__ void __launch_bounds__(NTHR, D == 32 ? 2 : 1) small_bwd_dq_kernel(Sma
   }
   const int64_t lrow = ((int64_t)z * a.H + hd) * a.S;
   if (lane < 32 && qlive) a.delta[lrow + qrow] = delta;
-  const float lse = a.lse[lrow + qc];
+  const float lse = qlive ? a.lse[lrow + qc] : INFINITY;
   const float LOG2E = 1.4426950408889634f;
-  const float inv_keep = a.pdrop > 0.f ? 1.f / (1.f - a.pdrop) : 1.f;
+  const float inv_keep = DROP ? 1.f / (1.f - a.pdrop) : 1.f;
   f32x16_t dq[D / 32];
 #pragma unroll
   for (int dt = 0; dt < D / 32; ++dt)
@@ -436,66 +433,58 @@ __global__ void __launch_bounds__(NTHR, D == 32 ? 2 : 1) small_bwd_dq_kernel(Sma
   const bool st4 = (a.S & 3) == 0;
 
   KT stg;
-  stg.load(a, Kp, Vp, b1p, b2blk, qb * BM, 0, tid);
-  stg.store(smem, tid, hb1, hb2);
+  stg.load(a, Kp, Vp, b1p, b2mat, qb * BM, 0, tid);
+  stg.store(smem, tid);
   __syncthreads();
   for (int j = 0; j < nt; ++j) {
-    const int cur = j & 1, k0 = j * BN;
-    if (j + 1 < nt) stg.load(a, Kp, Vp, b1p, b2blk, qb * BM, k0 + BN, tid);
-    const char* buf = smem + cur * KT::BYTES;
+    const int k0 = j * BN;
+    const char* buf = smem;
     const char* Vt = buf + KT::OFF_V;
-    f32x16_t s[2], dp[2];
+    const char* b1row = buf + KT::OFF_B1 + 16 * h;
+    const char* b2row = buf + KT::OFF_B2 + (wid * 32 + l32) * KT::B2RS + 8 * h;
+    V8 da[2][2];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < 2; ++t) {  // one 32-key half at a time, and in the schedule too (registers)
+      __builtin_amdgcn_sched_barrier(0);
+      f32x16_t s, dp;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) { s[t][r] = 0.f; dp[t][r] = 0.f; }
+      for (int r = 0; r < 16; ++r) { s[r] = 0.f; dp[r] = 0.f; }
 #pragma unroll
       for (int kk = 0; kk < D / 16; ++kk) {
         const V8 kv = *reinterpret_cast<const V8*>(buf + (t * 32 + l32) * RS<D>() + (2 * kk + h) * 16);
-        s[t] = MF<T>::mma(kv, qf[kk], s[t]);
+        s = MF<T>::mma(kv, qf[kk], s);
         const V8 vv = *reinterpret_cast<const V8*>(Vt + (t * 32 + l32) * RS<D>() + (2 * kk + h) * 16);
-        dp[t] = MF<T>::mma(vv, gf[kk], dp[t]);
+        dp = MF<T>::mma(vv, gf[kk], dp);
       }
-    }
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int kr = t * 32 + 8 * g + 4 * h, kb4 = k0 + kr;
         uint32_t kb = 0xfu;
-        if (a.pdrop > 0.f) kb = keep4(a.seed, drow, (uint32_t)(kb4 >> 2), a.thresh);
+        if constexpr (DROP) kb = keep4(a.seed, drow, (uint32_t)((k0 + t * 32 + 8 * g + 4 * h) >> 2), a.thresh);
         float bb[4];
-        tile_bias4<T, D>(buf, buf, hb1, hb2, wid * 32 + l32, kr, kb4, a.S, bb);
+        tile_bias4<T, PAIR>(b1row, b2row, t * 32 + 8 * g, bb);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int r = 4 * g + i;
-          const float x = s[t][r] * a.scale + bb[i];
-          const float p = (kb4 + i < a.S && qlive) ? __builtin_amdgcn_exp2f((x - lse) * LOG2E) : 0.f;
-          const float kf = ((kb >> i) & 1u) ? inv_keep : 0.f;
-          s[t][r] = p * (dp[t][r] * kf - delta);  // dS (natural units)
+          const float p = __builtin_amdgcn_exp2f((s[r] * a.scale + bb[i] - lse) * LOG2E);
+          if constexpr (DROP) dp[r] *= ((kb >> i) & 1u) ? inv_keep : 0.f;
+          s[r] = p * (dp[r] - delta);  // dS (natural units)
+          da[t][r >> 3][r & 7] = (T)s[r];
         }
-        if (db2p && qlive) {
-          if (st4) {
-            if (kb4 < a.S) {
-              f32x4 w;
+      }
+      if (db2p && qlive) {
 #pragma unroll
-              for (int i = 0; i < 4; ++i) w[i] = s[t][4 * g + i];
-              *reinterpret_cast<f32x4*>(db2p + kb4) = w;
-            }
+        for (int g = 0; g < 4; ++g) {
+          const int kb4 = k0 + t * 32 + 8 * g + 4 * h;
+          if (st4) {
+            if (kb4 < a.S) *reinterpret_cast<f32x4*>(db2p + kb4) = f32x4{s[4 * g], s[4 * g + 1], s[4 * g + 2], s[4 * g + 3]};
           } else {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-              if (kb4 + i < a.S) db2p[kb4 + i] = s[t][4 * g + i];
+              if (kb4 + i < a.S) db2p[kb4 + i] = s[4 * g + i];
           }
         }
       }
-    V8 da[2][2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int ss = 0; ss < 2; ++ss)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) da[t][ss][e] = (T)s[t][8 * ss + e];
+    }
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt) {
       const int ch0 = dt * 4 + colhalf * 2 + gch;
@@ -505,8 +494,12 @@ __global__ void __launch_bounds__(NTHR, D == 32 ? 2 : 1) small_bwd_dq_kernel(Sma
         for (int ss = 0; ss < 2; ++ss)
           dq[dt] = MF<T>::mma(da[t][ss], tr_read<V8>(buf, RS<D>(), t * 32 + 16 * ss + 4 * h, ch0, lane), dq[dt]);
     }
-    if (j + 1 < nt) stg.store(smem + (cur ^ 1) * KT::BYTES, tid, hb1, hb2);
     __syncthreads();
+    if (j + 1 < nt) {
+      stg.load(a, Kp, Vp, b1p, b2mat, qb * BM, k0 + BN, tid);
+      stg.store(smem, tid);
+      __syncthreads();
+    }
   }
   T* Gq = a.out + z * a.dz + hd * a.dh;
 #pragma unroll
@@ -521,17 +514,17 @@ __global__ void __launch_bounds__(NTHR, D == 32 ? 2 : 1) small_bwd_dq_kernel(Sma
 
 // ---------------------------------------------------------------- pass 2: dK, dV (key-outer), dB1
 // One 64-query tile: Q and dO rows, lse / delta of the 64 queries, and the [64 q][128 key] bias2 block of the
-// workgroup's keys (272-B rows; the wave reads 32 consecutive 2-B keys of one row).
-template <typename T, int D>
+// workgroup's keys (272-B rows, read transposed: the 32 keys of a wave by lane, the queries by register).
+template <typename T, int D, bool PAIR>
 struct QueryTile {
   static constexpr int PER = Tiles<T, D>::PER, CPR = Tiles<T, D>::CPR;
   static constexpr int B2RS = 2 * BM + 16;
   static constexpr int OFF_G = TILE<D>(), OFF_L = 2 * TILE<D>(), OFF_B2 = OFF_L + 2 * BN * 4;
-  static constexpr int BYTES = OFF_B2 + BN * B2RS;
+  static constexpr int BYTES = OFF_B2 + (PAIR ? BN * B2RS : 0);
   u32x4_t rq[PER], rg[PER], rb2[4];
   float rl;
   __device__ __forceinline__ void load(const SmallArgs<T>& a, const T* Qp, const T* Gp, int64_t lrow,
-                                       const T* b2blk, int key0, int q0, int tid) {
+                                       int64_t b2mat, int key0, int q0, int tid) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int c = tid + i * NTHR, row = c / CPR, ch = c % CPR;
@@ -539,20 +532,13 @@ struct QueryTile {
       rq[i] = *reinterpret_cast<const u32x4_t*>(Qp + (int64_t)q * a.qs + ch * 8);
       rg[i] = *reinterpret_cast<const u32x4_t*>(Gp + (int64_t)q * a.gs + ch * 8);
     }
-    if (tid < 2 * BN) {
-      const int q = min(q0 + (tid & (BN - 1)), a.S - 1);
-      rl = tid < BN ? a.lse[lrow + q] : a.delta[lrow + q];
+    if (tid < 2 * BN) {  // queries past the end weigh nothing
+      const int q = q0 + (tid & (BN - 1));
+      rl = tid < BN ? (q < a.S ? a.lse[lrow + q] : INFINITY) : (q < a.S ? a.delta[lrow + q] : 0.f);
     }
-    if (b2blk) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = tid + i * NTHR, row = c >> 4, ch = c & 15;
-        const int q = min(q0 + row, a.S - 1);
-        rb2[i] = bias_chunk(b2blk + (int64_t)q * a.S, key0 + ch * 8, a.S, a.vec_bias);
-      }
-    }
+    if constexpr (PAIR) bias_chunks<16>(a, b2mat, q0, key0, tid, rb2);
   }
-  __device__ __forceinline__ void store(char* buf, int tid, bool hb2) {
+  __device__ __forceinline__ void store(char* buf, int tid) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int c = tid + i * NTHR, row = c / CPR, ch = c % CPR;
@@ -560,7 +546,7 @@ struct QueryTile {
       *reinterpret_cast<u32x4_t*>(buf + OFF_G + row * RS<D>() + ch * 16) = rg[i];
     }
     if (tid < 2 * BN) reinterpret_cast<float*>(buf + OFF_L)[tid] = rl;
-    if (hb2) {
+    if constexpr (PAIR) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int c = tid + i * NTHR, row = c >> 4, ch = c & 15;
@@ -570,11 +556,11 @@ struct QueryTile {
   }
 };
 
-template <typename T, int D>
-__global__ void __launch_bounds__(NTHR, D == 32 ? 2 : 1) small_bwd_dkv_kernel(SmallArgs<T> a) {
+template <typename T, int D, bool DROP, bool PAIR>
+__global__ void __launch_bounds__(NTHR, 2) small_bwd_dkv_kernel(SmallArgs<T> a) {
   typedef typename MF<T>::V8 V8;
-  typedef QueryTile<T, D> QT;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+  typedef QueryTile<T, D, PAIR> QT;
+  __shared__ __attribute__((aligned(16))) char smem[QT::BYTES];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, h = lane >> 5, l32 = lane & 31;
   const int nkb = (a.S + BM - 1) / BM;
   const int kbk = blockIdx.x % nkb, hd = (blockIdx.x / nkb) % a.H, z = blockIdx.x / (nkb * a.H);
@@ -583,8 +569,7 @@ __global__ void __launch_bounds__(NTHR, D == 32 ? 2 : 1) small_bwd_dkv_kernel(Sm
   const bool klive = key < a.S;
   const T* Qp = a.q + z * a.qz + hd * a.qh;
   const T* Gp = a.dout + z * a.gz + hd * a.gh;
-  const T* b2blk = a.b2 ? a.b2 + ((int64_t)(z / a.b2_div) * a.H + hd) * a.S * a.S : nullptr;
-  const bool hb2 = b2blk != nullptr;
+  const int64_t b2mat = ((int64_t)(z / a.b2_div) * a.H + hd) * a.S * a.S;
 
   // B operands (column = this lane's key): K and V rows
   V8 kB[D / 16], vB[D / 16];
@@ -600,7 +585,7 @@ __global__ void __launch_bounds__(NTHR, D == 32 ? 2 : 1) small_bwd_dkv_kernel(Sm
   const float b1v = (a.b1 && klive) ? (float)a.b1[z * a.b1_zs + key] : 0.f;
   const int64_t lrow = ((int64_t)z * a.H + hd) * a.S;
   const float LOG2E = 1.4426950408889634f;
-  const float inv_keep = a.pdrop > 0.f ? 1.f / (1.f - a.pdrop) : 1.f;
+  const float inv_keep = DROP ? 1.f / (1.f - a.pdrop) : 1.f;
   f32x16_t dk[D / 32], dv[D / 32];
 #pragma unroll
   for (int dt = 0; dt < D / 32; ++dt)
@@ -611,20 +596,20 @@ __global__ void __launch_bounds__(NTHR, D == 32 ? 2 : 1) small_bwd_dkv_kernel(Sm
   const int gch = (lane >> 1) & 1, colhalf = (lane >> 4) & 1;
 
   QT stg;
-  stg.load(a, Qp, Gp, lrow, b2blk, kbk * BM, 0, tid);
-  stg.store(smem, tid, hb2);
+  stg.load(a, Qp, Gp, lrow, b2mat, kbk * BM, 0, tid);
+  stg.store(smem, tid);
   __syncthreads();
   for (int j = 0; j < nt; ++j) {
-    const int cur = j & 1, q0 = j * BN;
-    if (j + 1 < nt) stg.load(a, Qp, Gp, lrow, b2blk, kbk * BM, q0 + BN, tid);
-    const char* Qt = smem + cur * QT::BYTES;
+    const int q0 = j * BN;
+    const char* Qt = smem;
     const char* Gt = Qt + QT::OFF_G;
-    const float* lseT = reinterpret_cast<const float*>(Qt + QT::OFF_L);
+    const float* lseT = reinterpret_cast<const float*>(Qt + QT::OFF_L) + 4 * h;
     const float* delT = lseT + BN;
-    const char* b2t = Qt + QT::OFF_B2 + (wid * 32 + l32) * 2;
+    const char* b2t = Qt + QT::OFF_B2;
     // one 32-query half at a time (keeps the transient score / dP registers at 2 x 16)
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
+      __builtin_amdgcn_sched_barrier(0);
       f32x16_t s, dp;
 #pragma unroll
       for (int r = 0; r < 16; ++r) { s[r] = 0.f; dp[r] = 0.f; }
@@ -638,25 +623,30 @@ __global__ void __launch_bounds__(NTHR, D == 32 ? 2 : 1) small_bwd_dkv_kernel(Sm
       // rows = queries q0 + t*32 + crow(r, h), column = this lane's key
       V8 pa[2], da[2];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 l4 = *reinterpret_cast<const f32x4*>(lseT + t * 32 + 8 * g + 4 * h);
-        const f32x4 d4 = *reinterpret_cast<const f32x4*>(delT + t * 32 + 8 * g + 4 * h);
+      for (int ss = 0; ss < 2; ++ss) {
+        V8 b2;
+        if constexpr (PAIR) b2 = tr_read<V8>(b2t, QT::B2RS, t * 32 + 16 * ss + 4 * h, wid * 4 + colhalf * 2 + gch, lane);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = 4 * g + i, qr = t * 32 + 8 * g + 4 * h + i, q = q0 + qr;
-          const bool live = klive && q < a.S;
-          float x = s[r] * a.scale + b1v;
-          if (hb2) x += (float)*reinterpret_cast<const T*>(b2t + qr * QT::B2RS);
-          const float p = live ? __builtin_amdgcn_exp2f((x - l4[i]) * LOG2E) : 0.f;
-          float kf = 1.f;
-          if (a.pdrop > 0.f) {
-            const uint32_t kb = keep4(a.seed, (uint64_t)lrow + (uint64_t)q, (uint32_t)(key >> 2), a.thresh);
-            kf = ((kb >> (key & 3)) & 1u) ? inv_keep : 0.f;
+        for (int g = 2 * ss; g < 2 * ss + 2; ++g) {
+          const f32x4 l4 = *reinterpret_cast<const f32x4*>(lseT + t * 32 + 8 * g);
+          const f32x4 d4 = *reinterpret_cast<const f32x4*>(delT + t * 32 + 8 * g);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int r = 4 * g + i, e = r & 7;
+            float x = s[r] * a.scale + b1v;
+            if constexpr (PAIR) x += (float)b2[e];
+            const float p = __builtin_amdgcn_exp2f((x - l4[i]) * LOG2E);
+            float kf = 1.f;
+            if constexpr (DROP) {
+              const int q = q0 + t * 32 + 8 * g + 4 * h + i;
+              const uint32_t kb = keep4(a.seed, (uint64_t)lrow + (uint64_t)q, (uint32_t)(key >> 2), a.thresh);
+              kf = ((kb >> (key & 3)) & 1u) ? inv_keep : 0.f;
+            }
+            const float ds = p * (dp[r] * kf - d4[i]);
+            colsum += ds;
+            pa[ss][e] = (T)(p * kf);
+            da[ss][e] = (T)ds;
           }
-          const float ds = p * (dp[r] * kf - d4[i]);
-          colsum += ds;
-          pa[r >> 3][r & 7] = (T)(p * kf);
-          da[r >> 3][r & 7] = (T)ds;
         }
       }
 #pragma unroll
@@ -670,8 +660,12 @@ __global__ void __launch_bounds__(NTHR, D == 32 ? 2 : 1) small_bwd_dkv_kernel(Sm
         }
       }
     }
-    if (j + 1 < nt) stg.store(smem + (cur ^ 1) * QT::BYTES, tid, hb2);
     __syncthreads();
+    if (j + 1 < nt) {
+      stg.load(a, Qp, Gp, lrow, b2mat, kbk * BM, q0 + BN, tid);
+      stg.store(smem, tid);
+      __syncthreads();
+    }
   }
   if (a.db1) {
     colsum += __shfl_xor(colsum, 32, 64);
@@ -694,10 +688,11 @@ __global__ void __launch_bounds__(NTHR, D == 32 ? 2 : 1) small_bwd_dkv_kernel(Sm
 
 // ---------------------------------------------------------------- pass 3: dB2 summed over the z sharing it
 template <typename T, int D, bool DROP>
-__global__ void __launch_bounds__(NTHR, (D == 32 && !DROP) ? 2 : 1) small_bwd_db2_kernel(SmallArgs<T> a) {
+__global__ void __launch_bounds__(NTHR, 2) small_bwd_db2_kernel(SmallArgs<T> a) {
   typedef typename MF<T>::V8 V8;
-  typedef KeyTile<T, D> KT;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+  typedef KeyTile<T, D, true> Block;    // stages the bias2 block once
+  typedef KeyTile<T, D, false> KT;
+  __shared__ __attribute__((aligned(16))) char smem[2 * KT::BYTES > BM * Block::B2RS ? 2 * KT::BYTES : BM * Block::B2RS];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, h = lane >> 5, l32 = lane & 31;
   const int nqb = (a.S + BM - 1) / BM, nkt = (a.S + BN - 1) / BN;
   int bid = blockIdx.x;
@@ -705,23 +700,39 @@ __global__ void __launch_bounds__(NTHR, (D == 32 && !DROP) ? 2 : 1) small_bwd_db
   const int qb = bid % nqb; bid /= nqb;
   const int hd = bid % a.H; bid /= a.H;
   const int zb = bid % (a.Z / a.b2_div), split = bid / (a.Z / a.b2_div);
-  const int chunk = (a.b2_div + a.nsplit - 1) / a.nsplit;
-  const int n_lo = split * chunk, n_hi = min(a.b2_div, n_lo + chunk);
+  const int n_lo = (int)((int64_t)a.b2_div * split / a.nsplit), n_hi = (int)((int64_t)a.b2_div * (split + 1) / a.nsplit);
   const int q0w = qb * BM + wid * 32, qrow = q0w + l32;
   const int qc = min(qrow, a.S - 1);
   const bool qlive = qrow < a.S;
   const int k0 = kt * BN;
   const int64_t b2mat = ((int64_t)zb * a.H + hd) * a.S * a.S;
-  const bool hb1 = a.b1 != nullptr;
   const float LOG2E = 1.4426950408889634f;
-  const float inv_keep = a.pdrop > 0.f ? 1.f / (1.f - a.pdrop) : 1.f;
+  const float inv_keep = DROP ? 1.f / (1.f - a.pdrop) : 1.f;
   f32x16_t acc[2];
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
-  if (n_lo >= n_hi) return;  // uniform per workgroup (before any barrier)
 
+  // the lane's part of the bias2 block stays in its registers for all z
+  typedef T T4 __attribute__((ext_vector_type(4)));
+  T4 b2[2][4];
+  {
+    u32x4_t rb[4];
+    bias_chunks<8>(a, b2mat, qb * BM, k0, tid, rb);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = tid + i * NTHR, row = c >> 3, ch = c & 7;
+      st16_as_2x8(smem + row * Block::B2RS + ch * 16, rb[i]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        b2[t][g] = *reinterpret_cast<const T4*>(smem + (wid * 32 + l32) * Block::B2RS + (t * 32 + 8 * g + 4 * h) * 2);
+    __syncthreads();
+  }
   // per-z operands of the lane's query row, prefetched one z ahead
   V8 qf[D / 16], gf[D / 16];
   float lse = 0.f, delta = 0.f;
@@ -738,31 +749,30 @@ __global__ void __launch_bounds__(NTHR, (D == 32 && !DROP) ? 2 : 1) small_bwd_db
     delta = a.delta[lrow + qc];
   };
   KT stg;
-  {
-    const int z = zb * a.b2_div + n_lo;
-    stg.load(a, a.k + z * a.kz + hd * a.kh, a.v + z * a.vz + hd * a.vh, hb1 ? a.b1 + z * a.b1_zs : nullptr,
-             a.b2 + b2mat, qb * BM, k0, tid);
-    stg.store(smem, tid, hb1, true);  // the bias2 block lives in buffer 0 for the whole loop
-  }
+  auto load_keys = [&](int z) {
+    stg.load(a, a.k + z * a.kz + hd * a.kh, a.v + z * a.vz + hd * a.vh, a.b1 ? a.b1 + z * a.b1_zs : nullptr, 0, 0, k0, tid);
+  };
+  load_keys(zb * a.b2_div + n_lo);
+  stg.store(smem, tid);
   load_rows(zb * a.b2_div + n_lo);
   __syncthreads();
   for (int n = n_lo; n < n_hi; ++n) {
     const int z = zb * a.b2_div + n, cur = (n - n_lo) & 1;
     const bool more = n + 1 < n_hi;
-    if (more) {
-      const int zn = z + 1;
-      stg.load(a, a.k + zn * a.kz + hd * a.kh, a.v + zn * a.vz + hd * a.vh, hb1 ? a.b1 + zn * a.b1_zs : nullptr,
-               nullptr, qb * BM, k0, tid);
-    }
+    if (more) load_keys(z + 1);
     const char* buf = smem + cur * KT::BYTES;
-    const uint64_t drow = ((uint64_t)z * a.H + hd) * (uint64_t)a.S + (uint64_t)qrow;
     const float lse_n = lse, delta_n = delta;
     V8 qc_[D / 16], gc_[D / 16];
 #pragma unroll
     for (int kk = 0; kk < D / 16; ++kk) { qc_[kk] = qf[kk]; gc_[kk] = gf[kk]; }
     if (more) load_rows(z + 1);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {  // one 32-key half at a time
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) asm volatile("" : "+v"(b2[t][g]));  // (stays as it is: not held as 32 floats across the loop)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {  // one 32-key half at a time, and in the schedule too (registers)
+      __builtin_amdgcn_sched_barrier(0);
       f32x16_t s, dp;
 #pragma unroll
       for (int r = 0; r < 16; ++r) { s[r] = 0.f; dp[r] = 0.f; }
@@ -775,37 +785,33 @@ __global__ void __launch_bounds__(NTHR, (D == 32 && !DROP) ? 2 : 1) small_bwd_db
       }
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int kr = t * 32 + 8 * g + 4 * h, kb4 = k0 + kr;
         uint32_t kb = 0xfu;
-        if (DROP) kb = keep4(a.seed, drow, (uint32_t)(kb4 >> 2), a.thresh);
-        float bb[4];
-        tile_bias4<T, D>(buf, smem, hb1, true, wid * 32 + l32, kr, kb4, a.S, bb);
+        if constexpr (DROP)
+          kb = keep4(a.seed, ((uint64_t)z * a.H + hd) * (uint64_t)a.S + (uint64_t)qrow,
+                     (uint32_t)((k0 + t * 32 + 8 * g + 4 * h) >> 2), a.thresh);
+        const f32x4 b1 = *reinterpret_cast<const f32x4*>(buf + KT::OFF_B1 + 16 * h + (t * 32 + 8 * g) * 4);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int r = 4 * g + i;
-          const float x = s[r] * a.scale + bb[i];
-          const float p = (kb4 + i < a.S && qlive) ? __builtin_amdgcn_exp2f((x - lse_n) * LOG2E) : 0.f;
-          const float kf = ((kb >> i) & 1u) ? inv_keep : 0.f;
-          acc[t][r] += p * (dp[r] * kf - delta_n);
+          const float p = __builtin_amdgcn_exp2f((s[r] * a.scale + (b1[i] + (float)b2[t][g][i]) - lse_n) * LOG2E);
+          if constexpr (DROP) dp[r] *= ((kb >> i) & 1u) ? inv_keep : 0.f;
+          acc[t][r] += p * (dp[r] - delta_n);
         }
       }
     }
-    if (more) stg.store(smem + (cur ^ 1) * KT::BYTES, tid, hb1, false);
+    if (more) stg.store(smem + (cur ^ 1) * KT::BYTES, tid);
     __syncthreads();
   }
   if (!qlive) return;
-  float* out = a.db2 + b2mat + (int64_t)qrow * a.S;
+  // several workgroups: each writes its own sums, `sum_parts_kernel` adds them up in their order
+  float* out = (a.nsplit > 1 ? a.part + (int64_t)split * (a.Z / a.b2_div) * a.H * a.S * a.S : a.db2) + b2mat + (int64_t)qrow * a.S;
   const bool st4 = (a.S & 3) == 0;
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int kb4 = k0 + t * 32 + 8 * g + 4 * h;
-      if (a.nsplit > 1) {  // partial sums of several workgroups (dB2 zeroed by the caller)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (kb4 + i < a.S) unsafeAtomicAdd(out + kb4 + i, acc[t][4 * g + i]);
-      } else if (st4) {
+      if (st4) {
         if (kb4 < a.S) {
           f32x4 w;
 #pragma unroll
@@ -820,70 +826,87 @@ __global__ void __launch_bounds__(NTHR, (D == 32 && !DROP) ? 2 : 1) small_bwd_db
     }
 }
 
-template <typename K>
-void set_lds(K* fn, int bytes) {
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+// out[i] = sum over s of part[s][i]
+__global__ void __launch_bounds__(256) sum_parts_kernel(const float* __restrict__ part, float* __restrict__ out, int64_t n, int parts) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  if (n % 4 == 0) {
+    f32x4 v = *reinterpret_cast<const f32x4*>(part + i);
+    for (int s = 1; s < parts; ++s) v += *reinterpret_cast<const f32x4*>(part + s * n + i);
+    *reinterpret_cast<f32x4*>(out + i) = v;
+  } else {
+    for (int64_t e = i; e < min(i + 4, n); ++e) {
+      float v = part[e];
+      for (int s = 1; s < parts; ++s) v += part[s * n + e];
+      out[e] = v;
+    }
+  }
 }
 
-template <typename T, int D>
+// Workgroups that share the z of one pair-bias tile: as many as the chip holds at once (two a CU; [256, 256, 4, 32]: 47 us, with
+// 768 51, with 1024 53), at least four z each.
+int db2_splits(int Z, int H, int S, int b2_div) {
+  const int64_t base = (int64_t)(Z / b2_div) * H * ((S + BM - 1) / BM) * ((S + BN - 1) / BN);
+  return b2_div == 1 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(b2_div / 4, 512 / base));
+}
+
+template <typename T, int D, bool DROP, bool PAIR>
 int launch_small(SmallArgs<T> a, bool bwd, hipStream_t st) {
   const int nqb = (a.S + BM - 1) / BM;
   const dim3 grid(nqb * a.H * a.Z);
-  constexpr int lds_f = 2 * KeyTile<T, D>::BYTES + 4 * 32 * 4;
-  constexpr int lds_kv = 2 * QueryTile<T, D>::BYTES;
-  static bool attr = false;
-  if (!attr) {
-    set_lds(&small_fwd_kernel<T, D>, lds_f);
-    set_lds(&small_bwd_dq_kernel<T, D>, lds_f);
-    set_lds(&small_bwd_dkv_kernel<T, D>, lds_kv);
-    set_lds(&small_bwd_db2_kernel<T, D, false>, lds_f);
-    set_lds(&small_bwd_db2_kernel<T, D, true>, lds_f);
-    attr = true;
-  }
   if (!bwd) {
-    hipLaunchKernelGGL((small_fwd_kernel<T, D>), grid, dim3(NTHR), lds_f, st, a);
+    hipLaunchKernelGGL((small_fwd_kernel<T, D, DROP, PAIR>), grid, dim3(NTHR), 0, st, a);
     DS_CHECK_LAUNCH();
     return 0;
   }
-  hipLaunchKernelGGL((small_bwd_dq_kernel<T, D>), grid, dim3(NTHR), lds_f, st, a);
+  hipLaunchKernelGGL((small_bwd_dq_kernel<T, D, DROP, PAIR>), grid, dim3(NTHR), 0, st, a);
   DS_CHECK_LAUNCH();
-  hipLaunchKernelGGL((small_bwd_dkv_kernel<T, D>), grid, dim3(NTHR), lds_kv, st, a);
+  hipLaunchKernelGGL((small_bwd_dkv_kernel<T, D, DROP, PAIR>), grid, dim3(NTHR), 0, st, a);
   DS_CHECK_LAUNCH();
-  if (a.db2 && a.b2_div > 1) {
-    // enough workgroups to fill 256 CUs a few times over: split the sharing z when the tile grid is small
-    const int base = (a.Z / a.b2_div) * a.H * nqb * ((a.S + BN - 1) / BN);
-    a.nsplit = std::max(1, std::min(a.b2_div / 4, 1024 / base));
-    const dim3 g3(base * a.nsplit);
-    if (a.pdrop > 0.f)
-      hipLaunchKernelGGL((small_bwd_db2_kernel<T, D, true>), g3, dim3(NTHR), lds_f, st, a);
-    else
-      hipLaunchKernelGGL((small_bwd_db2_kernel<T, D, false>), g3, dim3(NTHR), lds_f, st, a);
+  if (PAIR && a.db2 && a.b2_div > 1) {
+    a.nsplit = db2_splits(a.Z, a.H, a.S, a.b2_div);
+    if (a.nsplit > 1 && a.part == nullptr) return (int)hipErrorInvalidValue;
+    const dim3 g3((a.Z / a.b2_div) * a.H * nqb * ((a.S + BN - 1) / BN) * a.nsplit);
+    hipLaunchKernelGGL((small_bwd_db2_kernel<T, D, DROP>), g3, dim3(NTHR), 0, st, a);
     DS_CHECK_LAUNCH();
+    if (a.nsplit > 1) {
+      const int64_t n = (int64_t)(a.Z / a.b2_div) * a.H * a.S * a.S;
+      hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, st, a.part, a.db2, n, a.nsplit);
+      DS_CHECK_LAUNCH();
+    }
   }
   return 0;
 }
 
 template <typename T>
 int dispatch_small(SmallArgs<T> a, int D, bool bwd, hipStream_t st) {
-  if (D == 32) return launch_small<T, 32>(a, bwd, st);
-  if (D == 64) return launch_small<T, 64>(a, bwd, st);
+  auto by_bias = [&](auto d, auto drop) {
+    constexpr int DD = decltype(d)::value;
+    constexpr bool DR = decltype(drop)::value;
+    return a.b2 ? launch_small<T, DD, DR, true>(a, bwd, st) : launch_small<T, DD, DR, false>(a, bwd, st);
+  };
+  auto by_drop = [&](auto d) { return a.pdrop > 0.f ? by_bias(d, std::true_type{}) : by_bias(d, std::false_type{}); };
+  if (D == 32) return by_drop(std::integral_constant<int, 32>{});
+  if (D == 64) return by_drop(std::integral_constant<int, 64>{});
   return (int)hipErrorInvalidValue;
 }
 
 }  // namespace
 
-// Forward. strides[12] = (q z,s,h)(k)(v)(o); dtype DS_BF16 / DS_F16; b1 / b2 may be null.
+// Forward. strides[12] = (q z,s,h)(k)(v)(o); dtype DS_BF16 / DS_F16; b1 / b2 may be null; b2_numel: elements that may be read
+// at b2, at least 8.
 extern "C" int ds_flash_small_fwd(const void* q, const void* k, const void* v, void* o, float* lse, const void* b1,
                                   const void* b2, const int64_t* st, int64_t b1_zs, int Z, int H, int S, int Sk, int D,
-                                  int b2_div, float scale, float pdrop, uint64_t seed, int vec_bias, int dtype,
+                                  int b2_div, float scale, float pdrop, uint64_t seed, int64_t b2_numel, int dtype,
                                   hipStream_t stream) {
-  if (Z <= 0 || H <= 0 || S <= 0 || Sk <= 0 || b2_div <= 0 || (D != 32 && D != 64) || pdrop < 0.f || pdrop >= 1.f)
+  if (Z <= 0 || H <= 0 || S <= 0 || Sk <= 0 || b2_div <= 0 || (D != 32 && D != 64) || pdrop < 0.f || pdrop >= 1.f ||
+      (b2 != nullptr && b2_numel < 8))
     return (int)hipErrorInvalidValue;
   const uint32_t thresh = (uint32_t)fminf(4294967295.f, pdrop * 4294967296.f);
 #define DS_SMALL_ARGS(T)                                                                                        \
   SmallArgs<T> a{(const T*)q, (const T*)k, (const T*)v, nullptr, nullptr, (T*)o, lse, (const T*)b1, (const T*)b2, \
                  nullptr, nullptr, nullptr, nullptr, nullptr, st[0], st[1], st[2], st[3], st[4], st[5], st[6], st[7],     \
-                 st[8], st[9], st[10], st[11], 0, 0, 0, 0, 0, 0, b1_zs, Z, H, S, b2_div, scale, pdrop, thresh, seed, vec_bias, 1, Sk};
+                 st[8], st[9], st[10], st[11], 0, 0, 0, 0, 0, 0, b1_zs, Z, H, S, b2_div, scale, pdrop, thresh, seed, b2_numel - 8, 1, nullptr, Sk};
   if (dtype == DS_BF16) {
     DS_SMALL_ARGS(bf16)
     return dispatch_small<bf16>(a, D, false, stream);
@@ -897,20 +920,24 @@ extern "C" int ds_flash_small_fwd(const void* q, const void* k, const void* v, v
 }
 
 // Backward. strides[18] = (q)(k)(v)(o)(dO)(dQ); dk / dv dense [Z, S, H, D] in the input dtype; delta fp32 [Z, H, S]
-// scratch; db1 [Z, S] fp32 (zeroed by the caller) or null; db2 [Z / b2_div, H, S, S] fp32 (fully written) or null.
+// scratch; db1 [Z, S] fp32 (zeroed by the caller) or null; db2 [Z / b2_div, H, S, S] fp32 (fully written) or null, db2_part
+// `ds_flash_small_db2_splits` times as much scratch when that is more than one.
+extern "C" int ds_flash_small_db2_splits(int Z, int H, int S, int b2_div) { return db2_splits(Z, H, S, b2_div); }
+
 extern "C" int ds_flash_small_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout,
                                   const float* lse, const void* b1, const void* b2, void* dq, void* dk, void* dv,
-                                  float* delta, float* db1, float* db2, const int64_t* st, int64_t b1_zs, int Z, int H, int S, int D,
-                                  int b2_div, float scale, float pdrop, uint64_t seed, int vec_bias, int dtype,
+                                  float* delta, float* db1, float* db2, float* db2_part, const int64_t* st, int64_t b1_zs, int Z, int H, int S, int D,
+                                  int b2_div, float scale, float pdrop, uint64_t seed, int64_t b2_numel, int dtype,
                                   hipStream_t stream) {
-  if (Z <= 0 || H <= 0 || S <= 0 || b2_div <= 0 || (D != 32 && D != 64) || pdrop < 0.f || pdrop >= 1.f)
+  if (Z <= 0 || H <= 0 || S <= 0 || b2_div <= 0 || (D != 32 && D != 64) || pdrop < 0.f || pdrop >= 1.f ||
+      (b2 != nullptr && b2_numel < 8))
     return (int)hipErrorInvalidValue;
   const uint32_t thresh = (uint32_t)fminf(4294967295.f, pdrop * 4294967296.f);
 #define DS_SMALL_ARGS(T)                                                                                           \
   SmallArgs<T> a{(const T*)q, (const T*)k, (const T*)v, (const T*)o, (const T*)dout, (T*)dq, (float*)lse,           \
                  (const T*)b1, (const T*)b2, (T*)dk, (T*)dv, delta, db1, db2, st[0], st[1], st[2], st[3], st[4], st[5], st[6],      \
                  st[7], st[8], st[9], st[10], st[11], st[12], st[13], st[14], st[15], st[16], st[17], b1_zs, Z, H, S, b2_div, scale, pdrop, \
-                 thresh, seed, vec_bias, 1, S};
+                 thresh, seed, b2_numel - 8, 1, db2_part, S};
   if (dtype == DS_BF16) {
     DS_SMALL_ARGS(bf16)
     return dispatch_small<bf16>(a, D, true, stream);

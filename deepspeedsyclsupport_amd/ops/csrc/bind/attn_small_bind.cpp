@@ -9,11 +9,12 @@
 
 extern "C" {
 int ds_flash_small_fwd(const void*, const void*, const void*, void*, float*, const void*, const void*,
-                       const int64_t*, int64_t, int, int, int, int, int, int, float, float, uint64_t, int, int,
+                       const int64_t*, int64_t, int, int, int, int, int, int, float, float, uint64_t, int64_t, int,
                        hipStream_t);
 int ds_flash_small_bwd(const void*, const void*, const void*, const void*, const void*, const float*, const void*,
-                       const void*, void*, void*, void*, float*, float*, float*, const int64_t*, int64_t, int, int, int, int,
-                       int, float, float, uint64_t, int, int, hipStream_t);
+                       const void*, void*, void*, void*, float*, float*, float*, float*, const int64_t*, int64_t, int, int, int,
+                       int, int, float, float, uint64_t, int64_t, int, hipStream_t);
+int ds_flash_small_db2_splits(int, int, int, int);
 }
 
 using torch::Tensor;
@@ -48,21 +49,19 @@ void operand(const Tensor& t, const Tensor& q, const char* name, bool any_s = fa
 struct Bias {
   const void* b1 = nullptr;
   const void* b2 = nullptr;
-  int64_t b1_zs = 0;
-  int vec = 1;
+  int64_t b1_zs = 0, b2_numel = 0;
+  Tensor padded;
 };
 
 Bias biases(const OptT& b1, const OptT& b2, const Tensor& q, int64_t Sk, int64_t b2_div) {
   const int64_t Z = q.size(0), S = q.size(1), H = q.size(2);
   Bias r;
-  r.vec = Sk % 8 == 0;  // bias rows are read in whole 16-B chunks of 8 keys
   if (b1.has_value() && b1->defined()) {
     TORCH_CHECK(b1->is_cuda() && b1->dim() == 2 && b1->size(0) == Z && b1->size(1) == Sk && b1->stride(1) == 1,
                 "flash_small: bias1 must be [Z, Sk] with a unit last stride");
     TORCH_CHECK(b1->scalar_type() == q.scalar_type(), "flash_small: bias1 dtype mismatch");
     r.b1 = b1->data_ptr();
     r.b1_zs = b1->stride(0);
-    r.vec &= aligned(r.b1, 16) && r.b1_zs % 8 == 0;
   }
   if (b2.has_value() && b2->defined()) {
     TORCH_CHECK(b2_div >= 1 && Z % b2_div == 0, "flash_small: b2_div must divide Z");
@@ -70,8 +69,9 @@ Bias biases(const OptT& b1, const OptT& b2, const Tensor& q, int64_t Sk, int64_t
                     b2->size(1) == H && b2->size(2) == S && b2->size(3) == Sk,
                 "flash_small: bias2 must be contiguous [Z / b2_div, H, S, Sk]");
     TORCH_CHECK(b2->scalar_type() == q.scalar_type(), "flash_small: bias2 dtype mismatch");
-    r.b2 = b2->data_ptr();
-    r.vec &= aligned(r.b2, 16);
+    r.padded = b2->numel() < 8 ? at::constant_pad_nd(b2->flatten(), {0, 8 - b2->numel()}) : *b2;  // (read in chunks of 8)
+    r.b2 = r.padded.data_ptr();
+    r.b2_numel = r.padded.numel();
   }
   return r;
 }
@@ -98,7 +98,7 @@ std::vector<Tensor> flash_small_fwd(Tensor q, Tensor k, Tensor v, OptT b1, OptT 
   push(st, q); push(st, k); push(st, v); push(st, o);
   check(ds_flash_small_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr<float>(), bs.b1,
                            bs.b2, st.data(), bs.b1_zs, (int)Z, (int)H, (int)S, (int)Sk, (int)D, (int)b2_div, (float)scale,
-                           (float)pdrop, (uint64_t)seed, bs.vec, dcode(q), at::hip::getCurrentHIPStream().stream()),
+                           (float)pdrop, (uint64_t)seed, bs.b2_numel, dcode(q), at::hip::getCurrentHIPStream().stream()),
         "flash_small_fwd");
   return {o, lse};
 }
@@ -126,14 +126,20 @@ std::vector<Tensor> flash_small_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, T
   auto dv = torch::empty({Z, S, H, D}, q.options());
   auto delta = torch::empty({Z, H, S}, f32);
   Tensor db1 = want_db1 ? torch::zeros({Z, S}, f32) : torch::empty({0}, f32);
-  Tensor db2 = want_db2 ? torch::zeros({Z / b2_div, H, S, S}, f32) : torch::empty({0}, f32);
+  Tensor db2 = torch::empty({want_db2 ? Z / b2_div : 0, H, S, S}, f32), part;
+  if (want_db2) {
+    const int splits = ds_flash_small_db2_splits((int)Z, (int)H, (int)S, (int)b2_div);
+    if (splits > 1) part = torch::empty({splits, db2.numel()}, f32);
+  } else {
+    db2 = torch::empty({0}, f32);
+  }
   std::vector<int64_t> st;
   push(st, q); push(st, k); push(st, v); push(st, o); push(st, dout); push(st, dq);
   check(ds_flash_small_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dout.data_ptr(),
                            lse.data_ptr<float>(), bs.b1, bs.b2, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
                            delta.data_ptr<float>(), want_db1 ? db1.data_ptr<float>() : nullptr,
-                           want_db2 ? db2.data_ptr<float>() : nullptr, st.data(), bs.b1_zs, (int)Z, (int)H, (int)S,
-                           (int)D, (int)b2_div, (float)scale, (float)pdrop, (uint64_t)seed, bs.vec, dcode(q),
+                           want_db2 ? db2.data_ptr<float>() : nullptr, part.defined() ? part.data_ptr<float>() : nullptr, st.data(), bs.b1_zs, (int)Z, (int)H, (int)S,
+                           (int)D, (int)b2_div, (float)scale, (float)pdrop, (uint64_t)seed, bs.b2_numel, dcode(q),
                            at::hip::getCurrentHIPStream().stream()),
         "flash_small_bwd");
   return {dq, dk, dv, db1, db2};

@@ -136,3 +136,29 @@ def test_cross_length_forward(D, Sk):
     assert _rel(out, FS.reference(q, k, v, b1)) < 2e-2
     with pytest.raises(NotImplementedError):
         FS.flash_small(q.requires_grad_(True), k, v)
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("Z,S,H,b2_div,p", [(1, 1, 3, 1, 0.0), (2, 3, 1, 2, 0.0), (3, 65, 2, 3, 0.0), (64, 129, 1, 64, 0.0),
+                                            (40, 71, 2, 20, 0.0), (24, 64, 2, 24, 0.3), (8, 250, 1, 2, 0.3)])
+def test_tile_edges_splits_and_unaligned_pair_biases(D, Z, S, H, b2_div, p):
+    """Sizes around the tiles, a pair bias at odd addresses whose last chunk ends with the tensor, one or several workgroups
+    adding up its gradient; masks of the type's lowest value: a query whose keys all have it attends to them alike."""
+    q, k, v, bias1, bias2 = _case(Z, S, H, D, torch.bfloat16, True, True, b2_div, seed=7)
+    bias1[0, 1:] = torch.finfo(torch.bfloat16).min
+    room = torch.empty(bias2.numel() + 1, device="cuda", dtype=torch.bfloat16)
+    odd = room[1:].view_as(bias2).copy_(bias2)
+    keep = FS.keep_mask(9, Z, H, S, p) if p else None
+    masked = torch.full_like(bias1, torch.finfo(torch.bfloat16).min)
+    assert _rel(FS.flash_small(q, k, v, masked), v.float().mean(1, keepdim=True).expand_as(v)) < 2e-2
+    ins = [t.detach().requires_grad_(True) for t in (q, k, v, bias1, odd)]
+    refs = [t.detach().float().clone().requires_grad_(True) for t in (q, k, v, bias1, bias2)]
+    out = FS.flash_small(*ins, b2_div=b2_div, dropout_p=p, seed=9)
+    ref = FS.reference(*refs, b2_div=b2_div, **(dict(keep=keep, p=p) if p else {}))
+    assert _rel(out, ref) < 2e-2
+    go = torch.randn_like(ref)
+    out.backward(go.bfloat16())
+    ref.backward(go)
+    # sums over keys, queries and the b2_div sharers of bf16-rounded factors: as in the tests above
+    for name, a, r in zip(("dq", "dk", "dv", "db1", "db2"), ins, refs):
+        assert (a.grad.float() - r.grad).abs().max() < 4e-2 * r.grad.abs().max() + 4e-2, name
