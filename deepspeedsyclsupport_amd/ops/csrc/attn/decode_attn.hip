@@ -5,13 +5,20 @@
 // blocked KV cache (`inference/v2/kernels/ragged_ops/blocked_flash`). One kernel serves both engines: a contiguous
 // per-sequence cache is the special case "one block of max_len tokens per sequence".
 //
-// Decode is HBM-bound (every cached K and V byte is read once per token), so the design is flash-decoding:
+// Every cached K and V byte is read once per token, but a step's caches are a few MB: what bounds it is the chain of latencies.
 //  * grid = (batch, kv_head, split): each workgroup reads ONE kv head's K/V for a contiguous slice of the sequence
 //    once and serves all G = Hq/Hk query heads of that GQA group from it (no K/V re-read per query head);
-//  * the sequence is split so the launch has >= ~2 workgroups per CU even at batch 1 (256 CUs);
-//  * scores for the slice live in LDS; softmax runs on LDS; P·V streams V rows with 16-B loads, 16 lanes per row;
-//  * partial (max, sum, unnormalised acc) per split are merged by a small combine kernel (log-sum-exp). (An in-kernel
-//    last-block merge was measured 2x slower: the device-scope fences it needs write back L2.)
+//  * eight waves take alternating groups of 16 keys, each with its own running maxima, sums and accumulators, and meet once, at
+//    the end. Scores are one MFMA tile, K . Q^T with the group's heads as columns (bf16 products, fp32 sums: what the vector
+//    units gave, at a fraction of their instructions); P . V stays on the vector units, with P in fp32: V rows are read
+//    whole, LPR lanes a row, and a row's probabilities reach its lanes through LDS. K and V of a group are loaded together
+//    (held a group ahead they cost the second workgroup of a CU, and time: 48 x 190 keys 16 us for 12);
+//  * a sequence is split only when that is long for one workgroup (see `ds_paged_decode_splits`): partial (max, sum,
+//    unnormalised acc) per split are merged by a small combine kernel (log-sum-exp). (An in-kernel last-block merge was
+//    measured 2x slower: the device-scope fences it needs write back L2.)
+// Measured, us (a workgroup of four waves per 64 to 1024 keys, scores and softmax in LDS between barriers; the read at 6.5 TB/s), 8
+// kv heads of 128: 1 sequence of 130 keys, 4 heads each 6 (14; 0.1), 1 of 8192 19 (44; 5), 12 of 700, 2 heads each 11 (20; 5),
+// 48 of 190, 4 each 12 (24; 6), 48 of 1024 42 (74; 31), 256 of 512 96 (183; 83).
 // Optional ALiBi slopes (BLOOM) are applied on the fly. With a sliding window (Mistral) or chunked visibility only the
 // keys in sight are split and read. A second instantiation takes key and value widths of their own (multiples of 8), a
 // tanh score cap, a softmax sink per head, a gate per token and head, and GQA groups of any size.
@@ -19,190 +26,208 @@
 
 namespace {
 
-constexpr int THREADS = 256;
+constexpr int WAVES = 8, THREADS = 64 * WAVES;
 constexpr int MAXG = 8;          // query heads per kv head handled per workgroup (GQA group)
-constexpr int MAX_CHUNK = 1024;  // keys per split (LDS: MAXG * MAX_CHUNK * 4 B = 32 KiB)
+constexpr int KEYS = 16;         // keys a wave takes at once
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
 // lanes per row of D elements, 8 each: D / 8 rounded up to a power of two
 constexpr int lanes_per_row(int d) { return d <= 64 ? 8 : (d <= 128 ? 16 : 32); }
 
-// DK, DV: the widths; 0: given at run time (dk, dv), LK / LV lanes per row
-template <int DK, int DV, int LK = lanes_per_row(DK), int LV = lanes_per_row(DV)>
-__global__ void __launch_bounds__(THREADS) paged_decode_kernel(
-    const bf16* __restrict__ q,          // [B, Hq, dk]
-    const bf16* __restrict__ kc,         // [NB, Hk, BS, dk]
-    const bf16* __restrict__ vc,         // [NB, Hk, BS, dv]
-    const int* __restrict__ block_table, // [B, max_blocks]
-    const int* __restrict__ seq_lens,    // [B]
-    const float* __restrict__ alibi,     // [Hq] or null
-    float* __restrict__ part_acc,        // [B, Hq, S, dv]  (only if S > 1)
-    float* __restrict__ part_ml,         // [B, Hq, S, 2]
-    bf16* __restrict__ out,              // [B, Hq, dv], rows ldo apart (written directly when S == 1)
-    const float* __restrict__ sink, const bf16* __restrict__ gate, int64_t ldg, int64_t ldo, int Hq, int Hk, int BS, int max_blocks, int chunk, float scale, int window, int mask_chunk, float softcap, int dk_rt,
-    int dv_rt) {
+struct DecodeArgs {
+  const bf16* q;           // [B, Hq, dk]
+  const bf16* kc;          // [NB, Hk, BS, dk]
+  const bf16* vc;          // [NB, Hk, BS, dv]
+  const int* block_table;  // [B, max_blocks]
+  const int* seq_lens;     // [B]
+  const float* alibi;      // [Hq] or null
+  float* part_acc;         // [B, Hq, S, dv]  (only if S > 1)
+  float* part_ml;          // [B, Hq, S, 2]
+  bf16* out;               // [B, Hq, dv], rows ldo apart (written directly when S == 1)
+  const float* sink;
+  const bf16* gate;
+  int64_t ldg, ldo;
+  int Hq, Hk, BS, bs_shift, max_blocks, chunk, window, mask_chunk, dk, dv;  // bs_shift: log2 BS, or -1
+  float scale, softcap;
+};
+
+// DK, DV: the widths; 0: given at run time, of which LPR lanes hold a row. GT: at least the query heads served.
+template <int DK, int DV, int GT, int LPR = lanes_per_row(DK)>
+__global__ void __launch_bounds__(THREADS, 2) paged_decode_kernel(DecodeArgs a) {
   constexpr bool EXT = DK == 0;
   static_assert(EXT || (DK % 16 == 0 && DK >= 64 && DK <= 256 && DK == DV), "head dim");
-  const int dk = EXT ? dk_rt : DK, dv = EXT ? dv_rt : DV;
-  extern __shared__ __attribute__((aligned(16))) float sm[];  // scores [G][chunk] + reduction scratch
-  const int b = blockIdx.x, kh = EXT ? blockIdx.y % Hk : blockIdx.y, split = blockIdx.z, S = gridDim.z;
-  const int g0 = EXT ? blockIdx.y / Hk * MAXG : 0;              // first query head of the group this block serves
-  const int GA = Hq / Hk, G = EXT ? min(MAXG, GA - g0) : GA, h0 = kh * GA + g0;
-  const int T = seq_lens[b];
-  int tlo = window > 0 ? max(0, T - window) : 0;                // first key in sight
-  if (mask_chunk > 0) tlo = max(tlo, (T - 1) / mask_chunk * mask_chunk);
-  const int t0 = tlo + split * chunk;
-  const int t1 = min(T, t0 + chunk);
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  float* scores = sm;                       // [G][chunk]
-  float* red = sm + MAXG * MAX_CHUNK;       // [THREADS/64 * MAXG * 2]
+  const int dk = EXT ? a.dk : DK, dv = EXT ? a.dv : DV;
+  // [WAVES][GT][dv] accumulators, [WAVES][GT][2] maxima and sums, [WAVES][KEYS + 1][GT] probabilities and the fade of what was
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  const int b = blockIdx.x, kh = EXT ? blockIdx.y % a.Hk : blockIdx.y, split = blockIdx.z, S = gridDim.z;
+  const int g0 = EXT ? blockIdx.y / a.Hk * MAXG : 0;          // first query head of the group this block serves
+  const int GA = a.Hq / a.Hk, G = EXT ? min(MAXG, GA - g0) : GA, h0 = kh * GA + g0;
+  const int T = a.seq_lens[b];
+  int tlo = a.window > 0 ? max(0, T - a.window) : 0;          // first key in sight
+  if (a.mask_chunk > 0) tlo = max(tlo, (T - 1) / a.mask_chunk * a.mask_chunk);
+  const int t0 = tlo + split * a.chunk, t1 = min(T, t0 + a.chunk);
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  // ---- q of the G heads of this GQA group; LPR lanes cover one row, 8 elements each. LPR is D/8 rounded up to a
-  // power of two (head dims 80 and 96 use 16 lanes per row): the surplus lanes carry a zero query, re-read the row's
-  // last chunk (a cache hit) and never write
-  const int CPR = dk / 8;                                      // 16-byte chunks per row
-  constexpr int LPR = LK;                                      // lanes per key row (16 for D=128)
-  constexpr int RPW = 64 / LPR;                                // rows per wave instruction
-  const int sub = lane / LPR, li_raw = lane % LPR, li = li_raw < CPR ? li_raw : CPR - 1;
-  const float lane_on = li_raw < CPR ? 1.f : 0.f;
-  float qv[MAXG][8];
-  // unconditional loads (clamped head index): a guarded load would make the compiler wait on each one in turn
+  // scores: lane (l16, q4) brings key l16 and holds those of head l16 with keys 4 q4 .. + 3; chunk 4 kk + q4 of 8 elements goes
+  // into MFMA kk (surplus chunks: a zero query, the row's last chunk again)
+  constexpr int KK = (LPR + 3) / 4;
+  const int l16 = lane & 15, q4 = lane >> 4;
+  bf16x8_t qf[KK];
+  const bool mine = l16 < G;
 #pragma unroll
-  for (int g = 0; g < MAXG; ++g) {
-    const int gc = g < G ? g : G - 1;
-    Vec8<bf16>::load(q + ((int64_t)b * Hq + h0 + gc) * dk + li * 8, qv[g]);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) qv[g][j] *= scale * lane_on;
+  for (int kk = 0; kk < KK; ++kk) {
+    const int c = 4 * kk + q4;
+    qf[kk] = *reinterpret_cast<const bf16x8_t*>(a.q + ((int64_t)b * a.Hq + h0 + min(l16, G - 1)) * dk + min(c, dk / 8 - 1) * 8);
+    if (c >= dk / 8 || !mine) qf[kk] = bf16x8_t{};
   }
-  // ---- phase 1: scores for keys of this split (UNR key rows per lane-group in flight per iteration)
-  constexpr int UNR = 4;
-  const int* bt = block_table + (int64_t)b * max_blocks;
-  const int kstride = (THREADS / 64) * RPW;
-  for (int tb = t0 + wid * RPW + sub; tb < t1; tb += kstride * UNR) {
-    float kv[UNR][8];
-    int blk[UNR];
+  const float slope = !EXT && a.alibi && mine ? a.alibi[h0 + l16] : 0.f;
+  // values: LPR lanes cover one row, 8 elements each
+  constexpr int RPW = 64 / LPR, UV = KEYS / RPW;              // rows per wave instruction, instructions
+  const int sub = lane / LPR, li = lane % LPR, lv = min(li, dv / 8 - 1);
+  float acc[GT][8], m = -INFINITY, l = 0.f;                   // m, l: of head l16
 #pragma unroll
-    for (int u = 0; u < UNR; ++u) blk[u] = bt[min(tb + u * kstride, t1 - 1) / BS];  // clamped: always valid
-#pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      const int tc = min(tb + u * kstride, t1 - 1);
-      Vec8<bf16>::load(kc + (((int64_t)blk[u] * Hk + kh) * BS + tc % BS) * dk + li * 8, kv[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      const int t = tb + u * kstride;
-      if (t >= t1) continue;  // uniform across the LPR lanes of one key row (the shuffle partners)
-#pragma unroll
-      for (int g = 0; g < MAXG; ++g) {
-        if (g < G) {
-          float s = 0.f;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) s = fmaf(qv[g][j], kv[u][j], s);
-#pragma unroll
-          for (int o = LPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-          if (li_raw == 0) {
-            if (alibi) s += alibi[h0 + g] * (float)(t - (T - 1));
-            if (EXT && softcap > 0.f) s = softcap * tanhf(s / softcap);
-            scores[g * MAX_CHUNK + (t - t0)] = s;
-          }
-        }
-      }
-    }
-  }
-  // V rows do not depend on the scores: start the first P.V pass's loads before the softmax phases
-  constexpr int ROWS = THREADS / LV;
-  const int CPV = dv / 8, r = tid / LV, c_raw = tid % LV, c = c_raw < CPV ? c_raw : CPV - 1;
-  float vpre[8];
-  if (t0 + r < t1) {
-    const int blk = bt[(t0 + r) / BS], off = (t0 + r) % BS;
-    Vec8<bf16>::load(vc + (((int64_t)blk * Hk + kh) * BS + off) * dv + c * 8, vpre);
-  }
-  __syncthreads();
-  // ---- phase 2: per-head max and sum over the split (one wave per head group, strided)
-  const int n = t1 - t0;
-  for (int g = wid; g < G; g += THREADS / 64) {
-    float m = -INFINITY;
-    for (int i = lane; i < n; i += 64) m = fmaxf(m, scores[g * MAX_CHUNK + i]);
-    m = wave_max(m);
-    float l = 0.f;
-    for (int i = lane; i < n; i += 64) {
-      const float p = (m == -INFINITY) ? 0.f : __expf(scores[g * MAX_CHUNK + i] - m);
-      scores[g * MAX_CHUNK + i] = p;
-      l += p;
-    }
-    l = wave_sum(l);
-    if (lane == 0) {
-      red[g * 2] = m;
-      red[g * 2 + 1] = l;
-    }
-  }
-  __syncthreads();
-  // ---- phase 3: acc[g][d] = sum_t p[g][t] * v[t][d]; LPR lanes per V row, THREADS/LPR rows in flight
-  float acc[MAXG][8];
-#pragma unroll
-  for (int g = 0; g < MAXG; ++g)
+  for (int g = 0; g < GT; ++g)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
-  for (int tb = t0 + r; tb < t1; tb += ROWS * UNR) {
-    float vv[UNR][8];
-    int vblk[UNR];
+  float* ml = sm + WAVES * GT * dv;
+  float* pw = ml + WAVES * GT * 2 + wid * (KEYS + 1) * GT;
+
+  constexpr int STEP = WAVES * KEYS;
+  const int* bt = a.block_table + (int64_t)b * a.max_blocks;
+  struct Group {
+    bf16x8_t k[KK], v[UV];
+  };
+  struct Blocks {
+    int k, v[UV];
+  };
+  // (keys past the end read the last one again)
+  auto blocks = [&](int t, Blocks& blk) {
+    auto of = [&](int key) {
+      const int tc = min(key, t1 - 1);
+      return bt[a.bs_shift >= 0 ? tc >> a.bs_shift : tc / a.BS];
+    };
+    blk.k = of(t + l16);
 #pragma unroll
-    for (int u = 0; u < UNR; ++u) vblk[u] = bt[min(tb + u * ROWS, t1 - 1) / BS];
+    for (int u = 0; u < UV; ++u) blk.v[u] = of(t + u * RPW + sub);
+  };
+  auto load = [&](int t, const Blocks& blk, Group& f) {
+    auto row = [&](int key, int block) {
+      const int tc = min(key, t1 - 1), off = a.bs_shift >= 0 ? tc & (a.BS - 1) : tc % a.BS;
+      return ((int64_t)block * a.Hk + kh) * a.BS + off;
+    };
+    const bf16* kr = a.kc + row(t + l16, blk.k) * dk;
 #pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      const int tc = min(tb + u * ROWS, t1 - 1);
-      if (u == 0 && tb == t0 + r) {
+    for (int kk = 0; kk < KK; ++kk) f.k[kk] = *reinterpret_cast<const bf16x8_t*>(kr + min(4 * kk + q4, dk / 8 - 1) * 8);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) vv[u][j] = vpre[j];
-      } else {
-        Vec8<bf16>::load(vc + (((int64_t)vblk[u] * Hk + kh) * BS + tc % BS) * dv + c * 8, vv[u]);
-      }
+    for (int u = 0; u < UV; ++u) f.v[u] = *reinterpret_cast<const bf16x8_t*>(a.vc + row(t + u * RPW + sub, blk.v[u]) * dv + lv * 8);
+  };
+  auto attend = [&](int t, const Group& f) {
+    f32x4 s{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.k[kk], qf[kk], s, 0, 0, 0);
+    float mx = m;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int key = t + 4 * q4 + i;
+      float x = s[i] * a.scale;
+      if (!EXT && a.alibi) x += slope * (float)(key - (T - 1));
+      if (EXT && a.softcap > 0.f) x = a.softcap * tanhf(x / a.softcap);
+      s[i] = key < t1 ? x : -INFINITY;
+      mx = fmaxf(mx, s[i]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float ref = mx == -INFINITY ? 0.f : mx, fade = __expf(m - ref);
+    m = mx;
+    l *= fade;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float p = __expf(s[i] - ref);
+      l += p;
+      if (l16 < GT) pw[(4 * q4 + i) * GT + l16] = p;
+    }
+    if (lane < GT) pw[KEYS * GT + lane] = fade;
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int g = 0; g < GT; ++g) {
+      const float w = pw[KEYS * GT + g];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[g][j] *= w;
     }
 #pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      const int t = tb + u * ROWS;
-      if (t >= t1) continue;
+    for (int u = 0; u < UV; ++u) {
+      if (t + u * RPW + sub >= t1) continue;
+      float p[GT];
 #pragma unroll
-      for (int g = 0; g < MAXG; ++g) {
-        if (g < G) {
-          const float p = scores[g * MAX_CHUNK + (t - t0)];
+      for (int g = 0; g < GT; ++g) p[g] = pw[(u * RPW + sub) * GT + g];
 #pragma unroll
-          for (int j = 0; j < 8; ++j) acc[g][j] = fmaf(p, vv[u][j], acc[g][j]);
-        }
-      }
+      for (int g = 0; g < GT; ++g)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[g][j] = fmaf(p[g], (float)f.v[u][j], acc[g][j]);
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  int t = t0 + wid * KEYS;
+  if (t < t1) {
+    Group f;
+    Blocks blk;
+    blocks(t, blk);
+    for (; t < t1; t += STEP) {
+      load(t, blk, f);
+      blocks(t + STEP, blk);
+      __builtin_amdgcn_sched_barrier(0);
+      attend(t, f);
     }
   }
-  __syncthreads();  // scores are dead: reuse their LDS as a [ROWS][D] buffer, one query head at a time
-  float* rb = sm;
+  // ---- the lane groups of a wave meet in registers (they share their maxima), the waves in LDS
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (lane < GT) {
+    ml[(wid * GT + lane) * 2] = m;
+    ml[(wid * GT + lane) * 2 + 1] = l;
+  }
 #pragma unroll
-  for (int g = 0; g < MAXG; ++g) {
-    if (g >= G) break;  // block-uniform
-    if (c_raw < CPV) {
+  for (int g = 0; g < GT; ++g) {
+    if (g >= G) break;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) rb[r * dv + c * 8 + j] = acc[g][j];
+    for (int o = LPR; o < 64; o *= 2)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[g][j] += __shfl_xor(acc[g][j], o, 64);
+    if (sub == 0 && li < dv / 8) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sm[(wid * GT + g) * dv + li * 8 + j] = acc[g][j];
     }
-    __syncthreads();
-    for (int idx = tid; idx < dv; idx += THREADS) {
-      float s = 0.f;
-      for (int rr = 0; rr < ROWS; ++rr) s += rb[rr * dv + idx];
-      const int hq = h0 + g;
-      const float m = red[g * 2], l = red[g * 2 + 1];
-      if (S == 1) {
-        float r = l > 0.f ? s / l : 0.f;
-        if (EXT && sink) {  // in the frame of the larger of the two
-          const float mn = fmaxf(m, sink[hq]), f = __expf(m - mn);
-          r = s * f / fmaf(l, f, __expf(sink[hq] - mn));
-        }
-        if (EXT && gate) r /= 1.f + __expf(-(float)gate[b * ldg + hq]);
-        out[(int64_t)b * ldo + hq * dv + idx] = (bf16)r;
-      } else {
-        part_acc[(((int64_t)b * Hq + hq) * S + split) * dv + idx] = s;
-        if (idx == 0) {
-          part_ml[(((int64_t)b * Hq + hq) * S + split) * 2] = m;
-          part_ml[(((int64_t)b * Hq + hq) * S + split) * 2 + 1] = l;
-        }
+  }
+  __syncthreads();
+  for (int i = tid; i < G * dv; i += THREADS) {
+    const int g = i / dv, d = i % dv, hq = h0 + g;
+    float mx = -INFINITY, num = 0.f, den = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) mx = fmaxf(mx, ml[(w * GT + g) * 2]);
+    const float ref = mx == -INFINITY ? 0.f : mx;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float f = __expf(ml[(w * GT + g) * 2] - ref);
+      num = fmaf(f, sm[(w * GT + g) * dv + d], num);
+      den = fmaf(f, ml[(w * GT + g) * 2 + 1], den);
+    }
+    if (S == 1) {
+      float r = den > 0.f ? num / den : 0.f;
+      if (EXT && a.sink) {  // in the frame of the larger of the two
+        const float mn = fmaxf(mx, a.sink[hq]), f = __expf(mx - mn);
+        r = num * f / fmaf(den, f, __expf(a.sink[hq] - mn));
+      }
+      if (EXT && a.gate) r /= 1.f + __expf(-(float)a.gate[b * a.ldg + hq]);
+      a.out[(int64_t)b * a.ldo + hq * dv + d] = (bf16)r;
+    } else {
+      const int64_t at = ((int64_t)b * a.Hq + hq) * S + split;
+      a.part_acc[at * dv + d] = num;
+      if (d == 0) {
+        a.part_ml[at * 2] = mx;
+        a.part_ml[at * 2 + 1] = den;
       }
     }
-    __syncthreads();
   }
 }
 
@@ -322,45 +347,71 @@ __global__ void __launch_bounds__(256) qkv_rope_append_kernel(
 
 }  // namespace
 
+// How many workgroups share a sequence: one up to 768 keys (the combine pass costs more than it saves: 12 x 8 heads x 700 keys 11.0
+// us whole, 12.1 in two; 1 x 8 x 512 9.7 and, in four, 9.1), then as many as fill the chip with one each, of at least 256 keys, 512
+// for long ones (1 x 8 x 1024: 15.0 whole, 10.4 in four; 12 x 8 x 2048: 27.9, 23.2 in two, 25.5 in four; 1 x 8 x 8192: 89, 19.2 in
+// sixteen, 24 in thirty-two).
 extern "C" int ds_paged_decode_splits(int B, int Hk, int max_len) {
-  // enough workgroups to cover the chip ~2x, splits of >= 64 keys, <= MAX_CHUNK keys per split
-  const int want = (512 + B * Hk - 1) / (B * Hk);
-  int chunk = (max_len + want - 1) / want;
-  chunk = ((chunk + 63) / 64) * 64;
-  if (chunk < 64) chunk = 64;
-  if (chunk > MAX_CHUNK) chunk = MAX_CHUNK;
+  const int64_t own = (int64_t)B * Hk;
+  int chunk = max_len;
+  if (max_len > 768) {
+    const int want = (int)(own < 256 ? 256 / own : 1), least = max_len > 4096 ? 512 : 256;
+    chunk = (max_len + want - 1) / want;
+    chunk = ((chunk < least ? least : chunk) + 63) / 64 * 64;
+  }
   return (max_len + chunk - 1) / chunk;
 }
+
+namespace {
+
+template <int DK, int DV, int LPR, int GT>
+int launch_decode(const DecodeArgs& a, dim3 grid, hipStream_t s) {
+  const int dv = DK ? DV : a.dv;
+  const int lds = WAVES * GT * (dv + 2 + KEYS + 1) * (int)sizeof(float);
+  auto* kernel = &paged_decode_kernel<DK, DV, GT, LPR>;
+  if (lds > 65536 &&
+      hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(kernel, grid, dim3(THREADS), lds, s, a);
+  DS_CHECK_LAUNCH();
+  if (grid.z > 1) {
+    hipLaunchKernelGGL(combine_kernel, dim3((unsigned)grid.x * a.Hq), dim3(dv), 0, s, a.part_acc, a.part_ml, a.out, a.sink, a.gate,
+                       a.ldg, a.Hq, a.ldo, (int)grid.z);
+    DS_CHECK_LAUNCH();
+  }
+  return 0;
+}
+
+// by the query heads a workgroup serves
+template <int DK, int DV, int LPR>
+int launch_decode(const DecodeArgs& a, dim3 grid, hipStream_t s) {
+  const int G = a.Hq / a.Hk;
+  if (G <= 1) return launch_decode<DK, DV, LPR, 1>(a, grid, s);
+  if (G <= 2) return launch_decode<DK, DV, LPR, 2>(a, grid, s);
+  if (G <= 4) return launch_decode<DK, DV, LPR, 4>(a, grid, s);
+  return launch_decode<DK, DV, LPR, MAXG>(a, grid, s);
+}
+
+int log2_of(int n) { return n > 0 && (n & (n - 1)) == 0 ? __builtin_ctz(n) : -1; }
+
+}  // namespace
 
 extern "C" int ds_paged_decode(const void* q, const void* kc, const void* vc, const int* block_table,
                                const int* seq_lens, const float* alibi, float* part_acc, float* part_ml, void* out,
                                int B, int Hq, int Hk, int D, int BS, int max_blocks, int max_len, int splits,
                                float scale, int window, hipStream_t s) {
-  if (Hq % Hk || Hq / Hk > MAXG) return (int)hipErrorInvalidValue;
+  if (Hk <= 0 || Hq % Hk || Hq / Hk > MAXG || splits <= 0) return (int)hipErrorInvalidValue;
   if (window > 0 && window < max_len) max_len = window;  // no more keys than that are in sight
   const int chunk = ((max_len + splits - 1) / splits + 63) / 64 * 64;
-  if (chunk > MAX_CHUNK) return (int)hipErrorInvalidValue;
-  const size_t lds = (size_t)(MAXG * MAX_CHUNK + 64) * sizeof(float);
-  dim3 grid(B, Hk, splits);
-#define LAUNCH(DD)                                                                                                  \
-  hipLaunchKernelGGL((paged_decode_kernel<DD, DD>), grid, dim3(THREADS), lds, s, (const bf16*)q, (const bf16*)kc,       \
-                     (const bf16*)vc, block_table, seq_lens, alibi, part_acc, part_ml, (bf16*)out, nullptr,          \
-                     nullptr, 0, (int64_t)Hq * DD, Hq, Hk, BS,                                                                   \
-                     max_blocks, chunk, scale, window, 0, 0.f, DD, DD);                                             \
-  DS_CHECK_LAUNCH();                                                                                                \
-  if (splits > 1) {                                                                                                 \
-    hipLaunchKernelGGL(combine_kernel, dim3(B * Hq), dim3(DD), 0, s, part_acc, part_ml, (bf16*)out, nullptr, nullptr, 0, Hq, \
-                       (int64_t)Hq * DD, splits);                                                                     \
-    DS_CHECK_LAUNCH();                                                                                              \
-  }
-  if (D == 64) { LAUNCH(64) }
-  else if (D == 80) { LAUNCH(80) }
-  else if (D == 96) { LAUNCH(96) }
-  else if (D == 128) { LAUNCH(128) }
-  else if (D == 256) { LAUNCH(256) }
-  else return (int)hipErrorInvalidValue;
-#undef LAUNCH
-  return 0;
+  const DecodeArgs a{(const bf16*)q, (const bf16*)kc, (const bf16*)vc, block_table, seq_lens, alibi, part_acc, part_ml, (bf16*)out,
+                     nullptr, nullptr, 0, (int64_t)Hq * D, Hq, Hk, BS, log2_of(BS), max_blocks, chunk, window, 0, D, D, scale, 0.f};
+  const dim3 grid(B, Hk, splits);
+  if (D == 64) return launch_decode<64, 64, 8>(a, grid, s);
+  if (D == 80) return launch_decode<80, 80, 16>(a, grid, s);
+  if (D == 96) return launch_decode<96, 96, 16>(a, grid, s);
+  if (D == 128) return launch_decode<128, 128, 16>(a, grid, s);
+  if (D == 256) return launch_decode<256, 256, 32>(a, grid, s);
+  return (int)hipErrorInvalidValue;
 }
 
 // Key / value widths of their own (multiples of 8 up to 256), chunked and / or windowed visibility, score cap, softmax sink
@@ -375,32 +426,14 @@ extern "C" int ds_paged_decode_ext(const void* q, const void* kc, const void* vc
       ldo < (int64_t)Hq * dv)
     return (int)hipErrorInvalidValue;
   const int chunk = ((span + splits - 1) / splits + 63) / 64 * 64;
-  if (chunk > MAX_CHUNK) return (int)hipErrorInvalidValue;
-  // scores [MAXG][MAX_CHUNK] + maxima / sums; the value reduction reuses it ([256 / lanes per row][dv] floats)
-  const size_t lds = (size_t)(MAXG * MAX_CHUNK + 64) * sizeof(float);
-  dim3 grid(B, Hk * ((Hq / Hk + MAXG - 1) / MAXG), splits);
-#define GO(LK, LV)                                                                                                  \
-  hipLaunchKernelGGL((paged_decode_kernel<0, 0, LK, LV>), grid, dim3(THREADS), lds, s, (const bf16*)q, (const bf16*)kc, \
-                     (const bf16*)vc, block_table, seq_lens, nullptr, part_acc, part_ml, (bf16*)out, sink, (const bf16*)gate, ldg, ldo, Hq, Hk, BS, \
-                     max_blocks, chunk, scale, window, mask_chunk, softcap, dk, dv)
-#define ROW(LK)                 \
-  {                             \
-    if (dv <= 64) GO(LK, 8);    \
-    else if (dv <= 128) GO(LK, 16); \
-    else GO(LK, 32);            \
-  }
-  if (dk <= 64) ROW(8)
-  else if (dk <= 128) ROW(16)
-  else ROW(32)
-#undef ROW
-#undef GO
-  DS_CHECK_LAUNCH();
-  if (splits > 1) {
-    hipLaunchKernelGGL(combine_kernel, dim3(B * Hq), dim3(dv), 0, s, part_acc, part_ml, (bf16*)out, sink,
-                       (const bf16*)gate, ldg, Hq, ldo, splits);
-    DS_CHECK_LAUNCH();
-  }
-  return 0;
+  const DecodeArgs a{(const bf16*)q, (const bf16*)kc, (const bf16*)vc, block_table, seq_lens, nullptr, part_acc, part_ml, (bf16*)out,
+                     sink, (const bf16*)gate, ldg, ldo, Hq, Hk, BS, log2_of(BS), max_blocks, chunk, window, mask_chunk, dk, dv, scale,
+                     softcap};
+  const dim3 grid(B, Hk * ((Hq / Hk + MAXG - 1) / MAXG), splits);
+  const int wide = dk > dv ? dk : dv;
+  if (wide <= 64) return launch_decode<0, 0, 8>(a, grid, s);
+  if (wide <= 128) return launch_decode<0, 0, 16>(a, grid, s);
+  return launch_decode<0, 0, 32>(a, grid, s);
 }
 
 extern "C" int ds_kv_append(const void* k, const void* v, void* kc, void* vc, const int* block_table,

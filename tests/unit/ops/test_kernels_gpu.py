@@ -327,6 +327,24 @@ def test_paged_decode_alibi_window_and_capacity():
     torch.testing.assert_close(out.float(), ref, rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("hq,hk", [(3, 3), (10, 5), (9, 3), (16, 2)])
+@pytest.mark.parametrize("D,BS,window", [(64, 24, 0), (128, 16, 100), (96, 64, 0)])
+def test_paged_decode_edges_of_key_groups(hq, hk, D, BS, window):
+    """Contexts around a wave's group, a workgroup's round and the length from which a sequence is split, one to eight heads a
+    group, a block size that is no power of two. Probabilities stay in fp32: against fp64 the result is off by its own
+    rounding (2^-9) and that of the fp32 sums (a few hundred terms of at most 5, 2^-24 each)."""
+    lens = [1, 15, 16, 17, 127, 128, 129, 768, 769, 1030]
+    kc, vc, bt, maxb = _paged_setup(len(lens), hk, D, BS, lens, seed=5)
+    q = torch.randn(len(lens), hq, D, device="cuda").bfloat16()
+    sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    room = torch.full((len(lens) + 1, hq, D), 7.0, device="cuda", dtype=torch.bfloat16)
+    for max_len in (max(lens), maxb * BS):
+        out = ops().paged_decode(q, kc, vc, bt, sl, max_len, D**-0.5, None, window, room[:-1])
+        ref = _paged_ref(q.double(), kc.double(), vc.double(), bt, lens, D**-0.5, None, window)
+        assert ((out.double() - ref).abs() <= 2.0**-8 * ref.abs() + 2e-4).all()
+        assert torch.equal(out, room[:-1]) and (room[-1] == 7).all()
+
+
 def test_kv_append():
     B, n, hk, D, BS = 3, 5, 4, 128, 16
     kc, vc, bt, maxb = _paged_setup(B, hk, D, BS, [64, 64, 64])
