@@ -426,6 +426,8 @@ class DSInferenceLayer(ProjectionLayer):
                                                                              qkv.dtype == torch.bfloat16)) \
             and kc.dtype == torch.bfloat16 and (not meta.prefill_from_zero or alibi is not None or bool(window)
                                                 or D != 128)
+        if n == 1 and pending is None and self._step_ok(qkv, kc):
+            return self._decode_step(qkv, meta, kc, vc, rope, alibi, scale, window).view(B, n, self.hq * D)
         if pending is not None or (qkv.is_cuda and qkv.dtype == torch.bfloat16 and kc.dtype == torch.bfloat16):
             # one fused HIP epilogue: split + RoPE(q, k) + scatter k/v into the paged cache (and, for a pending
             # weight-only GEMV, its finalize pass: the sums are read straight from the split-K workspace)
@@ -462,6 +464,22 @@ class DSInferenceLayer(ProjectionLayer):
             o = _cached_attention(q, kc, vc, meta, scale, alibi, window)
         return o.reshape(B, n, self.hq * D)
 
+    def _step_ok(self, qkv, kc):
+        """Whether a step of one token a sequence may take its rotation and cache append into the attention kernel."""
+        spec = self.spec
+        rot = spec.rotary_dim if spec.pos in ("rope", "rope_gptj") else 0
+        return qkv.is_cuda and qkv.dtype == torch.bfloat16 and kc.dtype == torch.bfloat16 and rot % 16 == 0 and \
+            spec.head_dim in PAGED_HEAD_DIMS
+
+    def _decode_step(self, qkv, meta, kc, vc, rope, alibi, scale, window):
+        """qkv of one token a sequence -> its attention [B, Hq, D], in one kernel (`csrc/attn/decode_attn.hip`)."""
+        from ...ops.native import hip_ops
+        spec = self.spec
+        rot = spec.rotary_dim if spec.pos in ("rope", "rope_gptj") else 0
+        return hip_ops().paged_decode_step(qkv.contiguous(), rope[0] if rot else None, rope[1] if rot else None, meta.pos_ids, kc,
+                                           vc, meta.block_tables, meta.seq_lens, meta.max_len, scale, alibi, window, self.hq, rot,
+                                           spec.pos == "rope_gptj")
+
     def _attend_ragged(self, qkv, meta: "RaggedMeta", cache, rope, alibi):
         """Ragged batch: qkv [1, T, (Hq+2Hk)*D] -> [1, T, Hq*D]. One fused epilogue (RoPE + paged-cache append) for
         all tokens, then the paged decode kernel for the leading single-token sequences and the ragged paged
@@ -474,6 +492,10 @@ class DSInferenceLayer(ProjectionLayer):
         pending = qkv if hasattr(qkv, "finalize_rms") else None
         if pending is not None and not (pending.acc.is_cuda and kc.dtype == torch.bfloat16):
             qkv, pending = pending.finalize(), None
+        scale = spec.attn_scale or 1.0 / math.sqrt(D)
+        window = spec.layer_windows[self.layer_idx] if spec.layer_windows else spec.sliding_window
+        if meta.n_decode == T and pending is None and self._step_ok(qkv, kc):
+            return self._decode_step(qkv, meta, kc, vc, rope, alibi, scale, window).view(1, T, self.hq * D)
         if pending is not None or (qkv.is_cuda and qkv.dtype == torch.bfloat16 and kc.dtype == torch.bfloat16):
             from ...ops.native import hip_ops
             src = pending._take() if pending is not None else qkv.reshape(T, -1).contiguous()
@@ -491,8 +513,6 @@ class DSInferenceLayer(ProjectionLayer):
                 DF.apply_rotary_pos_emb(k, rope[0], rope[1], position_ids=pos, rotary_dim=rot, interleaved=inter)
             _kv_append_ragged(k[0], v[0], kc, vc, meta)
             q = q[0]
-        scale = spec.attn_scale or 1.0 / math.sqrt(D)
-        window = spec.layer_windows[self.layer_idx] if spec.layer_windows else spec.sliding_window
         return _ragged_attention(q, kc, vc, meta, scale, alibi, window).reshape(1, T, self.hq * D)
 
     def _attention(self, x, meta: BatchMeta, cache, rope, alibi):

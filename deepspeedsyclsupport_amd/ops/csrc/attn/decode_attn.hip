@@ -18,7 +18,8 @@
 //    measured 2x slower: the device-scope fences it needs write back L2.)
 // Measured, us (a workgroup of four waves per 64 to 1024 keys, scores and softmax in LDS between barriers; the read at 6.5 TB/s), 8
 // kv heads of 128: 1 sequence of 130 keys, 4 heads each 6 (14; 0.1), 1 of 8192 19 (44; 5), 12 of 700, 2 heads each 11 (20; 5),
-// 48 of 190, 4 each 12 (24; 6), 48 of 1024 42 (74; 31), 256 of 512 96 (183; 83).
+// 48 of 190, 4 each 12 (24; 6), 48 of 1024 42 (74; 31), 256 of 512 96 (183; 83). A step's rotation and append in it: 0.5 to 1 us, a
+// kernel of their own 4 to 8.
 // Optional ALiBi slopes (BLOOM) are applied on the fly. With a sliding window (Mistral) or chunked visibility only the
 // keys in sight are split and read. A second instantiation takes key and value widths of their own (multiples of 8), a
 // tanh score cap, a softmax sink per head, a gate per token and head, and GQA groups of any size.
@@ -35,9 +36,9 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 constexpr int lanes_per_row(int d) { return d <= 64 ? 8 : (d <= 128 ? 16 : 32); }
 
 struct DecodeArgs {
-  const bf16* q;           // [B, Hq, dk]
-  const bf16* kc;          // [NB, Hk, BS, dk]
-  const bf16* vc;          // [NB, Hk, BS, dv]
+  const bf16* q;           // [B, Hq, dk]; NEW: [B, Hq + 2 Hk, dk], a step's q, k and v as projected
+  bf16* kc;                // [NB, Hk, BS, dk]
+  bf16* vc;                // [NB, Hk, BS, dv]
   const int* block_table;  // [B, max_blocks]
   const int* seq_lens;     // [B]
   const float* alibi;      // [Hq] or null
@@ -49,15 +50,53 @@ struct DecodeArgs {
   int64_t ldg, ldo;
   int Hq, Hk, BS, bs_shift, max_blocks, chunk, window, mask_chunk, dk, dv;  // bs_shift: log2 BS, or -1
   float scale, softcap;
+  const float *cosT, *sinT;  // NEW: [positions, rot / 2]
+  const int* pos;            // [B]
+  int rot, interleaved;
 };
 
-// DK, DV: the widths; 0: given at run time, of which LPR lanes hold a row. GT: at least the query heads served.
-template <int DK, int DV, int GT, int LPR = lanes_per_row(DK)>
+// Elements 8 c .. + 7 of a head, the first `rot` of them turned by cs, sn [rot / 2]: pairs (i, i + rot / 2), or (2 i, 2 i + 1)
+__device__ __forceinline__ bf16x8_t rope_chunk(const bf16* head, int chunk, const float* cs, const float* sn, int rot, int interleaved) {
+  const int d = 8 * chunk, half = rot / 2;
+  const bf16x8_t x = *reinterpret_cast<const bf16x8_t*>(head + d);
+  if (d >= rot) return x;
+  const bool low = d < half;
+  const int i = interleaved ? d / 2 : low ? d : d - half;
+  const bf16x8_t y = *reinterpret_cast<const bf16x8_t*>(head + (interleaved ? d : low ? d + half : i));
+  f32x4 c[2], s[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int at = min(i + 4 * e, half - 4);  // (pairs that stand together need the first four only)
+    c[e] = *reinterpret_cast<const f32x4*>(cs + at);
+    s[e] = *reinterpret_cast<const f32x4*>(sn + at);
+  }
+  bf16x8_t r;
+  if (interleaved) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float a = (float)x[2 * j], b = (float)x[2 * j + 1];
+      r[2 * j] = (bf16)(a * c[0][j] - b * s[0][j]);
+      r[2 * j + 1] = (bf16)(b * c[0][j] + a * s[0][j]);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float turn = (float)y[j] * s[j >> 2][j & 3];
+      r[j] = (bf16)((float)x[j] * c[j >> 2][j & 3] + (low ? -turn : turn));
+    }
+  }
+  return r;
+}
+
+// DK, DV: the widths; 0: given at run time, of which LPR lanes hold a row. GT: at least the query heads served. NEW: the step's
+// projection comes as it is: queries are turned here, and the last key and value are taken from it and written to the cache.
+template <int DK, int DV, int GT, int LPR, bool NEW>
 __global__ void __launch_bounds__(THREADS, 2) paged_decode_kernel(DecodeArgs a) {
   constexpr bool EXT = DK == 0;
   static_assert(EXT || (DK % 16 == 0 && DK >= 64 && DK <= 256 && DK == DV), "head dim");
   const int dk = EXT ? a.dk : DK, dv = EXT ? a.dv : DV;
-  // [WAVES][GT][dv] accumulators, [WAVES][GT][2] maxima and sums, [WAVES][KEYS + 1][GT] probabilities and the fade of what was
+  // [WAVES][GT][dv] accumulators, [WAVES][GT][2] maxima and sums, [WAVES][KEYS + 1][GT] probabilities and the fade of what was;
+  // NEW: [GT + 2][dk] rows of the step
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int b = blockIdx.x, kh = EXT ? blockIdx.y % a.Hk : blockIdx.y, split = blockIdx.z, S = gridDim.z;
   const int g0 = EXT ? blockIdx.y / a.Hk * MAXG : 0;          // first query head of the group this block serves
@@ -65,7 +104,7 @@ __global__ void __launch_bounds__(THREADS, 2) paged_decode_kernel(DecodeArgs a) 
   const int T = a.seq_lens[b];
   int tlo = a.window > 0 ? max(0, T - a.window) : 0;          // first key in sight
   if (a.mask_chunk > 0) tlo = max(tlo, (T - 1) / a.mask_chunk * a.mask_chunk);
-  const int t0 = tlo + split * a.chunk, t1 = min(T, t0 + a.chunk);
+  const int t0 = tlo + split * a.chunk, t1 = min(NEW ? T - 1 : T, t0 + a.chunk);  // (of the keys in the cache)
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   // scores: lane (l16, q4) brings key l16 and holds those of head l16 with keys 4 q4 .. + 3; chunk 4 kk + q4 of 8 elements goes
@@ -74,11 +113,10 @@ __global__ void __launch_bounds__(THREADS, 2) paged_decode_kernel(DecodeArgs a) 
   const int l16 = lane & 15, q4 = lane >> 4;
   bf16x8_t qf[KK];
   const bool mine = l16 < G;
+  if constexpr (!NEW) {
 #pragma unroll
-  for (int kk = 0; kk < KK; ++kk) {
-    const int c = 4 * kk + q4;
-    qf[kk] = *reinterpret_cast<const bf16x8_t*>(a.q + ((int64_t)b * a.Hq + h0 + min(l16, G - 1)) * dk + min(c, dk / 8 - 1) * 8);
-    if (c >= dk / 8 || !mine) qf[kk] = bf16x8_t{};
+    for (int kk = 0; kk < KK; ++kk)
+      qf[kk] = *reinterpret_cast<const bf16x8_t*>(a.q + ((int64_t)b * a.Hq + h0 + min(l16, G - 1)) * dk + min(4 * kk + q4, dk / 8 - 1) * 8);
   }
   const float slope = !EXT && a.alibi && mine ? a.alibi[h0 + l16] : 0.f;
   // values: LPR lanes cover one row, 8 elements each
@@ -121,7 +159,7 @@ __global__ void __launch_bounds__(THREADS, 2) paged_decode_kernel(DecodeArgs a) 
 #pragma unroll
     for (int u = 0; u < UV; ++u) f.v[u] = *reinterpret_cast<const bf16x8_t*>(a.vc + row(t + u * RPW + sub, blk.v[u]) * dv + lv * 8);
   };
-  auto attend = [&](int t, const Group& f) {
+  auto attend = [&](int t, int t1, const Group& f) {
     f32x4 s{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.k[kk], qf[kk], s, 0, 0, 0);
@@ -168,17 +206,50 @@ __global__ void __launch_bounds__(THREADS, 2) paged_decode_kernel(DecodeArgs a) 
     }
     __builtin_amdgcn_wave_barrier();
   };
+  // NEW: a thread turns one chunk of a query or of the key (the value's stay as they are) for all waves (turned by each wave for
+  // itself, a step took 2 to 4 us more)
+  bf16* rows = reinterpret_cast<bf16*>(sm + WAVES * GT * (dv + 2 + KEYS + 1));  // [G queries, key, value][dk]
+  const int own = T - 1 - t0;
+  const bool last = NEW && own >= 0 && own < a.chunk;                          // this split holds the step's own key
+  if constexpr (NEW) {
+    const int cpr = dk / 8, row = tid / cpr, c = tid % cpr;
+    if (row < G + 2) {
+      const int head = row < G ? h0 + row : row == G ? a.Hq + kh : a.Hq + a.Hk + kh, rot = row <= G ? a.rot : 0;
+      const int64_t p = a.rot ? (int64_t)a.pos[b] * (a.rot / 2) : 0;
+      const bf16x8_t x = rope_chunk(a.q + ((int64_t)b * (a.Hq + 2 * a.Hk) + head) * dk, c, a.cosT + p, a.sinT + p, rot, a.interleaved);
+      *reinterpret_cast<bf16x8_t*>(rows + row * dk + c * 8) = x;
+      if (last && row >= G) {
+        const int block = bt[a.bs_shift >= 0 ? (T - 1) >> a.bs_shift : (T - 1) / a.BS];
+        const int64_t at = ((int64_t)block * a.Hk + kh) * a.BS + (a.bs_shift >= 0 ? (T - 1) & (a.BS - 1) : (T - 1) % a.BS);
+        *reinterpret_cast<bf16x8_t*>((row == G ? a.kc : a.vc) + at * dk + c * 8) = x;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk)
+      qf[kk] = *reinterpret_cast<const bf16x8_t*>(rows + min(l16, G - 1) * dk + min(4 * kk + q4, dk / 8 - 1) * 8);
+  }
+#pragma unroll
+  for (int kk = 0; kk < KK; ++kk)
+    if (4 * kk + q4 >= dk / 8 || !mine) qf[kk] = bf16x8_t{};
+  Group f;
   int t = t0 + wid * KEYS;
   if (t < t1) {
-    Group f;
     Blocks blk;
     blocks(t, blk);
     for (; t < t1; t += STEP) {
       load(t, blk, f);
       blocks(t + STEP, blk);
       __builtin_amdgcn_sched_barrier(0);
-      attend(t, f);
+      attend(t, t1, f);
     }
+  }
+  if (last && wid == (own + KEYS - 1) / KEYS % WAVES) {  // the step's own key, by the wave with the fewest others
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) f.k[kk] = *reinterpret_cast<const bf16x8_t*>(rows + G * dk + min(4 * kk + q4, dk / 8 - 1) * 8);
+#pragma unroll
+    for (int u = 0; u < UV; ++u) f.v[u] = *reinterpret_cast<const bf16x8_t*>(rows + (G + 1) * dk + lv * 8);
+    attend(T - 1, T, f);
   }
   // ---- the lane groups of a wave meet in registers (they share their maxima), the waves in LDS
   l += __shfl_xor(l, 16, 64);
@@ -278,7 +349,36 @@ __global__ void __launch_bounds__(256) kv_append_kernel(const bf16* __restrict__
 // Fused QKV epilogue for inference: split the fused projection output, apply RoPE (rotate-half or GPT-J interleaved,
 // partial rotary dims allowed) to q and k, write q [T, Hq, D] and scatter k/v straight into the paged cache
 // (optionally also returning contiguous k/v for the prefill attention). Replaces split + 3 copies + 2 RoPE launches
-// + kv_append. One workgroup per token; token t belongs to sequence t / n_new at cache slot start_pos[b] + t % n_new.
+// + kv_append. One thread per 8 elements, a token's in adjacent workgroups; token t belongs to sequence t / n_new at cache slot
+// start_pos[b] + t % n_new, or (ragged) to seq_ids[t] at slot pos[t]. Bound by its read and write: 8192 tokens, 32 + 2 x 8 heads of
+// 128: 41 us, 4.9 TB/s (one thread per pair, four 2-byte accesses each: 125).
+__global__ void __launch_bounds__(256) qkv_rope_rows_kernel(
+    const bf16* __restrict__ qkv, const float* __restrict__ cosT, const float* __restrict__ sinT,
+    const int* __restrict__ pos, bf16* __restrict__ q_out, bf16* __restrict__ k_out, bf16* __restrict__ v_out,
+    bf16* __restrict__ kc, bf16* __restrict__ vc, const int* __restrict__ block_table,
+    const int* __restrict__ start_pos, const int* __restrict__ seq_ids, int n_new, int Hq, int Hk, int D, int rot,
+    int interleaved, int BS, int max_blocks) {
+  const int H3 = Hq + 2 * Hk, cpr = D / 8, t = blockIdx.x;
+  const int i = blockIdx.y * 256 + threadIdx.x, h = i / cpr, c = i % cpr;
+  if (h >= H3) return;
+  const bf16* head = qkv + ((int64_t)t * H3 + h) * D;
+  const int p = pos[t];
+  const bf16x8_t x = rope_chunk(head, c, cosT + (int64_t)p * (rot / 2), sinT + (int64_t)p * (rot / 2), h < Hq + Hk ? rot : 0, interleaved);
+  if (h < Hq) {
+    *reinterpret_cast<bf16x8_t*>(q_out + ((int64_t)t * Hq + h) * D + c * 8) = x;
+    return;
+  }
+  const bool isk = h < Hq + Hk;
+  const int kh = isk ? h - Hq : h - Hq - Hk, b = seq_ids ? seq_ids[t] : t / n_new;
+  const int slot = seq_ids ? p : start_pos[b] + t % n_new;
+  const int blk = block_table[(int64_t)b * max_blocks + slot / BS];
+  *reinterpret_cast<bf16x8_t*>((isk ? kc : vc) + (((int64_t)blk * Hk + kh) * BS + slot % BS) * D + c * 8) = x;
+  bf16* extra = isk ? k_out : v_out;
+  if (extra) *reinterpret_cast<bf16x8_t*>(extra + ((int64_t)t * Hk + kh) * D + c * 8) = x;
+}
+
+// The same for what that cannot take: sums that still sit in a GEMV's workspace, widths and rotations that are no whole chunks.
+// One thread per element pair.
 __global__ void __launch_bounds__(256) qkv_rope_append_kernel(
     const bf16* __restrict__ qkv, const float* __restrict__ cosT, const float* __restrict__ sinT,
     const int* __restrict__ pos, bf16* __restrict__ q_out, bf16* __restrict__ k_out, bf16* __restrict__ v_out,
@@ -364,11 +464,11 @@ extern "C" int ds_paged_decode_splits(int B, int Hk, int max_len) {
 
 namespace {
 
-template <int DK, int DV, int LPR, int GT>
+template <int DK, int DV, int LPR, bool NEW, int GT>
 int launch_decode(const DecodeArgs& a, dim3 grid, hipStream_t s) {
   const int dv = DK ? DV : a.dv;
-  const int lds = WAVES * GT * (dv + 2 + KEYS + 1) * (int)sizeof(float);
-  auto* kernel = &paged_decode_kernel<DK, DV, GT, LPR>;
+  const int lds = WAVES * GT * (dv + 2 + KEYS + 1) * (int)sizeof(float) + (NEW ? (GT + 2) * dv * 2 : 0);
+  auto* kernel = &paged_decode_kernel<DK, DV, GT, LPR, NEW>;
   if (lds > 65536 &&
       hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
     return (int)hipErrorInvalidValue;
@@ -383,41 +483,57 @@ int launch_decode(const DecodeArgs& a, dim3 grid, hipStream_t s) {
 }
 
 // by the query heads a workgroup serves
-template <int DK, int DV, int LPR>
+template <int DK, int DV, int LPR, bool NEW>
 int launch_decode(const DecodeArgs& a, dim3 grid, hipStream_t s) {
   const int G = a.Hq / a.Hk;
-  if (G <= 1) return launch_decode<DK, DV, LPR, 1>(a, grid, s);
-  if (G <= 2) return launch_decode<DK, DV, LPR, 2>(a, grid, s);
-  if (G <= 4) return launch_decode<DK, DV, LPR, 4>(a, grid, s);
-  return launch_decode<DK, DV, LPR, MAXG>(a, grid, s);
+  if (G <= 1) return launch_decode<DK, DV, LPR, NEW, 1>(a, grid, s);
+  if (G <= 2) return launch_decode<DK, DV, LPR, NEW, 2>(a, grid, s);
+  if (G <= 4) return launch_decode<DK, DV, LPR, NEW, 4>(a, grid, s);
+  return launch_decode<DK, DV, LPR, NEW, MAXG>(a, grid, s);
 }
 
 int log2_of(int n) { return n > 0 && (n & (n - 1)) == 0 ? __builtin_ctz(n) : -1; }
 
 }  // namespace
 
-extern "C" int ds_paged_decode(const void* q, const void* kc, const void* vc, const int* block_table,
+namespace {
+
+template <bool NEW>
+int decode_by_width(const DecodeArgs& a, dim3 grid, hipStream_t s) {
+  switch (a.dk) {
+    case 64: return launch_decode<64, 64, 8, NEW>(a, grid, s);
+    case 80: return launch_decode<80, 80, 16, NEW>(a, grid, s);
+    case 96: return launch_decode<96, 96, 16, NEW>(a, grid, s);
+    case 128: return launch_decode<128, 128, 16, NEW>(a, grid, s);
+    case 256: return launch_decode<256, 256, 32, NEW>(a, grid, s);
+    default: return (int)hipErrorInvalidValue;
+  }
+}
+
+}  // namespace
+
+// With `pos`: q is the step's projection [B, (Hq + 2 Hk) D], seq_lens counts its key, which is turned (like the queries, by the
+// tables' row pos[b]: the first `rot` elements, rot % 16 == 0) and goes into the cache with its value.
+extern "C" int ds_paged_decode(const void* q, void* kc, void* vc, const int* block_table,
                                const int* seq_lens, const float* alibi, float* part_acc, float* part_ml, void* out,
                                int B, int Hq, int Hk, int D, int BS, int max_blocks, int max_len, int splits,
-                               float scale, int window, hipStream_t s) {
-  if (Hk <= 0 || Hq % Hk || Hq / Hk > MAXG || splits <= 0) return (int)hipErrorInvalidValue;
+                               float scale, int window, const int* pos, const float* cosT, const float* sinT, int rot,
+                               int interleaved, hipStream_t s) {
+  if (Hk <= 0 || Hq % Hk || Hq / Hk > MAXG || splits <= 0 || rot < 0 || rot % 16 || rot > D || (rot && (!pos || !cosT || !sinT)))
+    return (int)hipErrorInvalidValue;
   if (window > 0 && window < max_len) max_len = window;  // no more keys than that are in sight
   const int chunk = ((max_len + splits - 1) / splits + 63) / 64 * 64;
-  const DecodeArgs a{(const bf16*)q, (const bf16*)kc, (const bf16*)vc, block_table, seq_lens, alibi, part_acc, part_ml, (bf16*)out,
-                     nullptr, nullptr, 0, (int64_t)Hq * D, Hq, Hk, BS, log2_of(BS), max_blocks, chunk, window, 0, D, D, scale, 0.f};
+  const DecodeArgs a{(const bf16*)q, (bf16*)kc, (bf16*)vc, block_table, seq_lens, alibi, part_acc, part_ml, (bf16*)out,
+                     nullptr, nullptr, 0, (int64_t)Hq * D, Hq, Hk, BS, log2_of(BS), max_blocks, chunk, window, 0, D, D, scale, 0.f,
+                     cosT, sinT, pos, rot, interleaved};
   const dim3 grid(B, Hk, splits);
-  if (D == 64) return launch_decode<64, 64, 8>(a, grid, s);
-  if (D == 80) return launch_decode<80, 80, 16>(a, grid, s);
-  if (D == 96) return launch_decode<96, 96, 16>(a, grid, s);
-  if (D == 128) return launch_decode<128, 128, 16>(a, grid, s);
-  if (D == 256) return launch_decode<256, 256, 32>(a, grid, s);
-  return (int)hipErrorInvalidValue;
+  return pos ? decode_by_width<true>(a, grid, s) : decode_by_width<false>(a, grid, s);
 }
 
 // Key / value widths of their own (multiples of 8 up to 256), chunked and / or windowed visibility, score cap, softmax sink
 // [Hq] (or null), gate [B, Hq] (or null), its rows ldg and rows of out ldo elements apart. `splits`
 // from ds_paged_decode_splits(B, Hk, span) with span = the most keys in sight.
-extern "C" int ds_paged_decode_ext(const void* q, const void* kc, const void* vc, const int* block_table,
+extern "C" int ds_paged_decode_ext(const void* q, void* kc, void* vc, const int* block_table,
                                    const int* seq_lens, float* part_acc, float* part_ml, void* out, int B, int Hq, int Hk,
                                    int dk, int dv, int BS, int max_blocks, int span, int splits, float scale,
                                    float softcap, int window, int mask_chunk, const float* sink, const void* gate,
@@ -426,14 +542,14 @@ extern "C" int ds_paged_decode_ext(const void* q, const void* kc, const void* vc
       ldo < (int64_t)Hq * dv)
     return (int)hipErrorInvalidValue;
   const int chunk = ((span + splits - 1) / splits + 63) / 64 * 64;
-  const DecodeArgs a{(const bf16*)q, (const bf16*)kc, (const bf16*)vc, block_table, seq_lens, nullptr, part_acc, part_ml, (bf16*)out,
+  const DecodeArgs a{(const bf16*)q, (bf16*)kc, (bf16*)vc, block_table, seq_lens, nullptr, part_acc, part_ml, (bf16*)out,
                      sink, (const bf16*)gate, ldg, ldo, Hq, Hk, BS, log2_of(BS), max_blocks, chunk, window, mask_chunk, dk, dv, scale,
-                     softcap};
+                     softcap, nullptr, nullptr, nullptr, 0, 0};
   const dim3 grid(B, Hk * ((Hq / Hk + MAXG - 1) / MAXG), splits);
   const int wide = dk > dv ? dk : dv;
-  if (wide <= 64) return launch_decode<0, 0, 8>(a, grid, s);
-  if (wide <= 128) return launch_decode<0, 0, 16>(a, grid, s);
-  return launch_decode<0, 0, 32>(a, grid, s);
+  if (wide <= 64) return launch_decode<0, 0, 8, false>(a, grid, s);
+  if (wide <= 128) return launch_decode<0, 0, 16, false>(a, grid, s);
+  return launch_decode<0, 0, 32, false>(a, grid, s);
 }
 
 extern "C" int ds_kv_append(const void* k, const void* v, void* kc, void* vc, const int* block_table,
@@ -455,6 +571,13 @@ extern "C" int ds_qkv_rope_append(const void* qkv, const float* cosT, const floa
   if (D % 2 || rot % 2 || rot > D || (D - rot) % 2 || T <= 0) return T == 0 ? 0 : (int)hipErrorInvalidValue;
   if (acc != nullptr && (NP < (Hq + 2 * Hk) * D || T > 16)) return (int)hipErrorInvalidValue;
   if (acc == nullptr && qkv == nullptr) return (int)hipErrorInvalidValue;
+  if (acc == nullptr && D % 8 == 0 && rot % 16 == 0) {
+    hipLaunchKernelGGL(qkv_rope_rows_kernel, dim3(T, ((Hq + 2 * Hk) * (D / 8) + 255) / 256), dim3(256), 0, s, (const bf16*)qkv, cosT,
+                       sinT, pos, (bf16*)q_out, (bf16*)k_out, (bf16*)v_out, (bf16*)kc, (bf16*)vc, block_table, start_pos, seq_ids,
+                       n_new, Hq, Hk, D, rot, interleaved, BS, max_blocks);
+    DS_CHECK_LAUNCH();
+    return 0;
+  }
   const int tph = D / 2 < 256 ? D / 2 : 256, hpb = 256 / tph;
   hipLaunchKernelGGL(qkv_rope_append_kernel, dim3(T, (Hq + 2 * Hk + hpb - 1) / hpb), dim3(256), 0, s, (const bf16*)qkv, cosT, sinT, pos,
                      (bf16*)q_out, (bf16*)k_out, (bf16*)v_out, (bf16*)kc, (bf16*)vc, block_table, start_pos, seq_ids,

@@ -22,8 +22,9 @@ int ds_qkv_rope_append(const void*, const float*, const float*, const int*, void
                        const void*, int, hipStream_t);
 int ds_paged_prefill(const void*, const void*, const void*, void*, const int*, const int*, const int*, const int*, int,
                      const float*, int, int, int, int, int, int, float, hipStream_t);
-int ds_paged_decode(const void*, const void*, const void*, const int*, const int*, const float*, float*, float*, void*,
-                    int, int, int, int, int, int, int, int, float, int, hipStream_t);
+int ds_paged_decode(const void*, void*, void*, const int*, const int*, const float*, float*, float*, void*,
+                    int, int, int, int, int, int, int, int, float, int, const int*, const float*, const float*, int, int,
+                    hipStream_t);
 int ds_kv_append(const void*, const void*, void*, void*, const int*, const int*, int, int, int, int, int, int,
                  hipStream_t);
 int ds_skinny_i8_ok(int, int, int);
@@ -70,15 +71,20 @@ void need(const Tensor& t, const char* n) {
   TORCH_CHECK(t.is_cuda() && t.is_contiguous(), n, " must be a contiguous device tensor");
 }
 
-// q [B, Hq, D] bf16; caches [NB, Hk, BS, D] bf16; block_table [B, max_blocks] int32; seq_lens [B] int32
-Tensor paged_decode(Tensor q, Tensor kc, Tensor vc, Tensor block_table, Tensor seq_lens, int64_t max_len, double scale,
-                    OptT alibi, int64_t window, OptT into) {
+// Where a step's own keys and values still have to be turned and appended
+struct NewKeys {
+  const int* pos = nullptr;
+  const float *cos = nullptr, *sin = nullptr;
+  int rot = 0, interleaved = 0;
+};
+
+Tensor run_paged_decode(const Tensor& q, int B, int Hq, const Tensor& kc, const Tensor& vc, const Tensor& block_table,
+                        const Tensor& seq_lens, int64_t max_len, double scale, const OptT& alibi, int64_t window, const OptT& into,
+                        const NewKeys& fresh) {
   need(q, "q"); need(kc, "k_cache"); need(vc, "v_cache"); need(block_table, "block_table"); need(seq_lens, "seq_lens");
   TORCH_CHECK(q.scalar_type() == at::kBFloat16 && kc.scalar_type() == at::kBFloat16, "bf16 q/cache");
   TORCH_CHECK(block_table.scalar_type() == at::kInt && seq_lens.scalar_type() == at::kInt, "int32 tables");
-  const int B = (int)q.size(0), Hq = (int)q.size(1), D = (int)q.size(2);
-  const int Hk = (int)kc.size(1), BS = (int)kc.size(2);
-  TORCH_CHECK(kc.size(3) == D, "head dim mismatch");
+  const int Hk = (int)kc.size(1), BS = (int)kc.size(2), D = (int)kc.size(3);
   const int max_blocks = (int)block_table.size(1);
   TORCH_CHECK((int64_t)max_blocks * BS >= max_len, "block table too small for max_len");
   const int64_t span = window > 0 && window < max_len ? window : max_len;  // keys in sight
@@ -87,7 +93,7 @@ Tensor paged_decode(Tensor q, Tensor kc, Tensor vc, Tensor block_table, Tensor s
     need(*into, "out");
     TORCH_CHECK(into->sizes() == q.sizes() && into->scalar_type() == at::kBFloat16, "paged_decode: out like q");
   }
-  auto out = into.has_value() ? *into : torch::empty_like(q);
+  auto out = into.has_value() ? *into : torch::empty({B, Hq, D}, q.options());
   auto fo = q.options().dtype(at::kFloat);
   Tensor pacc, pml;
   if (splits > 1) {
@@ -99,9 +105,37 @@ Tensor paged_decode(Tensor q, Tensor kc, Tensor vc, Tensor block_table, Tensor s
   check(ds_paged_decode(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), block_table.data_ptr<int>(),
                         seq_lens.data_ptr<int>(), al, splits > 1 ? pacc.data_ptr<float>() : nullptr,
                         splits > 1 ? pml.data_ptr<float>() : nullptr, out.data_ptr(), B, Hq, Hk, D, BS, max_blocks,
-                        (int)max_len, splits, (float)scale, (int)window, stream()),
+                        (int)max_len, splits, (float)scale, (int)window, fresh.pos, fresh.cos, fresh.sin, fresh.rot,
+                        fresh.interleaved, stream()),
         "paged_decode");
   return out;
+}
+
+// q [B, Hq, D] bf16; caches [NB, Hk, BS, D] bf16; block_table [B, max_blocks] int32; seq_lens [B] int32
+Tensor paged_decode(Tensor q, Tensor kc, Tensor vc, Tensor block_table, Tensor seq_lens, int64_t max_len, double scale,
+                    OptT alibi, int64_t window, OptT into) {
+  TORCH_CHECK(kc.size(3) == q.size(2), "head dim mismatch");
+  return run_paged_decode(q, (int)q.size(0), (int)q.size(1), kc, vc, block_table, seq_lens, max_len, scale, alibi, window, into, {});
+}
+
+// A decode step's projection qkv [B, (Hq + 2 Hk) D], one token a sequence -> its attention [B, Hq, D] over the cache, which takes
+// up the step's key (turned, like the queries, by row pos[b] of the tables: the first `rot` elements, rot % 16 == 0) and value at
+// place seq_lens[b] - 1
+Tensor paged_decode_step(Tensor qkv, OptT cos, OptT sin, Tensor pos, Tensor kc, Tensor vc, Tensor block_table, Tensor seq_lens,
+                         int64_t max_len, double scale, OptT alibi, int64_t window, int64_t Hq, int64_t rot, bool interleaved) {
+  need(pos, "pos");
+  const int64_t B = seq_lens.numel(), Hk = kc.size(1), D = kc.size(3);
+  TORCH_CHECK(qkv.numel() == B * (Hq + 2 * Hk) * D && pos.numel() == B && pos.scalar_type() == at::kInt && block_table.size(0) == B,
+              "paged_decode_step: one row of q, k and v, and one position, per sequence");
+  TORCH_CHECK(vc.sizes() == kc.sizes() && rot % 16 == 0 && rot >= 0 && rot <= D, "paged_decode_step: caches / rotation");
+  NewKeys fresh{pos.data_ptr<int>(), nullptr, nullptr, (int)rot, interleaved ? 1 : 0};
+  if (rot) {
+    TORCH_CHECK(cos.has_value() && sin.has_value(), "rope tables required");
+    need(*cos, "cos"); need(*sin, "sin");
+    fresh.cos = cos->data_ptr<float>();
+    fresh.sin = sin->data_ptr<float>();
+  }
+  return run_paged_decode(qkv, (int)B, (int)Hq, kc, vc, block_table, seq_lens, max_len, scale, alibi, window, c10::nullopt, fresh);
 }
 
 // k, v [B, n_new, Hk, D] -> caches at positions start_pos[b] + j
@@ -575,6 +609,7 @@ void register_inference_ops(pybind11::module& m) {
         py::arg("kc"), py::arg("vc"), py::arg("block_table"), py::arg("start_pos"), py::arg("n_new"), py::arg("Hq"),
         py::arg("Hk"), py::arg("rot"), py::arg("interleaved"), py::arg("want_kv"), py::arg("seq_ids") = py::none(), py::arg("acc_rows") = 0,
         py::arg("acc_bias") = py::none());
+  m.def("paged_decode_step", &paged_decode_step);
   m.def("paged_decode", &paged_decode, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_table"),
         py::arg("seq_lens"), py::arg("max_len"), py::arg("scale"), py::arg("alibi"), py::arg("window"), py::arg("out") = py::none());
   m.def("kv_append", &kv_append);

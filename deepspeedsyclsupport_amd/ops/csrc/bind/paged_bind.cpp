@@ -16,7 +16,7 @@ int ds_paged_prefill_ext(const void*, const void*, const void*, void*, const int
                          int, int, int, int, int, int, int, int, float, float, const float*, const void*, int64_t, int64_t,
                          hipStream_t);
 int ds_paged_decode_splits(int, int, int);
-int ds_paged_decode_ext(const void*, const void*, const void*, const int*, const int*, float*, float*, void*, int, int,
+int ds_paged_decode_ext(const void*, void*, void*, const int*, const int*, float*, float*, void*, int, int,
                         int, int, int, int, int, int, int, float, float, int, int, const float*, const void*, int64_t, int64_t,
                         hipStream_t);
 }

@@ -345,6 +345,26 @@ def test_paged_decode_edges_of_key_groups(hq, hk, D, BS, window):
         assert torch.equal(out, room[:-1]) and (room[-1] == 7).all()
 
 
+@pytest.mark.parametrize("D,rot,interleaved", [(128, 128, False), (128, 32, False), (64, 64, True), (80, 16, False), (256, 0, False)])
+@pytest.mark.parametrize("window", [0, 40])
+def test_paged_decode_step_equals_append_and_attention(D, rot, interleaved, window):
+    """A step that turns and appends its own keys, against the two kernels: the cache to the bit of rounding, its other rows
+    untouched, and the attention of what they made."""
+    hq, hk, BS, lens = 8, 2, 16, [1, 2, 16, 17, 113, 129, 900, 1500]   # with the step's own key
+    kc, vc, bt, maxb = _paged_setup(len(lens), hk, D, BS, lens, seed=6)
+    qkv = torch.randn(len(lens), (hq + 2 * hk) * D, device="cuda").bfloat16()
+    sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    pos, seqs = sl - 1, torch.arange(len(lens), dtype=torch.int32, device="cuda")
+    tables = R.rope_tables(2048, rot, device="cuda") if rot else (None, None)
+    k2, v2 = kc.clone(), vc.clone()
+    q = ops().qkv_rope_append(qkv, *tables, pos, k2, v2, bt, pos, 1, hq, hk, rot, interleaved, False, seqs)[0]
+    want = ops().paged_decode(q, k2, v2, bt, sl, maxb * BS, D**-0.5, None, window)
+    got = ops().paged_decode_step(qkv, *tables, pos, kc, vc, bt, sl, maxb * BS, D**-0.5, None, window, hq, rot, interleaved)
+    assert torch.equal(vc, v2)
+    torch.testing.assert_close(kc.float(), k2.float(), rtol=2.0**-7, atol=0)  # (a * c - b * s may be contracted either way)
+    torch.testing.assert_close(got.float(), want.float(), rtol=1e-2, atol=1e-2)
+
+
 def test_kv_append():
     B, n, hk, D, BS = 3, 5, 4, 128, 16
     kc, vc, bt, maxb = _paged_setup(B, hk, D, BS, [64, 64, 64])
@@ -677,3 +697,26 @@ def test_norm_forward_few_and_many_rows(rows, H, res):
         (DF.layer_norm(xg, g, b, 1e-5).float() * gy).sum().backward()
         (F.layer_norm(xf, (H, ), g.float(), b.float(), 1e-5) * gy).sum().backward()
         torch.testing.assert_close(xg.grad.float(), xf.grad, rtol=5e-2, atol=5e-2)
+
+
+@pytest.mark.parametrize("D,rot,interleaved", [(96, 16, False), (80, 80, True), (80, 80, False), (80, 20, False), (64, 8, True)])
+def test_qkv_rope_append_chunks_and_pairs(D, rot, interleaved):
+    """Widths and rotations of whole chunks of 8, and those that go pair by pair: rows of a ragged batch, without copies."""
+    hq, hk, BS, T = 3, 1, 8, 21
+    kc, vc, bt, maxb = _paged_setup(2, hk, D, BS, [64, 64])
+    qkv = torch.randn(T, (hq + 2 * hk) * D, device="cuda").bfloat16()
+    seqs = torch.tensor([0] * 9 + [1] * 12, dtype=torch.int32, device="cuda")
+    pos = torch.cat([torch.arange(5, 14), torch.arange(12)]).int().cuda()
+    cos, sin = R.rope_tables(256, rot, device="cuda")
+    start = torch.tensor([5, 0], dtype=torch.int32, device="cuda")
+    q = ops().qkv_rope_append(qkv, cos, sin, pos, kc, vc, bt, start, 1, hq, hk, rot, interleaved, False, seqs)[0]
+    x = qkv.view(T, hq + 2 * hk, D).float()
+    c, s = cos[pos.long()][:, None], sin[pos.long()][:, None]
+    y = x.clone()
+    a, b = (x[..., 0:rot:2], x[..., 1:rot:2]) if interleaved else (x[..., :rot // 2], x[..., rot // 2:rot])
+    lo, hi = (slice(0, rot, 2), slice(1, rot, 2)) if interleaved else (slice(0, rot // 2), slice(rot // 2, rot))
+    y[..., lo], y[..., hi] = a * c - b * s, b * c + a * s
+    torch.testing.assert_close(q.float(), y[:, :hq], rtol=1e-2, atol=1e-2)
+    blk, off = bt[seqs.long(), (pos // BS).long()].long(), (pos % BS).long()
+    torch.testing.assert_close(kc[blk, :, off].float(), y[:, hq:hq + hk], rtol=1e-2, atol=1e-2)
+    assert torch.equal(vc[blk, :, off].float(), x[:, hq + hk:])
