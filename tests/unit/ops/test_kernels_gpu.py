@@ -69,6 +69,47 @@ def test_adam_multi_and_fused_adam_optimizer():
         torch.testing.assert_close(p, r, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("pdt,gdt,ldt", [(torch.float32, torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32, None),
+                                         (torch.float32, torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16, None)])
+def test_adam_multi_block_edges(pdt, gdt, ldt):
+    """Sizes around a block's elements and tensors that start off the vector alignment, several in one launch; what lies between
+    the tensors stays."""
+    sizes, room = [1, 8, 1016, 1024, 1032, 4104, 1023, 40000], 8
+    def tensors(dt, scale=1.0):
+        flat = (torch.rand(sum(sizes) + room * (len(sizes) + 1), device="cuda") * scale).to(dt)
+        at, out = 0, []
+        for i, n in enumerate(sizes):
+            at += room + (i == 5)  # (one tensor at an odd address)
+            out.append(flat[at:at + n])
+            at += n
+        return flat, out
+    fp, p = tensors(pdt)
+    fm, m = tensors(pdt, 0.1)
+    fv, v = tensors(pdt, 0.01)
+    _, g = tensors(gdt)
+    flp, lp = tensors(ldt) if ldt else (None, [])
+    before = [f.clone() for f in (fp, fm, fv)]
+    ref = [[t.float().clone() for t in ts] for ts in (p, m, v)]
+    ops().adam_multi(p, m, v, g, lp, 1e-2, 0.9, 0.99, 1e-8, 0.1, 0.1, 0.01, 0.5, True)
+    tol = dict(rtol=1e-5, atol=1e-6) if pdt == torch.float32 else dict(rtol=1e-2, atol=1e-3)
+    for i in range(len(sizes)):
+        pr, mr, vr = (ref[k][i] for k in range(3))
+        R.adam_update(pr, mr, vr, g[i].float() * 0.5, 1e-2, 0.9, 0.99, 1e-8, 0.1, 1)
+        for a, b in ((p[i], pr), (m[i], mr), (v[i], vr)):
+            torch.testing.assert_close(a.float(), b, **tol)
+        if ldt:
+            # (half an ulp, or the other neighbour of a tie: the copy may be rounded from the unrounded update)
+            torch.testing.assert_close(lp[i].float(), p[i], rtol=2.0**-11 * 1.01 if ldt == torch.float16 else 2.0**-8 * 1.01, atol=1e-7)
+    used = torch.zeros_like(fp, dtype=torch.bool)
+    at = 0
+    for i, n in enumerate(sizes):
+        at += room + (i == 5)
+        used[at:at + n] = True
+        at += n
+    for f, b in zip((fp, fm, fv), before):
+        assert torch.equal(f[~used], b[~used])
+
+
 def test_lion_adagrad_lamb():
     torch.manual_seed(2)
     n = 100003
