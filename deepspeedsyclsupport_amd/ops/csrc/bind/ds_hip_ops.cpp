@@ -21,7 +21,8 @@ int ds_lion_flat(void*, void*, const void*, void*, int64_t, int, int, int, float
 int ds_adagrad_flat(void*, void*, const void*, void*, int64_t, int, int, int, float, float, float, float, hipStream_t);
 int ds_lamb_flat(void*, void*, void*, const void*, void*, float*, float*, float*, int64_t, int, int, int, float,
                  float, float, float, float, float, float, float, float, float, hipStream_t);
-int ds_sumsq_multi(const void**, const int64_t*, const int*, int, float*, int, float*, hipStream_t);
+int ds_sumsq_partials(int);
+int ds_sumsq_multi(const void**, const int64_t*, const int*, int, float*, float*, hipStream_t);
 int ds_norm_bwd_blocks(int64_t);
 int ds_rms_fwd(const void*, const void*, const void*, void*, void*, float*, int64_t, int, float, int, hipStream_t);
 int ds_rms_bwd(const void*, const void*, const void*, const float*, const void*, void*, void*, float*, int64_t, int,
@@ -189,10 +190,9 @@ Tensor lamb_flat(Tensor p, Tensor m, Tensor v, Tensor g, OptT lp, double lr, dou
 // sum of squares of all tensors (fp32 device scalar), deterministic
 Tensor sumsq_multi(std::vector<Tensor> xs) {
   TORCH_CHECK(!xs.empty(), "sumsq_multi: empty list");
-  const int cap = 512 * (int)xs.size();
   auto fopt = xs[0].options().dtype(at::kFloat);
-  auto partials = torch::empty({cap}, fopt);
-  auto out = torch::zeros({}, fopt);
+  auto partials = torch::empty({ds_sumsq_partials((int)xs.size())}, fopt);
+  auto out = torch::empty({}, fopt);
   std::vector<const void*> ptrs;
   std::vector<int64_t> ns;
   std::vector<int> dts;
@@ -202,7 +202,7 @@ Tensor sumsq_multi(std::vector<Tensor> xs) {
     ns.push_back(x.numel());
     dts.push_back(dcode(x));
   }
-  check(ds_sumsq_multi(ptrs.data(), ns.data(), dts.data(), (int)xs.size(), partials.data_ptr<float>(), cap,
+  check(ds_sumsq_multi(ptrs.data(), ns.data(), dts.data(), (int)xs.size(), partials.data_ptr<float>(),
                        out.data_ptr<float>(), stream()),
         "sumsq_multi");
   return out;

@@ -140,6 +140,18 @@ def test_sumsq_multi():
     assert abs(got - ref) / ref < 1e-5
 
 
+def test_sumsq_multi_many_tensors_and_edges():
+    """More tensors than a launch's table holds, empty ones, starts off the vector alignment, sizes around a block's round, all
+    types; each sum is of non-negative terms, so fp32 in any order is off by a few 2^-24 per term of a thread's chain."""
+    sizes = [8191, 0, 8192, 8193, 1, 7, 40000, 3 << 20] * 10
+    for dt in (torch.float32, torch.bfloat16, torch.float16):
+        xs = [torch.randn(n + i % 3, device="cuda").to(dt)[i % 3:] for i, n in enumerate(sizes)]
+        ref = sum(float(x.double().pow(2).sum()) for x in xs)
+        assert abs(float(ops().sumsq_multi(xs)) - ref) / ref < 1e-5
+    assert float(ops().sumsq_multi([torch.empty(0, device="cuda")])) == 0
+    assert math.isinf(float(ops().sumsq_multi([torch.ones(10, device="cuda"), torch.full((3, ), math.inf, device="cuda")])))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("H", [64, 1024, 4096, 5120, 8192])
 @pytest.mark.parametrize("residual", [False, True])
