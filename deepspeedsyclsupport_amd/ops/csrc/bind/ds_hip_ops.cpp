@@ -62,7 +62,8 @@ int ds_flash_bwd(const void*, const void*, const void*, const void*, const void*
                  const float*, int64_t, int64_t, hipStream_t);
 int ds_transpose16(const void*, void*, int, int, int, int64_t, hipStream_t);
 int ds_xent_fwd(const void*, const int64_t*, float*, float*, int64_t, int, int64_t, int, float, int, hipStream_t);
-int ds_xent_bwd(const void*, const int64_t*, const float*, const float*, float, void*, int64_t, int, int64_t, int64_t,
+int ds_xent_mean(const float*, const int64_t*, float*, float*, int64_t, int, hipStream_t);
+int ds_xent_bwd(const void*, const int64_t*, const float*, const float*, float, const float*, void*, int64_t, int, int64_t, int64_t,
                 int, float, int, hipStream_t);
 }
 
@@ -476,15 +477,27 @@ std::vector<Tensor> xent_fwd(Tensor logits, Tensor labels, int64_t ignore_index,
   return {loss, lse};
 }
 
+// -> (mean over the labels that are not ignored, lse [N], how many those are)
+std::vector<Tensor> xent_mean_fwd(Tensor logits, Tensor labels, int64_t ignore_index, double smoothing) {
+  auto r = xent_fwd(logits, labels, ignore_index, smoothing);
+  TORCH_CHECK(labels.numel() == logits.size(0) && labels.numel() < ((int64_t)1 << 31), "xent: one label per row");
+  auto mean = torch::empty({}, r[0].options()), of = torch::empty({}, r[0].options());
+  check(ds_xent_mean(r[0].data_ptr<float>(), labels.data_ptr<int64_t>(), mean.data_ptr<float>(), of.data_ptr<float>(),
+                     labels.numel(), (int)ignore_index, stream()), "xent_mean");
+  return {mean, r[1], of};
+}
+
+// mean_of from xent_mean_fwd: dloss is the gradient of its mean, one number
 Tensor xent_bwd(Tensor logits, Tensor labels, Tensor lse, OptT dloss, double dloss_scalar, bool inplace,
-                int64_t ignore_index, double smoothing) {
+                int64_t ignore_index, double smoothing, OptT mean_of) {
   const int64_t N = logits.size(0);
+  TORCH_CHECK(!mean_of.has_value() || (dloss.has_value() && dloss->numel() == 1), "xent_bwd: the gradient of a mean is one number");
   Tensor out = inplace ? logits : torch::empty_like(logits);
   const float* dl = nullptr;
   Tensor dlc;
   if (dloss.has_value()) { dlc = dloss->to(at::kFloat).contiguous(); dl = dlc.data_ptr<float>(); }
   check(ds_xent_bwd(logits.data_ptr(), labels.data_ptr<int64_t>(), lse.data_ptr<float>(), dl, (float)dloss_scalar,
-                    out.data_ptr(), N, (int)logits.size(1), logits.stride(0), out.stride(0), (int)ignore_index,
+                    mean_of.has_value() ? mean_of->data_ptr<float>() : nullptr, out.data_ptr(), N, (int)logits.size(1), logits.stride(0), out.stride(0), (int)ignore_index,
                     smoothing, dcode(logits), stream()),
         "xent_bwd");
   return out;
@@ -748,5 +761,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("work") = py::none(), py::arg("merges") = py::none(), py::arg("nslots") = 0, py::arg("kbias") = py::none(),
         py::arg("abias") = py::none(), py::arg("rpe") = py::none(), py::arg("check_plan") = true);
   m.def("xent_fwd", &xent_fwd);
-  m.def("xent_bwd", &xent_bwd);
+  m.def("xent_mean_fwd", &xent_mean_fwd);
+  m.def("xent_bwd", &xent_bwd, py::arg("logits"), py::arg("labels"), py::arg("lse"), py::arg("dloss"), py::arg("dloss_scalar"),
+        py::arg("inplace"), py::arg("ignore_index"), py::arg("smoothing"), py::arg("mean_of") = py::none());
 }

@@ -71,10 +71,45 @@ __global__ void __launch_bounds__(256) xent_fwd_kernel(const T* __restrict__ log
   }
 }
 
+// mean = sum of the rows' losses / max(n, 1), mean_of = max(n, 1), n the labels that are not ignored: one block, since what it
+// replaces (compare, convert, two sums, clamp, divide, and two more in the backward) was a launch each, 5 us or more.
+__global__ void __launch_bounds__(1024) xent_mean_kernel(const float* __restrict__ loss, const int64_t* __restrict__ labels,
+                                                         float* __restrict__ mean, float* __restrict__ mean_of, int64_t rows,
+                                                         int ignore_index) {
+  __shared__ float sum[16];
+  __shared__ int count[16];
+  float s = 0.f;
+  int n = 0;
+  for (int64_t i = threadIdx.x; i < rows; i += 1024) {
+    s += loss[i];
+    n += labels[i] != ignore_index;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    s += __shfl_xor(s, o, 64);
+    n += __shfl_xor(n, o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    sum[threadIdx.x >> 6] = s;
+    count[threadIdx.x >> 6] = n;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; ++w) {
+      s += sum[w];
+      n += count[w];
+    }
+    const float of = (float)(n > 1 ? n : 1);
+    *mean = s / of;
+    *mean_of = of;
+  }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) xent_bwd_kernel(const T* __restrict__ logits, const int64_t* __restrict__ labels,
                                                        const float* __restrict__ lse, const float* __restrict__ dloss,
-                                                       float dloss_scalar, T* __restrict__ dlogits, int64_t rows,
+                                                       float dloss_scalar, const float* __restrict__ mean_of,
+                                                       T* __restrict__ dlogits, int64_t rows,
                                                        int V, int64_t ld, int64_t ldo, int ignore_index,
                                                        float smoothing) {
   const int64_t row = blockIdx.x;
@@ -83,7 +118,8 @@ __global__ void __launch_bounds__(256) xent_bwd_kernel(const T* __restrict__ log
   T* dx = dlogits + row * ldo;
   const int64_t lab = labels[row];
   const bool ignored = (lab == ignore_index || lab < 0 || lab >= V);
-  const float g = ignored ? 0.f : (dloss ? dloss[row] : dloss_scalar);
+  // mean_of: dloss is the gradient of the mean over that many rows
+  const float g = ignored ? 0.f : mean_of ? *dloss / *mean_of : (dloss ? dloss[row] : dloss_scalar);
   const float L = lse[row];
   const float sm_off = smoothing / V;
   const bool vec = (V % 8 == 0) && ((((uintptr_t)x) & 15) == 0) && ((((uintptr_t)dx) & 15) == 0);
@@ -126,12 +162,20 @@ extern "C" int ds_xent_fwd(const void* logits, const int64_t* labels, float* los
   return 0;
 }
 
+extern "C" int ds_xent_mean(const float* loss, const int64_t* labels, float* mean, float* mean_of, int64_t rows, int ignore_index,
+                            hipStream_t s) {
+  hipLaunchKernelGGL(xent_mean_kernel, dim3(1), dim3(1024), 0, s, loss, labels, mean, mean_of, rows, ignore_index);
+  DS_CHECK_LAUNCH();
+  return 0;
+}
+
+// mean_of: null, or dloss is one number, the gradient of the mean over *mean_of rows.
 extern "C" int ds_xent_bwd(const void* logits, const int64_t* labels, const float* lse, const float* dloss,
-                           float dloss_scalar, void* dlogits, int64_t rows, int V, int64_t ld, int64_t ldo,
+                           float dloss_scalar, const float* mean_of, void* dlogits, int64_t rows, int V, int64_t ld, int64_t ldo,
                            int ignore_index, float smoothing, int dtype, hipStream_t s) {
   if (rows <= 0) return 0;
   DISPATCH_T(dtype, hipLaunchKernelGGL((xent_bwd_kernel<T>), dim3((unsigned)rows), dim3(256), 0, s, (const T*)logits,
-                                       labels, lse, dloss, dloss_scalar, (T*)dlogits, rows, V, ld, ldo, ignore_index,
+                                       labels, lse, dloss, dloss_scalar, mean_of, (T*)dlogits, rows, V, ld, ldo, ignore_index,
                                        smoothing));
   DS_CHECK_LAUNCH();
   return 0;

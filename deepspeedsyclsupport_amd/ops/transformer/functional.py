@@ -278,11 +278,30 @@ class _XentFn(torch.autograd.Function):
         return dlogits, None, None, None, None
 
 
+class _XentMeanFn(torch.autograd.Function):
+    """The mean over the labels that are not ignored."""
+
+    @staticmethod
+    def forward(ctx, logits, labels, ignore_index, smoothing, inplace_grad):
+        mean, lse, mean_of = hip_ops().xent_mean_fwd(logits, labels, ignore_index, smoothing)
+        ctx.save_for_backward(logits, labels, lse, mean_of)
+        ctx.ignore_index, ctx.smoothing, ctx.inplace = ignore_index, smoothing, inplace_grad
+        return mean
+
+    @staticmethod
+    def backward(ctx, dloss):
+        logits, labels, lse, mean_of = ctx.saved_tensors
+        dlogits = hip_ops().xent_bwd(logits, labels, lse, dloss, 0.0, ctx.inplace, ctx.ignore_index, ctx.smoothing, mean_of)
+        return dlogits, None, None, None, None
+
+
 def cross_entropy(logits, labels, ignore_index=-100, label_smoothing=0.0, reduction="mean", inplace_backward=True):
     """Fused softmax-CE over [N, V] logits (bf16/fp32). `inplace_backward` reuses the logits buffer for the grad."""
     if logits.is_cuda:
         logits2 = logits.reshape(-1, logits.shape[-1])
         labels2 = labels.reshape(-1).contiguous()
+        if reduction not in ("none", "sum"):
+            return _XentMeanFn.apply(logits2, labels2, ignore_index, label_smoothing, inplace_backward)
         per_tok = _XentFn.apply(logits2, labels2, ignore_index, label_smoothing, inplace_backward)
     else:
         per_tok = reference.cross_entropy(logits.reshape(-1, logits.shape[-1]), labels.reshape(-1), ignore_index,

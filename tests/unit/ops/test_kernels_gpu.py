@@ -321,6 +321,28 @@ def test_cross_entropy(V, dtype):
     torch.testing.assert_close(logits.grad.float(), lf.grad, **TOL[dtype])
 
 
+@pytest.mark.parametrize("N,ignored", [(1, 0), (67, 20), (67, 67), (2500, 7), (0, 0)])
+def test_cross_entropy_mean_is_that_of_the_rows(N, ignored):
+    """The fused mean against the rows' own losses: the same numbers, added up in another order; its gradient too. A label that no
+    row of the vocabulary has counts but weighs nothing; the result can be changed in place."""
+    from deepspeedsyclsupport_amd.ops.transformer import functional as DF
+    V = 264
+    x = torch.randn(N, V, device="cuda")
+    labels = torch.randint(0, V, (N, ), device="cuda")
+    labels[:ignored] = -7
+    if N > 60 and ignored < 60:
+        labels[60] = V + 3
+    a, b = (x.clone().requires_grad_(True) for _ in range(2))
+    rows = DF.cross_entropy(a, labels, ignore_index=-7, label_smoothing=0.1, reduction="none", inplace_backward=False)
+    want = rows.sum() / (labels != -7).sum().clamp(min=1)
+    got = DF.cross_entropy(b, labels, ignore_index=-7, label_smoothing=0.1, inplace_backward=False)
+    torch.testing.assert_close(got, want, rtol=1e-6, atol=0)
+    got /= 2
+    (want / 2 * 3).backward()
+    (got * 3).backward()
+    torch.testing.assert_close(b.grad, a.grad, rtol=1e-6, atol=1e-9)
+
+
 # ------------------------------------------------------------------------------------------------ inference kernels
 def _paged_setup(B, Hk, D, BS, lens, seed=0):
     g = torch.Generator(device="cuda").manual_seed(seed)
