@@ -12,6 +12,7 @@ import torch
 from torch import Tensor, nn
 from torch.nn import functional as F
 
+from ...models.llama import TokenEmbedding
 from .utils import DeQuantizer, Packed, Quantizer
 
 quantized_weight_registry = {}  # id(original weight) -> (codes, scale, minimum, shape, moved); cleared after a pass
@@ -95,4 +96,5 @@ class QuantizedEmbedding(nn.Module, _QuantizedWeight):
 QUANTIZATION_LAYER_MAPPINGS = {
     nn.Linear: QuantizedLinear,
     nn.Embedding: QuantizedEmbedding,
+    TokenEmbedding: QuantizedEmbedding,
 }

@@ -161,12 +161,21 @@ class LlamaDecoderLayer(nn.Module):
         return self.mlp(normed), residual
 
 
+class TokenEmbedding(nn.Embedding):
+    """nn.Embedding whose plain form (no padding row, norm bound, frequency scaling or sparse gradient) takes the gradient kernel."""
+
+    def forward(self, ids):
+        if self.padding_idx is None and self.max_norm is None and not self.scale_grad_by_freq and not self.sparse:
+            return DF.embedding(ids, self.weight)
+        return super().forward(ids)
+
+
 class LlamaModel(nn.Module):
 
     def __init__(self, cfg: LlamaConfig):
         super().__init__()
         self.cfg = cfg
-        self.embed_tokens = nn.Embedding(cfg.vocab_size, cfg.hidden_size)
+        self.embed_tokens = TokenEmbedding(cfg.vocab_size, cfg.hidden_size)
         self.layers = nn.ModuleList([LlamaDecoderLayer(cfg, i) for i in range(cfg.num_hidden_layers)])
         self.norm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps)
         self.rope = RotaryTables(cfg.head_dim, cfg.max_position_embeddings, cfg.rope_theta)

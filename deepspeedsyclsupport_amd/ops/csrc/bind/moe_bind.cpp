@@ -14,6 +14,8 @@ int ds_moe_gather(const void*, const float*, const int*, void*, int, int, int, h
 int ds_grouped_gemm_ok(int, int);
 int ds_grouped_gemm(const void*, const void*, void*, const int*, int, int, int, int, hipStream_t);
 int ds_embed_gather(const void*, const int64_t*, const void*, const int64_t*, void*, int64_t, int, hipStream_t);
+int ds_embed_grad_max();
+int ds_embed_grad(const void*, const int64_t*, void*, int64_t, int, int64_t, hipStream_t);
 int ds_rows_gather(const void*, const int64_t*, void*, int64_t, int, hipStream_t);
 int ds_rows_scatter(const void*, const int64_t*, void*, int64_t, int, hipStream_t);
 int ds_token_sort(int*, int, int, int, hipStream_t);
@@ -116,6 +118,16 @@ Tensor embed_gather(Tensor table, Tensor ids, std::optional<Tensor> pos_table, s
   return out;
 }
 
+// The gradient [V, H] of an embedding whose rows ids [T] gave dy [T, H]
+Tensor embed_grad(Tensor dy, Tensor ids, int64_t V) {
+  need_bf16(dy, "dy"); need(ids, "ids");
+  TORCH_CHECK(ids.scalar_type() == at::kLong && dy.dim() == 2 && dy.size(0) == ids.numel(), "embed_grad: int64 ids, one row each");
+  if ((uintptr_t)dy.data_ptr() % 16) dy = dy.clone();  // it is read by 16 bytes
+  auto out = torch::zeros({V, dy.size(1)}, dy.options());
+  check(ds_embed_grad(dy.data_ptr(), ids.data_ptr<int64_t>(), out.data_ptr(), ids.numel(), (int)dy.size(1), V, stream()), "embed_grad");
+  return out;
+}
+
 // out[i] = x[idx[i]] rows
 // In-place per-row sort of distinct int32 token positions in [0, S) (random-LTD token_sort_).
 Tensor token_sort_(Tensor idx, int64_t S) {
@@ -154,6 +166,8 @@ void register_moe_ops(pybind11::module& m) {
   m.def("grouped_gemm_ok", &grouped_gemm_ok);
   m.def("grouped_gemm", &grouped_gemm);
   m.def("embed_gather", &embed_gather);
+  m.def("embed_grad", &embed_grad);
+  m.def("embed_grad_max", []() { return ds_embed_grad_max(); });
   m.def("token_sort_", &token_sort_);
   m.def("rows_gather", &rows_gather);
   m.def("rows_scatter", &rows_scatter);

@@ -260,6 +260,30 @@ def apply_rotary_pos_emb(x, cos, sin, position_ids=None, pos_offset=0, rotary_di
     return x
 
 
+# --------------------------------------------------------------------------------------------------- embedding
+class _EmbeddingFn(torch.autograd.Function):
+
+    @staticmethod
+    def forward(ctx, ids, weight):
+        ctx.save_for_backward(ids)
+        ctx.rows = weight.shape[0]
+        return F.embedding(ids, weight)
+
+    @staticmethod
+    def backward(ctx, dy):
+        (ids, ) = ctx.saved_tensors
+        return None, hip_ops().embed_grad(dy.reshape(-1, dy.shape[-1]).contiguous(), ids.reshape(-1).contiguous(), ctx.rows)
+
+
+def embedding(ids, weight):
+    """Rows `ids` of weight, with the gradient kernel `embed_grad` (`csrc/moe/moe_kernels.hip`) for what it takes: bf16 rows of up to
+    4096 tokens."""
+    if weight.is_cuda and weight.dtype == torch.bfloat16 and weight.requires_grad and torch.is_grad_enabled() and \
+            ids.dtype == torch.int64 and weight.shape[1] % 8 == 0 and weight.numel() and ids.numel() <= hip_ops().embed_grad_max():
+        return _EmbeddingFn.apply(ids, weight)
+    return F.embedding(ids, weight)
+
+
 # --------------------------------------------------------------------------------------------------- cross entropy
 class _XentFn(torch.autograd.Function):
 

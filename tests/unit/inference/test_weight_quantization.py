@@ -99,6 +99,14 @@ def test_keys_select_modules_and_tied_weights_share_codes(bits):
             _Tied(), {"weight_quantization": {"post_init_quant": {"fc": c, "f": c}}})
 
 
+def test_token_embedding_of_the_models_is_quantized():
+    from deepspeedsyclsupport_amd.models.llama import LlamaConfig, LlamaForCausalLM
+    model = LlamaForCausalLM(LlamaConfig(vocab_size=128, hidden_size=64, intermediate_size=64, num_hidden_layers=1,
+                                         num_attention_heads=2, max_position_embeddings=32))
+    _init_group_wise_weight_quantization(model, {"weight_quantization": {"post_init_quant": {"embed": _cfg(8)}}})
+    assert isinstance(model.model.embed_tokens, QuantizedEmbedding)
+
+
 def test_quantized_initialization_covers_every_layer():
     m = _Tied()
     _init_group_wise_weight_quantization(m, {"weight_quantization": {"quantized_initialization": _cfg(8, 32)}})

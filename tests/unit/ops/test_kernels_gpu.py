@@ -303,6 +303,25 @@ def test_rope_inplace(interleaved):
     torch.testing.assert_close(back, x, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("T,W,V", [(1, 8, 3), (1023, 264, 40), (1025, 2048, 5000), (4096, 2056, 700), (2050, 64, 1), (4097, 64, 300)])
+def test_embedding_gradient(T, W, V):
+    """Ids that repeat once, often, always, around the sizes of a round of ids and a slice of columns, and one token more than the
+    kernel takes; for odd T dy starts 2 bytes off. fp32 sums of n bf16 rows are off by at most n 2^-24 of their magnitudes' sum, the result by 2^-9 of itself."""
+    from deepspeedsyclsupport_amd.ops.transformer import functional as DF
+    ids = torch.randint(0, V, (1, T), device="cuda")
+    w = torch.randn(V, W, device="cuda").bfloat16().requires_grad_(True)
+    dy = torch.randn(T * W + T % 2, device="cuda").bfloat16()[T % 2:].view(1, T, W)
+    y = DF.embedding(ids, w)
+    assert torch.equal(y, w.detach()[ids[0]][None])
+    y.backward(dy)
+    ref = torch.zeros(V, W, device="cuda", dtype=torch.float64).index_add_(0, ids[0], dy[0].double())
+    if T <= 4096:
+        err = T * 2.0**-24 * torch.zeros_like(ref).index_add_(0, ids[0], dy[0].double().abs())
+        assert ((w.grad.double() - ref).abs() <= 2.0**-8 * ref.abs() + err).all()
+    else:
+        torch.testing.assert_close(w.grad.double(), ref, rtol=0.1, atol=0.5)
+
+
 @pytest.mark.parametrize("V", [32000, 50257, 1000])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_cross_entropy(V, dtype):
