@@ -9,8 +9,8 @@ streams (`ops/int8_gemv.py`) — the matrix is re-laid ONCE:
 
     wsh[nb, kq, h, lane, :] = w[16 nb + (lane % 16), 64 kq + 16 (lane // 16) + 8 h : +8]      (2 KB per 16 x 64 tile)
 
-and every 16-byte-per-lane load reads 1 KB contiguous. A product owns all of K, so the norm of its input, bias, residual and
-activation are part of it (`DecodeProduct.finish`): one launch each. With more than `MAX_DECODE_ROWS` token rows (prefill) the
+and every 16-byte-per-lane load reads 1 KB contiguous. The norm of a product's input, bias, residual and
+activation are part of it (`DecodeProduct.finish`): one launch each, two where a wide batch cuts K into parts. With more than `MAX_DECODE_ROWS` token rows (prefill) the
 library GEMM runs on a row-major matrix: the copy kept next to the shuffled one when `keep_row_major` (twice the weight
 memory, sized for 288 GB of HBM), else a temporary un-shuffled right before the GEMM.
 """
@@ -21,8 +21,8 @@ from . import reference
 from .native import hip_ops
 
 # Rows up to which a decoder layer's products take the stream. Every workgroup reads all of x, so the library's blocking wins
-# from there on: layer of a 4096-wide, 14336-deep Llama, 40 rows 125 us against 143 + 17 for its norms and activation, 64 rows
-# 163 against 131 + 17.
+# from there on: layer of a 4096-wide, 14336-deep Llama, 40 rows 110 us against 143 + 17 for its norms and activation, 64 rows
+# (K uncut) 163 against 131 + 17.
 MAX_DECODE_ROWS = 48
 
 
@@ -92,7 +92,7 @@ class DecodeProduct:
         self.weight, self.x, self.bias = weight, x, bias
 
     def finish(self, norm=None, residual=None, act=None, gated=False):
-        """act(rms_norm(x) . w^T + bias) + residual in one launch: `norm` (weight, eps) of the input, `act` an activation code,
+        """act(rms_norm(x) . w^T + bias) + residual in one call: `norm` (weight, eps) of the input, `act` an activation code,
         `gated`: w is [gate | up] (N % 32 == 0) and the result act(gate) up."""
         x, N = self.x, self.weight.shape[0]
         norm_w, eps = norm or (None, 0.0)

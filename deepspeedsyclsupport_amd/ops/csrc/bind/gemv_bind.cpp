@@ -6,7 +6,8 @@ int ds_skinny_gemm(const void*, const void*, const void*, const void*, const voi
                    int, int, int, int, float, hipStream_t);
 int ds_decode_gemm_ok(int, int);
 int ds_decode_gemm(const void*, const void*, const void*, const void*, float, const void*, void*, int, int, int, int, int, float,
-                   hipStream_t);
+                   void*, hipStream_t);
+int64_t ds_decode_gemm_scratch(int, int, int, int, int);
 int ds_skinny_mfma_ok(int, int, int);
 int ds_skinny_mfma(const void*, const void*, const void*, const void*, const void*, const void*, void*, void*, int, int,
                    int, int, int, int, float, hipStream_t);
@@ -55,16 +56,19 @@ Tensor decode_linear_sh(Tensor x, Tensor wsh, int64_t N, std::optional<double> g
   sizes.back() = glu ? N / 2 : N;
   auto y = torch::empty(sizes, x.options());
   const int code = glu ? CLAMPED_GLU : act.has_value() ? UNARY + (int)*act : -1;
+  Tensor part;
+  if (const int64_t bytes = ds_decode_gemm_scratch((int)M, (int)N, (int)K, glu, 0))
+    part = torch::empty({bytes}, x.options().dtype(at::kByte));
   check(ds_decode_gemm(x.data_ptr(), wsh.data_ptr(), nullptr, nullptr, 0.f, nullptr, y.data_ptr(), (int)M, (int)N, (int)K, glu, code,
-                       glu ? (float)*glu_limit : 0.f, stream()), "decode_linear_sh");
+                       glu ? (float)*glu_limit : 0.f, part.defined() ? part.data_ptr() : nullptr, stream()), "decode_linear_sh");
   return y;
 }
-// Whether decode_linear_sh takes a product and is the faster one. Every workgroup reads all of x: over deep contractions the
-// library's blocking wins from 17 rows on ([4096, 14336], us: 24 rows 30 here, 29 there; 40 rows 41 and 33), over short ones
-// the stream up to its 48 ([2048, 5632], 40 rows: 18 and 20; [4096, 4096] 15 and 20).
+// Whether decode_linear_sh takes a product and is the faster one. Every workgroup reads all of x, or its part of it: over deep
+// contractions that are not cut the library's blocking wins from 17 rows on ([4096, 14336] uncut, us: 24 rows 30 here, 29 there; 40
+// rows 41 and 33; cut 25 and 27.5), over short ones the stream up to its 48 ([2048, 5632], 40 rows: 13 and 20; [4096, 4096] 14 and 20).
 bool decode_linear_sh_ok(int64_t M, int64_t N, int64_t K, bool glu) {
-  return M <= 48 && K < ((int64_t)1 << 31) && ds_decode_gemm_ok((int)M, (int)K) && (M <= 16 || K <= 8192) &&
-         (!glu || N % 32 == 0);
+  return M <= 48 && K < ((int64_t)1 << 31) && ds_decode_gemm_ok((int)M, (int)K) && (!glu || N % 32 == 0) &&
+         (M <= 16 || K <= 8192 || ds_decode_gemm_scratch((int)M, (int)N, (int)K, glu, 0) > 0);
 }
 }  // namespace
 

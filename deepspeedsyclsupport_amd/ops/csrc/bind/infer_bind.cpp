@@ -35,7 +35,8 @@ int64_t ds_skinny_i8_mfma_ws_floats(int);
 void ds_skinny_i8_tune(int, int, int);
 int ds_decode_gemm_ok(int, int);
 int ds_decode_gemm(const void*, const void*, const void*, const void*, float, const void*, void*, int, int, int, int, int, float,
-                   hipStream_t);
+                   void*, hipStream_t);
+int64_t ds_decode_gemm_scratch(int, int, int, int, int);
 int ds_unshuffle_sh16(const void*, void*, int, int, hipStream_t);
 void ds_skinny_b16_tune(int, int);
 int ds_dequant_sh(const int8_t*, const float*, void*, int, int, int, hipStream_t);
@@ -472,8 +473,12 @@ Tensor decode_gemm(Tensor x, Tensor wsh, int64_t N, OptT bias, OptT norm_w, doub
   for (const void* p : {(const void*)wsh.data_ptr(), (const void*)x.data_ptr(), np})
     TORCH_CHECK(reinterpret_cast<uintptr_t>(p) % 16 == 0, "decode_gemm: 16-B aligned x / weights");
   auto y = torch::empty({M, cols}, x.options());
+  Tensor part;
+  if (const int64_t bytes = ds_decode_gemm_scratch((int)M, (int)N, (int)K, gated, np != nullptr))
+    part = torch::empty({bytes}, x.options().dtype(at::kByte));
   check(ds_decode_gemm(x.data_ptr(), wsh.data_ptr(), bp, np, (float)eps, rp, y.data_ptr(), (int)M, (int)N, (int)K, gated,
-                       gated || act < 0 ? (int)act : (int)act + 16, (float)limit, stream()), "decode_gemm");
+                       gated || act < 0 ? (int)act : (int)act + 16, (float)limit, part.defined() ? part.data_ptr() : nullptr,
+                       stream()), "decode_gemm");
   return y;
 }
 bool decode_gemm_ok(int64_t M, int64_t K) { return ds_decode_gemm_ok((int)M, (int)K) != 0; }
@@ -597,7 +602,7 @@ void register_inference_ops(pybind11::module& m) {
         py::arg("norm_w") = py::none(), py::arg("eps") = 0.0, py::arg("res") = py::none(), py::arg("gated") = false,
         py::arg("act") = -1, py::arg("limit") = 0.0);
   m.def("unshuffle_sh16", &unshuffle_sh16);
-  m.def("skinny_b16_tune", [](int64_t cfg, int64_t wpc) { ds_skinny_b16_tune((int)cfg, (int)wpc); }, py::arg("cfg"),
+  m.def("skinny_b16_tune", [](int64_t cfg, int64_t parts) { ds_skinny_b16_tune((int)cfg, (int)parts); }, py::arg("cfg"),
         py::arg("wpc") = 0);
   m.def("skinny_finalize_rms", &skinny_finalize_rms);
   m.def("skinny_finalize_gated", &skinny_finalize_gated);

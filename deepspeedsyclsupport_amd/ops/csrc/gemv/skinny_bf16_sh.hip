@@ -11,16 +11,17 @@
 // so each 16-byte-per-lane load reads 1 KB contiguous and IS the A operand of one v_mfma_f32_16x16x32_bf16 (X is
 // loaded with the same k permutation).
 //  * a workgroup owns RB blocks of 16 weight rows over all of K and up to 48 token rows: its eight waves take alternating steps
-//    of 64 columns, straight into registers, and their sums meet in LDS once. No split over workgroups, so no fp32 sums in
-//    memory, no atomics and no second kernel: sums stay in one fixed order and the result leaves as bf16;
+//    of 64 columns, straight into registers, and their sums meet in LDS once. No atomics: sums stay in one fixed order and the
+//    result leaves as bf16, from this launch, or where wide batches cut K into parts (`cut_of`) from a second one;
 //  * the norm costs no pass: y = rs (X w) . W^T with rs the row's 1 / rms, and every workgroup sees all of X anyway. It
 //    multiplies X by the norm's weight on the way to the matrix cores, adds up the squares beside, and scales the sums;
 //  * a gated pair (gate block i, up block i + N / 32) sits in one workgroup: act(gate) up leaves, half of N;
-//  * X is read once per workgroup (from L2), which is what bounds wide batches; RB trades that against workgroups enough.
+//  * X is read once per workgroup (from L2), which is what bounds wide batches; RB and the parts trade that against workgroups
+//    enough.
 // Bound by the weights' read (6.5 TB/s here). Measured, us (the same products as split streams with fp32 atomics and a finalize
 // pass; the floor): 12 rows x [4096, 4096] 9 (14; 5), [4096, 14336] 23 (25; 18), gated [28672, 4096] 38 (45; 36), with the
 // norm 39, [32000, 4096] 42 (51; 40), [2048, 2048] 5.6 (7.6; 1.3). 24 and 40 rows (library GEMM): gated [28672, 4096] with the
-// norm 42 and 50 (52 and 52 without the norm and activation), [4096, 4096] 11 and 15 (20 and 20).
+// norm 42 and 50 (52 and 52 without the norm and activation), [4096, 4096] 12 and 14 (20 and 20).
 // Prefill (more rows) un-shuffles into a row-major temporary for the library GEMM (`ds_unshuffle_sh16`),
 // or uses the row-major copy the caller kept.
 #include "ds_hip.h"
@@ -41,6 +42,8 @@ struct ShArgs {
   float eps;
   int act;             // gated: activation code; else code + DS_ACT_UNARY, or -1
   float limit;         // of the clamped gated activation
+  int parts;           // of K, each with workgroups of its own (1: all of it)
+  f32x4* part;         // their sums [parts][blocks][MT][64], as the accumulators lie
 };
 
 __device__ __forceinline__ float act_any(int a, float x) {
@@ -58,6 +61,32 @@ struct Int {
   static constexpr int value = V;
 };
 
+// Token row `row`, columns n .. n + 3 of a product without a gate: bias, activation, residual
+__device__ __forceinline__ void store_plain(const ShArgs& a, f32x4 v, int row, int n) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int c = n + e;
+    if (c >= a.N) continue;
+    float r = v[e] + (a.bias ? (float)a.bias[c] : 0.f);
+    if (a.act >= 0) r = act_any(a.act - DS_ACT_UNARY, r);
+    if (a.res) r += (float)a.res[(int64_t)row * a.N + c];
+    v[e] = r;
+  }
+  bf16* yr = a.y + (int64_t)row * a.N + n;
+  if (a.N % 4 == 0) {
+    if (n < a.N) {
+      bf16x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (bf16)v[e];
+      *reinterpret_cast<bf16x4*>(yr) = o;
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < a.N) yr[e] = (bf16)v[e];
+  }
+}
+
 template <int MT, int RB, bool NORM, bool GATED>
 __global__ void __launch_bounds__(WAVES * 64, (MT <= 2 ? 4 : 2)) decode_gemm_kernel(ShArgs a) {
   static_assert(!GATED || RB % 2 == 0, "pairs");
@@ -68,6 +97,9 @@ __global__ void __launch_bounds__(WAVES * 64, (MT <= 2 ? 4 : 2)) decode_gemm_ker
   const int lane = threadIdx.x & 63, l16 = lane & 15, q4 = lane >> 4;
   const int wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int K = a.K, KQ = K / 64, NB = (a.N + 15) / 16, HB = a.N / 32;
+  const bool split = !NORM && !GATED && a.parts > 1;
+  const int first = split ? (int)((int64_t)KQ * blockIdx.y / a.parts) : 0,
+            end = split ? (int)((int64_t)KQ * (blockIdx.y + 1) / a.parts) : KQ;  // steps of K
   // block i of this workgroup
   auto block_of = [&](int i) {
     if (!GATED) return (int)blockIdx.x * RB + i;
@@ -105,12 +137,12 @@ __global__ void __launch_bounds__(WAVES * 64, (MT <= 2 ? 4 : 2)) decode_gemm_ker
 #pragma unroll
         for (int i = 0; i < RB; ++i)
           f.w[u][h][i] = __builtin_nontemporal_load(
-              reinterpret_cast<const bf16x8_t*>(wp[i] + (int64_t)min(s0 + WAVES * u, KQ - 1) * 1024 + 512 * h));
+              reinterpret_cast<const bf16x8_t*>(wp[i] + (int64_t)min(s0 + WAVES * u, end - 1) * 1024 + 512 * h));
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int k = min(s0 + WAVES * u, KQ - 1) * 64 + 8 * h;
+        const int k = min(s0 + WAVES * u, end - 1) * 64 + 8 * h;
         if constexpr (NORM) f.norm[u][h] = *reinterpret_cast<const bf16x8_t*>(np + k);
 #pragma unroll
         for (int m = 0; m < MT; ++m) f.x[u][h][m] = *reinterpret_cast<const bf16x8_t*>(xp[m] + k);
@@ -120,7 +152,7 @@ __global__ void __launch_bounds__(WAVES * 64, (MT <= 2 ? 4 : 2)) decode_gemm_ker
   auto products = [&](Steps& f, int s0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (u && s0 + WAVES * u >= KQ) break;
+      if (u && s0 + WAVES * u >= end) break;
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -141,8 +173,8 @@ __global__ void __launch_bounds__(WAVES * 64, (MT <= 2 ? 4 : 2)) decode_gemm_ker
     __builtin_amdgcn_sched_barrier(0);
   };
   constexpr int STRIDE = WAVES * U;
-  int s = wid;
-  if (s < KQ) {
+  int s = first + wid;
+  if (s < end) {
     Steps f0;
     if constexpr (RB <= 2) {  // the next steps' loads run while these are multiplied
       Steps f1;
@@ -150,13 +182,13 @@ __global__ void __launch_bounds__(WAVES * 64, (MT <= 2 ? 4 : 2)) decode_gemm_ker
       for (;;) {
         load(f1, s + STRIDE);
         products(f0, s);
-        if ((s += STRIDE) >= KQ) break;
+        if ((s += STRIDE) >= end) break;
         load(f0, s + STRIDE);
         products(f1, s);
-        if ((s += STRIDE) >= KQ) break;
+        if ((s += STRIDE) >= end) break;
       }
     } else {  // four blocks a step: the workgroups beside this one cover its waits, a second set of registers costs more of them
-      for (; s < KQ; s += STRIDE) {
+      for (; s < end; s += STRIDE) {
         load(f0, s);
         products(f0, s);
       }
@@ -210,35 +242,40 @@ __global__ void __launch_bounds__(WAVES * 64, (MT <= 2 ? 4 : 2)) decode_gemm_ker
       return v;
     };
     f32x4 v = total(j), u = GATED ? total(j + T / 2) : v;
+    if (split) {
+      if (block_of(i) < NB) a.part[(((int64_t)blockIdx.y * NB + block_of(i)) * MT + m) * 64 + lane] = v;
+      continue;
+    }
     if (row >= a.M) continue;
+    if constexpr (!GATED) {
+      store_plain(a, v, row, n);
+      continue;
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int c = n + e;
       if (c >= cols) continue;
       float r = v[e] + (a.bias ? (float)a.bias[c] : 0.f);
-      if constexpr (GATED) {
-        const float g = r, up = u[e] + (a.bias ? (float)a.bias[cols + c] : 0.f);
-        r = a.act == DS_ACT_CLAMPED_GLU ? clamped_glu_f(g, up, a.limit) : act_any(a.act, g) * up;
-      } else if (a.act >= 0) {
-        r = act_any(a.act - DS_ACT_UNARY, r);
-      }
+      const float g = r, up = u[e] + (a.bias ? (float)a.bias[cols + c] : 0.f);
+      r = a.act == DS_ACT_CLAMPED_GLU ? clamped_glu_f(g, up, a.limit) : act_any(a.act, g) * up;
       if (a.res) r += (float)a.res[(int64_t)row * cols + c];
       v[e] = r;
     }
-    bf16* yr = a.y + (int64_t)row * cols + n;
-    if (cols % 4 == 0) {
-      if (n < cols) {
-        bf16x4 o;
+    bf16x4 o;  // (whole blocks of columns)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = (bf16)v[e];
-        *reinterpret_cast<bf16x4*>(yr) = o;
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (n + e < cols) yr[e] = (bf16)v[e];
-    }
+    for (int e = 0; e < 4; ++e) o[e] = (bf16)v[e];
+    if (n < cols) *reinterpret_cast<bf16x4*>(a.y + (int64_t)row * cols + n) = o;
   }
+}
+
+// The parts' sums, always in the same order, and what is fused behind the product
+__global__ void __launch_bounds__(256) decode_gemm_sum_kernel(ShArgs a, int blocks, int mt) {
+  const int64_t per = (int64_t)blocks * mt * 64, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= per) return;
+  f32x4 v = a.part[i];
+  for (int p = 1; p < a.parts; ++p) v += a.part[p * per + i];
+  const int lane = (int)(i & 63), t = (int)(i >> 6), row = 16 * (t % mt) + (lane & 15);
+  if (row < a.M) store_plain(a, v, row, t / mt * 16 + 4 * (lane >> 4));
 }
 
 // Pre-shuffled bf16 -> row-major bf16 [N, K]. One thread per 16-byte lane chunk (8 weights of one row).
@@ -256,12 +293,40 @@ __global__ void __launch_bounds__(256) unshuffle_sh16_kernel(const bf16* __restr
   *reinterpret_cast<bf16x8*>(W + row * KQ * 64 + kq * 64 + 16 * (lane >> 4) + 8 * h) = v;
 }
 
-int g_blocks = 0;
+int g_blocks = 0, g_parts = 0;
+
+struct Cut {
+  int blocks, parts;  // blocks of 16 weight rows per workgroup, parts of K
+};
+// One block, until the blocks fill the chip's 256 CUs one and a half times (12 rows, us with one / two: [3072, 2048] 5.7 / 6.8, [4096,
+// 14336] 23 / 30; [6144, 4096] 15 / 11). Then two, and with more than 16 token rows four from 1024 blocks on (24 rows x [32000, 4096]
+// 48 with two, 46 with four; 12 rows 42 and 45). Gated pairs take four from 512 on ([11264, 2048] 13.0 with two, 11.0 with
+// four; [28672, 4096] 41 and 38).
+// More than 16 token rows of 4096 and more over fewer blocks: what a CU can read (30 bytes a nanosecond) bounds one block's workgroup,
+// and of that most is X. Several blocks share the reading, and parts of K keep the workgroups at 256; the parts' sums are a launch of
+// 4 us. 48 rows, us with one block and with this: [4096, 4096] 16.3 and 14.6, [4096, 14336] 45 and 28, [2048, 5632] 20.6 and 13.5,
+// [5120, 5120] 37 and 23 (two blocks, one part); 17 rows 10.9 and 11.4, 27 and 24, 12.3 and 10.0, 20.5 and 15.1. Over 2048 the launch
+// costs what it gives ([2048, 2048] 10.2 and 9.9). Four blocks for 33 rows and more of 8192 ([4096, 14336] 33 with two; 17 rows 24.6
+// with four, 23.6 with two).
+Cut cut_of(int M, int N, int K, bool gated, bool norm) {
+  const int blocks = gated ? N / 16 : (N + 15) / 16, mt = (M + 15) / 16;
+  int rb = blocks < 384 ? 1 : 2;
+  if (gated ? blocks >= 512 : mt > 1 && blocks >= 1024) rb = 4;
+  const bool plain = !gated && !norm, cut = plain && mt > 1 && K >= 4096 && blocks < 384;
+  if (cut) rb = mt == 3 && K >= 8192 ? 4 : 2;
+  if (g_blocks) rb = g_blocks >= 4 ? 4 : g_blocks == 3 ? 2 : g_blocks;
+  if (gated && rb < 2) rb = 2;
+  if (!gated && mt == 1 && rb == 4) rb = 2;
+  const int groups = (blocks + rb - 1) / rb;
+  int parts = cut ? max(min(min(256 / groups, K / 1024), 8), 1) : 1;  // (K / 1024: two steps a wave)
+  if (g_parts && plain) parts = min(g_parts, K / 64);
+  return {rb, parts};
+}
 
 template <int MT, int RB>
 int launch(const ShArgs& a, bool gated, hipStream_t st) {
   const int blocks = gated ? a.N / 16 : (a.N + 15) / 16;
-  const dim3 grid((blocks + RB - 1) / RB), threads(WAVES * 64);
+  const dim3 grid((blocks + RB - 1) / RB, a.parts), threads(WAVES * 64);
   if (gated) {
     if constexpr (RB > 1) {
       if (a.norm_w) hipLaunchKernelGGL((decode_gemm_kernel<MT, RB, true, true>), grid, threads, 0, st, a);
@@ -271,16 +336,23 @@ int launch(const ShArgs& a, bool gated, hipStream_t st) {
     if (a.norm_w) hipLaunchKernelGGL((decode_gemm_kernel<MT, RB, true, false>), grid, threads, 0, st, a);
     else hipLaunchKernelGGL((decode_gemm_kernel<MT, RB, false, false>), grid, threads, 0, st, a);
   }
+  if (a.parts > 1) hipLaunchKernelGGL(decode_gemm_sum_kernel, dim3((blocks * MT * 64 + 255) / 256), dim3(256), 0, st, a, blocks, MT);
   DS_CHECK_LAUNCH();
   return 0;
 }
 
 }  // namespace
 
-// Forces blocks per workgroup (1, 2, 4, where the product has such a kernel; 0: by the rule below).
-extern "C" void ds_skinny_b16_tune(int cfg, int) { g_blocks = cfg; }
+// Forces blocks per workgroup (1, 2, 4, where the product has such a kernel) and parts of K; 0: by the rule above.
+extern "C" void ds_skinny_b16_tune(int cfg, int parts) { g_blocks = cfg; g_parts = parts; }
 
 extern "C" int ds_decode_gemm_ok(int M, int K) { return M >= 1 && M <= 48 && K >= 64 && K % 64 == 0; }
+
+// Bytes of scratch memory that ds_decode_gemm wants for a product (0: none)
+extern "C" int64_t ds_decode_gemm_scratch(int M, int N, int K, int gated, int norm) {
+  const int parts = cut_of(M, N, K, gated, norm).parts;
+  return parts > 1 ? (int64_t)parts * ((N + 15) / 16) * ((M + 15) / 16) * 1024 : 0;
+}
 
 extern "C" int ds_unshuffle_sh16(const void* Wsh, void* W, int N, int K, hipStream_t st) {
   if (N <= 0 || K % 64) return (int)hipErrorInvalidValue;
@@ -294,29 +366,21 @@ extern "C" int ds_unshuffle_sh16(const void* Wsh, void* W, int N, int K, hipStre
 
 // X [M, K] bf16 (M <= 48, K % 64 == 0), Wsh in the shuffled layout above (N padded to a multiple of 16). norm_w [K] or null: X
 // is RMS-normed by it first. bias [N], res [M, N] or null. gated: N / 2 columns act(gate) up (N % 32 == 0); else act: a
-// code + DS_ACT_UNARY, or -1.
+// code + DS_ACT_UNARY, or -1. part: ds_decode_gemm_scratch bytes.
 extern "C" int ds_decode_gemm(const void* X, const void* Wsh, const void* bias, const void* norm_w, float eps, const void* res,
-                              void* Y, int M, int N, int K, int gated, int act, float limit, hipStream_t st) {
+                              void* Y, int M, int N, int K, int gated, int act, float limit, void* part, hipStream_t st) {
   if (!ds_decode_gemm_ok(M, K) || N <= 0 || (gated && N % 32)) return (int)hipErrorInvalidValue;
+  const Cut cut = cut_of(M, N, K, gated, norm_w != nullptr);
+  if (cut.parts > 1 && !part) return (int)hipErrorInvalidValue;
   const ShArgs a{(const bf16*)X, (const bf16*)Wsh, (const bf16*)bias, (const bf16*)norm_w, (const bf16*)res, (bf16*)Y, M, N, K,
-                 eps, act, limit};
-  // Blocks of 16 weight rows per workgroup. One, until the blocks fill the chip's 256 CUs one and a half times (12 rows, us with
-  // one / two: [3072, 2048] 5.7 / 6.8, [4096, 14336] 23 / 30; [6144, 4096] 15 / 11). Then two, and with more than 16 token rows
-  // four from 1024 blocks on (24 rows x [32000, 4096] 48 with two, 46 with four; 12 rows 42 and 45). Gated pairs take four
-  // from 512 on ([11264, 2048] 13.0 with two, 11.0 with four; [28672, 4096] 41 and 38).
-  const int mt = (M + 15) / 16, blocks = gated ? N / 16 : (N + 15) / 16;
-  int rb = blocks < 384 ? 1 : 2;
-  if (gated ? blocks >= 512 : mt > 1 && blocks >= 1024) rb = 4;
-  if (g_blocks) rb = g_blocks >= 4 ? 4 : g_blocks == 3 ? 2 : g_blocks;
-  if (gated && rb < 2) rb = 2;
-  if (!gated && mt == 1 && rb == 4) rb = 2;
+                 eps, act, limit, cut.parts, (f32x4*)part};
 #define GO(MT)                                  \
-  switch (rb) {                                 \
+  switch (cut.blocks) {                         \
     case 1: return launch<MT, 1>(a, gated, st); \
     case 2: return launch<MT, 2>(a, gated, st); \
     default: return launch<MT, 4>(a, gated, st); \
   }
-  switch (mt) {
+  switch ((M + 15) / 16) {
     case 1: GO(1)
     case 2: GO(2)
     default: GO(3)

@@ -116,3 +116,25 @@ def test_bf16_sh_products_with_what_stands_around_them_gpu(M, N, K, gated, norm)
     assert y.shape == ref.shape
     # (the activation's own exp is good to a few 2^-24, its error stays below that of the stored result)
     assert ((y.double() - ref).abs() <= 2.0**-8 * ref.abs() + 2 * err + 2.0**-20 * (1 + ref.abs().max())).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K", [(4096, 4096), (16, 4160), (37, 8192), (500, 9216), (5120, 4096), (6128, 4096), (6144, 4096), (2050, 4032)])
+@pytest.mark.parametrize("M", [17, 32, 33, 48])
+def test_wide_batches_cut_the_contraction(N, K, M):
+    """Few and ragged weight rows, parts of unequal length, both sides of the sizes from which K is cut, with bias, activation and
+    residual. The fp32 sum is off by at most K 2^-24 of its magnitudes' sum (sqrt(K) of that in truth), the result by 2^-9 of itself
+    twice (silu passes on at most 1.1 of an error)."""
+    torch.manual_seed(N + K + M)
+    x, w = torch.randn(M, K, device="cuda").bfloat16(), (torch.randn(N, K, device="cuda") * 0.05).bfloat16()
+    b, res = torch.randn(N, device="cuda").bfloat16(), torch.randn(M, N, device="cuda").bfloat16()
+    bw = Bf16Weight(w)
+    z = x.double() @ w.double().t()
+    err = K**0.5 * 2.0**-24 * (x.double().abs() @ w.double().abs().t())
+    for bias, act, r in ((None, None, None), (b, None, res), (b, 0, res)):
+        want = z if bias is None else z + b.double()
+        want = torch.nn.functional.silu(want) if act == 0 else want
+        want = want if r is None else want + r.double()
+        y = bw.raw(x, bias).finish(residual=r, act=act)
+        assert ((y.double() - want).abs() <= 1.1 * err + 2.0**-8 * want.abs() + 1e-6).all()
+        assert torch.equal(y, bw.raw(x, bias).finish(residual=r, act=act))
