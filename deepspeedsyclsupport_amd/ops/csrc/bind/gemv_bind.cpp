@@ -1,4 +1,4 @@
-// Module of the bf16 decode products (up to 64 token rows) of the hybrid decoders, with activation epilogues.
+// Module of the bf16 decode products (up to 48 token rows) of the hybrid decoders, with activation epilogues.
 #include "bind_util.h"
 
 extern "C" {
@@ -41,14 +41,14 @@ Tensor decode_linear(Tensor x, Tensor w, std::optional<double> glu_limit, std::o
   return y;
 }
 
-// The same for M <= 64 over a weight in the shuffled decode layout (ops/bf16_gemv.py: preshuffle16), w [N, K], K % 64 == 0;
+// The same for M <= 48 over a weight in the shuffled decode layout (ops/bf16_gemv.py: preshuffle16), w [N, K], K % 64 == 0;
 // with a limit: N % 32 == 0
 Tensor decode_linear_sh(Tensor x, Tensor wsh, int64_t N, std::optional<double> glu_limit, std::optional<int64_t> act) {
   need(x, "x"); need(wsh, "wsh");
   const int64_t K = x.size(-1), M = x.numel() / K, NB = (N + 15) / 16;
   const bool glu = glu_limit.has_value();
   TORCH_CHECK(x.scalar_type() == at::kBFloat16 && wsh.scalar_type() == at::kBFloat16 && wsh.numel() == NB * 16 * K &&
-              ds_decode_gemm_ok((int)M, (int)K), "decode_linear_sh: up to 64 bf16 rows, K % 64 == 0");
+              ds_decode_gemm_ok((int)M, (int)K), "decode_linear_sh: up to 48 bf16 rows, K % 64 == 0");
   TORCH_CHECK(NB * K < ((int64_t)1 << 40) && N < ((int64_t)1 << 31) / 16, "decode_linear_sh: matrix too large");
   TORCH_CHECK(!(glu && act.has_value()), "decode_linear_sh: one epilogue");
   TORCH_CHECK(!glu || N % 32 == 0, "decode_linear_sh: [gate | up] of whole blocks of 16 rows");

@@ -452,7 +452,7 @@ const void* opt_bf16(const OptT& t, int64_t numel, const char* what) {
   return t->data_ptr();
 }
 
-// bf16 product over the pre-shuffled weight (ops/bf16_gemv.py: preshuffle16): x [M, K] bf16 (M <= 64), wsh bf16 [ceil(N/16), K/64,
+// bf16 product over the pre-shuffled weight (ops/bf16_gemv.py: preshuffle16): x [M, K] bf16 (M <= 48), wsh bf16 [ceil(N/16), K/64,
 // 2, 64, 8] -> y [M, N] bf16. norm_w [K]: x is RMS-normed first. bias [N]; res [M, N] is added at the end. gated: w is a
 // fused [gate | up] weight, the result act(gate) up [M, N / 2] (limit: of the clamped activation); else act: an activation
 // code of the result, or -1.
