@@ -1,10 +1,9 @@
-// CDNA4 flash-attention backward (training), bf16, head dim 128, GQA-native, causal / full / block-sparse.
+// CDNA4 flash-attention backward (training), bf16, head dim 128, GQA-native, causal / full. Block-sparse: sparse_bwd.hip.
 //
 // Reference counterparts: the training attention backward of the BERT kernel (`csrc/transformer/softmax_kernels.cu:
-// 443-592` softmax backward + the strided-batched dQ/dK/dV GEMMs of `csrc/transformer/ds_transformer_cuda.cpp:302+`)
-// and the block-sparse Triton backward (`deepspeed/ops/sparse_attention/matmul.py:605` DSD/SDD transposes,
-// `softmax.py:213`). Both materialise the [B,H,S,S] probabilities; this kernel recomputes them from the forward's
-// natural-log LSE instead (FlashAttention-2 style), laid out for gfx950:
+// 443-592` softmax backward + the strided-batched dQ/dK/dV GEMMs of `csrc/transformer/ds_transformer_cuda.cpp:302+`),
+// which materialises the [B,H,S,S] probabilities; this kernel recomputes them from the forward's natural-log LSE instead
+// (FlashAttention-2 style), laid out for gfx950:
 //
 //  * one workgroup = 8 waves = 256 keys of one (batch, kv head); wave w owns keys 32w..32w+31 and keeps dK^T and dV^T
 //    of its keys (2 x 4 x 32x32 fp32 tiles = 128 accumulator registers) while the workgroup sweeps every query head of
@@ -29,14 +28,8 @@
 //  * causal: waves whose 32 keys lie entirely above a tile skip it, the dQ product stops at the diagonal, workgroups
 //    with the most tiles (low key blocks) start first, and each (batch, kv head)'s key blocks share an XCD (Q / dO
 //    reuse in L2);
-//  * block-sparse: each workgroup walks only the 32-row query tiles its key block meets in the layout (a host-built
-//    column plan) and masks by the 32 bits that the plan holds per tile (2 x 16 rows, 16 x 16 keys) — cost scales with the
-//    layout density. List, masks and the per-key bias reach the loop through scalar loads and registers: a vector load in
-//    there waits for everything in flight ahead of it, the dQ atomics of waves 0..3 and the tiles of waves 4..7 included;
-//  * a sweep that is much longer than the others (the global columns of BigBird), or too few of them to fill the chip
-//    (short sequences of grouped-query models), is cut into parts that leave fp32 dK / dV in a workspace; a second launch
-//    adds them up in a fixed order. B2 H8 S16384, BigBird of 64-key blocks with padding: 1641 -> 506 us, now bound by the
-//    dQ atomics (below); B3 Hq16 Hk4 S1000 causal (48 workgroups uncut): 313 -> 103 us.
+//  * too few sweeps to fill the chip (short sequences of grouped-query models) are cut into parts that leave fp32 dK / dV in a
+//    workspace; a second launch adds them up in a fixed order. B3 Hq16 Hk4 S1000 causal (48 workgroups uncut): 313 -> 103 us.
 // Measured (tools/bench_flash_bwd.py, profiles/flash_bwd_bench_r2_final.jsonl): B8 H32 S4096 D128 causal 4.2-4.3 ms
 // (round-2 start: 4.58). SQ PMC of the round-2 start: ~29 % MFMA busy, ~9 VALU per MFMA -- the VALU issue slots, not
 // the matrix pipe, are what the trims above (packed converts, pre-scaled row constants, uniform mask skip) buy back.
@@ -141,36 +134,16 @@ struct BwdArgs {
   int64_t qsb, qsh, qss, ksb, ksh, kss, vsb, vsh, vss, osb, osh, oss, dksb, dksh, dkss, dvsb, dvsh, dvss;
   float c;      // softmax scale * log2(e)
   float scale;
-  // block-sparse column plan, each for lut_heads (1 or Hk) kv heads: qtiles [nkb, maxt] = (query head within the kv group
-  // << 16 | 32-row query tile) for every tile key block kb meets, qmasks [nkb, maxt] (bit 16 r + k: its rows 16r.. see keys
-  // 16k.. of the block), work [nwork, 4] = (key block or -1, first entry of its list, entries, part slot or -1), merges
-  // [nmerge, 4] = (key block or -1, first slot, slots, 0)
-  const int* qtiles;
-  const int* qmasks;
-  const int* work;
-  const int* merges;
-  int maxt, lut_heads, nwork, nmerge;
   // parts: dense sweeps are cut into nsplit of them (part p of key block kb: slot kb * nsplit + p)
   int nsplit, nslots;
-  f32x4* part;  // [B * Hk or, with lists per head, B, nslots, 32, 512]
-  // additive score biases of the block-sparse path (see flash_fwd.hip SparseLut), any may be null
-  const float *kbias, *abias, *rpe;
-  int64_t kb_stride, ab_stride, rpe_hs, rpe_rs;
-  // 1 = kbias, 2 = abias, 4 = rpe are real; with any of them set the others point at one zero float and their
-  // strides and key multipliers (ab_km / rpe_km) are 0, so the kernel loads unconditionally (a uniform branch around
-  // these loads runs into a hipcc ROCm 7.2 code generation error)
-  int bias_flags, kb_km, ab_km, rpe_km;
+  f32x4* part;  // [B * Hk, nslots, 32, 512]
 };
-
-// read-only and wave-uniform: scalar loads, whatever the kernel writes or clobbers in between
-typedef __attribute__((address_space(4))) const int const_int;
-__device__ __forceinline__ const_int* uniform_ints(const int* p) { return (const_int*)(uintptr_t)p; }
 
 // NW waves per workgroup, each owning KPW = 256 / NW keys (NC = KPW / 32 column tiles of the S / dP accumulators).
 // NW = 4: one wave per SIMD with the whole 512-register file (dK^T/dV^T of 64 keys = 256 accumulator registers),
 // every wave also computes one 32-column slice of the tile's dQ; NW = 8: two waves per SIMD, 32 keys each, waves
 // 0..3 compute dQ.
-template <int NW, bool CAUSAL, bool SPARSE, int BIASED = 0>
+template <int NW, bool CAUSAL>
 __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
   constexpr int NTHR = NW * 64, KPW = KB / NW, NC = KPW / 32;
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -180,19 +153,10 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
   const int S = a.S;
   const int nkb = (S + KB - 1) / KB;
   const int logical = xcd_remap(blockIdx.x, gridDim.x);
-  const int per_bh = SPARSE ? a.nwork : nkb * a.nsplit;
+  const int per_bh = nkb * a.nsplit;
   const int bh = logical / per_bh, wi = logical % per_bh;
   const int b = bh / a.Hk, hk = bh % a.Hk, rep = a.Hq / a.Hk;
-  int kb = wi / a.nsplit, it0 = 0, slot = -1;  // causal: low key blocks (most tiles) first within a head
-  int n_it = 0;
-  if constexpr (SPARSE) {
-    const_int* wk = uniform_ints(a.work) + ((int64_t)(a.lut_heads == 1 ? 0 : hk) * a.nwork + wi) * 4;
-    kb = wk[0];
-    it0 = wk[1];
-    n_it = wk[2];
-    slot = wk[3];
-    if (kb < 0) return;  // (heads with fewer parts than the others)
-  }
+  const int kb = wi / a.nsplit;  // causal: low key blocks (most tiles) first within a head
   const int k0 = kb * KB;
   const int ntq = (S + QT - 1) / QT;
 
@@ -207,29 +171,12 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
   // ------------------------------------------------------------------ iteration space: (query head, query tile)
   const int t0 = CAUSAL ? k0 / QT : 0;
   const int per_head_dense = ntq - t0;
-  const_int* lut = nullptr;
-  const_int* lutm = nullptr;
-  if constexpr (SPARSE) {
-    const int64_t at = ((int64_t)(a.lut_heads == 1 ? 0 : hk) * nkb + kb) * a.maxt + it0;
-    lut = uniform_ints(a.qtiles) + at;
-    lutm = uniform_ints(a.qmasks) + at;
-    it0 = 0;
-  } else {
-    const int all = rep * per_head_dense, part = wi % a.nsplit;
-    it0 = (int)((int64_t)all * part / a.nsplit);
-    n_it = (int)((int64_t)all * (part + 1) / a.nsplit) - it0;
-    if (a.nsplit > 1) slot = wi;
-  }
-  // it -> (query head, query tile); the sparse list holds (head-in-group << 16 | tile) per (kv head, key block)
+  const int all = rep * per_head_dense, part = wi % a.nsplit, it0 = (int)((int64_t)all * part / a.nsplit);
+  const int n_it = (int)((int64_t)all * (part + 1) / a.nsplit) - it0, slot = a.nsplit > 1 ? wi : -1;
+  // it -> (query head, query tile)
   auto tile_at = [&](int it, int& hq, int& qt) {
-    if constexpr (SPARSE) {
-      const int code = lut[it];
-      hq = hk * rep + (code >> 16);
-      qt = code & 0xffff;
-    } else {
-      hq = hk * rep + (it0 + it) / per_head_dense;
-      qt = t0 + (it0 + it) % per_head_dense;
-    }
+    hq = hk * rep + (it0 + it) / per_head_dense;
+    qt = t0 + (it0 + it) % per_head_dense;
   };
 
   // ------------------------------------------------------------------ staging of one (Q, dO, lse, delta) tile
@@ -343,22 +290,12 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) dk[c][dt][r] = dv[c][dt][r] = 0.f;
 
-  float kbv[NC];  // BIASED: the per-key bias of this lane's keys, in units of log2
-#pragma unroll
-  for (int c = 0; c < NC; ++c)
-    kbv[c] = BIASED == 0 ? 0.f : a.kbias[(int64_t)b * a.kb_stride + (int64_t)min(kw0 + 32 * c + l32, S - 1) * a.kb_km] *
-                                     1.4426950408889634f;
-
   // K image / V rows landed before the DMA starts: consuming the V fragments here makes hipcc's own waitcnt pass
   // retire them now instead of waiting vmcnt(0) (= draining the DMA) at their first use inside the tile loop
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) asm volatile("" : : "v"(vf[c][kk]));
-  if constexpr (BIASED != 0) {
-#pragma unroll
-    for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(kbv[c]));
-  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   if (n_it > 0) stage(0, 0);
   if (n_it > 1) stage(1, 1);
@@ -380,7 +317,6 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
     char* DSc = DSimg + cur * DS_BYTES;
 
     // ---------------- which of this wave's 32-key slabs meet the tile? keep[c] bit r: accumulator row r unmasked
-    const unsigned tmask = SPARSE ? (unsigned)lutm[it] : 0xffffffffu;
     bool act[NC];
     unsigned keep[NC];
 #pragma unroll
@@ -388,12 +324,6 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
       const int ks = kw0 + 32 * c, mykey = ks + l32;
       act[c] = ks < S && (!CAUSAL || ks <= q0 + QT - 1);
       keep[c] = mykey < S ? 0xffffu : 0u;
-      if constexpr (SPARSE) {  // registers 0..7 are rows 0..15 of the tile, 8..15 rows 16..31
-        const unsigned mine = tmask >> ((ks - k0) / 16);
-        act[c] = act[c] && (mine & 0x00030003u) != 0;
-        const unsigned lane_bits = mine >> (l32 >> 4);
-        keep[c] &= ((lane_bits & 1u) ? 0x00ffu : 0u) | ((lane_bits & 0x10000u) ? 0xff00u : 0u);
-      }
       if (q0 + QT > S) {  // padded query rows of the last tile
 #pragma unroll
         for (int r = 0; r < 16; ++r)
@@ -456,27 +386,7 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
       // the per-element select costs 4 VALU and the VALU issue slots are the co-bottleneck beside the MFMAs.
       float pf[16], df[16];
       const bool need_mask = keep[c] != 0xffffu;
-      if constexpr (BIASED != 0) {
-        // P = exp2(c * S' + log2(e) * bias): the per-key bias is one constant per lane, attention-mask / relative
-        // position values are read per (query row, key) — consecutive lanes read consecutive keys of one row.
-        // BIASED == 1: per-key bias only (BERT padding masks); 2: all three terms.
-        const int mykey = min(kw0 + 32 * c + l32, S - 1);
-        const float l2e = 1.4426950408889634f;
-        const float* abp = a.abias + (int64_t)mykey * a.ab_km;
-        const float* rpp = a.rpe + (int64_t)hq * a.rpe_hs + (int64_t)mykey * a.rpe_km;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float bv = kbv[c];
-          if constexpr (BIASED == 2) {
-            const int qr = min(q0 + crow(r, h), S - 1);
-            bv = fmaf(abp[(int64_t)qr * a.ab_stride] + rpp[(int64_t)qr * a.rpe_rs], l2e, bv);
-          }
-          float p = __builtin_amdgcn_exp2f(fmaf(s[r], a.c, bv));
-          if (!((keep[c] >> r) & 1u)) p = 0.f;
-          pf[r] = p;
-          df[r] = p * dp[r];
-        }
-      } else if (__any(need_mask)) {
+      if (__any(need_mask)) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           float p = __builtin_amdgcn_exp2f(s[r] * a.c);
@@ -557,29 +467,18 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
       auto ld_b = [&](int s2) {
         return join(tr_read(Kimg + 4096 * s2 + kqoff[0]), tr_read(Kimg + 4096 * s2 + kqoff[1]));
       };
-      if constexpr (SPARSE) {
-#pragma unroll 1
-        for (int slab = 0; slab < 8; ++slab) {
-          if (!((tmask >> (2 * slab)) & 0x00030003u)) continue;
-          const bf16x8_t a0 = ld_a(2 * slab), b0 = ld_b(2 * slab), a1 = ld_a(2 * slab + 1), b1 = ld_b(2 * slab + 1);
-          dq = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b0, dq, 0, 0, 0);
-          dq = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, dq, 0, 0, 0);
-          ++nks;
-        }
-      } else {
-        // keys up to the diagonal (causal) / the sequence end, as 16-key MFMA steps
-        int kmax = min(KB, S - k0);
-        if (CAUSAL) kmax = min(kmax, q0 + QT - k0);
-        nks = (kmax + 15) >> 4;
-        if (nks == KB / 16) {  // every key block but the diagonal one: straight-line, scheduled by hipcc
+      // keys up to the diagonal (causal) / the sequence end, as 16-key MFMA steps
+      int kmax = min(KB, S - k0);
+      if (CAUSAL) kmax = min(kmax, q0 + QT - k0);
+      nks = (kmax + 15) >> 4;
+      if (nks == KB / 16) {  // every key block but the diagonal one: straight-line, scheduled by hipcc
 #pragma unroll
-          for (int s2 = 0; s2 < KB / 16; ++s2)
-            dq = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld_a(s2), ld_b(s2), dq, 0, 0, 0);
-        } else {
+        for (int s2 = 0; s2 < KB / 16; ++s2)
+          dq = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld_a(s2), ld_b(s2), dq, 0, 0, 0);
+      } else {
 #pragma unroll 1
-          for (int s2 = 0; s2 < nks; ++s2)
-            dq = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld_a(s2), ld_b(s2), dq, 0, 0, 0);
-        }
+        for (int s2 = 0; s2 < nks; ++s2)
+          dq = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld_a(s2), ld_b(s2), dq, 0, 0, 0);
       }
       if (nks > 0) {
         // lane part of the 16 destination rows, laundered so that hipcc forms each address next to its atomic
@@ -604,7 +503,7 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
   // ------------------------------------------------------------------ epilogue: dK = scale * dK^T^T, dV
   if (slot >= 0) {  // a part of the sweep: the accumulators as they are, 16 bytes per thread and piece
     static_assert(NC == 1 && NTHR == 512, "the parts' layout");
-    f32x4* po = a.part + ((int64_t)(a.lut_heads == 1 ? bh : b) * a.nslots + slot) * (32 * NTHR) + tid;
+    f32x4* po = a.part + ((int64_t)bh * a.nslots + slot) * (32 * NTHR) + tid;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -647,16 +546,9 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
 // thread layout is the main kernel's).
 __global__ void __launch_bounds__(512) flash_bwd_merge_kernel(BwdArgs a) {
   const int bh = blockIdx.y, b = bh / a.Hk, hk = bh % a.Hk, mi = blockIdx.x / 8, dt = blockIdx.x & 3, isv = (blockIdx.x >> 2) & 1;
-  int kb = mi, slot0 = mi * a.nsplit, n = a.nsplit;
-  if (a.merges != nullptr) {
-    const int* me = a.merges + ((int64_t)(a.lut_heads == 1 ? 0 : hk) * a.nmerge + mi) * 4;
-    kb = me[0];
-    slot0 = me[1];
-    n = me[2];
-    if (kb < 0) return;
-  }
+  const int kb = mi, slot0 = mi * a.nsplit, n = a.nsplit;
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, key = kb * KB + 32 * (tid >> 6) + (lane & 31);
-  const f32x4* src = a.part + ((int64_t)(a.lut_heads == 1 ? bh : b) * a.nslots + slot0) * (32 * 512) + (16 * isv + 4 * dt) * 512 + tid;
+  const f32x4* src = a.part + ((int64_t)bh * a.nslots + slot0) * (32 * 512) + (16 * isv + 4 * dt) * 512 + tid;
   f32x4 acc[4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) acc[g] = src[g * 512];
@@ -730,32 +622,22 @@ __global__ void __launch_bounds__(256) flash_bwd_post_kernel(const float* __rest
   *reinterpret_cast<bf16x8*>(dq + bb * sb + hh * sh + (int64_t)q * ss + sub * 8) = r;
 }
 
-template <int NW, bool C, bool SP, int BI = 0>
+template <int NW, bool C>
 int launch_main(const BwdArgs& a, hipStream_t st) {
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_bwd_kernel<NW, C, SP, BI>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes<NW>());
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_bwd_kernel<NW, C>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              lds_bytes<NW>());
     attr = true;
   }
   const int nkb = (a.S + KB - 1) / KB;
-  const int grid = a.B * a.Hk * (SP ? a.nwork : nkb * a.nsplit);
-  hipLaunchKernelGGL((flash_bwd_kernel<NW, C, SP, BI>), dim3(grid), dim3(NW * 64), lds_bytes<NW>(), st, a);
+  hipLaunchKernelGGL((flash_bwd_kernel<NW, C>), dim3(a.B * a.Hk * nkb * a.nsplit), dim3(NW * 64), lds_bytes<NW>(), st, a);
   DS_CHECK_LAUNCH();
-  const int nmerge = SP ? a.nmerge : (a.nsplit > 1 ? nkb : 0);
-  if (nmerge > 0) {
-    hipLaunchKernelGGL(flash_bwd_merge_kernel, dim3(nmerge * 8, a.B * a.Hk), dim3(512), 0, st, a);
+  if (a.nsplit > 1) {
+    hipLaunchKernelGGL(flash_bwd_merge_kernel, dim3(nkb * 8, a.B * a.Hk), dim3(512), 0, st, a);
     DS_CHECK_LAUNCH();
   }
   return 0;
-}
-
-template <int NW>
-int launch_mode(const BwdArgs& a, int mode, hipStream_t st) {
-  if (mode == 2 && a.bias_flags == 1) return launch_main<NW, false, true, 1>(a, st);
-  if (mode == 2 && a.bias_flags) return launch_main<NW, false, true, 2>(a, st);
-  return mode == 1 ? launch_main<NW, true, false>(a, st)
-                   : (mode == 2 ? launch_main<NW, false, true>(a, st) : launch_main<NW, false, false>(a, st));
 }
 
 }  // namespace
@@ -763,9 +645,8 @@ int launch_mode(const BwdArgs& a, int mode, hipStream_t st) {
 // Strides are (batch, head, seq) in elements, unit last stride everywhere, all bf16 rows 16-B aligned.
 // q/o/dout/dq [B,Hq,S,128], k/v/dk/dv [B,Hk,S,128], lse [B,Hq,S] natural-log (flash_fwd's), workspace:
 // delta [2*B*Hq*S] fp32 (the pre kernel's -delta and -LSE/scale rows) and dqacc [B*Hq*S*128] fp32.
-// mode: 0 full, 1 causal (top-left), 2 block-sparse (plan: see BwdArgs). part: the workspace of the parts,
-// B * Hk * slots * 256 KB, slots = ds_flash_bwd_split(..) * key blocks of 256 for the dense modes (none if it is 1) or nslots; with
-// lists per head nslots counts those of all heads: B * nslots * 256 KB.
+// mode: 0 full, 1 causal (top-left). part: the workspace of the parts, B * Hk * slots * 256 KB, slots = ds_flash_bwd_split(..) * key
+// blocks of 256 (none if the split is 1).
 
 // Parts per key block of a dense sweep. A workgroup takes a CU for itself, so anything below 256 of them idles the rest;
 // parts shorter than 4 tiles would spend their time on the K image and the accumulators. Measured, us, causal, for parts
@@ -782,16 +663,10 @@ extern "C" int ds_flash_bwd(const void* q, const void* k, const void* v, const v
                             const float* lse, float* delta, float* dqacc, void* dq, void* dk, void* dv, int B, int Hq,
                             int Hk, int S, const int64_t* qs, const int64_t* ks, const int64_t* vs, const int64_t* os,
                             const int64_t* dos, const int64_t* dqs, const int64_t* dks, const int64_t* dvs,
-                            float scale, int mode, const int* qtiles, const int* qmasks, const int* work, const int* merges,
-                            int maxt, int lut_heads, int nwork, int nmerge, int nslots, float* part, int bias_flags,
-                            const float* kbias, int64_t kb_stride, const float* abias, int64_t ab_stride, const float* rpe,
-                            int64_t rpe_hs, int64_t rpe_rs, hipStream_t st) {
+                            float scale, int mode, float* part, hipStream_t st) {
   if (Hk <= 0 || Hq % Hk != 0 || S <= 0 || B <= 0) return (int)hipErrorInvalidValue;
-  if (mode == 2 && (qtiles == nullptr || qmasks == nullptr || work == nullptr || (lut_heads != 1 && lut_heads != Hk) ||
-                    nwork <= 0 || (nmerge > 0 && (merges == nullptr || nslots <= 0))))
-    return (int)hipErrorInvalidValue;
-  const int nsplit = mode == 2 ? 1 : ds_flash_bwd_split(B, Hq, Hk, S);
-  if ((nsplit > 1 || (mode == 2 && nmerge > 0)) && part == nullptr) return (int)hipErrorInvalidValue;
+  const int nsplit = ds_flash_bwd_split(B, Hq, Hk, S);
+  if (nsplit > 1 && part == nullptr) return (int)hipErrorInvalidValue;
   const int64_t rows = (int64_t)B * Hq * S;
   const int pgrid = (int)((rows + 15) / 16);
   hipLaunchKernelGGL(flash_bwd_pre_kernel, dim3(pgrid), dim3(256), 0, st, (const bf16*)o, (const bf16*)dout, lse,
@@ -809,19 +684,10 @@ extern "C" int ds_flash_bwd(const void* q, const void* k, const void* v, const v
   a.dvsb = dvs[0]; a.dvsh = dvs[1]; a.dvss = dvs[2];
   a.c = scale * 1.4426950408889634f;
   a.scale = scale;
-  a.qtiles = qtiles; a.qmasks = qmasks; a.work = work; a.merges = mode == 2 ? merges : nullptr;
-  a.maxt = maxt; a.lut_heads = lut_heads; a.nwork = nwork; a.nmerge = nmerge;
   a.nsplit = nsplit;
-  a.nslots = mode == 2 ? nslots : nsplit * ((S + KB - 1) / KB);
+  a.nslots = nsplit * ((S + KB - 1) / KB);
   a.part = reinterpret_cast<f32x4*>(part);
-  // biases: block-sparse path only; with any bias present every pointer must be valid (see BwdArgs::bias_flags)
-  if (bias_flags && (mode != 2 || !kbias || !abias || !rpe)) return (int)hipErrorInvalidValue;
-  a.kbias = kbias; a.abias = abias; a.rpe = rpe;
-  a.bias_flags = bias_flags;
-  a.kb_km = bias_flags & 1; a.ab_km = (bias_flags >> 1) & 1; a.rpe_km = (bias_flags >> 2) & 1;
-  a.kb_stride = a.kb_km ? kb_stride : 0; a.ab_stride = a.ab_km ? ab_stride : 0;
-  a.rpe_hs = a.rpe_km ? rpe_hs : 0; a.rpe_rs = a.rpe_km ? rpe_rs : 0;
-  int rc = launch_mode<8>(a, mode, st);
+  const int rc = mode == 1 ? launch_main<8, true>(a, st) : launch_main<8, false>(a, st);
   if (rc) return rc;
   hipLaunchKernelGGL(flash_bwd_post_kernel, dim3(pgrid), dim3(256), 0, st, dqacc, (bf16*)dq, Hq, S, rows, dqs[0],
                      dqs[1], dqs[2], scale);

@@ -152,8 +152,12 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
   // count, so global-attention rows do not start last). Measured: query-block-major heavy-first order loses more
   // to L2 misses than it gains in tail length (tools/bench_sparse_attn.py).
   const int per_bh = SPARSE ? lut.nwork : nqb;
-  const int bh = logical / per_bh;
-  const int qbi = logical % per_bh;
+  int bh = logical / per_bh, qbi = logical % per_bh;
+  if (SPARSE && B * Hq % 8 == 0) {  // an XCD takes the longest lists of all its heads first
+    const int per = B * Hq / 8, at = blockIdx.x / 8;
+    bh = blockIdx.x % 8 * per + at % per;
+    qbi = at / per;
+  }
   const int b = bh / Hq, hq = bh % Hq, hk = hq / (Hq / Hk);
   const int lh = SPARSE ? (lut.lay_heads == 1 ? 0 : hq) : 0;
   int qb = CAUSAL ? nqb - 1 - qbi : qbi, first = 0, count = 0, slot = -1;  // heaviest first
@@ -262,12 +266,11 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
   const float rescale_thr = RESCALE_LOG2 / c;  // in raw score units
   const int qrow_lane = q0w + l32;  // the query row this lane's scores belong to
 
-  // the Q fragments are the only loads hipcc tracks: retire them before the first DMA so its own counted waits
-  // never have to look past transfers it does not know about
+  // the Q fragments are the only loads hipcc tracks: retired after the first DMA is on its way and before the loop, so that its
+  // own counted waits never have to look past transfers it does not know about
+  if (nt > 0) dma_tile(tile_of(0), 0);  // uniform per workgroup (a sparse row block may have no tiles)
 #pragma unroll
   for (int kk = 0; kk < 8; ++kk) asm volatile("" : : "v"(qf[kk]));
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  if (nt > 0) dma_tile(tile_of(0), 0);  // uniform per workgroup (a sparse row block may have no tiles)
   tile_barrier();
 
   // one tile; `cur` (the LDS buffer) is a compile-time constant so it folds into the displacements

@@ -54,12 +54,13 @@ int ds_flash_fwd_sparse(const void*, const void*, const void*, void*, float*, in
                         const int64_t*, const int64_t*, const int64_t*, float, const int*, const int*, const int*,
                         const int*, int, int, int, int, int, float*, float*, const float*, int64_t, const float*, int64_t,
                         const float*, int64_t, int64_t, hipStream_t);
+int ds_sparse_bwd(const void*, const void*, const void*, const void*, const void*, const float*, float*, void*, void*, void*, int, int,
+                  int, const int64_t*, float, const int* const*, const int*, float*, const int* const*, const int*, float*, const float*,
+                  int64_t, const float*, int64_t, const float*, int64_t, int64_t, hipStream_t);
 int ds_flash_bwd_split(int, int, int, int);
 int ds_flash_bwd(const void*, const void*, const void*, const void*, const void*, const float*, float*, float*, void*,
                  void*, void*, int, int, int, int, const int64_t*, const int64_t*, const int64_t*, const int64_t*,
-                 const int64_t*, const int64_t*, const int64_t*, const int64_t*, float, int, const int*, const int*,
-                 const int*, const int*, int, int, int, int, int, float*, int, const float*, int64_t, const float*, int64_t,
-                 const float*, int64_t, int64_t, hipStream_t);
+                 const int64_t*, const int64_t*, const int64_t*, const int64_t*, float, int, float*, hipStream_t);
 int ds_transpose16(const void*, void*, int, int, int, int64_t, hipStream_t);
 int ds_xent_fwd(const void*, const int64_t*, float*, float*, int64_t, int, int64_t, int, float, int, hipStream_t);
 int ds_xent_mean(const float*, const int64_t*, float*, float*, int64_t, int, hipStream_t);
@@ -589,8 +590,9 @@ struct SparsePlan {
   int T, heads, nwork, nmerge, nslots;
 };
 
+// blocks: lists; shared: blocks that the work goes by; ntile: tiles across
 SparsePlan sparse_plan(const OptT& tiles, const OptT& masks, const OptT& work, const OptT& merges, int64_t nslots, int64_t H,
-                       int64_t blocks, int64_t ntile, int64_t nhead, bool contents) {
+                       int64_t blocks, int64_t shared, int64_t ntile, bool contents) {
   for (const OptT* t : {&tiles, &masks, &work, &merges}) {
     TORCH_CHECK(t->has_value(), "block-sparse plan missing");
     need(**t, "plan");
@@ -605,11 +607,10 @@ SparsePlan sparse_plan(const OptT& tiles, const OptT& masks, const OptT& work, c
     auto in = [](const Tensor& t, int64_t lo, int64_t hi) {  // lo <= t < hi
       return t.numel() == 0 || (t.min().item<int>() >= lo && t.max().item<int>() < hi);
     };
-    TORCH_CHECK(in(code.bitwise_and(0xffff), 0, ntile) && in(torch::bitwise_right_shift(code, 16), 0, nhead),
-                "block-sparse plan: tile out of range");
-    TORCH_CHECK(in(wk.select(2, 0), -1, blocks) && in(wk.select(2, 1), 0, T + 1) && in(wk.select(2, 2), 0, T + 1) &&
+    TORCH_CHECK(in(code, 0, ntile), "block-sparse plan: tile out of range");
+    TORCH_CHECK(in(wk.select(2, 0), -1, shared) && in(wk.select(2, 1), 0, T + 1) && in(wk.select(2, 2), 0, T + 1) &&
                     in(wk.select(2, 1) + wk.select(2, 2), 0, T + 1) && in(wk.select(2, 3), -1, nslots) &&
-                    in(mg.select(2, 0), -1, blocks) && in(mg.select(2, 1), 0, nslots) &&
+                    in(mg.select(2, 0), -1, shared) && in(mg.select(2, 1), 0, nslots) &&
                     in(mg.select(2, 1) + mg.select(2, 2), 0, nslots + 1),
                 "block-sparse plan: entry out of range");
   }
@@ -632,7 +633,7 @@ std::vector<Tensor> flash_fwd_sparse(Tensor q, Tensor k, Tensor v, double scale,
   for (const Tensor* t : {&q, &k, &v})
     for (int d = 0; d < 3; ++d) TORCH_CHECK(t->stride(d) % 8 == 0, "flash_fwd_sparse: strides must be multiples of 8");
   TORCH_CHECK(S % 128 == 0, "flash_fwd_sparse: sequence length");
-  const SparsePlan pl = sparse_plan(tiles, masks, work, merges, nslots, Hq, S / 128, S / 64, 1, check_plan);
+  const SparsePlan pl = sparse_plan(tiles, masks, work, merges, nslots, Hq, S / 128, S / 128, S / 64, check_plan);
   Tensor parts, ml;
   if (pl.nmerge > 0) {
     const int64_t n = (pl.heads == 1 ? B * Hq : B) * nslots;
@@ -655,12 +656,10 @@ std::vector<Tensor> flash_fwd_sparse(Tensor q, Tensor k, Tensor v, double scale,
 }
 
 // Flash backward (csrc/attn/flash_bwd.hip): q/o/dout [B,Hq,S,128], k/v [B,Hk,S,128] bf16 views with unit last stride,
-// lse [B,Hq,S] fp32 from flash_fwd. mode 0 full, 1 causal, 2 block-sparse with the column LUT (qtiles int32
-// [Hk, nkb, T] of (head-in-group << 16 | 32-row tile), nqt int32 [Hk, nkb], layout uint8 [LH, nb, nb], granularity
-// blk). Returns dq, dk, dv laid out [B,S,H,128] in memory (viewed [B,H,S,128]) like flash_fwd's output.
+// lse [B,Hq,S] fp32 from flash_fwd. mode 0 full, 1 causal. Returns dq, dk, dv laid out [B,S,H,128] in memory (viewed [B,H,S,128]) like
+// flash_fwd's output.
 std::vector<Tensor> flash_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, Tensor dout, double scale,
-                              int64_t mode, OptT qtiles, OptT qmasks, OptT work, OptT merges, int64_t nslots, OptT kbias,
-                              OptT abias, OptT rpe, bool check_plan) {
+                              int64_t mode) {
   for (const Tensor* t : {&q, &k, &v, &o, &dout}) {
     TORCH_CHECK(t->is_cuda() && t->dim() == 4 && t->scalar_type() == at::kBFloat16, "flash_bwd: 4-D bf16 device tensors");
     TORCH_CHECK(t->size(3) == 128 && t->stride(3) == 1, "flash_bwd: head dim 128 with unit last stride");
@@ -673,27 +672,10 @@ std::vector<Tensor> flash_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse
   TORCH_CHECK(Hq % Hk == 0, "flash_bwd: Hq must be a multiple of Hk");
   TORCH_CHECK(lse.is_cuda() && lse.scalar_type() == at::kFloat && lse.is_contiguous() && lse.numel() == B * Hq * S,
               "flash_bwd: lse [B,Hq,S] fp32 contiguous");
-  TORCH_CHECK(mode >= 0 && mode <= 2, "flash_bwd: mode");
-  SparsePlan pl{};
-  pl.heads = 1;
-  const int64_t nkb = (S + 255) / 256;
-  if (mode == 2) {
-    TORCH_CHECK(S % 128 == 0, "flash_bwd: block-sparse sequence length");
-    pl = sparse_plan(qtiles, qmasks, work, merges, nslots, Hk, nkb, S / 32, Hq / Hk, check_plan);
-  }
-  const int64_t slots = mode == 2 ? (pl.nmerge > 0 ? nslots : 0) : [&] {
-    const int n = ds_flash_bwd_split((int)B, (int)Hq, (int)Hk, (int)S);
-    return n > 1 ? n * nkb : (int64_t)0;
-  }();
+  TORCH_CHECK(mode == 0 || mode == 1, "flash_bwd: mode");
+  const int nsplit = ds_flash_bwd_split((int)B, (int)Hq, (int)Hk, (int)S);
   Tensor parts;
-  if (slots) parts = torch::empty({(pl.heads == 1 ? B * Hk : B) * slots, 65536}, q.options().dtype(at::kFloat));
-  const AttnBias ab = attn_bias(kbias, abias, rpe, B, Hq, S);
-  TORCH_CHECK(mode == 2 || (!ab.kb && !ab.ab && !ab.rp), "flash_bwd: score biases need the block-sparse mode");
-  // the kernel loads all three bias terms unconditionally: absent ones read one zero float
-  const int flags = (ab.kb ? 1 : 0) | (ab.ab ? 2 : 0) | (ab.rp ? 4 : 0);
-  Tensor zero1;
-  if (flags) zero1 = torch::zeros({4}, q.options().dtype(at::kFloat));
-  auto zp = [&](const float* p) { return (p || !flags) ? p : zero1.data_ptr<float>(); };
+  if (nsplit > 1) parts = torch::empty({B * Hk * nsplit * ((S + 255) / 256), 65536}, q.options().dtype(at::kFloat));
   auto mk = [&](int64_t H) { return torch::empty({B, S, H, 128}, q.options()).transpose(1, 2); };
   auto dq = mk(Hq), dk = mk(Hk), dv = mk(Hk);
   auto delta = torch::empty({2 * B * Hq * S}, q.options().dtype(at::kFloat));  // -delta and -LSE/scale rows
@@ -703,11 +685,52 @@ std::vector<Tensor> flash_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse
   st3(q, qs); st3(k, ks); st3(v, vs); st3(o, os); st3(dout, gs); st3(dq, dqs); st3(dk, dks); st3(dv, dvs);
   check(ds_flash_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dout.data_ptr(), lse.data_ptr<float>(),
                      delta.data_ptr<float>(), dqacc.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-                     (int)B, (int)Hq, (int)Hk, (int)S, qs, ks, vs, os, gs, dqs, dks, dvs, (float)scale, (int)mode, pl.tiles,
-                     pl.masks, pl.work, pl.merges, pl.T, pl.heads, pl.nwork, pl.nmerge, pl.nslots,
-                     slots ? parts.data_ptr<float>() : nullptr, flags, zp(ab.kb), ab.kbs, zp(ab.ab), ab.abs_, zp(ab.rp),
-                     ab.rhs, ab.rrs, stream()),
+                     (int)B, (int)Hq, (int)Hk, (int)S, qs, ks, vs, os, gs, dqs, dks, dvs, (float)scale, (int)mode,
+                     nsplit > 1 ? parts.data_ptr<float>() : nullptr, stream()),
         "flash_bwd");
+  return {dq, dk, dv};
+}
+
+// Block-sparse backward (csrc/attn/sparse_bwd.hip): all tensors [B,H,S,128], lse from flash_fwd_sparse. `rows` and `cols`: tiles,
+// masks (by 128 rows and 64-key tiles, by 256 keys and 32-row tiles), work and merges (both by 64 rows or keys). Returns dq, dk, dv as flash_bwd does.
+std::vector<Tensor> sparse_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, Tensor dout, double scale, std::vector<Tensor> rows,
+                               int64_t row_slots, std::vector<Tensor> cols, int64_t col_slots, OptT kbias, OptT abias, OptT rpe,
+                               bool check_plan) {
+  for (const Tensor* t : {&q, &k, &v, &o, &dout}) {
+    TORCH_CHECK(t->is_cuda() && t->dim() == 4 && t->scalar_type() == at::kBFloat16, "sparse_bwd: 4-D bf16 device tensors");
+    TORCH_CHECK(t->size(3) == 128 && t->stride(3) == 1, "sparse_bwd: head dim 128 with unit last stride");
+    TORCH_CHECK(t->sizes() == q.sizes(), "sparse_bwd: shapes");
+    for (int d = 0; d < 3; ++d) TORCH_CHECK(t->stride(d) % 8 == 0, "sparse_bwd: strides must be multiples of 8");
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "sparse_bwd: 16-B aligned data required");
+  }
+  const int64_t B = q.size(0), H = q.size(1), S = q.size(2);
+  TORCH_CHECK(lse.is_cuda() && lse.scalar_type() == at::kFloat && lse.is_contiguous() && lse.numel() == B * H * S,
+              "sparse_bwd: lse [B,H,S] fp32 contiguous");
+  TORCH_CHECK(S % 128 == 0, "sparse_bwd: sequence length");
+  TORCH_CHECK(rows.size() == 4 && cols.size() == 4, "sparse_bwd: plans of tiles, masks, work, merges");
+  const SparsePlan pr = sparse_plan(rows[0], rows[1], rows[2], rows[3], row_slots, H, S / 128, S / 64, S / 64, check_plan);
+  const SparsePlan pc = sparse_plan(cols[0], cols[1], cols[2], cols[3], col_slots, H, (S + 255) / 256, S / 64, S / 32, check_plan);
+  const auto f32 = q.options().dtype(at::kFloat);
+  auto parts = [&](const SparsePlan& p, int64_t each) {
+    return p.nmerge > 0 ? torch::empty({(p.heads == 1 ? B * H : B) * p.nslots, each}, f32) : Tensor();
+  };
+  Tensor row_part = parts(pr, 64 * 128), col_part = parts(pc, 128 * 128);
+  const AttnBias ab = attn_bias(kbias, abias, rpe, B, H, S);
+  auto mk = [&] { return torch::empty({B, S, H, 128}, q.options()).transpose(1, 2); };
+  auto dq = mk(), dk = mk(), dv = mk();
+  auto nrow = torch::empty({2 * B * H * S}, f32);
+  int64_t strides[24], n = 0;
+  for (const Tensor* t : {&q, &k, &v, &o, &dout, &dq, &dk, &dv})
+    for (int d = 0; d < 3; ++d) strides[n++] = t->stride(d);
+  const int* row_lists[4] = {pr.tiles, pr.masks, pr.work, pr.merges};
+  const int* col_lists[4] = {pc.tiles, pc.masks, pc.work, pc.merges};
+  const int row_sizes[5] = {pr.T, pr.heads, pr.nwork, pr.nmerge, pr.nslots}, col_sizes[5] = {pc.T, pc.heads, pc.nwork, pc.nmerge, pc.nslots};
+  check(ds_sparse_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dout.data_ptr(), lse.data_ptr<float>(),
+                      nrow.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), (int)B, (int)H, (int)S, strides, (float)scale,
+                      row_lists, row_sizes, row_part.defined() ? row_part.data_ptr<float>() : nullptr, col_lists, col_sizes,
+                      col_part.defined() ? col_part.data_ptr<float>() : nullptr, ab.kb, ab.kbs, ab.ab, ab.abs_, ab.rp, ab.rhs, ab.rrs,
+                      stream()),
+        "sparse_bwd");
   return {dq, dk, dv};
 }
 
@@ -758,8 +781,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("tiles"), py::arg("masks"), py::arg("work"), py::arg("merges"), py::arg("nslots"), py::arg("want_lse"),
         py::arg("kbias") = py::none(), py::arg("abias") = py::none(), py::arg("rpe") = py::none(), py::arg("check_plan") = true);
   m.def("flash_bwd", &flash_bwd, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("o"), py::arg("lse"),
-        py::arg("dout"), py::arg("scale"), py::arg("mode"), py::arg("qtiles") = py::none(), py::arg("qmasks") = py::none(),
-        py::arg("work") = py::none(), py::arg("merges") = py::none(), py::arg("nslots") = 0, py::arg("kbias") = py::none(),
+        py::arg("dout"), py::arg("scale"), py::arg("mode"));
+  m.def("sparse_bwd", &sparse_bwd, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("o"), py::arg("lse"), py::arg("dout"),
+        py::arg("scale"), py::arg("rows"), py::arg("row_slots"), py::arg("cols"), py::arg("col_slots"), py::arg("kbias") = py::none(),
         py::arg("abias") = py::none(), py::arg("rpe") = py::none(), py::arg("check_plan") = true);
   m.def("xent_fwd", &xent_fwd);
   m.def("xent_mean_fwd", &xent_mean_fwd);

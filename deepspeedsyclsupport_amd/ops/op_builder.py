@@ -43,6 +43,7 @@ EXTENSIONS = {
             "attn/decode_attn.hip",
             "attn/flash_fwd.hip",
             "attn/flash_bwd.hip",
+            "attn/sparse_bwd.hip",
             "attn/paged_prefill.hip",
             "attn/flash_small.hip",
             "quant/quant_kernels.hip",

@@ -6,10 +6,10 @@ head) visits only the 64-key tiles its layout rows touch, listed in a LUT built 
 length), and masks inside a tile by 16 x 16 pieces. Work and K/V traffic therefore scale with the
 layout density. Head dims below 128 are zero-padded to 128 (zeros change neither QK^T nor the kept part of PV).
 
-Backward: `csrc/attn/flash_bwd.hip` in its SPARSE instantiation (reference: the transposed DSD/SDD products of
-`matmul.py:605` and the sparse softmax backward `softmax.py:213`) — every workgroup (256 keys of one head) visits
-only the 32-row query tiles its key block meets in the layout (a column LUT built here) and masks likewise,
-recomputing P from the forward's LSE. No [L, L] tensor is ever built; work scales with density.
+Backward: `csrc/attn/sparse_bwd.hip` (reference: the transposed DSD/SDD products of `matmul.py:605` and the sparse softmax
+backward `softmax.py:213`), one pass by rows for dQ over the forward's lists and one by columns for dK and dV, every workgroup
+64 rows (keys) of one head; the columns' lists are made here too (the 32-row query tiles that 256 keys meet). P is recomputed
+from the forward's LSE. No [L, L] tensor is ever built; work scales with density.
 
 `SparsePlan` holds what both passes read: the lists and their masks (`SparseLists`, one per layout), and how the lists are shared out
 over workgroups (a row or column that is much longer than the others is cut into parts), which depends on batch and heads.
@@ -103,34 +103,37 @@ def build_bwd_lut(layout, blk, L, H, device, key=None):
     return out
 
 
-# Workgroups that the chip holds at once (two of the forward's per CU, one of the backward's) and the shortest part worth cutting:
-# a part costs its operands' first load and a pass of its accumulators through memory, 64 KB in the forward, 256 KB in the
-# backward. Measured, us, BigBird of 64-key blocks, forward with parts of at least 4 / 8 / 16 / 32 tiles, backward with 8 / 16 /
-# 32 / 64: B2 H8 L16384 126 / 113 / 119 / 110 and 520 / 506 / 513 / 506; B1 H8 L4096 31 / 28 / 36 / 56 and 102 / 98 / 100 / 162;
-# B1 H4 L2048 23 / 21 / 32 / 52 and 47 / 72 / 89 / 154. A share of half a chip cuts layouts that fill it by themselves (Fixed,
-# L8192: forward 90 -> 107).
-_FWD_SHARE, _BWD_SHARE = (512, 8), (256, 8)
+# Workgroups that lists are shared out over, and the shortest part worth cutting, in tiles: by rows (64 keys), for the forward and
+# dQ, and by columns (32 rows). The chip holds 512 of either at once; a part costs its operands' first load and a pass of its
+# accumulators through memory, 32 to 64 KB. Measured, us, forward / backward: BigBird B2 H8 L16384 with (512, 8), (256, 8) 153 /
+# 387; (768, 8), (512, 16) 157 / 372; (1024, 16), (4096, 8) 152 / 407; Fixed B1 H8 L8192 98 / 352, 91 / 305, 110 / 419.
+_FWD_SHARE, _BWD_SHARE = (768, 8), (512, 16)
 
 PlanSide = namedtuple("PlanSide", "tiles masks work merges nslots")
 
 
-def _share_out(counts, copies, slots, least):
+def _share_out(counts, copies, slots, least, met=None):
     """counts [LH, n] list lengths; `copies` workgroups sets run side by side -> (work [LH, W, 4], merges [LH, M, 4], nslots):
     lists far longer than an equal share of all the work are cut evenly, the parts of all LH heads numbered through. Entries as in
-    the kernels; -1 pads."""
+    the kernels; -1 pads. met [LH, n, T] (numpy, bool): what counts in longer lists; a part runs from its first to its last."""
     limit = max(least, -(-int(counts.sum()) * copies // slots))
+    if met is not None:   # (first, and one past the last)
+        ends = np.stack([met.argmax(-1), np.where(met.any(-1), met.shape[-1] - met[..., ::-1].argmax(-1), 0)], -1).tolist()
     work, merges, used = [], [], 0
-    for row in counts.tolist():
+    for head, row in enumerate(counts.tolist()):
         entries, joins = [], []
         for i, n in enumerate(row):
-            parts = 1 if n <= limit * 3 // 2 else -(-n // limit)
+            if n <= limit * 3 // 2:
+                a, b = (0, n) if met is None else ends[head][i]
+                entries.append((n, (i, a, b - a, -1)))
+                continue
+            parts, at = -(-n // limit), range(n) if met is None else met[head, i].nonzero()[0].tolist()
             for p in range(parts):
-                a = n * p // parts
-                entries.append((i, a, n * (p + 1) // parts - a, used + p if parts > 1 else -1))
-            if parts > 1:
-                joins.append((i, used, parts, 0))
-                used += parts
-        work.append(sorted(entries, key=lambda e: -e[2]))   # longest first
+                a, b = n * p // parts, n * (p + 1) // parts
+                entries.append((b - a, (i, at[a], at[b - 1] + 1 - at[a], used + p)))
+            joins.append((i, used, parts, 0))
+            used += parts
+        work.append([e for _, e in sorted(entries, key=lambda e: -e[0])])   # longest first
         merges.append(joins)
 
     def pad(lists):
@@ -179,17 +182,28 @@ class SparseLists:
         else:
             tiles, counts, _, _ = build_bwd_lut(self.layout, self.blk, self.L, lay.shape[0], "cpu", self.key)
             masks = _tile_masks(bits, self.blk, self.L, 2, 16).transpose(1, 2)   # listed by key block
-        return *self._to_device([tiles, masks.gather(2, tiles.long())]), counts
+        masks = masks.gather(2, tiles.long())
+        return *self._to_device([tiles, masks]), counts, masks
 
-    def side(self, side, share, B, H):
+    def _split(self, side, parts):
+        """What blocks of 64 rows (columns), `parts` to a list, have to do with: (counts [LH, n], [LH, n, entries of the lists])."""
+        _, _, counts, masks = self.lists[side]
+        masks = np.where(np.arange(masks.shape[2]) < counts.numpy()[..., None], masks.numpy().view(np.uint32), 0)
+        bits = [0xffff << 16 * p if side == "fwd" else 0x000f000f << 4 * p for p in range(parts)]
+        met = (masks[:, :, None] & np.array(bits, np.uint32)[:, None]) != 0
+        met = met.reshape(met.shape[0], -1, met.shape[3])[:, :self.L // 64]
+        return torch.from_numpy(met.sum(-1)), met
+
+    def side(self, side, share, B, H, parts=1):
         if side not in self.lists:
             self.lists[side] = self._make(side)
-        tiles, masks, counts = self.lists[side]
-        key = side, *share, B * H if tiles.shape[0] == 1 else B
+        tiles, masks, counts, _ = self.lists[side]
+        key = side, parts, *share, B * H if tiles.shape[0] == 1 else B
         if key not in self.shares:
             if len(self.shares) > 64:
                 self.shares.clear()
-            work, merges, nslots = _share_out(counts, key[-1], *share)
+            counts, met = (counts, None) if parts == 1 else self._split(side, parts)
+            work, merges, nslots = _share_out(counts, key[-1], *share, met)
             self.shares[key] = (*self._to_device([work, merges]), nslots)
         return PlanSide(tiles, masks, *self.shares[key])
 
@@ -205,6 +219,13 @@ class SparsePlan:
 
     def backward(self):
         return self.lists.side("bwd", _BWD_SHARE, self.B, self.H)
+
+    # the same lists, shared out by blocks of 64 rows (keys): what the backward's kernels read
+    def rows(self):
+        return self.lists.side("fwd", _FWD_SHARE, self.B, self.H, 2)
+
+    def columns(self):
+        return self.lists.side("bwd", _BWD_SHARE, self.B, self.H, 4)
 
 
 _PLANS = {}
@@ -268,8 +289,9 @@ class BlockSparseAttnFn(torch.autograd.Function):
             q, k, v, do = (torch.nn.functional.pad(t, pad) for t in (q, k, v, do))
         elif do.stride(-1) != 1 or any(s % 8 for s in do.stride()[:3]):
             do = do.contiguous()
-        dq, dk, dv = hip_ops().flash_bwd(q, k, v, o, lse, do, ctx.scale, 2, *ctx.plan.backward(), kbias, abias, rpe,
-                                         check_plan=False)
+        rows, cols = ctx.plan.rows(), ctx.plan.columns()
+        dq, dk, dv = hip_ops().sparse_bwd(q, k, v, o, lse, do, ctx.scale, rows[:4], rows.nslots, cols[:4], cols.nslots, kbias, abias,
+                                          rpe, check_plan=False)
         if D < 128:
             dq, dk, dv = dq[..., :D], dk[..., :D], dv[..., :D]
         return dq, dk, dv, None, None, None, None, None, None

@@ -62,6 +62,42 @@ def test_plan_visits_the_layout_once(kind, blk, L, monkeypatch):
         assert plan.forward().nslots > 0 or L <= 256
 
 
+@pytest.mark.parametrize("kind", ["shared", "heads", "empty"])
+@pytest.mark.parametrize("blk,L", [(16, 128), (32, 640), (64, 1152), (256, 1280)])
+@pytest.mark.parametrize("least", [2, 10**6])
+def test_blocks_of_64_visit_the_layout_once(kind, blk, L, least, monkeypatch):
+    """The backward's shares: every block of 64 rows (keys) sees its own part of the lists once, over all its parts."""
+    monkeypatch.setattr(bs, "_FWD_SHARE", (1 << 20, least))
+    monkeypatch.setattr(bs, "_BWD_SHARE", (1 << 20, least))
+    bs._PLANS.clear()
+    lay = _layout(kind, 2, blk, L)
+    plan = bs.sparse_plan(lay, blk, L, 1, 2, "cpu")
+    bs._PLANS.clear()
+    want = (lay != 0).repeat_interleave(blk // 16, 1).repeat_interleave(blk // 16, 2)[:, :L // 16, :L // 16].long()
+    for side, parts, rows, cols in ((plan.rows(), 2, 8, 4), (plan.columns(), 4, 2, 16)):
+        for head in range(side.work.shape[0]):
+            seen, slots = torch.zeros(L // 16, -(-L // 256) * 16, dtype=torch.long), {}
+            for own, first, n, slot in side.work[head].tolist():
+                if own < 0:
+                    continue
+                slots.setdefault(own, []).append(slot)
+                blk_, part = divmod(own, parts)
+                for j in range(first, first + n):
+                    t, m = side.tiles[head, blk_, j].item(), side.masks[head, blk_, j].item()
+                    for r in range(rows):
+                        for k in range(cols):
+                            if parts == 2 and r // 4 == part:
+                                seen[8 * blk_ + r, 4 * t + k] += (m >> (r * cols + k)) & 1
+                            elif parts == 4 and k // 4 == part:
+                                seen[2 * t + r, 16 * blk_ + k] += (m >> (r * cols + k)) & 1
+            assert torch.equal(seen[:, :L // 16], want[head])
+            assert sorted(slots) == list(range(L // 64))
+            merged = {b: list(range(s, s + n)) for b, s, n, _ in side.merges[head].tolist() if b >= 0}
+            assert all(got == [-1] if b not in merged else sorted(got) == merged[b] for b, got in slots.items())
+            assert all(0 <= s < side.nslots for got in merged.values() for s in got)
+            assert L == 128 or bool(merged) == (least == 2)
+
+
 def test_parts_of_all_heads_are_numbered_through():
     """A workspace slot per part there is: a head or two with long rows among many must not reserve as much for each of the others."""
     H, blk, L = 8, 64, 4096
