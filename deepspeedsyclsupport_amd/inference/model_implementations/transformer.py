@@ -12,9 +12,8 @@ all-reduce each (bias added once after it), vocab-parallel LM head with an all-g
 Weight-only int8/int4 quantisation keeps group-quantised weights and dequantises into a per-layer workspace.
 """
 import math
-from array import array
 from dataclasses import dataclass, field
-from itertools import accumulate, repeat
+from itertools import accumulate
 from typing import Dict, List, Optional
 
 import torch
@@ -24,6 +23,8 @@ import torch.nn.functional as F
 from ... import comm as dist
 from ...ops import reference
 from ...ops import moe_ops
+from ...ops.bf16_gemv import Bf16Weight, decode_rows_ok
+from ...ops.native import cpu_ops, hip_ops
 from ...ops.transformer import functional as DF
 
 
@@ -111,7 +112,6 @@ class QuantLinearWeight:
     `i8` holds whichever stream object applies."""
 
     def __init__(self, w, bits=8, group_size=64):
-        from ...ops.bf16_gemv import Bf16Weight
         from ...ops.int4_gemv import Int4Weight
         from ...ops.int8_gemv import Int8Weight
         from ...ops.quantizer import quantize
@@ -188,6 +188,7 @@ class RaggedMeta:
     kv_offs: Optional[torch.Tensor] = None   # [S - n_short + 1] offsets of the other sequences' contexts laid end to end
     kv_total: int = 0                # ... and their end
     ids: Optional[torch.Tensor] = None       # the new tokens, where `build` was given them
+    ids_checked: bool = False        # ... and the caller has seen to it that the vocabulary has them
     seen: Dict[int, tuple] = field(default_factory=dict)   # `contexts` by window
 
     SHORT_TOKENS = 64    # portions up to this long count as short
@@ -217,71 +218,16 @@ class RaggedMeta:
     @staticmethod
     def build(starts, n_new, block_lists, n_decode, block_size, device, slots=None, logit_rows=None, ids=None):
         """`slots`: state slots of the sequences; `logit_rows`: rows (of the concatenated tokens) whose logits are
-        wanted instead of every sequence's last; `ids`: int64 tokens on the host that go along."""
-        S = len(starts)
-        cu = list(accumulate(n_new, initial=0))
-        T = cu[-1]
-        width = max(1, max(len(b) for b in block_lists))
-        lens = [st + n for st, n in zip(starts, n_new)]
-        last = [c - 1 for c in cu[1:]] if logit_rows is None else list(logit_rows)
-        slots = [] if slots is None else list(slots)
-        long = [i for i in range(S) if n_new[i] > RaggedMeta.STEP_TOKENS] if slots else []
-        short = [i for i in range(S) if n_new[i] <= RaggedMeta.STEP_TOKENS] if slots else []
-        # (a sequence is only counted as short if everything before it in the batch is)
-        n_short = next((i for i in range(n_decode, S) if n_new[i] > RaggedMeta.SHORT_TOKENS), S)
-        kv = list(accumulate(lens[n_short:], initial=0))
-        # everything in one array of 32-bit integers (a decode step is bound by the host: no detour over long lists)
-        flat, sizes = array("i"), []
-
-        def part(values=()):
-            flat.extend(values)
-            sizes.append(len(flat))
-
-        for st, n in zip(starts, n_new):
-            flat.extend((st, ) if n == 1 else range(st, st + n))
-        part()
-        for i, n in enumerate(n_new):
-            flat.extend((i, ) if n == 1 else repeat(i, n))
-        part()
-        part(starts)
-        part(lens)
-        part(cu)
-        for i in range(n_decode, S):
-            for qb in range(-(-n_new[i] // 128)):
-                flat.extend((i, qb))
-        part()
-        part(last)
-        for b in block_lists:
-            flat.extend(b)
-            flat.frombytes(bytes(4 * (width - len(b))))
-        part()
-        part(slots)
-        part(short)
-        chunks, chunk_seqs = [], []
-        for i in long:
-            chunk_seqs += [i, len(chunks) // 2]
-            for c in range(-(-n_new[i] // RaggedMeta.STATE_CHUNK)):
-                chunks += (i, c)
-        part(chunk_seqs)
-        part(chunks)
-        part(kv)
-        # ... behind the 64-bit ones: one copy, from pinned memory, so that no step waits for the steps before it
-        wide = torch.tensor(last, dtype=torch.int64)
-        wide = wide if ids is None else torch.cat([wide, ids])
-        cuda, n = device is not None and torch.device(device).type == "cuda", 2 * len(wide)
-        buf = torch.empty(n + len(flat), dtype=torch.int32, pin_memory=cuda)
-        buf[:n].view(torch.int64).copy_(wide)
-        buf[n:].copy_(torch.frombuffer(flat, dtype=torch.int32))
-        if cuda:
-            buf = buf.to(device, non_blocking=True)
-        wide, buf = buf[:n].view(torch.int64), buf[n:]
-        views = [buf[a:b] for a, b in zip([0] + sizes, sizes)]
+        wanted instead of every sequence's last; `ids`: int64 tokens on the host (a tensor or several) that go along."""
+        toks = [] if ids is None else [ids] if torch.is_tensor(ids) else list(ids)
+        views, last_idx, ids, cu, n_short, kv_total, width, all_rows = cpu_ops().ragged_tables(
+            starts, n_new, block_lists, n_decode, slots or [], logit_rows, toks, None if device is None else torch.device(device),
+            RaggedMeta.SHORT_TOKENS, RaggedMeta.STEP_TOKENS, RaggedMeta.STATE_CHUNK)
         pos_t, sid_t, st_t, len_t, cu_t, work_t, last_t, bt_t, slot_t, short_t, long_t, chunk_t, kv_t = views
-        return RaggedMeta(block_tables=bt_t.view(S, width), start_pos=st_t, seq_lens=len_t, pos_ids=pos_t,
-                          seq_ids=sid_t, cu_q=cu_t, work=work_t.view(-1, 2), last_idx=wide[:len(last)], last_rows=last_t,
-                          all_rows=len(last) == T and last == list(range(T)), ids=None if ids is None else wide[len(last):], n_decode=n_decode, cu_host=cu, start_host=list(starts), max_len=width * block_size,
-                          block_size=block_size, slots=slot_t, seq_list=short_t, chunk_seqs=long_t.view(-1, 2),
-                          chunk_work=chunk_t.view(-1, 2), n_short=n_short, kv_offs=kv_t, kv_total=kv[-1])
+        return RaggedMeta(block_tables=bt_t, start_pos=st_t, seq_lens=len_t, pos_ids=pos_t, seq_ids=sid_t, cu_q=cu_t, work=work_t,
+                          last_idx=last_idx, last_rows=last_t, all_rows=all_rows, ids=ids, n_decode=n_decode, cu_host=cu,
+                          start_host=list(starts), max_len=width * block_size, block_size=block_size, slots=slot_t, seq_list=short_t,
+                          chunk_seqs=long_t, chunk_work=chunk_t, n_short=n_short, kv_offs=kv_t, kv_total=kv_total)
 
 
 class ProjectionLayer(nn.Module):
@@ -317,7 +263,6 @@ class ProjectionLayer(nn.Module):
         """Keep a second copy of the four projection weights in MFMA operand order (`ops/bf16_gemv.py`): twice the
         weight memory — 288 GB of HBM is sized for it — for decode-sized batches. No-op for quantised, split or non-bf16
         weights."""
-        from ...ops.bf16_gemv import Bf16Weight
         if self.quant or self.split_w or self.spec.num_experts:
             return False
         ws = {n: getattr(self, n) for n in ("qkv_w", "o_w", "fc1_w", "fc2_w")}
@@ -427,7 +372,6 @@ class DSInferenceLayer(ProjectionLayer):
         if pending is not None or (qkv.is_cuda and qkv.dtype == torch.bfloat16 and kc.dtype == torch.bfloat16):
             # one fused HIP epilogue: split + RoPE(q, k) + scatter k/v into the paged cache (and, for a pending
             # weight-only GEMV, its finalize pass: the sums are read straight from the split-K workspace)
-            from ...ops.native import hip_ops
             rot = spec.rotary_dim if spec.pos in ("rope", "rope_gptj") else 0
             want_kv = meta.prefill_from_zero and n > 1 and not paged
             src = pending._take() if pending is not None else qkv.contiguous()
@@ -469,7 +413,6 @@ class DSInferenceLayer(ProjectionLayer):
 
     def _decode_step(self, qkv, meta, kc, vc, rope, alibi, scale, window):
         """qkv of one token a sequence -> its attention [B, Hq, D], in one kernel (`csrc/attn/decode_attn.hip`)."""
-        from ...ops.native import hip_ops
         spec = self.spec
         rot = spec.rotary_dim if spec.pos in ("rope", "rope_gptj") else 0
         return hip_ops().paged_decode_step(qkv.contiguous(), rope[0] if rot else None, rope[1] if rot else None, meta.pos_ids, kc,
@@ -494,7 +437,6 @@ class DSInferenceLayer(ProjectionLayer):
         if meta.n_decode == len(meta.start_host) and pending is None and self._step_ok(qkv, kc):
             return self._decode_step(qkv, meta, kc, vc, rope, alibi, scale, window).view(1, T, self.hq * D)
         if pending is not None or (qkv.is_cuda and qkv.dtype == torch.bfloat16 and kc.dtype == torch.bfloat16):
-            from ...ops.native import hip_ops
             src = pending._take() if pending is not None else qkv.reshape(T, -1).contiguous()
             q = hip_ops().qkv_rope_append(src, rope[0] if rot else None,
                                           rope[1] if rot else None, meta.pos_ids, kc, vc, meta.block_tables,
@@ -566,7 +508,6 @@ class DSInferenceLayer(ProjectionLayer):
     def _forward_skinny(self, h, residual, meta, cache, rope, alibi):
         """Decode (<= 8 token rows): 4 weight-streaming GEMVs with RMSNorm / residual / gated activation fused into
         their input stage, plus the fused QKV epilogue and the paged decode attention."""
-        from ...ops.native import hip_ops
         from ...ops.transformer.functional import ACT_CODES
         ops, eps, tp1 = hip_ops(), self.spec.norm_eps, self.tp == 1
         res1 = torch.empty_like(h)
@@ -600,19 +541,29 @@ class DSInferenceLayer(ProjectionLayer):
         if (not self.quant and not self.sh) or self.split_w or spec.norm != "rms" or spec.parallel_residual \
                 or spec.num_experts or self.tp != 1 or not torch.is_tensor(h):
             return None
-        from ...ops.bf16_gemv import Bf16Weight, decode_rows_ok
         ws = self.sh or {n: w.i8 for n, w in self.quant.items()}
         return ws if decode_rows_ok(h) and all(isinstance(ws.get(n), Bf16Weight) for n in self.projection_names()) else None
 
     def _forward_decode(self, h, residual, meta, cache, rope, alibi, ws):
         """Four products, each with what stands around it: the norms are part of the products that read them, residuals,
         biases and the activation of those that make them (`csrc/gemv/skinny_bf16_sh.hip`)."""
-        from ...ops.transformer.functional import ACT_CODES
         spec = self.spec
         x = h if residual is None else h + residual
+        kc = cache.k[self.layer_idx]
+        if isinstance(meta, RaggedMeta) and meta.n_decode == len(meta.start_host) and self._step_ok(x, kc):
+            # one token a sequence: the same launches in one call
+            rot = spec.rotary_dim if spec.pos in ("rope", "rope_gptj") else 0
+            cos, sin = rope if rot else (None, None)
+            window = spec.layer_windows[self.layer_idx] if spec.layer_windows else spec.sliding_window
+            qkv, o, fc1, fc2 = ws["qkv_w"], ws["o_w"], ws["fc1_w"], ws["fc2_w"]
+            return hip_ops().decode_layer(
+                x, qkv.wsh, qkv.shape[0], self.qkv_b, self.ln1_w, o.wsh, self.o_b, self.ln2_w, fc1.wsh, fc1.shape[0], self.fc1_b,
+                fc2.wsh, self.fc2_b, spec.norm_eps, DF.ACT_CODES[spec.act], spec.gated_mlp, cos, sin, meta.pos_ids, kc,
+                cache.v[self.layer_idx], meta.block_tables, meta.seq_lens, meta.max_len, spec.attn_scale or 1.0 / math.sqrt(spec.head_dim),
+                alibi, window, self.hq, rot, spec.pos == "rope_gptj"), None
         qkv = ws["qkv_w"].raw(x, self.qkv_b).finish(norm=(self.ln1_w, spec.norm_eps))
         x = ws["o_w"].raw(self._attend(qkv, meta, cache, rope, alibi), self.o_b).finish(residual=x)
-        mid = ws["fc1_w"].raw(x, self.fc1_b).finish(norm=(self.ln2_w, spec.norm_eps), act=ACT_CODES[spec.act],
+        mid = ws["fc1_w"].raw(x, self.fc1_b).finish(norm=(self.ln2_w, spec.norm_eps), act=DF.ACT_CODES[spec.act],
                                                     gated=spec.gated_mlp)
         return ws["fc2_w"].raw(mid, self.fc2_b).finish(residual=x), None
 
@@ -623,7 +574,6 @@ class DSInferenceLayer(ProjectionLayer):
         if not self.quant or self.split_w or spec.norm != "rms" or spec.parallel_residual or spec.num_experts \
                 or self.tp != 1:
             return None
-        from ...ops.bf16_gemv import Bf16Weight
         from ...ops.int8_gemv import PendingAcc, raw_ok
         q = {n: self.quant[n].i8 if n in self.quant else None for n in self.projection_names()}
         if any(w is None or isinstance(w, Bf16Weight) for w in q.values()):
@@ -686,7 +636,6 @@ class DSInferenceLayer(ProjectionLayer):
 # ------------------------------------------------------------------------------------------------ attention impls
 def _kv_append(k, v, kc, vc, meta):
     if k.is_cuda and kc.dtype == torch.bfloat16:
-        from ...ops.native import hip_ops
         hip_ops().kv_append(k, v, kc, vc, meta.block_tables, meta.start_pos)
         return
     B, n, Hk, D = k.shape
@@ -856,7 +805,6 @@ def _seq_cached_attention(q, kc, vc, meta, i, scale, alibi, window):
 
 def _decode_attention(q, kc, vc, meta, scale, alibi, window):
     if q.is_cuda and q.dtype == torch.bfloat16 and q.shape[-1] in PAGED_HEAD_DIMS:
-        from ...ops.native import hip_ops
         return hip_ops().paged_decode(q, kc, vc, meta.block_tables, meta.seq_lens, meta.max_len, scale,
                                       alibi, window)
     B, Hq, D = q.shape
@@ -928,6 +876,9 @@ class DSInferenceModel(nn.Module):
             # token + learned position rows in one gather kernel (reference `ragged_ops/embed/embed.cu:19`)
             pos = meta.pos_ids.view(input_ids.shape).long() + self.spec.learned_pos_offset
             h = moe_ops.embed_gather(self.embed, input_ids, self.pos_embed, pos).view(*input_ids.shape, -1)
+        elif getattr(meta, "ids_checked", False):
+            # (torch's lookup of up to 16 rows is one workgroup: 12 rows of 2048 10 us, here 3; it alone checks the ids)
+            h = moe_ops.embed_gather(self.embed, input_ids).view(*input_ids.shape, -1)
         else:
             h = F.embedding(input_ids, self.embed)
         if self.spec.embed_norm:
@@ -942,14 +893,12 @@ class DSInferenceModel(nn.Module):
         spec = self.spec
         if not (h.is_cuda and h.dtype == torch.bfloat16 and spec.final_norm and spec.norm == "rms"):
             return None
-        from ...ops.bf16_gemv import decode_rows_ok
         sh = getattr(self, "lm_head_sh", None)
         if sh is not None and decode_rows_ok(h):
             x = h if residual is None else h + residual
             return self._gather_vocab(sh.raw(x, self.lm_head_b).finish(norm=(self.norm_w, spec.norm_eps)))
         if not _skinny_rows_ok(h.shape[0], spec.hidden_size):
             return None
-        from ...ops.native import hip_ops
         return self._gather_vocab(hip_ops().skinny_gemm(h, self.lm_head, self.lm_head_b, None, 1, False, 0, residual, self.norm_w,
                                                         spec.norm_eps, None))
 
@@ -1020,7 +969,6 @@ class DSInferenceModel(nn.Module):
         """Second, shuffled copy of every layer's projection weights for batched decode (see the layer method);
         returns the number of layers that took one."""
         n = sum(bool(layer.add_decode_layout()) for layer in self.layers)
-        from ...ops.bf16_gemv import Bf16Weight
         if n and self.tp_size == 1 and self.lm_head.is_cuda and Bf16Weight.supported(self.lm_head.data):
             self.lm_head_sh = Bf16Weight(self.lm_head.data)  # the LM head streams every decode step too
         return n

@@ -14,6 +14,7 @@ from typing import Iterable, Tuple
 
 import torch
 
+from ...ops.native import cpu_ops
 from ..model_implementations.transformer import DSInferenceModel
 from .config_v2 import AllocationMode, RaggedInferenceEngineConfig
 from .ragged import DSStateManager, PlaceholderSequenceDescriptor, RaggedBatchWrapper
@@ -82,27 +83,26 @@ class InferenceEngineV2:
         the device: a step is prepared while the one before it runs. On another stream than that one it starts behind it."""
         uids = list(batch_uids)
         toks = [t.reshape(-1) for t in batch_tokens]
+        lens = [t.numel() for t in toks]
         if do_checks:
-            res = self.can_schedule(uids, [t.numel() for t in toks])
+            res = self.can_schedule(uids, lens)
             if res != SchedulingResult.Success:
                 raise SchedulingError(res)
-            host = [t for t in toks if not t.is_cuda and t.numel()]
-            if host:  # an id the embedding does not have must not reach the device
-                lo, hi = torch.aminmax(torch.cat(host))
-                if int(lo) < 0 or int(hi) >= self._model.spec.vocab_size:
-                    raise ValueError(f"token ids {int(lo)} to {int(hi)} outside the vocabulary of "
-                                     f"{self._model.spec.vocab_size}")
+            lo, hi = cpu_ops().int_range([t for t in toks if not t.is_cuda])
+            if lo < 0 or hi >= self._model.spec.vocab_size:  # an id the embedding does not have must not reach the device
+                raise ValueError(f"token ids {lo} to {hi} outside the vocabulary of {self._model.spec.vocab_size}")
         self._follow_last_step()
         batch = self._batch
         batch.clear()
         seqs = []
-        for uid, t in zip(uids, toks):
+        for uid, t, n in zip(uids, toks, lens):
             seq = self._state_manager.get_or_create_sequence(uid)
-            self._state_manager.allocate_blocks(seq, t.numel())
-            seq.pre_forward(t.numel())
+            self._state_manager.allocate_blocks(seq, n)
+            seq.pre_forward(n)
             batch.insert_sequence(seq, t, do_checks=False)
             seqs.append(seq)
-        batch.finalize(logit_positions=[(t.numel() - 1, ) for t in toks] if logit_positions is None else logit_positions)
+        batch.finalize(logit_positions=[(n - 1, ) for n in lens] if logit_positions is None else logit_positions,
+                       ids_checked=do_checks)
         logits = self._model.forward_ragged(batch.input_ids(), batch.meta)
         for s in seqs:
             s.post_forward()

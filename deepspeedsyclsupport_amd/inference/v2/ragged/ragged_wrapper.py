@@ -58,10 +58,10 @@ class RaggedBatchWrapper:
         self._toks.append(tokens)
         self._n_tokens += tokens.numel()
 
-    def finalize(self, padding=False, logit_positions=None) -> None:
+    def finalize(self, padding=False, logit_positions=None, ids_checked=False) -> None:
         """Build and upload the index tables. `padding` is accepted for signature parity: the in-tree kernels take
         exact counts, nothing is padded. `logit_positions`: per inserted sequence, the places among its new tokens
-        whose logits are wanted (default: the last one of each)."""
+        whose logits are wanted (default: the last one of each); `ids_checked`: the host tokens are in the vocabulary."""
         if not self._seqs:
             raise RuntimeError("cannot finalize an empty ragged batch")
         n = [t.numel() for t in self._toks]
@@ -77,15 +77,17 @@ class RaggedBatchWrapper:
                 at += n[i]
             rows = [first[i] + int(p) for i, want in enumerate(logit_positions) for p in want]
         slots = [s.slot for s in seqs] if seqs[0].slot is not None else None
-        ids = torch.cat([self._toks[i] for i in self.order])
-        packed = ids.dtype == torch.int64 and not ids.is_cuda
+        toks = [self._toks[i] for i in self.order]
+        packed = all(t.dtype == torch.int64 and not t.is_cuda for t in toks)   # (they go along with the tables)
         self.meta = RaggedMeta.build([s.seen_tokens for s in seqs], [n[i] for i in self.order],
                                      [s.blocks for s in seqs], sum(is_decode), bs, self._device, slots, rows,
-                                     ids if packed else None)
+                                     toks if packed else None)
         if packed:
-            ids = self.meta.ids
-        elif self._device is not None:
-            ids = ids.to(self._device, non_blocking=True)
+            ids, self.meta.ids_checked = self.meta.ids, ids_checked
+        else:
+            ids = torch.cat(toks)
+            if self._device is not None:
+                ids = ids.to(self._device, non_blocking=True)
         self._ids = ids
         self._is_finalized = True
 

@@ -137,10 +137,11 @@ EXTENSIONS = {
         ],
         "bindings": ["bind/hybrid_bind.cpp"],
     },
-    # host ops: CPU Adam/Adagrad/Lion (ZeRO-Offload, Twin-Flow), async tensor I/O (ZeRO-Infinity), shm all-reduce
+    # host ops: CPU Adam/Adagrad/Lion (ZeRO-Offload, Twin-Flow), async tensor I/O (ZeRO-Infinity), shm all-reduce,
+    # index tables of ragged batches
     "ds_cpu_ops": {
         "kind": "cpu",
-        "sources": ["cpu/cpu_optim.cpp", "cpu/aio.cpp", "cpu/shm_comm.cpp", "cpu/cpu_module.cpp"],
+        "sources": ["cpu/cpu_optim.cpp", "cpu/aio.cpp", "cpu/shm_comm.cpp", "cpu/ragged.cpp", "cpu/cpu_module.cpp"],
         "libs": "-lrt -lpthread",
     },
 }
