@@ -13,7 +13,7 @@
 //    value must not become -inf), online softmax, P reused as the A operand of O += P.V (V by the hardware transposed
 //    read); dropout multiplies P by keep / (1 - p) after the normaliser (Philox-4x32 keyed by (z, h, query, key),
 //    regenerated in the backward);
-//  * backward: passes without atomics on the big tensors (dQ query-outer; dK/dV key-outer; the shared pair-bias gradient summed
+//  * backward: passes without atomics on the big tensors (dQ query-outer; dK/dV key-outer; short sequences both in one; the shared pair-bias gradient summed
 //    over the z that share it in registers), P recomputed from the saved LSE in each — see the backward section.
 // All passes are bound by the vector instructions around the exponentials (about ten a score) and by latency: tiles are small and
 // few, so each has ONE buffer in LDS and nothing is held in registers for the next one: three workgroups share a CU and cover each
@@ -96,6 +96,7 @@ struct SmallArgs {
   int64_t b2_last; // elements of bias2 - 8 (at least 0): where its last whole chunk begins
   int nsplit;      // dB2 pass: the b2_div sharing z are split over this many workgroups
   float* part;     // ... whose sums go here [nsplit, Z / b2_div, H, S, S] when they are several
+  T* order;        // backward: the pair bias in the accumulators' order (small_order_elements), or null
   int Sk;          // keys (the forward may attend to a context of another length; the backward needs Sk == S)
 };
 
@@ -701,6 +702,244 @@ __global__ void __launch_bounds__(NTHR, 2) small_bwd_dkv_kernel(SmallArgs<T> a) 
   }
 }
 
+// ---------------------------------------------------------------- passes 1 and 2 in one: sequences of up to 256, width 32, a pair bias
+// One workgroup has all of a (z, h): a wave per 32 keys, with dK and dV of its keys in registers, and Q, dO and K whole in LDS (64-byte
+// rows, chunks swizzled by the row). Scores, their exponentials and dS are made once for all three gradients instead of twice:
+// the vector instructions around them are what bounds both passes. dS of a tile of 32 queries crosses LDS for dQ, 16 x 16
+// pieces of which go to four waves in turn, while the others begin the next tile. The pair bias comes in the order of the
+// accumulators (small_bias_order_kernel), 2 x 16 bytes a lane and tile from L2. Two workgroups of eight waves share a CU.
+// [256, 256, 4, 32], us: 50 + 51 in two passes, 72 here, 20 of it the loads of two rounds of workgroups that all begin at once, the
+// others 6000 clocks a tile (four waves a SIMD, 1000 each of vector instructions).
+constexpr int WHOLE_S = 256, WHOLE_LDS = 3 * WHOLE_S * 64 + WHOLE_S * 64 + 2 * WHOLE_S * 4;
+
+// bias2 [groups, S, S] -> [groups, query tiles, key tiles, 2, 64, 8]: element j of half g and lane l is query crow(8 g + j, l / 32), key
+// l % 32 of the tile; zero past the end. A wave per tile.
+template <typename T>
+__global__ void __launch_bounds__(256) small_bias_order_kernel(const T* __restrict__ b2, T* __restrict__ out, int S, int nt, int64_t tiles) {
+  const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (w >= tiles) return;
+  const int lane = threadIdx.x & 63, kt = (int)(w % nt), qt = (int)(w / nt % nt), key = 32 * kt + (lane & 31);
+  const T* src = b2 + w / nt / nt * S * S;
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    typename MF<T>::V8 v;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int q = 32 * qt + crow(8 * g + j, lane >> 5);
+      v[j] = q < S && key < S ? src[(int64_t)q * S + key] : (T)0.f;
+    }
+    *reinterpret_cast<typename MF<T>::V8*>(out + w * 1024 + (g * 64 + lane) * 8) = v;
+  }
+}
+
+__device__ __forceinline__ f32x4 mma16(bf16x8_t a, bf16x8_t b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f32x4 mma16(f16x8_t a, f16x8_t b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+
+// 4 + 4 rows' transposed read at two places
+template <typename V8>
+__device__ __forceinline__ V8 tr_pair(const char* lo_p, const char* hi_p) {
+  const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)lo_p);
+  const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)hi_p);
+  s16x8 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) { v[e] = lo[e]; v[4 + e] = hi[e]; }
+  return __builtin_bit_cast(V8, v);
+}
+
+template <typename T, bool DB1>
+__global__ void __launch_bounds__(WHOLE_S * 2, 4) small_bwd_whole_kernel(SmallArgs<T> a, const T* b2o) {
+  typedef typename MF<T>::V8 V8;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int nt = blockDim.x / 64, rows = 32 * nt;   // tiles of 32, one a wave
+  char *Qi = smem, *Gi = Qi + rows * 64, *Ki = Gi + rows * 64, *DS = Ki + rows * 64;   // DS: [key][32 queries]
+  float *lseS = reinterpret_cast<float*>(DS + rows * 64), *delS = lseS + rows;
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int S = a.S, hd = blockIdx.x % a.H, z = blockIdx.x / a.H;
+  const float LOG2E = 1.4426950408889634f;
+  const T* Qp = a.q + z * a.qz + hd * a.qh;
+  const T* Gp = a.dout + z * a.gz + hd * a.gh;
+  const T* Kp = a.k + z * a.kz + hd * a.kh;
+  const int64_t lrow = ((int64_t)z * a.H + hd) * S;
+
+  // ---- Q, dO, K whole: chunk ch of row r at 64 r + 16 (ch ^ r / 4 % 4)
+  u32x4_t st[3][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = tid + i * blockDim.x, r = min(c >> 2, S - 1), ch = c & 3;
+    st[0][i] = *reinterpret_cast<const u32x4_t*>(Qp + (int64_t)r * a.qs + ch * 8);
+    st[1][i] = *reinterpret_cast<const u32x4_t*>(Gp + (int64_t)r * a.gs + ch * 8);
+    st[2][i] = *reinterpret_cast<const u32x4_t*>(Kp + (int64_t)r * a.ks + ch * 8);
+  }
+  // ---- this wave's keys as B operands (column: the lane's key), and its 32 queries' delta
+  const int key = 32 * wid + l32, kc = min(key, S - 1);
+  const bool live = key < S;
+  V8 kB[2], vB[2];
+  float delta = 0.f;
+  {
+    const T* kr = Kp + (int64_t)kc * a.ks;
+    const T* vr = a.v + z * a.vz + hd * a.vh + (int64_t)kc * a.vs;
+    const T* gr = Gp + (int64_t)kc * a.gs;
+    const T* orow = a.o + z * a.oz + hd * a.oh + (int64_t)kc * a.os_;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      kB[kk] = *reinterpret_cast<const V8*>(kr + 16 * kk + 8 * h);
+      vB[kk] = *reinterpret_cast<const V8*>(vr + 16 * kk + 8 * h);
+      const V8 g = *reinterpret_cast<const V8*>(gr + 16 * kk + 8 * h), o = *reinterpret_cast<const V8*>(orow + 16 * kk + 8 * h);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) delta += (float)g[e] * (float)o[e];
+    }
+    delta += __shfl_xor(delta, 32, 64);
+  }
+  const float b1v = !live ? -INFINITY : a.b1 ? (float)a.b1[z * a.b1_zs + key] : 0.f;
+  const T* bp = b2o + (((int64_t)(z / a.b2_div) * a.H + hd) * nt * nt + wid) * 1024;  // tile (0, wid); the next: nt tiles on
+  V8 bias[2] = {*reinterpret_cast<const V8*>(bp + lane * 8), *reinterpret_cast<const V8*>(bp + 512 + lane * 8)};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = tid + i * blockDim.x, r = c >> 2, at = r * 64 + 16 * ((c & 3) ^ ((r >> 2) & 3));
+    *reinterpret_cast<u32x4_t*>(Qi + at) = st[0][i];
+    *reinterpret_cast<u32x4_t*>(Gi + at) = st[1][i];
+    *reinterpret_cast<u32x4_t*>(Ki + at) = st[2][i];
+  }
+  if (lane < 32) {  // queries past the end weigh nothing
+    lseS[key] = live ? a.lse[lrow + key] : INFINITY;
+    delS[key] = live ? -delta : 0.f;
+    if (live) a.delta[lrow + key] = delta;
+  }
+
+  f32x16_t dk, dv;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) dk[r] = dv[r] = 0.f;
+  float colsum = 0.f;
+  // (LDS alone: neither the bias on its way nor what is stored of dQ is waited for)
+  auto sync = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  sync();
+  for (int t = 0; t < nt; ++t) {
+    // where a lane reads rows (A operands), columns of 32 (B of dK, dV) and of 16 (dQ), and writes dS: worked out anew for every
+    // tile from a lane that the compiler takes for another each time (kept over the loop they would spill)
+    int ln = tid & 63;
+    asm volatile("" : "+v"(ln));
+    const int hh = ln >> 5, k32 = ln & 31, gq = (ln >> 2) & 3, gch = (ln >> 1) & 1, gb = 8 * (ln & 1), colhalf = (ln >> 4) & 1;
+    int ra[2], ta[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) ra[kk] = k32 * 64 + 16 * ((2 * kk + hh) ^ ((k32 >> 2) & 3));
+#pragma unroll
+    for (int hi = 0; hi < 2; ++hi) ta[hi] = (4 * hh + 8 * hi + gq) * 64 + 16 * ((colhalf * 2 + gch) ^ (hh + 2 * hi)) + gb;
+    f32x16_t s, dp;  // dP starts at -delta; a zero of its own for every tile (one for all would hold 16 registers)
+    float zero = 0.f;
+    asm volatile("" : "+v"(zero));
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 d4 = *reinterpret_cast<const f32x4*>(delS + 32 * t + 8 * g + 4 * hh);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[4 * g + i] = zero;
+        dp[4 * g + i] = d4[i];
+      }
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      s = MF<T>::mma(*reinterpret_cast<const V8*>(Qi + t * 2048 + ra[kk]), kB[kk], s);
+      dp = MF<T>::mma(*reinterpret_cast<const V8*>(Gi + t * 2048 + ra[kk]), vB[kk], dp);
+    }
+    V8 pa[2], da[2];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      if (g) __builtin_amdgcn_sched_barrier(0);  // (one group's constants at a time: registers)
+      const f32x4 l4 = *reinterpret_cast<const f32x4*>(lseS + 32 * t + 8 * g + 4 * hh);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 4 * g + i;
+        const float x = s[r] * a.scale + b1v + (float)bias[r >> 3][r & 7];
+        const float p = __builtin_amdgcn_exp2f((x - l4[i]) * LOG2E), ds = p * dp[r];
+        if constexpr (DB1) colsum += ds;
+        pa[r >> 3][r & 7] = (T)p;
+        da[r >> 3][r & 7] = (T)ds;
+      }
+    }
+    if (t + 1 < nt) {  // (the next tile's bias comes while dQ is made)
+      bp += (int64_t)nt * 1024;
+      bias[0] = *reinterpret_cast<const V8*>(bp + ln * 8);
+      bias[1] = *reinterpret_cast<const V8*>(bp + 512 + ln * 8);
+    }
+    if (t) sync();  // dS of the tile before has been read
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const s16x8 d8 = __builtin_bit_cast(s16x8, da[g >> 1]);
+      s16x4 v4;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v4[i] = d8[4 * (g & 1) + i];
+      // unit 2 g + h of the key's row
+      *reinterpret_cast<s16x4*>(DS + (32 * wid + k32) * 64 + 8 * (hh ^ ((k32 >> 1) & 1)) + 16 * (g ^ ((k32 >> 2) & 3))) = v4;
+    }
+#pragma unroll
+    for (int ss = 0; ss < 2; ++ss) {
+      const int at = t * 2048 + ss * 1024;
+      dv = MF<T>::mma(pa[ss], tr_pair<V8>(Gi + at + ta[0], Gi + at + ta[1]), dv);
+      dk = MF<T>::mma(da[ss], tr_pair<V8>(Qi + at + ta[0], Qi + at + ta[1]), dk);
+    }
+    sync();
+    // ---- dQ of the tile: four pieces of 16 x 16, over all keys, piece j by wave (4 t + j) % nt
+#pragma unroll 1
+    for (int j = (wid + 4 * nt * t - 4 * t) % nt; j < 4; j += nt) {
+      const int qh = j >> 1, dh = j & 1, g4 = ln >> 4;
+      int da_[2], kb_[2];
+#pragma unroll
+      for (int hi = 0; hi < 2; ++hi) {
+        const int kr = 8 * g4 + 4 * hi + gq;
+        da_[hi] = kr * 64 + 8 * ((4 * qh + (ln & 3)) ^ ((kr >> 1) & 7));
+        kb_[hi] = kr * 64 + 16 * ((2 * dh + gch) ^ ((kr >> 2) & 3)) + gb;
+      }
+      f32x4 dq{0.f, 0.f, 0.f, 0.f};
+      for (int c0 = 0; c0 < nt; c0 += 4) {  // four tiles' reads fly together
+        V8 ds4[4], k4[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int at = min(c0 + c, nt - 1) * 2048;
+          ds4[c] = tr_pair<V8>(DS + at + da_[0], DS + at + da_[1]);
+          k4[c] = tr_pair<V8>(Ki + at + kb_[0], Ki + at + kb_[1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (c0 + c < nt) dq = mma16(ds4[c], k4[c], dq);
+      }
+      T* out = a.out + z * a.dz + hd * a.dh + 16 * dh + (ln & 15);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int q = 32 * t + 16 * qh + 4 * g4 + i;
+        if (q < S) out[(int64_t)q * a.ds] = (T)(dq[i] * a.scale);
+      }
+    }
+  }
+  if constexpr (DB1) {
+    colsum += __shfl_xor(colsum, 32, 64);
+    const int k = 32 * wid + (threadIdx.x & 63);
+    if ((threadIdx.x & 63) < 32 && k < S) unsafeAtomicAdd(a.db1 + (int64_t)z * S + k, colsum);
+  }
+  // this wave's rows of dK and dV through its rows of the Q and dO images, which nobody reads any more, into 16-byte pieces
+  int ln = tid & 63;
+  asm volatile("" : "+v"(ln));
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int at = (32 * wid + crow(r, ln >> 5)) * 64 + (ln & 31) * 2;
+    *reinterpret_cast<T*>(Qi + at) = (T)(dk[r] * a.scale);
+    *reinterpret_cast<T*>(Gi + at) = (T)dv[r];
+  }
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = 32 * wid + 16 * i + (ln >> 2), ch = ln & 3;
+    const u32x4_t k4 = *reinterpret_cast<const u32x4_t*>(Qi + r * 64 + ch * 16), v4 = *reinterpret_cast<const u32x4_t*>(Gi + r * 64 + ch * 16);
+    if (r < S) {
+      const int64_t at = (((int64_t)z * S + r) * a.H + hd) * 32 + ch * 8;
+      *reinterpret_cast<u32x4_t*>(a.dk + at) = k4;
+      *reinterpret_cast<u32x4_t*>(a.dv + at) = v4;
+    }
+  }
+}
+
 // ---------------------------------------------------------------- pass 3: dB2 summed over the z sharing it
 template <typename T, int D, bool DROP>
 __global__ void __launch_bounds__(NTHR, 2) small_bwd_db2_kernel(SmallArgs<T> a) {
@@ -865,6 +1104,32 @@ int db2_splits(int Z, int H, int S, int b2_div) {
   return b2_div == 1 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(b2_div / 4, 512 / base));
 }
 
+// Elements of the pair bias in the accumulators' order, for what goes through one pass for dQ, dK and dV; 0: two passes. Pair biases
+// of their own for every z would be read and written once more than they are used, and fewer than a workgroup a CU leave the chip
+// idle (dQ, dK and dV in two passes and in one, us: [32, 256, 4, 32] 23 and 24, [24, 40, 4, 32] 13 and 14; [128, 200, 4, 32] 54 and 36,
+// [100, 133, 8, 32] 69 and 49, [512, 32, 8, 32] 61 and 23, [256, 250, 8, 32] 185 and 133).
+int64_t small_order_elements(int Z, int H, int S, int D, int b2_div, bool drop) {
+  const int64_t nt = (S + 31) / 32;
+  return D == 32 && S <= WHOLE_S && !drop && b2_div > 1 && (int64_t)Z * H >= 256 ? (int64_t)(Z / b2_div) * H * nt * nt * 1024 : 0;
+}
+
+template <typename T, bool DB1>
+int launch_whole(const SmallArgs<T>& a, hipStream_t st) {
+  static bool attr = false;
+  if (!attr) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&small_bwd_whole_kernel<T, DB1>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              WHOLE_LDS);
+    attr = true;
+  }
+  const int nt = (a.S + 31) / 32;
+  const int64_t tiles = (int64_t)(a.Z / a.b2_div) * a.H * nt * nt;
+  hipLaunchKernelGGL(small_bias_order_kernel<T>, dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, st, a.b2, a.order, a.S, nt, tiles);
+  DS_CHECK_LAUNCH();
+  hipLaunchKernelGGL((small_bwd_whole_kernel<T, DB1>), dim3(a.H * a.Z), dim3(64 * nt), WHOLE_LDS / 8 * nt, st, a, (const T*)a.order);
+  DS_CHECK_LAUNCH();
+  return 0;
+}
+
 template <typename T, int D, bool DROP, bool PAIR>
 int launch_small(SmallArgs<T> a, bool bwd, hipStream_t st) {
   const int nqb = (a.S + BM - 1) / BM;
@@ -874,10 +1139,20 @@ int launch_small(SmallArgs<T> a, bool bwd, hipStream_t st) {
     DS_CHECK_LAUNCH();
     return 0;
   }
-  hipLaunchKernelGGL((small_bwd_dq_kernel<T, D, DROP, PAIR>), grid, dim3(NTHR), 0, st, a);
-  DS_CHECK_LAUNCH();
-  hipLaunchKernelGGL((small_bwd_dkv_kernel<T, D, DROP, PAIR>), grid, dim3(NTHR), 0, st, a);
-  DS_CHECK_LAUNCH();
+  bool whole = false;
+  if constexpr (D == 32 && !DROP && PAIR) {
+    if (small_order_elements(a.Z, a.H, a.S, D, a.b2_div, false) > 0) {
+      whole = true;
+      if (a.order == nullptr) return (int)hipErrorInvalidValue;
+      if (int rc = a.db1 ? launch_whole<T, true>(a, st) : launch_whole<T, false>(a, st)) return rc;
+    }
+  }
+  if (!whole) {
+    hipLaunchKernelGGL((small_bwd_dq_kernel<T, D, DROP, PAIR>), grid, dim3(NTHR), 0, st, a);
+    DS_CHECK_LAUNCH();
+    hipLaunchKernelGGL((small_bwd_dkv_kernel<T, D, DROP, PAIR>), grid, dim3(NTHR), 0, st, a);
+    DS_CHECK_LAUNCH();
+  }
   if (PAIR && a.db2 && a.b2_div > 1) {
     a.nsplit = db2_splits(a.Z, a.H, a.S, a.b2_div);
     if (a.nsplit > 1 && a.part == nullptr) return (int)hipErrorInvalidValue;
@@ -921,7 +1196,7 @@ extern "C" int ds_flash_small_fwd(const void* q, const void* k, const void* v, v
 #define DS_SMALL_ARGS(T)                                                                                        \
   SmallArgs<T> a{(const T*)q, (const T*)k, (const T*)v, nullptr, nullptr, (T*)o, lse, (const T*)b1, (const T*)b2, \
                  nullptr, nullptr, nullptr, nullptr, nullptr, st[0], st[1], st[2], st[3], st[4], st[5], st[6], st[7],     \
-                 st[8], st[9], st[10], st[11], 0, 0, 0, 0, 0, 0, b1_zs, Z, H, S, b2_div, scale, pdrop, thresh, seed, b2_numel - 8, 1, nullptr, Sk};
+                 st[8], st[9], st[10], st[11], 0, 0, 0, 0, 0, 0, b1_zs, Z, H, S, b2_div, scale, pdrop, thresh, seed, b2_numel - 8, 1, nullptr, nullptr, Sk};
   if (dtype == DS_BF16) {
     DS_SMALL_ARGS(bf16)
     return dispatch_small<bf16>(a, D, false, stream);
@@ -939,9 +1214,14 @@ extern "C" int ds_flash_small_fwd(const void* q, const void* k, const void* v, v
 // `ds_flash_small_db2_splits` times as much scratch when that is more than one.
 extern "C" int ds_flash_small_db2_splits(int Z, int H, int S, int b2_div) { return db2_splits(Z, H, S, b2_div); }
 
+// order: ds_flash_small_order elements of the inputs' type when that is not zero
+extern "C" int64_t ds_flash_small_order(int Z, int H, int S, int D, int b2_div, float pdrop, int has_b2) {
+  return has_b2 ? small_order_elements(Z, H, S, D, b2_div, pdrop > 0.f) : 0;
+}
+
 extern "C" int ds_flash_small_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout,
                                   const float* lse, const void* b1, const void* b2, void* dq, void* dk, void* dv,
-                                  float* delta, float* db1, float* db2, float* db2_part, const int64_t* st, int64_t b1_zs, int Z, int H, int S, int D,
+                                  float* delta, float* db1, float* db2, float* db2_part, void* order, const int64_t* st, int64_t b1_zs, int Z, int H, int S, int D,
                                   int b2_div, float scale, float pdrop, uint64_t seed, int64_t b2_numel, int dtype,
                                   hipStream_t stream) {
   if (Z <= 0 || H <= 0 || S <= 0 || b2_div <= 0 || (D != 32 && D != 64) || pdrop < 0.f || pdrop >= 1.f ||
@@ -952,7 +1232,7 @@ extern "C" int ds_flash_small_bwd(const void* q, const void* k, const void* v, c
   SmallArgs<T> a{(const T*)q, (const T*)k, (const T*)v, (const T*)o, (const T*)dout, (T*)dq, (float*)lse,           \
                  (const T*)b1, (const T*)b2, (T*)dk, (T*)dv, delta, db1, db2, st[0], st[1], st[2], st[3], st[4], st[5], st[6],      \
                  st[7], st[8], st[9], st[10], st[11], st[12], st[13], st[14], st[15], st[16], st[17], b1_zs, Z, H, S, b2_div, scale, pdrop, \
-                 thresh, seed, b2_numel - 8, 1, db2_part, S};
+                 thresh, seed, b2_numel - 8, 1, db2_part, (T*)order, S};
   if (dtype == DS_BF16) {
     DS_SMALL_ARGS(bf16)
     return dispatch_small<bf16>(a, D, true, stream);

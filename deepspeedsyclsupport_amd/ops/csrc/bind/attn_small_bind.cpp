@@ -12,8 +12,9 @@ int ds_flash_small_fwd(const void*, const void*, const void*, void*, float*, con
                        const int64_t*, int64_t, int, int, int, int, int, int, float, float, uint64_t, int64_t, int,
                        hipStream_t);
 int ds_flash_small_bwd(const void*, const void*, const void*, const void*, const void*, const float*, const void*,
-                       const void*, void*, void*, void*, float*, float*, float*, float*, const int64_t*, int64_t, int, int, int,
+                       const void*, void*, void*, void*, float*, float*, float*, float*, void*, const int64_t*, int64_t, int, int, int,
                        int, int, float, float, uint64_t, int64_t, int, hipStream_t);
+int64_t ds_flash_small_order(int, int, int, int, int, float, int);
 int ds_flash_small_db2_splits(int, int, int, int);
 }
 
@@ -133,12 +134,16 @@ std::vector<Tensor> flash_small_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, T
   } else {
     db2 = torch::empty({0}, f32);
   }
+  Tensor order;
+  if (const int64_t n = ds_flash_small_order((int)Z, (int)H, (int)S, (int)D, (int)b2_div, (float)pdrop, bs.b2 != nullptr))
+    order = torch::empty({n}, q.options());
   std::vector<int64_t> st;
   push(st, q); push(st, k); push(st, v); push(st, o); push(st, dout); push(st, dq);
   check(ds_flash_small_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dout.data_ptr(),
                            lse.data_ptr<float>(), bs.b1, bs.b2, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
                            delta.data_ptr<float>(), want_db1 ? db1.data_ptr<float>() : nullptr,
-                           want_db2 ? db2.data_ptr<float>() : nullptr, part.defined() ? part.data_ptr<float>() : nullptr, st.data(), bs.b1_zs, (int)Z, (int)H, (int)S,
+                           want_db2 ? db2.data_ptr<float>() : nullptr, part.defined() ? part.data_ptr<float>() : nullptr,
+                           order.defined() ? order.data_ptr() : nullptr, st.data(), bs.b1_zs, (int)Z, (int)H, (int)S,
                            (int)D, (int)b2_div, (float)scale, (float)pdrop, (uint64_t)seed, bs.b2_numel, dcode(q),
                            at::hip::getCurrentHIPStream().stream()),
         "flash_small_bwd");

@@ -182,3 +182,25 @@ def test_a_row_of_the_pair_bias_stays_with_its_query(D, S, bad):
     for name, clean, other in zip(("o", "dq"), *got):
         assert torch.isnan(other[:, rows]).any(), name
         assert torch.equal(clean[:, ~rows], other[:, ~rows]), name
+
+
+@pytest.mark.parametrize("dtype,masked", [(torch.bfloat16, True), (torch.float16, False)])
+@pytest.mark.parametrize("Z,S,H,b2_div", [(256, 1, 1, 256), (128, 31, 2, 64), (86, 33, 3, 43), (64, 130, 4, 64), (40, 225, 7, 20),
+                                          (32, 256, 8, 16), (32, 257, 8, 16)])
+def test_short_sequences_in_one_pass(Z, S, H, b2_div, dtype, masked):
+    """Enough short sequences that one pass makes dQ, dK and dV (257: two again): one to eight tiles of 32 with remainders, a pair
+    bias at odd addresses, with a per-key mask and its gradient and without."""
+    q, k, v, bias1, bias2 = _case(Z, S, H, 32, dtype, masked, True, b2_div, seed=5)
+    if masked:
+        bias1[0, 1:] = torch.finfo(dtype).min
+    odd = torch.empty(bias2.numel() + 1, device="cuda", dtype=dtype)[1:].view_as(bias2).copy_(bias2)
+    ins = [t if t is None else t.detach().requires_grad_(True) for t in (q, k, v, bias1, odd)]
+    refs = [t if t is None else t.detach().double().requires_grad_(True) for t in (q, k, v, bias1, bias2)]
+    out, ref = FS.flash_small(*ins, b2_div=b2_div), FS.reference(*refs, b2_div=b2_div)
+    go = torch.randn(ref.shape, device="cuda")
+    out.backward(go.to(dtype))
+    ref.backward(go.to(dtype).double())
+    tol = 4e-2 if dtype == torch.bfloat16 else 1e-2   # as above
+    for name, a, r in zip(("dq", "dk", "dv", "db1", "db2"), ins, refs):
+        if a is not None:
+            assert (a.grad.double() - r.grad).abs().max() < tol * r.grad.abs().max() + tol, name
