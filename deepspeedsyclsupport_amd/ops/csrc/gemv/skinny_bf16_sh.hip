@@ -19,6 +19,8 @@
 //    blocks (no norm) leave as sums, and a second launch pairs them;
 //  * X is read once per workgroup (from L2), which is what bounds wide batches; RB and the parts trade that against workgroups
 //    enough.
+// Two workgroups fit a CU with up to four blocks (128 registers a lane: 33 rows x gated [28672, 4096] 54 us with one, 47 with two), one
+// with eight.
 // Bound by the weights' read (6.5 TB/s here). Measured, us (the same products as split streams with fp32 atomics and a finalize
 // pass; the floor): 12 rows x [4096, 4096] 9 (14; 5), [4096, 14336] 23 (25; 18), gated [28672, 4096] 38 (45; 36), with the
 // norm 39, [32000, 4096] 42 (51; 40), [2048, 2048] 5.6 (7.6; 1.3). 24 and 40 rows (library GEMM): gated [28672, 4096] 44 and 51 (60
@@ -62,6 +64,14 @@ struct Int {
   static constexpr int value = V;
 };
 
+// The address as a wave's base and a lane's bytes. APART: the asm keeps it so, and the base in scalar registers: 10 to 20 vector
+// registers less. (Few token rows have them to spare: a step of one sequence took 0.2 % longer with it.)
+template <bool APART>
+__device__ __forceinline__ const bf16x8_t* at(const bf16* base, uint32_t bytes) {
+  if constexpr (APART) asm("" : "+v"(bytes));
+  return reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const char*>(base) + bytes);
+}
+
 // Token row `row`, columns n .. n + 3 of a product without a gate: bias, activation, residual
 __device__ __forceinline__ void store_plain(const ShArgs& a, f32x4 v, int row, int n) {
 #pragma unroll
@@ -97,7 +107,7 @@ __device__ __forceinline__ float gate_up(const ShArgs& a, float g, float up, int
 }
 
 template <int MT, int RB, bool NORM, bool GATED>
-__global__ void __launch_bounds__(WAVES * 64, (MT <= 2 ? 4 : 2)) decode_gemm_kernel(ShArgs a) {
+__global__ void __launch_bounds__(WAVES * 64, (MT <= 2 || RB == 4 ? 4 : 2)) decode_gemm_kernel(ShArgs a) {
   static_assert(!GATED || RB % 2 == 0, "pairs");
   constexpr int T = MT * RB, HALF = WAVES / 2;
   constexpr int U = T == 1 ? 2 : 1;  // steps loaded together
@@ -118,12 +128,11 @@ __global__ void __launch_bounds__(WAVES * 64, (MT <= 2 ? 4 : 2)) decode_gemm_ker
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
     const int last = GATED ? (i < RB / 2 ? HB : 2 * HB) - 1 : NB - 1;
-    wp[i] = a.w + (int64_t)min(block_of(i), last) * KQ * 1024 + lane * 8;
+    wp[i] = a.w + (int64_t)min(block_of(i), last) * KQ * 1024;
   }
-  const bf16* xp[MT];
+  uint32_t xo[MT];  // bytes
 #pragma unroll
-  for (int m = 0; m < MT; ++m) xp[m] = a.x + (int64_t)min(16 * m + l16, a.M - 1) * K + 16 * q4;
-  const bf16* np = NORM ? a.norm_w + 16 * q4 : nullptr;
+  for (int m = 0; m < MT; ++m) xo[m] = ((uint32_t)min(16 * m + l16, a.M - 1) * K + 16 * q4) * 2;
 
   f32x4 acc[RB][MT];
   float ss[MT];
@@ -146,15 +155,15 @@ __global__ void __launch_bounds__(WAVES * 64, (MT <= 2 ? 4 : 2)) decode_gemm_ker
 #pragma unroll
         for (int i = 0; i < RB; ++i)
           f.w[u][h][i] = __builtin_nontemporal_load(
-              reinterpret_cast<const bf16x8_t*>(wp[i] + (int64_t)min(s0 + WAVES * u, end - 1) * 1024 + 512 * h));
+              at<MT == 3>(wp[i] + (int64_t)min(s0 + WAVES * u, end - 1) * 1024 + 512 * h, lane * 16));
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int k = min(s0 + WAVES * u, end - 1) * 64 + 8 * h;
-        if constexpr (NORM) f.norm[u][h] = *reinterpret_cast<const bf16x8_t*>(np + k);
+        if constexpr (NORM) f.norm[u][h] = *at<MT == 3>(a.norm_w + k, 32 * q4);
 #pragma unroll
-        for (int m = 0; m < MT; ++m) f.x[u][h][m] = *reinterpret_cast<const bf16x8_t*>(xp[m] + k);
+        for (int m = 0; m < MT; ++m) f.x[u][h][m] = *at<MT == 3>(a.x + k, xo[m]);
       }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -325,6 +334,11 @@ struct Cut {
 // 14; 48 rows with two / four: [8192, 4096] 19 / 24, [9216, 3072] 28 / 19, [12288, 4096] 35 / 26). Products with more blocks than that
 // holds take the most that there are (24 rows x [32000, 4096] 48 with two, 46 with four), up to 16 token rows two (12 rows 42 and 45).
 // Gated pairs take two or four (12 rows: [11264, 2048] 13.0 and 11.0, [28672, 4096] 41 and 38).
+// Eight blocks for 33 rows and more of 4096 and more, where they still make more than 144 workgroups: X, a quarter to a half of what a
+// CU reads, is then read half as often. 33 / 48 rows, us with four and with eight: gated [22016, 4096] 47 / 51 and 41 / 42, [28672, 4096]
+// 47 / 51.5 and 49 / 51, [57344, 8192] 170 / 187 and 158 / 160, [32000, 4096] 52 / 58 and 49 / 49, [20480, 5120] 53 / 59 and 45 / 48. Fewer
+// workgroups leave too many CUs idle (48 rows x [16384, 8192], 128 of them, 51 and 67), and X of 2048 gives nothing (48 rows x
+// [32000, 2048] 29.1 and 31.6). Up to 32 rows it pays for long X alone (32 rows x gated [28672, 4096] 46 and 49).
 // More than 16 token rows of 4096 and more over few blocks: what a CU can read (30 bytes a nanosecond) bounds one block's workgroup,
 // and of that most is X. Several blocks share the reading, and parts of K keep the workgroups at 256; the parts' sums are a launch of
 // 4 us. 48 rows, us with one block and with this: [4096, 4096] 16.3 and 14.6, [4096, 14336] 45 and 28, [2048, 5632] 20.6 and 13.5; 17
@@ -337,7 +351,7 @@ struct Cut {
 // 6.9, x [1024, 8192] 9.6 and 8.4), and where long ones stand a quarter over one round (16 rows x [10240, 8192] 40 and 35).
 Cut cut_of(int M, int N, int K, bool gated, bool norm) {
   const int blocks = gated ? N / 16 : (N + 15) / 16, mt = (M + 15) / 16, most = gated || mt > 1 ? 4 : 2;
-  int rb = blocks <= 256 && !gated ? 1 : blocks <= 512 ? 2 : most, parts = 1;
+  int rb = blocks <= 256 && !gated ? 1 : blocks <= 512 ? 2 : mt == 3 && blocks > 1152 && K >= 4096 ? 8 : most, parts = 1;
   if (!gated && !norm) {
     int fill = 0;  // workgroups that parts may make
     if (mt == 1) {
@@ -351,9 +365,10 @@ Cut cut_of(int M, int N, int K, bool gated, bool norm) {
     }
     parts = max(min(min(fill / ((blocks + rb - 1) / rb), K / 1024), 8), 1);  // (K / 1024: two steps a wave)
   }
-  if (g_blocks) rb = g_blocks >= 4 ? 4 : g_blocks == 3 ? 2 : g_blocks;
+  if (g_blocks) rb = g_blocks >= 8 ? 8 : g_blocks >= 4 ? 4 : g_blocks == 3 ? 2 : g_blocks;
   if (gated && rb < 2) rb = 2;
-  if (!gated && mt == 1 && rb == 4) rb = 2;
+  if (mt < 3 && rb == 8) rb = 4;
+  if (mt == 1 && !gated && rb == 4) rb = 2;
   if (g_parts && !gated && !norm) parts = min(g_parts, K / 64);
   return {rb, parts};
 }
@@ -380,7 +395,7 @@ int launch(const ShArgs& a, bool gated, bool loose, hipStream_t st) {
 
 }  // namespace
 
-// Forces blocks per workgroup (1, 2, 4, where the product has such a kernel) and parts of K; 0: by the rule above.
+// Forces blocks per workgroup (1, 2, 4, 8, where the product has such a kernel) and parts of K; 0: by the rule above.
 extern "C" void ds_skinny_b16_tune(int cfg, int parts) { g_blocks = cfg; g_parts = parts; }
 
 extern "C" int ds_decode_gemm_ok(int M, int K) { return M >= 1 && M <= 48 && K >= 64 && K % 64 == 0; }
@@ -415,11 +430,14 @@ extern "C" int ds_decode_gemm(const void* X, const void* Wsh, const void* bias, 
   else if (!part) return (int)hipErrorInvalidValue;
   const ShArgs a{(const bf16*)X, (const bf16*)Wsh, (const bf16*)bias, (const bf16*)norm_w, (const bf16*)res, (bf16*)Y, M, N, K,
                  eps, act, limit, cut.parts, (f32x4*)part};
-#define GO(MT)                                         \
-  switch (cut.blocks) {                                \
-    case 1: return launch<MT, 1>(a, gated, loose, st); \
-    case 2: return launch<MT, 2>(a, gated, loose, st); \
-    default: return launch<MT, 4>(a, gated, loose, st); \
+#define GO(MT)                                                          \
+  switch (cut.blocks) {                                                 \
+    case 1: return launch<MT, 1>(a, gated, loose, st);                  \
+    case 2: return launch<MT, 2>(a, gated, loose, st);                  \
+    case 4: return launch<MT, 4>(a, gated, loose, st);                  \
+    default:                                                            \
+      if constexpr (MT == 3) return launch<MT, 8>(a, gated, loose, st); \
+      return (int)hipErrorInvalidValue;                                 \
   }
   switch ((M + 15) / 16) {
     case 1: GO(1)
