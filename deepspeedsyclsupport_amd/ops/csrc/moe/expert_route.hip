@@ -30,81 +30,93 @@ struct RouteArgs {
   int* slots;        // [T, K]: place of the pair within its expert's
 };
 
-// One wave: logits z [E] of a token in LDS (overwritten), gs scratch [groups]
-__device__ __forceinline__ void choose(float* z, float* gs, int tok, const RouteArgs& a, int* hist) {
+// The largest of the wave's values, in registers alone (a step of the ladder is one instruction with a lane move; a shuffle goes
+// through LDS)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float max_step(float v) {
+  const int b = __float_as_int(v);
+  return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(b, b, CTRL, ROWS, 0xf, false)));
+}
+__device__ __forceinline__ float max_all(float v) {
+  v = max_step<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: lane 15 of each 16 has their largest
+  v = max_step<0x112, 0xf>(v);
+  v = max_step<0x114, 0xf>(v);
+  v = max_step<0x118, 0xf>(v);
+  v = max_step<0x142, 0xa>(v);  // lane 15 to the next 16, lane 31 to the upper half
+  v = max_step<0x143, 0xc>(v);
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+// One wave: logits z [E] of a token in LDS (overwritten), gs scratch [groups], up to 64 NI experts. Lane k gets choice k and, with
+// hist, its place among the workgroup's pairs of that expert.
+template <int NI>
+__device__ __forceinline__ void choose(float* z, float* gs, int tok, const RouteArgs& a, int* hist, int& my_e, int& my_slot) {
   const int lane = threadIdx.x & 63, E = a.E, per = E / a.groups;
-  float s[MAXE / 64], mx = -INFINITY, den = 0.f;
+  float s[NI], mx = -INFINITY, den = 0.f;
 #pragma unroll
-  for (int i = 0; i < MAXE / 64; ++i) {
+  for (int i = 0; i < NI; ++i) {
     s[i] = lane + 64 * i < E ? z[lane + 64 * i] : -INFINITY;
     mx = fmaxf(mx, s[i]);
   }
   if (a.sigmoid) {
 #pragma unroll
-    for (int i = 0; i < MAXE / 64; ++i) s[i] = 1.f / (1.f + expf(-s[i]));
+    for (int i = 0; i < NI; ++i) s[i] = 1.f / (1.f + expf(-s[i]));
   } else {
-    mx = wave_max(mx);
+    mx = max_all(mx);
 #pragma unroll
-    for (int i = 0; i < MAXE / 64; ++i) {
+    for (int i = 0; i < NI; ++i) {
       s[i] = lane + 64 * i < E ? expf(s[i] - mx) : 0.f;
       den += s[i];
     }
     den = wave_sum(den);
 #pragma unroll
-    for (int i = 0; i < MAXE / 64; ++i) s[i] /= den;
+    for (int i = 0; i < NI; ++i) s[i] /= den;
   }
+  if (a.keep < a.groups) {
 #pragma unroll
-  for (int i = 0; i < MAXE / 64; ++i)
-    if (lane + 64 * i < E) z[lane + 64 * i] = s[i];
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  for (int g = lane; g < a.groups; g += 64) {
-    float b = 0.f, c = 0.f;
-    for (int e = g * per; e < (g + 1) * per; ++e) {
-      c = fmaxf(c, fminf(b, z[e]));
-      b = fmaxf(b, z[e]);
+    for (int i = 0; i < NI; ++i)
+      if (lane + 64 * i < E) z[lane + 64 * i] = s[i];
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int g = lane; g < a.groups; g += 64) {
+      float b = 0.f, c = 0.f;
+      for (int e = g * per; e < (g + 1) * per; ++e) {
+        c = fmaxf(c, fminf(b, z[e]));
+        b = fmaxf(b, z[e]);
+      }
+      gs[g] = a.best == 2 ? b + c : b;
     }
-    gs[g] = a.best == 2 ? b + c : b;
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-  for (int i = 0; i < MAXE / 64; ++i) {
+  for (int i = 0; i < NI; ++i) {
     const int e = lane + 64 * i;
     if (e >= E) {
       s[i] = -1.f;
-      continue;
+    } else if (a.keep < a.groups) {
+      const int g = e / per;
+      const float b = gs[g];
+      int better = 0;
+      for (int o = 0; o < a.groups; ++o) better += gs[o] > b || (gs[o] == b && o < g);
+      if (better >= a.keep) s[i] = -1.f;
     }
-    const int g = e / per;
-    const float b = gs[g];
-    int better = 0;
-    for (int o = 0; o < a.groups; ++o) better += gs[o] > b || (gs[o] == b && o < g);
-    if (better >= a.keep) s[i] = -1.f;
   }
-  float mine = 0.f, sum = 0.f;  // lane k keeps choice k
-  int my_e = 0;
+  float mine = 0.f, sum = 0.f;
   for (int k = 0; k < a.K; ++k) {
     float bv = -1.f;
-    int be = MAXE;
+    int be = E - 1;  // logits that are not numbers choose nothing: stay in bounds
 #pragma unroll
-    for (int i = 0; i < MAXE / 64; ++i)
-      if (s[i] > bv) {
-        bv = s[i];
-        be = lane + 64 * i;
-      }
+    for (int i = 0; i < NI; ++i) bv = fmaxf(bv, s[i]);
+    bv = max_all(bv);
+    if (bv > -1.f) {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int oe = __shfl_xor(be, o, 64);
-      if (ov > bv || (ov == bv && oe < be)) {
-        bv = ov;
-        be = oe;
-      }
+      for (int i = NI - 1; i >= 0; --i)
+        if (const uint64_t at = __ballot(s[i] == bv)) be = 64 * i + __builtin_ctzll(at);
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        if (be == lane + 64 * i) s[i] = -1.f;
     }
-#pragma unroll
-    for (int i = 0; i < MAXE / 64; ++i)
-      if (be == lane + 64 * i) s[i] = -1.f;
-    be = min(be, E - 1);      // (logits that are not numbers choose nothing: stay in bounds)
     sum += bv;
     if (lane == k) {
       mine = bv;
@@ -115,23 +127,24 @@ __device__ __forceinline__ void choose(float* z, float* gs, int tok, const Route
     const int64_t i = (int64_t)tok * a.K + lane;
     a.experts[i] = my_e;
     a.weights[i] = mine / (sum + 1e-20f) * a.scale;
-    if (hist) a.slots[i] = atomicAdd(hist + my_e, 1);  // within the workgroup; the base is added below
+    if (hist) my_slot = atomicAdd(hist + my_e, 1);
   }
 }
 
-// The workgroup's pairs take a run of every expert's places
-__device__ __forceinline__ void claim(const RouteArgs& a, int first, int n, int* hist) {
+// The workgroup's pairs take a run of every expert's places; afterwards hist holds where it begins
+__device__ __forceinline__ void claim(const RouteArgs& a, int* hist) {
   __syncthreads();
   for (int e = threadIdx.x; e < a.E; e += blockDim.x)
     if (const int c = hist[e]) hist[e] = atomicAdd(a.counts + e, c);
   __syncthreads();
-  for (int i = threadIdx.x; i < n * a.K; i += blockDim.x) {
-    const int64_t p = (int64_t)first * a.K + i;
-    a.slots[p] += hist[a.experts[p]];
-  }
 }
 
-// bf16, W a multiple of 8. NW waves share the width of 16 TM tokens and up to 16 ET experts.
+// bf16, W a multiple of 8. NW waves share the width of 16 TM tokens and up to 16 ET experts. With few tokens there is one workgroup,
+// and what bounds it is a CU's path to memory (35 bytes a nanosecond) and then the chain of steps that follows; so the
+// width's remainder is loaded by 4, 2 and 1 steps at a time, the waves' shares meet after two barriers, the maxima of the choice stay
+// in registers, and places go to memory once. us before and after: 16 tokens of 2048 among 32 experts 13.2 and 10.0, 64 tokens
+// among 64 experts with lists 28 and 21, 64 of 4096 among 128 73 and 43, 8192 of 4096 among 32 43 and 34. (Whole cache lines a wave,
+// or all loads held ahead of the products, measured the same.)
 template <int ET, int TM, int NW>
 __global__ void __launch_bounds__(64 * NW) route_mfma_kernel(const bf16* __restrict__ h, const bf16* __restrict__ rw,
                                                              RouteArgs a) {
@@ -182,37 +195,61 @@ __global__ void __launch_bounds__(64 * NW) route_mfma_kernel(const bf16* __restr
   const int whole = a.W / 32;
   int k = w;
   for (; k + NW * (U - 1) < whole; k += NW * U) steps(Int<U>{}, 32 * k, false);
-  for (; k < whole; k += NW) steps(Int<1>{}, 32 * k, false);
+  if constexpr (U == 8)
+    if (k + NW * 3 < whole) {
+      steps(Int<4>{}, 32 * k, false);
+      k += NW * 4;
+    }
+  if constexpr (U >= 4)
+    if (k + NW < whole) {
+      steps(Int<2>{}, 32 * k, false);
+      k += NW * 2;
+    }
+  if (k < whole) steps(Int<1>{}, 32 * k, false);
   if (a.W % 32 && whole % NW == w) steps(Int<1>{}, 32 * whole, true);
-#pragma unroll
-  for (int half = NW / 2; half >= 1; half /= 2) {  // the waves' shares, pairwise
-    if (w >= half && w < 2 * half) {
-#pragma unroll
-      for (int m = 0; m < TM; ++m)
-#pragma unroll
-        for (int e = 0; e < ET; ++e) red[w - half][m * ET + e][lane] = acc[m][e];
-    }
-    __syncthreads();
-    if (w < half) {
-#pragma unroll
-      for (int m = 0; m < TM; ++m)
-#pragma unroll
-        for (int e = 0; e < ET; ++e) acc[m][e] += red[w][m * ET + e][lane];
-    }
-    __syncthreads();
-  }
-  if (w == 0) {
+  // the waves' shares: pairs of them in their registers, the rest spread over all threads, always in the same order
+  constexpr int H = NW / 2;
+  if (w >= H) {
 #pragma unroll
     for (int m = 0; m < TM; ++m)
 #pragma unroll
-      for (int e = 0; e < ET; ++e)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)  // token 16 m + l16, expert 16 e + 4 q4 + r
-          z[(16 * m + l16) * ZP + 16 * e + 4 * q4 + r] = acc[m][e][r];
+      for (int e = 0; e < ET; ++e) red[w - H][m * ET + e][lane] = acc[m][e];
   }
   __syncthreads();
-  for (int i = w; i < n; i += NW) choose(z + i * ZP, gs[w], t0 + i, a, a.counts ? hist : nullptr);
-  if (a.counts) claim(a, t0, n, hist);
+  if (w < H) {
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int e = 0; e < ET; ++e) red[w][m * ET + e][lane] += acc[m][e];
+  }
+  __syncthreads();
+  for (int i = tid; i < TM * ET * 64; i += 64 * NW) {
+    const int c = i / 64, m = c / ET, e = c % ET;  // lane = tid % 64 throughout
+    f32x4 v[H];
+#pragma unroll
+    for (int j = 0; j < H; ++j) v[j] = red[j][c][lane];
+#pragma unroll
+    for (int half = H / 2; half >= 1; half /= 2)
+#pragma unroll
+      for (int j = 0; j < half; ++j) v[j] += v[j + half];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)  // token 16 m + l16, expert 16 e + 4 q4 + r
+      z[(16 * m + l16) * ZP + 16 * e + 4 * q4 + r] = v[0][r];
+  }
+  __syncthreads();
+  int my_e[TOK / NW], my_slot[TOK / NW];
+#pragma unroll
+  for (int j = 0; j < TOK / NW; ++j) {
+    const int i = w + NW * j;
+    if (i < n) choose<(ET + 3) / 4>(z + i * ZP, gs[w], t0 + i, a, a.counts ? hist : nullptr, my_e[j], my_slot[j]);
+  }
+  if (!a.counts) return;
+  claim(a, hist);
+#pragma unroll
+  for (int j = 0; j < TOK / NW; ++j) {
+    const int i = w + NW * j;
+    if (i < n && lane < a.K) a.slots[(int64_t)(t0 + i) * a.K + lane] = hist[my_e[j]] + my_slot[j];
+  }
 }
 
 // fp32, or widths the matrix kernel does not take: a workgroup per token
@@ -231,8 +268,11 @@ __global__ void __launch_bounds__(256) route_any_kernel(const T* __restrict__ h,
     if (lane == 0) z[e] = s;
   }
   __syncthreads();
-  if (threadIdx.x < 64) choose(z, gs, t, a, a.counts ? hist : nullptr);
-  if (a.counts) claim(a, t, 1, hist);
+  int my_e = 0, my_slot = 0;
+  if (threadIdx.x < 64) choose<MAXE / 64>(z, gs, t, a, a.counts ? hist : nullptr, my_e, my_slot);
+  if (!a.counts) return;
+  claim(a, hist);
+  if (threadIdx.x < a.K) a.slots[(int64_t)t * a.K + threadIdx.x] = hist[my_e] + my_slot;
 }
 
 // Exclusive prefix of counts [E] in LDS (pre[E]: the total), by the first wave

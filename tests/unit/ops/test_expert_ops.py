@@ -90,6 +90,39 @@ def test_route(device, dtype, tol, E, top, groups, keep, W, T):
     assert (full - got)[same.all(-1)].abs().max() < 1e-5
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,top,groups,keep,best,W,T", [(16, 1, 1, 1, 1, 7712, 17), (32, 4, 4, 2, 1, 2048, 16), (32, 32, 4, 4, 2, 4616, 4097),
+                                                        (33, 8, 3, 2, 2, 1312, 9), (64, 5, 8, 4, 1, 1920, 4100), (192, 64, 4, 2, 2, 808, 5)])
+@pytest.mark.parametrize("sigmoid", [0, 1])
+def test_route_widths_and_ties(E, top, groups, keep, best, W, T, sigmoid):
+    """Widths that end in every number of steps a wave takes at once, whole and partial; all experts alike in pairs, so that every
+    choice is a tie and goes to the lower index; logits that are not numbers choose expert E - 1. fp32 sums of W products are off by at
+    most W 2^-23 of their magnitudes' sum; here the operands are small integers and every sum is exact."""
+    from deepspeedsyclsupport_amd.ops.native import expert_ops as native
+    h = torch.randint(-2, 3, (T, W)).bfloat16()
+    r = torch.zeros(E, W)
+    r[torch.arange(E)[:, None], torch.stack([torch.randperm(W)[:8] for _ in range(E)])] = 1.0
+    r[1::2] = r[:E - E % 2:2]
+    h[-1] = float("nan")
+    e, w, offs, order, at = native().route(h.cuda(), r.bfloat16().cuda(), top, groups, keep, True, sigmoid, best, 2.0)
+    z = h[:-1].double() @ r.double().t()
+    s = z.sigmoid() if sigmoid else z.softmax(-1)
+    z = z.view(T - 1, groups, -1)
+    per = z.shape[-1]
+    g = s.view(T - 1, groups, per).sort(-1, descending=True).values[..., :min(best, per)].float().sum(-1)
+    alive = torch.zeros(T - 1, groups, dtype=torch.bool).scatter_(1, g.sort(dim=-1, descending=True, stable=True).indices[:, :keep], True)
+    masked = s.masked_fill(~alive.repeat_interleave(per, 1), -1.0)
+    want = z.reshape(T - 1, E).masked_fill(~alive.repeat_interleave(per, 1), -1e9).sort(dim=-1, descending=True, stable=True).indices[:, :top]
+    assert (e.cpu()[:-1].long() == want).float().mean() > 0.999  # (groups whose sums of two are equal but for rounding)
+    picked = masked.gather(1, e.cpu()[:-1].long())
+    torch.testing.assert_close(w.cpu()[:-1].double(), 2.0 * picked / picked.sum(-1, keepdim=True), rtol=2e-5, atol=1e-7)
+    assert (e[-1] == E - 1).all()
+    flat = e.view(-1).cpu().long()
+    assert torch.equal(offs[1:].cpu(), torch.bincount(flat, minlength=E).cumsum(0).int())
+    assert torch.equal(flat[order.cpu().long()], flat.sort().values) and torch.equal(order[at.view(-1).long()].cpu().long(),
+                                                                                     torch.arange(T * top))
+
+
 SIZES = [(12, 3, 64, 96), (8, 2, 40, 24), (4, 1, 256, 200), (9, 4, 136, 72), (16, 6, 320, 128), (5, 2, 33, 27), (64, 8, 128, 64),
          (32, 3, 256, 128), (3, 2, 448, 192), (6, 5, 128, 320)]
 
