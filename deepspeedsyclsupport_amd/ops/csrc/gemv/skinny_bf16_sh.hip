@@ -64,11 +64,9 @@ struct Int {
   static constexpr int value = V;
 };
 
-// The address as a wave's base and a lane's bytes. APART: the asm keeps it so, and the base in scalar registers: 10 to 20 vector
-// registers less. (Few token rows have them to spare: a step of one sequence took 0.2 % longer with it.)
-template <bool APART>
+// The address as a wave's base in scalar registers and a lane's bytes; the asm keeps it so: 10 to 20 vector registers less.
 __device__ __forceinline__ const bf16x8_t* at(const bf16* base, uint32_t bytes) {
-  if constexpr (APART) asm("" : "+v"(bytes));
+  asm("" : "+v"(bytes));
   return reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const char*>(base) + bytes);
 }
 
@@ -124,15 +122,28 @@ __global__ void __launch_bounds__(WAVES * 64, (MT <= 2 || RB == 4 ? 4 : 2)) deco
     if (!GATED) return (int)blockIdx.x * RB + i;
     return (int)blockIdx.x * (RB / 2) + i % (RB / 2) + (i < RB / 2 ? 0 : HB);
   };
+  // 33 rows and more: bases per wave and bytes per lane (`at`); up to 32, which have the registers, pointers per lane. (Those as a
+  // base and bytes too: hipcc 7.2 gave a step's addresses registers of the sums in <1, 2, false, true>.)
+  constexpr bool APART = MT == 3;
   const bf16* wp[RB];
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
     const int last = GATED ? (i < RB / 2 ? HB : 2 * HB) - 1 : NB - 1;
-    wp[i] = a.w + (int64_t)min(block_of(i), last) * KQ * 1024;
+    wp[i] = a.w + (int64_t)min(block_of(i), last) * KQ * 1024 + (APART ? 0 : lane * 8);
   }
-  uint32_t xo[MT];  // bytes
+  const bf16* xp[MT];
+  uint32_t xo[MT];
 #pragma unroll
-  for (int m = 0; m < MT; ++m) xo[m] = ((uint32_t)min(16 * m + l16, a.M - 1) * K + 16 * q4) * 2;
+  for (int m = 0; m < MT; ++m) {
+    const int row = min(16 * m + l16, a.M - 1);
+    xo[m] = ((uint32_t)row * K + 16 * q4) * 2;
+    xp[m] = APART ? a.x : a.x + (int64_t)row * K + 16 * q4;
+  }
+  const bf16* np = NORM ? a.norm_w + (APART ? 0 : 16 * q4) : nullptr;
+  auto from = [&](const bf16* p, uint32_t bytes) {
+    if constexpr (APART) return at(p, bytes);
+    else return reinterpret_cast<const bf16x8_t*>(p);
+  };
 
   f32x4 acc[RB][MT];
   float ss[MT];
@@ -155,15 +166,15 @@ __global__ void __launch_bounds__(WAVES * 64, (MT <= 2 || RB == 4 ? 4 : 2)) deco
 #pragma unroll
         for (int i = 0; i < RB; ++i)
           f.w[u][h][i] = __builtin_nontemporal_load(
-              at<MT == 3>(wp[i] + (int64_t)min(s0 + WAVES * u, end - 1) * 1024 + 512 * h, lane * 16));
+              from(wp[i] + (int64_t)min(s0 + WAVES * u, end - 1) * 1024 + 512 * h, lane * 16));
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int k = min(s0 + WAVES * u, end - 1) * 64 + 8 * h;
-        if constexpr (NORM) f.norm[u][h] = *at<MT == 3>(a.norm_w + k, 32 * q4);
+        if constexpr (NORM) f.norm[u][h] = *from(np + k, 32 * q4);
 #pragma unroll
-        for (int m = 0; m < MT; ++m) f.x[u][h][m] = *at<MT == 3>(a.x + k, xo[m]);
+        for (int m = 0; m < MT; ++m) f.x[u][h][m] = *from(xp[m] + k, xo[m]);
       }
     __builtin_amdgcn_sched_barrier(0);
   };
