@@ -8,7 +8,7 @@
 //
 // Tensors are [Z, S, H, D] with arbitrary (z, s, h) strides (Z = B*N for Evoformer, B for BERT); bias1 is indexed
 // [z, key] (per-key mask bias), bias2 is [Z / b2_div, H, S, S] (pair bias shared by b2_div consecutive z).
-//  * forward: one workgroup = 4 waves x 32 query rows of one (z, h); 64-key K/V tiles in LDS (rows padded to 2D + 16 bytes:
+//  * forward (one of its own for width 32, a pair bias and up to 256 keys, see there): one workgroup = 4 waves x 32 query rows of one (z, h); 64-key K/V tiles in LDS (rows padded to 2D + 16 bytes:
 //    conflict-free b128 row reads without a swizzle); S^T = K.Q^T on v_mfma_f32_32x32x16 so each lane owns one query row's scores, biases added in natural units (a mask of the type's lowest
 //    value must not become -inf), online softmax, P reused as the A operand of O += P.V (V by the hardware transposed
 //    read); dropout multiplies P by keep / (1 - p) after the normaliser (Philox-4x32 keyed by (z, h, query, key),
@@ -226,6 +226,17 @@ __device__ __forceinline__ V8 tr_read(const char* img, int rs, int rb, int ch0, 
   return __builtin_bit_cast(V8, v);
 }
 
+// 4 + 4 rows' transposed read at two places
+template <typename V8>
+__device__ __forceinline__ V8 tr_pair(const char* lo_p, const char* hi_p) {
+  const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)lo_p);
+  const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)hi_p);
+  s16x8 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) { v[e] = lo[e]; v[4 + e] = hi[e]; }
+  return __builtin_bit_cast(V8, v);
+}
+
 // ================================================================================================== forward
 template <typename T, int D, bool DROP, bool PAIR>
 __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
@@ -382,6 +393,184 @@ __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
 #pragma unroll
       for (int dt = 0; dt < D / 32; ++dt) Op[(int64_t)qi * a.os_ + dt * 32 + l32] = (T)(o[dt][r] * iv[r]);
     }
+  }
+  if (lane < 32 && qrow < a.S)
+    a.lse[((int64_t)z * a.H + hd) * a.S + qrow] = l_tot > 0.f ? m_run + __logf(l_tot) : INFINITY;
+}
+
+// ---------------------------------------------------------------- forward, 8 to 256 keys, width 32, a pair bias
+// Bound by the vector instructions of a score (eleven and the exponential, four's time). Up to 256 queries of a (z, h) share a
+// workgroup, K and V whole in LDS: one barrier, then a wave's tiles of 32 keys wait for nobody. The rows of K go into the matrix cores
+// in an order that leaves a lane with 16 neighbouring keys of its query (register r of half h: key 16 h + r of the tile), so the pair
+// bias comes from memory as it lies, 2 x 16 bytes a lane and tile, a tile ahead, and not through LDS; the scale of exp2 goes into
+// one fma with the maximum, which moves only when a new one is well above it. 64-byte rows, chunk ch of row r at 16 (ch ^ swz32(r)):
+// K's rows in that order and V's transposed reads touch every bank once. Two workgroups of eight waves share a CU.
+// us, the general kernel and this one: [256, 256, 4, 32] 43.7 and 39, [180, 230, 8, 32] 58 and 48, [128, 200, 4, 32] 25 and 18, [100, 133,
+// 8, 32] 32 and 25, [512, 32, 8, 32] 29 and 13; fewer workgroups than two a CU [140, 256, 4, 32] 26.6 and 26.6, [77, 199, 4, 32] 17.6 and 17.9.
+// (Several z a workgroup, the next one's K and V on their way, 40.5; four waves 43.)
+constexpr int FWD_WHOLE = 256, FWD_WAVES = 8;
+__device__ __forceinline__ int swz32(int r) { return ((r >> 2) & 1) | ((r >> 3) & 2); }
+
+// 16 bytes a lane from memory to LDS byte dst + 16 * lane, past the compiler, which would wait for it before every LDS read
+__device__ __forceinline__ void small_dma(const void* g, uint32_t dst) {
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
+               "s_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "v"(g), "s"(dst)
+               : "memory");
+}
+
+// the larger of the two halves' values of a row (v_permlane32_swap: a shuffle through LDS is a wait of a hundred clocks)
+__device__ __forceinline__ float half_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, x), false, false);
+  return fmaxf(__builtin_bit_cast(float, r[0]), __builtin_bit_cast(float, r[1]));
+}
+
+template <typename T>
+__global__ void __launch_bounds__(64 * FWD_WAVES, 4) small_fwd_whole_kernel(SmallArgs<T> a) {
+  typedef typename MF<T>::V8 V8;
+  typedef __attribute__((address_space(3))) char lds_char;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int nt = (a.Sk + 31) / 32, rows = nt * 32, waves = blockDim.x / 64;
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  float *b1S = reinterpret_cast<float*>(smem + 2 * rows * 64), *scratch = b1S + rows + wid * 32;  // (behind K and V)
+  const int nqb = (a.S + 32 * waves - 1) / (32 * waves);
+  const int qb = blockIdx.x % nqb, hd = blockIdx.x / nqb % a.H, z = blockIdx.x / (nqb * a.H);
+  const int q0w = (qb * waves + wid) * 32, qrow = q0w + l32;
+  const T* bp = a.b2 + ((int64_t)(z / a.b2_div) * a.H + hd) * a.S * a.Sk + (int64_t)min(qrow, a.S - 1) * a.Sk;
+  const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_char*)smem);
+
+  for (int p = wid; p < 4 * nt; p += waves) {  // 16 rows of K or V
+    const bool v = p >= 2 * nt;
+    const int r = (v ? p - 2 * nt : p) * 16 + (lane >> 2), key = min(r, a.Sk - 1);
+    const T* src = v ? a.v + z * a.vz + hd * a.vh + (int64_t)key * a.vs : a.k + z * a.kz + hd * a.kh + (int64_t)key * a.ks;
+    small_dma(src + 8 * ((lane & 3) ^ swz32(r)), lds + p * 1024);
+  }
+  V8 qf[2];
+  {
+    const T* qr = a.q + z * a.qz + hd * a.qh + (int64_t)min(qrow, a.S - 1) * a.qs + 8 * h;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) qf[kk] = *reinterpret_cast<const V8*>(qr + 16 * kk);
+  }
+  V8 bias[2];  // of 16 keys of this lane's query
+  auto load_bias = [&](int k0) {
+    const int key = k0 + 16 * h;
+    if (k0 + 32 <= a.Sk) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g) __builtin_memcpy(&bias[g], bp + key + 8 * g, 16);
+    } else {  // the row's end: its last eight, shifted (what is past it is another row's, or nobody's)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const int at = key + 8 * g, from = min(at, a.Sk - 8);
+        unsigned __int128 v;
+        __builtin_memcpy(&v, bp + from, 16);
+        v = at - from >= 8 ? 0 : v >> 16 * (at - from);
+        bias[g] = __builtin_bit_cast(V8, v);
+      }
+    }
+  };
+  load_bias(0);
+  for (int i = tid; i < rows; i += blockDim.x) b1S[i] = i >= a.Sk ? -INFINITY : a.b1 ? (float)a.b1[z * a.b1_zs + i] : 0.f;
+  int ka[2], va[2];
+  {
+    const int key = 16 * ((l32 >> 2) & 1) + (l32 & 3) + 4 * (l32 >> 3);
+    const int gq = (lane >> 2) & 3, gch = (lane >> 1) & 1, gb = 8 * (lane & 1), colhalf = (lane >> 4) & 1;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = 16 * h + 4 * i + gq;
+      ka[i] = key * 64 + 16 * ((2 * i + h) ^ swz32(key));
+      va[i] = rows * 64 + r * 64 + 16 * ((colhalf * 2 + gch) ^ swz32(r)) + gb;
+    }
+  }
+  const float LOG2E = 1.4426950408889634f;
+  // the largest score of before is kept until a new one is e^5.5 times as large: most tiles leave O as it is
+  constexpr float KEPT = 5.5f;
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  f32x16_t o;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) o[r] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+#pragma unroll 1
+  for (int j = 0; j < nt; ++j) {
+    f32x16_t s;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) s = MF<T>::mma(*reinterpret_cast<const V8*>(smem + j * 2048 + ka[kk]), qf[kk], s);
+    // natural units: scale q.k + bias1[key] + bias2[q, key]
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 b1 = *reinterpret_cast<const f32x4*>(b1S + 32 * j + 16 * h + 4 * g);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 4 * g + i;
+        s[r] = fmaf(s[r], a.scale, b1[i] + (float)bias[r >> 3][r & 7]);
+      }
+    }
+    if (j + 1 < nt) load_bias(32 * (j + 1));
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; r += 2) asm("v_max3_f32 %0, %0, %1, %2" : "+v"(mx) : "v"(s[r]), "v"(s[r + 1]));
+    mx = half_max(mx);
+    const float m_new = mx > m_run + KEPT ? mx : m_run;
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;
+    // rows that the type's lowest value masks throughout: their differences alone can be scaled
+    const bool deep = !(fabsf(m_use) < 1e30f);
+    const float mc = deep ? 0.f : -m_use * LOG2E;
+    if (__any(deep)) {
+      const float by = deep ? m_use : 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] -= by;
+    }
+    f32x4 psum{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], LOG2E, mc));
+      psum[r & 3] += s[r];
+    }
+    if (!__all(m_new == m_run)) {
+      const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * LOG2E);
+      l_run *= alpha;
+      if (j) {
+        if (lane < 32) scratch[lane] = alpha;
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(scratch + 8 * g + 4 * h);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[4 * g + i] *= v[i];
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+    l_run += (psum[0] + psum[1]) + (psum[2] + psum[3]);
+    m_run = m_new;
+#pragma unroll
+    for (int ss = 0; ss < 2; ++ss) {
+      V8 p;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) p[e] = (T)s[8 * ss + e];
+      const char* at = smem + j * 2048 + ss * 512;
+      o = MF<T>::mma(p, tr_pair<V8>(at + va[0], at + va[1]), o);
+    }
+  }
+  const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  if (lane < 32) scratch[lane] = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  int ln = lane;  // (anew: the rows' addresses are not kept over the loop)
+  asm volatile("" : "+v"(ln));
+  const int row = q0w + 4 * (ln >> 5);
+  T* Op = a.out + z * a.oz + hd * a.oh + (int64_t)row * a.os_ + (ln & 31);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(scratch + 8 * g + 4 * (ln >> 5));
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (row + 8 * g + i < a.S) Op[(8 * g + i) * a.os_] = (T)(o[4 * g + i] * v[i]);
   }
   if (lane < 32 && qrow < a.S)
     a.lse[((int64_t)z * a.H + hd) * a.S + qrow] = l_tot > 0.f ? m_run + __logf(l_tot) : INFINITY;
@@ -734,17 +923,6 @@ __global__ void __launch_bounds__(256) small_bias_order_kernel(const T* __restri
 
 __device__ __forceinline__ f32x4 mma16(bf16x8_t a, bf16x8_t b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ f32x4 mma16(f16x8_t a, f16x8_t b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
-
-// 4 + 4 rows' transposed read at two places
-template <typename V8>
-__device__ __forceinline__ V8 tr_pair(const char* lo_p, const char* hi_p) {
-  const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)lo_p);
-  const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)hi_p);
-  s16x8 v;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) { v[e] = lo[e]; v[4 + e] = hi[e]; }
-  return __builtin_bit_cast(V8, v);
-}
 
 template <typename T, bool DB1>
 __global__ void __launch_bounds__(WHOLE_S * 2, 4) small_bwd_whole_kernel(SmallArgs<T> a, const T* b2o) {
@@ -1135,6 +1313,16 @@ int launch_small(SmallArgs<T> a, bool bwd, hipStream_t st) {
   const int nqb = (a.S + BM - 1) / BM;
   const dim3 grid(nqb * a.H * a.Z);
   if (!bwd) {
+    if constexpr (D == 32 && !DROP && PAIR) {
+      if (a.Sk >= 8 && a.Sk <= FWD_WHOLE) {
+        // (below 8 keys a row has no 16 bytes of bias; above 256 K and V would leave a CU one workgroup)
+        const int qt = (a.S + 31) / 32, nqb = (qt + FWD_WAVES - 1) / FWD_WAVES, waves = (qt + nqb - 1) / nqb;
+        const int rows = (a.Sk + 31) / 32 * 32;
+        hipLaunchKernelGGL(small_fwd_whole_kernel<T>, dim3(nqb * a.H * a.Z), dim3(64 * waves), rows * (2 * 64 + 4) + waves * 128, st, a);
+        DS_CHECK_LAUNCH();
+        return 0;
+      }
+    }
     hipLaunchKernelGGL((small_fwd_kernel<T, D, DROP, PAIR>), grid, dim3(NTHR), 0, st, a);
     DS_CHECK_LAUNCH();
     return 0;

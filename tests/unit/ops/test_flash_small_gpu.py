@@ -204,3 +204,29 @@ def test_short_sequences_in_one_pass(Z, S, H, b2_div, dtype, masked):
     for name, a, r in zip(("dq", "dk", "dv", "db1", "db2"), ins, refs):
         if a is not None:
             assert (a.grad.double() - r.grad).abs().max() < tol * r.grad.abs().max() + tol, name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("S,Sk", [(1, 8), (40, 7), (33, 31), (32, 33), (130, 95), (257, 250), (300, 256), (64, 257)])
+def test_forward_with_a_pair_bias_by_keys(S, Sk, dtype):
+    """Keys around tiles of 32, the ends of the kernel that holds all of them (8 and 256) and what is past them; rows of one packed
+    buffer, a pair bias at odd addresses; keys masked by the type's lowest value, for one z all of them (who then count alike).
+    P is rounded to 2^-9 (2^-12): twice that of the largest value, and the result's own rounding. Scores of keys masked by half's
+    lowest value stand 2^-8 apart in single precision, and so may the weights of a z that has no others."""
+    Z, H, D = 6, 2, 32
+    g = torch.Generator(device="cuda").manual_seed(S + Sk)
+    q = torch.randn(Z, S, H, D, device="cuda", generator=g).to(dtype)
+    k, v = torch.randn(Z, Sk, 2, H, D, device="cuda", generator=g).to(dtype).unbind(2)
+    b1 = torch.zeros(Z, Sk, device="cuda", dtype=dtype)
+    b1[torch.rand(Z, Sk, device="cuda", generator=g) < 0.3] = torch.finfo(dtype).min
+    b1[0] = torch.finfo(dtype).min
+    b2 = torch.randn(Z // 3, H, S, Sk, device="cuda", generator=g).to(dtype)
+    odd = torch.empty(b2.numel() + 1, device="cuda", dtype=dtype)[1:].view_as(b2).copy_(b2)
+    with torch.no_grad():
+        out = FS.flash_small(q, k, v, b1, odd, b2_div=3)
+    ref = FS.reference(q, k, v, b1, b2, b2_div=3)
+    step = 2.0**-9 if dtype == torch.bfloat16 else 2.0**-12
+    loose = torch.full((Z, 1, 1, 1), 2 * step, device="cuda")
+    if dtype == torch.float16:
+        loose[0] += 2.0**-7
+    assert ((out.float() - ref).abs() <= step * ref.abs() + loose * v.float().abs().max()).all()
