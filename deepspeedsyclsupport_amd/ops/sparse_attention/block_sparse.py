@@ -168,27 +168,33 @@ class SparseLists:
 
     def __init__(self, bits, blk, L, device):
         self.layout, self.blk, self.L, self.device = torch.from_numpy(bits), blk, L, device
-        self.key, self.lists, self.shares = _lut_key(bits, blk, L, "cpu"), {}, {}
+        self.lists, self.shares = {}, {}
 
     def _to_device(self, parts):
         flat = torch.cat([t.reshape(-1) for t in parts]).to(self.device)   # one copy
         return [t.view(p.shape) for t, p in zip(flat.split([p.numel() for p in parts]), parts)]
 
     def _make(self, side):
-        tiles, counts, lay, _ = build_lut(self.layout, self.blk, self.L, "cpu", self.key)
-        bits = self.layout[:lay.shape[0]].numpy()
-        if side == "fwd":
-            masks = _tile_masks(bits, self.blk, self.L, 8, 4)
-        else:
-            tiles, counts, _, _ = build_bwd_lut(self.layout, self.blk, self.L, lay.shape[0], "cpu", self.key)
-            masks = _tile_masks(bits, self.blk, self.L, 2, 16).transpose(1, 2)   # listed by key block
-        masks = masks.gather(2, tiles.long())
+        """(tiles and masks on the device, the lists' lengths, the masks here): what a list has to do with, ascending, from the masks."""
+        bits = self.layout.numpy()
+        if bits.shape[0] > 1 and (bits == bits[:1]).all():
+            bits = bits[:1]
+        masks = _tile_masks(bits, self.blk, self.L, *((8, 4) if side == "fwd" else (2, 16))).numpy()
+        if side != "fwd":
+            masks = masks.transpose(0, 2, 1)   # listed by key block
+        met = masks != 0
+        ends = met.cumsum(-1, dtype=np.int32)
+        counts = torch.from_numpy(ends[..., -1].copy())
+        lists = np.zeros((2, *met.shape[:2], max(int(counts.max()), 1)), np.int32)
+        head, block, tile = met.nonzero()
+        at = head, block, ends[met] - 1
+        lists[0][at], lists[1][at] = tile, masks[met]
+        tiles, masks = torch.from_numpy(lists)
         return *self._to_device([tiles, masks]), counts, masks
 
     def _split(self, side, parts):
         """What blocks of 64 rows (columns), `parts` to a list, have to do with: (counts [LH, n], [LH, n, entries of the lists])."""
-        _, _, counts, masks = self.lists[side]
-        masks = np.where(np.arange(masks.shape[2]) < counts.numpy()[..., None], masks.numpy().view(np.uint32), 0)
+        masks = self.lists[side][3].numpy().view(np.uint32)
         bits = [0xffff << 16 * p if side == "fwd" else 0x000f000f << 4 * p for p in range(parts)]
         met = (masks[:, :, None] & np.array(bits, np.uint32)[:, None]) != 0
         met = met.reshape(met.shape[0], -1, met.shape[3])[:, :self.L // 64]
