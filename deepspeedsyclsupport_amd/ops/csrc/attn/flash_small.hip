@@ -406,7 +406,8 @@ __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
 // one fma with the maximum, which moves only when a new one is well above it. 64-byte rows, chunk ch of row r at 16 (ch ^ swz32(r)):
 // K's rows in that order and V's transposed reads touch every bank once. Two workgroups of eight waves share a CU.
 // us, the general kernel and this one: [256, 256, 4, 32] 43.7 and 39, [180, 230, 8, 32] 58 and 48, [128, 200, 4, 32] 25 and 18, [100, 133,
-// 8, 32] 32 and 25, [512, 32, 8, 32] 29 and 13; fewer workgroups than two a CU [140, 256, 4, 32] 26.6 and 26.6, [77, 199, 4, 32] 17.6 and 17.9.
+// 8, 32] 32 and 25, [512, 32, 8, 32] 29 and 13; [140, 256, 4, 32] 26.6 and 26.6. Where few CUs
+// get a second large workgroup the general kernel's smaller ones are shared out better ([77, 199, 4, 32], 308 of them, 18 and 20).
 // (Several z a workgroup, the next one's K and V on their way, 40.5; four waves 43.)
 constexpr int FWD_WHOLE = 256, FWD_WAVES = 8;
 __device__ __forceinline__ int swz32(int r) { return ((r >> 2) & 1) | ((r >> 3) & 2); }
@@ -1258,20 +1259,46 @@ __global__ void __launch_bounds__(NTHR, 2) small_bwd_db2_kernel(SmallArgs<T> a) 
     }
 }
 
-// out[i] = sum over s of part[s][i]
+// out[i] = sum over s of part[s][i], in a fixed order: a wave's lanes have four results each, its workgroup's waves a quarter of the parts,
+// eight of them on their way at once (a thread to itself waited for one part after the other: 64 parts of [8, 32, 32] 20 us, now 7; 16 of
+// [4, 256, 256] 5.8 and 4.8)
 __global__ void __launch_bounds__(256) sum_parts_kernel(const float* __restrict__ part, float* __restrict__ out, int64_t n, int parts) {
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-  if (i >= n) return;
-  if (n % 4 == 0) {
-    f32x4 v = *reinterpret_cast<const f32x4*>(part + i);
-    for (int s = 1; s < parts; ++s) v += *reinterpret_cast<const f32x4*>(part + s * n + i);
-    *reinterpret_cast<f32x4*>(out + i) = v;
-  } else {
-    for (int64_t e = i; e < min(i + 4, n); ++e) {
-      float v = part[e];
-      for (int s = 1; s < parts; ++s) v += part[s * n + e];
-      out[e] = v;
+  __shared__ f32x4 sums[4][64];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, lo = parts * wid / 4, hi = parts * (wid + 1) / 4;
+  const int64_t i = ((int64_t)blockIdx.x * 64 + lane) * 4;
+  const bool whole = n % 4 == 0;
+  auto at = [&](int s) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (whole) {
+      if (i < n) v = *reinterpret_cast<const f32x4*>(part + s * n + i);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (i + e < n) v[e] = part[s * n + i + e];
     }
+    return v;
+  };
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+  int s = lo;
+  for (; s + 8 <= hi; s += 8) {
+    f32x4 v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = at(s + u);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) sum += v[u];
+  }
+  for (; s < hi; ++s) sum += at(s);
+  sums[wid][lane] = sum;
+  __syncthreads();
+  if (wid) return;
+#pragma unroll
+  for (int w = 1; w < 4; ++w) sum += sums[w][lane];
+  if (whole) {
+    if (i < n) *reinterpret_cast<f32x4*>(out + i) = sum;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (i + e < n) out[i + e] = sum[e];
   }
 }
 
@@ -1314,11 +1341,12 @@ int launch_small(SmallArgs<T> a, bool bwd, hipStream_t st) {
   const dim3 grid(nqb * a.H * a.Z);
   if (!bwd) {
     if constexpr (D == 32 && !DROP && PAIR) {
-      if (a.Sk >= 8 && a.Sk <= FWD_WHOLE) {
-        // (below 8 keys a row has no 16 bytes of bias; above 256 K and V would leave a CU one workgroup)
-        const int qt = (a.S + 31) / 32, nqb = (qt + FWD_WAVES - 1) / FWD_WAVES, waves = (qt + nqb - 1) / nqb;
+      // (below 8 keys a row has no 16 bytes of bias; above 256 K and V would leave a CU one workgroup)
+      const int qt = (a.S + 31) / 32, blocks = (qt + FWD_WAVES - 1) / FWD_WAVES, waves = (qt + blocks - 1) / blocks;
+      const int64_t groups = (int64_t)blocks * a.H * a.Z;
+      if (a.Sk >= 8 && a.Sk <= FWD_WHOLE && !(waves > 4 && groups > 256 && groups < 320)) {
         const int rows = (a.Sk + 31) / 32 * 32;
-        hipLaunchKernelGGL(small_fwd_whole_kernel<T>, dim3(nqb * a.H * a.Z), dim3(64 * waves), rows * (2 * 64 + 4) + waves * 128, st, a);
+        hipLaunchKernelGGL(small_fwd_whole_kernel<T>, dim3((unsigned)groups), dim3(64 * waves), rows * (2 * 64 + 4) + waves * 128, st, a);
         DS_CHECK_LAUNCH();
         return 0;
       }
@@ -1349,7 +1377,7 @@ int launch_small(SmallArgs<T> a, bool bwd, hipStream_t st) {
     DS_CHECK_LAUNCH();
     if (a.nsplit > 1) {
       const int64_t n = (int64_t)(a.Z / a.b2_div) * a.H * a.S * a.S;
-      hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, st, a.part, a.db2, n, a.nsplit);
+      hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a.part, a.db2, n, a.nsplit);
       DS_CHECK_LAUNCH();
     }
   }
