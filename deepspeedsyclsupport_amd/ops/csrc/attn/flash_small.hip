@@ -898,8 +898,8 @@ __global__ void __launch_bounds__(NTHR, 2) small_bwd_dkv_kernel(SmallArgs<T> a) 
 // the vector instructions around them are what bounds both passes. dS of a tile of 32 queries crosses LDS for dQ, 16 x 16
 // pieces of which go to four waves in turn, while the others begin the next tile. The pair bias comes in the order of the
 // accumulators (small_bias_order_kernel), 2 x 16 bytes a lane and tile from L2. Two workgroups of eight waves share a CU.
-// [256, 256, 4, 32], us: 50 + 51 in two passes, 72 here, 20 of it the loads of two rounds of workgroups that all begin at once, the
-// others 6000 clocks a tile (four waves a SIMD, 1000 each of vector instructions).
+// [256, 256, 4, 32], us: 50 + 51 in two passes, 67 here, 20 of it the loads of two rounds of workgroups that all begin at once;
+// four waves a SIMD, 900 clocks a tile each of vector instructions.
 constexpr int WHOLE_S = 256, WHOLE_LDS = 3 * WHOLE_S * 64 + WHOLE_S * 64 + 2 * WHOLE_S * 4;
 
 // bias2 [groups, S, S] -> [groups, query tiles, key tiles, 2, 64, 8]: element j of half g and lane l is query crow(8 g + j, l / 32), key
@@ -925,11 +925,11 @@ __global__ void __launch_bounds__(256) small_bias_order_kernel(const T* __restri
 __device__ __forceinline__ f32x4 mma16(bf16x8_t a, bf16x8_t b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ f32x4 mma16(f16x8_t a, f16x8_t b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 
-template <typename T, bool DB1>
-__global__ void __launch_bounds__(WHOLE_S * 2, 4) small_bwd_whole_kernel(SmallArgs<T> a, const T* b2o) {
+template <typename T, bool DB1, int NT>
+__global__ void __launch_bounds__(NT ? NT * 64 : WHOLE_S * 2, 4) small_bwd_whole_kernel(SmallArgs<T> a, const T* b2o) {
   typedef typename MF<T>::V8 V8;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int nt = blockDim.x / 64, rows = 32 * nt;   // tiles of 32, one a wave
+  const int nt = NT ? NT : blockDim.x / 64, rows = 32 * nt;   // tiles of 32, one a wave
   char *Qi = smem, *Gi = Qi + rows * 64, *Ki = Gi + rows * 64, *DS = Ki + rows * 64;   // DS: [key][32 queries]
   float *lseS = reinterpret_cast<float*>(DS + rows * 64), *delS = lseS + rows;
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
@@ -945,7 +945,7 @@ __global__ void __launch_bounds__(WHOLE_S * 2, 4) small_bwd_whole_kernel(SmallAr
   u32x4_t st[3][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int c = tid + i * blockDim.x, r = min(c >> 2, S - 1), ch = c & 3;
+    const int c = tid + i * 64 * nt, r = min(c >> 2, S - 1), ch = c & 3;
     st[0][i] = *reinterpret_cast<const u32x4_t*>(Qp + (int64_t)r * a.qs + ch * 8);
     st[1][i] = *reinterpret_cast<const u32x4_t*>(Gp + (int64_t)r * a.gs + ch * 8);
     st[2][i] = *reinterpret_cast<const u32x4_t*>(Kp + (int64_t)r * a.ks + ch * 8);
@@ -975,7 +975,7 @@ __global__ void __launch_bounds__(WHOLE_S * 2, 4) small_bwd_whole_kernel(SmallAr
   V8 bias[2] = {*reinterpret_cast<const V8*>(bp + lane * 8), *reinterpret_cast<const V8*>(bp + 512 + lane * 8)};
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int c = tid + i * blockDim.x, r = c >> 2, at = r * 64 + 16 * ((c & 3) ^ ((r >> 2) & 3));
+    const int c = tid + i * 64 * nt, r = c >> 2, at = r * 64 + 16 * ((c & 3) ^ ((r >> 2) & 3));
     *reinterpret_cast<u32x4_t*>(Qi + at) = st[0][i];
     *reinterpret_cast<u32x4_t*>(Gi + at) = st[1][i];
     *reinterpret_cast<u32x4_t*>(Ki + at) = st[2][i];
@@ -1318,19 +1318,24 @@ int64_t small_order_elements(int Z, int H, int S, int D, int b2_div, bool drop) 
   return D == 32 && S <= WHOLE_S && !drop && b2_div > 1 && (int64_t)Z * H >= 256 ? (int64_t)(Z / b2_div) * H * nt * nt * 1024 : 0;
 }
 
-template <typename T, bool DB1>
+// Kernels of their own for one tile and for five to eight: in the one for any number, addresses and the turns at dQ are a quarter of a
+// tile's instructions ([256, 256, 4, 32] 81 us for 67, [200, 251, 8, 32] 135 and 107, [100, 133, 8, 32] 51 and 43, [512, 32, 8, 32] 23 and 20). (Two to four have the registers for it no more: 30 to 100 of them in scratch memory.)
+template <typename T, bool DB1, int NT>
 int launch_whole(const SmallArgs<T>& a, hipStream_t st) {
+  const int nt = (a.S + 31) / 32;
+  if constexpr (NT != 0) {
+    if (nt != NT) return launch_whole<T, DB1, NT == 1 ? 0 : NT == 5 ? 1 : NT - 1>(a, st);
+  }
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&small_bwd_whole_kernel<T, DB1>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              WHOLE_LDS);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&small_bwd_whole_kernel<T, DB1, NT>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, WHOLE_LDS);
     attr = true;
   }
-  const int nt = (a.S + 31) / 32;
   const int64_t tiles = (int64_t)(a.Z / a.b2_div) * a.H * nt * nt;
   hipLaunchKernelGGL(small_bias_order_kernel<T>, dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, st, a.b2, a.order, a.S, nt, tiles);
   DS_CHECK_LAUNCH();
-  hipLaunchKernelGGL((small_bwd_whole_kernel<T, DB1>), dim3(a.H * a.Z), dim3(64 * nt), WHOLE_LDS / 8 * nt, st, a, (const T*)a.order);
+  hipLaunchKernelGGL((small_bwd_whole_kernel<T, DB1, NT>), dim3(a.H * a.Z), dim3(64 * nt), WHOLE_LDS / 8 * nt, st, a, (const T*)a.order);
   DS_CHECK_LAUNCH();
   return 0;
 }
@@ -1360,7 +1365,7 @@ int launch_small(SmallArgs<T> a, bool bwd, hipStream_t st) {
     if (small_order_elements(a.Z, a.H, a.S, D, a.b2_div, false) > 0) {
       whole = true;
       if (a.order == nullptr) return (int)hipErrorInvalidValue;
-      if (int rc = a.db1 ? launch_whole<T, true>(a, st) : launch_whole<T, false>(a, st)) return rc;
+      if (int rc = a.db1 ? launch_whole<T, true, WHOLE_S / 32>(a, st) : launch_whole<T, false, WHOLE_S / 32>(a, st)) return rc;
     }
   }
   if (!whole) {
