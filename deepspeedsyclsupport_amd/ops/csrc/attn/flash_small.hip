@@ -424,8 +424,8 @@ __device__ __forceinline__ void small_dma(const void* g, uint32_t dst) {
 
 // the larger of the two halves' values of a row (v_permlane32_swap: a shuffle through LDS is a wait of a hundred clocks)
 __device__ __forceinline__ float half_max(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, x), false, false);
-  return fmaxf(__builtin_bit_cast(float, r[0]), __builtin_bit_cast(float, r[1]));
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
 template <typename T>

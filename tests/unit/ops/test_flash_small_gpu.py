@@ -245,3 +245,17 @@ def test_one_pass_by_number_of_tiles(S):
     ref.backward(go.bfloat16().double())
     for name, a, r in zip(("dq", "dk", "dv", "db1", "db2"), ins, refs):
         assert (a.grad.double() - r.grad).abs().max() < 4e-2 * r.grad.abs().max() + 4e-2, name
+
+
+@pytest.mark.parametrize("run", [4, 8, 16, 32, 64])
+@pytest.mark.parametrize("odd", [0, 1])
+def test_masked_runs_of_keys(run, odd):
+    """Every other run of keys masked, the others with scores far above: the maximum of a row is that of all its keys, whichever lanes
+    and tiles hold them (of the masked ones alone, the others' exponentials would be infinite). Tolerance as in the tests above."""
+    Z, S, H = 8, 200, 2
+    q, k, v, _, bias2 = _case(Z, S, H, 32, torch.bfloat16, False, True, Z, seed=run)
+    keys = torch.arange(S, device="cuda") // run % 2
+    bias1 = torch.where(keys == odd, -1e9, 100.0).expand(Z, S).bfloat16().contiguous()
+    with torch.no_grad():
+        out = FS.flash_small(q, k, v, bias1, bias2, b2_div=Z)
+    assert _rel(out, FS.reference(q, k, v, bias1, bias2, b2_div=Z)) < 2e-2
