@@ -15,6 +15,12 @@
 //    row reads of K (`ds_read_b128`) and the transposed reads of V;
 //  * global->LDS staging is split (issue the next tile's loads before the current tile's MFMAs, write LDS after them),
 //    so HBM latency hides under the MFMA work; one barrier per tile;
+//    What bounds it: a tile's 32 products of a wave take a SIMD 1024 clocks, and the 32 KB that it reads of K and V for its
+//    32 rows take LDS as long, with eight waves of a CU; the exponentials 512 more where nothing else runs, at 1.7 GHz under
+//    this load. (Tried: reads further ahead; the products of the next keys and of the last ones between a tile's
+//    exponentials: the same time; 64 rows per wave, half the reads: one wave per SIMD, 28 spilled registers, 988 us.)
+//    B1 Hq32 Hkv8 S8192 causal 599 -> 589 us, B2 Hq32 S4096 341 -> 335, with the row maximum in short chains and no
+//    arithmetic for a rescale where no maximum moves;
 //  * causal: fully-masked tiles are skipped per wave, heavy query blocks are launched first, and the block->tile map
 //    keeps every (batch, head) on one XCD so its K/V stay in that XCD's L2.
 //  * block-sparse variant (SPARSE=true, reference `ops/sparse_attention` SDD/softmax/DSD Triton kernels): each
@@ -372,18 +378,21 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
           }
       }
       // ---------------- online softmax (row = this lane's query; partner lane^32 holds the other 32 keys)
-      // row max: one v_max3 per register pair (fmaxf on MFMA outputs makes hipcc canonicalise every input first)
-      float mx = -INFINITY;
+      // row max: one v_max3 per register pair (fmaxf on MFMA outputs makes hipcc canonicalise every input first), in four
+      // chains of four and not one of sixteen, whose latency nothing covers; the partner's half by a swap of the wave's
+      // halves in registers. (The swap's results are taken by value: a __builtin_bit_cast of the second reads the first.)
+      float m4[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mx = max3f(mx, s[0][r], s[1][r]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      for (int r = 0; r < 16; ++r) m4[r & 3] = max3f(m4[r & 3], s[0][r], s[1][r]);
+      float mx = max3f(max3f(m4[0], m4[1], m4[2]), m4[3], m4[3]);
+      const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = max3f(__uint_as_float(halves[0]), __uint_as_float(halves[1]), mx);
       // deferred rescale: the running reference maximum only moves when the new maximum exceeds it by more than
       // RESCALE_LOG2 in the exponent's units, so most tiles skip the rescale of O entirely; until then the
       // probabilities are at most 2^RESCALE_LOG2 (exact in fp32, in range for bf16), and l / LSE use the same
-      // reference, so the result is unchanged.
+      // reference, so the result is unchanged. Where no row of the wave moves, nothing is computed for it.
       const float m_new = mx > m_run + rescale_thr ? mx : m_run;
       const float m_use = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = fast_exp2((m_run - m_use) * c);
       const float mc = m_use * c;
       float psum = 0.f;
 #pragma unroll
@@ -394,10 +403,11 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
           s[t][r] = p;
           psum += p;
         }
-      l_run = l_run * alpha + psum;
-      m_run = m_new;
       // ---------------- rescale O rows (alpha lives on the lane of its row; O rows live in registers)
-      if (!__all(alpha == 1.f)) {
+      if (!__all(m_new == m_run)) {
+        const float alpha = fast_exp2((m_run - m_use) * c);
+        l_run *= alpha;
+        m_run = m_new;
         if (lane < 32) scratch[lane] = alpha;
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -414,6 +424,7 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
           for (int r = 0; r < 16; ++r) o[dt][r] *= a4[r];
         __builtin_amdgcn_wave_barrier();
       }
+      l_run += psum;
       // ---------------- O += P . V  (P straight from the score registers; V via transposed LDS reads)
       // two probabilities per v_cvt_pk_bf16_f32 (hipcc lowers an element-wise fptrunc to one convert plus a
       // v_perm per element, and the VALU issue slots are what this loop runs out of)

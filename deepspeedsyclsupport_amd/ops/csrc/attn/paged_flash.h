@@ -247,17 +247,17 @@ __global__ void __launch_bounds__(NTHR, 2) paged_flash_kernel(PagedArgs a, int p
           }
       }
       // ---------------- online softmax; the reference maximum moves only past 2^8 (flash_fwd.hip)
-      float alpha = 1.f, mc = a.cap_out;
+      float m_new = m_run, m_use = 0.f, mc = a.cap_out;
       if (!fixed) {
-        float mx = -INFINITY;
+        float m4[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmax3(mx, s[0][r], s[1][r]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = mx > m_run + rescale_thr ? mx : m_run;
-        const float m_use = m_new == -INFINITY ? 0.f : m_new;
-        alpha = __builtin_amdgcn_exp2f((m_run - m_use) * a.c);
+        for (int r = 0; r < 16; ++r) m4[r & 3] = fmax3(m4[r & 3], s[0][r], s[1][r]);
+        float mx = fmax3(fmax3(m4[0], m4[1], m4[2]), m4[3], m4[3]);
+        const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+        mx = fmax3(__uint_as_float(halves[0]), __uint_as_float(halves[1]), mx);
+        m_new = mx > m_run + rescale_thr ? mx : m_run;
+        m_use = m_new == -INFINITY ? 0.f : m_new;
         mc = m_use * a.c;
-        m_run = m_new;
       }
       float psum = 0.f;
 #pragma unroll
@@ -268,8 +268,10 @@ __global__ void __launch_bounds__(NTHR, 2) paged_flash_kernel(PagedArgs a, int p
           s[t][r] = p;
           psum += p;
         }
-      l_run = l_run * alpha + psum;
-      if (!fixed && !__all(alpha == 1.f)) {
+      if (!fixed && !__all(m_new == m_run)) {
+        const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * a.c);
+        l_run *= alpha;
+        m_run = m_new;
         if (lane < 32) scratch[lane] = alpha;
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -286,6 +288,7 @@ __global__ void __launch_bounds__(NTHR, 2) paged_flash_kernel(PagedArgs a, int p
           for (int r = 0; r < 16; ++r) o[dt][r] *= a4[r];
         __builtin_amdgcn_wave_barrier();
       }
+      l_run += psum;
       // ---------------- O += P . V, 16 keys at a time; EXT: weights as two bf16 terms, the second what the first leaves out
       bf16x8_t ph, pl;
 #pragma unroll

@@ -52,6 +52,22 @@ def _case(lens, starts, Hq, Hk, BS, alibi, window, seed=0, D=128):
                                    msg=lambda m: f"seq {i} (start {starts[i]}, n {lens[i]}): {m}")
 
 
+@pytest.mark.parametrize("n", [128, 40])
+def test_paged_prefill_peak_at_every_key(n):
+    """Each of 128 cached keys in turn is one row's only large score: a maximum that misses any overflows its weights."""
+    from deepspeedsyclsupport_amd.inference.model_implementations.transformer import RaggedMeta
+    from deepspeedsyclsupport_amd.ops.native import hip_ops
+    g = torch.Generator().manual_seed(n)
+    perm = torch.randperm(128, generator=g)[:n].cuda()
+    kc = torch.zeros(4, 1, 64, 128, device="cuda", dtype=torch.bfloat16)
+    kc[:2] = torch.eye(128, device="cuda").bfloat16().view(2, 1, 64, 128)
+    vc = torch.randn(4, 1, 64, 128, generator=g).cuda().bfloat16()
+    q = 300 * torch.eye(128, device="cuda").bfloat16()[perm][:, None]
+    meta = RaggedMeta.build([128], [n], [[0, 1, 2, 3]], 0, 64, torch.device("cuda"))
+    out = hip_ops().paged_prefill(q, kc, vc, meta.block_tables, meta.start_pos, meta.cu_q, meta.work, None, 0, 1.0)
+    assert torch.equal(out[:, 0], vc[:2].reshape(128, 128)[perm])  # one weight is 1, the others e^-300 = 0 in fp32
+
+
 @pytest.mark.parametrize("Hq,Hk", [(8, 8), (8, 2)])
 @pytest.mark.parametrize("BS", [16, 64])
 def test_paged_prefill_mixed_chunks(Hq, Hk, BS):

@@ -38,6 +38,20 @@ def test_flash_fwd(causal, B, Hq, Hk, S):
     assert o.transpose(1, 2).is_contiguous()  # memory is [B,S,H,D]
 
 
+@pytest.mark.parametrize("S", [128, 96, 33])
+def test_flash_fwd_peak_at_every_key(S):
+    """Each key in turn is one row's only large score: a maximum that misses any of them overflows that row's weights."""
+    from deepspeedsyclsupport_amd.ops.native import hip_ops
+    g = torch.Generator().manual_seed(S)
+    perm = torch.randperm(S, generator=g).cuda()
+    k = torch.eye(S, 128, device="cuda").bfloat16()[None, None]
+    v = torch.randn(1, 1, S, 128, generator=g).cuda().bfloat16()
+    q = 300 * k[:, :, perm]
+    o, lse = hip_ops().flash_fwd(q, k, v, False, 1.0, True)
+    assert torch.equal(o, v[:, :, perm])  # one weight is 1, the others e^-300 = 0 in fp32
+    torch.testing.assert_close(lse, torch.full_like(lse, 300), rtol=2**-22, atol=0)  # two roundings of the base change
+
+
 def test_flash_fwd_strided_inputs():
     """q/k/v as views of a packed [B,S,H,D] buffer (non-contiguous head-major views)."""
     from deepspeedsyclsupport_amd.ops.native import hip_ops
