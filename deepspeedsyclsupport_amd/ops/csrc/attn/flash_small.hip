@@ -399,11 +399,11 @@ __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
 }
 
 // ---------------------------------------------------------------- forward, 8 to 256 keys, width 32, a pair bias
-// Bound by the vector instructions of a score (eleven and the exponential, four's time). Up to 256 queries of a (z, h) share a
+// Bound by the vector instructions of a score (twelve and the exponential, four's time). Up to 256 queries of a (z, h) share a
 // workgroup, K and V whole in LDS: one barrier, then a wave's tiles of 32 keys wait for nobody. The rows of K go into the matrix cores
 // in an order that leaves a lane with 16 neighbouring keys of its query (register r of half h: key 16 h + r of the tile), so the pair
-// bias comes from memory as it lies, 2 x 16 bytes a lane and tile, a tile ahead, and not through LDS; the scale of exp2 goes into
-// one fma with the maximum, which moves only when a new one is well above it. 64-byte rows, chunk ch of row r at 16 (ch ^ swz32(r)):
+// bias comes from memory as it lies, 2 x 16 bytes a lane and tile, a tile ahead, and not through LDS; the maximum
+// moves only when a new one is well above it. 64-byte rows, chunk ch of row r at 16 (ch ^ swz32(r)):
 // K's rows in that order and V's transposed reads touch every bank once. Two workgroups of eight waves share a CU.
 // us, the general kernel and this one: [256, 256, 4, 32] 43.7 and 39, [180, 230, 8, 32] 58 and 48, [128, 200, 4, 32] 25 and 18, [100, 133,
 // 8, 32] 32 and 25, [512, 32, 8, 32] 29 and 13; [140, 256, 4, 32] 26.6 and 26.6. Where few CUs
@@ -517,18 +517,11 @@ __global__ void __launch_bounds__(64 * FWD_WAVES, 4) small_fwd_whole_kernel(Smal
     mx = half_max(mx);
     const float m_new = mx > m_run + KEPT ? mx : m_run;
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    // rows that the type's lowest value masks throughout: their differences alone can be scaled
-    const bool deep = !(fabsf(m_use) < 1e30f);
-    const float mc = deep ? 0.f : -m_use * LOG2E;
-    if (__any(deep)) {
-      const float by = deep ? m_use : 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] -= by;
-    }
     f32x4 psum{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], LOG2E, mc));
+      // (the difference first: in an fma with a maximum that is scaled, and rounded, before, a mask of -1e10 is an exponent of 328)
+      s[r] = __builtin_amdgcn_exp2f((s[r] - m_use) * LOG2E);
       psum[r & 3] += s[r];
     }
     if (!__all(m_new == m_run)) {

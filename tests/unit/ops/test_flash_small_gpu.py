@@ -259,3 +259,36 @@ def test_masked_runs_of_keys(run, odd):
     with torch.no_grad():
         out = FS.flash_small(q, k, v, bias1, bias2, b2_div=Z)
     assert _rel(out, FS.reference(q, k, v, bias1, bias2, b2_div=Z)) < 2e-2
+
+
+_MASKS = [-1e4, -1e5, -1e6, -1e7, -1e9, -5e9, -1e10, -1e15, -1e20, torch.finfo(torch.bfloat16).min]
+
+
+def _masked_case(mask):
+    """Whole rows masked by `mask`, rows whose first 32 (64) keys are, a third of the keys at random. Queries and keys are small whole
+    numbers and their products exact, so that the scores can be told to the last bit: fma(q k, scale, bias1 + bias2) in single precision."""
+    Z, S, H, D = 128, 100, 2, 32
+    g = torch.Generator(device="cuda").manual_seed(17)
+    q, k = (torch.randint(-2, 3, (Z, S, H, D), device="cuda", generator=g).bfloat16() for _ in range(2))
+    v, do = (torch.randn(Z, S, H, D, device="cuda", generator=g).bfloat16() for _ in range(2))
+    b2 = torch.randn(2, H, S, S, device="cuda", generator=g)
+    b2[1, 1] *= 40   # (beside 1e9, single precision has steps of 64)
+    gone = torch.rand(Z, S, device="cuda", generator=g) < 0.3
+    gone[0::4], gone[1::4, :32], gone[3::4, :64] = True, True, True
+    b1 = torch.zeros(Z, S, device="cuda").masked_fill_(gone, mask)
+    b1, b2 = b1.bfloat16(), b2.bfloat16()
+    bias = (b1.float()[:, None, None] + b2.float().repeat_interleave(Z // 2, 0)).double()
+    s = (q.double().transpose(1, 2) @ k.double().permute(0, 2, 3, 1) * torch.tensor(D**-0.5).double() + bias).float().double()
+    return q, k, v, do, b1, b2, s
+
+
+@pytest.mark.parametrize("mask", _MASKS)
+def test_finite_masks_forward(mask):
+    """P is rounded to 2^-9, as is the result; LSE is a maximum plus a logarithm in single precision."""
+    from deepspeedsyclsupport_amd.ops.native import hip_ops
+    q, k, v, _, b1, b2, s = _masked_case(mask)
+    o, lse = hip_ops().flash_small_fwd(q, k, v, b1, b2, 64, 32**-0.5, 0.0, 0)
+    want = (torch.softmax(s, -1) @ v.double().transpose(1, 2)).transpose(1, 2)
+    assert ((o.double() - want).abs() <= 2.0**-9 * want.abs() + 2.0**-8 * v.double().abs().max()).all()
+    want = torch.logsumexp(s, -1)
+    assert ((lse.double() - want).abs() <= 2.0**-22 * want.abs() + 1e-5).all()
