@@ -402,13 +402,14 @@ __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
 // Bound by the vector instructions of a score (twelve and the exponential, four's time). Up to 256 queries of a (z, h) share a
 // workgroup, K and V whole in LDS: one barrier, then a wave's tiles of 32 keys wait for nobody. The rows of K go into the matrix cores
 // in an order that leaves a lane with 16 neighbouring keys of its query (register r of half h: key 16 h + r of the tile), so the pair
-// bias comes from memory as it lies, 2 x 16 bytes a lane and tile, a tile ahead, and not through LDS; the maximum
-// moves only when a new one is well above it. 64-byte rows, chunk ch of row r at 16 (ch ^ swz32(r)):
+// bias comes from memory as it lies, 2 x 16 bytes a lane and tile, a tile ahead, and not through LDS. The largest
+// weight is 1, which no type rounds: a maximum kept until a new one is well above it saves the rescaling of O, and costs a tenth of
+// the result's accuracy (0.0023 for 0.0020 off 64 bits). 64-byte rows, chunk ch of row r at 16 (ch ^ swz32(r)):
 // K's rows in that order and V's transposed reads touch every bank once. Two workgroups of eight waves share a CU.
-// us, the general kernel and this one: [256, 256, 4, 32] 43.7 and 39, [180, 230, 8, 32] 58 and 48, [128, 200, 4, 32] 25 and 18, [100, 133,
-// 8, 32] 32 and 25, [512, 32, 8, 32] 29 and 13; [140, 256, 4, 32] 26.6 and 26.6. Where few CUs
-// get a second large workgroup the general kernel's smaller ones are shared out better ([77, 199, 4, 32], 308 of them, 18 and 20).
-// (Several z a workgroup, the next one's K and V on their way, 40.5; four waves 43.)
+// us, the general kernel and this one: [256, 256, 4, 32] 43.5 and 40.3, [180, 230, 8, 32] 57 and 51, [128, 200, 4, 32] 23.5 and 19.2,
+// [100, 133, 8, 32] 29.6 and 24.9, [512, 32, 8, 32] 28.7 and 12.6; [140, 256, 4, 32] 26.4 and 28.1. Where few CUs
+// get a second large workgroup the general kernel's smaller ones are shared out better ([77, 199, 4, 32], 308 of them, 17.1 and 18.4).
+// (Tried beside 39 with another rule for the maximum: several z a workgroup, the next one's K and V on their way, 40.5; four waves 43.)
 constexpr int FWD_WHOLE = 256, FWD_WAVES = 8;
 __device__ __forceinline__ int swz32(int r) { return ((r >> 2) & 1) | ((r >> 3) & 2); }
 
@@ -486,8 +487,6 @@ __global__ void __launch_bounds__(64 * FWD_WAVES, 4) small_fwd_whole_kernel(Smal
     }
   }
   const float LOG2E = 1.4426950408889634f;
-  // the largest score of before is kept until a new one is e^5.5 times as large: most tiles leave O as it is
-  constexpr float KEPT = 5.5f;
   asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   f32x16_t o;
 #pragma unroll
@@ -515,7 +514,7 @@ __global__ void __launch_bounds__(64 * FWD_WAVES, 4) small_fwd_whole_kernel(Smal
 #pragma unroll
     for (int r = 0; r < 16; r += 2) asm("v_max3_f32 %0, %0, %1, %2" : "+v"(mx) : "v"(s[r]), "v"(s[r + 1]));
     mx = half_max(mx);
-    const float m_new = mx > m_run + KEPT ? mx : m_run;
+    const float m_new = fmaxf(m_run, mx);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     f32x4 psum{0.f, 0.f, 0.f, 0.f};
 #pragma unroll

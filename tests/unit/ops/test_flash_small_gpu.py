@@ -292,3 +292,23 @@ def test_finite_masks_forward(mask):
     assert ((o.double() - want).abs() <= 2.0**-9 * want.abs() + 2.0**-8 * v.double().abs().max()).all()
     want = torch.logsumexp(s, -1)
     assert ((lse.double() - want).abs() <= 2.0**-22 * want.abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("dtype,unit", [(torch.bfloat16, 2.0**-8), (torch.float16, 2.0**-11)], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("S,top", [(64, 40), (250, 100), (256, 255)])
+def test_largest_weight_is_exact(dtype, unit, S, top):
+    """One key stands up to e^5 above the tiles before it, and it alone has a value: its weight is 1 whatever stood before, so that
+    the result is rounded once (2 percent beside that for the exponentials and sums in single precision)."""
+    from deepspeedsyclsupport_amd.ops.native import hip_ops
+    Z, H, D = 2, 8, 32
+    q = torch.zeros(Z, S, H, D, device="cuda", dtype=dtype)
+    v = torch.zeros_like(q)
+    v[:, top] = 1
+    above = torch.linspace(0.5, 5.4, H * S, device="cuda").view(1, H, S).to(dtype)
+    b2 = torch.zeros(1, H, S, S, device="cuda", dtype=dtype)
+    b2[..., top] = above
+    o, lse = hip_ops().flash_small_fwd(q, q, v, None, b2, Z, D**-0.5, 0.0, 0)
+    e = above.double().exp().transpose(1, 2)[..., None]
+    want = e / (e + S - 1)
+    assert ((o.double() - want).abs() <= 1.02 * unit * want).all()
+    assert (lse.double() - (e[..., 0] + S - 1).log().transpose(1, 2)).abs().max() < 1e-5
