@@ -38,6 +38,7 @@ constexpr int STAGE = 2 * PIECE;
 constexpr int LIST = 512;             // steps listed at a time
 constexpr float LOG2E = 1.4426950408889634f;
 
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
@@ -84,10 +85,10 @@ __device__ __forceinline__ void settle() { asm volatile("s_waitcnt vmcnt(0)\n\ts
 // LDS work is done; then the barrier. Unlike __syncthreads it waits for no load.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-__device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {  // round to nearest even, lo in bits 0..15
-  unsigned r;
-  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(lo), "v"(hi));
-  return r;
+// Round to nearest even, lo in bits 0..15: one v_cvt_pk_bf16_f32. Not in asm: a swap of the wave's halves stands two wait states
+// behind what writes its operands, and hipcc sees to that where it sees the writer.
+__device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2_t{lo, hi}, bf16x2));
 }
 __device__ __forceinline__ bf16x8 pack8(const f32x16& x, int at) {
   u32x4_t u;
