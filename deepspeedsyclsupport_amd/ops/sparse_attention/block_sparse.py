@@ -167,6 +167,8 @@ class SparseLists:
     side (batch and heads); each side is made when it is first needed."""
 
     def __init__(self, bits, blk, L, device):
+        # blocks that make up tiles of 64 evenly, and as many of them as the sequence has, both ways
+        assert min(bits.shape[1:]) * blk >= L and L % 128 == 0 and L % blk == 0 and (64 % blk == 0 or blk % 64 == 0)
         self.layout, self.blk, self.L, self.device = torch.from_numpy(bits), blk, L, device
         self.lists, self.shares = {}, {}
 

@@ -135,6 +135,26 @@ def test_batch_sizes_share_the_lists(kind, monkeypatch):
     bs._PLANS.clear()
 
 
+@pytest.mark.parametrize("shape,blk,L", [((1, 16, 16), 64, 2048), ((1, 32, 16), 64, 2048), ((1, 16, 32), 64, 2048), ((2, 32, 31), 64, 2048),
+                                         ((1, 8, 8), 48, 384), ((1, 4, 4), 96, 384), ((1, 3, 3), 64, 192), ((1, 5, 5), 32, 144)])
+def test_layouts_that_do_not_fit_are_refused(shape, blk, L):
+    """Fewer blocks than the sequence has, blocks that do not make up tiles, sequences of no whole tiles: refused, every time."""
+    bs._PLANS.clear()
+    for _ in range(2):
+        with pytest.raises(AssertionError):
+            bs.sparse_plan(torch.ones(shape, dtype=torch.long), blk, L, 1, shape[0], "cpu").forward()
+    assert not bs._PLANS
+
+
+def test_a_layout_for_longer_sequences_is_cut():
+    H, blk, L = 2, 32, 640
+    lay = _layout("heads", H, blk, 2 * L)
+    whole, cut = (bs.sparse_plan(x, blk, L, 1, H, "cpu") for x in (lay, lay[:, :L // blk, :L // blk].contiguous()))
+    for a, b in ((whole.forward(), cut.forward()), (whole.rows(), cut.rows()), (whole.columns(), cut.columns())):
+        assert all(torch.equal(x, y) for x, y in zip(a[:4], b[:4])) and a.nslots == b.nslots
+    bs._PLANS.clear()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("D,blk,L,kind,bias", [(128, 64, 1152, "shared", False), (64, 32, 1024, "heads", True),
                                                (128, 16, 512, "empty", False), (128, 128, 1408, "shared", True)])
