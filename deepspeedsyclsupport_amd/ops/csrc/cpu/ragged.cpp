@@ -5,12 +5,19 @@
 
 #include <algorithm>
 #include <optional>
+#include <stdexcept>
+#include <string>
 #include <vector>
 
 namespace {
 
 using Ints = std::vector<int64_t>;
 using torch::Tensor;
+
+int64_t narrow(int64_t v) {
+  if ((int32_t)v != v) throw std::overflow_error("ragged_tables: " + std::to_string(v) + " does not fit 32 bits");
+  return v;
+}
 
 // See RaggedMeta (inference/model_implementations/transformer.py) for the tables. One array of 32-bit integers behind the 64-bit
 // ones (logit rows, then the tokens), one copy, from pinned memory, so that no step waits for the steps before it.
@@ -25,14 +32,16 @@ pybind11::tuple ragged_tables(const Ints& starts, const Ints& n_new, const std::
   size_t width = 1;
   for (size_t i = 0; i < S; ++i) {
     TORCH_CHECK(n_new[i] >= 0, "ragged_tables: token counts");
-    cu[i + 1] = cu[i] + n_new[i];
+    cu[i + 1] = cu[i] + narrow(n_new[i]);
+    narrow(cu[i + 1]);
+    narrow(narrow(starts[i]) + n_new[i]);
     width = std::max(width, blocks[i].size());
   }
   const int64_t T = cu[S];
   std::vector<int32_t> flat;
   flat.reserve(2 * T + S * (width + 8) + T / 32 + 64);
   std::vector<int64_t> ends;
-  auto put = [&](int64_t v) { flat.push_back((int32_t)v); };
+  auto put = [&](int64_t v) { flat.push_back((int32_t)narrow(v)); };
   auto part = [&] { ends.push_back((int64_t)flat.size()); };
   for (size_t i = 0; i < S; ++i)
     for (int64_t j = 0; j < n_new[i]; ++j) put(starts[i] + j);

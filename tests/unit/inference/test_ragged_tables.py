@@ -40,6 +40,17 @@ def test_tables_hold_the_batch(seed):
     assert m.kv_offs.tolist() == [sum(ctx[:i]) for i in range(len(ctx) + 1)] and m.kv_total == sum(ctx)
 
 
+@pytest.mark.parametrize("what", ["starts", "tokens", "sum", "block", "slot", "row"])
+def test_what_32_bits_do_not_hold_is_refused(what):
+    big = 1 << 31
+    a = dict(starts=[4, 0], n_new=[1, 2], block_lists=[[1], [2]], n_decode=1, block_size=16, device=None, slots=[0, 1], logit_rows=[0, 2])
+    RaggedMeta.build(**a)
+    a.update({"starts": dict(starts=[big, 0]), "tokens": dict(n_new=[1, big]), "sum": dict(starts=[4, big - 2]), "block": dict(block_lists=[[1], [big]]),
+              "slot": dict(slots=[0, -big - 1]), "row": dict(logit_rows=[0, big + 2])}[what])
+    with pytest.raises(OverflowError):
+        RaggedMeta.build(**a)
+
+
 def test_range_of_host_tokens():
     f = cpu_ops().int_range
     assert f([]) == (0, -1) and f([torch.empty(0, dtype=torch.int64)]) == (0, -1)
