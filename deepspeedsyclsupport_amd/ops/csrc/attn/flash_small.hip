@@ -407,8 +407,14 @@ __global__ void __launch_bounds__(NTHR, 2) small_fwd_kernel(SmallArgs<T> a) {
 // the result's accuracy (0.0023 for 0.0020 off 64 bits). 64-byte rows, chunk ch of row r at 16 (ch ^ swz32(r)):
 // K's rows in that order and V's transposed reads touch every bank once. Two workgroups of eight waves share a CU.
 // us, the general kernel and this one: [256, 256, 4, 32] 43.5 and 40.3, [180, 230, 8, 32] 57 and 51, [128, 200, 4, 32] 23.5 and 19.2,
-// [100, 133, 8, 32] 29.6 and 24.9, [512, 32, 8, 32] 28.7 and 12.6; [140, 256, 4, 32] 26.4 and 28.1. Where few CUs
-// get a second large workgroup the general kernel's smaller ones are shared out better ([77, 199, 4, 32], 308 of them, 17.1 and 18.4).
+// [100, 133, 8, 32] 29.6 and 24.9, [512, 32, 8, 32] 28.7 and 12.6.
+// Large workgroups share out worse than the general kernel's of four waves where a CU has at most one and could have two of those,
+// and where some CUs get a second one and most do not; those shapes stay with it. General and this, us, at 4 heads: 128
+// workgroups of six waves (180 tokens) 8.4 and 9.1, of seven (210) 10.0 and 10.2, of eight (250) 10.2 and 11.2, but of five (150) 8.5 and
+// 8.2; 160 of them 10.2 and 9.2, 11.9 and 10.3, 12.3 and 11.5, 10.0 and 8.3. 264 / 384 of eight 17.1 and 18.4 / 18.8 and 19.4, of seven 16.1 and
+// 15.2 / 17.9 and 16.9; 416 of eight 23.6 and 19.6. (A third one has no such bound: 528 / 600 of eight 26.6 and 26.9 / 27.9 and 27.5.)
+// What the line leaves slower: two waves, up to 256 workgroups, 4.9 and 5.1; 1200 of four (128 tokens) 18.3 and 19.5; and keys of another
+// number than the queries, 560 of four waves and 256 keys 16.4 and 19.0, 640 of eight and 100 keys 16.6 and 18.3.
 // (Tried beside 39 with another rule for the maximum: several z a workgroup, the next one's K and V on their way, 40.5; four waves 43.)
 constexpr int FWD_WHOLE = 256, FWD_WAVES = 8;
 __device__ __forceinline__ int swz32(int r) { return ((r >> 2) & 1) | ((r >> 3) & 2); }
@@ -1341,7 +1347,8 @@ int launch_small(SmallArgs<T> a, bool bwd, hipStream_t st) {
       // (below 8 keys a row has no 16 bytes of bias; above 256 K and V would leave a CU one workgroup)
       const int qt = (a.S + 31) / 32, blocks = (qt + FWD_WAVES - 1) / FWD_WAVES, waves = (qt + blocks - 1) / blocks;
       const int64_t groups = (int64_t)blocks * a.H * a.Z;
-      if (a.Sk >= 8 && a.Sk <= FWD_WHOLE && !(waves > 4 && groups > 256 && groups < 320)) {
+      const bool shared_worse = (waves > 5 && groups <= 128) || (waves == FWD_WAVES && groups > 256 && groups <= 384);
+      if (a.Sk >= 8 && a.Sk <= FWD_WHOLE && !shared_worse) {
         const int rows = (a.Sk + 31) / 32 * 32;
         hipLaunchKernelGGL(small_fwd_whole_kernel<T>, dim3((unsigned)groups), dim3(64 * waves), rows * (2 * 64 + 4) + waves * 128, st, a);
         DS_CHECK_LAUNCH();

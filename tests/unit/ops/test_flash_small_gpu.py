@@ -232,6 +232,17 @@ def test_forward_with_a_pair_bias_by_keys(S, Sk, dtype):
     assert ((out.float() - ref).abs() <= step * ref.abs() + loose * v.float().abs().max()).all()
 
 
+@pytest.mark.parametrize("S", [180, 256])
+@pytest.mark.parametrize("groups", [128, 132, 256, 260, 384, 388])
+def test_forward_on_either_side_of_its_lines(S, groups):
+    """The numbers of workgroups at which the forward's kernel changes, against fp64; P and the result are rounded to 2^-8."""
+    q, k, v, bias1, bias2 = _case(groups // 4, S, 4, 32, torch.bfloat16, True, True, groups // 4, seed=groups)
+    with torch.no_grad():
+        out = FS.flash_small(q, k, v, bias1, bias2, b2_div=groups // 4)
+    ref = FS.reference(*(t.double() for t in (q, k, v, bias1, bias2)), b2_div=groups // 4)
+    assert ((out.double() - ref).abs() <= 2.0**-8 * (ref.abs() + v.double().abs().max())).all()
+
+
 @pytest.mark.parametrize("S", [32, 64, 97, 160, 161, 192, 193, 224, 255])
 def test_one_pass_by_number_of_tiles(S):
     """Gradients of every kernel there is for a number of tiles of 32, at their ends, against fp64: bf16 factors as in the tests above."""
@@ -252,7 +263,7 @@ def test_one_pass_by_number_of_tiles(S):
 def test_masked_runs_of_keys(run, odd):
     """Every other run of keys masked, the others with scores far above: the maximum of a row is that of all its keys, whichever lanes
     and tiles hold them (of the masked ones alone, the others' exponentials would be infinite). Tolerance as in the tests above."""
-    Z, S, H = 8, 200, 2
+    Z, S, H = 72, 200, 2   # (more than 128 workgroups)
     q, k, v, _, bias2 = _case(Z, S, H, 32, torch.bfloat16, False, True, Z, seed=run)
     keys = torch.arange(S, device="cuda") // run % 2
     bias1 = torch.where(keys == odd, -1e9, 100.0).expand(Z, S).bfloat16().contiguous()
@@ -300,7 +311,7 @@ def test_largest_weight_is_exact(dtype, unit, S, top):
     """One key stands up to e^5 above the tiles before it, and it alone has a value: its weight is 1 whatever stood before, so that
     the result is rounded once (2 percent beside that for the exponentials and sums in single precision)."""
     from deepspeedsyclsupport_amd.ops.native import hip_ops
-    Z, H, D = 2, 8, 32
+    Z, H, D = 18, 8, 32   # (more than 128 workgroups)
     q = torch.zeros(Z, S, H, D, device="cuda", dtype=dtype)
     v = torch.zeros_like(q)
     v[:, top] = 1
