@@ -123,7 +123,8 @@ __global__ void __launch_bounds__(WAVES * 64, (MT <= 2 || RB == 4 ? 4 : 2)) deco
     return (int)blockIdx.x * (RB / 2) + i % (RB / 2) + (i < RB / 2 ? 0 : HB);
   };
   // 33 rows and more: bases per wave and bytes per lane (`at`); up to 32, which have the registers, pointers per lane. (Those as a
-  // base and bytes too: hipcc 7.2 gave a step's addresses registers of the sums in <1, 2, false, true>.)
+  // base and bytes without the asm: hipcc 7.2 forms a step's addresses in the upper registers of the second block's sums, <1, 2, false,
+  // true> and <2, 2, false, true>. A test reads the assembly for that.)
   constexpr bool APART = MT == 3;
   const bf16* wp[RB];
 #pragma unroll
