@@ -19,8 +19,10 @@
 //    blocks (no norm) leave as sums, and a second launch pairs them;
 //  * X is read once per workgroup (from L2), which is what bounds wide batches; RB and the parts trade that against workgroups
 //    enough.
-// Two workgroups fit a CU with up to four blocks (128 registers a lane: 33 rows x gated [28672, 4096] 54 us with one, 47 with two), one
-// with eight.
+// Two workgroups fit a CU with up to four blocks where X is normed (128 registers a lane: 33 / 48 rows x gated [28672, 4096] 51.8 / 52.4 us
+// with one, 47.3 / 50.2 with two), whose products wait for vector instructions; without, one with all its registers is faster (33 / 48
+// rows x [16384, 8192] 47 / 48, with two 56 / 49; [4096, 14336] in parts 28 / 28 and 31 / 29; gated [22016, 4096] 42 / 45 and 45 / 46). One with
+// eight.
 // Bound by the weights' read (6.5 TB/s here). Measured, us (the same products as split streams with fp32 atomics and a finalize
 // pass; the floor): 12 rows x [4096, 4096] 9 (14; 5), [4096, 14336] 23 (25; 18), gated [28672, 4096] 38 (45; 36), with the
 // norm 39, [32000, 4096] 42 (51; 40), [2048, 2048] 5.6 (7.6; 1.3). 24 and 40 rows (library GEMM): gated [28672, 4096] 44 and 51 (60
@@ -105,7 +107,7 @@ __device__ __forceinline__ float gate_up(const ShArgs& a, float g, float up, int
 }
 
 template <int MT, int RB, bool NORM, bool GATED>
-__global__ void __launch_bounds__(WAVES * 64, (MT <= 2 || RB == 4 ? 4 : 2)) decode_gemm_kernel(ShArgs a) {
+__global__ void __launch_bounds__(WAVES * 64, (MT <= 2 || (RB == 4 && NORM) ? 4 : 2)) decode_gemm_kernel(ShArgs a) {
   static_assert(!GATED || RB % 2 == 0, "pairs");
   constexpr int T = MT * RB, HALF = WAVES / 2;
   constexpr int U = T == 1 ? 2 : 1;  // steps loaded together
@@ -217,7 +219,7 @@ __global__ void __launch_bounds__(WAVES * 64, (MT <= 2 || RB == 4 ? 4 : 2)) deco
         products(f1, s);
         if ((s += STRIDE) >= end) break;
       }
-    } else {  // four blocks a step: the workgroups beside this one cover its waits, a second set of registers costs more of them
+    } else {  // four blocks and more: other waves cover a step's waits (two to four on a SIMD), a second set of registers costs more of them
       for (; s < end; s += STRIDE) {
         load(f0, s);
         products(f0, s);
@@ -346,11 +348,16 @@ struct Cut {
 // 14; 48 rows with two / four: [8192, 4096] 19 / 24, [9216, 3072] 28 / 19, [12288, 4096] 35 / 26). Products with more blocks than that
 // holds take the most that there are (24 rows x [32000, 4096] 48 with two, 46 with four), up to 16 token rows two (12 rows 42 and 45).
 // Gated pairs take two or four (12 rows: [11264, 2048] 13.0 and 11.0, [28672, 4096] 41 and 38).
-// Eight blocks for 33 rows and more of 4096 and more, where they still make more than 144 workgroups: X, a quarter to a half of what a
-// CU reads, is then read half as often. 33 / 48 rows, us with four and with eight: gated [22016, 4096] 47 / 51 and 41 / 42, [28672, 4096]
-// 47 / 51.5 and 49 / 51, [57344, 8192] 170 / 187 and 158 / 160, [32000, 4096] 52 / 58 and 49 / 49, [20480, 5120] 53 / 59 and 45 / 48. Fewer
-// workgroups leave too many CUs idle (48 rows x [16384, 8192], 128 of them, 51 and 67), and X of 2048 gives nothing (48 rows x
-// [32000, 2048] 29.1 and 31.6). Up to 32 rows it pays for long X alone (32 rows x gated [28672, 4096] 46 and 49).
+// Eight blocks for 33 rows and more of 4096 and more: X, a quarter to a half of what a CU reads, is then read half as often. One workgroup
+// has a CU to itself, so their number decides: where four blocks (two a CU with a norm) fill their rounds as well or better, it stays at
+// four. 33 / 48 rows, us with four and with eight. Normed, 129 to 256 workgroups of eight: [18432, 4096] 42 / 47 and 36 / 38, gated [22016, 4096]
+// 43 / 48 and 40 / 41, [28672, 4096] 47 / 50 and 45 / 46, [32000, 4096] 48 / 53 and 48 / 50; 272 to 384 of them, a second round that is half
+// empty: gated [38912, 4096] 65 / 71 and 78 / 82; 385 and more: [50304, 4096] 86 / 94 and 84 / 86, gated [57344, 8192] 162 / 184 and 156 / 161 ([128256,
+// 4096], four rounds, 184 / 204 and 191 / 197). Without a norm, up to 200: [17408, 4096] 41 / 45 and 39 / 39, [20480, 5120] 52 / 57 and 48 / 49, gated
+// [22016, 4096] 42 / 45 and 43 / 42; but gated [28672, 4096] 43.5 / 47 and 46 / 47, [32000, 4096] 48.6 / 49.6 and 52 / 51, [40960, 4096] 67 / 69 and
+// 83 / 84, [65536, 4096] 93 / 97 and 102 / 103. Up to 1024 blocks four make one round (48 rows x [16384, 8192] 48 and 69), and X of 2048
+// gives nothing (33 / 48 rows x [32000, 2048] 27 / 28 and 30 / 31). Up to 32 rows it pays for long X alone (32 rows x gated [28672, 4096] 46
+// and 49).
 // More than 16 token rows of 4096 and more over few blocks: what a CU can read (30 bytes a nanosecond) bounds one block's workgroup,
 // and of that most is X. Several blocks share the reading, and parts of K keep the workgroups at 256; the parts' sums are a launch of
 // 4 us. 48 rows, us with one block and with this: [4096, 4096] 16.3 and 14.6, [4096, 14336] 45 and 28, [2048, 5632] 20.6 and 13.5; 17
@@ -363,7 +370,9 @@ struct Cut {
 // 6.9, x [1024, 8192] 9.6 and 8.4), and where long ones stand a quarter over one round (16 rows x [10240, 8192] 40 and 35).
 Cut cut_of(int M, int N, int K, bool gated, bool norm) {
   const int blocks = gated ? N / 16 : (N + 15) / 16, mt = (M + 15) / 16, most = gated || mt > 1 ? 4 : 2;
-  int rb = blocks <= 256 && !gated ? 1 : blocks <= 512 ? 2 : mt == 3 && blocks > 1152 && K >= 4096 ? 8 : most, parts = 1;
+  const int eights = (blocks + 7) / 8;  // workgroups of eight blocks
+  const bool eight = mt == 3 && K >= 4096 && blocks > 1024 && (norm ? (eights - 1) % 256 >= 128 : eights <= 200);
+  int rb = blocks <= 256 && !gated ? 1 : blocks <= 512 ? 2 : eight ? 8 : most, parts = 1;
   if (!gated && !norm) {
     int fill = 0;  // workgroups that parts may make
     if (mt == 1) {
