@@ -105,9 +105,10 @@ def build_bwd_lut(layout, blk, L, H, device, key=None):
 
 # Workgroups that lists are shared out over, and the shortest part worth cutting, in tiles: by rows (64 keys), for the forward and
 # dQ, and by columns (32 rows). The chip holds 512 of either at once; a part costs its operands' first load and a pass of its
-# accumulators through memory, 32 to 64 KB. Measured, us, forward / backward: BigBird B2 H8 L16384 with (512, 8), (256, 8) 153 /
-# 387; (768, 8), (512, 16) 157 / 372; (1024, 16), (4096, 8) 152 / 407; Fixed B1 H8 L8192 98 / 352, 91 / 305, 110 / 419.
-_FWD_SHARE, _BWD_SHARE = (768, 8), (512, 16)
+# accumulators through memory, 32 to 64 KB. Measured, us, forward / forward and backward, rows over 512, 640 and 768: BigBird B2 H8
+# L16384 105 / 416, 111 / 420, 114 / 424; a random 15 % B2 H8 L4096 44 / 155, 56 / 165, 60 / 169; Fixed B1 H4 L4096 of 32 tokens 54 / 172, 62 /
+# 184, 62 / 184. Columns over 256 with parts of at least 8 and over 512 of 16, backward alone: 387 and 372 (BigBird), 352 and 305 (Fixed, L8192).
+_FWD_SHARE, _BWD_SHARE = (512, 8), (512, 16)
 
 PlanSide = namedtuple("PlanSide", "tiles masks work merges nslots")
 
