@@ -1310,10 +1310,12 @@ int db2_splits(int Z, int H, int S, int b2_div) {
 // Elements of the pair bias in the accumulators' order, for what goes through one pass for dQ, dK and dV; 0: two passes. Pair biases
 // of their own for every z would be read and written once more than they are used, and fewer than a workgroup a CU leave the chip
 // idle (dQ, dK and dV in two passes and in one, us: [32, 256, 4, 32] 23 and 24, [24, 40, 4, 32] 13 and 14; [128, 200, 4, 32] 54 and 36,
-// [100, 133, 8, 32] 69 and 49, [512, 32, 8, 32] 61 and 23, [256, 250, 8, 32] 185 and 133).
+// [100, 133, 8, 32] 69 and 49, [512, 32, 8, 32] 61 and 23, [256, 250, 8, 32] 185 and 133). Of four tiles, which fill the two passes'
+// workgroups and have no kernel of their own here, more of them: [100, 128, 4, 32] 21.6 and 23.1, [128, 128, 4, 32] 22.7 and 24.8, [160, 128, 4,
+// 32] 28.6 and 28.5, [256, 128, 4, 32] 42 and 34.
 int64_t small_order_elements(int Z, int H, int S, int D, int b2_div, bool drop) {
-  const int64_t nt = (S + 31) / 32;
-  return D == 32 && S <= WHOLE_S && !drop && b2_div > 1 && (int64_t)Z * H >= 256 ? (int64_t)(Z / b2_div) * H * nt * nt * 1024 : 0;
+  const int64_t nt = (S + 31) / 32, least = nt == 4 ? 640 : 256;
+  return D == 32 && S <= WHOLE_S && !drop && b2_div > 1 && (int64_t)Z * H >= least ? (int64_t)(Z / b2_div) * H * nt * nt * 1024 : 0;
 }
 
 // Kernels of their own for one tile and for five to eight: in the one for any number, addresses and the turns at dQ are a quarter of a
