@@ -277,10 +277,10 @@ def test_masked_runs_of_keys(run, odd):
 _MASKS = [-1e4, -1e5, -1e6, -1e7, -1e9, -5e9, -1e10, -1e15, -1e20, torch.finfo(torch.bfloat16).min]
 
 
-def _masked_case(mask):
+def _masked_case(mask, S=100):
     """Whole rows masked by `mask`, rows whose first 32 (64) keys are, a third of the keys at random. Queries and keys are small whole
     numbers and their products exact, so that the scores can be told to the last bit: fma(q k, scale, bias1 + bias2) in single precision."""
-    Z, S, H, D = 128, 100, 2, 32
+    Z, H, D = 128, 2, 32
     g = torch.Generator(device="cuda").manual_seed(17)
     q, k = (torch.randint(-2, 3, (Z, S, H, D), device="cuda", generator=g).bfloat16() for _ in range(2))
     v, do = (torch.randn(Z, S, H, D, device="cuda", generator=g).bfloat16() for _ in range(2))
@@ -305,6 +305,31 @@ def test_finite_masks_forward(mask):
     assert ((o.double() - want).abs() <= 2.0**-9 * want.abs() + 2.0**-8 * v.double().abs().max()).all()
     want = torch.logsumexp(s, -1)
     assert ((lse.double() - want).abs() <= 2.0**-22 * want.abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("mask", _MASKS)
+@pytest.mark.parametrize("S", [70, 100])
+def test_finite_masks_backward(S, mask):
+    """In one pass for all gradients (70) and in two (100). Where some keys are not masked, against fp64 as in the tests above. Rows
+    masked throughout: their scores, and LSE, stand 64 apart at -1e9, so that a weight may come out as 1 for 1 / S, but as no more:
+    the gradients are bounded by those of such weights."""
+    from deepspeedsyclsupport_amd.ops.native import hip_ops
+    q, k, v, do, b1, b2, s = _masked_case(mask, S)
+    scale = 32**-0.5
+    o, lse = hip_ops().flash_small_fwd(q, k, v, b1, b2, 64, scale, 0.0, 0)
+    dq, dk, dv, db1, db2 = hip_ops().flash_small_bwd(do, q, k, v, o, lse, b1, b2, 64, scale, 0.0, 0, True, True)
+    assert all(bool(t.isfinite().all()) for t in (dq, dk, dv, db1, db2))
+    qd, kd, vd, dod = (t.double().transpose(1, 2) for t in (q, k, v, do))
+    p = torch.softmax(s, -1)
+    dp = dod @ vd.transpose(-1, -2) - (dod * o.double().transpose(1, 2)).sum(-1, keepdim=True)
+    ds = p * dp
+    want = [t.transpose(1, 2) for t in (scale * (ds @ kd), scale * (ds.transpose(-1, -2) @ qd), p.transpose(-1, -2) @ dod)]
+    most = [t.transpose(1, 2) for t in (scale * (dp.abs() @ kd.abs()), scale * (dp.abs().transpose(-1, -2) @ qd.abs()),
+                                        dod.abs().sum(-2, keepdim=True).expand_as(vd))]
+    some = torch.arange(q.shape[0], device="cuda") % 4 != 0
+    for name, a, w, m in zip(("dq", "dk", "dv"), (dq, dk, dv), want, most):
+        assert ((a.double() - w)[some].abs() < 4e-2 * w[some].abs().max() + 4e-2).all(), name
+        assert (a.double().abs()[~some] <= 1.02 * m[~some] + 1e-3).all(), name
 
 
 @pytest.mark.parametrize("dtype,unit", [(torch.bfloat16, 2.0**-8), (torch.float16, 2.0**-11)], ids=["bf16", "fp16"])
