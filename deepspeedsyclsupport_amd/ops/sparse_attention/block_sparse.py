@@ -21,29 +21,23 @@ import torch
 
 from ..native import hip_ops
 
-_LUTS = {}
-
 
 def _bits(layout):
     return layout.detach().cpu().contiguous().numpy() != 0
 
 
-def _lut_key(layout, blk, L, device):
-    """The layout's contents (one bit per block) and what else a LUT depends on."""
-    bits = layout if isinstance(layout, np.ndarray) else _bits(layout)
+def _plan_key(bits, blk, L, device):
+    """The layout's contents (one bit per block) and what else a plan depends on."""
     return (np.packbits(bits).tobytes(), bits.shape, blk, L, str(device))
 
 
-def build_lut(layout, blk, L, device, key=None):
+def build_lut(layout, blk, L, device):
     """layout [H, nb, nb] (0/1) -> (tiles int32 [LH, nqb, T], ntiles int32 [LH, nqb], layout uint8 [LH, nb, nb],
     qorder int32 [LH, nqb] = query blocks by descending tile count, the kernel's launch order).
 
     LH = 1 when every head shares one layout. Tile t of query block qb is listed when any key of 64-key tile t is
-    allowed for any of the 128 query rows of qb; the tile lists are ascending."""
-    key = key or _lut_key(layout, blk, L, device)
-    hit = _LUTS.get(key)
-    if hit is not None:
-        return hit
+    allowed for any of the 128 query rows of qb; the tile lists are ascending. For statistics and tests: the kernels read the
+    lists of `SparseLists`, which come from the masks and say the same."""
     lay = layout.to(torch.bool)
     if lay.shape[0] > 1 and bool((lay == lay[:1]).all()):
         lay = lay[:1]
@@ -57,24 +51,13 @@ def build_lut(layout, blk, L, device, key=None):
     T = max(int(ntiles.max()), 1)
     order = torch.sort((~t64).to(torch.int8), dim=-1, stable=True).indices[..., :T].to(torch.int32)
     qorder = torch.sort(ntiles, dim=-1, descending=True, stable=True).indices.to(torch.int32)  # heaviest first
-    lut = (order.contiguous().to(device), ntiles.contiguous().to(device),
-           lay.to(torch.uint8).contiguous().to(device), qorder.contiguous().to(device))
-    if len(_LUTS) > 64:
-        _LUTS.clear()
-    _LUTS[key] = lut
-    return lut
+    return (order.contiguous().to(device), ntiles.contiguous().to(device), lay.to(torch.uint8).contiguous().to(device),
+            qorder.contiguous().to(device))
 
 
-_BWD_LUTS = {}
-
-
-def build_bwd_lut(layout, blk, L, H, device, key=None):
+def build_bwd_lut(layout, blk, L, H, device):
     """Column LUT of the sparse backward: (qtiles int32 [H, nkb, T] = 32-row query tiles met by each 256-key block,
-    ascending, nqt int32 [H, nkb], layout uint8 [LH, nb, nb] at granularity blk' = min(blk, 128), blk')."""
-    key = (key or _lut_key(layout, blk, L, device)) + (H,)
-    hit = _BWD_LUTS.get(key)
-    if hit is not None:
-        return hit
+    ascending, nqt int32 [H, nkb], layout uint8 [LH, nb, nb] at granularity blk' = min(blk, 128), blk'). For tests, as above."""
     lay = layout.to(torch.bool)
     if lay.shape[0] > 1 and bool((lay == lay[:1]).all()):
         lay = lay[:1]
@@ -95,12 +78,7 @@ def build_bwd_lut(layout, blk, L, H, device, key=None):
     order = torch.sort((~met).to(torch.int8), dim=-1, stable=True).indices[..., :T].to(torch.int32)
     if LH == 1 and H > 1:
         order, nqt = order.expand(H, nkb, T), nqt.expand(H, nkb)
-    out = (order.contiguous().to(device), nqt.contiguous().to(device), lay.to(torch.uint8).contiguous().to(device),
-           blk)
-    if len(_BWD_LUTS) > 64:
-        _BWD_LUTS.clear()
-    _BWD_LUTS[key] = out
-    return out
+    return order.contiguous().to(device), nqt.contiguous().to(device), lay.to(torch.uint8).contiguous().to(device), blk
 
 
 # Workgroups that lists are shared out over, and the shortest part worth cutting, in tiles: by rows (64 keys), for the forward and
@@ -226,7 +204,7 @@ class SparsePlan:
     def forward(self):
         return self.lists.side("fwd", _FWD_SHARE, self.B, self.H)
 
-    def backward(self):
+    def backward(self):   # (by 256 keys, whole lists: for tests; the kernels read `rows` and `columns`)
         return self.lists.side("bwd", _BWD_SHARE, self.B, self.H)
 
     # the same lists, shared out by blocks of 64 rows (keys): what the backward's kernels read
@@ -242,7 +220,7 @@ _PLANS = {}
 
 def sparse_plan(layout, blk, L, B, H, device):
     bits = _bits(layout)
-    key = _lut_key(bits, blk, L, device)
+    key = _plan_key(bits, blk, L, device)
     lists = _PLANS.get(key)
     if lists is None:
         if len(_PLANS) > 64:

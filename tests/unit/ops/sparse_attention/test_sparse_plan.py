@@ -106,7 +106,7 @@ def test_parts_of_all_heads_are_numbered_through():
     lay[3] = lay[5] = 1
     bs._PLANS.clear()
     plan = bs.sparse_plan(lay, blk, L, 1, H, "cpu")
-    for side in (plan.forward(), plan.backward()):
+    for side in (plan.forward(), plan.backward(), plan.rows(), plan.columns()):
         used = sorted(e[3] for head in side.work.tolist() for e in head if e[3] >= 0)
         assert used and used == list(range(side.nslots))
         joined = sorted(s for head in side.merges.tolist() for b, first, k, _ in head if b >= 0 for s in range(first, first + k))
@@ -132,6 +132,23 @@ def test_batch_sizes_share_the_lists(kind, monkeypatch):
         assert [side.tiles.data_ptr() for side in (plan.forward(), plan.backward())] == want
         work, merges, nslots = bs._share_out(bs.build_lut(lay, blk, L, "cpu")[1], B * H if kind == "shared" else B, *bs._FWD_SHARE)
         assert torch.equal(plan.forward().work, work) and plan.forward().nslots == nslots
+        assert [side.tiles.data_ptr() for side in (plan.rows(), plan.columns())] == want
+    bs._PLANS.clear()
+
+
+@pytest.mark.parametrize("kind", ["shared", "heads", "empty"])
+@pytest.mark.parametrize("blk,L", [(16, 256), (32, 640), (64, 1152), (128, 1280), (256, 1280)])
+def test_lists_are_those_of_the_layout(kind, blk, L):
+    """The plan's lists, made from its masks, against those made from the layout."""
+    lay = _layout(kind, 2, blk, L)
+    plan = bs.sparse_plan(lay, blk, L, 1, 2, "cpu")
+    for side, (tiles, counts) in ((plan.rows(), bs.build_lut(lay, blk, L, "cpu")[:2]), (plan.columns(), bs.build_bwd_lut(lay, blk, L, 2, "cpu")[:2])):
+        listed = (side.masks != 0).sum(-1)
+        for head in range(2):
+            mine = min(head, side.tiles.shape[0] - 1), min(head, tiles.shape[0] - 1)
+            assert torch.equal(listed[mine[0]].int(), counts[mine[1]])
+            for block, n in enumerate(counts[mine[1]].tolist()):
+                assert torch.equal(side.tiles[mine[0], block, :n], tiles[mine[1], block, :n])
     bs._PLANS.clear()
 
 
