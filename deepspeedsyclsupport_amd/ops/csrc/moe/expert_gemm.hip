@@ -11,8 +11,8 @@
 //    operand order and every wave has rows of its own, so they go from memory to registers in 512-byte runs, one step of 64
 //    ahead; only the entries' rows pass through LDS (swizzled, two buffers). Two workgroups share a CU. Workgroups walk groups
 //    of 4 column tiles by all row tiles of an expert, so that those at work on an XCD at a time share both operands in its L2.
-//  * big tile: a hundred rows per expert or more. 256 entries x 256 weight rows per workgroup of 8 waves, both operands through LDS
-//    by DMA (two buffers of 64 columns, 128 KB): see expert_big_kernel.
+//  * big tile: a hundred rows per expert or more. 256 entries x 256 weight rows per workgroup of 4 waves, entries' rows through LDS by
+//    DMA (four buffers of 64 columns, 128 KB), weights straight into registers: see expert_big_kernel.
 //  * any: a workgroup per entry and 64 columns; fp32 and widths that are no multiple of 8.
 #include "ds_hip.h"
 
@@ -29,6 +29,10 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.f + expf(-g)) * u; }
+// By the hardware's exponential and reciprocal; the quarter keeps the latter's result a normal number
+__device__ __forceinline__ float silu_mul_fast(float g, float u) {
+  return 0.25f * g * __builtin_amdgcn_rcpf(fmaf(0.25f, __expf(-g), 0.25f)) * u;
+}
 enum : int { NONE = 0, SILU_GLU = 1, RELU2 = 2 };  // activation codes
 __device__ __forceinline__ float plain_act(float x, int act) {
   if (act != RELU2) return x;
@@ -44,6 +48,7 @@ struct ExpertArgs {
   const int* offs;       // [E + 1] and
   const int* order;      // [entries], or null (up to FEW entries)
   int entries, E, N, K, div, act;
+  uint32_t xbytes;       // of x, 0 if that is not 32 bits
 };
 
 // Operand order of a weight matrix [rows, K] (ops/bf16_gemv.py): 16 x 64 tiles of 1024 elements, tile by tile along K;
@@ -223,65 +228,59 @@ __global__ void __launch_bounds__(256) expert_stream_kernel(ExpertArgs a) {
 // ------------------------------------------------------------------------------------------------ many rows per expert
 constexpr int BM = 128, BN = 256, GROUP = 4;
 
+// Row tiles (of TM entries) of all experts laid end to end; this workgroup's place among them.
 struct Place {
-  int pre[MAXE + 1], offs[MAXE + 1], found;
+  int e, first, left, n0;  // expert, its first entry here (as listed), entries from there on, first column
 };
-// Row tiles (of TM entries) of all experts laid end to end; this workgroup's place among them: expert, first entry, first column.
-// false: there is nothing for it. block-uniform.
+// false: there is nothing for this workgroup. Every wave finds it by itself, four experts a lane: no LDS, no barrier.
 template <int TM, int GROUPS>
-__device__ __forceinline__ bool place_of(const ExpertArgs& a, Place& pl, int per, int& e, int& m0, int& n0) {
-  const int tid = threadIdx.x, lane = tid & 63, threads = blockDim.x, nt = (a.N + per - 1) / per;
-  for (int i = tid; i <= a.E; i += threads) pl.offs[i] = a.offs[i];
-  __syncthreads();
-  if (tid < 64) {
-    int c[4], s = 0;
+__device__ __forceinline__ bool place_of(const ExpertArgs& a, int per, Place& p) {
+  const int lane = threadIdx.x & 63, nt = (a.N + per - 1) / per;
+  int o[5], c[4], s = 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int x = 4 * lane + i;
-      c[i] = x < a.E ? (pl.offs[x + 1] - pl.offs[x] + TM - 1) / TM : 0;
-      s += c[i];
-    }
-    int run = s;
+  for (int i = 0; i < 5; ++i) o[i] = a.offs[min(4 * lane + i, a.E)];  // (past the last expert: no entries)
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(run, o, 64);
-      if (lane >= o) run += y;
-    }
-    int at = run - s;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (4 * lane + i < a.E) pl.pre[4 * lane + i] = at;
-      at += c[i];
-    }
-    if (lane == 63) pl.pre[a.E] = run;
+  for (int i = 0; i < 4; ++i) {
+    c[i] = (o[i + 1] - o[i] + TM - 1) / TM;
+    s += c[i];
   }
-  __syncthreads();
-  const int total = pl.pre[a.E] * nt;
+  int run = s;
+#pragma unroll
+  for (int k = 1; k < 64; k <<= 1) {
+    const int y = __shfl_up(run, k, 64);
+    if (lane >= k) run += y;
+  }
+  const int total = __builtin_amdgcn_readlane(run, 63) * nt;
   if ((int)blockIdx.x >= total) return false;
   const int id = xcd_remap(blockIdx.x, total);
-  for (int x = tid; x < a.E; x += threads)
-    if (pl.pre[x] * nt <= id && id < pl.pre[x + 1] * nt) pl.found = x;
-  __syncthreads();
-  e = pl.found;
-  const int mt = pl.pre[e + 1] - pl.pre[e], local = id - pl.pre[e] * nt, g = local / (mt * GROUPS);
-  const int rest = local - g * mt * GROUPS, width = min(GROUPS, nt - g * GROUPS);
-  m0 = rest / width * TM;
-  n0 = (g * GROUPS + rest % width) * per;
+  const int owner = __builtin_ctzll(__ballot(id < run * nt));  // the first lane whose experts reach that far
+  int at = run - s, e = 0, lo = 0, hi = 0, mt = 1;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {  // (each lane for its own experts; the owner's count)
+    if (at * nt <= id && id < (at + c[i]) * nt) e = 4 * lane + i, lo = o[i], hi = o[i + 1], mt = c[i], s = at;
+    at += c[i];
+  }
+  auto of = [&](int v) { return __builtin_amdgcn_readlane(v, owner); };
+  const int tiles = of(mt), local = id - of(s) * nt, g = local / (tiles * GROUPS);
+  const int rest = local - g * tiles * GROUPS, width = min(GROUPS, nt - g * GROUPS), m0 = rest / width * TM;
+  p.e = of(e);
+  p.first = of(lo) + m0;
+  p.left = of(hi) - p.first;
+  p.n0 = (g * GROUPS + rest % width) * per;
   return true;
 }
 
 template <bool GLU>
 __global__ void __launch_bounds__(256, 2) expert_tile_kernel(ExpertArgs a) {
   __shared__ __attribute__((aligned(16))) bf16 xs[2][BM * 64];
-  __shared__ Place pl;
   __shared__ int ents[BM];
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int N = a.N, K = a.K, KQ = K / 64;
-  int e, m0, n0;
-  if (!place_of<BM, GROUP>(a, pl, GLU ? BN / 2 : BN, e, m0, n0)) return;
-  const int left = min(BM, pl.offs[e + 1] - pl.offs[e] - m0);
-  if (tid < BM) ents[tid] = a.order[pl.offs[e] + m0 + min(tid, left - 1)];
+  Place pl;
+  if (!place_of<BM, GROUP>(a, GLU ? BN / 2 : BN, pl)) return;
+  const int e = pl.e, n0 = pl.n0, left = min(BM, pl.left);
+  if (tid < BM) ents[tid] = a.order[pl.first + min(tid, left - 1)];
   __syncthreads();
   // ---- entries' rows on their way to LDS: 8 rows of 8 pieces per wave and access, piece p of row r holding columns
   // 8 (p ^ (r / 2 % 8)) .. + 7
@@ -375,7 +374,7 @@ __global__ void __launch_bounds__(256, 2) expert_tile_kernel(ExpertArgs a) {
         bf16x4 o;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          o[i] = (bf16)(GLU ? silu_mul(acc[0][m][4 * q + i], acc[1][m][4 * q + i]) : plain_act(acc[t][m][4 * q + i], a.act));
+          o[i] = (bf16)(GLU ? silu_mul_fast(acc[0][m][4 * q + i], acc[1][m][4 * q + i]) : plain_act(acc[t][m][4 * q + i], a.act));
         *reinterpret_cast<bf16x4*>(yr + n + 8 * q + 4 * hh) = o;
       }
     }
@@ -384,207 +383,194 @@ __global__ void __launch_bounds__(256, 2) expert_tile_kernel(ExpertArgs a) {
 
 // ------------------------------------------------------------------------------------------------ hundreds of rows per expert
 // What bounds the tile kernel above is traffic into the CU: for each step of 64 columns its two workgroups take 2 x (128 + 256)
-// rows, 48 bytes a clock at the full matrix rate. One tile of 256 x 256 takes 32, all of it by DMA, without registers. Eight
-// waves, 64 weight rows (gated: 32 of either part) x 128 entries each: two on a SIMD, so that one has products to issue while the
-// other's transfers wait to be taken (four waves of 128 x 128, with a third less to read from LDS: 1.08 times the time). The
-// barrier comes ahead of a step's last quarter, whose operands are in registers by then, and the next step's first reads right
-// behind it; transfers are issued a quarter at a time, between products. Rows come swizzled (the source address carries it),
-// weights in operand order: reads without bank conflicts. Workgroups walk groups of 8 column tiles by all row tiles of an expert.
-// 32 experts, 1024 rows each on average: 3584 gated columns of 4096: 2180 -> 1790 us (1076 TFLOP/s; a third of the requests
-// miss the L2, the matrix cores are busy 55 % of the time); 4096 plain columns of 3584: 1115 -> 950 us.
-constexpr int TM = 256, TN = 256, BIG_BUF = (TM + TN) * 128, BIG_LDS = 2 * BIG_BUF;
+// rows, 48 bytes a clock at the full matrix rate. One tile of 256 x 256 takes 32. Of that tile's step (2048 clocks of the matrix
+// cores) LDS would be busy as long with both operands in it and waves of 64 x 128; so
+//  * four waves, one on a SIMD with all its registers, have 64 weight rows (gated: 32 of either part) by all 256 entries each: no
+//    wave reads another's weights, which go from memory (operand order: 512-byte runs) to registers two steps ahead. LDS carries the
+//    entries' rows alone, 1280 of the 2048 clocks, by DMA three steps ahead into four buffers; swizzled by the source address,
+//    read without bank conflicts a quarter step ahead;
+//  * a step is 64 products of 32 x 32 x 16; one LDS read, at most one transfer and one load of weights go between two of them. One barrier a
+//    step. Every wait counts what may still be on its way: buffers are arrays apart, and all accesses buffer instructions (hipcc waits
+//    for everything where LDS transfers are global ones), so the compiler's own waits for weights count too. Tail steps issue the last
+//    step's transfers again, so that the counts stand;
+//  * rows in units of 64 (MT): a short tile moves and multiplies no others.
+// Workgroups walk groups of 8 column tiles by all row tiles of an expert. Then bound by power: 1.6 GHz, matrix cores busy 77 % of the time in
+// a long loop; without any transfers 1.75 GHz and 83 %. 16 x 16 x 32 products: hipcc moves accumulators about, 1.05 times the time.
+// 32 experts, 1024 rows each on average, at random: 3584 gated columns of 4096: 1805 -> 1600 us (all even 1680 -> 1490), 4096 plain columns of
+// 3584: 978 -> 891 us (eight waves, both operands in LDS, a wait for all transfers every step); 256 rows: 657 -> 574; 8 x 128 rows: 111 -> 92.
+// Of these the gate by the hardware's exponential and reciprocal 4 % (32 outputs a lane and tile, 8 us), finding the place in registers 2 %.
+constexpr int TM = 256, TN = 256;
 typedef __attribute__((address_space(3))) char lds_char;
 typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
+typedef __attribute__((address_space(3))) void lds_void;
 
-// 16 bytes per lane from global memory to LDS byte `dst` + OFF + 16 * lane. Inline asm: hipcc waits for its own such loads before
-// every LDS read that it cannot prove apart from them.
-template <int OFF>
-__device__ __forceinline__ void dma16(const void* g, uint32_t dst) {
-  uint32_t keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
-               "s_mov_b32 m0, %0"
-               : "=&s"(keep)
-               : "v"(g), "s"(dst), "n"(OFF)
-               : "memory", "scc");
+// 16 bytes per lane to LDS bytes dst + 16 lane. (The host's pass does not know the size.)
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t from, uint32_t lane_bytes, uint32_t bytes, lds_char* dst) {
+#ifdef __HIP_DEVICE_COMPILE__
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void*)dst, 16, lane_bytes, bytes, 0, 0);
+#endif
 }
-template <int OFF>
-__device__ __forceinline__ void dma16_s(const void* base, uint32_t voff, uint32_t dst) {  // wave-uniform base, offset per lane
-  uint32_t keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_add_u32 m0, %3, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\t"
-               "s_mov_b32 m0, %0"
-               : "=&s"(keep)
-               : "v"(voff), "s"(base), "s"(dst), "n"(OFF)
-               : "memory", "scc");
+// All of this wave's LDS accesses and all but its NEWER latest loads are done, then those of all waves.
+template <int NEWER>
+__device__ __forceinline__ void meet() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((NEWER & 15) | 7 << 4 | (NEWER >> 4) << 14);
+  asm volatile("s_barrier" ::: "memory");
 }
 
-template <bool GLU, int NW>
-__global__ void __launch_bounds__(NW * 64, NW / 4) expert_big_kernel(ExpertArgs a) {
-  constexpr int NP = 16 / NW, WT = 16 / NW, XP = 32 / NW;  // weight parts of 32 rows; weight tiles and rows' pieces moved per wave
-  extern __shared__ __attribute__((aligned(16))) char smem[];  // [2][256 rows x 64 | 16 weight tiles of 16 x 64]
-  __shared__ Place pl;
+template <bool GLU>
+__global__ void __launch_bounds__(256, 1) expert_big_kernel(ExpertArgs a) {
+  // rows of a step each, as arrays apart: the compiler then knows which transfers a read has to wait for
+  __shared__ __attribute__((aligned(16))) char b0[TM * 128], b1[TM * 128], b2[TM * 128], b3[TM * 128];
   __shared__ int ents[TM];
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
-  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), wc = wid % (NW / 2), wr = wid / (NW / 2);
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int N = a.N, K = a.K, KQ = K / 64;
-  int e, m0, n0;
-  if (!place_of<TM, 8>(a, pl, GLU ? TN / 2 : TN, e, m0, n0)) return;
-  e = __builtin_amdgcn_readfirstlane(e);
-  m0 = __builtin_amdgcn_readfirstlane(m0);
-  n0 = __builtin_amdgcn_readfirstlane(n0);
-  const int left = min(TM, __builtin_amdgcn_readfirstlane(pl.offs[e + 1] - pl.offs[e]) - m0);
-  if (tid < TM) ents[tid] = a.order[pl.offs[e] + m0 + min(tid, left - 1)];
-  __syncthreads();
-  // ---- what this wave moves per step: pieces of 8 entries' rows (piece p of row r: columns 8 (p ^ (r / 2 % 8)) .. + 7) and
-  // weight tiles, a piece per half
-  const bf16* xp[XP];
-  const bf16* wp[WT];
+  Place pl;
+  if (!place_of<TM, 8>(a, GLU ? TN / 2 : TN, pl)) return;
+  const int e = pl.e, n0 = pl.n0, left = min(TM, pl.left);
+  const auto xs = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, (int)a.xbytes, 0x00020000);
+  // ---- this wave's 2 x 32 weight rows: gate and up of the same columns, or 64 neighbours
+  __amdgpu_buffer_rsrc_t ws[2];
 #pragma unroll
-  for (int i = 0; i < XP; ++i) {
-    const int r = wid * 8 * XP + i * 8 + (lane >> 3);
-    xp[i] = (const bf16*)a.x + (int64_t)(ents[r] / a.div) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7));
+  for (int t = 0; t < 2; ++t) {
+    const int row = GLU ? min(n0 + 32 * wid, N - 32) + t * N : min(n0 + 64 * wid + 32 * t, N - 32);
+    ws[t] = __builtin_amdgcn_make_buffer_rsrc((bf16*)a.w + ((int64_t)e * (GLU ? 2 : 1) * N + row) * K, 0, 64 * K, 0x00020000);
   }
-#pragma unroll
-  for (int i = 0; i < WT; ++i) {
-    const int t = WT * wid + i, row = GLU ? min(n0 + 16 * (t & 7), N - 16) + (t >> 3) * N : min(n0 + 16 * t, N - 16);
-    wp[i] = (const bf16*)a.w + ((int64_t)e * (GLU ? 2 : 1) * N + row) * K;
-  }
-  // the entries are the loads that the compiler tracks: done before the first transfer
-#pragma unroll
-  for (int i = 0; i < XP; ++i) asm volatile("" : "+v"(xp[i]));
-  const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_char*)smem + 1024 * XP * wid);
-  // piece p of 2 XP of step kq: the first half entries' rows, the others weight tiles
-  auto move = [&](int kq, auto buf_c, auto p_c) {
-    constexpr int B = decltype(buf_c)::value * BIG_BUF, p = decltype(p_c)::value;
-    if constexpr (p < XP) dma16<B + 1024 * p>(xp[p] + (int64_t)kq * 64, dst);
-    else dma16_s<B + TM * 128 + 1024 * (p - XP)>(wp[(p - XP) / 2] + (int64_t)kq * 1024 + (p & 1) * 512, lane * 16, dst);
+  const uint32_t wo = (uint32_t)(l32 >> 4) * KQ * 2048 + hh * 256 + (l32 & 15) * 16;
+  auto buffer = [&](auto b_c) -> lds_char* {
+    constexpr int b = decltype(b_c)::value & 3;
+    if constexpr (b == 0) return (lds_char*)b0;
+    else if constexpr (b == 1) return (lds_char*)b1;
+    else if constexpr (b == 2) return (lds_char*)b2;
+    else return (lds_char*)b3;
   };
-  auto settle = [&]() { asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-
-  // ---- operand reads: entry 128 wr + 32 m + l32, row l32 of weight part t; step (h, j): columns 16 (2 j + hh) + 8 h .. + 7 of
-  // either
-  const lds_char* s3 = (const lds_char*)smem;
-  uint32_t xa[4], wa;
+  auto weights = [&](int kq, int i, int t) {
+    return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(ws[t], wo + (i >> 1) * 1024 + (i & 1) * 512,
+                                                                            min(kq, KQ - 1) * 2048, 0));
+  };
+  // ---- operand reads: entry 32 m + l32, columns 16 (2 j + hh) + 8 h .. + 7 of step (h, j) = (i / 2, i % 2)
+  uint32_t xa[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int h = i >> 1, j = i & 1;
-    xa[i] = (uint32_t)((128 * wr + l32) * 128 + 16 * ((4 * j + 2 * hh + h) ^ ((l32 >> 1) & 7)));
+    xa[i] = (uint32_t)(l32 * 128 + 16 * ((4 * j + 2 * hh + h) ^ ((l32 >> 1) & 7)));
   }
-  wa = (uint32_t)(TM * 128 + ((GLU ? 1 : 2) * NP * wc + (l32 >> 4)) * 2048 + hh * 256 + (l32 & 15) * 16);
-  f32x16 acc[NP][4];  // [weight part][entries]; GLU: the first half gate, the others up
-#pragma unroll
-  for (int t = 0; t < NP; ++t)
-#pragma unroll
-    for (int m = 0; m < 4; ++m)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[t][m][r] = 0.f;
+  auto rows = [&](auto b_c, int i, int m) { return *reinterpret_cast<const lds_bf16x8*>(buffer(b_c) + xa[i] + m * 4096); };
 
-  auto all = [&](int kq, auto buf_c, auto from, auto to, auto&& self) {
-    if constexpr (decltype(from)::value < decltype(to)::value) {
-      move(kq, buf_c, from);
-      self(kq, buf_c, Int<decltype(from)::value + 1>{}, to, self);
-    }
-  };
-  all(0, Int<0>{}, Int<0>{}, Int<2 * XP>{}, all);
-  settle();
-  if (KQ > 1) all(1, Int<1>{}, Int<0>{}, Int<XP>{}, all);
-  // MT: 32-entry tiles that this wave has (every wave passes the same barriers)
+  // MT: 32-entry tiles
   auto sweep = [&](auto mt_c) {
     constexpr int MT = decltype(mt_c)::value;
-    bf16x8 w0[NP], x0[4], w1[NP], x1[4];
-    auto read_w = [&](int i, int t, auto buf_c) {
-      const int tile = GLU ? (t % (NP / 2)) * 2 + t / (NP / 2) * 8 : 2 * t;
-      return *reinterpret_cast<const lds_bf16x8*>(
-          s3 + wa + (decltype(buf_c)::value * BIG_BUF + tile * 2048 + (i >> 1) * 1024 + (i & 1) * 512));
-    };
-    auto read_x = [&](int i, int m, auto buf_c) {
-      return *reinterpret_cast<const lds_bf16x8*>(s3 + xa[i] + (decltype(buf_c)::value * BIG_BUF + m * 4096));
-    };
-    // four columns steps of 16, in quarters; the next one's operands are read and pieces of a later step are
-    // moved between the quarters (a run of transfers would hold the wave, and with it its products, until they are taken)
-    auto part = [&](int kq, auto buf_c, auto i_c) {
-      constexpr int buf = decltype(buf_c)::value, i = decltype(i_c)::value, ni = (i + 1) & 3;
-      const bool more = i < 3 || kq + 1 < KQ;
-      if (i == 3 && more) settle();  // the next step has come, and nobody reads this one any more
-      auto quarter = [&](auto q_c) {
-        constexpr int q = decltype(q_c)::value;
-        if constexpr (MT > 0) {
-          if (more) {
-            using Next = Int<i == 3 ? buf ^ 1 : buf>;
-            if constexpr (q < 2) {
+    f32x16 acc[2][MT];
 #pragma unroll
-              for (int t = q * NP / 2; t < (q + 1) * NP / 2; ++t) w1[t] = read_w(ni, t, Next{});
-              if (q < MT) x1[q] = read_x(ni, q, Next{});
-            } else if constexpr (q == 2) {
-              if (2 < MT) x1[2] = read_x(ni, 2, Next{});
-              if (3 < MT) x1[3] = read_x(ni, 3, Next{});
-            }
-          }
-        }
-        constexpr int some = XP / 4;  // pieces per quarter
-        if constexpr (i == 3) {
-          if (kq + 2 < KQ) all(kq + 2, buf_c, Int<some * q>{}, Int<some * (q + 1)>{}, all);
-        } else if constexpr (i == 0) {
-          if (kq + 1 < KQ) all(kq + 1, Int<buf ^ 1>{}, Int<XP + some * q>{}, Int<XP + some * (q + 1)>{}, all);
-        }
-        __builtin_amdgcn_sched_barrier(0x6);
-        if constexpr (q < MT) {
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int t = 0; t < NP; ++t) acc[t][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w0[t], x0[q], acc[t][q], 0, 0, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0x6);
-      };
-      quarter(Int<0>{});
-      quarter(Int<1>{});
-      quarter(Int<2>{});
-      quarter(Int<3>{});
+      for (int m = 0; m < MT; ++m)
 #pragma unroll
-      for (int t = 0; t < NP; ++t) w0[t] = w1[t];
+        for (int r = 0; r < 16; ++r) acc[t][m][r] = 0.f;
+    // ---- rows on their way: MT pieces of 8 rows of 128 bytes per wave (16 bytes p of row r: columns 8 (p ^ (r / 2 % 8)) .. + 7)
+    const int mine = 8 * MT * wid, entry = a.order[pl.first + min(mine + lane, left - 1)];
+    uint32_t xo[MT];
 #pragma unroll
-      for (int m = 0; m < 4; ++m) x0[m] = x1[m];
-    };
-    if constexpr (MT > 0) {
-#pragma unroll
-      for (int t = 0; t < NP; ++t) w0[t] = read_w(0, t, Int<0>{});
-#pragma unroll
-      for (int m = 0; m < MT; ++m) x0[m] = read_x(0, m, Int<0>{});
+    for (int i = 0; i < MT; ++i) {
+      const int r = i * 8 + (lane >> 3);
+      xo[i] = ((uint32_t)__shfl(entry / a.div, r, 64) * K + 8 * ((lane & 7) ^ (((mine + r) >> 1) & 7))) * 2;
     }
-    auto step = [&](int kq, auto buf_c) {
-      part(kq, buf_c, Int<0>{});
-      part(kq, buf_c, Int<1>{});
-      part(kq, buf_c, Int<2>{});
-      part(kq, buf_c, Int<3>{});
+    if (lane < 8 * MT) ents[mine + lane] = entry;
+    // those of step kq that part p issues; past the end the last step again, into a buffer that nobody reads
+    auto move = [&](int kq, auto b_c, int p, int only) {
+#pragma unroll
+      for (int i = p * MT / 4; i < (p + 1) * MT / 4; ++i)
+        if (only < 0 || only == i - p * MT / 4)
+          dma16(xs, xo[i], min(kq, KQ - 1) * 128, buffer(b_c) + 128 * mine + 1024 * i);
     };
-    for (int kq = 0; kq < KQ; kq += 2) {
+    bf16x8 w[2][4][2], x[2][MT];
+    // (in the order of the loop, which waits by it)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) move(0, Int<0>{}, i, -1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) move(1, Int<1>{}, i, -1);
+#pragma unroll
+    for (int i = 0; i < 7; ++i) {
+      if (i >= 3) move(2, Int<2>{}, i - 3, -1);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) w[i >> 2][i & 3][t] = weights(i >> 2, i & 3, t);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    meet<2 * MT + 14>();
+#pragma unroll
+    for (int m = 0; m < MT; ++m) x[0][m] = rows(Int<0>{}, 0, m);
+    auto part = [&](int kq, auto s_c, auto i_c) {
+      constexpr int s = decltype(s_c)::value, i = decltype(i_c)::value, ni = (i + 1) & 3;
+      using Next = Int<i == 3 ? s + 1 : s>;
+      if constexpr (i == 3) {  // the next step has come, and nobody reads the one before this any more
+        meet<MT + 14 + 3 * MT / 4>();
+      }
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        x[(i + 1) & 1][m] = rows(Next{}, ni, m);
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+          if (l * MT / 4 != m) continue;
+          if (l < 2) move(kq + 3, Int<s + 3>{}, i, l);
+          else if (i == 0) w[(s & 1) ^ 1][3][l - 2] = weights(kq + 1, 3, l - 2);
+          else w[s & 1][i ? i - 1 : 0][l - 2] = weights(kq + 2, i - 1, l - 2);
+        }
+        __builtin_amdgcn_sched_barrier(0x6);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          acc[t][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[s & 1][i][t], x[i & 1][m], acc[t][m], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0x6);
+      }
+    };
+    auto step = [&](int kq, auto s_c) {
+      part(kq, s_c, Int<0>{});
+      part(kq, s_c, Int<1>{});
+      part(kq, s_c, Int<2>{});
+      part(kq, s_c, Int<3>{});
+    };
+    int kq = 0;
+    for (; kq + 4 <= KQ; kq += 4) {
       step(kq, Int<0>{});
-      if (kq + 1 < KQ) step(kq + 1, Int<1>{});
+      step(kq + 1, Int<1>{});
+      step(kq + 2, Int<2>{});
+      step(kq + 3, Int<3>{});
     }
-  };
-  const int tiles = min(max((left - 128 * wr + 31) / 32, 0), 4);
-  if (tiles == 4) sweep(Int<4>{});
-  else if (tiles == 3) sweep(Int<3>{});
-  else if (tiles == 2) sweep(Int<2>{});
-  else if (tiles == 1) sweep(Int<1>{});
-  else sweep(Int<0>{});
-  // lane: entry l32 of a tile, weight rows 8 q + 4 hh + 0..3
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const int r = 128 * wr + 32 * m + l32;
-    if (r >= left) continue;
-    bf16* yr = (bf16*)a.y + (int64_t)ents[r] * N;
-#pragma unroll
-    for (int t = 0; t < (GLU ? NP / 2 : NP); ++t) {
-      const int n = n0 + (GLU ? 16 : 32) * NP * wc + 32 * t;
-      if (n >= N) continue;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        bf16x4 o;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          o[i] = (bf16)(GLU ? silu_mul(acc[t][m][4 * q + i], acc[t + (GLU ? NP / 2 : 0)][m][4 * q + i]) : plain_act(acc[t][m][4 * q + i], a.act));
-        *reinterpret_cast<bf16x4*>(yr + n + 8 * q + 4 * hh) = o;
+    if (kq < KQ) {
+      step(kq, Int<0>{});
+      if (kq + 1 < KQ) {
+        step(kq + 1, Int<1>{});
+        if (kq + 2 < KQ) step(kq + 2, Int<2>{});
       }
     }
-  }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // lane: entry l of a tile, weight rows 8 q + 4 h + 0..3 (found anew: held over the loop they are spilled)
+    const int l = __lane_id() & 31, h = __lane_id() >> 5;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const int r = 32 * m + l;
+      if (r >= left) continue;
+      bf16* yr = (bf16*)a.y + (int64_t)ents[r] * N;
+#pragma unroll
+      for (int t = 0; t < (GLU ? 1 : 2); ++t) {
+        const int n = n0 + (GLU ? 32 : 64) * wid + 32 * t;
+        if (n >= N) continue;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          bf16x4 o;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            o[i] = (bf16)(GLU ? silu_mul_fast(acc[0][m][4 * q + i], acc[1][m][4 * q + i]) : plain_act(acc[t][m][4 * q + i], a.act));
+          *reinterpret_cast<bf16x4*>(yr + n + 8 * q + 4 * h) = o;
+        }
+      }
+    }
+  };
+  const int tiles = (left + 63) / 64;
+  if (tiles == 4) sweep(Int<8>{});
+  else if (tiles == 3) sweep(Int<6>{});
+  else if (tiles == 2) sweep(Int<4>{});
+  else sweep(Int<2>{});
 }
 
 template <typename T, bool GLU>
@@ -621,27 +607,19 @@ __global__ void __launch_bounds__(256) expert_sum_kernel(const T* __restrict__ y
   }
 }
 
-// Rows per expert on average from which 256-row tiles pay. Measured against the tile kernel, us, gated / plain: 32 experts of 3584
-// by 4096, 96 rows 387 -> 429 / 187 -> 211, 128 rows 583 -> 452 / 295 -> 225, 256 rows 783 -> 645 / 392 -> 317; 32 of 1408 by 2048,
-// 96 rows 82 -> 108 / 46 -> 36, 128 rows 129 -> 109 / 55 -> 38; 8 of 3584 by 4096, 128 rows 151 -> 111 / 90 -> 82. The
-// host knows the average alone. What is far from it costs up to 300 rows (an eighth of 32 experts of 3584 by 4096 with 83 % of the
-// rows, 192 on average 581 -> 639 / 297 -> 338, 512 1140 -> 1087 / 590 -> 558), and so does exactly 128 rows each where they fill the
-// smaller tiles and the chip (32 of 3584 by 4096 373 -> 448 / 186 -> 219; 8 of them 141 -> 114 / 100 -> 68); routed at random, 128 to
-// 1024 rows gain 1.04 to 1.5, but where the second round of workgroups is a short one (256 rows, 32 of 1408 by 2048 141 -> 157 / 69 ->
-// 92). A choice on the device, one large tile or two small ones per workgroup, lost more than it saved: two small ones behind one
-// barrier take 1.25 times as long as in two workgroups.
-constexpr int BIG_ROWS = 128, BIG_WAVES = 8;
+// Rows per expert on average from which 256-row tiles pay. Measured against the tile kernel, gated / plain, times as fast: 32 experts of 3584 by
+// 4096, 96 rows 0.97 / 0.98, 128 rows 1.25 / 1.39, 256 rows 1.21 / 1.31; 32 of 1408 by 2048, 96 rows 0.88 / 1.28, 128 rows 0.90 / 1.45, 192
+// rows 1.11 / 1.16; 8 of 3584 by 4096, 128 rows 1.55 / 1.67. The host knows the average alone. What is far from it costs up to 256 rows (an
+// eighth of 32 experts of 3584 by 4096 with 83 % of the rows: 128 on average 1.08 / 0.92, 192 0.93 / 0.96, 320 1.16 / 1.08), and so does
+// exactly 128 rows each where they fill the smaller tiles and the chip (32 of 3584 by 4096 0.98 / 0.96, of 1408 by 2048 0.88 / 1.24). A
+// choice on the device, one large tile or two small ones per workgroup, lost more than it saved: two small ones behind one barrier take
+// 1.25 times as long as in two workgroups.
+constexpr int BIG_ROWS = 128;
 
 template <bool GLU>
 int launch_big(const ExpertArgs& a, int per, hipStream_t st) {  // per: columns of a tile
-  static bool attr = false;
-  if (!attr) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_big_kernel<GLU, BIG_WAVES>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              BIG_LDS);
-    attr = true;
-  }
   const int64_t grid = ((int64_t)a.entries / TM + a.E) * ((a.N + per - 1) / per);
-  hipLaunchKernelGGL((expert_big_kernel<GLU, BIG_WAVES>), dim3((unsigned)grid), dim3(BIG_WAVES * 64), BIG_LDS, st, a);
+  hipLaunchKernelGGL((expert_big_kernel<GLU>), dim3((unsigned)grid), dim3(256), 0, st, a);
   DS_CHECK_LAUNCH();
   return 0;
 }
@@ -662,12 +640,13 @@ extern "C" int ds_expert_gemm(const void* x, const void* w, void* y, const int* 
     return (int)hipErrorInvalidValue;
   const bool lists = offs != nullptr, gated = act == SILU_GLU;
   if (operand && (dtype != DS_BF16 || !ds_expert_order_ok(N, K) || (!lists && entries > FEW))) return (int)hipErrorInvalidValue;
-  const ExpertArgs a{x, w, y, experts, offs, order, entries, E, N, K, div, act};
+  const int64_t xbytes = ((int64_t)(entries - 1) / div + 1) * K * 2;
+  const ExpertArgs a{x, w, y, experts, offs, order, entries, E, N, K, div, act, xbytes <= UINT32_MAX ? (uint32_t)xbytes : 0};
   if (operand && lists && tile) {
     const int per = gated ? BN / 2 : BN;
     const int64_t grid = ((int64_t)entries / BM + E) * ((N + per - 1) / per);
     if (grid > INT32_MAX) return (int)hipErrorInvalidValue;
-    if (entries >= (int64_t)BIG_ROWS * E) return gated ? launch_big<true>(a, per, st) : launch_big<false>(a, per, st);
+    if (entries >= (int64_t)BIG_ROWS * E && a.xbytes) return gated ? launch_big<true>(a, per, st) : launch_big<false>(a, per, st);
     if (gated) hipLaunchKernelGGL(expert_tile_kernel<true>, dim3((unsigned)grid), dim3(256), 0, st, a);
     else hipLaunchKernelGGL(expert_tile_kernel<false>, dim3((unsigned)grid), dim3(256), 0, st, a);
     DS_CHECK_LAUNCH();

@@ -208,6 +208,52 @@ def test_big_tiles_at_their_edges(N, K, act):
     assert ((y.float() - z).norm() / z.norm()).item() < 3e-3
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["silu_glu", "none"])
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 384, 448, 512, 832])
+def test_big_tiles_over_steps(K, act):
+    """256 x 256 tiles: every remainder of the four buffers, fewer steps than buffers and several rounds of them, for every number of
+    64-row units; the same bits each time. Gates far out on both sides: silu goes to 0 and to the gate itself."""
+    from deepspeedsyclsupport_amd.ops.expert_ops import ACTS, expert_ops, operand_order
+    N, counts = 96, [64, 128, 192, 256, 300, 1, 65]
+    g = torch.Generator(device="cuda").manual_seed(K)
+    E, n, parts = len(counts), sum(counts), 2 if act == "silu_glu" else 1
+    assert n >= 128 * E
+    w = (torch.randn(E, parts * N, K, device="cuda", generator=g) * K**-0.5).bfloat16()
+    x = torch.randn(n, K, device="cuda", generator=g).bfloat16()
+    x[:8] *= 64.0
+    experts = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    order = torch.randperm(n, generator=torch.Generator().manual_seed(2))
+    experts[order.clone()] = experts.clone()
+    order, offs = torch.argsort(experts, stable=True).int().cuda(), torch.tensor([0, *counts]).cumsum(0).int().cuda()
+    run = lambda: expert_ops().expert_gemm(x, operand_order(w), experts.int().cuda(), offs, order, 1, ACTS[act], True, True)  # noqa: E731
+    y = run()
+    z = (w.double()[experts.cuda()] @ x.double()[:, :, None]).squeeze(-1)
+    if act == "silu_glu":
+        z = z[:, :N] * torch.sigmoid(z[:, :N]) * z[:, N:]
+    # one rounding to bf16 (2^-9 of the value); sums of K products in fp32, each off by at most K 2^-24 of the sum of magnitudes (of order
+    # sqrt K times the value's scale, 64 in the first rows): far below 1e-4 of that scale
+    scale = z.abs().amax(-1, keepdim=True)
+    assert ((y.double() - z).abs() <= z.abs() * 2**-8 + 1e-4 * scale).all()
+    for _ in range(3):
+        assert torch.equal(run(), y)
+
+
+@pytest.mark.gpu
+def test_big_tiles_leave_long_inputs():
+    """Rows that 32 bits of bytes do not reach go by the tile kernel."""
+    from deepspeedsyclsupport_amd.ops.expert_ops import expert_ops, operand_order
+    N, K, n = 32, 8192, (1 << 18) + 96    # 4 GiB and a little
+    w = (torch.randn(1, N, K, device="cuda") * K**-0.5).bfloat16()
+    x = torch.zeros(n, K, device="cuda", dtype=torch.bfloat16)
+    rows = torch.tensor([0, 1, (1 << 18) - 1, 1 << 18, n - 1], device="cuda")
+    x[rows] = torch.randn(len(rows), K, device="cuda").bfloat16()
+    order, offs = torch.arange(n, dtype=torch.int32, device="cuda"), torch.tensor([0, n], dtype=torch.int32, device="cuda")
+    y = expert_ops().expert_gemm(x, operand_order(w), torch.zeros(n, dtype=torch.int32, device="cuda"), offs, order, 1, 0, True, True)
+    torch.testing.assert_close(y[rows].float(), x[rows].float() @ w[0].float().t(), rtol=2**-7, atol=1e-3)
+    assert y.ne(0).any(-1).sum() == len(rows)
+
+
 @pytest.mark.parametrize("device", [pytest.param("cpu"), pytest.param("cuda", marks=GPU)])
 def test_rope_table(device):
     """Angles of far positions, fp32 to the last digits."""
