@@ -6,12 +6,15 @@ operands are MN-major, a layout the library GEMMs run at ~1.0-1.1 PF/s on MI355X
 So for long token dimensions the backward first streams dY and X through the HBM-speed transpose kernel
 (`csrc/act/transpose.hip`) and then issues the K-major GEMM. The function also saves the Parameter (not a view of
 it), so under ZeRO-3 a released gathered weight is not kept alive by autograd (reference
-`runtime/zero/linear.py:43` LinearFunctionForZeroStage3).
+`runtime/zero/linear.py:43` LinearFunctionForZeroStage3). Short token dimensions take the products of
+`csrc/gemm/narrow_gemm.hip`.
 """
 import os
 
 import torch
 import torch.nn.functional as F
+
+from .native import hip_ops
 
 KMAJOR_MIN_ROWS = int(os.environ.get("DS_WGRAD_KMAJOR_MIN_ROWS", "8192"))
 _ENABLED = os.environ.get("DS_WGRAD_KMAJOR", "1") != "0"
@@ -44,9 +47,25 @@ def _kmajor_of(t2d, given, Tp):
     if given is not None and given.shape == (t2d.shape[1], Tp) and given.dtype == t2d.dtype:
         STATS["kmajor_from_producer"] += 1
         return given
-    from .native import hip_ops
     STATS["kmajor_transposed"] += 1
     return hip_ops().transpose16(_rows16(t2d), Tp)
+
+
+# (no public predicate says that a torch function mode is on)
+_function_modes = torch._C._len_torch_function_stack
+
+
+def _narrow(a, b):
+    """Whether a product may go to the extension, which takes the short ones and gives torch the others and all that a transform,
+    dispatch mode, tracer or autocast has to see. Function modes and the compiler see calls from Python alone."""
+    return a.is_cuda and b.is_cuda and not _function_modes() and not torch.compiler.is_compiling()
+
+
+def plain_linear(x, weight, bias=None):
+    """x W^T + b without a gradient of its own: the narrow products where they pay, else torch's."""
+    if bias is None and _narrow(x, weight):
+        return hip_ops().linear(x, weight)
+    return F.linear(x, weight, bias)
 
 
 def weight_grad(go2d, x2d, go_kmajor=None, x_kmajor=None):
@@ -61,6 +80,8 @@ def weight_grad(go2d, x2d, go_kmajor=None, x_kmajor=None):
             STATS["kmajor_from_producer"] += 1
         xt = x_kmajor if x2d is None else _kmajor_of(x2d, x_kmajor, Tp)          # [in, Tp]
         return torch.mm(got, xt.t())
+    if _narrow(go2d, x2d):
+        return hip_ops().linear_weight_grad(go2d, x2d)
     return go2d.t().mm(x2d)
 
 
@@ -69,9 +90,10 @@ def input_grad(go2d, weight):
     a K-major copy W^T [in, out] (one HBM-speed transpose of the weight, ~0.04 ms for a 7B layer's QKV) turns the
     product into the TN layout of the forward GEMMs."""
     if _DGRAD_ENABLED and _kmajor_ok(go2d, weight) and weight.dim() == 2 and weight.stride(1) == 1:
-        from .native import hip_ops
         wt = hip_ops().transpose16(_rows16(weight))   # [in, out]
         return torch.mm(go2d, wt.t())
+    if _narrow(go2d, weight):
+        return hip_ops().linear_input_grad(go2d, weight)
     return go2d.mm(weight)
 
 
@@ -87,7 +109,7 @@ class LinearFunction(torch.autograd.Function):
         else:
             ctx.save_for_backward(x, weight, bias)
             ctx.kmajor_saved = False
-        return F.linear(x, weight, bias)
+        return plain_linear(x, weight, bias)
 
     @staticmethod
     def backward(ctx, go):

@@ -38,6 +38,7 @@ EXTENSIONS = {
             "act/act_kernels.hip",
             "act/dropout_kernels.hip",
             "act/transpose.hip",
+            "gemm/narrow_gemm.hip",
             "rope/rope_kernels.hip",
             "xent/xent_kernels.hip",
             "attn/decode_attn.hip",

@@ -1,0 +1,116 @@
+"""Products around a short batch of tokens (`csrc/gemm/narrow_gemm.hip`) and the linear layer that takes them."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from deepspeedsyclsupport_amd.ops.linear import LinearFunction, plain_linear
+from deepspeedsyclsupport_amd.ops.native import hip_ops
+
+GPU = pytest.mark.gpu
+
+
+def _rnd(*shape, seed=0):
+    return torch.randn(*shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(seed)).bfloat16()
+
+
+def _check(got, a, b):
+    """One rounding to bf16 (2^-9 of the value) and sums of K products in fp32, off by less than K 2^-23 of the magnitudes' sum."""
+    a, b = a.double(), b.double()
+    want, size = a @ b.t(), a.abs() @ b.abs().t()
+    assert got.shape == want.shape
+    assert ((got.double() - want).abs() <= want.abs() * 2**-8 + size * a.shape[1] * 2**-23).all()
+
+
+@GPU
+@pytest.mark.parametrize("tile,parts", [(0, 0), (32, 1), (32, 3), (64, 1), (64, 2)])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (8, 40, 64), (31, 64, 128), (33, 72, 192), (64, 136, 256), (72, 200, 320), (128, 96, 448),
+                                   (127, 264, 576), (136, 1032, 1088)])
+def test_products_at_their_edges(M, N, K, tile, parts):
+    """Both forms of both operands; tiles that rows, columns or the inner dimension do not fill; fewer steps than buffers, and every
+    remainder of them; operands that are columns of wider matrices; the same bits each time."""
+    ops = hip_ops()
+    a, b = _rnd(M, K, seed=1), _rnd(N, K, seed=2)
+    wide_a, wide_b = _rnd(M, K + 24, seed=3), _rnd(K, N + 16, seed=4)
+    ops.narrow_gemm_tune(tile, parts)
+    try:
+        got = ops.narrow_gemm(a, b, True, True)
+        _check(got, a, b)
+        assert torch.equal(got, ops.narrow_gemm(a, b, True, True))
+        _check(ops.narrow_gemm(a, b.t().contiguous(), True, False), a, b)
+        _check(ops.narrow_gemm(wide_a[:, 8:8 + K], wide_b[:, 8:8 + N], True, False), wide_a[:, 8:8 + K], wide_b[:, 8:8 + N].t())
+        if M % 8 == 0:
+            at = a.t().contiguous()
+            _check(ops.narrow_gemm(at, b, False, True), a, b)
+            for rows in (K, K - 1, K - 37, 1):   # (an inner dimension of any length)
+                _check(ops.narrow_gemm(at[:rows], b.t().contiguous()[:rows], False, False), a[:, :rows], b[:, :rows])
+    finally:
+        ops.narrow_gemm_tune(0, 0)
+
+
+@GPU
+def test_values_that_do_not_mix():
+    """Infinities and NaN stay in their rows; nothing from past the end of an operand comes in."""
+    a, b = _rnd(40, 128), _rnd(48, 128, seed=1)
+    a[3, 5], a[4, 7] = float("inf"), float("nan")
+    y = hip_ops().narrow_gemm(a, b, True, True)
+    keep = [i for i in range(40) if i not in (3, 4)]
+    _check(y[keep], a[keep], b)
+    assert not y[3].isfinite().any() and y[4].isnan().all()
+    big = _rnd(64, 256)
+    big[40:] = float("nan")
+    _check(hip_ops().narrow_gemm(big[:40, :128].contiguous(), b, True, True), big[:40, :128], b)
+    _check(hip_ops().narrow_gemm(big[:37, :40], big[:37, 40:104], False, False), big[:37, :40].t(), big[:37, 40:104].t())
+
+
+@GPU
+@pytest.mark.parametrize("lead", [(2, 33), (128, )])
+def test_linear_layer(lead):
+    """What differentiates, transforms, counts or casts torch's linear does so here; the products are the narrow ones."""
+    I, O = 128, 192
+    x, w = _rnd(*lead, I).requires_grad_(), _rnd(O, I, seed=1).requires_grad_()
+    go = _rnd(*lead, O, seed=2)
+    y = LinearFunction.apply(x, w, None, None)
+    gx, gw = torch.autograd.grad(y, (x, w), go)
+    x2, go2 = x.detach().reshape(-1, I), go.reshape(-1, O)
+    assert torch.equal(y.reshape(-1, O), hip_ops().narrow_gemm(x2, w.detach(), True, True))
+    assert torch.equal(gx.reshape(-1, I), hip_ops().narrow_gemm(go2, w.detach(), True, False))
+    assert torch.equal(gw, hip_ops().narrow_gemm(go2, x2, False, False))
+    # (the gradient's gradient, and a batch of vectors through the Jacobian: torch's own products)
+    for f in (lambda a, b: LinearFunction.apply(a, b, None, None), F.linear):
+        out = f(x, w)
+        (g1, ) = torch.autograd.grad(out.float().pow(2).sum(), x, create_graph=True)
+        (g2, ) = torch.autograd.grad(g1.float().pow(2).sum(), w)
+        rows = torch.autograd.grad(f(x, w), (x, w), torch.stack([go, 2 * go]), is_grads_batched=True)
+        if f is F.linear:
+            for got, want in zip(kept, (g1, g2, *rows)):
+                torch.testing.assert_close(got.float(), want.float(), rtol=0.03, atol=0.03 * want.float().abs().max().item())
+        kept = (g1, g2, *rows)
+    from torch.utils.flop_counter import FlopCounterMode
+    with FlopCounterMode(display=False) as count:
+        LinearFunction.apply(x, w, None, None).backward(go)
+    assert count.get_total_flops() == 3 * 2 * x2.shape[0] * I * O
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert plain_linear(x.detach(), w.detach()).dtype == torch.float16
+    from torch.fx.experimental.proxy_tensor import make_fx
+    with torch.no_grad():
+        assert any("mm" in str(n.target) for n in make_fx(lambda a, b: plain_linear(a, b))(x.detach(), w.detach()).graph.nodes)
+        assert torch.equal(torch.func.vmap(plain_linear, (0, None))(x.detach()[None], w.detach())[0],
+                           torch.func.vmap(F.linear, (0, None))(x.detach()[None], w.detach())[0])
+
+
+@GPU
+def test_linear_layer_leaves_what_it_does_not_take():
+    """Other types, odd widths, unaligned and strided inputs, empty ones, long ones: torch's answer."""
+    def same(x, w):
+        assert torch.equal(plain_linear(x, w), F.linear(x, w))
+    with torch.no_grad():
+        same(_rnd(8, 64).float(), _rnd(16, 64).float())
+        same(_rnd(8, 72), _rnd(16, 72))                        # no whole steps of 64
+        same(_rnd(8, 64), _rnd(17, 64))                        # no whole pieces of columns
+        same(_rnd(64 * 8 + 1)[1:].view(8, 64), _rnd(16, 64))   # not aligned
+        same(_rnd(64, 8).t(), _rnd(16, 64))
+        same(_rnd(0, 64), _rnd(16, 64))
+        same(_rnd(64), _rnd(16, 64))
+        same(_rnd(4096, 1024), _rnd(1024, 1024))
+        x, w = _rnd(16, 64), _rnd(32, 64, seed=1)
+        torch.testing.assert_close(plain_linear(x, w).float(), F.linear(x, w).float(), rtol=2**-6, atol=2**-4)
