@@ -24,6 +24,7 @@ from ... import comm as dist
 from ...ops import reference
 from ...ops import moe_ops
 from ...ops.bf16_gemv import Bf16Weight, decode_rows_ok
+from ...ops.linear import plain_linear
 from ...ops.native import cpu_ops, hip_ops
 from ...ops.transformer import functional as DF
 
@@ -282,7 +283,7 @@ class ProjectionLayer(nn.Module):
         qw = self.quant.get(name)
         if qw is not None and qw.i8 is not None:
             return qw.i8.linear(x, bias)
-        return F.linear(x, self._w(name), bias)
+        return plain_linear(x, self._w(name), bias)
 
     def _w(self, name):
         return self.quant[name].materialize() if name in self.quant else getattr(self, name)

@@ -250,15 +250,15 @@ int g_tile = 0, g_parts = 0;
 struct Cut {
   int tm, tn, parts;  // tile, parts of K
 };
-// Tiles of 64 from 128 of them on (y of 128 tokens, us with 32 / 64: [3072, 1024] 6.4 / 6.9, [5632, 1024] 9.3 / 7.1). Operands that run across
-// the inner dimension come in rows of 64, never 32 (half a cache line: dX of 128 tokens by [3072, 1024] 14.9 for 11.3). Parts where the
+// Tiles of 64 where those of 32 are more than two a CU (y of 128 tokens, us with 32 / 64: [3072, 1024] 6.4 / 6.9, [4096, 2048] 9.1 / 10.4,
+// [5632, 1024] 9.3 / 7.1), with an operand across the inner dimension from 128 of them on. Such operands come in rows of 64, never 32 (half a cache line: dX of 128 tokens by [3072, 1024] 14.9 for 11.3). Parts where the
 // tiles leave the chip idle: a sum costs 2 us and its traffic, so both operands along K want 2560 of it each (y of 64 tokens, [2048, 5632] 12.6
 // whole, 10.5 in two; [1024, 2816] 7.7 and 7.7), while rows across it come slower (dX of 128 tokens by [5632, 1024] 42 whole, 15.8
 // in four, 13.4 in eight; of 256 by [1024, 2816] 10.2 whole, 12.4 in two).
 Cut cut_of(int64_t M, int64_t N, int64_t K, bool along) {
   auto tiles = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
   int tn = along ? 32 : 64, tm = 32;
-  if (g_tile ? g_tile == 64 : tiles(64, 64) >= 128) tm = tn = 64;
+  if (g_tile ? g_tile == 64 : along ? tiles(32, 32) > 512 : tiles(64, 64) >= 128) tm = tn = 64;
   const int64_t fill = (K >= 2048 ? 512 : 256) / tiles(tm, tn), longest = K / (along ? 2560 : 512);
   const int64_t parts = g_parts ? std::min<int64_t>(g_parts, (K + 63) / 64) : std::min<int64_t>(std::min(fill, longest), 8);
   return {tm, tn, (int)std::max<int64_t>(parts, 1)};
