@@ -65,7 +65,7 @@ int ds_flash_bwd(const void*, const void*, const void*, const void*, const void*
 int ds_transpose16(const void*, void*, int, int, int, int64_t, hipStream_t);
 int ds_narrow_gemm_ok(int64_t, int64_t, int64_t, int64_t, int64_t, int, int);
 int64_t ds_narrow_gemm_scratch(int64_t, int64_t, int64_t, int, int);
-int ds_narrow_gemm_pays(int64_t, int64_t, int64_t, int);
+int ds_narrow_gemm_pays(int64_t, int64_t, int64_t, int, int);
 int ds_narrow_gemm(const void*, const void*, void*, int64_t, int64_t, int64_t, int64_t, int64_t, int, int, void*, hipStream_t);
 void ds_narrow_gemm_tune(int, int);
 int ds_xent_fwd(const void*, const int64_t*, float*, float*, int64_t, int, int64_t, int, float, int, hipStream_t);
@@ -533,7 +533,7 @@ Tensor narrow_product(const Tensor& a, const Tensor& b, bool a_along, bool b_alo
     return Tensor();
   const int64_t M = a.size(a_along ? 0 : 1), K = a.size(a_along ? 1 : 0), N = b.size(b_along ? 0 : 1);
   const int64_t lda = a.size(0) > 1 ? a.stride(0) : a.size(1), ldb = b.size(0) > 1 ? b.stride(0) : b.size(1);
-  if (b.size(b_along ? 1 : 0) != K || !ds_narrow_gemm_ok(M, N, K, lda, ldb, a_along, b_along) || (!any && !ds_narrow_gemm_pays(M, N, K, a_along)))
+  if (b.size(b_along ? 1 : 0) != K || !ds_narrow_gemm_ok(M, N, K, lda, ldb, a_along, b_along) || (!any && !ds_narrow_gemm_pays(M, N, K, a_along, b_along)))
     return Tensor();
   const char *pa = (const char*)a.const_data_ptr(), *pb = (const char*)b.const_data_ptr();
   if ((uintptr_t)pa % 16 || (uintptr_t)pb % 16) return Tensor();

@@ -3,17 +3,17 @@
 //
 // What bounds them is latency and the count of workgroups, not the matrix cores: 128 tokens of a 1024-wide layer make 32 tiles of
 // 64 x 64. Hence
-//  * tiles of 64 x 64 (four waves of 32 x 32) or, where those are too few, of 32 rows by 32 or 64 (the waves share each step's inner
-//    dimension and meet in LDS at the end, always in the same order), and K in parts with a second launch for their sums;
+//  * tiles of 128 x 128 or 64 x 64 (four waves of 64 x 64 or 32 x 32) or, where those are too few, of 32 rows by 32 or 64 (the waves share
+//    each step's inner dimension and meet in LDS at the end, always in the same order), and K in parts with a second launch for their sums;
 //  * both operands come by DMA into four LDS buffers, three steps ahead; one barrier a step, whose wait counts what may still be on its
-//    way (buffers are arrays apart, accesses buffer instructions: see moe/expert_gemm.hip);
+//    way;
 //  * an operand whose rows run along the inner dimension is stored row by row, 128 bytes a step; one whose rows run across it (W in dX, both in
 //    dW) as it lies, and read transposed (ds_read_b64_tr_b16). Chunks are swizzled by the source address, against bank conflicts;
 //  * what lies past the end of a buffer reads as zero: ragged tokens need no other treatment, along the inner dimension neither.
 // Besides, the library's call takes the host 18 to 23 us, this one 5 to 7: a training step of 128 tokens has 27 of them and waits for the host.
 // Measured, us (the library's kernel): 128 tokens, layers [3072, 1024], [1024, 1024], [5632, 1024], [1024, 2816], head [8000, 1024]: y 6.4
-// (9.5), 4.8 (8.3), 7.1 (9.7), 7.8 (7.9), 7.3 (10.1); dX 10.8 (13.4), 8.1 (11.0), 13.4 (20.9), 9.8 (11.3), 15.3 (30); dW 6.3 (7.1), 3.3 (5.3),
-// 9.0 (9.3), 5.7 (7.1), 11.6 (10.1).
+// (9.4), 4.5 (8.2), 6.7 (9.8), 6.9 (7.9), 7.0 (10.1); dX 8.4 (13.4), 5.2 (11.0), 9.9 (21.1), 5.6 (11.3), 11.9 (30.9); dW 6.2 (7.2), 3.3 (5.3),
+// 10.4 (9.3), 5.6 (7.4), 11.0 (10.1). 512 tokens, [3072, 1024]: 9.4 (10.6), 11.0 (16.1), 9.6 (11.9).
 #include "ds_hip.h"
 
 #include <algorithm>
@@ -40,11 +40,21 @@ struct NarrowArgs {
   f32x4* part;             // their sums [parts][M][N] (null: the result leaves from here)
 };
 
-// 16 bytes per lane to LDS bytes dst + 16 lane. (The host's pass does not know the size.)
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t from, uint32_t lane_bytes, lds_char* dst) {
-#ifdef __HIP_DEVICE_COMPILE__
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void*)dst, 16, lane_bytes, 0, 0, 0);
-#endif
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+// A buffer of `bytes` bytes: what lies past its end reads as zero
+__device__ __forceinline__ i32x4 buffer_of(const void* p, uint32_t bytes) {
+  const uint64_t at = (uint64_t)p;
+  return i32x4{__builtin_amdgcn_readfirstlane((int)at), __builtin_amdgcn_readfirstlane((int)(at >> 32)), __builtin_amdgcn_readfirstlane((int)bytes),
+               0x00020000};
+}
+// 16 bytes per lane to LDS bytes dst + 16 lane. Inline asm: hipcc waits for all of its own such loads before a transposed read.
+__device__ __forceinline__ void dma16(i32x4 from, uint32_t lane_bytes, uint32_t dst) {
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "s"(dst), "v"(lane_bytes), "s"(from)
+               : "memory");
 }
 
 // All of this wave's LDS accesses and all but its NEWER latest loads are done, then those of all waves.
@@ -59,12 +69,12 @@ __device__ __forceinline__ void meet() {
 template <bool ALONG, int R>
 struct Operand {
   static constexpr int BYTES = R * 128, PIECES = R / 32;  // LDS bytes a step, transfers of 1 KB a wave
-  __amdgpu_buffer_rsrc_t from;
+  i32x4 from;
   uint32_t src[PIECES], step;  // per lane: bytes of step 0; bytes from a step to the next
   int dst;
 
   __device__ __forceinline__ void init(const bf16* p, uint32_t bytes, uint32_t ld, int r0, int lane, int wid) {
-    from = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(p), 0, (int)bytes, 0x00020000);
+    from = buffer_of(p, bytes);
     step = ALONG ? 128 : 128 * ld;
     dst = wid * PIECES * 1024;
 #pragma unroll
@@ -73,14 +83,16 @@ struct Operand {
       if constexpr (ALONG) {  // 8 rows of 8 chunks: chunk c of row r at c ^ (r / 2 % 8)
         const int r = 8 * piece + (lane >> 3);
         src[i] = (uint32_t)(r0 + r) * ld * 2 + 16 * ((lane & 7) ^ ((r >> 1) & 7));
-      } else {  // R / 8 chunks of a step's 64 / PIECES / 4 rows each; of 64 columns chunk c of row r at c ^ (4 (r / 2 % 2))
+      } else {  // R / 8 chunks of a step's 64 / PIECES / 4 rows each, those of row r swizzled by `turn`
         constexpr int CH = R / 8;
         const int r = (64 / CH) * piece + lane / CH, c = lane % CH;
-        src[i] = (uint32_t)r * ld * 2 + 2 * r0 + 16 * (CH == 8 ? c ^ (((r >> 1) & 1) << 2) : c);
+        src[i] = (uint32_t)r * ld * 2 + 2 * r0 + 16 * (c ^ turn(r));
       }
     }
   }
-  __device__ __forceinline__ void move(int kq, lds_char* buf) const {
+  // A transposed read takes 64 bytes of eight rows in two goes: rows of 256 bytes, or pairs of rows of 128, that meet in a bank are apart
+  static __device__ __forceinline__ int turn(int r) { return R == 128 ? (r & 3) << 2 : R == 64 ? ((r >> 1) & 1) << 2 : 0; }
+  __device__ __forceinline__ void move(int kq, uint32_t buf) const {
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) dma16(from, src[i] + (uint32_t)kq * step, buf + dst + 1024 * i);
   }
@@ -97,8 +109,7 @@ struct Operand {
       return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     } else {
       const int gq = (lane >> 2) & 3, row = 16 * j + 4 * h + gq;
-      int c = r0 / 8 + ((lane >> 4) & 1) * 2 + ((lane >> 1) & 1);
-      if constexpr (R == 64) c ^= ((gq >> 1) & 1) << 2;
+      const int c = (r0 / 8 + ((lane >> 4) & 1) * 2 + ((lane >> 1) & 1)) ^ turn(gq);
       const lds_char* at = buf + row * (2 * R) + 16 * c + 8 * (lane & 1);
       s16x8 v;
 #ifdef __HIP_DEVICE_COMPILE__
@@ -119,15 +130,16 @@ __device__ __forceinline__ bf16x4 narrowed(f32x4 v) {
 
 // AK, BK: the operand's rows run along the inner dimension. TM x TN: tile of C. U: steps of 64 a buffer holds.
 template <bool AK, bool BK, int TM, int TN, int U>
-__global__ void __launch_bounds__(256, 2) narrow_gemm_kernel(NarrowArgs a) {
+__global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(NarrowArgs a) {
   typedef Operand<AK, TM> A;
   typedef Operand<BK, TN> B;
   constexpr int STEP = A::BYTES + B::BYTES, BUF = STEP * U;
-  constexpr int WM = TM / 32, WN = TN / 32, WK = 4 / (WM * WN), SLICES = 4 / WK;  // waves over rows, columns, slices of 16 of a step
+  constexpr int WM = TM > 32 ? 2 : 1, WN = TN > 32 ? 2 : 1, WK = 4 / (WM * WN), SLICES = 4 / WK;  // waves over rows, columns, slices of 16
+  constexpr int MR = TM / 32 / WM, NR = TN / 32 / WN;                                            // pieces of 32 x 32 of a wave
   constexpr bool PLAIN = AK && BK;
-  __shared__ __attribute__((aligned(16))) char b0[BUF], b1[BUF], b2[BUF], b3[BUF];
+  __shared__ __attribute__((aligned(16))) char lds[4 * BUF];
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wid % WM * 32, wn = wid / WM % WN * 32, wk = wid / (WM * WN);
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wid % WM * 32 * MR, wn = wid / WM % WN * 32 * NR, wk = wid / (WM * WN);
   const int mt = (a.M + TM - 1) / TM, id = xcd_remap(blockIdx.x, gridDim.x), m0 = id % mt * TM, n0 = id / mt * TN;
   const int all = (a.K + 63) / 64, first = (int)((int64_t)all * blockIdx.y / a.parts);  // steps of 64: of K, and of this part
   const int steps = (int)((int64_t)all * (blockIdx.y + 1) / a.parts) - first, rounds = (steps + U - 1) / U;
@@ -135,38 +147,43 @@ __global__ void __launch_bounds__(256, 2) narrow_gemm_kernel(NarrowArgs a) {
   B ob;
   oa.init(a.a, a.abytes, a.lda, m0, lane, wid);
   ob.init(a.b, a.bbytes, a.ldb, n0, lane, wid);
-  auto buffer = [&](auto b_c) -> lds_char* {
-    constexpr int b = decltype(b_c)::value & 3;
-    if constexpr (b == 0) return (lds_char*)b0;
-    else if constexpr (b == 1) return (lds_char*)b1;
-    else if constexpr (b == 2) return (lds_char*)b2;
-    else return (lds_char*)b3;
-  };
+  auto buffer = [&](auto b_c) -> lds_char* { return (lds_char*)lds + (decltype(b_c)::value & 3) * BUF; };
   // round r; past the end the last step again, into a place that nobody reads
   auto move = [&](int r, auto b_c) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int kq = first + min(r * U + u, steps - 1);
-      oa.move(kq, buffer(b_c) + STEP * u);
-      ob.move(kq, buffer(b_c) + STEP * u + A::BYTES);
+      const uint32_t to = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)buffer(b_c) + STEP * u);
+      oa.move(kq, to);
+      ob.move(kq, to + A::BYTES);
     }
   };
-  f32x16 acc;
+  f32x16 acc[MR][NR];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  for (int m = 0; m < MR; ++m)
+#pragma unroll
+    for (int n = 0; n < NR; ++n)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[m][n][i] = 0.f;
   auto products = [&](int r, auto b_c) {
     const lds_char* buf = buffer(b_c);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (u && r * U + u >= steps) break;
-      bf16x8 x[SLICES], w[SLICES];
+      bf16x8 x[SLICES][MR], w[SLICES][NR];
 #pragma unroll
       for (int j = 0; j < SLICES; ++j) {
-        w[j] = ob.template read<PLAIN>(buf + STEP * u + A::BYTES, wk * SLICES + j, wn, lane);
-        x[j] = oa.template read<PLAIN>(buf + STEP * u, wk * SLICES + j, wm, lane);
+#pragma unroll
+        for (int n = 0; n < NR; ++n) w[j][n] = ob.template read<PLAIN>(buf + STEP * u + A::BYTES, wk * SLICES + j, wn + 32 * n, lane);
+#pragma unroll
+        for (int m = 0; m < MR; ++m) x[j][m] = oa.template read<PLAIN>(buf + STEP * u, wk * SLICES + j, wm + 32 * m, lane);
       }
 #pragma unroll
-      for (int j = 0; j < SLICES; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[j], x[j], acc, 0, 0, 0);
+      for (int j = 0; j < SLICES; ++j)
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+#pragma unroll
+          for (int n = 0; n < NR; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[j][n], x[j][m], acc[m][n], 0, 0, 0);
     }
   };
   if (rounds <= 3) {  // all at once
@@ -202,15 +219,16 @@ __global__ void __launch_bounds__(256, 2) narrow_gemm_kernel(NarrowArgs a) {
   __syncthreads();
   const int l32 = lane & 31, h = lane >> 5;
   constexpr int ROW = TN * 4 + 16, PART = TM * ROW;  // bytes
-  constexpr int FIRST = WK > 1 ? WK / 2 : 1;         // parts in b0 (64 x 64: its one begins there and ends in b1)
-  auto place = [&](int w, int m, int n) {            // of row m, columns n .. of the wave group w
-    if constexpr (WK > 1) return (w < FIRST ? b0 : b1) + w % FIRST * PART + m * ROW + n * 4;
-    else return (m < TM / 2 ? b0 : b1) + m % (TM / 2) * ROW + n * 4;
-  };
-  static_assert((WK > 1 ? FIRST * PART : PART / 2) <= BUF, "room for the sums");
+  auto place = [&](int w, int m, int n) { return lds + w * PART + m * ROW + n * 4; };  // of row m, columns n .. of the wave group w
+  static_assert(WK * PART <= 4 * BUF, "room for the sums");
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
-    *reinterpret_cast<f32x4*>(place(wk, wm + l32, wn + 8 * q + 4 * h)) = f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+  for (int m = 0; m < MR; ++m)
+#pragma unroll
+    for (int n = 0; n < NR; ++n)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f32x4*>(place(wk, wm + 32 * m + l32, wn + 32 * n + 8 * q + 4 * h)) =
+            f32x4{acc[m][n][4 * q], acc[m][n][4 * q + 1], acc[m][n][4 * q + 2], acc[m][n][4 * q + 3]};
   __syncthreads();
   constexpr int PIECES = TM * TN / 8;  // of 8 columns
 #pragma unroll
@@ -250,23 +268,32 @@ int g_tile = 0, g_parts = 0;
 struct Cut {
   int tm, tn, parts;  // tile, parts of K
 };
-// Tiles of 64 where those of 32 are more than two a CU (y of 128 tokens, us with 32 / 64: [3072, 1024] 6.4 / 6.9, [4096, 2048] 9.1 / 10.4,
-// [5632, 1024] 9.3 / 7.1), with an operand across the inner dimension from 128 of them on. Such operands come in rows of 64, never 32 (half a cache line: dX of 128 tokens by [3072, 1024] 14.9 for 11.3). Parts where the
-// tiles leave the chip idle: a sum costs 2 us and its traffic, so both operands along K want 2560 of it each (y of 64 tokens, [2048, 5632] 12.6
-// whole, 10.5 in two; [1024, 2816] 7.7 and 7.7), while rows across it come slower (dX of 128 tokens by [5632, 1024] 42 whole, 15.8
-// in four, 13.4 in eight; of 256 by [1024, 2816] 10.2 whole, 12.4 in two).
-Cut cut_of(int64_t M, int64_t N, int64_t K, bool along) {
-  auto tiles = [&](int tm, int tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
-  int tn = along ? 32 : 64, tm = 32;
-  if (g_tile ? g_tile == 64 : along ? tiles(32, 32) > 512 : tiles(64, 64) >= 128) tm = tn = 64;
-  const int64_t fill = (K >= 2048 ? 512 : 256) / tiles(tm, tn), longest = K / (along ? 2560 : 512);
-  const int64_t parts = g_parts ? std::min<int64_t>(g_parts, (K + 63) / 64) : std::min<int64_t>(std::min(fill, longest), 8);
+// us, on one machine, of 32-row tiles / 64 / 128, whole or in parts of K (x2, x4).
+// Both operands along K (y): 32 x 32 up to two tiles a CU (128 tokens by [3072, 1024] 6.4 / 6.4, [4096, 2048] 9.0 / 9.4, [5632, 1024] 8.6 / 6.7), 128 x
+// 128 from 140 of them on (512 by [5632, 1024] 13.7 with 64, 12.7; 768 by [3072, 1024], 144 of them, 13.8, 12.1; 256 by [8000, 1024], 126, 9.8, 12.2). Parts
+// of 2560 or more of K: a sum costs 2 us and its traffic (64 by [2048, 5632] 12.6, x2 10.5; [1024, 2816] 7.7, 7.7).
+// One across (dX): those rows come in runs of 64 columns, never 32 (half a cache line). 64 x 64 from 160 tiles on, of long K from 64
+// (256 tokens by [5632, 1024] 32x2 13.0, 64x4 11.8; 512 17.5, 64x2 15.8; by [3072, 1024] 9.5, 10.5). Parts of 768 up to a workgroup a CU
+// (128 by [3072, 1024] 10.6, x2 9.4, x4 8.9; by [1024, 1024] 5.3, 6.4, 6.9).
+// Both across (dW): 64 x 64, 128 x 128 from 176 of them on (512 by [3072, 1024] 11.0, 9.8; by [1536, 1024] 7.6, 8.7).
+Cut cut_of(int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) {
+  auto tiles = [&](int t, int u) { return ((M + t - 1) / t) * ((N + u - 1) / u); };
+  const bool along = a_along && b_along, across = !a_along && !b_along;
+  int tm = 32, tn = along ? 32 : 64;
+  if (tiles(128, 128) >= (across ? 176 : 140) && (along || across)) tm = tn = 128;
+  else if (along ? tiles(32, 32) > 512 : across || tiles(64, 64) >= (K >= 4096 ? 64 : 160)) tm = tn = 64;
+  if (g_tile) {
+    tm = g_tile;
+    tn = g_tile == 32 && !along ? 64 : g_tile;
+  }
+  int64_t parts = std::min<int64_t>(std::min<int64_t>((along ? 512 : 256) / tiles(tm, tn), K / (along ? 2560 : 768)), 8);
+  if (g_parts) parts = std::min<int64_t>(g_parts, (K + 63) / 64);
   return {tm, tn, (int)std::max<int64_t>(parts, 1)};
 }
 
 }  // namespace
 
-// Forces tiles of 64 or 32 rows and parts of K; 0: by the rule above.
+// Forces tiles of 32, 64 or 128 rows and parts of K; 0: by the rule above.
 extern "C" void ds_narrow_gemm_tune(int tile, int parts) { g_tile = tile; g_parts = parts; }
 
 // Whether the kernel takes the product: whole 16-byte pieces of rows, whole steps of 64 along an operand's rows, offsets of 32 bits
@@ -278,14 +305,20 @@ extern "C" int ds_narrow_gemm_ok(int64_t M, int64_t N, int64_t K, int64_t lda, i
   return (ar + 128) * lda * 2 < UINT32_MAX && (br + 128) * ldb * 2 < UINT32_MAX && ((M + 31) / 32) * ((N + 31) / 32) <= INT32_MAX;
 }
 
-// Whether it is as fast as the library's there. y, dX: up to 2^31 products (256 tokens by [8000, 1024] 9.8 us and 13.2, 21 and 31; of 2^32,
-// 128 tokens by [11264, 2048] 22 and 18). dW: up to 2^30 (256 tokens by [3072, 1024] 9.5 and 8.8, by [5632, 1024], 1.4 times 2^30, 13.8 and
-// 11.4).
-extern "C" int ds_narrow_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along) { return M * N <= (1LL << (a_along ? 31 : 30)) / K; }
+// Whether it is as fast as the library's there, us here (there); up to 1024 tokens. y: 2^31 products, of up to 2^24 weights 2^32 (512 tokens by
+// [8000, 1024] 13.7 (16.0); 128 by [11264, 2048] 21.6 (18.1); 1024 by [5632, 1024], 1.4 times 2^32, 23 (20.2)). dX: 3 2^32 and fewer than 3 2^20
+// results (512 by [11264, 2048] 61 (76), by [5632, 1024] 15.9 (25.3); 768 by [4096, 4096] 52 (42), 512 by [1024, 8192] 16.9 (15.2); 1500 by [4096, 2048]
+// 45 (35)). dW: 2^22 weights, 2^23 from up to 224 tokens (1024 by [3072, 1024] 13.3 (15.5); 200 by [8000, 1024] 14.5 (14.3), 256 15.2 (12.6)).
+extern "C" int ds_narrow_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along) {
+  if ((a_along ? M : K) > 1024) return 0;
+  if (!a_along) return M * N <= (K <= 224 ? 1 << 23 : 1 << 22);
+  if (!b_along) return M * N < (3 << 20) && M * N <= (3LL << 32) / K;
+  return M * N <= (1LL << (N * K <= (1 << 24) ? 32 : 31)) / K;
+}
 
 // Bytes of scratch memory that the product wants (0: none)
 extern "C" int64_t ds_narrow_gemm_scratch(int64_t M, int64_t N, int64_t K, int a_along, int b_along) {
-  const Cut c = cut_of(M, N, K, a_along && b_along);
+  const Cut c = cut_of(M, N, K, a_along, b_along);
   return c.parts > 1 ? c.parts * M * N * 4 : 0;
 }
 
@@ -294,7 +327,7 @@ extern "C" int64_t ds_narrow_gemm_scratch(int64_t M, int64_t N, int64_t K, int a
 extern "C" int ds_narrow_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_along,
                               int b_along, void* part, hipStream_t st) {
   if (!ds_narrow_gemm_ok(M, N, K, lda, ldb, a_along, b_along)) return (int)hipErrorInvalidValue;
-  const Cut cut = cut_of(M, N, K, a_along && b_along);
+  const Cut cut = cut_of(M, N, K, a_along, b_along);
   if (cut.parts == 1) part = nullptr;
   else if (!part) return (int)hipErrorInvalidValue;
   const int64_t ar = a_along ? M : K, ac = a_along ? K : M, br = b_along ? N : K, bc = b_along ? K : N;
@@ -302,7 +335,12 @@ extern "C" int ds_narrow_gemm(const void* A, const void* B, void* C, int64_t M, 
                      (uint32_t)(((ar - 1) * lda + ac) * 2), (uint32_t)(((br - 1) * ldb + bc) * 2), cut.parts, (f32x4*)part};
   const dim3 grid((unsigned)(((M + cut.tm - 1) / cut.tm) * ((N + cut.tn - 1) / cut.tn)), cut.parts);
 #define GO(AK, BK, TM, TN, U) hipLaunchKernelGGL((narrow_gemm_kernel<AK, BK, TM, TN, U>), grid, dim3(256), 0, st, a)
-  if (cut.tm == 64) {
+  if (cut.tm == 128) {
+    if (a_along && b_along) GO(true, true, 128, 128, 1);
+    else if (a_along) GO(true, false, 128, 128, 1);
+    else if (b_along) GO(false, true, 128, 128, 1);
+    else GO(false, false, 128, 128, 1);
+  } else if (cut.tm == 64) {
     if (a_along && b_along) GO(true, true, 64, 64, 1);
     else if (a_along) GO(true, false, 64, 64, 1);
     else if (b_along) GO(false, true, 64, 64, 1);

@@ -22,7 +22,7 @@ def _check(got, a, b):
 
 
 @GPU
-@pytest.mark.parametrize("tile,parts", [(0, 0), (32, 1), (32, 3), (64, 1), (64, 2)])
+@pytest.mark.parametrize("tile,parts", [(0, 0), (32, 1), (32, 3), (64, 1), (64, 2), (128, 1), (128, 2)])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 64), (8, 40, 64), (31, 64, 128), (33, 72, 192), (64, 136, 256), (72, 200, 320), (128, 96, 448),
                                    (127, 264, 576), (136, 1032, 1088)])
 def test_products_at_their_edges(M, N, K, tile, parts):
