@@ -192,31 +192,28 @@ __global__ void __launch_bounds__(256) rms_bwd_kernel(const T* __restrict__ dy, 
     dw_part[(int64_t)blockIdx.x * H + c] = sm[c] + sm[H + c] + sm[2 * H + c] + sm[3 * H + c];
 }
 
-// Column sum of nb partial rows, two deterministic stages so the reduction uses the whole chip:
-// stage 1 (grid H/256 x CS): block (x, y) sums rows y, y+CS, ... of its 256 columns into stage[y][c];
-// stage 2 (grid H/256): sums the CS stage rows and casts.
-constexpr int CS = 32;
-__global__ void __launch_bounds__(256) colsum_stage1(const float* __restrict__ part, int nb, int H, int ld,
-                                                     float* __restrict__ stage) {
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= H) return;
-  float acc = 0.f;
-  for (int b = blockIdx.y; b < nb; b += CS) acc += part[(int64_t)b * ld + c];
-  stage[(int64_t)blockIdx.y * H + c] = acc;
-}
+// Column sums of nb partial rows, in a fixed order: a block has 32 columns, its 32 groups of lanes every 32nd row, and they meet in LDS. Bound by
+// latency and the launch; in two launches (by rows, then over 32 sums) the second cost as much as the first. RMSNorm / LayerNorm backward, us,
+// before and now: 128 x 1024 8.2 / 12.2, 6.7 / 9.0; 3000 x 2048 17.5 / 26.6, 13.6 / 18.3; 8192 x 1024 25.6 / 33.7, 21.0 / 26.5; 32768 x 8192 the same.
 template <typename T>
-__global__ void __launch_bounds__(256) colsum_stage2(const float* __restrict__ stage, int H, T* __restrict__ out) {
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= H) return;
+__global__ void __launch_bounds__(1024) colsum_kernel(const float* __restrict__ part, int nb, int H, int ld, T* __restrict__ out) {
+  __shared__ float sums[32][33];
+  const int l = threadIdx.x & 31, g = threadIdx.x >> 5, c = blockIdx.x * 32 + l;
   float acc = 0.f;
+  if (c < H) {
+#pragma unroll 4
+    for (int b = g; b < nb; b += 32) acc += part[(int64_t)b * ld + c];
+  }
+  sums[g][l] = acc;
+  __syncthreads();
+  if (g || c >= H) return;
 #pragma unroll
-  for (int y = 0; y < CS; ++y) acc += stage[(int64_t)y * H + c];
+  for (int i = 1; i < 32; ++i) acc += sums[i][l];
   out[c] = (T)acc;
 }
 template <typename T>
-static void colsum(const float* part, int nb, int H, int ld, float* stage, T* out, hipStream_t s) {
-  hipLaunchKernelGGL(colsum_stage1, dim3((H + 255) / 256, CS), dim3(256), 0, s, part, nb, H, ld, stage);
-  hipLaunchKernelGGL((colsum_stage2<T>), dim3((H + 255) / 256), dim3(256), 0, s, stage, H, out);
+static void colsum(const float* part, int nb, int H, int ld, T* out, hipStream_t s) {
+  hipLaunchKernelGGL((colsum_kernel<T>), dim3((H + 31) / 32), dim3(1024), 0, s, part, nb, H, ld, out);
 }
 
 // ------------------------------------------------------------------------------------------------ LayerNorm
@@ -658,8 +655,8 @@ static constexpr int kMaxHidden = 8192;      // backward kernels
 static constexpr int kMaxHiddenFwd = 16384;  // forward kernels
 static int norm_grid(int64_t rows) { return ds_grid_for((rows + 3) / 4, 1, 256 * 8); }
 
-// Number of fp32 partial rows the backward writes for `rows`. The host allocates part[(nb + 32) * H] for RMSNorm
-// and part[(nb + 32) * 2H] for LayerNorm (the trailing 32 rows are the column-sum stage buffer).
+// Number of fp32 partial rows the backward writes for `rows`. The host allocates part[nb * H] for RMSNorm
+// and part[nb * 2H] for LayerNorm.
 // (512 = two persistent blocks per CU: measured best for the wide-row backward against 256 / 768 / 1024 / 2048)
 extern "C" int ds_norm_bwd_blocks(int64_t rows) { return ds_grid_for((rows + 3) / 4, 1, 512); }
 
@@ -694,7 +691,7 @@ extern "C" int ds_rms_bwd(const void* dy, const void* x, const void* w, const fl
   if (block_rows(H) && !bwd_wave_rows()) {
     DISPATCH_T(dtype, (launch_block_norm_bwd<T, false>(dy, x, w, nullptr, rstd, dres, dx, part, nb, rows, H, s)));
     DS_CHECK_LAUNCH();
-    DISPATCH_T(dtype, colsum<T>(part, nb, H, H, part + (int64_t)nb * H, (T*)dw, s));
+    DISPATCH_T(dtype, colsum<T>(part, nb, H, H, (T*)dw, s));
     DS_CHECK_LAUNCH();
     return 0;
   }
@@ -708,7 +705,7 @@ extern "C" int ds_rms_bwd(const void* dy, const void* x, const void* w, const fl
                          (const T*)w, rstd, nullptr, (T*)dx, part, rows, H);
   }));
   DS_CHECK_LAUNCH();
-  DISPATCH_T(dtype, colsum<T>(part, nb, H, H, part + (int64_t)nb * H, (T*)dw, s));
+  DISPATCH_T(dtype, colsum<T>(part, nb, H, H, (T*)dw, s));
   DS_CHECK_LAUNCH();
   return 0;
 }
@@ -755,10 +752,9 @@ extern "C" int ds_ln_bwd(const void* dy, const void* x, const void* g, const flo
                          (const T*)g, mean, rstd, nullptr, (T*)dx, part, rows, H);
   }));
   DS_CHECK_LAUNCH();
-  float* stage = part + (int64_t)nb * 2 * H;
   DISPATCH_T(dtype, {
-    colsum<T>(part, nb, H, 2 * H, stage, (T*)dg, s);
-    colsum<T>(part + H, nb, H, 2 * H, stage + (int64_t)CS * H, (T*)db, s);
+    colsum<T>(part, nb, H, 2 * H, (T*)dg, s);
+    colsum<T>(part + H, nb, H, 2 * H, (T*)db, s);
   });
   DS_CHECK_LAUNCH();
   return 0;
