@@ -16,6 +16,8 @@ import os
 import torch
 import torch.nn.functional as F
 
+from .native import hip_ops, unseen_from_python
+
 try:
     from torch.nn.attention import SDPBackend, sdpa_kernel
     _PREF = [SDPBackend.EFFICIENT_ATTENTION, SDPBackend.FLASH_ATTENTION, SDPBackend.MATH]
@@ -46,7 +48,6 @@ class FlashAttnFunc(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, causal, scale):
-        from .native import hip_ops
         need_grad = any(t.requires_grad for t in (q, k, v))
         o, lse = hip_ops().flash_fwd(q, k, v, bool(causal), float(scale), need_grad)
         if need_grad:
@@ -56,7 +57,6 @@ class FlashAttnFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, do):
-        from .native import hip_ops
         q, k, v, o, lse = ctx.saved_tensors
         if do.stride(-1) != 1 or any(s % 8 for s in do.stride()[:3]) or do.data_ptr() % 16:
             do = do.contiguous()
@@ -76,5 +76,6 @@ def attention(q, k, v, causal=True, softmax_scale=None, attn_mask=None, dropout_
     """q [B, Hq, S, D], k/v [B, Hk, S, D] -> o [B, Hq, S, D]."""
     if flash_supported(q, k, v, attn_mask, dropout_p):
         scale = softmax_scale if softmax_scale is not None else q.shape[-1]**-0.5
-        return FlashAttnFunc.apply(q, k, v, causal, scale)
+        o = hip_ops().flash_node(q, k, v, bool(causal), float(scale)) if unseen_from_python() else None
+        return FlashAttnFunc.apply(q, k, v, causal, scale) if o is None else o
     return _sdpa(q, k, v, causal, softmax_scale, attn_mask, dropout_p)

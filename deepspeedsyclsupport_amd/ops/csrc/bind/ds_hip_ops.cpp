@@ -3,6 +3,7 @@
 // expose a C ABI taking raw pointers + hipStream_t. Every op launches on torch's current HIP stream, so ops compose
 // with torch streams, events and hipGraph capture.
 #include <torch/extension.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/HIPContext.h>
 #include <hip/hip_runtime_api.h>
@@ -135,6 +136,35 @@ void adam_multi(std::vector<Tensor> p, std::vector<Tensor> m, std::vector<Tensor
         "adam_multi");
 }
 
+// The same over flat state: p, m and v of item i begin at element offs[i]
+void adam_multi_flat(Tensor p, Tensor m, Tensor v, std::vector<int64_t> offs, std::vector<Tensor> g, std::vector<Tensor> lp, double lr, double b1,
+                     double b2, double eps, double wd, double bc1, double bc2, double grad_scale, bool adamw) {
+  const size_t n = g.size();
+  if (n == 0) return;
+  need(p, "p"); need(m, "m"); need(v, "v");
+  TORCH_CHECK(offs.size() == n && lp.size() == n, "list sizes");
+  TORCH_CHECK(m.scalar_type() == at::kFloat && v.scalar_type() == at::kFloat && m.numel() == p.numel() && v.numel() == p.numel(),
+              "adam_multi_flat: fp32 moments of the flat's size");
+  std::vector<void*> pp(n), mp(n), vp(n), lpp(n);
+  std::vector<const void*> gp(n);
+  std::vector<int64_t> nn(n);
+  const int pd = dcode(p), gd = dcode(g[0]), ld = dcode(lp[0]);
+  for (size_t i = 0; i < n; ++i) {
+    need(g[i], "g"); need(lp[i], "lp");
+    nn[i] = g[i].numel();
+    TORCH_CHECK(dcode(g[i]) == gd && dcode(lp[i]) == ld, "adam_multi_flat: mixed dtypes within one call");
+    TORCH_CHECK(offs[i] >= 0 && nn[i] <= p.numel() - offs[i] && lp[i].numel() == nn[i], "adam_multi_flat: size mismatch");
+    pp[i] = (char*)p.data_ptr() + offs[i] * p.element_size();
+    mp[i] = m.data_ptr<float>() + offs[i];
+    vp[i] = v.data_ptr<float>() + offs[i];
+    gp[i] = g[i].data_ptr();
+    lpp[i] = lp[i].data_ptr();
+  }
+  check(ds_adam_multi(pp.data(), mp.data(), vp.data(), gp.data(), lpp.data(), nn.data(), (int)n, pd, gd, ld, lr, b1, b2, eps, wd, bc1, bc2,
+                      grad_scale, adamw ? 1 : 0, stream()),
+        "adam_multi_flat");
+}
+
 // split-master Adam: lo int16 residuals, m/v fp32, g any dtype, hi bf16 weights updated in place
 void adam_multi_split(std::vector<Tensor> lo, std::vector<Tensor> m, std::vector<Tensor> v, std::vector<Tensor> g,
                       std::vector<Tensor> hi, double lr, double b1, double b2, double eps, double wd, double bc1,
@@ -239,7 +269,7 @@ std::vector<Tensor> rms_bwd(Tensor dy, Tensor x, Tensor w, Tensor rstd, OptT dre
   auto dx = torch::empty_like(x);
   auto dw = torch::empty_like(w);
   const int nb = ds_norm_bwd_blocks(rows);
-  auto part = torch::empty({((int64_t)nb + 32) * H}, x.options().dtype(at::kFloat));
+  auto part = torch::empty({(int64_t)nb * H}, x.options().dtype(at::kFloat));
   if (dres.has_value()) need(*dres, "dres");
   check(ds_rms_bwd(dy.data_ptr(), x.data_ptr(), w.data_ptr(), rstd.data_ptr<float>(), ptr_or_null(dres),
                    dx.data_ptr(), dw.data_ptr(), part.data_ptr<float>(), rows, H, dcode(x), stream()),
@@ -270,7 +300,7 @@ std::vector<Tensor> ln_bwd(Tensor dy, Tensor x, Tensor g, Tensor mean, Tensor rs
   auto dx = torch::empty_like(x);
   auto dg = torch::empty_like(g), db = torch::empty_like(g);
   const int nb = ds_norm_bwd_blocks(rows);
-  auto part = torch::empty({((int64_t)nb + 32) * 2 * H}, x.options().dtype(at::kFloat));
+  auto part = torch::empty({(int64_t)nb * 2 * H}, x.options().dtype(at::kFloat));
   check(ds_ln_bwd(dy.data_ptr(), x.data_ptr(), g.data_ptr(), mean.data_ptr<float>(), rstd.data_ptr<float>(),
                   ptr_or_null(dres), dx.data_ptr(), dg.data_ptr(), db.data_ptr(), part.data_ptr<float>(), rows, H,
                   dcode(x), stream()),
@@ -515,14 +545,20 @@ Tensor xent_bwd(Tensor logits, Tensor labels, Tensor lse, OptT dloss, double dlo
 // out [B,S,Hq,128] so the o_proj GEMM reads it without a transpose copy, lse [B,Hq,S] fp32).
 // x [R, C] (16-bit, unit last stride) -> x^T contiguous [C, Rp] at HBM speed (K-major wgrad GEMM operands);
 // pad_to > R appends zero columns (the contraction dimension rounded up for the GEMM)
-// Nothing but the kernels looks at this call: no autograd, transform, dispatch mode, tracer or autocast, and no lazy bit on a tensor
-bool unwatched(const Tensor& a, const Tensor& b) {
+// No transform, dispatch mode, tracer or autocast has to see what becomes of these tensors, and none carries a tangent or a lazy bit
+bool unseen(std::initializer_list<const Tensor*> ts) {
   using K = c10::DispatchKey;
   static const c10::DispatchKeySet special({K::Python, K::PythonTLSSnapshot, K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Batched,
                                             K::Functionalize, K::Conjugate, K::Negative, K::ZeroTensor});
-  const auto tls = c10::impl::tls_local_dispatch_key_set();
-  return (tls.included_ - c10::default_included_set).empty() && !at::autocast::is_autocast_enabled(at::kCUDA) && !(a.key_set() | b.key_set()).has_any(special) &&
-         !(at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad())) && !a._fw_grad(0).defined() && !b._fw_grad(0).defined();
+  if (!(c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty() || at::autocast::is_autocast_enabled(at::kCUDA))
+    return false;
+  for (const Tensor* t : ts)
+    if (t->defined() && (t->key_set().has_any(special) || t->_fw_grad(0).defined())) return false;
+  return true;
+}
+// ... nor autograd
+bool unwatched(const Tensor& a, const Tensor& b) {
+  return !(at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad())) && unseen({&a, &b});
 }
 
 // A B^T over the inner dimension: a [M, K], or [K, M] if not a_along; b [N, K], or [K, N]. Undefined where the kernel does not take it
@@ -551,7 +587,7 @@ Tensor narrow_gemm(Tensor a, Tensor b, bool a_along, bool b_along) {
 }
 
 // x [.., I] W [O, I]^T
-Tensor linear(Tensor x, Tensor w) {
+Tensor linear_product(Tensor x, Tensor w) {
   if (unwatched(x, w) && x.dim() >= 2 && x.is_contiguous() && w.dim() == 2 && x.size(-1) == w.size(1) && x.numel()) {
     const Tensor y = narrow_product(x.view({-1, x.size(-1)}), w, true, true, false);
     if (y.defined()) {
@@ -800,6 +836,151 @@ std::vector<Tensor> sparse_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor ls
   return {dq, dk, dv};
 }
 
+// ------------------------------------------------------------------------------------------ autograd nodes of the training path
+// The functions of ops/linear.py, ops/attention.py and ops/transformer/functional.py as nodes in C++: the same kernels, saved tensors and
+// products, without Python between them (a training step of 1 x 128 tokens is the host's: 21 functions, 10 to 25 us each way). Every
+// `*_node` returns nothing where its Python function has to take the call: what transforms, traces, casts or counts it, and types and
+// layouts that are not the kernel's.
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+template <class T>
+using Node = torch::autograd::Function<T>;
+
+bool bf16_rows(const Tensor& t) { return t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.is_contiguous() && t.numel(); }
+
+struct LinearNode : Node<LinearNode> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
+    ctx->save_for_backward({x, w});  // (the parameter itself: a gathered weight that is released is not kept alive)
+    return linear_product(x, w);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &w = saved[1], go = grads[0].reshape({-1, w.size(0)});
+    Tensor gx, gw;
+    if (ctx->needs_input_grad(0)) gx = linear_input_grad(go, w).view(x.sizes());
+    if (ctx->needs_input_grad(1)) gw = linear_weight_grad(go, x.reshape({-1, x.size(-1)}));
+    return {gx, gw};
+  }
+};
+// x W^T of fewer than `rows` tokens
+OptT linear_node(Tensor x, Tensor w, int64_t rows) {
+  if (!bf16_rows(x) || x.dim() < 2 || x.numel() / x.size(-1) >= rows || !w.is_cuda() || w.scalar_type() != at::kBFloat16 || w.dim() != 2 ||
+      w.device() != x.device() || w.size(1) != x.size(-1) || !unseen({&x, &w}))
+    return c10::nullopt;
+  return LinearNode::apply(x, w);
+}
+
+struct RmsNormNode : Node<RmsNormNode> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, double eps, const OptT& residual) {
+    auto r = rms_fwd(x, residual, w, eps);
+    const bool sum = residual.has_value();
+    ctx->saved_data["sum"] = sum;
+    ctx->save_for_backward({sum ? r[1] : x, w, r[2]});
+    ctx->set_materialize_grads(false);
+    return sum ? variable_list{r[0], r[1]} : variable_list{r[0]};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const bool sum = ctx->saved_data["sum"].toBool();
+    const Tensor dy = grads[0].defined() ? grads[0].contiguous() : torch::zeros_like(saved[0]);
+    OptT dres;
+    if (sum && grads[1].defined()) dres = grads[1].contiguous();
+    auto d = rms_bwd(dy, saved[0], saved[1], saved[2], dres);
+    return {d[0], d[1], Tensor(), sum ? d[0] : Tensor()};  // (of what the forward added up the gradient is the same)
+  }
+};
+std::optional<std::vector<Tensor>> rms_norm_node(Tensor x, Tensor w, double eps, OptT residual) {
+  const Tensor none, &r = residual.has_value() ? *residual : none;
+  if (!bf16_rows(x) || !w.is_cuda() || w.scalar_type() != at::kBFloat16 || !w.is_contiguous() || w.device() != x.device() ||
+      (r.defined() && (!bf16_rows(r) || r.device() != x.device() || r.sizes() != x.sizes())) || !unseen({&x, &w, &r}))
+    return c10::nullopt;
+  return RmsNormNode::apply(x, w, eps, residual);
+}
+
+struct GatedActNode : Node<GatedActNode> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& gu, int64_t act) {
+    ctx->saved_data["act"] = act;
+    ctx->save_for_backward({gu});
+    return gated_act_fwd(gu, act);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    return {gated_act_bwd(grads[0].contiguous(), ctx->get_saved_variables()[0], ctx->saved_data["act"].toInt()), Tensor()};
+  }
+};
+OptT gated_act_node(Tensor gu, int64_t act) {
+  if (!bf16_rows(gu) || !unseen({&gu})) return c10::nullopt;
+  return GatedActNode::apply(gu, act);
+}
+
+struct QkvRopeNode : Node<QkvRopeNode> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& cos, const Tensor& sin, const OptT& pos, int64_t hq, int64_t hk,
+                               int64_t rot, int64_t offset, bool token_major) {
+    ctx->saved_data["rot"] = rot;
+    ctx->saved_data["offset"] = offset;
+    ctx->save_for_backward({cos, sin, pos.has_value() ? *pos : Tensor()});
+    return qkv_rope_fwd(qkv, cos, sin, pos, hq, hk, rot, offset, token_major);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    OptT pos;
+    if (saved[2].defined()) pos = saved[2];
+    const Tensor d = qkv_rope_bwd(grads[0], grads[1], grads[2], saved[0], saved[1], pos, ctx->saved_data["rot"].toInt(),
+                                  ctx->saved_data["offset"].toInt());
+    return {d, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+std::optional<std::vector<Tensor>> qkv_rope_node(Tensor qkv, Tensor cos, Tensor sin, OptT pos, int64_t hq, int64_t hk, int64_t rot, int64_t offset,
+                                                 bool token_major) {
+  const Tensor none, &p = pos.has_value() ? *pos : none;
+  if (!bf16_rows(qkv) || !unseen({&qkv, &cos, &sin, &p}) || cos.requires_grad() || sin.requires_grad()) return c10::nullopt;
+  return QkvRopeNode::apply(qkv, cos, sin, pos, hq, hk, rot, offset, token_major);
+}
+
+struct FlashNode : Node<FlashNode> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, bool causal, double scale) {
+    const bool grad = q.requires_grad() || k.requires_grad() || v.requires_grad();
+    auto r = flash_fwd(q, k, v, causal, scale, grad);
+    if (grad) ctx->save_for_backward({q, k, v, r[0], r[1]});
+    ctx->saved_data["causal"] = causal;
+    ctx->saved_data["scale"] = scale;
+    return r[0];
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto s = ctx->get_saved_variables();
+    Tensor go = grads[0];
+    bool rows = go.stride(-1) == 1 && (uintptr_t)go.data_ptr() % 16 == 0;
+    for (int d = 0; d < 3; ++d) rows = rows && go.stride(d) % 8 == 0;
+    if (!rows) go = go.contiguous();
+    auto d = flash_bwd(s[0], s[1], s[2], s[3], s[4], go, ctx->saved_data["scale"].toDouble(), ctx->saved_data["causal"].toBool() ? 1 : 0);
+    return {d[0], d[1], d[2], Tensor(), Tensor()};
+  }
+};
+OptT flash_node(Tensor q, Tensor k, Tensor v, bool causal, double scale) {
+  if (!unseen({&q, &k, &v})) return c10::nullopt;
+  return FlashNode::apply(q, k, v, causal, scale);
+}
+
+struct XentMeanNode : Node<XentMeanNode> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& labels, int64_t ignore_index, double smoothing, bool inplace) {
+    auto r = xent_mean_fwd(logits, labels, ignore_index, smoothing);
+    ctx->save_for_backward({logits, labels, r[1], r[2]});
+    ctx->saved_data["ignore"] = ignore_index;
+    ctx->saved_data["smoothing"] = smoothing;
+    ctx->saved_data["inplace"] = inplace;
+    return r[0];
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto s = ctx->get_saved_variables();
+    const Tensor d = xent_bwd(s[0], s[1], s[2], grads[0], 0., ctx->saved_data["inplace"].toBool(), ctx->saved_data["ignore"].toInt(),
+                              ctx->saved_data["smoothing"].toDouble(), s[3]);
+    return {d, Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+OptT xent_mean_node(Tensor logits, Tensor labels, int64_t ignore_index, double smoothing, bool inplace) {
+  if (!logits.is_cuda() || !unseen({&logits, &labels})) return c10::nullopt;
+  return XentMeanNode::apply(logits, labels, ignore_index, smoothing, inplace);
+}
+
 }  // namespace
 
 // other binding translation units of this extension
@@ -818,6 +999,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "deepspeedsyclsupport_amd gfx950 kernels";
   m.def("adam_flat", &adam_flat);
   m.def("adam_multi", &adam_multi);
+  m.def("adam_multi_flat", &adam_multi_flat);
   m.def("adam_multi_split", &adam_multi_split);
   m.def("lion_flat", &lion_flat);
   m.def("adagrad_flat", &adagrad_flat);
@@ -842,8 +1024,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("qkv_rope_bwd", &qkv_rope_bwd);
   m.def("rope_inplace", &rope_inplace);
   m.def("narrow_gemm", &narrow_gemm);
-  m.def("linear", &linear);
+  m.def("linear", &linear_product);
   m.def("linear_input_grad", &linear_input_grad);
+  m.def("linear_node", &linear_node);
+  m.def("rms_norm_node", &rms_norm_node);
+  m.def("gated_act_node", &gated_act_node);
+  m.def("qkv_rope_node", &qkv_rope_node);
+  m.def("flash_node", &flash_node);
+  m.def("xent_mean_node", &xent_mean_node);
   m.def("linear_weight_grad", &linear_weight_grad);
   m.def("narrow_gemm_tune", [](int64_t tile, int64_t parts) { ds_narrow_gemm_tune((int)tile, (int)parts); });
   m.def("transpose16", &transpose16, py::arg("x"), py::arg("pad_to") = 0);

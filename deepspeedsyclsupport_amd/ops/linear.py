@@ -14,7 +14,7 @@ import os
 import torch
 import torch.nn.functional as F
 
-from .native import hip_ops
+from .native import hip_ops, unseen_from_python
 
 KMAJOR_MIN_ROWS = int(os.environ.get("DS_WGRAD_KMAJOR_MIN_ROWS", "8192"))
 _ENABLED = os.environ.get("DS_WGRAD_KMAJOR", "1") != "0"
@@ -51,14 +51,10 @@ def _kmajor_of(t2d, given, Tp):
     return hip_ops().transpose16(_rows16(t2d), Tp)
 
 
-# (no public predicate says that a torch function mode is on)
-_function_modes = torch._C._len_torch_function_stack
-
-
 def _narrow(a, b):
     """Whether a product may go to the extension, which takes the short ones and gives torch the others and all that a transform,
-    dispatch mode, tracer or autocast has to see. Function modes and the compiler see calls from Python alone."""
-    return a.is_cuda and b.is_cuda and not _function_modes() and not torch.compiler.is_compiling()
+    dispatch mode, tracer or autocast has to see."""
+    return a.is_cuda and b.is_cuda and unseen_from_python()
 
 
 def plain_linear(x, weight, bias=None):
@@ -132,4 +128,10 @@ class LinearFunction(torch.autograd.Function):
 
 
 def linear(x, weight, bias=None):
+    """x W^T + b. Short token dimensions without a bias take the same as a node in C++."""
+    if bias is None and _narrow(x, weight):
+        y = hip_ops().linear_node(x, weight, KMAJOR_MIN_ROWS)
+        if y is not None:
+            return y
+    # a producer kernel may have written x's token-contiguous copy for the weight-gradient GEMM (`_ds_kmajor`)
     return LinearFunction.apply(x, weight, bias, getattr(x, "_ds_kmajor", None))

@@ -13,6 +13,16 @@ from . import op_builder
 DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 
 
+# (no public predicate says that a torch function mode is on)
+_function_modes = torch._C._len_torch_function_stack
+
+
+def unseen_from_python():
+    """Whether neither a torch function mode nor the compiler has to see the torch calls behind an op (dispatch modes, transforms,
+    tracers and autocast are looked for in the extension)."""
+    return not _function_modes() and not torch.compiler.is_compiling()
+
+
 @functools.lru_cache(None)
 def hip_ops():
     return op_builder.load("ds_hip_ops")

@@ -8,7 +8,7 @@ import torch
 import torch.nn.functional as F
 
 from .. import reference
-from ..native import hip_ops
+from ..native import hip_ops, unseen_from_python
 
 ACT_CODES = {"silu": 0, "swiglu": 0, "gelu_tanh": 1, "gelu_new": 1, "gelu_pytorch_tanh": 1, "gelu": 2, "geglu": 2,
              "relu": 3, "reglu": 3, "identity": 4}
@@ -54,6 +54,10 @@ def rms_norm(x, weight, eps=1e-6, residual=None):
         x = x.contiguous()
         if residual is not None:
             residual = residual.contiguous()
+        if unseen_from_python():
+            out = hip_ops().rms_norm_node(x, weight, eps, residual)  # (the same in C++, for bf16)
+            if out is not None:
+                return out[0] if residual is None else tuple(out)
         return _RMSNormFn.apply(x, weight, eps, residual)
     h = x + residual if residual is not None else x
     y = (h.float() * torch.rsqrt(h.float().pow(2).mean(-1, keepdim=True) + eps) * weight.float()).to(x.dtype)
@@ -137,7 +141,9 @@ def gated_activation(gate_up, act="silu"):
             out, out_t = _GatedActKMajorFn.apply(gate_up.contiguous(), code)
             out._ds_kmajor = out_t
             return out
-        return _GatedActFn.apply(gate_up.contiguous(), code)
+        gate_up = gate_up.contiguous()
+        out = hip_ops().gated_act_node(gate_up, code) if unseen_from_python() else None
+        return _GatedActFn.apply(gate_up, code) if out is None else out
     g, u = gate_up.chunk(2, dim=-1)
     return reference.ACTS[code](g) * u
 
@@ -229,7 +235,9 @@ def qkv_rope_split(qkv, cos, sin, num_heads, num_kv_heads, rotary_dim=None, posi
     rot = rotary_dim or D
     if qkv.is_cuda and D % 8 == 0 and rot % 16 == 0:
         pos = position_ids.to(torch.int32).contiguous() if position_ids is not None else None
-        return _QKVRopeFn.apply(qkv.contiguous(), cos, sin, pos, num_heads, num_kv_heads, rot, pos_offset, token_major)
+        args = (qkv.contiguous(), cos, sin, pos, num_heads, num_kv_heads, rot, pos_offset, token_major)
+        out = hip_ops().qkv_rope_node(*args) if unseen_from_python() else None
+        return _QKVRopeFn.apply(*args) if out is None else tuple(out)
     q, k, v = qkv.split([num_heads, num_kv_heads, num_kv_heads], dim=2)
     p = position_ids if position_ids is not None else torch.arange(pos_offset, pos_offset + S, device=qkv.device)
     q = reference.apply_rope_half(q, cos, sin, p)
@@ -350,7 +358,9 @@ def cross_entropy(logits, labels, ignore_index=-100, label_smoothing=0.0, reduct
         # the mean's kernel is one block: 65536 rows of 512 take 122 us forward and backward, 148 with torch's sums, 262144 of 128 455 and
         # 430
         if reduction not in ("none", "sum") and labels2.numel() <= XENT_MEAN_MAX:
-            return _XentMeanFn.apply(logits2, labels2, ignore_index, label_smoothing, inplace_backward)
+            args = (logits2, labels2, ignore_index, label_smoothing, inplace_backward)
+            mean = hip_ops().xent_mean_node(*args) if unseen_from_python() else None
+            return _XentMeanFn.apply(*args) if mean is None else mean
         per_tok = _XentFn.apply(logits2, labels2, ignore_index, label_smoothing, inplace_backward)
     else:
         per_tok = reference.cross_entropy(logits.reshape(-1, logits.shape[-1]), labels.reshape(-1), ignore_index,

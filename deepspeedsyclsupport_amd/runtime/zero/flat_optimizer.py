@@ -202,6 +202,7 @@ class FlatZeroOptimizer(ZeROOptimizer):
         zc_set = getattr(self.zc, "model_fields_set", set()) if self.zc is not None else set()
         overlap = not ("overlap_comm" in zc_set and not self.zc.overlap_comm)
         self.rs_stream = self.acc.Stream() if self.device.type == "cuda" and overlap else None
+        self._rs_issued = False  # something is on rs_stream that the compute stream has not waited for
         self.ag_stream = self.acc.Stream() if self.device.type == "cuda" and overlap else None
         # `reduce_scatter: false` (reference stage 1/2): all-reduce the whole bucket and keep the owner's slice
         self.use_reduce_scatter = bool(getattr(self.zc, "reduce_scatter", True)) if self.zc is not None else True
@@ -686,6 +687,7 @@ class FlatZeroOptimizer(ZeROOptimizer):
         ctx = self.acc.stream(self.rs_stream) if self.rs_stream is not None else _nullctx()
         if self.rs_stream is not None:
             self.rs_stream.wait_stream(compute)
+            self._rs_issued = True
         with ctx:
             comm = src if src.dtype == self.comm_dtype else src.to(self.comm_dtype)
             pre = self._pre_factor(g)
@@ -800,8 +802,7 @@ class FlatZeroOptimizer(ZeROOptimizer):
                     if g.grad_flat is None:
                         g.grad_flat = torch.zeros(g.padded, dtype=self.dtype, device=self.device)
                     self._reduce_group(g)
-        if self.rs_stream is not None:
-            self.acc.current_stream().wait_stream(self.rs_stream)
+        self._join_reductions()
         if self.coordinator is not None:
             self.coordinator.end_backward()
         self.micro_step += 1
@@ -815,7 +816,12 @@ class FlatZeroOptimizer(ZeROOptimizer):
                 if g.grad_flat is None:
                     g.grad_flat = torch.zeros(g.padded, dtype=self.dtype, device=self.device)
                 self._reduce_group(g)
-        if self.rs_stream is not None:
+        self._join_reductions()
+
+    def _join_reductions(self):
+        """The current stream waits for the reductions issued since it last did (55 us of host time where there are none)."""
+        if self._rs_issued:
+            self._rs_issued = False
             self.acc.current_stream().wait_stream(self.rs_stream)
 
     # ================================================================================ step
@@ -876,7 +882,9 @@ class FlatZeroOptimizer(ZeROOptimizer):
                             continue
                         if p.grad.is_sparse:
                             p.grad = p.grad.to_dense()
-                        gr = p.grad.reshape(-1)[lo - a:hi - a]
+                        gr = p.grad.reshape(-1)
+                        if hi - lo != n:
+                            gr = gr[lo - a:hi - a]
                         items.append((og, moff + lo - g.seg_lo - s, hi - lo, gr, g.shard[lo - g.seg_lo:hi - g.seg_lo],
                                       1.0 / div))
                 elif g._acc_valid:
@@ -893,13 +901,19 @@ class FlatZeroOptimizer(ZeROOptimizer):
         classes = defaultdict(list)
         for (og, moff, n, gr, lp, scale) in items:
             classes[(og, scale, gr.device.type)].append(gr)
-        sq = torch.zeros((), dtype=torch.float32, device=self.device)
+        sq = None
         for (og, scale, devtype), ts in classes.items():
             if devtype == "cuda":
                 s = native.hip_ops().sumsq_multi([t.contiguous() for t in ts])
             else:
                 s = sum((t.float().pow(2).sum() for t in ts), torch.zeros(())).to(self.device)
-            sq = sq + s * (scale * scale) / self._og_replicas(og)
+            if scale != 1.0:
+                s = s * (scale * scale)
+            if self._og_replicas(og) != 1:
+                s = s / self._og_replicas(og)
+            sq = s if sq is None else sq + s
+        if sq is None:
+            sq = torch.zeros((), dtype=torch.float32, device=self.device)
         if self.off is not None:
             for og, s in self.off.staged_norm_sq().items():
                 s = s.to(self.device) if torch.is_tensor(s) else torch.tensor(float(s), device=self.device)
@@ -914,8 +928,8 @@ class FlatZeroOptimizer(ZeROOptimizer):
         """Optimizer step at the accumulation boundary (the engine only calls it there)."""
         items = self._grad_items()
         scale = self._unscale_factor()
-        norm = self._global_norm_sq(items).sqrt() * scale
-        norm_f = float(norm)  # the one device->host sync per step (overflow / clipping decisions)
+        norm = self._global_norm_sq(items).sqrt()
+        norm_f = float(norm if scale == 1.0 else norm * scale)  # the one device->host sync per step (overflow / clipping decisions)
         self._global_grad_norm = norm_f
         overflow = not math.isfinite(norm_f)
         self.overflow = overflow
@@ -986,9 +1000,11 @@ class FlatZeroOptimizer(ZeROOptimizer):
                 for (_, moff, n, gr, lp, s) in by_og[og]:
                     classes[(gr.dtype, s)].append((moff, n, gr, lp))
                 for (gdt, s), lst in classes.items():
-                    ps = [master[moff:moff + n] for moff, n, _, _ in lst]
-                    ms = [st["exp_avg"][moff:moff + n] for moff, n, _, _ in lst]
-                    vs = [st["exp_avg_sq"][moff:moff + n] for moff, n, _, _ in lst]
+                    whole = master.is_cuda and not self.split_master  # (the kernel takes the flats and offsets in them)
+                    if not whole:
+                        ps = [master[moff:moff + n] for moff, n, _, _ in lst]
+                        ms = [st["exp_avg"][moff:moff + n] for moff, n, _, _ in lst]
+                        vs = [st["exp_avg_sq"][moff:moff + n] for moff, n, _, _ in lst]
                     gs = [gr for _, _, gr, _ in lst]
                     lps = [lp for _, _, _, lp in lst]
                     if master.is_cuda:
@@ -1001,8 +1017,9 @@ class FlatZeroOptimizer(ZeROOptimizer):
                             native.hip_ops().adam_multi_split(ps, ms, vs, gs, lps, group["lr"], b1, b2, group["eps"],
                                                               group["weight_decay"], bc1, bc2, grad_scale * s, adamw)
                         else:
-                            native.hip_ops().adam_multi(ps, ms, vs, gs, lps, group["lr"], b1, b2, group["eps"],
-                                                        group["weight_decay"], bc1, bc2, grad_scale * s, adamw)
+                            native.hip_ops().adam_multi_flat(master, st["exp_avg"], st["exp_avg_sq"], [it[0] for it in lst], gs,
+                                                             lps, group["lr"], b1, b2, group["eps"], group["weight_decay"],
+                                                             bc1, bc2, grad_scale * s, adamw)
                         for i, lp in back:
                             lp.copy_(lps[i], non_blocking=lp.is_pinned())
                     else:

@@ -9,19 +9,18 @@ import types
 
 import torch.nn as nn
 
-from ...ops.linear import LinearFunction
+from ...ops.linear import LinearFunction, linear
 
 # the training linear of ops/linear.py (saves the Parameter; K-major weight-gradient GEMM for long token dims)
 LinearFunctionForZeroStage3 = LinearFunction
 
 
 def zero3_linear_wrap(input, weight, bias=None):
-    return LinearFunctionForZeroStage3.apply(input, weight, bias, getattr(input, "_ds_kmajor", None))
+    return linear(input, weight, bias)
 
 
 def _zero3_linear_forward(self, x):
-    # a producer kernel may have written x's token-contiguous copy for the weight-gradient GEMM (`_ds_kmajor`)
-    return LinearFunctionForZeroStage3.apply(x, self.weight, self.bias, getattr(x, "_ds_kmajor", None))
+    return linear(x, self.weight, self.bias)
 
 
 def install_zero3_linear(module: nn.Module):
