@@ -770,9 +770,9 @@ class MatrixMemory(HeadScan):
 
     def heads(self, layer, proj, meta, cache, carry, out):
         w = self.weight
-        y = mixer_ops.matrix_memory(proj, mixer_ops.ScanLayout(rows=proj.shape[1], **self.at), cache.state[layer.layer_idx], meta,
-                                    self.gate + self.cols, w(layer, "i_b"), w(layer, "f_b"), self.cap, self.dk**-0.5)
-        mixer_ops.gated_norm(y, proj, self.gate, w(layer, "head_norm"), self.H, layer.spec.norm_eps, "sigmoid_after", out)
+        mixer_ops.matrix_memory_read_out(proj, mixer_ops.ScanLayout(rows=proj.shape[1], **self.at), cache.state[layer.layer_idx],
+                                         meta, self.gate + self.cols, w(layer, "i_b"), w(layer, "f_b"), self.cap, self.dk**-0.5,
+                                         w(layer, "head_norm"), layer.spec.norm_eps, out)
 
 
 class Retention(HeadScan):
@@ -798,9 +798,9 @@ class Retention(HeadScan):
         ld = w(layer, "log_decay")
         if self.H < len(self.decay):
             ld = ld[layer.tp_rank * self.H:(layer.tp_rank + 1) * self.H]
-        y = mixer_ops.retention(proj, mixer_ops.ScanLayout(rows=proj.shape[1], **self.at), cache.state[layer.layer_idx]["state"],
-                                meta, ld, self.rot.angles(w(layer, "rot_freq"), meta, carry), self.dk**-0.5)
-        mixer_ops.gated_norm(y, proj, self.gate, None, self.H, layer.spec.norm_eps, "silu_after", out)
+        mixer_ops.retention_read_out(proj, mixer_ops.ScanLayout(rows=proj.shape[1], **self.at), cache.state[layer.layer_idx]["state"],
+                                     meta, ld, self.rot.angles(w(layer, "rot_freq"), meta, carry), self.dk**-0.5,
+                                     layer.spec.norm_eps, out)
 
 
 class ParallelMixer(Mixer):

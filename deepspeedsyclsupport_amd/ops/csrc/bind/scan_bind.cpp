@@ -15,6 +15,10 @@ int ds_scan_recur(const void*, const void*, const float*, const float*, const fl
                   const float*, void*, int, const int*, int, int, const int*, const int*, const int*, void*, const int*, int,
                   int, hipStream_t);
 int ds_scan_chunk_ok(int);
+int ds_scan_step_ok(int, int);
+int ds_scan_step(const void*, const float*, int, const float*, int, int, const float*, const float*, float, float*, float, float*,
+                 float*, const int*, int, const int*, const int*, const int*, int, int, const float*, float, void*, int64_t, const int*,
+                 int, int, hipStream_t);
 int ds_scan_chunk(const void*, const void*, const float*, const float*, const float*, float, const void*, float*, float*,
                   const float*, void*, int, const int*, int, const int*, const int*, const int*, void*, const int*, int,
                   hipStream_t);
@@ -191,6 +195,43 @@ void scan_chunk(Tensor qk, Tensor v, OptT gb, OptT log_decay, OptT skip, double 
                       i32(cu, S + 1, "cu"), i32(start, S, "start"), i32(slots, S, "slots"), out.data_ptr(), D.v, (int)T, stream()),
         "scan_chunk");
 }
+
+// Whether `scan_step` takes heads of these sizes
+bool scan_step_ok(int64_t dk, int64_t dv) { return ds_scan_step_ok((int)dk, (int)dv); }
+
+// From the projection to the gated read-out in one launch, for the sequences in `list`: scan_split, scan_recur and gated_norm (mode 0
+// or 2, a part per head) with constant decays, or (gates = first of 2 H gate columns, with bi, bf, cap, peak and zstate) exp_gates too.
+// Writes their rows of out [T, H dv] (it may be columns of a wider matrix) and their slots
+void scan_step(Tensor proj, std::vector<int64_t> dims, OptT cs, OptT log_decay, int64_t gates, OptT bi, OptT bf, double cap,
+               OptT peak, double scale, Tensor state, OptT zstate, Tensor list, Tensor cu, Tensor start, Tensor slots, int64_t gate,
+               OptT w, double eps, int64_t mode, Tensor out) {
+  need(proj, "proj"); need(state, "state"); need_rows(out, "out");
+  const Dims D = dims_of(dims);
+  const int64_t T = proj.size(0), S = start.numel(), half = has(cs) ? cs->numel() / 2 / std::max<int64_t>(T, 1) : 0, C = D.H() * D.dv();
+  TORCH_CHECK(proj.dim() == 2 && proj.size(1) == D.rows() && 2 * half <= D.dk() && D.taps() == 1 && gate >= 0 && gate + C <= D.rows(),
+              "scan_step: proj [T, rows]");
+  TORCH_CHECK(out.size(0) == T && out.size(1) == C && out.scalar_type() == proj.scalar_type(), "scan_step: out [T, H dv]");
+  TORCH_CHECK(state.scalar_type() == at::kFloat && state.dim() == 4 && state.size(1) == D.H() && state.size(2) == D.dv() &&
+              state.size(3) == D.dks(), "scan_step: state [slots, H, dv, dks] fp32");
+  TORCH_CHECK(has(log_decay) != has(zstate) && has(bi) == has(zstate) && has(bf) == has(zstate) && has(peak) == has(zstate),
+              "scan_step: decays per head, or gates with a normaliser");
+  if (has(zstate)) {
+    need(*zstate, "normaliser"); need(*peak, "peak");
+    TORCH_CHECK(zstate->scalar_type() == at::kFloat && zstate->dim() == 4 && zstate->size(0) == state.size(0) &&
+                zstate->size(1) == D.H() && zstate->size(2) == (D.dv() + 31) / 32 && zstate->size(3) == D.dks(),
+                "scan_step: normaliser [slots, H, dv / 32, dks] fp32");
+    TORCH_CHECK(peak->scalar_type() == at::kFloat && peak->dim() == 2 && peak->size(0) == state.size(0) && peak->size(1) == D.H(),
+                "scan_step: peak [slots, H] fp32");
+    TORCH_CHECK(gates >= 0 && gates + 2 * D.H() <= D.rows() && cap > 0, "scan_step: gate columns outside the projection");
+  }
+  check(ds_scan_step(proj.data_ptr(), has(cs) ? f32(*cs, T * half * 2, "angles") : nullptr, (int)half,
+                     opt_f32(log_decay, D.H(), "log_decay"), (int)gates, (int)gates + D.H(), opt_f32(bi, D.H(), "input bias"),
+                     opt_f32(bf, D.H(), "forget bias"), (float)cap, has(peak) ? peak->data_ptr<float>() : nullptr, (float)scale,
+                     state.data_ptr<float>(), has(zstate) ? zstate->data_ptr<float>() : nullptr, i32(list, list.numel(), "list"),
+                     (int)list.numel(), i32(cu, S + 1, "cu"), i32(start, S, "start"), i32(slots, S, "slots"), (int)gate, (int)mode,
+                     opt_f32(w, C, "norm"), (float)eps, out.data_ptr(), T > 1 ? out.stride(0) : C, D.v, (int)T, dcode(proj), stream()),
+        "scan_step");
+}
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -200,4 +241,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("exp_gates", &exp_gates);
   m.def("scan_recur", &scan_recur);
   m.def("scan_chunk", &scan_chunk);
+  m.def("scan_step_ok", &scan_step_ok);
+  m.def("scan_step", &scan_step);
 }

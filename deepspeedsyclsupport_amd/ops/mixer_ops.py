@@ -93,6 +93,12 @@ def latent_attention(q, lat, ukv, ukt, freq, sink, meta, scale, d, e, window=0, 
 
 
 # ------------------------------------------------------------------------------------------------ recurrences
+# Tokens of a portion up to which gates, recurrence and gated norm go in one launch (recur/scan_step.hip has the figures): 16 sequences
+# of 16 heads of 128 take 7.4 us for 13.1 at one token, 11.5 for 19.8 at four, a matrix memory's 8.4 for 14.9 and 14.8 for 19.0;
+# at 16 tokens, where two barriers a token count and the separate gates see all tokens at once, the memory's take 40 for 34
+STEP_LONGEST = 4
+
+
 @dataclass(frozen=True)
 class ScanLayout:
     """Where a fused projection row [rows] holds what. q, k [Hk heads of dk], v [H heads of dv] and the output gate start
@@ -170,6 +176,35 @@ def matrix_memory(proj, lay, slots, meta, gates, bi, bf, cap, scale):
 
 
 # ------------------------------------------------------------------------------------------------ selective recurrences
+def _steps(proj, lay, meta):
+    """The extension if this batch goes from the projection to the read-out in one launch."""
+    cu = meta.cu_host
+    if not use_native(proj) or (meta.n_decode < len(cu) - 1 and max(b - a for a, b in zip(cu, cu[1:])) > STEP_LONGEST):
+        return None
+    ops = scan_ops()
+    return ops if ops.scan_step_ok(lay.dk, lay.dv) else None
+
+
+def retention_read_out(proj, lay, state, meta, log_decay, cs, scale, eps, out):
+    """`retention`, divided by its rms head by head, times silu of the gate columns -> out [T, H dv]."""
+    if (ops := _steps(proj, lay, meta)):
+        ops.scan_step(proj, lay.dims, cs, log_decay, 0, None, None, 1.0, None, scale, state, None, meta.seq_list, meta.cu_q,
+                      meta.start_pos, meta.slots, lay.gate, None, eps, GATES["silu_after"], out)
+    else:
+        y = retention(proj, lay, state, meta, log_decay, cs, scale)
+        gated_norm(y, proj, lay.gate, None, lay.H, eps, "silu_after", out)
+
+
+def matrix_memory_read_out(proj, lay, slots, meta, gates, bi, bf, cap, scale, w, eps, out):
+    """`matrix_memory`, divided by its rms head by head, times w and the sigmoid of the gate columns -> out [T, H dv]."""
+    if (ops := _steps(proj, lay, meta)):
+        ops.scan_step(proj, lay.dims, None, None, gates, bi, bf, cap, slots["peak"], scale, slots["state"], slots["norm"],
+                      meta.seq_list, meta.cu_q, meta.start_pos, meta.slots, lay.gate, w, eps, GATES["sigmoid_after"], out)
+    else:
+        y = matrix_memory(proj, lay, slots, meta, gates, bi, bf, cap, scale)
+        gated_norm(y, proj, lay.gate, w, lay.H, eps, "sigmoid_after", out)
+
+
 def causal_conv(x, w, b, conv_state, meta):
     """silu(conv(x) + b): x [T, C] (it may be columns of a wider matrix), w [C, taps] (last column: the current token), inputs
     before a portion from its slot of conv_state [slots, taps - 1, C]. This op or the `selective_scan` that must follow moves the

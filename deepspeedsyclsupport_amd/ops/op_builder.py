@@ -91,6 +91,7 @@ EXTENSIONS = {
             "recur/exp_gates.hip",
             "recur/decayed_scan.hip",
             "recur/decayed_chunk.hip",
+            "recur/scan_step.hip",
         ],
         "bindings": ["bind/scan_bind.cpp"],
     },

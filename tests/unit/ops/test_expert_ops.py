@@ -500,6 +500,62 @@ def test_chunked_memory_is_fp32(dk, dv):
         assert ((o - outs[0]).abs() <= 1.6e-2 * outs[0].abs() + 1e-3).all()
 
 
+# in one launch: key rows padded to 32, 64, 128 and 256, up to 128 value columns; the last two of a kind that is not taken
+STEP_HEADS = [(3, 16, 24), (1, 5, 8), (2, 64, 40), (4, 33, 31), (2, 128, 128), (2, 200, 64), (1, 256, 72), (2, 128, 130), (2, 128, 24)]
+
+
+@pytest.mark.parametrize("device,dtype,tol", CASES)
+@pytest.mark.parametrize("H,dk,dv", STEP_HEADS)
+@pytest.mark.parametrize("memory", [False, True])
+def test_read_out(device, dtype, tol, H, dk, dv, memory):
+    """From the projection to the gated read-out over portions of 1 to 4 tokens, which go in one launch, with longer ones between
+    them, in reused slots, into columns of a wider matrix. The sum over dv columns of a read-out at unit size carries the error of
+    the read-out itself, so the tolerance is that of its parts; in 16 bits the result is rounded once."""
+    first, cap, eps, pad = 8, 6.0, 1e-2, 8
+    gates = first + H * (2 * dk + 2 * dv)
+    la = mixer_ops.ScanLayout(rows=gates + 2 * H + 3, q=first, k=first + H * dk, v=first + 2 * H * dk, gate=gates - H * dv, Hk=H,
+                              H=H, dk=dk, dv=dv)
+    cuts = [[(0, 1), (1, 4), (2, 1)], [(0, 1), (2, 1), (1, 1)], [(0, 40), (1, 2)], [(2, 5), (0, 3)], [(1, 4), (0, 2), (2, 1)]]
+    n = [sum(c for step in cuts for j, c in step if j == i) for i in range(3)]
+    proj = [rnd(m, la.rows, seed=i).to(dtype) for i, m in enumerate(n)]
+    b, weight, rot = rnd(2, H, seed=9), 1 + rnd(H * dv, seed=3, scale=0.3), dk // 2 // 2 * 2
+    decay = torch.tensor([0.05, 1.0, 0.97, 0.9][:H], dtype=torch.float64)
+    slots = {"state": torch.full((3, H, dv, la.dks), 7.0, device=device), "peak": torch.full((3, H), 9.0, device=device),
+             "norm": torch.full((3, H, -(-dv // 32), la.dks), -5.0, device=device)}
+    for name in ("state", "norm"):
+        slots[name][..., dk:] = 0
+    freq = torch.tensor([50.0**(-2 * i / max(rot, 1)) for i in range(rot // 2)], dtype=torch.float64, device=device)
+    d, ld, slot, at, got = b.to(device), decay.log().float().to(device), (2, 0, 1), [0, 0, 0], [[], [], []]
+    for step in cuts:
+        mm, _ = meta([(at[i], c) for i, c in step], device, slots=[slot[i] for i, _ in step])
+        x = torch.cat([proj[i][at[i]:at[i] + c] for i, c in step]).to(device)
+        wide = torch.full((len(x), H * dv + 2 * pad), 9.0, dtype=dtype, device=device)
+        out = wide[:, pad:pad + H * dv]
+        if memory:
+            mixer_ops.matrix_memory_read_out(x, la, slots, mm, gates, d[0], d[1], cap, dk**-0.5, weight.to(device), eps, out)
+        else:
+            mixer_ops.retention_read_out(x, la, slots["state"], mm, ld, hybrid_ops.rope_table(mm.pos_ids, freq) if rot else None,
+                                         dk**-0.5, eps, out)
+        assert (wide[:, :pad] == 9).all() and (wide[:, pad + H * dv:] == 9).all()
+        row = 0
+        for i, c in step:
+            got[i].append(out[row:row + c])
+            row, at[i] = row + c, at[i] + c
+    for i, x in enumerate(proj):
+        li, lf = _gates(la, x, gates, b, cap, H)
+        x = x.double()
+        part = lambda at, w: x[:, at:at + H * w].view(-1, H, w)
+        q, k, v, g = part(la.q, dk) * dk**-0.5, part(la.k, dk), part(la.v, dv), x[:, la.gate:la.gate + H * dv]
+        turn = lambda y: O.rotate(y, rot, 50.0)
+        o = torch.stack([O.matrix_memory(q[:, h], k[:, h], v[:, h], li[:, h], lf[:, h]) if memory else
+                         O.decayed_scan(turn(q[:, h]), turn(k[:, h]), v[:, h], decay[h]) for h in range(H)], 1)
+        want = O.rms(o, eps).reshape(-1, H * dv) * (weight.double() * O.sigmoid(g) if memory else O.silu(g))
+        close(torch.cat(got[i]), want, tol if dtype != torch.float32 else 2e-4)
+    assert not slots["state"][..., dk:].any()
+    if memory:
+        assert not slots["norm"][..., dk:].any() and (slots["norm"] == slots["norm"][:, :, :1]).all()
+
+
 @pytest.mark.parametrize("device,dtype,tol", CASES)
 @pytest.mark.parametrize("P,parts", [(24, 3), (64, 5), (96, 4), (128, 16), (192, 2), (500, 1), (37, 2), (1024, 3), (8, 9)])
 def test_gated_norm_of_heads(device, dtype, tol, P, parts):
