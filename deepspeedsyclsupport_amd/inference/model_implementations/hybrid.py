@@ -146,8 +146,8 @@ class PreNormResidual(nn.Module):
         return x, expert_ops.pre_norm(x, None, model.layers[0].res1.norm_w, spec.norm_eps, ids=ids, embed=model.embed,
                                       mult=spec.embed_scale)
 
-    def enter(self, spec, x, pending):
-        return expert_ops.pre_norm(x, pending[0], self.norm_w, spec.norm_eps)
+    def enter(self, spec, x, pending, router=None):
+        return expert_ops.pre_norm(x, pending[0], self.norm_w, spec.norm_eps, router=router)
 
     def finish(self, model, x, y, rows, gate=None):
         return expert_ops.pre_norm(x, y, model.norm_w, model.spec.norm_eps, rows=rows)
@@ -174,9 +174,9 @@ class SandwichResidual(PreNormResidual):
         """How `pre_norm` takes this sublayer's output."""
         return dict(post_w=self.post_w, gate=gate, gate_b=None if gate is None else self.gate_b)
 
-    def enter(self, spec, x, pending):
+    def enter(self, spec, x, pending, router=None):
         y, prev, gate = pending
-        return expert_ops.pre_norm(x, y, None if self.side else self.norm_w, spec.norm_eps, **prev._close(gate))
+        return expert_ops.pre_norm(x, y, None if self.side else self.norm_w, spec.norm_eps, **prev._close(gate), router=router)
 
     def finish(self, model, x, y, rows, gate=None):
         return expert_ops.pre_norm(x, y, model.norm_w, model.spec.norm_eps, rows=rows, **self._close(gate))
@@ -864,6 +864,9 @@ class MLP:
         """Copies for decoding of weights that are no plain projections."""
         return {}
 
+    def router(self, layer):
+        """What the norm ahead of this takes along to route its rows, if there is anything to route."""
+
 
 class ClampedMLP(MLP):
     """Gated feed-forward whose branches are clamped before the product."""
@@ -943,8 +946,7 @@ class RoutedMLP(MLP):
         self.E, self.top = int(ro["experts"]), int(ro["top"])
         self.groups, self.keep = int(groups.get("count", 1)), int(groups.get("keep", 1))
         self.act, self.shared = ml.get("act", "silu_glu"), int((ml.get("shared") or {}).get("ff") or 0)
-        self.how = dict(score=ro.get("score", "softmax"), best=int(groups.get("best", 1)), scale=float(ro.get("scale", 1.0)),
-                        act=self.act)
+        self.how = dict(score=ro.get("score", "softmax"), best=int(groups.get("best", 1)), scale=float(ro.get("scale", 1.0)))
         if ml["expert"]["ff"] % tp or self.shared % tp:
             raise ValueError(f"expert widths {ml['expert']['ff']}, {self.shared} over {tp} ranks")
         if self.groups < 1 or self.E % self.groups or not 1 <= self.keep <= self.groups or \
@@ -976,10 +978,13 @@ class RoutedMLP(MLP):
         both = expert_ops.operand_order(layer.fc1_w.data), expert_ops.operand_order(layer.fc2_w.data)
         return {} if any(w is None for w in both) else {"experts": both}
 
+    def router(self, layer):
+        return expert_ops.Router(layer.router_w, self.top, self.groups, self.keep, layer.sh.get("experts"), **self.how)
+
     def run(self, layer, h, carry):
         first = layer.project(h, carry, self) if self.shared or layer.gated else None
         y = expert_ops.experts(h, layer.router_w, layer.fc1_w, layer.fc2_w, self.top, self.groups, self.keep,
-                               layer.sh.get("experts"), **self.how)
+                               layer.sh.get("experts"), **self.how, act=self.act, routed=carry.pop("routed", None))
         if self.shared:
             y.base = layer._linear(expert_ops.row_act(first, self.act), "shared2_w")
         return y if layer.tp == 1 else y.sum()   # ranks exchange plain sums
@@ -1104,7 +1109,11 @@ class DSHybridLayer(ProjectionLayer):
         y = self._allreduce(self._linear(self.mixer.run(self, h, meta, cache, carry), "o_w"))
         pending = (y, self.res1, carry.pop("gate", None))
         if self.mlp:
-            h = self.res2.enter(self.spec, x, pending)
+            router = self.mlp.router(self) if isinstance(self.res2, PreNormResidual) else None
+            if router is None:
+                h = self.res2.enter(self.spec, x, pending)
+            else:
+                h, carry["routed"] = self.res2.enter(self.spec, x, pending, router)
             y = self._allreduce(self.mlp.run(self, h, carry))
             pending = (y, self.res2, carry.pop("gate", None))
         if self.side:

@@ -4,7 +4,7 @@ sublayers' inputs and, optionally, on their gated outputs, grouped routing, expe
 Device tensors run the gfx950 kernels of `ds_expert_ops` (fp32 or bf16 storage); host tensors the plain versions in
 `ops/reference.py`, as everywhere in `ops`. Residual, norms, router logits and scores are fp32 whatever the storage type."""
 from dataclasses import dataclass
-from typing import Optional
+from typing import NamedTuple, Optional
 
 import torch
 
@@ -25,14 +25,39 @@ class ExpertSum:
         return (expert_ops() if use_native(self.y) else reference).expert_sum(self.y, self.w, self.rows, self.base)
 
 
-def pre_norm(x, y, w, eps, ids=None, embed=None, mult=1.0, rows=None, post_w=None, gate=None, gate_b=None):
+class Router(NamedTuple):
+    """How a sublayer picks its experts: the arguments of `experts` that its routing goes by."""
+    w: torch.Tensor
+    top: int
+    groups: int = 1
+    keep: int = 1
+    order: Optional[tuple] = None
+    score: str = "softmax"
+    best: int = 1
+    scale: float = 1.0
+
+    def lists(self, ops, dtype, tokens):
+        """Whether the products take lists of every expert's rows, and whether they tile the rows."""
+        rows = tokens * self.top
+        tile = self.order is not None and rows >= TILE_ROWS * self.w.shape[0]
+        return not (dtype != torch.bfloat16 or (rows <= ops.expert_few() and not tile)), tile
+
+
+def pre_norm(x, y, w, eps, ids=None, embed=None, mult=1.0, rows=None, post_w=None, gate=None, gate_b=None, router=None):
     """Residual x [T, W] fp32, in place: x += y (a tensor or an `ExpertSum`), or x = mult embed[ids]. Returns x / rms(x) * w (w
     None: x) in y's (embed's) type. With `rows`: x stays, and those rows come back. What is added may first be multiplied by
     sigmoid(gate + gate_b), gate [T, W] (it may be columns of a wider matrix), and then be divided by its own rms, times
-    post_w."""
-    f = (expert_ops() if use_native(x) else reference).pre_norm
+    post_w. With a `router`: (the result, its routing for `experts` where it came in the same pass)."""
+    ops = expert_ops() if use_native(x) else reference
     parts = (y.y, y.w, y.rows, y.base) if isinstance(y, ExpertSum) else (y, None, None, None)
-    return f(x, *parts, w, eps, ids, embed, mult, rows, post_w, gate, gate_b)
+    if router is None:
+        return ops.pre_norm(x, *parts, w, eps, ids, embed, mult, rows, post_w, gate, gate_b)
+    r, lists = router, ops is not reference and router.lists(ops, parts[0].dtype, x.shape[0])[0]
+    if ops is reference or parts[0].dtype != torch.bfloat16 or not ops.pre_norm_route_ok(x, r.w, gate, r.top, lists):
+        return ops.pre_norm(x, *parts, w, eps, None, None, 1.0, None, post_w, gate, gate_b), None
+    h, *routed = ops.pre_norm_route(x, *parts, w, eps, post_w, gate, gate_b, r.w, r.top, r.groups, r.keep, lists, SCORES[r.score], r.best,
+                                    r.scale)
+    return h, routed
 
 
 ACTS = {"none": 0, "silu_glu": 1, "relu2": 2}   # of a product's rows; silu_glu: silu(first half) times the second
@@ -60,11 +85,13 @@ def operand_order(w):
     return torch.stack([preshuffle16(e) for e in w]).view(E, N, K)
 
 
-def experts(h, router, fc1, fc2, top, groups=1, keep=1, order=None, score="softmax", best=1, scale=1.0, act="silu_glu"):
+def experts(h, router, fc1, fc2, top, groups=1, keep=1, order=None, score="softmax", best=1, scale=1.0, act="silu_glu",
+            routed=None):
     """Routed feed-forwards: h [T, W], router [E, W], fc1 [E, F, W] (gated: [E, 2 F, W], gate rows, up rows), fc2 [E, W, F] ->
     `ExpertSum`. Experts are scored by the softmax over all or by their own sigmoids. Those of the `keep` best of `groups` equal
     groups compete (a group counts as much as its `best` best members together); the `top` best are taken, weighted by their
-    scores divided by the scores' sum, times `scale`. `order`: (fc1, fc2) in operand order, if they are kept."""
+    scores divided by the scores' sum, times `scale`. `order`: (fc1, fc2) in operand order, if they are kept. `routed`: the routing that
+    `pre_norm` made with the same router."""
     code, routing = ACTS[act], (top, groups, keep)
     how = (SCORES[score], best, scale)
     if not use_native(h):
@@ -72,10 +99,9 @@ def experts(h, router, fc1, fc2, top, groups=1, keep=1, order=None, score="softm
         return ExpertSum(reference.expert_gemm(reference.expert_gemm(h, fc1, e, top, code), fc2, e, 1, 0), w)
     ops = expert_ops()
     rows, E = h.shape[0] * top, router.shape[0]
-    tile = order is not None and rows >= TILE_ROWS * E
-    few = h.dtype != torch.bfloat16 or (rows <= ops.expert_few() and not tile)
-    e, w, offs, entries, at = ops.route(h, router, *routing, not few, *how)
-    if order is None and not few and rows >= LIBRARY_ROWS * E and all(n % 128 == 0 for n in (*fc1.shape[1:], fc2.shape[2])):
+    lists, tile = Router(router, *routing, order).lists(ops, h.dtype, h.shape[0])
+    e, w, offs, entries, at = routed or ops.route(h, router, *routing, lists, *how)
+    if order is None and lists and rows >= LIBRARY_ROWS * E and all(n % 128 == 0 for n in (*fc1.shape[1:], fc2.shape[2])):
         ends = offs[1:]
         mid = ops.row_act(torch._grouped_mm(ops.expert_spread(h, at), fc1.transpose(1, 2), offs=ends), code)
         return ExpertSum(torch._grouped_mm(mid, fc2.transpose(1, 2), offs=ends), w, at)

@@ -90,6 +90,52 @@ def test_route(device, dtype, tol, E, top, groups, keep, W, T):
     assert (full - got)[same.all(-1)].abs().max() < 1e-5
 
 
+@pytest.mark.parametrize("device,dtype,tol", CASES)
+@pytest.mark.parametrize("E,top,groups,keep,W", [(12, 3, 3, 2, 64), (7, 7, 1, 1, 2040), (33, 4, 3, 1, 2056), (64, 8, 8, 3, 8192),
+                                                 (160, 6, 8, 3, 96), (256, 10, 16, 5, 128), (16, 4, 4, 2, 8200), (12, 3, 3, 2, 37)])
+@pytest.mark.parametrize("T", [1, 21, 256, 512, 513])
+def test_norm_and_route(device, dtype, tol, E, top, groups, keep, W, T):
+    """Norm and routing in one pass: the rows are those of the norm by itself but for sums in another order (a last bit in fp32, at
+    times one in 16 bits), the routing is what fp64 makes of the rows as they came back, the lists hold every pair once. Beyond 512
+    (few experts: 256) rows, with too many pairs an expert, for widths that are no multiple of 8 or exceed 8192 and in fp32 the
+    routing is left to `experts`. A logit sums W exact
+    products, W / 64 of them one by one, then a tree: off by (W / 64 + 8) 2^-24 of their sizes' sum at most, a weight by twice that."""
+    if device == "cpu" and T > 21:
+        pytest.skip("sizes of device kernels")
+    eps, K, post = 1e-3, 3, T % 2
+    x, y, g = rnd(T, W, seed=1), rnd(T * K, W, seed=2).to(dtype), torch.softmax(rnd(T, K, seed=3), -1)
+    r, w = rnd(E, W, seed=4, scale=1.5 * W**-0.5).to(dtype), 1 + rnd(W, seed=5, scale=0.2)
+    d = lambda t: None if t is None else t.to(device)
+    side = dict(post_w=d(1 + rnd(W, seed=6, scale=0.2)), gate=d(rnd(T, W + 8, seed=7).to(dtype))[:, 8:], gate_b=d(rnd(W, seed=8))) \
+        if post else {}
+    e = expert_ops.ExpertSum(d(y), d(g), None, d(rnd(T, W, seed=9).to(dtype)))
+    a, b = d(x).clone(), d(x).clone()
+    plain = expert_ops.pre_norm(a, e, d(w), eps, **side)
+    h, routed = expert_ops.pre_norm(b, e, d(w), eps, **side, router=expert_ops.Router(d(r), top, groups, keep))
+    many = E >= 64
+    lists = device == "cuda" and expert_ops.Router(r, top).lists(expert_ops.expert_ops(), dtype, T)[0]
+    fits = device == "cuda" and dtype == torch.bfloat16 and T <= (512 if many else 256) and W % 8 == 0 and W <= 8192 and \
+        (not lists or T * top <= (64 if many else 32) * E)
+    assert (routed is not None) == fits
+    if not fits:
+        assert torch.equal(h, plain) and torch.equal(a, b)
+        return
+    close(b, a.cpu(), 1e-6)
+    assert ((h.float() - plain.float()).abs() <= 2**-7 * plain.float().abs() + 1e-5).all()
+    ge, gw, offs, order, rows = routed
+    hd, rd = h.cpu().double(), r.double()
+    we, ww = O.route(hd @ rd.t(), top, groups, keep)
+    same = (ge.cpu() == we).all(-1)
+    assert same.float().mean() >= (1.0 if T < 100 else 0.99)
+    bound = (W / 64 + 8) * 2**-24 * (hd.abs() @ rd.abs().t()).max()
+    assert (gw.cpu().double() - ww)[same].abs().max() <= 2 * bound
+    if offs is not None:
+        assert torch.equal(order.cpu().sort().values, torch.arange(T * top, dtype=torch.int32))
+        assert torch.equal(rows.cpu().view(-1)[order.long().cpu()], torch.arange(T * top, dtype=torch.int32))
+        assert torch.equal(ge.cpu().view(-1)[order.long().cpu()].sort().values, ge.cpu().view(-1)[order.long().cpu()])
+        assert torch.equal(offs.cpu()[1:], torch.bincount(ge.cpu().view(-1).long(), minlength=E).cumsum(0).int())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("E,top,groups,keep,best,W,T", [(16, 1, 1, 1, 1, 7712, 17), (32, 4, 4, 2, 1, 2048, 16), (32, 32, 4, 4, 2, 4616, 4097),
                                                         (33, 8, 3, 2, 2, 1312, 9), (64, 5, 8, 4, 1, 1920, 4100), (192, 64, 4, 2, 2, 808, 5)])
