@@ -143,6 +143,10 @@ __global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(Nar
   const int mt = (a.M + TM - 1) / TM, id = xcd_remap(blockIdx.x, gridDim.x), m0 = id % mt * TM, n0 = id / mt * TN;
   const int all = (a.K + 63) / 64, first = (int)((int64_t)all * blockIdx.y / a.parts);  // steps of 64: of K, and of this part
   const int steps = (int)((int64_t)all * (blockIdx.y + 1) / a.parts) - first, rounds = (steps + U - 1) / U;
+  // Rows that lie a multiple of 8 KB apart meet in a memory channel at each step of K, in all workgroups at once: each begins elsewhere.
+  // (Not where two of them share weights. 64 rows by [28672, 4096] 54.5 -> 47.9 us, [8192, 8192] 39.9 -> 32.7; 28 KB apart, 4096 by
+  // 14336, 30.5 -> 33.7.)
+  const int rot = TN == 128 && BK && mt == 1 && a.ldb % 4096 == 0 ? id * 7 % steps : 0;
   A oa;
   B ob;
   oa.init(a.a, a.abytes, a.lda, m0, lane, wid);
@@ -152,7 +156,8 @@ __global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(Nar
   auto move = [&](int r, auto b_c) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int kq = first + min(r * U + u, steps - 1);
+      int kq = min(r * U + u, steps - 1) + rot;
+      kq = first + (kq >= steps ? kq - steps : kq);
       const uint32_t to = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)buffer(b_c) + STEP * u);
       oa.move(kq, to);
       ob.move(kq, to + A::BYTES);
@@ -272,6 +277,9 @@ struct Cut {
 // Both operands along K (y): 32 x 32 up to two tiles a CU (128 tokens by [3072, 1024] 6.4 / 6.4, [4096, 2048] 9.0 / 9.4, [5632, 1024] 8.6 / 6.7), 128 x
 // 128 from 140 of them on (512 by [5632, 1024] 13.7 with 64, 12.7; 768 by [3072, 1024], 144 of them, 13.8, 12.1; 256 by [8000, 1024], 126, 9.8, 12.2). Parts
 // of 2560 or more of K: a sum costs 2 us and its traffic (64 by [2048, 5632] 12.6, x2 10.5; [1024, 2816] 7.7, 7.7).
+// From K = 4096 on weights come from memory and a CU's share of the operands bounds: 128 x 128 tiles, in parts of 768 or more, where those make
+// 192 to 256 workgroups (128 by [4096, 14336] 63.9 with 64x1, 34.8 with 128x8; by [6144, 4096] 22.2, 128x5 20.7; but 256 by [4096, 4096] 21.2
+// with 64x1, 128x4 22.4), else 64 x 64 in parts of 1024 or more (128 by [2048, 5632] 18.2 with 32x2, 13.9; by [1024, 8192] 18.4, 13.1).
 // One across (dX): those rows come in runs of 64 columns, never 32 (half a cache line). 64 x 64 from 160 tiles on, of long K from 64
 // (256 tokens by [5632, 1024] 32x2 13.0, 64x4 11.8; 512 17.5, 64x2 15.8; by [3072, 1024] 9.5, 10.5). Parts of 768 up to a workgroup a CU
 // (128 by [3072, 1024] 10.6, x2 9.4, x4 8.9; by [1024, 1024] 5.3, 6.4, 6.9).
@@ -282,11 +290,22 @@ Cut cut_of(int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) {
   int tm = 32, tn = along ? 32 : 64;
   if (tiles(128, 128) >= (across ? 176 : 140) && (along || across)) tm = tn = 128;
   else if (along ? tiles(32, 32) > 512 : across || tiles(64, 64) >= (K >= 4096 ? 64 : 160)) tm = tn = 64;
+  int64_t parts = 0;
+  if (along && K >= 4096) {
+    const int64_t big = tiles(128, 128), mid = tiles(64, 64), cut = std::min<int64_t>(256 / std::max<int64_t>(big, 1), 8);
+    if (cut >= 2 && cut * big >= 192 && K / cut >= 768 && (K >= 8192 || mid <= 224 || mid > 256)) {
+      tm = tn = 128;
+      parts = cut;
+    } else if (mid >= (K >= 8192 ? 32 : 64) && mid <= 128) {
+      tm = tn = 64;
+      parts = std::min<int64_t>(std::min<int64_t>(256 / mid, K / 1024), 8);
+    }
+  }
   if (g_tile) {
     tm = g_tile;
     tn = g_tile == 32 && !along ? 64 : g_tile;
   }
-  int64_t parts = std::min<int64_t>(std::min<int64_t>((along ? 512 : 256) / tiles(tm, tn), K / (along ? 2560 : 768)), 8);
+  if (!parts || g_tile) parts = std::min<int64_t>(std::min<int64_t>((along ? 512 : 256) / tiles(tm, tn), K / (along ? 2560 : 768)), 8);
   if (g_parts) parts = std::min<int64_t>(g_parts, (K + 63) / 64);
   return {tm, tn, (int)std::max<int64_t>(parts, 1)};
 }
@@ -305,7 +324,9 @@ extern "C" int ds_narrow_gemm_ok(int64_t M, int64_t N, int64_t K, int64_t lda, i
   return (ar + 128) * lda * 2 < UINT32_MAX && (br + 128) * ldb * 2 < UINT32_MAX && ((M + 31) / 32) * ((N + 31) / 32) <= INT32_MAX;
 }
 
-// Whether it is as fast as the library's there, us here (there); up to 1024 tokens. y: 2^31 products, of up to 2^24 weights 2^32 (512 tokens by
+// Whether it is as fast as the library's there, us here (there); up to 1024 tokens. y: of K from 4096 on in three parts or more up to 128 tokens, in two
+// up to 256 (128 by [4096, 14336] 36 (75), [6144, 4096] 21 (25), [8192, 8192] 38 (50), 64 33 (34); 256 by [5120, 13824] 58 (120), [8192, 8192] 55 (78);
+// 64 by [12288, 4096] in two 28.7 (26.7)); else 2^31 products, of up to 2^24 weights 2^32 (512 tokens by
 // [8000, 1024] 13.7 (16.0); 128 by [11264, 2048] 21.6 (18.1); 1024 by [5632, 1024], 1.4 times 2^32, 23 (20.2)). dX: 3 2^32 and fewer than 3 2^20
 // results (512 by [11264, 2048] 61 (76), by [5632, 1024] 15.9 (25.3); 768 by [4096, 4096] 52 (42), 512 by [1024, 8192] 16.9 (15.2); 1500 by [4096, 2048]
 // 45 (35)). dW: 2^22 weights, 2^23 from up to 224 tokens (1024 by [3072, 1024] 13.3 (15.5); 200 by [8000, 1024] 14.5 (14.3), 256 15.2 (12.6)).
@@ -313,6 +334,7 @@ extern "C" int ds_narrow_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along,
   if ((a_along ? M : K) > 1024) return 0;
   if (!a_along) return M * N <= (K <= 224 ? 1 << 23 : 1 << 22);
   if (!b_along) return M * N < (3 << 20) && M * N <= (3LL << 32) / K;
+  if (K >= 4096 && M <= 256 && cut_of(M, N, K, true, true).parts >= (M <= 128 ? 3 : 2)) return 1;
   return M * N <= (1LL << (N * K <= (1 << 24) ? 32 : 31)) / K;
 }
 

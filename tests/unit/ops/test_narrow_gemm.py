@@ -48,6 +48,20 @@ def test_products_at_their_edges(M, N, K, tile, parts):
 
 
 @GPU
+@pytest.mark.parametrize("M,N,K", [(52, 6152, 4096), (1, 6144, 4096), (128, 6200, 4160), (129, 4104, 8192), (256, 5120, 5120), (100, 2056, 5632),
+                                   (33, 1024, 8192), (255, 4096, 4096), (300, 4096, 4160)])
+def test_long_inner_dimensions(M, N, K):
+    """Tiles and parts as the rule chooses them for K from 4096 on: 128 x 128 (rows a multiple of 8 KB apart begin elsewhere in K, unless
+    tiles share weights) and 64 x 64, and beyond them; the same bits each time."""
+    ops = hip_ops()
+    a, b = _rnd(M, K, seed=1), _rnd(N, K, seed=2)
+    got = ops.narrow_gemm(a, b, True, True)
+    _check(got, a, b)
+    assert torch.equal(got, ops.narrow_gemm(a, b, True, True))
+    _check(plain_linear(a, b), a, b)
+
+
+@GPU
 def test_values_that_do_not_mix():
     """Infinities and NaN stay in their rows; nothing from past the end of an operand comes in."""
     a, b = _rnd(40, 128), _rnd(48, 128, seed=1)
