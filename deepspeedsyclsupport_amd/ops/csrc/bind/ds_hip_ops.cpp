@@ -8,6 +8,8 @@
 #include <ATen/hip/HIPContext.h>
 #include <hip/hip_runtime_api.h>
 
+#include "narrow_bind.h"
+
 #include <optional>
 #include <vector>
 
@@ -64,11 +66,6 @@ int ds_flash_bwd(const void*, const void*, const void*, const void*, const void*
                  void*, void*, int, int, int, int, const int64_t*, const int64_t*, const int64_t*, const int64_t*,
                  const int64_t*, const int64_t*, const int64_t*, const int64_t*, float, int, float*, hipStream_t);
 int ds_transpose16(const void*, void*, int, int, int, int64_t, hipStream_t);
-int ds_narrow_gemm_ok(int64_t, int64_t, int64_t, int64_t, int64_t, int, int);
-int64_t ds_narrow_gemm_scratch(int64_t, int64_t, int64_t, int, int);
-int ds_narrow_gemm_pays(int64_t, int64_t, int64_t, int, int);
-int ds_narrow_gemm(const void*, const void*, void*, int64_t, int64_t, int64_t, int64_t, int64_t, int, int, void*, hipStream_t);
-void ds_narrow_gemm_tune(int, int);
 int ds_xent_fwd(const void*, const int64_t*, float*, float*, int64_t, int, int64_t, int, float, int, hipStream_t);
 int ds_xent_mean(const float*, const int64_t*, float*, float*, int64_t, int, hipStream_t);
 int ds_xent_bwd(const void*, const int64_t*, const float*, const float*, float, const float*, void*, int64_t, int, int64_t, int64_t,
@@ -545,58 +542,10 @@ Tensor xent_bwd(Tensor logits, Tensor labels, Tensor lse, OptT dloss, double dlo
 // out [B,S,Hq,128] so the o_proj GEMM reads it without a transpose copy, lse [B,Hq,S] fp32).
 // x [R, C] (16-bit, unit last stride) -> x^T contiguous [C, Rp] at HBM speed (K-major wgrad GEMM operands);
 // pad_to > R appends zero columns (the contraction dimension rounded up for the GEMM)
-// No transform, dispatch mode, tracer or autocast has to see what becomes of these tensors, and none carries a tangent or a lazy bit
-bool unseen(std::initializer_list<const Tensor*> ts) {
-  using K = c10::DispatchKey;
-  static const c10::DispatchKeySet special({K::Python, K::PythonTLSSnapshot, K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Batched,
-                                            K::Functionalize, K::Conjugate, K::Negative, K::ZeroTensor});
-  if (!(c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty() || at::autocast::is_autocast_enabled(at::kCUDA))
-    return false;
-  for (const Tensor* t : ts)
-    if (t->defined() && (t->key_set().has_any(special) || t->_fw_grad(0).defined())) return false;
-  return true;
-}
-// ... nor autograd
-bool unwatched(const Tensor& a, const Tensor& b) {
-  return !(at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad())) && unseen({&a, &b});
-}
-
-// A B^T over the inner dimension: a [M, K], or [K, M] if not a_along; b [N, K], or [K, N]. Undefined where the kernel does not take it
-// or (unless asked to take what it can) the library's is faster.
-Tensor narrow_product(const Tensor& a, const Tensor& b, bool a_along, bool b_along, bool any) {
-  if (!a.is_cuda() || a.device() != b.device() || a.scalar_type() != at::kBFloat16 || b.scalar_type() != at::kBFloat16 || a.dim() != 2 || b.dim() != 2 ||
-      a.stride(1) != 1 || b.stride(1) != 1)
-    return Tensor();
-  const int64_t M = a.size(a_along ? 0 : 1), K = a.size(a_along ? 1 : 0), N = b.size(b_along ? 0 : 1);
-  const int64_t lda = a.size(0) > 1 ? a.stride(0) : a.size(1), ldb = b.size(0) > 1 ? b.stride(0) : b.size(1);
-  if (b.size(b_along ? 1 : 0) != K || !ds_narrow_gemm_ok(M, N, K, lda, ldb, a_along, b_along) || (!any && !ds_narrow_gemm_pays(M, N, K, a_along, b_along)))
-    return Tensor();
-  const char *pa = (const char*)a.const_data_ptr(), *pb = (const char*)b.const_data_ptr();
-  if ((uintptr_t)pa % 16 || (uintptr_t)pb % 16) return Tensor();
-  Tensor c = torch::empty({M, N}, a.options());
-  const int64_t scratch = ds_narrow_gemm_scratch(M, N, K, a_along, b_along);
-  const Tensor part = scratch ? torch::empty({scratch}, a.options().dtype(at::kByte)) : Tensor();
-  check(ds_narrow_gemm(pa, pb, c.data_ptr(), M, N, K, lda, ldb, a_along, b_along, scratch ? part.data_ptr() : nullptr, stream()), "narrow_gemm");
-  return c;
-}
-
 Tensor narrow_gemm(Tensor a, Tensor b, bool a_along, bool b_along) {
   Tensor c = narrow_product(a, b, a_along, b_along, true);
   TORCH_CHECK(c.defined(), "narrow_gemm: bf16 matrices with contiguous, aligned rows and sizes that the kernel takes");
   return c;
-}
-
-// x [.., I] W [O, I]^T
-Tensor linear_product(Tensor x, Tensor w) {
-  if (unwatched(x, w) && x.dim() >= 2 && x.is_contiguous() && w.dim() == 2 && x.size(-1) == w.size(1) && x.numel()) {
-    const Tensor y = narrow_product(x.view({-1, x.size(-1)}), w, true, true, false);
-    if (y.defined()) {
-      auto sizes = x.sizes().vec();
-      sizes.back() = w.size(0);
-      return y.view(sizes);
-    }
-  }
-  return at::linear(x, w);
 }
 
 // dY [T, O] W [O, I]

@@ -1,5 +1,7 @@
-// Module of the bf16 decode products (up to 48 token rows) of the hybrid decoders, with activation epilogues.
+// Module of the bf16 products of the hybrid decoders: decode products (up to 48 token rows), with activation epilogues, and those of
+// short prompts.
 #include "bind_util.h"
+#include "narrow_bind.h"
 
 extern "C" {
 int ds_skinny_gemm(const void*, const void*, const void*, const void*, const void*, const void*, void*, void*, int, int,
@@ -84,4 +86,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_linear_sh_ok", &decode_linear_sh_ok);
   m.def("decode_linear_sh", &decode_linear_sh, py::arg("x"), py::arg("wsh"), py::arg("N"),
         py::arg("glu_limit") = py::none(), py::arg("act") = py::none());
+  m.def("linear", &linear_product);
 }

@@ -7,7 +7,7 @@ import torch
 import torch.nn.functional as F
 
 from . import mixer_ops, reference
-from .native import attn_ops, gemv_ops, hybrid_ops, use_native
+from .native import attn_ops, gemv_ops, hybrid_ops, unseen_from_python, use_native
 
 DECODE_ROWS = 16
 ACTS = {"gelu": 2}  # epilogue codes of the decode products (csrc/gemv/skinny_*.hip)
@@ -88,7 +88,7 @@ def delta_rule(proj, conv_w, a_log, dt_bias, norm_w, eps, state, conv_state, met
 
 def linear(x, w, sh=None, act=None):
     """x . w^T: a weight stream for decode-sized bf16 batches (over the shuffled copy `sh`, a `Bf16Weight`, from two
-    rows up), else the library product. act "gelu": the exact gelu of it (the stream's epilogue, else a pass of its own)."""
+    rows up), a narrow product for a short prompt, else the library's. act "gelu": the exact gelu of it (the stream's epilogue, else a pass of its own)."""
     rows = x.numel() // x.shape[-1]
     code = None if act is None else ACTS[act]
     if x.is_cuda and x.is_contiguous():
@@ -96,8 +96,12 @@ def linear(x, w, sh=None, act=None):
             return gemv_ops().decode_linear_sh(x, sh.wsh, sh.shape[0], act=code)
         if x.dtype == torch.bfloat16 and 0 < rows <= DECODE_ROWS and gemv_ops().decode_linear_ok(rows, x.shape[-1]):
             return gemv_ops().decode_linear(x, w, act=code)
-    y = F.linear(x, w)
+    y = _plain(x, w)
     return y if act is None else mixer_ops.gelu(y)
+
+
+def _plain(x, w):
+    return gemv_ops().linear(x, w) if x.is_cuda and unseen_from_python() else F.linear(x, w)
 
 
 def glu_linear(x, w, sh, limit):
@@ -108,4 +112,4 @@ def glu_linear(x, w, sh, limit):
             return gemv_ops().decode_linear_sh(x, sh.wsh, sh.shape[0], limit)
         if 0 < rows <= DECODE_ROWS and gemv_ops().decode_linear_ok(rows, x.shape[-1]):
             return gemv_ops().decode_linear(x, w, limit)
-    return clamped_glu(F.linear(x, w), limit)
+    return clamped_glu(_plain(x, w), limit)

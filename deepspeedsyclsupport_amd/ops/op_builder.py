@@ -61,13 +61,14 @@ EXTENSIONS = {
                      "bind/comm_bind.cpp", "bind/attn_small_bind.cpp"],
     },
     # what serving the hybrid decoders (inference/model_implementations/hybrid.py) needs, mechanism by mechanism: in a fresh
-    # checkout such a model starts after compiling the decode products and the sources of what it is made of
+    # checkout such a model starts after compiling the products and the sources of what it is made of
     "ds_gemv_ops": {
         "kind": "hip",
         "kernels": [
             "gemv/skinny_gemm.hip",
             "gemv/skinny_mfma.hip",
             "gemv/skinny_bf16_sh.hip",
+            "gemm/narrow_gemm.hip",
         ],
         "bindings": ["bind/gemv_bind.cpp"],
     },

@@ -128,3 +128,15 @@ def test_linear_layer_leaves_what_it_does_not_take():
         same(_rnd(4096, 1024), _rnd(1024, 1024))
         x, w = _rnd(16, 64), _rnd(32, 64, seed=1)
         torch.testing.assert_close(plain_linear(x, w).float(), F.linear(x, w).float(), rtol=2**-6, atol=2**-4)
+
+
+@GPU
+@pytest.mark.parametrize("T,W,N", [(49, 256, 512), (100, 4096, 6144), (200, 2048, 2048), (1500, 256, 256)])
+def test_products_of_hybrid_decoders(T, W, N):
+    """Short prompts of the hybrid decoders take the same products, longer ones and fp32 torch's."""
+    from deepspeedsyclsupport_amd.ops import hybrid_ops
+    x, w = _rnd(T, W, seed=1), _rnd(N, W, seed=2)
+    _check(hybrid_ops.linear(x, w), x, w)
+    if T <= 256:
+        assert torch.equal(hybrid_ops.linear(x, w), hip_ops().narrow_gemm(x, w, True, True))
+    assert torch.equal(hybrid_ops.linear(x.float(), w.float()), F.linear(x.float(), w.float()))
