@@ -98,6 +98,7 @@ struct SmallArgs {
   float* part;     // ... whose sums go here [nsplit, Z / b2_div, H, S, S] when they are several
   T* order;        // backward: the pair bias in the accumulators' order (small_order_elements), or null
   int Sk;          // keys (the forward may attend to a context of another length; the backward needs Sk == S)
+  int db2_as_in;   // with several parts: db2 is of the inputs' type, rounded once
 };
 
 // 4 consecutive 16-bit values (8-B aligned) added to f as fp32 / stored from fp32
@@ -1206,7 +1207,10 @@ __global__ void __launch_bounds__(NTHR, 2) small_bwd_db2_kernel(SmallArgs<T> a) 
       __builtin_amdgcn_sched_barrier(0);
       f32x16_t s, dp;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) { s[r] = 0.f; dp[r] = 0.f; }
+      for (int r = 0; r < 16; ++r) {
+        s[r] = 0.f;
+        dp[r] = DROP ? 0.f : -delta_n;  // (a vector instruction a score less: [256, 256, 4, 32] 38.0 -> 37.3 us)
+      }
 #pragma unroll
       for (int kk = 0; kk < D / 16; ++kk) {
         const V8 kv = *reinterpret_cast<const V8*>(buf + (t * 32 + l32) * RS<D>() + (2 * kk + h) * 16);
@@ -1226,7 +1230,7 @@ __global__ void __launch_bounds__(NTHR, 2) small_bwd_db2_kernel(SmallArgs<T> a) 
           const int r = 4 * g + i;
           const float p = __builtin_amdgcn_exp2f((s[r] * a.scale + (b1[i] + (float)b2[t][g][i]) - lse_n) * LOG2E);
           if constexpr (DROP) dp[r] *= ((kb >> i) & 1u) ? inv_keep : 0.f;
-          acc[t][r] += p * (dp[r] - delta_n);
+          acc[t][r] += p * (DROP ? dp[r] - delta_n : dp[r]);
         }
       }
     }
@@ -1259,8 +1263,11 @@ __global__ void __launch_bounds__(NTHR, 2) small_bwd_db2_kernel(SmallArgs<T> a) 
 
 // out[i] = sum over s of part[s][i], in a fixed order: a wave's lanes have four results each, its workgroup's waves a quarter of the parts,
 // eight of them on their way at once (a thread to itself waited for one part after the other: 64 parts of [8, 32, 32] 20 us, now 7; 16 of
-// [4, 256, 256] 5.8 and 4.8)
-__global__ void __launch_bounds__(256) sum_parts_kernel(const float* __restrict__ part, float* __restrict__ out, int64_t n, int parts) {
+// [4, 256, 256] 5.8 and 4.8). O: float, or the inputs' type, where that is the gradient's (a launch of 4 us for the cast less: forward and
+// backward of [256, 256, 4, 32] 154 -> 149 us)
+template <typename O>
+__global__ void __launch_bounds__(256) sum_parts_kernel(const float* __restrict__ part, O* __restrict__ out, int64_t n, int parts) {
+  typedef O O4 __attribute__((ext_vector_type(4)));
   __shared__ f32x4 sums[4][64];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, lo = parts * wid / 4, hi = parts * (wid + 1) / 4;
   const int64_t i = ((int64_t)blockIdx.x * 64 + lane) * 4;
@@ -1292,11 +1299,11 @@ __global__ void __launch_bounds__(256) sum_parts_kernel(const float* __restrict_
 #pragma unroll
   for (int w = 1; w < 4; ++w) sum += sums[w][lane];
   if (whole) {
-    if (i < n) *reinterpret_cast<f32x4*>(out + i) = sum;
+    if (i < n) *reinterpret_cast<O4*>(out + i) = O4{(O)sum[0], (O)sum[1], (O)sum[2], (O)sum[3]};
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (i + e < n) out[i + e] = sum[e];
+      if (i + e < n) out[i + e] = (O)sum[e];
   }
 }
 
@@ -1383,7 +1390,9 @@ int launch_small(SmallArgs<T> a, bool bwd, hipStream_t st) {
     DS_CHECK_LAUNCH();
     if (a.nsplit > 1) {
       const int64_t n = (int64_t)(a.Z / a.b2_div) * a.H * a.S * a.S;
-      hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a.part, a.db2, n, a.nsplit);
+      const dim3 g4((unsigned)((n + 255) / 256));
+      if (a.db2_as_in) hipLaunchKernelGGL(sum_parts_kernel<T>, g4, dim3(256), 0, st, a.part, (T*)a.db2, n, a.nsplit);
+      else hipLaunchKernelGGL(sum_parts_kernel<float>, g4, dim3(256), 0, st, a.part, a.db2, n, a.nsplit);
       DS_CHECK_LAUNCH();
     }
   }
@@ -1433,7 +1442,7 @@ extern "C" int ds_flash_small_fwd(const void* q, const void* k, const void* v, v
 
 // Backward. strides[18] = (q)(k)(v)(o)(dO)(dQ); dk / dv dense [Z, S, H, D] in the input dtype; delta fp32 [Z, H, S]
 // scratch; db1 [Z, S] fp32 (zeroed by the caller) or null; db2 [Z / b2_div, H, S, S] fp32 (fully written) or null, db2_part
-// `ds_flash_small_db2_splits` times as much scratch when that is more than one.
+// `ds_flash_small_db2_splits` times as much scratch when that is more than one; then, with db2_as_in, db2 is of the inputs' type.
 extern "C" int ds_flash_small_db2_splits(int Z, int H, int S, int b2_div) { return db2_splits(Z, H, S, b2_div); }
 
 // order: ds_flash_small_order elements of the inputs' type when that is not zero
@@ -1443,7 +1452,8 @@ extern "C" int64_t ds_flash_small_order(int Z, int H, int S, int D, int b2_div, 
 
 extern "C" int ds_flash_small_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout,
                                   const float* lse, const void* b1, const void* b2, void* dq, void* dk, void* dv,
-                                  float* delta, float* db1, float* db2, float* db2_part, void* order, const int64_t* st, int64_t b1_zs, int Z, int H, int S, int D,
+                                  float* delta, float* db1, float* db2, float* db2_part, int db2_as_in, void* order,
+                                  const int64_t* st, int64_t b1_zs, int Z, int H, int S, int D,
                                   int b2_div, float scale, float pdrop, uint64_t seed, int64_t b2_numel, int dtype,
                                   hipStream_t stream) {
   if (Z <= 0 || H <= 0 || S <= 0 || b2_div <= 0 || (D != 32 && D != 64) || pdrop < 0.f || pdrop >= 1.f ||
@@ -1454,7 +1464,7 @@ extern "C" int ds_flash_small_bwd(const void* q, const void* k, const void* v, c
   SmallArgs<T> a{(const T*)q, (const T*)k, (const T*)v, (const T*)o, (const T*)dout, (T*)dq, (float*)lse,           \
                  (const T*)b1, (const T*)b2, (T*)dk, (T*)dv, delta, db1, db2, st[0], st[1], st[2], st[3], st[4], st[5], st[6],      \
                  st[7], st[8], st[9], st[10], st[11], st[12], st[13], st[14], st[15], st[16], st[17], b1_zs, Z, H, S, b2_div, scale, pdrop, \
-                 thresh, seed, b2_numel - 8, 1, db2_part, (T*)order, S};
+                 thresh, seed, b2_numel - 8, 1, db2_part, (T*)order, S, db2_as_in};
   if (dtype == DS_BF16) {
     DS_SMALL_ARGS(bf16)
     return dispatch_small<bf16>(a, D, true, stream);

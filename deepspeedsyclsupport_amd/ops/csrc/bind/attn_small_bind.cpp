@@ -12,7 +12,7 @@ int ds_flash_small_fwd(const void*, const void*, const void*, void*, float*, con
                        const int64_t*, int64_t, int, int, int, int, int, int, float, float, uint64_t, int64_t, int,
                        hipStream_t);
 int ds_flash_small_bwd(const void*, const void*, const void*, const void*, const void*, const float*, const void*,
-                       const void*, void*, void*, void*, float*, float*, float*, float*, void*, const int64_t*, int64_t, int, int, int,
+                       const void*, void*, void*, void*, float*, float*, float*, float*, int, void*, const int64_t*, int64_t, int, int, int,
                        int, int, float, float, uint64_t, int64_t, int, hipStream_t);
 int64_t ds_flash_small_order(int, int, int, int, int, float, int);
 int ds_flash_small_db2_splits(int, int, int, int);
@@ -105,10 +105,10 @@ std::vector<Tensor> flash_small_fwd(Tensor q, Tensor k, Tensor v, OptT b1, OptT 
 }
 
 // Returns dq (contiguous, q dtype), dk, dv (q dtype), db1 [Z, S] fp32 / db2 [Z / b2_div, H, S, S] fp32 (empty when
-// not requested).
+// not requested). db2_as_in: db2 in q's type where it is summed from parts (else the caller's cast is the shorter way).
 std::vector<Tensor> flash_small_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, OptT b1,
                                     OptT b2, int64_t b2_div, double scale, double pdrop, int64_t seed, bool want_db1,
-                                    bool want_db2) {
+                                    bool want_db2, bool db2_as_in) {
   operand(q, q, "q");
   operand(k, q, "k");
   operand(v, q, "v");
@@ -127,10 +127,11 @@ std::vector<Tensor> flash_small_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, T
   auto dv = torch::empty({Z, S, H, D}, q.options());
   const int64_t order_n = ds_flash_small_order((int)Z, (int)H, (int)S, (int)D, (int)b2_div, (float)pdrop, bs.b2 != nullptr);
   Tensor db1 = want_db1 ? torch::zeros({Z, S}, f32) : torch::empty({0}, f32);
-  Tensor db2 = want_db2 ? torch::empty({Z / b2_div, H, S, S}, f32) : torch::empty({0}, f32);
   // delta, the parts of db2 and the ordered pair bias in one allocation: the host bounds calls of up to some 150 us ([74, 197, 4, 32]
   // forward and backward 3 % slower with three)
   const int splits = want_db2 ? ds_flash_small_db2_splits((int)Z, (int)H, (int)S, (int)b2_div) : 1;
+  db2_as_in = db2_as_in && splits > 1;
+  Tensor db2 = want_db2 ? torch::empty({Z / b2_div, H, S, S}, db2_as_in ? q.options() : f32) : torch::empty({0}, f32);
   auto floats = [](int64_t n) { return (n + 63) / 64 * 64; };
   const int64_t delta_n = floats(Z * H * S), part_n = splits > 1 ? floats(splits * db2.numel()) : 0;
   Tensor scratch = torch::empty({delta_n + part_n + floats((order_n + 1) / 2)}, f32);
@@ -139,8 +140,8 @@ std::vector<Tensor> flash_small_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, T
   push(st, q); push(st, k); push(st, v); push(st, o); push(st, dout); push(st, dq);
   check(ds_flash_small_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dout.data_ptr(),
                            lse.data_ptr<float>(), bs.b1, bs.b2, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-                           delta, want_db1 ? db1.data_ptr<float>() : nullptr, want_db2 ? db2.data_ptr<float>() : nullptr,
-                           splits > 1 ? part : nullptr, order_n ? order : nullptr, st.data(), bs.b1_zs, (int)Z, (int)H, (int)S,
+                           delta, want_db1 ? db1.data_ptr<float>() : nullptr, want_db2 ? (float*)db2.data_ptr() : nullptr,
+                           splits > 1 ? part : nullptr, db2_as_in, order_n ? order : nullptr, st.data(), bs.b1_zs, (int)Z, (int)H, (int)S,
                            (int)D, (int)b2_div, (float)scale, (float)pdrop, (uint64_t)seed, bs.b2_numel, dcode(q),
                            at::hip::getCurrentHIPStream().stream()),
         "flash_small_bwd");
@@ -157,5 +158,5 @@ void register_attn_small_ops(pybind11::module& m) {
         pybind11::arg("v"), pybind11::arg("o"), pybind11::arg("lse"), pybind11::arg("b1") = pybind11::none(),
         pybind11::arg("b2") = pybind11::none(), pybind11::arg("b2_div") = 1, pybind11::arg("scale"),
         pybind11::arg("pdrop") = 0.0, pybind11::arg("seed") = 0, pybind11::arg("want_db1") = false,
-        pybind11::arg("want_db2") = false);
+        pybind11::arg("want_db2") = false, pybind11::arg("db2_as_in") = false);
 }

@@ -57,7 +57,8 @@ class FlashSmallFunc(torch.autograd.Function):
         q, k, v, o, lse, b1, b2 = ctx.saved_tensors
         b2_div, scale, pdrop, seed = ctx.cfg
         dq, dk, dv, db1, db2 = hip_ops().flash_small_bwd(_fix(do), q, k, v, o, lse, b1, b2, b2_div, scale, pdrop,
-                                                         seed, ctx.want[0], ctx.want[1])
+                                                         seed, ctx.want[0], ctx.want[1],
+                                                         ctx.want[1] and b2.dtype == q.dtype)
         db1 = db1.to(b1.dtype) if ctx.want[0] else None
         db2 = db2.to(b2.dtype) if ctx.want[1] else None
         return dq, dk, dv, db1, db2, None, None, None, None

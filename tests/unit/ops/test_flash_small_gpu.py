@@ -332,6 +332,21 @@ def test_finite_masks_backward(S, mask):
         assert (a.double().abs()[~some] <= 1.02 * m[~some] + 1e-3).all(), name
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("Z,S,H,N", [(64, 40, 4, 64), (16, 37, 3, 8), (40, 131, 1, 40), (6, 33, 2, 3), (4, 24, 2, 1)])
+def test_pair_bias_gradient_in_the_inputs_type(dtype, Z, S, H, N):
+    """Sums of several parts leave in the inputs' type as they would after a cast, at lengths whose square 4 divides and does not;
+    where there is one part, or none, they stay in fp32."""
+    from deepspeedsyclsupport_amd.ops.native import hip_ops
+    g = torch.Generator(device="cuda").manual_seed(0)
+    q, k, v, do = (torch.randn(Z, S, H, 32, device="cuda", generator=g).to(dtype) for _ in range(4))
+    b2 = torch.randn(Z // N, H, S, S, device="cuda", generator=g).to(dtype)
+    o, lse = hip_ops().flash_small_fwd(q, k, v, None, b2, N, 0.2, 0.0, 0)
+    plain, cast = (hip_ops().flash_small_bwd(do, q, k, v, o, lse, None, b2, N, 0.2, 0.0, 0, False, True, c)[4] for c in (False, True))
+    assert plain.dtype == torch.float32 and cast.dtype == (dtype if N >= 8 else torch.float32)
+    assert torch.equal(plain.to(dtype), cast.to(dtype))
+
+
 @pytest.mark.parametrize("dtype,unit", [(torch.bfloat16, 2.0**-8), (torch.float16, 2.0**-11)], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("S,top", [(64, 40), (250, 100), (256, 255)])
 def test_largest_weight_is_exact(dtype, unit, S, top):
