@@ -67,10 +67,8 @@ Tensor decode_linear_sh(Tensor x, Tensor wsh, int64_t N, std::optional<double> g
 }
 // Whether decode_linear_sh takes a product and is the faster one. Every workgroup reads all of x, or its part of it: over deep
 // contractions that are not cut the library's blocking wins from 17 rows on ([4096, 14336] uncut, us: 24 rows 30 here, 29 there; 40
-// rows 41 and 33; cut 25 and 27.5), over short ones the stream up to its 48 ([2048, 5632], 40 rows: 13 and 15; [14368, 4096] 32 rows 26
-// and 27, 48 rows 28.7 and 28.0). Few blocks of 2048 to 4096 columns are the library's from 33 rows on by the kernel ([2048, 3072] 40
-// rows 11.8 and 10.2), not in a decode step, which its call on the host holds up: 40 sequences of a 2048-wide hybrid 520 us a step, 570
-// with that product in the library.
+// rows 41 and 33; cut 25 and 27.5), over short ones the stream up to its 48 ([14368, 4096] 32 rows 26 and 27, 48 rows 25 and 28.0; [2048,
+// 5632], 40 rows: 11.4 and 15).
 bool decode_linear_sh_ok(int64_t M, int64_t N, int64_t K, bool glu) {
   if (M > 48 || K >= ((int64_t)1 << 31) || !ds_decode_gemm_ok((int)M, (int)K) || (glu && N % 2)) return false;
   if (M <= 16) return true;

@@ -38,7 +38,20 @@ struct NarrowArgs {
   uint32_t lda, ldb, abytes, bbytes;
   int parts;               // of K, each with workgroups of its own (1: all of it)
   f32x4* part;             // their sums [parts][M][N] (null: the result leaves from here)
+  const bf16 *bias, *res;  // behind a product with an ordered operand: [N] or null, [M, N] or null
+  int act;                 // ... an activation code + DS_ACT_UNARY, or -1
 };
+
+// Columns n .. n + 3 of row m: bias, activation, residual
+__device__ __forceinline__ f32x4 behind(const NarrowArgs& a, f32x4 v, int64_t m, int n) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (a.bias) v[i] += (float)a.bias[n + i];
+    if (a.act >= 0) v[i] = act_any(a.act - DS_ACT_UNARY, v[i]);
+    if (a.res) v[i] += (float)a.res[m * a.N + n + i];
+  }
+  return v;
+}
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
@@ -66,7 +79,11 @@ __device__ __forceinline__ void meet() {
 }
 
 // One operand's R rows (or columns) of a step of 64: its way into LDS and out of it
-template <bool ALONG, int R>
+// How an operand lies: its rows across the inner dimension, along it, or in operand order (blocks of 16 rows, of which 64 columns at a time are
+// 2 KB: `preshuffle16` of ops/bf16_gemv.py)
+enum : int { ACROSS = 0, ALONG = 1, ORDERED = 2 };
+
+template <int LAY, int R>
 struct Operand {
   static constexpr int BYTES = R * 128, PIECES = R / 32;  // LDS bytes a step, transfers of 1 KB a wave
   i32x4 from;
@@ -75,12 +92,14 @@ struct Operand {
 
   __device__ __forceinline__ void init(const bf16* p, uint32_t bytes, uint32_t ld, int r0, int lane, int wid) {
     from = buffer_of(p, bytes);
-    step = ALONG ? 128 : 128 * ld;
+    step = LAY == ORDERED ? 2048 : LAY == ALONG ? 128 : 128 * ld;
     dst = wid * PIECES * 1024;
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
       const int piece = wid * PIECES + i;
-      if constexpr (ALONG) {  // 8 rows of 8 chunks: chunk c of row r at c ^ (r / 2 % 8)
+      if constexpr (LAY == ORDERED) {  // half a block as it lies: chunk 2 q + h of its row r at 64 h + 16 q + r
+        src[i] = (uint32_t)((r0 >> 4) + (piece >> 1)) * 32 * ld + 1024 * (piece & 1) + 16 * lane;
+      } else if constexpr (LAY == ALONG) {  // 8 rows of 8 chunks: chunk c of row r at c ^ (r / 2 % 8)
         const int r = 8 * piece + (lane >> 3);
         src[i] = (uint32_t)(r0 + r) * ld * 2 + 16 * ((lane & 7) ^ ((r >> 1) & 7));
       } else {  // R / 8 chunks of a step's 64 / PIECES / 4 rows each, those of row r swizzled by `turn`
@@ -101,7 +120,11 @@ struct Operand {
   template <bool PLAIN>
   __device__ __forceinline__ bf16x8 read(const lds_char* buf, int j, int r0, int lane) const {
     const int l32 = lane & 31, h = lane >> 5;
-    if constexpr (ALONG) {
+    if constexpr (LAY == ORDERED) {
+      static_assert(PLAIN, "beside rows along the inner dimension");
+      const int r = r0 + l32;
+      return *reinterpret_cast<const lds_bf16x8*>(buf + (r >> 4) * 2048 + h * 1024 + (j * 16 + (r & 15)) * 16);
+    } else if constexpr (LAY == ALONG) {
       const int r = r0 + l32, sw = (r >> 1) & 7;
       if constexpr (PLAIN) return *reinterpret_cast<const lds_bf16x8*>(buf + r * 128 + 16 * ((2 * j + h) ^ sw));
       const bf16x4 lo = *reinterpret_cast<const lds_bf16x4*>(buf + r * 128 + 16 * ((2 * j) ^ sw) + 8 * h);
@@ -128,8 +151,8 @@ __device__ __forceinline__ bf16x4 narrowed(f32x4 v) {
   return o;
 }
 
-// AK, BK: the operand's rows run along the inner dimension. TM x TN: tile of C. U: steps of 64 a buffer holds.
-template <bool AK, bool BK, int TM, int TN, int U>
+// AK, BK: how the operands lie. TM x TN: tile of C. U: steps of 64 a buffer holds.
+template <int AK, int BK, int TM, int TN, int U>
 __global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(NarrowArgs a) {
   typedef Operand<AK, TM> A;
   typedef Operand<BK, TN> B;
@@ -146,7 +169,7 @@ __global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(Nar
   // Rows that lie a multiple of 8 KB apart meet in a memory channel at each step of K, in all workgroups at once: each begins elsewhere.
   // (Not where two of them share weights. 64 rows by [28672, 4096] 54.5 -> 47.9 us, [8192, 8192] 39.9 -> 32.7; 28 KB apart, 4096 by
   // 14336, 30.5 -> 33.7.)
-  const int rot = TN == 128 && BK && mt == 1 && a.ldb % 4096 == 0 ? id * 7 % steps : 0;
+  const int rot = TN == 128 && BK == ALONG && mt == 1 && a.ldb % 4096 == 0 ? id * 7 % steps : 0;
   A oa;
   B ob;
   oa.init(a.a, a.abytes, a.lda, m0, lane, wid);
@@ -254,18 +277,24 @@ __global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(Nar
       out[0] = lo;
       out[1] = hi;
     } else {
+      if constexpr (BK == ORDERED) {
+        lo = behind(a, lo, m0 + m, n0 + n);
+        hi = behind(a, hi, m0 + m, n0 + n + 4);
+      }
       *reinterpret_cast<bf16x8*>(a.c + at) = __builtin_shufflevector(narrowed(lo), narrowed(hi), 0, 1, 2, 3, 4, 5, 6, 7);
     }
   }
 }
 
 // The parts' sums, always in the same order
-__global__ void __launch_bounds__(256) narrow_sum_kernel(const f32x4* __restrict__ part, bf16* __restrict__ c, int64_t n4, int parts) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+template <bool BEHIND>
+__global__ void __launch_bounds__(256) narrow_sum_kernel(NarrowArgs a) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, n4 = (int64_t)a.M * a.N / 4;
   if (i >= n4) return;
-  f32x4 v = part[i];
-  for (int p = 1; p < parts; ++p) v += part[p * n4 + i];
-  *reinterpret_cast<bf16x4*>(c + 4 * i) = narrowed(v);
+  f32x4 v = a.part[i];
+  for (int p = 1; p < a.parts; ++p) v += a.part[p * n4 + i];
+  if constexpr (BEHIND) v = behind(a, v, 4 * i / a.N, (int)(4 * i % a.N));
+  *reinterpret_cast<bf16x4*>(a.c + 4 * i) = narrowed(v);
 }
 
 int g_tile = 0, g_parts = 0;
@@ -354,30 +383,81 @@ extern "C" int ds_narrow_gemm(const void* A, const void* B, void* C, int64_t M, 
   else if (!part) return (int)hipErrorInvalidValue;
   const int64_t ar = a_along ? M : K, ac = a_along ? K : M, br = b_along ? N : K, bc = b_along ? K : N;
   const NarrowArgs a{(const bf16*)A, (const bf16*)B, (bf16*)C, (int)M, (int)N, (int)K, (uint32_t)lda, (uint32_t)ldb,
-                     (uint32_t)(((ar - 1) * lda + ac) * 2), (uint32_t)(((br - 1) * ldb + bc) * 2), cut.parts, (f32x4*)part};
+                     (uint32_t)(((ar - 1) * lda + ac) * 2), (uint32_t)(((br - 1) * ldb + bc) * 2), cut.parts, (f32x4*)part,
+                     nullptr, nullptr, -1};
   const dim3 grid((unsigned)(((M + cut.tm - 1) / cut.tm) * ((N + cut.tn - 1) / cut.tn)), cut.parts);
 #define GO(AK, BK, TM, TN, U) hipLaunchKernelGGL((narrow_gemm_kernel<AK, BK, TM, TN, U>), grid, dim3(256), 0, st, a)
   if (cut.tm == 128) {
-    if (a_along && b_along) GO(true, true, 128, 128, 1);
-    else if (a_along) GO(true, false, 128, 128, 1);
-    else if (b_along) GO(false, true, 128, 128, 1);
-    else GO(false, false, 128, 128, 1);
+    if (a_along && b_along) GO(ALONG, ALONG, 128, 128, 1);
+    else if (a_along) GO(ALONG, ACROSS, 128, 128, 1);
+    else if (b_along) GO(ACROSS, ALONG, 128, 128, 1);
+    else GO(ACROSS, ACROSS, 128, 128, 1);
   } else if (cut.tm == 64) {
-    if (a_along && b_along) GO(true, true, 64, 64, 1);
-    else if (a_along) GO(true, false, 64, 64, 1);
-    else if (b_along) GO(false, true, 64, 64, 1);
-    else GO(false, false, 64, 64, 1);
+    if (a_along && b_along) GO(ALONG, ALONG, 64, 64, 1);
+    else if (a_along) GO(ALONG, ACROSS, 64, 64, 1);
+    else if (b_along) GO(ACROSS, ALONG, 64, 64, 1);
+    else GO(ACROSS, ACROSS, 64, 64, 1);
   } else {
-    if (a_along && b_along) GO(true, true, 32, 32, 2);
-    else if (a_along) GO(true, false, 32, 64, 1);
-    else if (b_along) GO(false, true, 32, 64, 1);
-    else GO(false, false, 32, 64, 1);
+    if (a_along && b_along) GO(ALONG, ALONG, 32, 32, 2);
+    else if (a_along) GO(ALONG, ACROSS, 32, 64, 1);
+    else if (b_along) GO(ACROSS, ALONG, 32, 64, 1);
+    else GO(ACROSS, ACROSS, 32, 64, 1);
   }
 #undef GO
-  if (part) {
-    const int64_t n4 = M * N / 4;
-    hipLaunchKernelGGL(narrow_sum_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, (const f32x4*)part, (bf16*)C, n4, cut.parts);
-  }
+  if (part) hipLaunchKernelGGL(narrow_sum_kernel<false>, dim3((unsigned)((M * N / 4 + 255) / 256)), dim3(256), 0, st, a);
+  DS_CHECK_LAUNCH();
+  return 0;
+}
+
+namespace {
+// Decode batches of 33 to 48 rows by weights in operand order. Against ds_decode_gemm's kernels (eight waves that load what they multiply) the
+// transfers run three steps ahead without registers, a workgroup's tile has 64 weight rows (there 32, or 64 with a CU to itself) and
+// the parts' sums are as many rows as there are. 64 x 64 in parts up to a workgroup a CU, whole from 129 tiles on, 128 x 128 of long K there;
+// few blocks 32 x 32. us before and now, 48 rows: [1024, 4096] 10.5 / 7.8, [2048, 2048] 9.8 / 6.1, [4096, 2048] 10.1 / 7.6, [4096, 4096] 14.3 / 12.2, [5120,
+// 5120] 22.8 / 15.6, [2048, 5632] 13.0 / 11.6, [4096, 14336] 28.5 / 26.4, [10240, 8192] 39.6 / 37.0, [16384, 4096] 28.2 / 26.9.
+Cut ordered_cut(int64_t M, int64_t N, int64_t K) {
+  const int64_t mid = (N + 63) / 64, low = (M + 31) / 32 * ((N + 31) / 32), big = (N + 127) / 128;
+  auto parts = [&](int64_t tiles) { return (int)std::max<int64_t>(std::min<int64_t>(std::min<int64_t>(256 / tiles, K / 1024), 8), 1); };
+  Cut c = {32, 32, 1};
+  if (mid > 128) c = K >= 8192 ? Cut{128, 128, parts(big)} : Cut{64, 64, 1};
+  else if (K >= 3072) c = mid >= (K >= 8192 ? 32 : 64) ? Cut{64, 64, parts(mid)} : Cut{32, 32, parts(low)};
+  if (g_tile) c.tm = c.tn = g_tile;
+  if (g_parts) c.parts = (int)std::min<int64_t>(g_parts, K / 64);
+  return c;
+}
+}  // namespace
+
+// Whether ds_narrow_ordered takes x [M, K] by w [N, K] in operand order, and is the faster way. Not over short K from 4096 rows on (33 rows by [8192,
+// 2048] 11.3, before 10.4), nor where the weights' read is what counts ([16384, 8192] 55, before 49; [32000, 4096] 52.5, 53.5, with 33 rows 51
+// and 50). Up to 32 rows small products (24 by [2048, 2048] 6.0, before 6.9, [3072, 1024] 4.8, 5.4; [4096, 2048] 7.8, 7.3) and those a quarter over
+// one round of single blocks (24 by [5120, 5120] 14.4, 16.5).
+extern "C" int ds_narrow_ordered_ok(int64_t M, int64_t N, int64_t K) {
+  if (M > 48 || N <= 0 || N > 16384 || N % 8 || K <= 0 || K % 64 || N * K > (3 << 25)) return 0;
+  if (M > 32) return K >= 3072 || N <= 4096;
+  return (M > 20 && K <= 2048 && N * K <= (1 << 22)) || (M > 16 && N > 4096 && N <= 5440 && K >= 4096 && K < 8192);
+}
+
+extern "C" int64_t ds_narrow_ordered_scratch(int64_t M, int64_t N, int64_t K) {
+  const Cut c = ordered_cut(M, N, K);
+  return c.parts > 1 ? c.parts * M * N * 4 : 0;
+}
+
+// y [M, N] = act(x w^T + bias) + res, rows of x K apart; part: ds_narrow_ordered_scratch bytes
+extern "C" int ds_narrow_ordered(const void* X, const void* W, const void* bias, const void* res, void* Y, int64_t M, int64_t N, int64_t K, int act,
+                                 void* part, hipStream_t st) {
+  if (!ds_narrow_ordered_ok(M, N, K)) return (int)hipErrorInvalidValue;
+  const Cut cut = ordered_cut(M, N, K);
+  if (cut.parts == 1) part = nullptr;
+  else if (!part) return (int)hipErrorInvalidValue;
+  const NarrowArgs a{(const bf16*)X, (const bf16*)W, (bf16*)Y, (int)M, (int)N, (int)K, (uint32_t)K, (uint32_t)K, (uint32_t)(M * K * 2),
+                     (uint32_t)((N + 15) / 16 * 16 * K * 2), cut.parts, (f32x4*)part, (const bf16*)bias, (const bf16*)res, act};
+  const dim3 grid((unsigned)(((M + cut.tm - 1) / cut.tm) * ((N + cut.tn - 1) / cut.tn)), cut.parts);
+#define GO(TM, U) hipLaunchKernelGGL((narrow_gemm_kernel<ALONG, ORDERED, TM, TM, U>), grid, dim3(256), 0, st, a)
+  if (cut.tm == 128) GO(128, 1);
+  else if (cut.tm == 64) GO(64, 1);
+  else GO(32, 2);
+#undef GO
+  if (part) hipLaunchKernelGGL(narrow_sum_kernel<true>, dim3((unsigned)((M * N / 4 + 255) / 256)), dim3(256), 0, st, a);
   DS_CHECK_LAUNCH();
   return 0;
 }

@@ -51,16 +51,6 @@ struct ShArgs {
   f32x4* part;         // their sums [parts][blocks][MT][64], as the accumulators lie (null: the result leaves from here)
 };
 
-__device__ __forceinline__ float act_any(int a, float x) {
-  switch (a) {
-    case 0: return x / (1.f + __expf(-x));  // silu
-    case 1: return 0.5f * x * (1.f + tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x)));
-    case 2: return 0.5f * x * (1.f + erff(x * 0.7071067811865476f));
-    case 3: return fmaxf(x, 0.f);
-    default: return x;
-  }
-}
-
 template <int V>
 struct Int {
   static constexpr int value = V;
@@ -367,7 +357,9 @@ struct Cut {
 // without and with: [5120, 13824] 33 / 41 / 52 and 28 / 31 / 33, [8192, 8192] 27 / 29 / 35 and 28 / 28 / 31, [10240, 8192] 35 / 40 / 45
 // and 34 / 35 / 40; shorter ones stay whole ([7168, 7168] 21 / 24 and 23 / 24).
 // Up to 16 rows parts pay at the ends alone: where a few blocks leave most CUs idle (16 rows x [1024, 4096] 8.7 and 7.7, 2 rows 6.1 and
-// 6.9, x [1024, 8192] 9.6 and 8.4), and where long ones stand a quarter over one round (16 rows x [10240, 8192] 40 and 35).
+// 6.9, x [1024, 8192] 9.6 and 8.4), and where long ones stand a quarter over one round (16 rows x [10240, 8192] 40 and 35); from 12 rows on
+// also over long K, in two blocks, which halve the reading of X (12 / 16 rows x [2048, 5632] 10.4 / 11.7 and 9.5 / 9.7, [4096, 14336] 23.7 / 26.0 and 22.8 / 23.3,
+// [5120, 13824] 29.9 / 31.6 and 27.6 / 28.5, [3072, 8192] 13.9 / 15.4 and 14.0 / 14.4).
 Cut cut_of(int M, int N, int K, bool gated, bool norm) {
   const int blocks = gated ? N / 16 : (N + 15) / 16, mt = (M + 15) / 16, most = gated || mt > 1 ? 4 : 2;
   const int eights = (blocks + 7) / 8;  // workgroups of eight blocks
@@ -377,6 +369,10 @@ Cut cut_of(int M, int N, int K, bool gated, bool norm) {
     int fill = 0;  // workgroups that parts may make
     if (mt == 1) {
       fill = blocks <= 64 && (K >= 8192 || (M > 8 && K >= 4096)) ? 256 : blocks > 512 && blocks <= 680 && K >= 8192 ? 1024 : 0;
+      if (M >= 12 && blocks > 64 && blocks <= 340 && K >= (blocks <= 256 ? 5120 : 8192)) {
+        rb = 2;
+        fill = blocks <= 256 ? 256 : 512;
+      }
     } else if (blocks <= 256 && K >= 4096) {
       rb = mt == 3 && K >= 8192 ? 4 : 2;
       fill = 256;
@@ -421,8 +417,17 @@ extern "C" void ds_skinny_b16_tune(int cfg, int parts) { g_blocks = cfg; g_parts
 
 extern "C" int ds_decode_gemm_ok(int M, int K) { return M >= 1 && M <= 48 && K >= 64 && K % 64 == 0; }
 
+// Most products of 33 rows and more, and some of 17, without a norm or a gate: the narrow products' kernel over the same weights (gemm/narrow_gemm.hip)
+extern "C" int ds_narrow_ordered_ok(int64_t, int64_t, int64_t);
+extern "C" int64_t ds_narrow_ordered_scratch(int64_t, int64_t, int64_t);
+extern "C" int ds_narrow_ordered(const void*, const void*, const void*, const void*, void*, int64_t, int64_t, int64_t, int, void*, hipStream_t);
+static bool narrow_instead(int M, int N, int K, int gated, bool norm) {
+  return !gated && !norm && !g_blocks && !g_parts && ds_narrow_ordered_ok(M, N, K);
+}
+
 // Bytes of scratch memory that ds_decode_gemm wants for a product (0: none)
 extern "C" int64_t ds_decode_gemm_scratch(int M, int N, int K, int gated, int norm) {
+  if (narrow_instead(M, N, K, gated, norm)) return ds_narrow_ordered_scratch(M, N, K);
   const bool loose = gated && N % 32;
   const int parts = cut_of(M, N, K, gated && !loose, norm).parts;
   return parts > 1 || loose ? (int64_t)parts * ((N + 15) / 16) * ((M + 15) / 16) * 1024 : 0;
@@ -445,6 +450,7 @@ extern "C" int ds_decode_gemm(const void* X, const void* Wsh, const void* bias, 
                               void* Y, int M, int N, int K, int gated, int act, float limit, void* part, hipStream_t st) {
   const bool loose = gated && N % 32;
   if (!ds_decode_gemm_ok(M, K) || N <= 0 || (loose && (N % 2 || norm_w))) return (int)hipErrorInvalidValue;
+  if (narrow_instead(M, N, K, gated, norm_w != nullptr)) return ds_narrow_ordered(X, Wsh, bias, res, Y, M, N, K, act, part, st);
   if (loose) gated = 0;
   const Cut cut = cut_of(M, N, K, gated, norm_w != nullptr);
   if (cut.parts == 1 && !loose) part = nullptr;

@@ -13,21 +13,6 @@
 
 namespace {
 
-enum Act : int { ACT_SILU = 0, ACT_GELU_TANH = 1, ACT_GELU_ERF = 2, ACT_RELU = 3, ACT_IDENTITY = 4 };
-
-__device__ __forceinline__ float act_any(int a, float x) {
-  switch (a) {
-    case ACT_SILU: return x / (1.f + __expf(-x));
-    case ACT_GELU_TANH: {
-      const float k0 = 0.7978845608028654f, k1 = 0.044715f;
-      return 0.5f * x * (1.f + tanhf(k0 * (x + k1 * x * x * x)));
-    }
-    case ACT_GELU_ERF: return 0.5f * x * (1.f + erff(x * 0.7071067811865476f));
-    case ACT_RELU: return fmaxf(x, 0.f);
-    default: return x;
-  }
-}
-
 // One block per token row. v = acc + bias + residual -> res_out; y = v * rsqrt(mean(v^2) + eps) * w.
 // Elements are kept in registers between the two phases (EPT per thread, N <= 1024 * EPT).
 template <int EPT>

@@ -81,6 +81,15 @@ template <typename T> __device__ __forceinline__ T from_f32(float x) { return (T
 #define DS_ACT_CLAMPED_GLU 5
 // activation codes from here on: code - DS_ACT_UNARY applied to the result of an ungated decode product
 #define DS_ACT_UNARY 16
+__device__ __forceinline__ float act_any(int a, float x) {
+  switch (a) {
+    case 0: return x / (1.f + __expf(-x));  // silu
+    case 1: return 0.5f * x * (1.f + tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x)));
+    case 2: return 0.5f * x * (1.f + erff(x * 0.7071067811865476f));
+    case 3: return fmaxf(x, 0.f);
+    default: return x;
+  }
+}
 __device__ __forceinline__ float clamped_glu_f(float g, float u, float limit, float alpha = 1.702f, float shift = 1.f) {
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
