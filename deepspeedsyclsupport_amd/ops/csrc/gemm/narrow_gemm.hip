@@ -355,7 +355,9 @@ extern "C" int ds_narrow_gemm_ok(int64_t M, int64_t N, int64_t K, int64_t lda, i
 
 // Whether it is as fast as the library's there, us here (there); up to 1024 tokens. y: of K from 4096 on in three parts or more up to 128 tokens, in two
 // up to 256 (128 by [4096, 14336] 36 (75), [6144, 4096] 21 (25), [8192, 8192] 38 (50), 64 33 (34); 256 by [5120, 13824] 58 (120), [8192, 8192] 55 (78);
-// 64 by [12288, 4096] in two 28.7 (26.7)); else 2^31 products, of up to 2^24 weights 2^32 (512 tokens by
+// 64 by [12288, 4096] in two 28.7 (26.7)); where 128 x 128 tiles, whole, nearly fill one round: up to 128 tokens with rows 8 KB apart (64 / 128 by
+// [28672, 4096] 47 / 53 (57 / 59), by [22016, 4096], 172 tiles, 44 / 53 (47 / 49)), in two tiles of tokens over K up to 2048, from 192 up to 4096 (160 /
+// 256 by [11264, 2048] 22 / 24 (24.5 / 27.6); 192 / 256 by [12288, 4096] 39.5 / 44 (41 / 49), 160 by it 38.5 (37.8)); else 2^31 products, of up to 2^24 weights 2^32 (512 tokens by
 // [8000, 1024] 13.7 (16.0); 128 by [11264, 2048] 21.6 (18.1); 1024 by [5632, 1024], 1.4 times 2^32, 23 (20.2)). dX: 3 2^32 and fewer than 3 2^20
 // results (512 by [11264, 2048] 61 (76), by [5632, 1024] 15.9 (25.3); 768 by [4096, 4096] 52 (42), 512 by [1024, 8192] 16.9 (15.2); 1500 by [4096, 2048]
 // 45 (35)). dW: 2^22 weights, 2^23 from up to 224 tokens (1024 by [3072, 1024] 13.3 (15.5); 200 by [8000, 1024] 14.5 (14.3), 256 15.2 (12.6)).
@@ -364,6 +366,9 @@ extern "C" int ds_narrow_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along,
   if (!a_along) return M * N <= (K <= 224 ? 1 << 23 : 1 << 22);
   if (!b_along) return M * N < (3 << 20) && M * N <= (3LL << 32) / K;
   if (K >= 4096 && M <= 256 && cut_of(M, N, K, true, true).parts >= (M <= 128 ? 3 : 2)) return 1;
+  const int64_t big = (N + 127) / 128;
+  if (K % 4096 == 0 && M <= 128 && big >= 200 && big <= 256) return 1;
+  if (M > (K <= 2048 ? 128 : 191) && M <= 256 && K <= 4096 && big >= 80 && big <= (K <= 2048 ? 128 : 112)) return 1;
   return M * N <= (1LL << (N * K <= (1 << 24) ? 32 : 31)) / K;
 }
 

@@ -49,7 +49,7 @@ def test_products_at_their_edges(M, N, K, tile, parts):
 
 @GPU
 @pytest.mark.parametrize("M,N,K", [(52, 6152, 4096), (1, 6144, 4096), (128, 6200, 4160), (129, 4104, 8192), (256, 5120, 5120), (100, 2056, 5632),
-                                   (33, 1024, 8192), (255, 4096, 4096), (300, 4096, 4160)])
+                                   (33, 1024, 8192), (255, 4096, 4096), (300, 4096, 4160), (100, 25608, 4096), (129, 11264, 2048), (193, 14328, 4096)])
 def test_long_inner_dimensions(M, N, K):
     """Tiles and parts as the rule chooses them for K from 4096 on: 128 x 128 (rows a multiple of 8 KB apart begin elsewhere in K, unless
     tiles share weights) and 64 x 64, and beyond them; the same bits each time."""
