@@ -25,7 +25,7 @@ from ...ops import reference
 from ...ops import moe_ops
 from ...ops.bf16_gemv import Bf16Weight, decode_rows_ok
 from ...ops.linear import plain_linear
-from ...ops.native import cpu_ops, hip_ops
+from ...ops.native import cpu_ops, gemv_ops, hip_ops
 from ...ops.transformer import functional as DF
 
 
@@ -163,8 +163,8 @@ class BatchMeta:
 @dataclass
 class RaggedMeta:
     """One ragged batch (inference v2 `put()`): the new tokens of every sequence concatenated, decode sequences (one
-    token each) first, then short portions (up to `SHORT_TOKENS`), then longer prompts and portions. Device tensors come from ONE packed host->device copy
-    (`RaggedMeta.build`); the host lists are kept so no step needs a device->host sync."""
+    token each) first, then short portions (up to `SHORT_TOKENS`), then longer prompts and portions. Device tensors are parts of one: short tables come
+    as a kernel's arguments, long ones in a copy (`RaggedMeta.build`); the host lists are kept so no step needs a device->host sync."""
     block_tables: torch.Tensor       # [S, max_blocks] int32
     start_pos: torch.Tensor          # [S] tokens cached before this step
     seq_lens: torch.Tensor           # [S] start + new
@@ -221,9 +221,15 @@ class RaggedMeta:
         """`slots`: state slots of the sequences; `logit_rows`: rows (of the concatenated tokens) whose logits are
         wanted instead of every sequence's last; `ids`: int64 tokens on the host (a tensor or several) that go along."""
         toks = [] if ids is None else [ids] if torch.is_tensor(ids) else list(ids)
+        device = None if device is None else torch.device(device)
+        upload, most = None, 0
+        if device is not None and device.type == "cuda":
+            if device.index is None:
+                device = torch.device("cuda", torch.cuda.current_device())
+            upload, most = gemv_ops().upload, gemv_ops().upload_most()
         views, last_idx, ids, cu, n_short, kv_total, width, all_rows = cpu_ops().ragged_tables(
-            starts, n_new, block_lists, n_decode, slots or [], logit_rows, toks, None if device is None else torch.device(device),
-            RaggedMeta.SHORT_TOKENS, RaggedMeta.STEP_TOKENS, RaggedMeta.STATE_CHUNK)
+            starts, n_new, block_lists, n_decode, slots or [], logit_rows, toks, device, RaggedMeta.SHORT_TOKENS, RaggedMeta.STEP_TOKENS,
+            RaggedMeta.STATE_CHUNK, upload, most)
         pos_t, sid_t, st_t, len_t, cu_t, work_t, last_t, bt_t, slot_t, short_t, long_t, chunk_t, kv_t = views
         return RaggedMeta(block_tables=bt_t, start_pos=st_t, seq_lens=len_t, pos_ids=pos_t, seq_ids=sid_t, cu_q=cu_t, work=work_t,
                           last_idx=last_idx, last_rows=last_t, all_rows=all_rows, ids=ids, n_decode=n_decode, cu_host=cu,

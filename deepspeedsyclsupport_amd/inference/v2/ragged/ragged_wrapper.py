@@ -2,7 +2,7 @@
 
 Sequences are inserted one by one with their new tokens; `finalize()` orders them (single-token decodes of known
 sequences first: the paged decode kernel takes a leading slice; then short portions, then prompts and long portions), builds every index
-table the kernels need and ships them to the device in ONE packed pinned copy (`RaggedMeta.build`). The kernels of
+table the kernels need and ships them to the device in one piece (`RaggedMeta.build`). The kernels of
 `inference/v2/kernels/ragged_ops.py` and `DSInferenceModel.forward_ragged` read the tables from `.meta`.
 """
 from typing import List

@@ -1,5 +1,5 @@
 // Module of the bf16 products of the hybrid decoders: decode products (up to 48 token rows), with activation epilogues, and those of
-// short prompts.
+// short prompts; a batch's tables on their way to the device.
 #include "bind_util.h"
 #include "narrow_bind.h"
 
@@ -10,6 +10,8 @@ int ds_decode_gemm_ok(int, int);
 int ds_decode_gemm(const void*, const void*, const void*, const void*, float, const void*, void*, int, int, int, int, int, float,
                    void*, hipStream_t);
 int64_t ds_decode_gemm_scratch(int, int, int, int, int);
+int ds_upload_most();
+int ds_upload(const void*, void*, int, hipStream_t);
 int ds_skinny_mfma_ok(int, int, int);
 int ds_skinny_mfma(const void*, const void*, const void*, const void*, const void*, const void*, void*, void*, int, int,
                    int, int, int, int, float, hipStream_t);
@@ -75,6 +77,17 @@ bool decode_linear_sh_ok(int64_t M, int64_t N, int64_t K, bool glu) {
   if (glu && N % 32) return false;
   return ds_decode_gemm_scratch((int)M, (int)N, (int)K, glu, 0) > 0 || K <= 8192;
 }
+
+// 32-bit words on the host -> on the device, in a launch; the host's may change as soon as this returns. Longer ones: undefined
+OptT upload(Tensor words, int64_t device) {
+  TORCH_CHECK(words.device().is_cpu() && words.dim() == 1 && words.is_contiguous() && words.scalar_type() == at::kInt, "upload: int32 words on the host");
+  if (words.numel() > ds_upload_most()) return std::nullopt;
+  const c10::Device dev(c10::kCUDA, (c10::DeviceIndex)device);
+  const c10::DeviceGuard guard(dev);
+  auto out = torch::empty({words.numel()}, words.options().device(dev));
+  check(ds_upload(words.data_ptr(), out.data_ptr(), (int)words.numel(), stream()), "upload");
+  return out;
+}
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -85,4 +98,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_linear_sh", &decode_linear_sh, py::arg("x"), py::arg("wsh"), py::arg("N"),
         py::arg("glu_limit") = py::none(), py::arg("act") = py::none());
   m.def("linear", &linear_product);
+  m.def("upload", &upload);
+  m.def("upload_most", &ds_upload_most);
 }

@@ -20,12 +20,14 @@ int64_t narrow(int64_t v) {
 }
 
 // See RaggedMeta (inference/model_implementations/transformer.py) for the tables. One array of 32-bit integers behind the 64-bit
-// ones (logit rows, then the tokens), one copy, from pinned memory, so that no step waits for the steps before it.
+// ones (logit rows, then the tokens), taken to the device by `upload` where it has up to `most` words (a decode step's: 12 sequences
+// of 600 tokens 400), else by one copy from pinned memory, so that no step waits for the steps before it.
 // -> (the tables in the order of RaggedMeta.build, logit rows, tokens or None, offsets, n_short, end of the long contexts, width of
 // the block tables, whether the logit rows are all rows)
 pybind11::tuple ragged_tables(const Ints& starts, const Ints& n_new, const std::vector<Ints>& blocks, int64_t n_decode, const Ints& slots,
                               const std::optional<Ints>& logit_rows, const std::vector<Tensor>& ids, const std::optional<c10::Device>& device,
-                              int64_t short_tokens, int64_t step_tokens, int64_t state_chunk) {
+                              int64_t short_tokens, int64_t step_tokens, int64_t state_chunk, const std::optional<pybind11::function>& upload,
+                              int64_t most) {
   const size_t S = starts.size();
   TORCH_CHECK(S > 0 && n_new.size() == S && blocks.size() == S && (slots.empty() || slots.size() == S), "ragged_tables: one entry a sequence");
   Ints cu(S + 1, 0);
@@ -113,7 +115,9 @@ pybind11::tuple ragged_tables(const Ints& starts, const Ints& n_new, const std::
   }
   const int64_t wide = (int64_t)last.size() + tokens;
   const bool cuda = device && device->is_cuda();
-  Tensor buf = torch::empty({2 * wide + (int64_t)flat.size()}, torch::TensorOptions().dtype(at::kInt).pinned_memory(cuda));
+  const int64_t words = 2 * wide + (int64_t)flat.size();
+  const bool small = cuda && upload && words <= most;
+  Tensor buf = torch::empty({words}, torch::TensorOptions().dtype(at::kInt).pinned_memory(cuda && !small));
   int64_t* w = reinterpret_cast<int64_t*>(buf.data_ptr<int32_t>());
   w = std::copy(last.begin(), last.end(), w);
   for (const Tensor& t : ids) {
@@ -121,7 +125,8 @@ pybind11::tuple ragged_tables(const Ints& starts, const Ints& n_new, const std::
     w = std::copy(c.data_ptr<int64_t>(), c.data_ptr<int64_t>() + c.numel(), w);
   }
   std::copy(flat.begin(), flat.end(), buf.data_ptr<int32_t>() + 2 * wide);
-  if (cuda) buf = buf.to(*device, /*non_blocking=*/true);
+  if (small) buf = (*upload)(buf, device->index()).cast<Tensor>();
+  else if (cuda) buf = buf.to(*device, /*non_blocking=*/true);
   const Tensor head = buf.narrow(0, 0, 2 * wide).view(at::kLong);
   std::vector<Tensor> views;
   int64_t at = 2 * wide, from = 0;

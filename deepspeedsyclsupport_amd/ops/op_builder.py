@@ -69,6 +69,7 @@ EXTENSIONS = {
             "gemv/skinny_mfma.hip",
             "gemv/skinny_bf16_sh.hip",
             "gemm/narrow_gemm.hip",
+            "ragged/upload.hip",
         ],
         "bindings": ["bind/gemv_bind.cpp"],
     },

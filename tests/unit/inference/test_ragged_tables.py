@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from deepspeedsyclsupport_amd.inference.model_implementations.transformer import RaggedMeta
-from deepspeedsyclsupport_amd.ops.native import cpu_ops
+from deepspeedsyclsupport_amd.ops.native import cpu_ops, gemv_ops
 
 
 @pytest.mark.parametrize("seed", range(6))
@@ -55,3 +55,34 @@ def test_range_of_host_tokens():
     f = cpu_ops().int_range
     assert f([]) == (0, -1) and f([torch.empty(0, dtype=torch.int64)]) == (0, -1)
     assert f([torch.tensor([3, -1]), torch.tensor([7], dtype=torch.int32)]) == (-1, 7)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,new", [(1, 1), (12, 1), (50, 1), (60, 1), (90, 1), (3, 40), (2, 700)])
+def test_tables_on_the_device(S, new):
+    """Short tables go as a kernel's arguments, long ones as a copy: the same tables either way, twice in a row."""
+    args = [5 + i for i in range(S)], [new] * S, [[i, 2 * i + 1, 7] for i in range(S)], S if new == 1 else 0, 256
+    toks = [torch.arange(new) + i for i in range(S)]
+    for slots in (list(range(S)), list(range(S, 2 * S))):
+        want = RaggedMeta.build(*args, None, slots, None, toks)
+        for device in ("cuda", "cuda:0", torch.device("cuda")):
+            got = RaggedMeta.build(*args, device, slots, None, toks)
+            for name, a in vars(want).items():
+                b = getattr(got, name)
+                if torch.is_tensor(a):
+                    assert b.device == torch.device("cuda:0") and b.dtype == a.dtype and torch.equal(b.cpu(), a), name
+                else:
+                    assert b == a, name
+
+
+@pytest.mark.gpu
+def test_words_as_arguments():
+    most = gemv_ops().upload_most()
+    assert gemv_ops().upload(torch.zeros(most + 1, dtype=torch.int32), 0) is None
+    for n in (0, 1, 239, 240, 241, 256, 257, most - 1, most):
+        host, outs, want = torch.empty(n, dtype=torch.int32), [], []
+        for k in range(4):
+            host.copy_(torch.randint(-2**31, 2**31 - 1, (n, )))   # (free again as soon as the call returns)
+            want.append(host.clone())
+            outs.append(gemv_ops().upload(host, 0))
+        assert all(torch.equal(a.cpu(), b) for a, b in zip(outs, want))
