@@ -40,6 +40,7 @@ struct NarrowArgs {
   f32x4* part;             // their sums [parts][M][N] (null: the result leaves from here)
   const bf16 *bias, *res;  // behind a product with an ordered operand: [N] or null, [M, N] or null
   int act;                 // ... an activation code + DS_ACT_UNARY, or -1
+  int band;                // row tiles that are walked together, column by column
 };
 
 // Columns n .. n + 3 of row m: bias, activation, residual
@@ -163,7 +164,9 @@ __global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(Nar
   __shared__ __attribute__((aligned(16))) char lds[4 * BUF];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wid % WM * 32 * MR, wn = wid / WM % WN * 32 * NR, wk = wid / (WM * WN);
-  const int mt = (a.M + TM - 1) / TM, id = xcd_remap(blockIdx.x, gridDim.x), m0 = id % mt * TM, n0 = id / mt * TN;
+  const int mt = (a.M + TM - 1) / TM, nt = (a.N + TN - 1) / TN, id = xcd_remap(blockIdx.x, gridDim.x);
+  const int strip = id / (a.band * nt), spot = id - strip * a.band * nt, deep = min(a.band, mt - strip * a.band);
+  const int m0 = (strip * a.band + spot % deep) * TM, n0 = spot / deep * TN;
   const int all = (a.K + 63) / 64, first = (int)((int64_t)all * blockIdx.y / a.parts);  // steps of 64: of K, and of this part
   const int steps = (int)((int64_t)all * (blockIdx.y + 1) / a.parts) - first, rounds = (steps + U - 1) / U;
   // Rows that lie a multiple of 8 KB apart meet in a memory channel at each step of K, in all workgroups at once: each begins elsewhere.
@@ -297,6 +300,14 @@ __global__ void __launch_bounds__(256) narrow_sum_kernel(NarrowArgs a) {
   *reinterpret_cast<bf16x4*>(a.c + 4 * i) = narrowed(v);
 }
 
+// Each XCD, with an L2 of its own, has an eighth of the tiles in a row: as nearly a square of them as bands allow (dW of 1000 / 8000 tokens, us, with
+// all row tiles first and in bands: [2048, 1024] 10.5 / 88 and 9.1 / 57, [2048, 512] 7.0 / 49 and 6.1 / 28.5, [11264, 2048] 77 / 439 and 68 / 400)
+int band_of(int64_t mt, int64_t nt) {
+  int64_t band = 1;
+  while (band < mt && 4 * band * band <= mt * nt / 8) band *= 2;
+  return (int)std::min(band, mt);
+}
+
 int g_tile = 0, g_parts = 0;
 
 struct Cut {
@@ -312,12 +323,13 @@ struct Cut {
 // One across (dX): those rows come in runs of 64 columns, never 32 (half a cache line). 64 x 64 from 160 tiles on, of long K from 64
 // (256 tokens by [5632, 1024] 32x2 13.0, 64x4 11.8; 512 17.5, 64x2 15.8; by [3072, 1024] 9.5, 10.5). Parts of 768 up to a workgroup a CU
 // (128 by [3072, 1024] 10.6, x2 9.4, x4 8.9; by [1024, 1024] 5.3, 6.4, 6.9).
-// Both across (dW): 64 x 64, 128 x 128 from 176 of them on (512 by [3072, 1024] 11.0, 9.8; by [1536, 1024] 7.6, 8.7).
+// Both across (dW): 64 x 64, 128 x 128 from 140 of them on (512 by [3072, 1024] 11.0, 9.8; 500 / 2000 / 8000 by [1536, 1536], 144, 9.0 / 21.7 / 77, 8.9 / 21.0 /
+// 64; by [1024, 2048], 128, 6.7 / 15.4 / 56, 8.9 / 20.4 / 63).
 Cut cut_of(int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) {
   auto tiles = [&](int t, int u) { return ((M + t - 1) / t) * ((N + u - 1) / u); };
   const bool along = a_along && b_along, across = !a_along && !b_along;
   int tm = 32, tn = along ? 32 : 64;
-  if (tiles(128, 128) >= (across ? 176 : 140) && (along || across)) tm = tn = 128;
+  if (tiles(128, 128) >= 140 && (along || across)) tm = tn = 128;
   else if (along ? tiles(32, 32) > 512 : across || tiles(64, 64) >= (K >= 4096 ? 64 : 160)) tm = tn = 64;
   int64_t parts = 0;
   if (along && K >= 4096) {
@@ -360,10 +372,18 @@ extern "C" int ds_narrow_gemm_ok(int64_t M, int64_t N, int64_t K, int64_t lda, i
 // 256 by [11264, 2048] 22 / 24 (24.5 / 27.6); 192 / 256 by [12288, 4096] 39.5 / 44 (41 / 49), 160 by it 38.5 (37.8)); else 2^31 products, of up to 2^24 weights 2^32 (512 tokens by
 // [8000, 1024] 13.7 (16.0); 128 by [11264, 2048] 21.6 (18.1); 1024 by [5632, 1024], 1.4 times 2^32, 23 (20.2)). dX: 3 2^32 and fewer than 3 2^20
 // results (512 by [11264, 2048] 61 (76), by [5632, 1024] 15.9 (25.3); 768 by [4096, 4096] 52 (42), 512 by [1024, 8192] 16.9 (15.2); 1500 by [4096, 2048]
-// 45 (35)). dW: 2^22 weights, 2^23 from up to 224 tokens (1024 by [3072, 1024] 13.3 (15.5); 200 by [8000, 1024] 14.5 (14.3), 256 15.2 (12.6)).
+// 45 (35)). Beyond, up to 2048, by [1024, 1024] (1400: y 8.3 (10.3), dX 8.2 (10.7)), dX by [3072, 1024] 23.6 (29.3). dW: one
+// round of 128 x 128 tiles, up to 8192 tokens (1000 / 3000 / 8000 by [2048, 2048] 14 / 30 / 73 (20 / 40 / 90), [1024, 2816] 13 / 27.5 / 64 (20 / 40 / 81),
+// [2048, 512] 6 / 13 / 28.5 (13 / 28 / 54), [1024, 1024] 6.4 / 14 / 31 (14 / 28 / 54)); one and a half or two, up to 2048 (300 / 1000 / 2000 by [3072, 2048]
+// 13.6 / 24 / 39 (15 / 27.5 / 45), [8000, 1024] 13.3 / 25.5 / 42 (16 / 30 / 46); 3000 by [3072, 2048] 53.4 (53.5)); nearly three where the library is slow (300 /
+// 1400 by [2048, 5632] 19 / 44 (28 / 53), but 800 by [5632, 2048] 31 (28)); five and a half (500 / 1000 by [11264, 2048] 43.5 / 68.5 (45 / 77)).
 extern "C" int ds_narrow_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along) {
-  if ((a_along ? M : K) > 1024) return 0;
-  if (!a_along) return M * N <= (K <= 224 ? 1 << 23 : 1 << 22);
+  if (!a_along) {
+    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
+    if (tiles <= 512) return tiles <= 256 ? K <= 8192 : K <= 2048;
+    return K >= 256 && ((tiles >= 640 && tiles <= 768 && N >= 2 * M && K <= 1500) || (tiles >= 1280 && tiles <= 1536 && K <= 1024));
+  }
+  if (M > 1024) return M <= 2048 && N <= 1024 && K <= (b_along ? 1024 : 3072);
   if (!b_along) return M * N < (3 << 20) && M * N <= (3LL << 32) / K;
   if (K >= 4096 && M <= 256 && cut_of(M, N, K, true, true).parts >= (M <= 128 ? 3 : 2)) return 1;
   const int64_t big = (N + 127) / 128;
@@ -389,7 +409,7 @@ extern "C" int ds_narrow_gemm(const void* A, const void* B, void* C, int64_t M, 
   const int64_t ar = a_along ? M : K, ac = a_along ? K : M, br = b_along ? N : K, bc = b_along ? K : N;
   const NarrowArgs a{(const bf16*)A, (const bf16*)B, (bf16*)C, (int)M, (int)N, (int)K, (uint32_t)lda, (uint32_t)ldb,
                      (uint32_t)(((ar - 1) * lda + ac) * 2), (uint32_t)(((br - 1) * ldb + bc) * 2), cut.parts, (f32x4*)part,
-                     nullptr, nullptr, -1};
+                     nullptr, nullptr, -1, band_of((M + cut.tm - 1) / cut.tm, (N + cut.tn - 1) / cut.tn)};
   const dim3 grid((unsigned)(((M + cut.tm - 1) / cut.tm) * ((N + cut.tn - 1) / cut.tn)), cut.parts);
 #define GO(AK, BK, TM, TN, U) hipLaunchKernelGGL((narrow_gemm_kernel<AK, BK, TM, TN, U>), grid, dim3(256), 0, st, a)
   if (cut.tm == 128) {
@@ -455,7 +475,7 @@ extern "C" int ds_narrow_ordered(const void* X, const void* W, const void* bias,
   if (cut.parts == 1) part = nullptr;
   else if (!part) return (int)hipErrorInvalidValue;
   const NarrowArgs a{(const bf16*)X, (const bf16*)W, (bf16*)Y, (int)M, (int)N, (int)K, (uint32_t)K, (uint32_t)K, (uint32_t)(M * K * 2),
-                     (uint32_t)((N + 15) / 16 * 16 * K * 2), cut.parts, (f32x4*)part, (const bf16*)bias, (const bf16*)res, act};
+                     (uint32_t)((N + 15) / 16 * 16 * K * 2), cut.parts, (f32x4*)part, (const bf16*)bias, (const bf16*)res, act, (int)((M + cut.tm - 1) / cut.tm)};
   const dim3 grid((unsigned)(((M + cut.tm - 1) / cut.tm) * ((N + cut.tn - 1) / cut.tn)), cut.parts);
 #define GO(TM, U) hipLaunchKernelGGL((narrow_gemm_kernel<ALONG, ORDERED, TM, TM, U>), grid, dim3(256), 0, st, a)
   if (cut.tm == 128) GO(128, 1);

@@ -62,6 +62,19 @@ def test_long_inner_dimensions(M, N, K):
 
 
 @GPU
+@pytest.mark.parametrize("T,O,I", [(1027, 2056, 520), (1027, 520, 2056), (1500, 1608, 1608), (3001, 256, 1032), (8192, 136, 264), (300, 2048, 5632), (2049, 1032, 1024)])
+def test_gradients_of_many_tokens(T, O, I):
+    """Tiles in bands of rows, the last one of fewer, over inner dimensions of any length; what the layer takes."""
+    ops = hip_ops()
+    go, x, w = _rnd(T, O, seed=1), _rnd(T, I, seed=2), _rnd(O, I, seed=3)
+    got = ops.narrow_gemm(go, x, False, False)
+    _check(got, go.t(), x.t())
+    assert torch.equal(got, ops.narrow_gemm(go, x, False, False)) and torch.equal(got, ops.linear_weight_grad(go, x))
+    _check(ops.linear_input_grad(go, w), go, w.t())
+    _check(ops.linear(x, w), x, w)
+
+
+@GPU
 def test_values_that_do_not_mix():
     """Infinities and NaN stay in their rows; nothing from past the end of an operand comes in."""
     a, b = _rnd(40, 128), _rnd(48, 128, seed=1)
