@@ -9,6 +9,9 @@
 //    way;
 //  * an operand whose rows run along the inner dimension is stored row by row, 128 bytes a step; one whose rows run across it (W in dX, both in
 //    dW) as it lies, and read transposed (ds_read_b64_tr_b16). Chunks are swizzled by the source address, against bank conflicts;
+//  * tiles of 128 x 128 have a CU to themselves, a wave on a SIMD: it reads a quarter of a step while it multiplies the one before, the first of the
+//    next step too, behind a barrier that stands before the last (1536 x 1536 over 8000 tokens 64 -> 50 us, 1000 tokens by [11264, 2048] 61 ->
+//    53). Then bound by what the L2s hand out: 256 workgroups 64 bytes a nanosecond each, 144 of them 84;
 //  * what lies past the end of a buffer reads as zero: ragged tokens need no other treatment, along the inner dimension neither.
 // Besides, the library's call takes the host 18 to 23 us, this one 5 to 7: a training step of 128 tokens has 27 of them and waits for the host.
 // Measured, us (the library's kernel): 128 tokens, layers [3072, 1024], [1024, 1024], [5632, 1024], [1024, 2816], head [8000, 1024]: y 6.4
@@ -178,12 +181,16 @@ __global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(Nar
   oa.init(a.a, a.abytes, a.lda, m0, lane, wid);
   ob.init(a.b, a.bbytes, a.ldb, n0, lane, wid);
   auto buffer = [&](auto b_c) -> lds_char* { return (lds_char*)lds + (decltype(b_c)::value & 3) * BUF; };
+  // where step i of this part stands in K; past the end the last one again
+  auto place_in = [&](int i) {
+    const int kq = min(i, steps - 1) + rot;
+    return first + (kq >= steps ? kq - steps : kq);
+  };
   // round r; past the end the last step again, into a place that nobody reads
   auto move = [&](int r, auto b_c) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      int kq = min(r * U + u, steps - 1) + rot;
-      kq = first + (kq >= steps ? kq - steps : kq);
+      const int kq = place_in(r * U + u);
       const uint32_t to = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)buffer(b_c) + STEP * u);
       oa.move(kq, to);
       ob.move(kq, to + A::BYTES);
@@ -230,19 +237,70 @@ __global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(Nar
     move(0, Int<0>{});
     move(1, Int<1>{});
     move(2, Int<2>{});
-    auto round = [&](int r, auto b_c) {
-      meet<2 * PER>();  // this round's operands have come, and nobody reads the buffer of the round before any more
-      move(r + 3, Int<decltype(b_c)::value + 3>{});
-      products(r, b_c);
-    };
-    for (int r = 0; r < rounds; r += 4) {
-      round(r, Int<0>{});
-      if (r + 1 >= rounds) break;
-      round(r + 1, Int<1>{});
-      if (r + 2 >= rounds) break;
-      round(r + 2, Int<2>{});
-      if (r + 3 >= rounds) break;
-      round(r + 3, Int<3>{});
+    if constexpr (TM == 128) {
+      bf16x8 x[2][MR], w[2][NR];
+      auto fetch = [&](auto b_c, int j, int s) {
+        const lds_char* buf = buffer(b_c);
+#pragma unroll
+        for (int n = 0; n < NR; ++n) w[s][n] = ob.template read<PLAIN>(buf + A::BYTES, j, wn + 32 * n, lane);
+#pragma unroll
+        for (int m = 0; m < MR; ++m) x[s][m] = oa.template read<PLAIN>(buf, j, wm + 32 * m, lane);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto multiply = [&](int s) {
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+#pragma unroll
+          for (int n = 0; n < NR; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[s][n], x[s][m], acc[m][n], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto round = [&](int r, auto b_c) {
+        using Next = Int<decltype(b_c)::value + 1>;
+        const int kq = place_in(r + 3);
+        const uint32_t to = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)buffer(Int<decltype(b_c)::value + 3>{}));
+        fetch(b_c, 1, 1);
+        oa.move(kq, to);
+        multiply(0);
+        fetch(b_c, 2, 0);
+        ob.move(kq, to + A::BYTES);
+        multiply(1);
+        fetch(b_c, 3, 1);
+        multiply(0);
+        meet<2 * PER>();
+        fetch(Next{}, 0, 0);
+        multiply(1);
+      };
+      meet<2 * PER>();
+      fetch(Int<0>{}, 0, 0);
+      int r = 0;
+      for (; r + 4 <= rounds; r += 4) {
+        round(r, Int<0>{});
+        round(r + 1, Int<1>{});
+        round(r + 2, Int<2>{});
+        round(r + 3, Int<3>{});
+      }
+      if (r < rounds) {
+        round(r, Int<0>{});
+        if (r + 1 < rounds) {
+          round(r + 1, Int<1>{});
+          if (r + 2 < rounds) round(r + 2, Int<2>{});
+        }
+      }
+    } else {
+      auto round = [&](int r, auto b_c) {
+        meet<2 * PER>();  // this round's operands have come, and nobody reads the buffer of the round before any more
+        move(r + 3, Int<decltype(b_c)::value + 3>{});
+        products(r, b_c);
+      };
+      for (int r = 0; r < rounds; r += 4) {
+        round(r, Int<0>{});
+        if (r + 1 >= rounds) break;
+        round(r + 1, Int<1>{});
+        if (r + 2 >= rounds) break;
+        round(r + 2, Int<2>{});
+        if (r + 3 >= rounds) break;
+        round(r + 3, Int<3>{});
+      }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the surplus transfers)
   }
@@ -315,21 +373,22 @@ struct Cut {
 };
 // us, on one machine, of 32-row tiles / 64 / 128, whole or in parts of K (x2, x4).
 // Both operands along K (y): 32 x 32 up to two tiles a CU (128 tokens by [3072, 1024] 6.4 / 6.4, [4096, 2048] 9.0 / 9.4, [5632, 1024] 8.6 / 6.7), 128 x
-// 128 from 140 of them on (512 by [5632, 1024] 13.7 with 64, 12.7; 768 by [3072, 1024], 144 of them, 13.8, 12.1; 256 by [8000, 1024], 126, 9.8, 12.2). Parts
+// 128 from 140 of them on (512 by [5632, 1024] 13.3 with 64, 11.1; 768 by [3072, 1024], 144 of them, 13.1, 11.0; 200 by [8000, 1024], 126, 9.4, 10.7). Parts
 // of 2560 or more of K: a sum costs 2 us and its traffic (64 by [2048, 5632] 12.6, x2 10.5; [1024, 2816] 7.7, 7.7).
 // From K = 4096 on weights come from memory and a CU's share of the operands bounds: 128 x 128 tiles, in parts of 768 or more, where those make
 // 192 to 256 workgroups (128 by [4096, 14336] 63.9 with 64x1, 34.8 with 128x8; by [6144, 4096] 22.2, 128x5 20.7; but 256 by [4096, 4096] 21.2
 // with 64x1, 128x4 22.4), else 64 x 64 in parts of 1024 or more (128 by [2048, 5632] 18.2 with 32x2, 13.9; by [1024, 8192] 18.4, 13.1).
 // One across (dX): those rows come in runs of 64 columns, never 32 (half a cache line). 64 x 64 from 160 tiles on, of long K from 64
-// (256 tokens by [5632, 1024] 32x2 13.0, 64x4 11.8; 512 17.5, 64x2 15.8; by [3072, 1024] 9.5, 10.5). Parts of 768 up to a workgroup a CU
+// (256 tokens by [5632, 1024] 32x2 13.0, 64x4 11.8; 512 17.5, 64x2 15.8; by [3072, 1024] 9.5, 10.5), 128 x 128 from 150 (800 by [1024, 2816], 154, 13.3 with
+// 64, 12.8; 300 by [2048, 5632], 132, 18.9, 19.5). Parts of 768 up to a workgroup a CU
 // (128 by [3072, 1024] 10.6, x2 9.4, x4 8.9; by [1024, 1024] 5.3, 6.4, 6.9).
-// Both across (dW): 64 x 64, 128 x 128 from 140 of them on (512 by [3072, 1024] 11.0, 9.8; 500 / 2000 / 8000 by [1536, 1536], 144, 9.0 / 21.7 / 77, 8.9 / 21.0 /
-// 64; by [1024, 2048], 128, 6.7 / 15.4 / 56, 8.9 / 20.4 / 63).
+// Both across (dW): 64 x 64, 128 x 128 from 140 of them on (500 / 2000 / 8000 by [1536, 1536], 144, 9.0 / 21.7 / 77, 8.2 / 17.7 / 50; by [1024, 2048], 128, 6.7 /
+// 15.4 / 56, 8.1 / 17.8 / 50).
 Cut cut_of(int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) {
   auto tiles = [&](int t, int u) { return ((M + t - 1) / t) * ((N + u - 1) / u); };
   const bool along = a_along && b_along, across = !a_along && !b_along;
   int tm = 32, tn = along ? 32 : 64;
-  if (tiles(128, 128) >= 140 && (along || across)) tm = tn = 128;
+  if (tiles(128, 128) >= (along || across ? 140 : 150)) tm = tn = 128;
   else if (along ? tiles(32, 32) > 512 : across || tiles(64, 64) >= (K >= 4096 ? 64 : 160)) tm = tn = 64;
   int64_t parts = 0;
   if (along && K >= 4096) {
@@ -346,7 +405,7 @@ Cut cut_of(int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) {
     tm = g_tile;
     tn = g_tile == 32 && !along ? 64 : g_tile;
   }
-  if (!parts || g_tile) parts = std::min<int64_t>(std::min<int64_t>((along ? 512 : 256) / tiles(tm, tn), K / (along ? 2560 : 768)), 8);
+  if (!parts || g_tile) parts = std::min<int64_t>(std::min<int64_t>((along && tm < 128 ? 512 : 256) / tiles(tm, tn), K / (along ? 2560 : 768)), 8);
   if (g_parts) parts = std::min<int64_t>(g_parts, (K + 63) / 64);
   return {tm, tn, (int)std::max<int64_t>(parts, 1)};
 }
@@ -365,30 +424,30 @@ extern "C" int ds_narrow_gemm_ok(int64_t M, int64_t N, int64_t K, int64_t lda, i
   return (ar + 128) * lda * 2 < UINT32_MAX && (br + 128) * ldb * 2 < UINT32_MAX && ((M + 31) / 32) * ((N + 31) / 32) <= INT32_MAX;
 }
 
-// Whether it is as fast as the library's there, us here (there); up to 1024 tokens. y: of K from 4096 on in three parts or more up to 128 tokens, in two
-// up to 256 (128 by [4096, 14336] 36 (75), [6144, 4096] 21 (25), [8192, 8192] 38 (50), 64 33 (34); 256 by [5120, 13824] 58 (120), [8192, 8192] 55 (78);
-// 64 by [12288, 4096] in two 28.7 (26.7)); where 128 x 128 tiles, whole, nearly fill one round: up to 128 tokens with rows 8 KB apart (64 / 128 by
-// [28672, 4096] 47 / 53 (57 / 59), by [22016, 4096], 172 tiles, 44 / 53 (47 / 49)), in two tiles of tokens over K up to 2048, from 192 up to 4096 (160 /
-// 256 by [11264, 2048] 22 / 24 (24.5 / 27.6); 192 / 256 by [12288, 4096] 39.5 / 44 (41 / 49), 160 by it 38.5 (37.8)); else 2^31 products, of up to 2^24 weights 2^32 (512 tokens by
-// [8000, 1024] 13.7 (16.0); 128 by [11264, 2048] 21.6 (18.1); 1024 by [5632, 1024], 1.4 times 2^32, 23 (20.2)). dX: 3 2^32 and fewer than 3 2^20
-// results (512 by [11264, 2048] 61 (76), by [5632, 1024] 15.9 (25.3); 768 by [4096, 4096] 52 (42), 512 by [1024, 8192] 16.9 (15.2); 1500 by [4096, 2048]
-// 45 (35)). Beyond, up to 2048, by [1024, 1024] (1400: y 8.3 (10.3), dX 8.2 (10.7)), dX by [3072, 1024] 23.6 (29.3). dW: one
-// round of 128 x 128 tiles, up to 8192 tokens (1000 / 3000 / 8000 by [2048, 2048] 14 / 30 / 73 (20 / 40 / 90), [1024, 2816] 13 / 27.5 / 64 (20 / 40 / 81),
-// [2048, 512] 6 / 13 / 28.5 (13 / 28 / 54), [1024, 1024] 6.4 / 14 / 31 (14 / 28 / 54)); one and a half or two, up to 2048 (300 / 1000 / 2000 by [3072, 2048]
-// 13.6 / 24 / 39 (15 / 27.5 / 45), [8000, 1024] 13.3 / 25.5 / 42 (16 / 30 / 46); 3000 by [3072, 2048] 53.4 (53.5)); nearly three where the library is slow (300 /
-// 1400 by [2048, 5632] 19 / 44 (28 / 53), but 800 by [5632, 2048] 31 (28)); five and a half (500 / 1000 by [11264, 2048] 43.5 / 68.5 (45 / 77)).
+// Whether it is as fast as the library's there, us here (there).
+// y and dX: where 128 x 128 tiles, whole, nearly fill one round, 176 to 256 of them (y: 200 / 2000 by [11264, 2048] / [2048, 2048] 17.1 / 20.5 (21.7 / 21.6), 1000
+// by [4096, 4096] 34.4 (36.6), 4096 by [1024, 2816] 25.6 (28.2); dX: 500 by [2048, 5632] 20.6 (26.8), 800 by [4096, 4096] 36 (40), 2000 by [11264, 2048] 98
+// (105); 384 tiles, 3000 by [2048, 2048], 34 (27)), over weights of up to 2^26 or from 512 tokens on (160 by [16384, 8192] 95 (80)).
+// y besides: of K from 4096 on in three parts or more up to 128 tokens, in two up to 256 (128 by [4096, 14336] 36 (75), [6144, 4096] 21 (25), [8192, 8192]
+// 38 (50), 64 33 (34); 256 by [5120, 13824] 58 (120); 64 by [12288, 4096] in two 28.7 (26.7)); up to 128 tokens in 200 to 256 tiles with rows 8 KB
+// apart (64 / 128 by [28672, 4096] 47 / 53 (57 / 59); by [22016, 4096], 172 tiles, 44 / 53 (47 / 49)); up to 1024 2^31 products, of up to 2^24 weights 2^32 (512
+// by [8000, 1024] 13.7 (16.0); 128 by [11264, 2048] 21.6 (18.1)); up to 2048 by [1024, 1024] (1400 8.3 (10.3)).
+// dX besides: up to 1024 tokens 3 2^32 products and fewer than 3 2^20 results (500 by [11264, 2048] 41 (62), by [5632, 1024] 16 (26); 800 by the first 80
+// (78)); up to 2048 of 1024 columns, from 1800 on of any K (1400 by [3072, 1024] 23.6 (29.4), [5632, 1024] 40 (38); 2000 39 (45)).
+// dW: up to two rounds, up to 8192 tokens (1000 / 3000 / 8000 by [2048, 2048] 12.7 / 27 / 64 (21 / 43 / 88), [1024, 2816] 11.6 / 23 / 52 (20 / 40 / 82), [2048, 512] 6 /
+// 13 / 28.5 (13 / 28 / 53), [3072, 2048] 22 / 47 / 112 (27 / 57 / 113), [8000, 1024] 24 / 52 / - (32 / 63 / -)); nearly three up to 4096 (300 / 3000 by [2048,
+// 5632] 18 / 74 (28 / 87)), five and a half up to 3000 (1000 / 3000 by [11264, 2048] 64 / 148 (80 / 152)); four, [4096, 4096], 500 / 1000 28 / 44 (30 / 43).
 extern "C" int ds_narrow_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along) {
+  const int64_t big = (N + 127) / 128, tiles = (M + 127) / 128 * big;
   if (!a_along) {
-    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-    if (tiles <= 512) return tiles <= 256 ? K <= 8192 : K <= 2048;
-    return K >= 256 && ((tiles >= 640 && tiles <= 768 && N >= 2 * M && K <= 1500) || (tiles >= 1280 && tiles <= 1536 && K <= 1024));
+    if (tiles <= 512) return K <= 8192;
+    return (tiles >= 640 && tiles <= 768 && K >= 256 && K <= 4096) || (tiles >= 1280 && tiles <= 1536 && K >= 256 && K <= 3000);
   }
-  if (M > 1024) return M <= 2048 && N <= 1024 && K <= (b_along ? 1024 : 3072);
+  if (M > 128 && tiles >= 176 && tiles <= 256 && (M > 512 || N * K <= (1 << 26))) return 1;
+  if (M > 1024) return M <= 2048 && N <= 1024 && (b_along ? K <= 1024 : K <= 3072 || M >= 1800);
   if (!b_along) return M * N < (3 << 20) && M * N <= (3LL << 32) / K;
   if (K >= 4096 && M <= 256 && cut_of(M, N, K, true, true).parts >= (M <= 128 ? 3 : 2)) return 1;
-  const int64_t big = (N + 127) / 128;
   if (K % 4096 == 0 && M <= 128 && big >= 200 && big <= 256) return 1;
-  if (M > (K <= 2048 ? 128 : 191) && M <= 256 && K <= 4096 && big >= 80 && big <= (K <= 2048 ? 128 : 112)) return 1;
   return M * N <= (1LL << (N * K <= (1 << 24) ? 32 : 31)) / K;
 }
 
