@@ -3,15 +3,17 @@
 //
 // What bounds them is latency and the count of workgroups, not the matrix cores: 128 tokens of a 1024-wide layer make 32 tiles of
 // 64 x 64. Hence
-//  * tiles of 128 x 128 or 64 x 64 (four waves of 64 x 64 or 32 x 32) or, where those are too few, of 32 rows by 32 or 64 (the waves share
-//    each step's inner dimension and meet in LDS at the end, always in the same order), and K in parts with a second launch for their sums;
-//  * both operands come by DMA into four LDS buffers, three steps ahead; one barrier a step, whose wait counts what may still be on its
-//    way;
+//  * tiles of 128 x 256, 128 x 128 or 64 x 64 (four waves of 64 x 128, 64 x 64 or 32 x 32) or, where those are too few, of 32 rows by 32 or 64 (the
+//    waves share each step's inner dimension and meet in LDS at the end, always in the same order), and K in parts with a second launch
+//    for their sums;
+//  * both operands come by DMA into four LDS buffers, three steps ahead (128 x 256: into three, two ahead); one barrier a step, whose wait
+//    counts what may still be on its way;
 //  * an operand whose rows run along the inner dimension is stored row by row, 128 bytes a step; one whose rows run across it (W in dX, both in
 //    dW) as it lies, and read transposed (ds_read_b64_tr_b16). Chunks are swizzled by the source address, against bank conflicts;
-//  * tiles of 128 x 128 have a CU to themselves, a wave on a SIMD: it reads a quarter of a step while it multiplies the one before, the first of the
-//    next step too, behind a barrier that stands before the last (1536 x 1536 over 8000 tokens 64 -> 50 us, 1000 tokens by [11264, 2048] 61 ->
-//    53). Then bound by what the L2s hand out: 256 workgroups 64 bytes a nanosecond each, 144 of them 84;
+//  * tiles of 128 rows have a CU to themselves, a wave on a SIMD: before each product it reads one operand of the next quarter step and sends
+//    one transfer, the next step's first quarter too, behind a barrier that stands before the last. 3000 tokens by [11264, 2048], dW, us: a step's
+//    reads, then its products 179; quarters 146; product by product 138, in tiles of 128 x 256 119 (library 147). Matrix cores busy 71 % of
+//    the time, at 1.5 GHz;
 //  * what lies past the end of a buffer reads as zero: ragged tokens need no other treatment, along the inner dimension neither.
 // Besides, the library's call takes the host 18 to 23 us, this one 5 to 7: a training step of 128 tokens has 27 of them and waits for the host.
 // Measured, us (the library's kernel): 128 tokens, layers [3072, 1024], [1024, 1024], [5632, 1024], [1024, 2816], head [8000, 1024]: y 6.4
@@ -114,10 +116,11 @@ struct Operand {
     }
   }
   // A transposed read takes 64 bytes of eight rows in two goes: rows of 256 bytes, or pairs of rows of 128, that meet in a bank are apart
-  static __device__ __forceinline__ int turn(int r) { return R == 128 ? (r & 3) << 2 : R == 64 ? ((r >> 1) & 1) << 2 : 0; }
+  static __device__ __forceinline__ int turn(int r) { return R >= 128 ? (r & 3) << 2 : R == 64 ? ((r >> 1) & 1) << 2 : 0; }
+  __device__ __forceinline__ void piece(int i, int kq, uint32_t buf) const { dma16(from, src[i] + (uint32_t)kq * step, buf + dst + 1024 * i); }
   __device__ __forceinline__ void move(int kq, uint32_t buf) const {
 #pragma unroll
-    for (int i = 0; i < PIECES; ++i) dma16(from, src[i] + (uint32_t)kq * step, buf + dst + 1024 * i);
+    for (int i = 0; i < PIECES; ++i) piece(i, kq, buf);
   }
   // Rows r0 .. + 31 (row: the lane's l32), inner columns of slice j of 16: 8 h .. + 7 where both operands lie along it (PLAIN), else
   // 4 h .. + 3 and 8 + 4 h .. + 3
@@ -164,7 +167,8 @@ __global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(Nar
   constexpr int WM = TM > 32 ? 2 : 1, WN = TN > 32 ? 2 : 1, WK = 4 / (WM * WN), SLICES = 4 / WK;  // waves over rows, columns, slices of 16
   constexpr int MR = TM / 32 / WM, NR = TN / 32 / WN;                                            // pieces of 32 x 32 of a wave
   constexpr bool PLAIN = AK && BK;
-  __shared__ __attribute__((aligned(16))) char lds[4 * BUF];
+  constexpr int NB = 4 * BUF <= 160 * 1024 ? 4 : 3;  // buffers
+  __shared__ __attribute__((aligned(16))) char lds[NB * BUF];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wid % WM * 32 * MR, wn = wid / WM % WN * 32 * NR, wk = wid / (WM * WN);
   const int mt = (a.M + TM - 1) / TM, nt = (a.N + TN - 1) / TN, id = xcd_remap(blockIdx.x, gridDim.x);
@@ -180,7 +184,7 @@ __global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(Nar
   B ob;
   oa.init(a.a, a.abytes, a.lda, m0, lane, wid);
   ob.init(a.b, a.bbytes, a.ldb, n0, lane, wid);
-  auto buffer = [&](auto b_c) -> lds_char* { return (lds_char*)lds + (decltype(b_c)::value & 3) * BUF; };
+  auto buffer = [&](auto b_c) -> lds_char* { return (lds_char*)lds + decltype(b_c)::value % NB * BUF; };
   // where step i of this part stands in K; past the end the last one again
   auto place_in = [&](int i) {
     const int kq = min(i, steps - 1) + rot;
@@ -224,7 +228,7 @@ __global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(Nar
           for (int n = 0; n < NR; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[j][n], x[j][m], acc[m][n], 0, 0, 0);
     }
   };
-  if (rounds <= 3) {  // all at once
+  if (NB == 4 && rounds <= 3) {  // all at once
     move(0, Int<0>{});
     if (rounds > 1) move(1, Int<1>{});
     if (rounds > 2) move(2, Int<2>{});
@@ -236,54 +240,56 @@ __global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(Nar
     constexpr int PER = (A::PIECES + B::PIECES) * U;
     move(0, Int<0>{});
     move(1, Int<1>{});
-    move(2, Int<2>{});
+    if constexpr (NB == 4) move(2, Int<2>{});
     if constexpr (TM == 128) {
       bf16x8 x[2][MR], w[2][NR];
-      auto fetch = [&](auto b_c, int j, int s) {
+      // a product at a time, with a read of the next quarter and a transfer of step r + NB - 1 before each
+      auto read = [&](auto b_c, int j, int s, int i) {
         const lds_char* buf = buffer(b_c);
-#pragma unroll
-        for (int n = 0; n < NR; ++n) w[s][n] = ob.template read<PLAIN>(buf + A::BYTES, j, wn + 32 * n, lane);
-#pragma unroll
-        for (int m = 0; m < MR; ++m) x[s][m] = oa.template read<PLAIN>(buf, j, wm + 32 * m, lane);
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      auto multiply = [&](int s) {
-#pragma unroll
-        for (int m = 0; m < MR; ++m)
-#pragma unroll
-          for (int n = 0; n < NR; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[s][n], x[s][m], acc[m][n], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
+        if (i < NR) w[s][i] = ob.template read<PLAIN>(buf + A::BYTES, j, wn + 32 * i, lane);
+        else if (i < NR + MR) x[s][i - NR] = oa.template read<PLAIN>(buf, j, wm + 32 * (i - NR), lane);
       };
       auto round = [&](int r, auto b_c) {
         using Next = Int<decltype(b_c)::value + 1>;
-        const int kq = place_in(r + 3);
-        const uint32_t to = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)buffer(Int<decltype(b_c)::value + 3>{}));
-        fetch(b_c, 1, 1);
-        oa.move(kq, to);
-        multiply(0);
-        fetch(b_c, 2, 0);
-        ob.move(kq, to + A::BYTES);
-        multiply(1);
-        fetch(b_c, 3, 1);
-        multiply(0);
-        meet<2 * PER>();
-        fetch(Next{}, 0, 0);
-        multiply(1);
+        const int kq = place_in(r + NB - 1);
+        const uint32_t to = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)buffer(Int<decltype(b_c)::value + NB - 1>{}));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (q == 3) meet<(NB - 2) * PER>();
+#pragma unroll
+          for (int i = 0; i < MR * NR; ++i) {
+            if (q < 3) read(b_c, q + 1, (q + 1) & 1, i);
+            else read(Next{}, 0, 0, i);
+            constexpr int SLOTS = 3 * MR * NR;
+            const int slot = q * MR * NR + i;
+#pragma unroll
+            for (int p = 0; p < A::PIECES + B::PIECES; ++p)
+              if (q < 3 && p * SLOTS / (A::PIECES + B::PIECES) == slot) {
+                if (p < A::PIECES) oa.piece(p, kq, to);
+                else ob.piece(p - A::PIECES, kq, to + A::BYTES);
+              }
+            __builtin_amdgcn_sched_barrier(0);
+            const int m = i / NR, n = i % NR;
+            acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[q & 1][n], x[q & 1][m], acc[m][n], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
       };
-      meet<2 * PER>();
-      fetch(Int<0>{}, 0, 0);
+      meet<(NB - 2) * PER>();
+#pragma unroll
+      for (int i = 0; i < MR + NR; ++i) read(Int<0>{}, 0, 0, i);
       int r = 0;
-      for (; r + 4 <= rounds; r += 4) {
+      for (; r + NB <= rounds; r += NB) {
         round(r, Int<0>{});
         round(r + 1, Int<1>{});
         round(r + 2, Int<2>{});
-        round(r + 3, Int<3>{});
+        if constexpr (NB == 4) round(r + 3, Int<3>{});
       }
       if (r < rounds) {
         round(r, Int<0>{});
         if (r + 1 < rounds) {
           round(r + 1, Int<1>{});
-          if (r + 2 < rounds) round(r + 2, Int<2>{});
+          if (NB == 4 && r + 2 < rounds) round(r + 2, Int<2>{});
         }
       }
     } else {
@@ -309,7 +315,7 @@ __global__ void __launch_bounds__(256, TM == 128 ? 1 : 2) narrow_gemm_kernel(Nar
   const int l32 = lane & 31, h = lane >> 5;
   constexpr int ROW = TN * 4 + 16, PART = TM * ROW;  // bytes
   auto place = [&](int w, int m, int n) { return lds + w * PART + m * ROW + n * 4; };  // of row m, columns n .. of the wave group w
-  static_assert(WK * PART <= 4 * BUF, "room for the sums");
+  static_assert(WK * PART <= NB * BUF, "room for the sums");
 #pragma unroll
   for (int m = 0; m < MR; ++m)
 #pragma unroll
@@ -371,25 +377,46 @@ int g_tile = 0, g_parts = 0;
 struct Cut {
   int tm, tn, parts;  // tile, parts of K
 };
+
+// Rounds that the chip makes of tiles of 128 x 128, or 128 x 256, which take 1.8 times as long (dW of 3000 tokens, us: 256 of the first 25, of the
+// second 44): `wide` where those are the faster ones
+struct Rounds {
+  int64_t tiles;  // of 128 x 128
+  bool wide;
+  int full;       // percent of the chosen one's rounds that is work
+  int64_t count;  // ... and their number
+  Rounds(int64_t M, int64_t N) {
+    tiles = (M + 127) / 128 * ((N + 127) / 128);
+    const int64_t half = (M + 127) / 128 * ((N + 255) / 256), a = (tiles + 255) / 256, b = (half + 255) / 256;
+    wide = 9 * b < 5 * a;
+    count = wide ? b : a;
+    full = (int)(100 * (wide ? half : tiles) / (256 * count));
+  }
+};
 // us, on one machine, of 32-row tiles / 64 / 128, whole or in parts of K (x2, x4).
 // Both operands along K (y): 32 x 32 up to two tiles a CU (128 tokens by [3072, 1024] 6.4 / 6.4, [4096, 2048] 9.0 / 9.4, [5632, 1024] 8.6 / 6.7), 128 x
-// 128 from 140 of them on (512 by [5632, 1024] 13.3 with 64, 11.1; 768 by [3072, 1024], 144 of them, 13.1, 11.0; 200 by [8000, 1024], 126, 9.4, 10.7). Parts
-// of 2560 or more of K: a sum costs 2 us and its traffic (64 by [2048, 5632] 12.6, x2 10.5; [1024, 2816] 7.7, 7.7).
+// 128 from 126 of them on (512 by [5632, 1024] 13.5 with 64, 10.7; 768 by [3072, 1024], 144, 13.6, 10.4; 1000 by [2048, 2048], 128, 15.6, 15.4; 700, 96,
+// 15.1, 15.2). Parts of 2560 or more of K: a sum costs 2 us and its traffic (64 by [2048, 5632] 12.6, x2 10.5; [1024, 2816] 7.7, 7.7).
+// 128 x 256 by `Rounds` (us with 128, 256: y 500 by [11264, 2048] 33.4, 28.0; dX 700 by [2048, 5632] 33.0, 27.5; dW 3000 by [11264, 2048] 145, 124; in one
+// round anyhow, y 1000 by [4096, 4096], 34.3, 44.2).
 // From K = 4096 on weights come from memory and a CU's share of the operands bounds: 128 x 128 tiles, in parts of 768 or more, where those make
 // 192 to 256 workgroups (128 by [4096, 14336] 63.9 with 64x1, 34.8 with 128x8; by [6144, 4096] 22.2, 128x5 20.7; but 256 by [4096, 4096] 21.2
 // with 64x1, 128x4 22.4), else 64 x 64 in parts of 1024 or more (128 by [2048, 5632] 18.2 with 32x2, 13.9; by [1024, 8192] 18.4, 13.1).
 // One across (dX): those rows come in runs of 64 columns, never 32 (half a cache line). 64 x 64 from 160 tiles on, of long K from 64
-// (256 tokens by [5632, 1024] 32x2 13.0, 64x4 11.8; 512 17.5, 64x2 15.8; by [3072, 1024] 9.5, 10.5), 128 x 128 from 150 (800 by [1024, 2816], 154, 13.3 with
-// 64, 12.8; 300 by [2048, 5632], 132, 18.9, 19.5). Parts of 768 up to a workgroup a CU
+// (256 tokens by [5632, 1024] 32x2 13.0, 64x4 11.8; 512 17.5, 64x2 15.8; by [3072, 1024] 9.5, 10.5), 128 x 128 from 88 (1400 by [8000, 1024], 88, 57 with 64,
+// 49, x2 35; 600 by [1024, 2816], 110, 10.0, 10.5; 300 by [2048, 5632], 132, 19.6, 16.3). Parts of 768 up to a workgroup a CU, of 128 x 128 2560
 // (128 by [3072, 1024] 10.6, x2 9.4, x4 8.9; by [1024, 1024] 5.3, 6.4, 6.9).
-// Both across (dW): 64 x 64, 128 x 128 from 140 of them on (500 / 2000 / 8000 by [1536, 1536], 144, 9.0 / 21.7 / 77, 8.2 / 17.7 / 50; by [1024, 2048], 128, 6.7 /
-// 15.4 / 56, 8.1 / 17.8 / 50).
+// Both across (dW): 64 x 64, 128 x 128 from 140 of them on (500 / 2000 / 8000 by [1536, 1536], 144, 9.4 / 21.8 / 78, 8.0 / 16.7 / 49; 500 / 2000 by [1024, 2048],
+// 128, 7.3 / 15.9, 7.9 / 15.8).
 Cut cut_of(int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) {
   auto tiles = [&](int t, int u) { return ((M + t - 1) / t) * ((N + u - 1) / u); };
   const bool along = a_along && b_along, across = !a_along && !b_along;
   int tm = 32, tn = along ? 32 : 64;
-  if (tiles(128, 128) >= (along || across ? 140 : 150)) tm = tn = 128;
-  else if (along ? tiles(32, 32) > 512 : across || tiles(64, 64) >= (K >= 4096 ? 64 : 160)) tm = tn = 64;
+  const Rounds rounds(M, N);
+  if (rounds.tiles >= (along ? 126 : across ? 140 : 88)) {
+    tm = 128;
+    tn = rounds.wide ? 256 : 128;
+  } else if (along ? tiles(32, 32) > 512 : across || tiles(64, 64) >= (K >= 4096 ? 64 : 160)) tm = tn = 64;
   int64_t parts = 0;
   if (along && K >= 4096) {
     const int64_t big = tiles(128, 128), mid = tiles(64, 64), cut = std::min<int64_t>(256 / std::max<int64_t>(big, 1), 8);
@@ -404,15 +431,16 @@ Cut cut_of(int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) {
   if (g_tile) {
     tm = g_tile;
     tn = g_tile == 32 && !along ? 64 : g_tile;
+    if (g_tile == 256) tm = 128;
   }
-  if (!parts || g_tile) parts = std::min<int64_t>(std::min<int64_t>((along && tm < 128 ? 512 : 256) / tiles(tm, tn), K / (along ? 2560 : 768)), 8);
+  if (!parts || g_tile) parts = std::min<int64_t>(std::min<int64_t>((along && tm < 128 ? 512 : 256) / tiles(tm, tn), K / (along || tm == 128 ? 2560 : 768)), 8);
   if (g_parts) parts = std::min<int64_t>(g_parts, (K + 63) / 64);
   return {tm, tn, (int)std::max<int64_t>(parts, 1)};
 }
 
 }  // namespace
 
-// Forces tiles of 32, 64 or 128 rows and parts of K; 0: by the rule above.
+// Forces tiles of 32, 64 or 128 rows, or 128 x 256 (256), and parts of K; 0: by the rule above.
 extern "C" void ds_narrow_gemm_tune(int tile, int parts) { g_tile = tile; g_parts = parts; }
 
 // Whether the kernel takes the product: whole 16-byte pieces of rows, whole steps of 64 along an operand's rows, offsets of 32 bits
@@ -421,33 +449,43 @@ extern "C" int ds_narrow_gemm_ok(int64_t M, int64_t N, int64_t K, int64_t lda, i
   if (N % 8 || lda % 8 || ldb % 8 || ((a_along || b_along) && K % 64) || (!a_along && M % 8)) return 0;
   if (lda < (a_along ? K : M) || ldb < (b_along ? K : N)) return 0;
   const int64_t ar = a_along ? M : K, br = b_along ? N : K;
-  return (ar + 128) * lda * 2 < UINT32_MAX && (br + 128) * ldb * 2 < UINT32_MAX && ((M + 31) / 32) * ((N + 31) / 32) <= INT32_MAX;
+  return (ar + 128) * lda * 2 < UINT32_MAX && (br + 256) * ldb * 2 < UINT32_MAX && ((M + 31) / 32) * ((N + 31) / 32) <= INT32_MAX;
 }
 
 // Whether it is as fast as the library's there, us here (there).
-// y and dX: where 128 x 128 tiles, whole, nearly fill one round, 176 to 256 of them (y: 200 / 2000 by [11264, 2048] / [2048, 2048] 17.1 / 20.5 (21.7 / 21.6), 1000
-// by [4096, 4096] 34.4 (36.6), 4096 by [1024, 2816] 25.6 (28.2); dX: 500 by [2048, 5632] 20.6 (26.8), 800 by [4096, 4096] 36 (40), 2000 by [11264, 2048] 98
-// (105); 384 tiles, 3000 by [2048, 2048], 34 (27)), over weights of up to 2^26 or from 512 tokens on (160 by [16384, 8192] 95 (80)).
-// y besides: of K from 4096 on in three parts or more up to 128 tokens, in two up to 256 (128 by [4096, 14336] 36 (75), [6144, 4096] 21 (25), [8192, 8192]
-// 38 (50), 64 33 (34); 256 by [5120, 13824] 58 (120); 64 by [12288, 4096] in two 28.7 (26.7)); up to 128 tokens in 200 to 256 tiles with rows 8 KB
-// apart (64 / 128 by [28672, 4096] 47 / 53 (57 / 59); by [22016, 4096], 172 tiles, 44 / 53 (47 / 49)); up to 1024 2^31 products, of up to 2^24 weights 2^32 (512
-// by [8000, 1024] 13.7 (16.0); 128 by [11264, 2048] 21.6 (18.1)); up to 2048 by [1024, 1024] (1400 8.3 (10.3)).
-// dX besides: up to 1024 tokens 3 2^32 products and fewer than 3 2^20 results (500 by [11264, 2048] 41 (62), by [5632, 1024] 16 (26); 800 by the first 80
-// (78)); up to 2048 of 1024 columns, from 1800 on of any K (1400 by [3072, 1024] 23.6 (29.4), [5632, 1024] 40 (38); 2000 39 (45)).
-// dW: up to two rounds, up to 8192 tokens (1000 / 3000 / 8000 by [2048, 2048] 12.7 / 27 / 64 (21 / 43 / 88), [1024, 2816] 11.6 / 23 / 52 (20 / 40 / 82), [2048, 512] 6 /
-// 13 / 28.5 (13 / 28 / 53), [3072, 2048] 22 / 47 / 112 (27 / 57 / 113), [8000, 1024] 24 / 52 / - (32 / 63 / -)); nearly three up to 4096 (300 / 3000 by [2048,
-// 5632] 18 / 74 (28 / 87)), five and a half up to 3000 (1000 / 3000 by [11264, 2048] 64 / 148 (80 / 152)); four, [4096, 4096], 500 / 1000 28 / 44 (30 / 43).
+// dX, up to 9 2^20 results: up to 1024 tokens (500 by [2048, 2048] 10.5 (15.1), [11264, 2048] 42 (63), [4096, 4096] 27.5 (34.6); 1024 by [11264, 2048]
+// 54 (79), [4096, 4096] 35.5 (41.3), [12288, 4096] 94 (111)); up to 2048 in one round of 88 tiles or more (1400 / 2000 by [3072, 2048] 23.7 / 29.5 (28.4 /
+// 32.6), [8000, 1024] 35 / 44 (72 / 64)); beyond in one that is 62 % full (3000 / 4096 by [2048, 2048] 29.6 / 35.5 (30.2 / 36.4), 3000 by [11264, 2048] 125
+// (130), [32000, 2048] 393 (344)), or 88 % of several (2000 by [2048, 5632] 53.5 (55.2); 1032 by [5632, 8192], 75 %, 120 (96)).
+// dW: up to 768 tiles (256 / 1024 / 4096 by [2048, 2048] 7.8 / 14.5 / 35.7 (10 / 17.2 / 45.5), [2048, 5632] 17 / 34 / 93 (24 / 41 / 96), 8000 by [1024, 1024] 30 (56));
+// more of them from 1280 tokens on ([4096, 4096] 512 / 1024 / 2048 30 / 42 / 67 (26 / 40 / 67), 6000 by [12288, 4096] 480 (513)), five rounds and more from 704
+// ([11264, 2048] 768 / 3000 48 / 123 (62 / 150)). Its rows must not meet in memory channels: 32 KB apart ([16384, 2048] 320 45 (35)), or 8 and 16 KB ([12288,
+// 8192] 528 158 (149)). From 8192 tokens on the layer makes copies along them for the library.
+// y: in one round of 176 to 256 tiles of 128 x 128 (200 / 256 by [11264, 2048] 16.9 / 17.3 (22.4 / 23.7), 1000 by [4096, 4096] 34 (38), 2000 by [2048, 2048] 21.2
+// (22.4), 4096 by [1024, 2816] 26.2 (28.3); 175 by [16384, 1024] 14.1 (13.2)), over weights of up to 2^26 or from 512 tokens on (160 by [16384, 8192] 73 (65)); of
+// 128 x 256 over K up to 2048 (500 by [11264, 2048] 27.4 (31.1), 1400 by [4096, 2048] 27.8 (30.8); 320 by [16384, 2048] 28 (26), 3000 by [2048, 2048] 28.7 (28.3)); in
+// several over K up to 1024 (1400 / 2000 by [8000, 1024] 33.2 / 40.6 (34.9 / 42.2)). Of K from 4096 on in three parts or more up to 128 tokens, in two up to 256
+// (128 by [4096, 14336] 36 (75), [6144, 4096] 21 (25), [8192, 8192] 38 (50), 64 33 (34); 256 by [5120, 13824] 58 (120); 64 by [12288, 4096] in two 28.7 (26.7)); up to 128
+// tokens in 200 to 256 tiles with rows 8 KB apart (64 / 128 by [28672, 4096] 47 / 53 (57 / 59); by [22016, 4096], 172 tiles, 44 / 53 (47 / 49)). Else up to 1024
+// tokens 2^31 products, of up to 2^24 weights 2^32 (512 by [8000, 1024] 12.6 (17.2), [5632, 1024] 10.7 (14.1); 128 by [11264, 2048] 16.1 (16.5)), but not in more
+// than 256 of 64 x 64 (700 by [2048, 2048] 15.2 (13.8)); up to 2048 by [1024, 1024] (1400 8.9 (10.8)).
 extern "C" int ds_narrow_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along) {
-  const int64_t big = (N + 127) / 128, tiles = (M + 127) / 128 * big;
+  const Rounds rounds(M, N);
   if (!a_along) {
-    if (tiles <= 512) return K <= 8192;
-    return (tiles >= 640 && tiles <= 768 && K >= 256 && K <= 4096) || (tiles >= 1280 && tiles <= 1536 && K >= 256 && K <= 3000);
+    if (M % 16384 == 0 || (M % 4096 == 0 && N % 8192 == 0 && M * N > (1 << 25))) return 0;
+    return K <= 8192 && (rounds.tiles <= 768 || K >= 1280 || (K >= 704 && rounds.tiles >= 1280 && rounds.tiles <= 1536));
   }
-  if (M > 128 && tiles >= 176 && tiles <= 256 && (M > 512 || N * K <= (1 << 26))) return 1;
-  if (M > 1024) return M <= 2048 && N <= 1024 && (b_along ? K <= 1024 : K <= 3072 || M >= 1800);
-  if (!b_along) return M * N < (3 << 20) && M * N <= (3LL << 32) / K;
+  if (!b_along) {
+    if (M <= 1024 || M * N > (9 << 20)) return M * N <= (9 << 20);
+    return rounds.count == 1 ? (M <= 2048 ? rounds.tiles >= 88 : rounds.full >= 62 && K <= 16384) : rounds.full >= 88;
+  }
+  if (M >= 192 && rounds.count == 1 && !rounds.wide && rounds.tiles >= 176 && (M > 512 || N * K <= (1 << 26))) return 1;
+  if (M > 384 && rounds.count == 1 && rounds.wide) return rounds.full >= 62 && M <= 2048 && K <= 2048;
+  if (M > 256 && K >= 2048 && (M + 63) / 64 * ((N + 63) / 64) > 256) return 0;
+  if (M > 512 && M <= 2048 && K <= 1024 && N <= 8192 && rounds.full >= 90) return 1;
+  if (M > 1024) return M <= 2048 && N <= 1024 && K <= 1024;
   if (K >= 4096 && M <= 256 && cut_of(M, N, K, true, true).parts >= (M <= 128 ? 3 : 2)) return 1;
-  if (K % 4096 == 0 && M <= 128 && big >= 200 && big <= 256) return 1;
+  if (K % 4096 == 0 && M <= 128 && rounds.tiles >= 200 && rounds.tiles <= 256) return 1;
   return M * N <= (1LL << (N * K <= (1 << 24) ? 32 : 31)) / K;
 }
 
@@ -471,7 +509,12 @@ extern "C" int ds_narrow_gemm(const void* A, const void* B, void* C, int64_t M, 
                      nullptr, nullptr, -1, band_of((M + cut.tm - 1) / cut.tm, (N + cut.tn - 1) / cut.tn)};
   const dim3 grid((unsigned)(((M + cut.tm - 1) / cut.tm) * ((N + cut.tn - 1) / cut.tn)), cut.parts);
 #define GO(AK, BK, TM, TN, U) hipLaunchKernelGGL((narrow_gemm_kernel<AK, BK, TM, TN, U>), grid, dim3(256), 0, st, a)
-  if (cut.tm == 128) {
+  if (cut.tn == 256) {
+    if (a_along && b_along) GO(ALONG, ALONG, 128, 256, 1);
+    else if (a_along) GO(ALONG, ACROSS, 128, 256, 1);
+    else if (b_along) GO(ACROSS, ALONG, 128, 256, 1);
+    else GO(ACROSS, ACROSS, 128, 256, 1);
+  } else if (cut.tm == 128) {
     if (a_along && b_along) GO(ALONG, ALONG, 128, 128, 1);
     else if (a_along) GO(ALONG, ACROSS, 128, 128, 1);
     else if (b_along) GO(ACROSS, ALONG, 128, 128, 1);
@@ -505,7 +548,7 @@ Cut ordered_cut(int64_t M, int64_t N, int64_t K) {
   Cut c = {32, 32, 1};
   if (mid > 128) c = K >= 8192 ? Cut{128, 128, parts(big)} : Cut{64, 64, 1};
   else if (K >= 3072) c = mid >= (K >= 8192 ? 32 : 64) ? Cut{64, 64, parts(mid)} : Cut{32, 32, parts(low)};
-  if (g_tile) c.tm = c.tn = g_tile;
+  if (g_tile) c.tm = c.tn = std::min(g_tile, 128);
   if (g_parts) c.parts = (int)std::min<int64_t>(g_parts, K / 64);
   return c;
 }

@@ -48,6 +48,25 @@ def test_products_at_their_edges(M, N, K, tile, parts):
 
 
 @GPU
+@pytest.mark.parametrize("parts", [1, 2])
+@pytest.mark.parametrize("M,N,K", [(8, 8, 64), (72, 264, 128), (128, 256, 192), (136, 248, 256), (128, 520, 320), (264, 1032, 576)])
+def test_tiles_of_256_columns(M, N, K, parts):
+    """One step to several times as many as buffers; the last tile's second half empty, or short of columns; every form."""
+    test_products_at_their_edges(M, N, K, 256, parts)
+
+
+@GPU
+@pytest.mark.parametrize("M,N", [(2048, 2304), (2000, 4104), (1032, 4864), (2944, 5632)])
+def test_more_than_one_round(M, N):
+    """Where the rule goes from one round of 128 x 128 to one or two of 128 x 256, and back."""
+    a, b = _rnd(M, 192, seed=1), _rnd(N, 192, seed=2)
+    at, bt = a.t().contiguous(), b.t().contiguous()
+    _check(hip_ops().narrow_gemm(a, b, True, True), a, b)
+    _check(hip_ops().narrow_gemm(a, bt, True, False), a, b)
+    _check(hip_ops().narrow_gemm(at, bt, False, False), a, b)
+
+
+@GPU
 @pytest.mark.parametrize("M,N,K", [(52, 6152, 4096), (1, 6144, 4096), (128, 6200, 4160), (129, 4104, 8192), (256, 5120, 5120), (100, 2056, 5632),
                                    (33, 1024, 8192), (255, 4096, 4096), (300, 4096, 4160), (100, 25608, 4096), (129, 11264, 2048), (193, 14328, 4096)])
 def test_long_inner_dimensions(M, N, K):
