@@ -123,14 +123,21 @@ __device__ __forceinline__ uint4 pack8(const float (&v)[8]) {
   return r;
 }
 
+template <typename T>
+__device__ __forceinline__ void unpack8(u32x4 w, float (&v)[8]) {
+  const T* h = reinterpret_cast<const T*>(&w);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = (float)h[j];
+}
+
 // out[r, i] = act(g) * u, outT[i, r] the same values token-contiguous
 template <typename T, int A>
 __global__ void __launch_bounds__(256) gated_fwd_t_kernel(const T* __restrict__ gu, T* __restrict__ out,
                                                           T* __restrict__ outT, int64_t rows, int64_t Tp, int I,
                                                           int tiles_r, int tiles_c) {
   __shared__ uint32_t tile[GT_TS * GT_LROW];
-  const int bid = xcd_remap(blockIdx.x, gridDim.x);
-  const int tr = bid % tiles_r, tc = bid / tiles_r;
+  int tr, tc;
+  transpose_tile(tiles_r, tiles_c, tr, tc);
   const int r0 = tr * GT_TS, c0 = tc * GT_TS;
   const int t = threadIdx.x, lr = t >> 3, lc = t & 7;
 #pragma unroll
@@ -141,8 +148,8 @@ __global__ void __launch_bounds__(256) gated_fwd_t_kernel(const T* __restrict__ 
     uint4 v = make_uint4(0u, 0u, 0u, 0u);
     if (gr < rows && gc < I) {
       float g[8], u[8], o[8];
-      Vec8<T>::load(gu + gr * 2 * I + gc, g);
-      Vec8<T>::load(gu + gr * 2 * I + I + gc, u);
+      unpack8<T>(load_once(gu + gr * 2 * I + gc), g);
+      unpack8<T>(load_once(gu + gr * 2 * I + I + gc), u);
 #pragma unroll
       for (int j = 0; j < 8; ++j) o[j] = act_f<A>(g[j]) * u[j];
       v = pack8<T>(o);
@@ -162,8 +169,8 @@ __global__ void __launch_bounds__(256) gated_bwd_t_kernel(const T* __restrict__ 
                                                           int64_t Tp, int I, int tiles_r, int tiles_c) {
   __shared__ uint32_t tile_g[GT_TS * GT_LROW];
   __shared__ uint32_t tile_u[GT_TS * GT_LROW];
-  const int bid = xcd_remap(blockIdx.x, gridDim.x);
-  const int tr = bid % tiles_r, tc = bid / tiles_r;
+  int tr, tc;
+  transpose_tile(tiles_r, tiles_c, tr, tc);
   const int r0 = tr * GT_TS, c0 = tc * GT_TS;
   const int t = threadIdx.x, lr = t >> 3, lc = t & 7;
 #pragma unroll
@@ -174,9 +181,9 @@ __global__ void __launch_bounds__(256) gated_bwd_t_kernel(const T* __restrict__ 
     uint4 vg = make_uint4(0u, 0u, 0u, 0u), vu = vg;
     if (gr < rows && gc < I) {
       float g[8], u[8], d[8], dg[8], du[8];
-      Vec8<T>::load(gu + gr * 2 * I + gc, g);
-      Vec8<T>::load(gu + gr * 2 * I + I + gc, u);
-      Vec8<T>::load(dout + gr * I + gc, d);
+      unpack8<T>(load_once(gu + gr * 2 * I + gc), g);
+      unpack8<T>(load_once(gu + gr * 2 * I + I + gc), u);
+      unpack8<T>(load_once(dout + gr * I + gc), d);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         dg[j] = d[j] * u[j] * act_df<A>(g[j]);

@@ -6,8 +6,7 @@
 //
 // One workgroup moves a 64 x 64 tile: 16-B global loads along the input rows (8 lanes per 128-B row segment), the
 // tile parked in LDS with rows padded to 33 dwords (column reads by consecutive lanes hit consecutive banks), then
-// 16-B global stores along the output rows. Tiles are walked in an order that keeps each XCD on a contiguous band
-// of output rows.
+// 16-B global stores along the output rows.
 #include "../include/ds_hip.h"
 
 namespace {
@@ -19,19 +18,18 @@ __global__ void __launch_bounds__(256) transpose16_kernel(const uint16_t* __rest
                                                           int R, int Rp, int C, int64_t ld, int tiles_r,
                                                           int tiles_c) {
   __shared__ uint32_t tile[TS * LROW];
-  const int nwg = gridDim.x;
-  const int bid = xcd_remap(blockIdx.x, nwg);
-  const int tr = bid % tiles_r, tc = bid / tiles_r;  // consecutive ids walk down the input rows = along out rows
+  int tr, tc;
+  transpose_tile(tiles_r, tiles_c, tr, tc);
   const int r0 = tr * TS, c0 = tc * TS;
   const int t = threadIdx.x, lr = t >> 3, lc = t & 7;
   // load: rows lr and lr + 32, 8 x 16-bit at column 8 * lc
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
     const int r = lr + 32 * p, gr = r0 + r, gc = c0 + 8 * lc;
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (gr < R && gc < C) v = *reinterpret_cast<const uint4*>(in + (int64_t)gr * ld + gc);
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (gr < R && gc < C) v = load_once(in + (int64_t)gr * ld + gc);
     uint32_t* dst = tile + r * LROW + 4 * lc;
-    dst[0] = v.x; dst[1] = v.y; dst[2] = v.z; dst[3] = v.w;
+    dst[0] = v[0]; dst[1] = v[1]; dst[2] = v[2]; dst[3] = v[3];
   }
   __syncthreads();
   // store: output row oc = c0 + j holds input column j; 8 consecutive output elements = input rows 8 * lc .. + 7

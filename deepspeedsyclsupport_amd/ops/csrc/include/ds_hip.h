@@ -145,3 +145,16 @@ __device__ __forceinline__ int xcd_remap(int orig, int nwg) {
   const int q = nwg / 8, r = nwg % 8, xcd = orig % 8;
   return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + orig / 8;
 }
+
+// Tile of a transposing kernel's workgroup: an XCD's share in columns of 16 tiles, row by row. Single columns of tiles read 128 bytes of each row
+// (us on data that a product has just written, 8192 x 11008 / 8192 x 8192: transpose16 70 / 56, this 64 / 53, with `load_once` 63 / 45; gated_fwd_t
+// 147 / 104, 131 / 96, 120 / 92; gated_bwd_t 266 / 192, 244 / 181, 224 / 179; up to 3000 rows of 5632 the same).
+__device__ __forceinline__ void transpose_tile(int tiles_r, int tiles_c, int& tr, int& tc) {
+  const int id = xcd_remap(blockIdx.x, gridDim.x), col = id / (tiles_r * 16) * 16, w = min(16, tiles_c - col), in = id - col * tiles_r;
+  tr = in / w;
+  tc = col + in % w;
+}
+
+// 16 bytes that this kernel has no second use for
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x4 load_once(const void* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); }

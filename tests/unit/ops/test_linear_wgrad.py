@@ -35,6 +35,20 @@ def test_transpose16(R, C, ld):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("R,C", [(8, 8), (72, 1016), (128, 1024), (200, 1032), (64, 2056), (1024, 3112)])
+def test_transposing_tiles(R, C):
+    """A column of 16 tiles or less, whole columns of them, remainders of 1 and 17; rows short of a tile."""
+    from deepspeedsyclsupport_amd.ops.native import hip_ops
+    gu = torch.randn(R, 2 * C, device="cuda", generator=torch.Generator(device="cuda").manual_seed(R)).bfloat16()
+    assert torch.equal(hip_ops().transpose16(gu[:, 8:8 + C], R + 72)[:, :R], gu[:, 8:8 + C].t())
+    for act in (0, 1):
+        out, out_t = hip_ops().gated_act_fwd_t(gu, act, 256)
+        assert torch.equal(out, hip_ops().gated_act_fwd(gu, act)) and torch.equal(out_t[:, :R], out.t()) and not out_t[:, R:].any()
+        dgu, dgu_t = hip_ops().gated_act_bwd_t(out, gu, act, 256)
+        assert torch.equal(dgu, hip_ops().gated_act_bwd(out, gu, act)) and torch.equal(dgu_t[:, :R], dgu.t()) and not dgu_t[:, R:].any()
+
+
+@pytest.mark.gpu
 def test_kmajor_weight_grad_gpu():
     torch.manual_seed(0)
     T, n_in, n_out = 8200, 512, 384
