@@ -13,11 +13,12 @@
 //    units gave, at a fraction of their instructions); P . V stays on the vector units, with P in fp32: V rows are read
 //    whole, LPR lanes a row, and a row's probabilities reach its lanes through LDS. K and V of a group are loaded together
 //    (held a group ahead they cost the second workgroup of a CU, and time: 48 x 190 keys 16 us for 12);
+//  * where a workgroup a (sequence, head) leaves half of the CUs idle, two share its values (`launch_decode`);
 //  * a sequence is split only when that is long for one workgroup (see `ds_paged_decode_splits`): partial (max, sum,
 //    unnormalised acc) per split are merged by a small combine kernel (log-sum-exp). (An in-kernel last-block merge was
 //    measured 2x slower: the device-scope fences it needs write back L2.)
 // Measured, us (a workgroup of four waves per 64 to 1024 keys, scores and softmax in LDS between barriers; the read at 6.5 TB/s), 8
-// kv heads of 128: 1 sequence of 130 keys, 4 heads each 6 (14; 0.1), 1 of 8192 19 (44; 5), 12 of 700, 2 heads each 11 (20; 5),
+// kv heads of 128: 1 sequence of 130 keys, 4 heads each 6 (14; 0.1), 1 of 8192 19 (44; 5), 12 of 700, 2 heads each 10 (20; 5),
 // 48 of 190, 4 each 12 (24; 6), 48 of 1024 42 (74; 31), 256 of 512 96 (183; 83). A step's rotation and append in it: 0.5 to 1 us, a
 // kernel of their own 4 to 8.
 // Optional ALiBi slopes (BLOOM) are applied on the fly. With a sliding window (Mistral) or chunked visibility only the
@@ -87,15 +88,17 @@ __device__ __forceinline__ bf16x8_t rope_chunk(const bf16* head, int chunk, cons
 
 // DK, DV: the widths; 0: given at run time. LPR: lanes that hold a row, 8 elements each (the width / 8 rounded up to a power of two). GT: at least the query heads served. NEW: the step's
 // projection comes as it is: queries are turned here, and the last key and value are taken from it and written to the cache.
-template <int DK, int DV, int GT, int LPR, bool NEW>
+// VP: workgroups that share a head's values, each with all of its keys.
+template <int DK, int DV, int GT, int LPR, bool NEW, int VP>
 __global__ void __launch_bounds__(THREADS, 2) paged_decode_kernel(DecodeArgs a) {
   constexpr bool EXT = DK == 0;
   static_assert(EXT || (DK % 16 == 0 && DK >= 64 && DK <= 256 && DK == DV), "head dim");
-  const int dk = EXT ? a.dk : DK, dv = EXT ? a.dv : DV;
+  static_assert(VP == 1 || (!EXT && DV == 8 * LPR), "values in parts");
+  const int dk = EXT ? a.dk : DK, dv = EXT ? a.dv : DV / VP, ldv = dv * VP;
   // [WAVES][GT][dv] accumulators, [WAVES][GT][2] maxima and sums, [WAVES][KEYS + 1][GT] probabilities and the fade of what was;
   // NEW: [GT + 2][dk] rows of the step
   extern __shared__ __attribute__((aligned(16))) float sm[];
-  const int b = blockIdx.x, kh = EXT ? blockIdx.y % a.Hk : blockIdx.y, split = blockIdx.z, S = gridDim.z;
+  const int b = blockIdx.x, kh = EXT ? blockIdx.y % a.Hk : blockIdx.y, split = blockIdx.z / VP, S = gridDim.z / VP, v0 = blockIdx.z % VP * dv;
   const int g0 = EXT ? blockIdx.y / a.Hk * MAXG : 0;          // first query head of the group this block serves
   const int GA = a.Hq / a.Hk, G = EXT ? min(MAXG, GA - g0) : GA, h0 = kh * GA + g0;
   const int T = a.seq_lens[b];
@@ -116,9 +119,9 @@ __global__ void __launch_bounds__(THREADS, 2) paged_decode_kernel(DecodeArgs a) 
       qf[kk] = *reinterpret_cast<const bf16x8_t*>(a.q + ((int64_t)b * a.Hq + h0 + min(l16, G - 1)) * dk + min(4 * kk + q4, dk / 8 - 1) * 8);
   }
   const float slope = !EXT && a.alibi && mine ? a.alibi[h0 + l16] : 0.f;
-  // values: LPR lanes cover one row, 8 elements each
-  constexpr int RPW = 64 / LPR, UV = KEYS / RPW;              // rows per wave instruction, instructions
-  const int sub = lane / LPR, li = lane % LPR, lv = min(li, dv / 8 - 1);
+  // values: lanes cover one row, 8 elements each
+  constexpr int LV = LPR / VP, RPW = 64 / LV, UV = KEYS / RPW;  // lanes of a row, rows per wave instruction, instructions
+  const int sub = lane / LV, li = lane % LV, lv = min(li, dv / 8 - 1);
   float acc[GT][8], m = -INFINITY, l = 0.f;                   // m, l: of head l16
 #pragma unroll
   for (int g = 0; g < GT; ++g)
@@ -154,7 +157,7 @@ __global__ void __launch_bounds__(THREADS, 2) paged_decode_kernel(DecodeArgs a) 
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) f.k[kk] = *reinterpret_cast<const bf16x8_t*>(kr + min(4 * kk + q4, dk / 8 - 1) * 8);
 #pragma unroll
-    for (int u = 0; u < UV; ++u) f.v[u] = *reinterpret_cast<const bf16x8_t*>(a.vc + row(t + u * RPW + sub, blk.v[u]) * dv + lv * 8);
+    for (int u = 0; u < UV; ++u) f.v[u] = *reinterpret_cast<const bf16x8_t*>(a.vc + row(t + u * RPW + sub, blk.v[u]) * ldv + v0 + lv * 8);
   };
   auto attend = [&](int t, int t1, const Group& f) {
     f32x4 s{0.f, 0.f, 0.f, 0.f};
@@ -215,7 +218,7 @@ __global__ void __launch_bounds__(THREADS, 2) paged_decode_kernel(DecodeArgs a) 
       const int64_t p = a.rot ? (int64_t)a.pos[b] * (a.rot / 2) : 0;
       const bf16x8_t x = rope_chunk(a.q + ((int64_t)b * (a.Hq + 2 * a.Hk) + head) * dk, c, a.cosT + p, a.sinT + p, rot, a.interleaved);
       *reinterpret_cast<bf16x8_t*>(rows + row * dk + c * 8) = x;
-      if (last && row >= G) {
+      if (last && row >= G && v0 == 0) {
         const int block = bt[a.bs_shift >= 0 ? (T - 1) >> a.bs_shift : (T - 1) / a.BS];
         const int64_t at = ((int64_t)block * a.Hk + kh) * a.BS + (a.bs_shift >= 0 ? (T - 1) & (a.BS - 1) : (T - 1) % a.BS);
         *reinterpret_cast<bf16x8_t*>((row == G ? a.kc : a.vc) + at * dk + c * 8) = x;
@@ -245,7 +248,7 @@ __global__ void __launch_bounds__(THREADS, 2) paged_decode_kernel(DecodeArgs a) 
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) f.k[kk] = *reinterpret_cast<const bf16x8_t*>(rows + G * dk + min(4 * kk + q4, dk / 8 - 1) * 8);
 #pragma unroll
-    for (int u = 0; u < UV; ++u) f.v[u] = *reinterpret_cast<const bf16x8_t*>(rows + (G + 1) * dk + lv * 8);
+    for (int u = 0; u < UV; ++u) f.v[u] = *reinterpret_cast<const bf16x8_t*>(rows + (G + 1) * dk + v0 + lv * 8);
     attend(T - 1, T, f);
   }
   // ---- the lane groups of a wave meet in registers (they share their maxima), the waves in LDS
@@ -259,7 +262,7 @@ __global__ void __launch_bounds__(THREADS, 2) paged_decode_kernel(DecodeArgs a) 
   for (int g = 0; g < GT; ++g) {
     if (g >= G) break;
 #pragma unroll
-    for (int o = LPR; o < 64; o *= 2)
+    for (int o = LV; o < 64; o *= 2)
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[g][j] += __shfl_xor(acc[g][j], o, 64);
     if (sub == 0 && li < dv / 8) {
@@ -287,11 +290,11 @@ __global__ void __launch_bounds__(THREADS, 2) paged_decode_kernel(DecodeArgs a) 
         r = num * f / fmaf(den, f, __expf(a.sink[hq] - mn));
       }
       if (EXT && a.gate) r /= 1.f + __expf(-(float)a.gate[b * a.ldg + hq]);
-      a.out[(int64_t)b * a.ldo + hq * dv + d] = (bf16)r;
+      a.out[(int64_t)b * a.ldo + hq * ldv + v0 + d] = (bf16)r;
     } else {
       const int64_t at = ((int64_t)b * a.Hq + hq) * S + split;
-      a.part_acc[at * dv + d] = num;
-      if (d == 0) {
+      a.part_acc[at * ldv + v0 + d] = num;
+      if (v0 + d == 0) {
         a.part_ml[at * 2] = mx;
         a.part_ml[at * 2 + 1] = den;
       }
@@ -461,15 +464,15 @@ extern "C" int ds_paged_decode_splits(int B, int Hk, int max_len) {
 
 namespace {
 
-template <int DK, int DV, int LPR, bool NEW, int GT>
-int launch_decode(const DecodeArgs& a, dim3 grid, hipStream_t s) {
+template <int DK, int DV, int LPR, bool NEW, int GT, int VP>
+int launch_parts(const DecodeArgs& a, dim3 grid, hipStream_t s) {
   const int dv = DK ? DV : a.dv;
-  const int lds = WAVES * GT * (dv + 2 + KEYS + 1) * (int)sizeof(float) + (NEW ? (GT + 2) * dv * 2 : 0);
-  auto* kernel = &paged_decode_kernel<DK, DV, GT, LPR, NEW>;
+  const int lds = WAVES * GT * (dv / VP + 2 + KEYS + 1) * (int)sizeof(float) + (NEW ? (GT + 2) * dv * 2 : 0);
+  auto* kernel = &paged_decode_kernel<DK, DV, GT, LPR, NEW, VP>;
   if (lds > 65536 &&
       hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
     return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(kernel, grid, dim3(THREADS), lds, s, a);
+  hipLaunchKernelGGL(kernel, dim3(grid.x, grid.y, grid.z * VP), dim3(THREADS), lds, s, a);
   DS_CHECK_LAUNCH();
   if (grid.z > 1) {
     hipLaunchKernelGGL(combine_kernel, dim3((unsigned)grid.x * a.Hq), dim3(dv), 0, s, a.part_acc, a.part_ml, a.out, a.sink, a.gate,
@@ -477,6 +480,17 @@ int launch_decode(const DecodeArgs& a, dim3 grid, hipStream_t s) {
     DS_CHECK_LAUNCH();
   }
   return 0;
+}
+
+// Values in two parts where that leaves no CU with more than one workgroup: a CU reads 60 B/ns at most, here three quarters of what it had to, and
+// needs no second launch. us whole / in parts, 12 sequences of 33 / 300 / 700 keys: 8 key heads of 128, 2 query heads each 4.8 / 8.0 / 13.0, 4.6 /
+// 7.5 / 12.0; 4 each 5.6 / 9.1 / 14.7, 6.1 / 9.1 / 13.9 (hence from 384 keys there); 4 of 256, 4 each 6.6 / 12.3 / 25.0, 6.1 / 11.3 / 20.2.
+template <int DK, int DV, int LPR, bool NEW, int GT>
+int launch_decode(const DecodeArgs& a, dim3 grid, hipStream_t s) {
+  if constexpr (DK >= 128) {
+    if (grid.z == 1 && grid.x * grid.y <= 128 && a.chunk >= (DK == 128 && GT >= 4 ? 384 : 0)) return launch_parts<DK, DV, LPR, NEW, GT, 2>(a, grid, s);
+  }
+  return launch_parts<DK, DV, LPR, NEW, GT, 1>(a, grid, s);
 }
 
 // by the query heads a workgroup serves

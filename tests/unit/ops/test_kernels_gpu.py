@@ -476,6 +476,27 @@ def test_paged_decode_step_equals_append_and_attention(D, rot, interleaved, wind
     torch.testing.assert_close(got.float(), want.float(), rtol=1e-2, atol=1e-2)
 
 
+@pytest.mark.parametrize("D,hq,hk", [(128, 4, 4), (128, 16, 8), (128, 32, 8), (128, 40, 5), (256, 3, 3), (256, 12, 6), (256, 16, 2)])
+def test_paged_decode_values_in_parts(D, hq, hk):
+    """Up to 128 (sequence, key head) two workgroups share a head's values, one more of them and none does (bounds as above); the
+    step's key and value are written once."""
+    for B in (128 // hk, 128 // hk + 1):
+        BS, lens = 32, [(1, 15, 16, 17, 127, 129, 330, 400, 513, 700, 768)[i % 11] for i in range(B)]
+        kc, vc, bt, maxb = _paged_setup(B, hk, D, BS, lens, seed=8)
+        sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+        pos, seqs = sl - 1, torch.arange(B, dtype=torch.int32, device="cuda")
+        tables = R.rope_tables(1024, D, device="cuda")
+        qkv = torch.randn(B, (hq + 2 * hk) * D, device="cuda", generator=torch.Generator(device="cuda").manual_seed(9)).bfloat16()
+        k2, v2 = kc.clone(), vc.clone()
+        q = ops().qkv_rope_append(qkv, *tables, pos, k2, v2, bt, pos, 1, hq, hk, D, False, False, seqs)[0]
+        ref = _paged_ref(q.double(), k2.double(), v2.double(), bt, lens, D**-0.5)
+        out = ops().paged_decode(q, k2, v2, bt, sl, max(lens), D**-0.5, None, 0)
+        assert ((out.double() - ref).abs() <= 2.0**-8 * ref.abs() + 2e-4).all()
+        got = ops().paged_decode_step(qkv, *tables, pos, kc, vc, bt, sl, max(lens), D**-0.5, None, 0, hq, D, False)
+        assert torch.equal(vc, v2)
+        torch.testing.assert_close(got.float(), out.float(), rtol=1e-2, atol=1e-2)
+
+
 def test_kv_append():
     B, n, hk, D, BS = 3, 5, 4, 128, 16
     kc, vc, bt, maxb = _paged_setup(B, hk, D, BS, [64, 64, 64])
