@@ -555,12 +555,12 @@ Cut ordered_cut(int64_t M, int64_t N, int64_t K) {
 }  // namespace
 
 // Whether ds_narrow_ordered takes x [M, K] by w [N, K] in operand order, and is the faster way. Not over short K from 4096 rows on (33 rows by [8192,
-// 2048] 11.3, before 10.4), nor where the weights' read is what counts ([16384, 8192] 55, before 49; [32000, 4096] 52.5, 53.5, with 33 rows 51
+// 2048] 11.3, before 10.4), nor 33 to 40 by [8192, 4096], 128 tiles in two parts (18.2 and 18.5, before 16.3 and 17.6), nor where the weights' read is what counts ([16384, 8192] 55, before 49; [32000, 4096] 52.5, 53.5, with 33 rows 51
 // and 50). Up to 32 rows small products (24 by [2048, 2048] 6.0, before 6.9, [3072, 1024] 4.8, 5.4; [4096, 2048] 7.8, 7.3) and those a quarter over
 // one round of single blocks (24 by [5120, 5120] 14.4, 16.5).
 extern "C" int ds_narrow_ordered_ok(int64_t M, int64_t N, int64_t K) {
   if (M > 48 || N <= 0 || N > 16384 || N % 8 || K <= 0 || K % 64 || N * K > (3 << 25)) return 0;
-  if (M > 32) return K >= 3072 || N <= 4096;
+  if (M > 32) return (K >= 3072 && (M > 40 || N <= 6144 || N > 8192 || K > 4096)) || N <= 4096;
   return (M > 20 && K <= 2048 && N * K <= (1 << 22)) || (M > 16 && N > 4096 && N <= 5440 && K >= 4096 && K < 8192);
 }
 
