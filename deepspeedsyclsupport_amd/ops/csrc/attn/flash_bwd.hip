@@ -31,13 +31,13 @@
 //  * too few sweeps to fill the chip (short sequences of grouped-query models) are cut into parts that leave fp32 dK / dV in a
 //    workspace; a second launch adds them up in a fixed order. B3 Hq16 Hk4 S1000 causal (48 workgroups uncut): 313 -> 103 us.
 // Measured (tools/bench_flash_bwd.py, profiles/flash_bwd_bench_r2_final.jsonl): B8 H32 S4096 D128 causal 4.2-4.3 ms
-// (round-2 start: 4.58). SQ PMC of the round-2 start: ~29 % MFMA busy, ~9 VALU per MFMA -- the VALU issue slots, not
+// (before the trims above: 4.58). SQ PMC before them: ~29 % MFMA busy, ~9 VALU per MFMA -- the VALU issue slots, not
 // the matrix pipe, are what the trims above (packed converts, pre-scaled row constants, uniform mask skip) buy back.
 // Where the time goes now: the dQ sum. Every 32-row query tile receives one 16-KB fp32 tile-add per 256-key block it
 // meets: B8 H32 S4096 causal = 278.5k tile-adds = 4.56 GB of float atomics, and the memory-side atomic units retire
 // ~1.3 TB/s chip-wide (one 256-B wave-instruction per ~50 ns per CU), i.e. a 3.5 ms floor for the main kernel at
 // this key-block size whatever the MFMA loop does (measured 3.8 ms + 0.3 ms pre/post; 4 heads x 32k: floor 3.3 ms,
-// measured 3.9 + 0.3). Pipelining the S / dP operand reads two MFMAs ahead (round 3) therefore bought only 2 %.
+// measured 3.9 + 0.3). Pipelining the S / dP operand reads two MFMAs ahead therefore bought only 2 %.
 // Going below the floor needs fewer adds per dQ element (512 keys per workgroup: the dK/dV accumulators no longer
 // fit two waves per SIMD) or bf16 atomics (2-3x the rounding error on dQ) -- neither taken.
 // Tried and measured slower: dQ partial stores + a summing pass instead of atomics (5.5 ms), pairing heavy and light
