@@ -359,7 +359,7 @@ struct Cut {
 // Up to 16 rows parts pay at the ends alone: where a few blocks leave most CUs idle (16 rows x [1024, 4096] 8.7 and 7.7, 2 rows 6.1 and
 // 6.9, x [1024, 8192] 9.6 and 8.4), and where long ones stand a quarter over one round (16 rows x [10240, 8192] 40 and 35); from 12 rows on
 // also over long K, in two blocks, which halve the reading of X (12 / 16 rows x [2048, 5632] 10.4 / 11.7 and 9.5 / 9.7, [4096, 14336] 23.7 / 26.0 and 22.8 / 23.3,
-// [5120, 13824] 29.9 / 31.6 and 27.6 / 28.5, [3072, 8192] 13.9 / 15.4 and 14.0 / 14.4).
+// [5120, 13824] 29.9 / 31.6 and 27.6 / 28.5, [3072, 8192] 13.9 / 15.4 and 14.0 / 14.4; not [4096, 6144] 12.4 / 13.5 and 13.3 / 13.7).
 Cut cut_of(int M, int N, int K, bool gated, bool norm) {
   const int blocks = gated ? N / 16 : (N + 15) / 16, mt = (M + 15) / 16, most = gated || mt > 1 ? 4 : 2;
   const int eights = (blocks + 7) / 8;  // workgroups of eight blocks
@@ -369,7 +369,7 @@ Cut cut_of(int M, int N, int K, bool gated, bool norm) {
     int fill = 0;  // workgroups that parts may make
     if (mt == 1) {
       fill = blocks <= 64 && (K >= 8192 || (M > 8 && K >= 4096)) ? 256 : blocks > 512 && blocks <= 680 && K >= 8192 ? 1024 : 0;
-      if (M >= 12 && blocks > 64 && blocks <= 340 && K >= (blocks <= 256 ? 5120 : 8192)) {
+      if (M >= 12 && blocks > 64 && blocks <= 340 && K >= (blocks <= 128 ? 5120 : 8192)) {
         rb = 2;
         fill = blocks <= 256 ? 256 : 512;
       }
