@@ -459,7 +459,9 @@ extern "C" int ds_narrow_gemm_ok(int64_t M, int64_t N, int64_t K, int64_t lda, i
 // (130), [32000, 2048] 393 (344)), or 88 % of several (2000 by [2048, 5632] 53.5 (55.2); 1032 by [5632, 8192], 75 %, 120 (96)).
 // dW: up to 768 tiles (256 / 1024 / 4096 by [2048, 2048] 7.8 / 14.5 / 35.7 (10 / 17.2 / 45.5), [2048, 5632] 17 / 34 / 93 (24 / 41 / 96), 8000 by [1024, 1024] 30 (56));
 // more of them from 1280 tokens on ([4096, 4096] 512 / 1024 / 2048 30 / 42 / 67 (26 / 40 / 67), 6000 by [12288, 4096] 480 (513)), five rounds and more from 704
-// ([11264, 2048] 768 / 3000 48 / 123 (62 / 150)). Its rows must not meet in memory channels: 32 KB apart ([16384, 2048] 320 45 (35)), or 8 and 16 KB ([12288,
+// ([11264, 2048] 768 / 3000 48 / 123 (62 / 150)); of token counts that are no whole 32, which the library pays for (100 by [22016, 4096] 64 (98), [4096, 11008]
+// 37 (52), [11264, 2048] 22 (26), [32000, 2048] 49 (53); 500 41 (47) by [6144, 4096], 98 (99) by [32000, 2048]; 333 by [4096, 4096] 32 (24), 900 by [27648,
+// 5120] 312 (292)). Its rows must not meet in memory channels: 32 KB apart ([16384, 2048] 320 45 (35)), or 8 and 16 KB ([12288,
 // 8192] 528 158 (149)). From 8192 tokens on the layer makes copies along them for the library.
 // y: in one round of 176 to 256 tiles of 128 x 128 (200 / 256 by [11264, 2048] 16.9 / 17.3 (22.4 / 23.7), 1000 by [4096, 4096] 34 (38), 2000 by [2048, 2048] 21.2
 // (22.4), 4096 by [1024, 2816] 26.2 (28.3); 175 by [16384, 1024] 14.1 (13.2)), over weights of up to 2^26 or from 512 tokens on (160 by [16384, 8192] 73 (65)); of
@@ -473,7 +475,9 @@ extern "C" int ds_narrow_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along,
   const Rounds rounds(M, N);
   if (!a_along) {
     if (M % 16384 == 0 || (M % 4096 == 0 && N % 8192 == 0 && M * N > (1 << 25))) return 0;
-    return K <= 8192 && (rounds.tiles <= 768 || K >= 1280 || (K >= 704 && rounds.tiles >= 1280 && rounds.tiles <= 1536));
+    if (K > 8192) return 0;
+    if (rounds.tiles <= 768 || K >= 1280 || (K >= 704 && rounds.tiles >= 1280 && rounds.tiles <= 1536)) return 1;
+    return K % 32 && (K <= 256 || (rounds.tiles <= 6000 && (K >= 500 || (rounds.tiles > 1024 && rounds.tiles < 3000))));
   }
   if (!b_along) {
     if (M <= 1024 || M * N > (9 << 20)) return M * N <= (9 << 20);
