@@ -35,8 +35,9 @@ bool unwatched(const Tensor& a, const Tensor& b) {
 }
 
 // A B^T over the inner dimension: a [M, K], or [K, M] if not a_along; b [N, K], or [K, N]. Undefined where the kernel does not take it
-// or (unless asked to take what it can) the library's is faster.
-Tensor narrow_product(const Tensor& a, const Tensor& b, bool a_along, bool b_along, bool any) {
+// or (unless asked to take what it can) the library's is faster. sizes: the result's where it is no matrix (a view of one, made in an autograd
+// function, could not be changed in place).
+Tensor narrow_product(const Tensor& a, const Tensor& b, bool a_along, bool b_along, bool any, at::OptionalIntArrayRef sizes = c10::nullopt) {
   if (!a.is_cuda() || a.device() != b.device() || a.scalar_type() != at::kBFloat16 || b.scalar_type() != at::kBFloat16 || a.dim() != 2 || b.dim() != 2 ||
       a.stride(1) != 1 || b.stride(1) != 1)
     return Tensor();
@@ -46,7 +47,7 @@ Tensor narrow_product(const Tensor& a, const Tensor& b, bool a_along, bool b_alo
     return Tensor();
   const char *pa = (const char*)a.const_data_ptr(), *pb = (const char*)b.const_data_ptr();
   if ((uintptr_t)pa % 16 || (uintptr_t)pb % 16) return Tensor();
-  Tensor c = torch::empty({M, N}, a.options());
+  Tensor c = torch::empty(sizes ? *sizes : at::IntArrayRef{M, N}, a.options());
   const int64_t scratch = ds_narrow_gemm_scratch(M, N, K, a_along, b_along);
   const Tensor part = scratch ? torch::empty({scratch}, a.options().dtype(at::kByte)) : Tensor();
   const int rc = ds_narrow_gemm(pa, pb, c.data_ptr(), M, N, K, lda, ldb, a_along, b_along, scratch ? part.data_ptr() : nullptr,
@@ -58,12 +59,10 @@ Tensor narrow_product(const Tensor& a, const Tensor& b, bool a_along, bool b_alo
 // x [.., I] W [O, I]^T
 Tensor linear_product(Tensor x, Tensor w) {
   if (unwatched(x, w) && x.dim() >= 2 && x.is_contiguous() && w.dim() == 2 && x.size(-1) == w.size(1) && x.numel()) {
-    const Tensor y = narrow_product(x.view({-1, x.size(-1)}), w, true, true, false);
-    if (y.defined()) {
-      auto sizes = x.sizes().vec();
-      sizes.back() = w.size(0);
-      return y.view(sizes);
-    }
+    auto sizes = x.sizes().vec();
+    sizes.back() = w.size(0);
+    const Tensor y = narrow_product(x.view({-1, x.size(-1)}), w, true, true, false, sizes);
+    if (y.defined()) return y;
   }
   return at::linear(x, w);
 }

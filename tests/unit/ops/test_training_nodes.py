@@ -137,6 +137,47 @@ def _grads_free(f, inputs):
     return out if isinstance(out, (tuple, list)) else (out, )
 
 
+@pytest.mark.parametrize("case", CASES, ids=lambda c: c.__name__[1:])
+def test_outputs_change_in_place(case):
+    """Outputs may be changed in place where the function's may, and the gradients are the function's."""
+    node, function, inputs = case()
+
+    def run(f):
+        try:
+            out = f(*inputs)
+            first = out[0] if isinstance(out, (tuple, list)) else out
+            return True, torch.autograd.grad(first.mul_(2).float().sum(), inputs, allow_unused=True)
+        except RuntimeError:
+            return False, ()
+    (ok, a), (want, b) = run(node), run(function)
+    assert ok == want
+    _same(a, b, case is not _flash)
+
+
+@pytest.mark.parametrize("lead", [(96, ), (2, 48), (1, 96)])
+def test_linear_changes_in_place(lead):
+    """A linear layer's output of a short batch, changed in place by itself and through views, as torch's may be."""
+    x, w, go = _leaf(*lead, 128), _leaf(256, 128, seed=1), _rnd(*lead, 256, seed=2)
+    rows = lambda y: y.view(-1, 8, 32)[:, 2:5]  # noqa: E731
+
+    def changed(f):
+        y = f(x, w)
+        y.mul_(2)
+        y += go
+        rows(y).relu_()
+        return y
+    want = torch.nn.functional.linear(x, w)
+    for f in (L.linear, lambda a, b: L.LinearFunction.apply(a, b, None, None)):
+        y, z = changed(f), 2 * f(x, w) + go
+        mask = torch.ones_like(z)
+        rows(mask)[rows(z) <= 0] = 0
+        assert torch.equal(y, z * mask)
+        for a, b in zip(torch.autograd.grad(y, (x, w), go), torch.autograd.grad(z * mask, (x, w), go)):
+            assert torch.equal(a, b)
+        # (sums of 128 products in fp32, one rounding on either side)
+        assert ((f(x, w).float() - want.float()).abs() <= 2**-7 * want.float().abs() + 1e-4).all()
+
+
 def test_released_weight():
     """A weight whose storage is released after the forward pass and filled again before the backward one, as gathered weights are."""
     x, w = _leaf(8, 64), torch.nn.Parameter(_rnd(24, 64, seed=1))
