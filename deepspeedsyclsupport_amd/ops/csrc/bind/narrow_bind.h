@@ -47,6 +47,7 @@ Tensor narrow_product(const Tensor& a, const Tensor& b, bool a_along, bool b_alo
     return Tensor();
   const char *pa = (const char*)a.const_data_ptr(), *pb = (const char*)b.const_data_ptr();
   if ((uintptr_t)pa % 16 || (uintptr_t)pb % 16) return Tensor();
+  const c10::DeviceGuard guard(a.device());  // (the stream below is the tensors' device's, whichever is current)
   Tensor c = torch::empty(sizes ? *sizes : at::IntArrayRef{M, N}, a.options());
   const int64_t scratch = ds_narrow_gemm_scratch(M, N, K, a_along, b_along);
   const Tensor part = scratch ? torch::empty({scratch}, a.options().dtype(at::kByte)) : Tensor();

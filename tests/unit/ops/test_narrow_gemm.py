@@ -145,6 +145,31 @@ def test_linear_layer(lead):
 
 
 @GPU
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="tensors beside the current device")
+def test_products_on_another_device():
+    """Short products run on their tensors' device and its stream, in order with what made the tensors there, while another is current."""
+    from deepspeedsyclsupport_amd.ops import hybrid_ops
+    from deepspeedsyclsupport_amd.ops.linear import input_grad, linear, weight_grad
+    a, b, go = _rnd(128, 1024, seed=1), _rnd(1024, 1024, seed=2), _rnd(128, 1024, seed=3)
+    want = hip_ops().narrow_gemm(a, b, True, True), hip_ops().narrow_gemm(go, b, True, False), hip_ops().narrow_gemm(go, a, False, False)
+    side = torch.cuda.Stream(1)
+    with torch.cuda.stream(side):
+        slow = torch.randn(4096, 4096, device="cuda:1")
+        for _ in range(20):
+            slow = slow @ slow * 1e-2
+        x, w, g = (t.to("cuda:1") for t in (a, b, go))
+        x, w, g = ((t + 0 * slow[0, 0].nan_to_num(0, 0, 0).to(t.dtype)) for t in (x, w, g))
+        torch.cuda.set_device(0)
+        assert torch.cuda.current_stream(1) == side
+        got = [f(x, w) for f in (plain_linear, hybrid_ops.linear, linear)], input_grad(g, w), weight_grad(g, x)
+    side.synchronize()
+    for t in got[0]:
+        assert t.device.index == 1 and torch.equal(t.to("cuda:0"), want[0])
+    assert torch.equal(got[1].to("cuda:0"), want[1]) and torch.equal(got[2].to("cuda:0"), want[2])
+    assert torch.cuda.current_device() == 0
+
+
+@GPU
 def test_linear_layer_leaves_what_it_does_not_take():
     """Other types, odd widths, unaligned and strided inputs, empty ones, long ones: torch's answer."""
     def same(x, w):
