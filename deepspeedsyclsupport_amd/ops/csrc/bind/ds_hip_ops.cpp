@@ -813,8 +813,8 @@ struct LinearNode : Node<LinearNode> {
 };
 // x W^T of fewer than `rows` tokens
 OptT linear_node(Tensor x, Tensor w, int64_t rows) {
-  if (!bf16_rows(x) || x.dim() < 2 || x.numel() / x.size(-1) >= rows || !w.is_cuda() || w.scalar_type() != at::kBFloat16 || w.dim() != 2 ||
-      w.device() != x.device() || w.size(1) != x.size(-1) || !unseen({&x, &w}))
+  if (!unseen({&x, &w}) || !bf16_rows(x) || x.dim() < 2 || x.numel() / x.size(-1) >= rows || !w.is_cuda() || w.scalar_type() != at::kBFloat16 ||
+      w.dim() != 2 || w.device() != x.device() || w.size(1) != x.size(-1))
     return c10::nullopt;
   return LinearNode::apply(x, w);
 }
@@ -840,8 +840,8 @@ struct RmsNormNode : Node<RmsNormNode> {
 };
 std::optional<std::vector<Tensor>> rms_norm_node(Tensor x, Tensor w, double eps, OptT residual) {
   const Tensor none, &r = residual.has_value() ? *residual : none;
-  if (!bf16_rows(x) || !w.is_cuda() || w.scalar_type() != at::kBFloat16 || !w.is_contiguous() || w.device() != x.device() ||
-      (r.defined() && (!bf16_rows(r) || r.device() != x.device() || r.sizes() != x.sizes())) || !unseen({&x, &w, &r}))
+  if (!unseen({&x, &w, &r}) || !bf16_rows(x) || !w.is_cuda() || w.scalar_type() != at::kBFloat16 || !w.is_contiguous() ||
+      w.device() != x.device() || (r.defined() && (!bf16_rows(r) || r.device() != x.device() || r.sizes() != x.sizes())))
     return c10::nullopt;
   return RmsNormNode::apply(x, w, eps, residual);
 }
@@ -857,7 +857,7 @@ struct GatedActNode : Node<GatedActNode> {
   }
 };
 OptT gated_act_node(Tensor gu, int64_t act) {
-  if (!bf16_rows(gu) || !unseen({&gu})) return c10::nullopt;
+  if (!unseen({&gu}) || !bf16_rows(gu)) return c10::nullopt;
   return GatedActNode::apply(gu, act);
 }
 
@@ -881,7 +881,7 @@ struct QkvRopeNode : Node<QkvRopeNode> {
 std::optional<std::vector<Tensor>> qkv_rope_node(Tensor qkv, Tensor cos, Tensor sin, OptT pos, int64_t hq, int64_t hk, int64_t rot, int64_t offset,
                                                  bool token_major) {
   const Tensor none, &p = pos.has_value() ? *pos : none;
-  if (!bf16_rows(qkv) || !unseen({&qkv, &cos, &sin, &p}) || cos.requires_grad() || sin.requires_grad()) return c10::nullopt;
+  if (!unseen({&qkv, &cos, &sin, &p}) || !bf16_rows(qkv) || cos.requires_grad() || sin.requires_grad()) return c10::nullopt;
   return QkvRopeNode::apply(qkv, cos, sin, pos, hq, hk, rot, offset, token_major);
 }
 

@@ -18,7 +18,8 @@ void ds_narrow_gemm_tune(int, int);
 namespace {
 using torch::Tensor;
 
-// No transform, dispatch mode, tracer or autocast has to see what becomes of these tensors, and none carries a tangent or a lazy bit
+// No transform, dispatch mode, tracer or autocast has to see what becomes of these tensors, and none carries a tangent or a lazy bit or is
+// anything but strided (asked first: such tensors may have no sizes)
 bool unseen(std::initializer_list<const Tensor*> ts) {
   using K = c10::DispatchKey;
   static const c10::DispatchKeySet special({K::Python, K::PythonTLSSnapshot, K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Batched,
@@ -26,7 +27,7 @@ bool unseen(std::initializer_list<const Tensor*> ts) {
   if (!(c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty() || at::autocast::is_autocast_enabled(at::kCUDA))
     return false;
   for (const Tensor* t : ts)
-    if (t->defined() && (t->key_set().has_any(special) || t->_fw_grad(0).defined())) return false;
+    if (t->defined() && (t->key_set().has_any(special) || t->layout() != at::kStrided || t->is_nested() || t->_fw_grad(0).defined())) return false;
   return true;
 }
 // ... nor autograd

@@ -188,6 +188,22 @@ def test_linear_layer_leaves_what_it_does_not_take():
 
 
 @GPU
+@pytest.mark.parametrize("layout", [torch.strided, torch.jagged])
+def test_nested_inputs(layout):
+    """Sequences of unequal length in one nested tensor, which torch's linear takes."""
+    from deepspeedsyclsupport_amd.ops import hybrid_ops
+    from deepspeedsyclsupport_amd.ops.linear import linear
+    parts, w = [_rnd(3, 128), _rnd(5, 128, seed=1)], _rnd(64, 128, seed=2)
+    x = torch.nested.nested_tensor(parts, layout=layout)
+    with torch.no_grad():
+        for f in (plain_linear, hybrid_ops._plain, linear, lambda a, b: LinearFunction.apply(a, b, None, None)):
+            y = f(x, w)
+            assert y.is_nested and y.layout == layout
+            for got, want in zip(y.unbind(), F.linear(x, w).unbind()):
+                assert torch.equal(got, want)
+
+
+@GPU
 @pytest.mark.parametrize("T,W,N", [(49, 256, 512), (100, 4096, 6144), (200, 2048, 2048), (1500, 256, 256)])
 def test_products_of_hybrid_decoders(T, W, N):
     """Short prompts of the hybrid decoders take the same products, longer ones and fp32 torch's."""
