@@ -76,6 +76,6 @@ def attention(q, k, v, causal=True, softmax_scale=None, attn_mask=None, dropout_
     """q [B, Hq, S, D], k/v [B, Hk, S, D] -> o [B, Hq, S, D]."""
     if flash_supported(q, k, v, attn_mask, dropout_p):
         scale = softmax_scale if softmax_scale is not None else q.shape[-1]**-0.5
-        o = hip_ops().flash_node(q, k, v, bool(causal), float(scale)) if unseen_from_python() else None
+        o = hip_ops().flash_node(q, k, v, bool(causal), float(scale)) if unseen_from_python(q, k, v) else None
         return FlashAttnFunc.apply(q, k, v, causal, scale) if o is None else o
     return _sdpa(q, k, v, causal, softmax_scale, attn_mask, dropout_p)

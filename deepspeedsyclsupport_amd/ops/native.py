@@ -7,20 +7,17 @@ implementations in `ops/reference.py` instead, which is the only place non-nativ
 import functools
 
 import torch
+from torch.overrides import has_torch_function_variadic
 
 from . import op_builder
 
 DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 
 
-# (no public predicate says that a torch function mode is on)
-_function_modes = torch._C._len_torch_function_stack
-
-
-def unseen_from_python():
-    """Whether neither a torch function mode nor the compiler has to see the torch calls behind an op (dispatch modes, transforms,
-    tracers and autocast are looked for in the extension)."""
-    return not _function_modes() and not torch.compiler.is_compiling()
+def unseen_from_python(*tensors):
+    """Whether neither the compiler nor a torch function, a mode's or one of these tensors' own, has to see the torch calls behind an op
+    (dispatch modes, transforms, tracers and autocast are looked for in the extension)."""
+    return not torch.compiler.is_compiling() and not has_torch_function_variadic(*tensors)
 
 
 @functools.lru_cache(None)

@@ -54,7 +54,7 @@ def rms_norm(x, weight, eps=1e-6, residual=None):
         x = x.contiguous()
         if residual is not None:
             residual = residual.contiguous()
-        if unseen_from_python():
+        if unseen_from_python(x, weight, residual):
             out = hip_ops().rms_norm_node(x, weight, eps, residual)  # (the same in C++, for bf16)
             if out is not None:
                 return out[0] if residual is None else tuple(out)
@@ -142,7 +142,7 @@ def gated_activation(gate_up, act="silu"):
             out._ds_kmajor = out_t
             return out
         gate_up = gate_up.contiguous()
-        out = hip_ops().gated_act_node(gate_up, code) if unseen_from_python() else None
+        out = hip_ops().gated_act_node(gate_up, code) if unseen_from_python(gate_up) else None
         return _GatedActFn.apply(gate_up, code) if out is None else out
     g, u = gate_up.chunk(2, dim=-1)
     return reference.ACTS[code](g) * u
@@ -236,7 +236,7 @@ def qkv_rope_split(qkv, cos, sin, num_heads, num_kv_heads, rotary_dim=None, posi
     if qkv.is_cuda and D % 8 == 0 and rot % 16 == 0:
         pos = position_ids.to(torch.int32).contiguous() if position_ids is not None else None
         args = (qkv.contiguous(), cos, sin, pos, num_heads, num_kv_heads, rot, pos_offset, token_major)
-        out = hip_ops().qkv_rope_node(*args) if unseen_from_python() else None
+        out = hip_ops().qkv_rope_node(*args) if unseen_from_python(*args[:4]) else None
         return _QKVRopeFn.apply(*args) if out is None else tuple(out)
     q, k, v = qkv.split([num_heads, num_kv_heads, num_kv_heads], dim=2)
     p = position_ids if position_ids is not None else torch.arange(pos_offset, pos_offset + S, device=qkv.device)
@@ -359,7 +359,7 @@ def cross_entropy(logits, labels, ignore_index=-100, label_smoothing=0.0, reduct
         # 430
         if reduction not in ("none", "sum") and labels2.numel() <= XENT_MEAN_MAX:
             args = (logits2, labels2, ignore_index, label_smoothing, inplace_backward)
-            mean = hip_ops().xent_mean_node(*args) if unseen_from_python() else None
+            mean = hip_ops().xent_mean_node(*args) if unseen_from_python(logits2, labels2) else None
             return _XentMeanFn.apply(*args) if mean is None else mean
         per_tok = _XentFn.apply(logits2, labels2, ignore_index, label_smoothing, inplace_backward)
     else:

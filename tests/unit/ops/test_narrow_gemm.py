@@ -187,6 +187,34 @@ def test_linear_layer_leaves_what_it_does_not_take():
         torch.testing.assert_close(plain_linear(x, w).float(), F.linear(x, w).float(), rtol=2**-6, atol=2**-4)
 
 
+class _Seen(torch.Tensor):
+    """A subclass that sees torch's calls by `__torch_function__` alone."""
+    calls = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        _Seen.calls.append(getattr(func, "__name__", ""))
+        return super().__torch_function__(func, types, args, kwargs or {})
+
+
+@GPU
+@pytest.mark.parametrize("which", [(True, False), (False, True), (True, True)])
+def test_subclasses_with_a_torch_function(which):
+    """They see torch's linear, and what comes out is one of them."""
+    from deepspeedsyclsupport_amd.ops import hybrid_ops
+    from deepspeedsyclsupport_amd.ops.linear import input_grad, linear, weight_grad
+    x, w, go = _rnd(96, 128), _rnd(64, 128, seed=1), _rnd(96, 64, seed=2)
+    sx, sw = (t.as_subclass(_Seen) if s else t for t, s in zip((x, w), which))
+    for f in (plain_linear, hybrid_ops._plain, linear, lambda a, b: LinearFunction.apply(a, b, None, None)):
+        _Seen.calls.clear()
+        y = f(sx, sw)
+        assert type(y) is _Seen and "linear" in _Seen.calls and torch.equal(y.as_subclass(torch.Tensor), F.linear(x, w))
+    for f, a, b in ((input_grad, go, sw), (weight_grad, go, sx)):
+        if isinstance(b, _Seen):
+            _Seen.calls.clear()
+            assert type(f(a, b)) is _Seen and "mm" in _Seen.calls
+
+
 @GPU
 @pytest.mark.parametrize("layout", [torch.strided, torch.jagged])
 def test_nested_inputs(layout):
