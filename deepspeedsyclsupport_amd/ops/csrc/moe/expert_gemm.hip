@@ -29,10 +29,6 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.f + expf(-g)) * u; }
-// By the hardware's exponential and reciprocal; the quarter keeps the latter's result a normal number
-__device__ __forceinline__ float silu_mul_fast(float g, float u) {
-  return 0.25f * g * __builtin_amdgcn_rcpf(fmaf(0.25f, __expf(-g), 0.25f)) * u;
-}
 enum : int { NONE = 0, SILU_GLU = 1, RELU2 = 2 };  // activation codes
 __device__ __forceinline__ float plain_act(float x, int act) {
   if (act != RELU2) return x;
@@ -374,7 +370,7 @@ __global__ void __launch_bounds__(256, 2) expert_tile_kernel(ExpertArgs a) {
         bf16x4 o;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          o[i] = (bf16)(GLU ? silu_mul_fast(acc[0][m][4 * q + i], acc[1][m][4 * q + i]) : plain_act(acc[t][m][4 * q + i], a.act));
+          o[i] = (bf16)(GLU ? silu_mul(acc[0][m][4 * q + i], acc[1][m][4 * q + i]) : plain_act(acc[t][m][4 * q + i], a.act));
         *reinterpret_cast<bf16x4*>(yr + n + 8 * q + 4 * hh) = o;
       }
     }
@@ -396,9 +392,10 @@ __global__ void __launch_bounds__(256, 2) expert_tile_kernel(ExpertArgs a) {
 //  * rows in units of 64 (MT): a short tile moves and multiplies no others.
 // Workgroups walk groups of 8 column tiles by all row tiles of an expert. Then bound by power: 1.6 GHz, matrix cores busy 77 % of the time in
 // a long loop; without any transfers 1.75 GHz and 83 %. 16 x 16 x 32 products: hipcc moves accumulators about, 1.05 times the time.
-// 32 experts, 1024 rows each on average, at random: 3584 gated columns of 4096: 1805 -> 1600 us (all even 1680 -> 1490), 4096 plain columns of
-// 3584: 978 -> 891 us (eight waves, both operands in LDS, a wait for all transfers every step); 256 rows: 657 -> 574; 8 x 128 rows: 111 -> 92.
-// Of these the gate by the hardware's exponential and reciprocal 4 % (32 outputs a lane and tile, 8 us), finding the place in registers 2 %.
+// 32 experts, 1024 rows each on average, at random: 3584 gated columns of 4096: 1812 -> 1683 us (all even 1680 -> 1561), 4096 plain columns of
+// 3584: 990 -> 880 us (eight waves, both operands in LDS, a wait for all transfers every step); 256 rows: 655 -> 579; 8 x 128 rows: 115 -> 97.
+// Finding the place in registers is 2 % of it. A gate by the hardware's exponential and reciprocal would be another 3 to 5 % (1617, 1510), but its error
+// grows as |g| 2^-24, past that of expf and a division from |g| = 5 on.
 constexpr int TM = 256, TN = 256;
 typedef __attribute__((address_space(3))) char lds_char;
 typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
@@ -560,7 +557,7 @@ __global__ void __launch_bounds__(256, 1) expert_big_kernel(ExpertArgs a) {
           bf16x4 o;
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            o[i] = (bf16)(GLU ? silu_mul_fast(acc[0][m][4 * q + i], acc[1][m][4 * q + i]) : plain_act(acc[t][m][4 * q + i], a.act));
+            o[i] = (bf16)(GLU ? silu_mul(acc[0][m][4 * q + i], acc[1][m][4 * q + i]) : plain_act(acc[t][m][4 * q + i], a.act));
           *reinterpret_cast<bf16x4*>(yr + n + 8 * q + 4 * h) = o;
         }
       }
@@ -607,13 +604,13 @@ __global__ void __launch_bounds__(256) expert_sum_kernel(const T* __restrict__ y
   }
 }
 
-// Rows per expert on average from which 256-row tiles pay. Measured against the tile kernel, gated / plain, times as fast: 32 experts of 3584 by
-// 4096, 96 rows 0.97 / 0.98, 128 rows 1.25 / 1.39, 256 rows 1.21 / 1.31; 32 of 1408 by 2048, 96 rows 0.88 / 1.28, 128 rows 0.90 / 1.45, 192
-// rows 1.11 / 1.16; 8 of 3584 by 4096, 128 rows 1.55 / 1.67. The host knows the average alone. What is far from it costs up to 256 rows (an
-// eighth of 32 experts of 3584 by 4096 with 83 % of the rows: 128 on average 1.08 / 0.92, 192 0.93 / 0.96, 320 1.16 / 1.08), and so does
-// exactly 128 rows each where they fill the smaller tiles and the chip (32 of 3584 by 4096 0.98 / 0.96, of 1408 by 2048 0.88 / 1.24). A
-// choice on the device, one large tile or two small ones per workgroup, lost more than it saved: two small ones behind one barrier take
-// 1.25 times as long as in two workgroups.
+// Rows per expert on average from which 256-row tiles pay: of 864 products of 128 to 1024 rows (12 sets of 8 to 256 experts, gated and plain, four
+// distributions of the rows) 717 are faster with them by more than 4 %, 91 slower. Their time by that of 128-row tiles, median and worst: shares at
+// random, 128 rows 0.78 and 1.16, 192 rows 0.84 and 0.99, 512 rows 0.82 and 1.24 (a last round of few tiles), 1024 rows 0.81 and 0.97. All even 1.01 and 1.16
+// with 128 rows, which fill the smaller tiles, 0.75 and 0.88 with 160. An eighth of the experts with 83 % of the rows 1.01 and 1.31 with 128, 1.10 and
+// 1.33 with 160, 1.08 and 1.48 with 192, 1.02 and 1.48 with 256, 0.89 and 1.07 with 320, 0.94 and 1.17 with 384: the host knows the
+// average alone. With 96 it goes either way (even shares, gated 32 of 1408 by 2048 1.18, 8 of 3584 by 4096 0.71). A choice on the device, one large tile or two small ones
+// per workgroup, lost more than it saved: two small ones behind one barrier take 1.25 times as long as in two workgroups.
 constexpr int BIG_ROWS = 128;
 
 template <bool GLU>

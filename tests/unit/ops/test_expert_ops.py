@@ -286,6 +286,28 @@ def test_big_tiles_over_steps(K, act):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [128, 64])
+def test_gates_of_tiles_are_exact_to_fp32(rows):
+    """Both tile kernels' silu(g) u over gates from -80 to 20. Rows of the unit matrix make every product a weight, exactly, so that only
+    the gate's own error is there: expf is good to 1 ulp (2^-23), sum, quotient and product round by 2^-24 each, which makes less
+    than 3 2^-23 together. A result has to be what a value that close rounds to."""
+    from deepspeedsyclsupport_amd.ops.expert_ops import ACTS, expert_ops, operand_order
+    E, N, K = 2, 256, 64
+    n, d = rows * E, 3 * 2.0**-23
+    experts = torch.arange(n, dtype=torch.int32, device="cuda") // rows
+    order, offs = torch.arange(n, dtype=torch.int32, device="cuda"), torch.arange(E + 1, dtype=torch.int32, device="cuda") * rows
+    x = torch.eye(K, device="cuda").bfloat16().repeat(n // K, 1)
+    for seed in range(4):
+        gen = torch.Generator(device="cuda").manual_seed(seed)
+        w = torch.cat([torch.rand(E, N, K, device="cuda", generator=gen) * 100 - 80, 1 + torch.rand(E, N, K, device="cuda", generator=gen)], 1).bfloat16()
+        y = expert_ops().expert_gemm(x, operand_order(w), experts, offs, order, 1, ACTS["silu_glu"], True, True)
+        z = w.double()[experts.long(), :, torch.arange(n, device="cuda") % K]
+        z = z[:, :N] * torch.sigmoid(z[:, :N]) * z[:, N:]
+        ends = torch.stack([(z * (1 - d)).bfloat16(), (z * (1 + d)).bfloat16()]).sort(0).values
+        assert ((ends[0] <= y) & (y <= ends[1])).all()
+
+
+@pytest.mark.gpu
 def test_big_tiles_leave_long_inputs():
     """Rows that 32 bits of bytes do not reach go by the tile kernel."""
     from deepspeedsyclsupport_amd.ops.expert_ops import expert_ops, operand_order
