@@ -372,7 +372,7 @@ int band_of(int64_t mt, int64_t nt) {
   return (int)std::min(band, mt);
 }
 
-int g_tile = 0, g_parts = 0;
+thread_local int g_tile = 0, g_parts = 0;  // (a thread's own: another's products go by the rules, and keep to the scratch they asked for)
 
 struct Cut {
   int tm, tn, parts;  // tile, parts of K
@@ -440,7 +440,7 @@ Cut cut_of(int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) {
 
 }  // namespace
 
-// Forces tiles of 32, 64 or 128 rows, or 128 x 256 (256), and parts of K; 0: by the rule above.
+// Forces tiles of 32, 64 or 128 rows, or 128 x 256 (256), and parts of K, for the calling thread's products; 0: by the rule above.
 extern "C" void ds_narrow_gemm_tune(int tile, int parts) { g_tile = tile; g_parts = parts; }
 
 // Whether the kernel takes the product: whole 16-byte pieces of rows, whole steps of 64 along an operand's rows, offsets of 32 bits

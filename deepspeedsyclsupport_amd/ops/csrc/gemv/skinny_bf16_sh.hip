@@ -328,7 +328,7 @@ __global__ void __launch_bounds__(256) unshuffle_sh16_kernel(const bf16* __restr
   *reinterpret_cast<bf16x8*>(W + row * KQ * 64 + kq * 64 + 16 * (lane >> 4) + 8 * h) = v;
 }
 
-int g_blocks = 0, g_parts = 0;
+thread_local int g_blocks = 0, g_parts = 0;  // (a thread's own: another's products go by the rules, and keep to the scratch they asked for)
 
 struct Cut {
   int blocks, parts;  // blocks of 16 weight rows per workgroup, parts of K
@@ -412,7 +412,8 @@ int launch(const ShArgs& a, bool gated, bool loose, hipStream_t st) {
 
 }  // namespace
 
-// Forces blocks per workgroup (1, 2, 4, 8, where the product has such a kernel) and parts of K; 0: by the rule above.
+// Forces blocks per workgroup (1, 2, 4, 8, where the product has such a kernel) and parts of K, for the calling thread's products; 0: by
+// the rule above.
 extern "C" void ds_skinny_b16_tune(int cfg, int parts) { g_blocks = cfg; g_parts = parts; }
 
 extern "C" int ds_decode_gemm_ok(int M, int K) { return M >= 1 && M <= 48 && K >= 64 && K % 64 == 0; }

@@ -108,6 +108,28 @@ def test_values_that_do_not_mix():
     _check(hip_ops().narrow_gemm(big[:37, :40], big[:37, 40:104], False, False), big[:37, :40].t(), big[:37, 40:104].t())
 
 
+def test_tuning_is_a_threads_own():
+    """What one thread forces for a measurement leaves another's products, and the scratch memory that they ask for, as they are."""
+    import ctypes
+    import threading
+    from deepspeedsyclsupport_amd.ops import op_builder
+    op_builder.load("ds_hip_ops")
+    lib = ctypes.CDLL(op_builder.so_path("ds_hip_ops"))
+    lib.ds_narrow_gemm_scratch.restype = lib.ds_decode_gemm_scratch.restype = ctypes.c_int64
+    n = ctypes.c_int64
+    query = lambda: (lib.ds_narrow_gemm_scratch(n(128), n(1024), n(1024), 1, 1), lib.ds_decode_gemm_scratch(4, 2048, 2048, 0, 0))  # noqa: E731
+    before, seen = query(), []
+
+    def other():
+        lib.ds_narrow_gemm_tune(32, 8)
+        lib.ds_skinny_b16_tune(1, 8)
+        seen.append(query())
+    thread = threading.Thread(target=other)
+    thread.start()
+    thread.join()
+    assert all(s > b for s, b in zip(seen[0], before)) and query() == before
+
+
 @GPU
 @pytest.mark.parametrize("lead", [(2, 33), (128, )])
 def test_linear_layer(lead):
