@@ -56,6 +56,7 @@ Tensor decode_linear_sh(Tensor x, Tensor wsh, int64_t N, std::optional<double> g
   TORCH_CHECK(NB * K < ((int64_t)1 << 40) && N < ((int64_t)1 << 31) / 16, "decode_linear_sh: matrix too large");
   TORCH_CHECK(!(glu && act.has_value()), "decode_linear_sh: one epilogue");
   TORCH_CHECK(!glu || N % 2 == 0, "decode_linear_sh: [gate | up] rows");
+  if ((uintptr_t)x.data_ptr() % 16) x = x.clone();  // (its rows go to LDS in pieces of 16 bytes as they lie)
   auto sizes = x.sizes().vec();
   sizes.back() = glu ? N / 2 : N;
   auto y = torch::empty(sizes, x.options());
