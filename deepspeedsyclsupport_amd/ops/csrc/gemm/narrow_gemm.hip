@@ -452,45 +452,72 @@ extern "C" int ds_narrow_gemm_ok(int64_t M, int64_t N, int64_t K, int64_t lda, i
   return (ar + 128) * lda * 2 < UINT32_MAX && (br + 256) * ldb * 2 < UINT32_MAX && ((M + 31) / 32) * ((N + 31) / 32) <= INT32_MAX;
 }
 
-// Whether it is as fast as the library's there, us here (there).
-// dX, up to 9 2^20 results: up to 1024 tokens (500 by [2048, 2048] 10.5 (15.1), [11264, 2048] 42 (63), [4096, 4096] 27.5 (34.6); 1024 by [11264, 2048]
-// 54 (79), [4096, 4096] 35.5 (41.3), [12288, 4096] 94 (111)); up to 2048 in one round of 88 tiles or more (1400 / 2000 by [3072, 2048] 23.7 / 29.5 (28.4 /
-// 32.6), [8000, 1024] 35 / 44 (72 / 64)); beyond in one that is 62 % full (3000 / 4096 by [2048, 2048] 29.6 / 35.5 (30.2 / 36.4), 3000 by [11264, 2048] 125
-// (130), [32000, 2048] 393 (344)), or 88 % of several (2000 by [2048, 5632] 53.5 (55.2); 1032 by [5632, 8192], 75 %, 120 (96)).
-// dW: up to 768 tiles (256 / 1024 / 4096 by [2048, 2048] 7.8 / 14.5 / 35.7 (10 / 17.2 / 45.5), [2048, 5632] 17 / 34 / 93 (24 / 41 / 96), 8000 by [1024, 1024] 30 (56));
-// more of them from 1280 tokens on ([4096, 4096] 512 / 1024 / 2048 30 / 42 / 67 (26 / 40 / 67), 6000 by [12288, 4096] 480 (513)), five rounds and more from 704
-// ([11264, 2048] 768 / 3000 48 / 123 (62 / 150)); of token counts that are no whole 32, which the library pays for (100 by [22016, 4096] 64 (98), [4096, 11008]
-// 37 (52), [11264, 2048] 22 (26), [32000, 2048] 49 (53); 500 41 (47) by [6144, 4096], 98 (99) by [32000, 2048]; 333 by [4096, 4096] 32 (24), 900 by [27648,
-// 5120] 312 (292)). Its rows must not meet in memory channels: 32 KB apart ([16384, 2048] 320 45 (35)), or 8 and 16 KB ([12288,
-// 8192] 528 158 (149)). From 8192 tokens on the layer makes copies along them for the library.
-// y: in one round of 176 to 256 tiles of 128 x 128 (200 / 256 by [11264, 2048] 16.9 / 17.3 (22.4 / 23.7), 1000 by [4096, 4096] 34 (38), 2000 by [2048, 2048] 21.2
-// (22.4), 4096 by [1024, 2816] 26.2 (28.3); 175 by [16384, 1024] 14.1 (13.2)), over weights of up to 2^26 or from 512 tokens on (160 by [16384, 8192] 73 (65)); of
-// 128 x 256 over K up to 2048 (500 by [11264, 2048] 27.4 (31.1), 1400 by [4096, 2048] 27.8 (30.8); 320 by [16384, 2048] 28 (26), 3000 by [2048, 2048] 28.7 (28.3)); in
-// several over K up to 1024 (1400 / 2000 by [8000, 1024] 33.2 / 40.6 (34.9 / 42.2)). Of K from 4096 on in three parts or more up to 128 tokens, in two up to 256
-// (128 by [4096, 14336] 36 (75), [6144, 4096] 21 (25), [8192, 8192] 38 (50), 64 33 (34); 256 by [5120, 13824] 58 (120); 64 by [12288, 4096] in two 28.7 (26.7)); up to 128
-// tokens in 200 to 256 tiles with rows 8 KB apart (64 / 128 by [28672, 4096] 47 / 53 (57 / 59); by [22016, 4096], 172 tiles, 44 / 53 (47 / 49)). Else up to 1024
-// tokens 2^31 products, of up to 2^24 weights 2^32 (512 by [8000, 1024] 12.6 (17.2), [5632, 1024] 10.7 (14.1); 128 by [11264, 2048] 16.1 (16.5)), but not in more
-// than 256 of 64 x 64 (700 by [2048, 2048] 15.2 (13.8)); up to 2048 by [1024, 1024] (1400 8.9 (10.8)).
+// Whether the kernel is as fast as the library's, for each product of a linear layer of `tokens` rows by a weight [out, in]; us here (there).
+// A cost model was not found that orders the library's side, which jumps with its own choice of tiles. What the lines go by is stated with each:
+// whole rounds of the chip (`Rounds`), which products of its size the library is bad at, and rows that meet in memory channels. On 300 layers at
+// random (33 to 8000 tokens, widths of 256 to 32768, none of which the lines were drawn by) 601 products go here, 580 of them faster by more than 4 %, 4
+// slower by as much (12.6 (12.1), 37.6 (30.1), 46.5 (43.2), 28.6 (27.0)); y / dX / dW of all 300 take 0.86 / 0.73 / 0.61 of the library's time in the mean
+// (profiles/narrow_products_at_random.csv).
+namespace {
+
+// y: a tile's operands come as the library's do; what is gained is its launch, and tiles that fill the chip.
+bool y_pays(int64_t tokens, int64_t out, int64_t in, const Rounds& rounds) {
+  const bool one = rounds.count == 1;
+  // one round of 128 x 128 that is 69 % full (200 / 256 by [11264, 2048] 16.9 / 17.3 (22.4 / 23.7), 1000 by [4096, 4096] 34 (38), 4096 by [1024, 2816]
+  // 26.2 (28.3); 175 by [16384, 1024] 14.1 (13.2)); of few tokens over weights up to 2^26 (160 by [16384, 8192] 73 (65))
+  if (tokens >= 192 && one && !rounds.wide && rounds.tiles >= 176 && (tokens > 512 || out * in <= (1 << 26))) return true;
+  // one round of 128 x 256 over short K (500 by [11264, 2048] 27.4 (31.1), 1400 by [4096, 2048] 27.8 (30.8); 320 by [16384, 2048] 28 (26), 3000 by
+  // [2048, 2048] 28.7 (28.3))
+  if (tokens > 384 && one && rounds.wide) return rounds.full >= 62 && tokens <= 2048 && in <= 2048;
+  // more than a round of 64 x 64 (700 by [2048, 2048] 15.2 (13.8))
+  if (tokens > 256 && in >= 2048 && (tokens + 63) / 64 * ((out + 63) / 64) > 256) return false;
+  // several rounds that are full, over short K (1400 / 2000 by [8000, 1024] 33.2 / 40.6 (34.9 / 42.2))
+  if (tokens > 512 && tokens <= 2048 && in <= 1024 && out <= 8192 && rounds.full >= 90) return true;
+  if (tokens > 1024) return tokens <= 2048 && out <= 1024 && in <= 1024;  // (1400 by [1024, 1024] 8.9 (10.8))
+  // long K in parts (128 by [4096, 14336] 36 (75), [6144, 4096] 21 (25), [8192, 8192] 38 (50), 64 33 (34); 256 by [5120, 13824] 58 (120); 64 by [12288, 4096]
+  // in two 28.7 (26.7))
+  if (in >= 4096 && tokens <= 256 && cut_of(tokens, out, in, true, true).parts >= (tokens <= 128 ? 3 : 2)) return true;
+  // rows 8 KB apart, which the library reads in step, in a round that is 78 % full (64 / 128 by [28672, 4096] 47 / 53 (57 / 59); by [22016, 4096], 172
+  // tiles, 44 / 53 (47 / 49))
+  if (in % 4096 == 0 && tokens <= 128 && rounds.tiles >= 200 && rounds.tiles <= 256) return true;
+  // else by the work: 2^31 products, over weights up to 2^24 2^32 (512 by [8000, 1024] 12.6 (17.2), [5632, 1024] 10.7 (14.1); 128 by [11264, 2048] 16.1 (16.5))
+  return tokens * out <= (1LL << (out * in <= (1 << 24) ? 32 : 31)) / in;
+}
+
+// dX: the library is slow over a weight read across its rows, up to 9 2^20 results.
+bool dx_pays(int64_t tokens, int64_t out, int64_t in, const Rounds& rounds) {
+  if (tokens * in > (9 << 20)) return false;
+  // 500 by [2048, 2048] 10.5 (15.1), [11264, 2048] 42 (63), [4096, 4096] 27.5 (34.6); 1024 by [11264, 2048] 54 (79), [12288, 4096] 94 (111)
+  if (tokens <= 1024) return true;
+  // several rounds: 88 % full (2000 by [2048, 5632] 53.5 (55.2); 1032 by [5632, 8192], 75 %, 120 (96))
+  if (rounds.count > 1) return rounds.full >= 88;
+  // one: of 88 tiles (1400 / 2000 by [3072, 2048] 23.7 / 29.5 (28.4 / 32.6), [8000, 1024] 35 / 44 (72 / 64)), of many tokens 62 % full (3000 / 4096 by
+  // [2048, 2048] 29.6 / 35.5 (30.2 / 36.4), 3000 by [11264, 2048] 125 (130), [32000, 2048] 393 (344))
+  return tokens <= 2048 ? rounds.tiles >= 88 : rounds.full >= 62 && out <= 16384;
+}
+
+// dW: both operands lie across the inner dimension, as the library likes least.
+bool dw_pays(int64_t tokens, int64_t out, int64_t in, const Rounds& rounds) {
+  // From 8192 tokens on the layer makes copies along them for the library. Rows that meet in memory channels: 32 KB apart ([16384, 2048] 320 45 (35)), or
+  // 8 and 16 KB ([12288, 8192] 528 158 (149))
+  if (tokens > 8192 || out % 16384 == 0 || (out % 4096 == 0 && in % 8192 == 0 && out * in > (1 << 25))) return false;
+  // up to three rounds of 128 x 128 (256 / 1024 / 4096 by [2048, 2048] 7.8 / 14.5 / 35.7 (10 / 17.2 / 45.5), [2048, 5632] 17 / 34 / 93 (24 / 41 / 96), 8000 by
+  // [1024, 1024] 30 (56)); more over long dimensions ([4096, 4096] 512 / 1024 / 2048 30 / 42 / 67 (26 / 40 / 67), 6000 by [12288, 4096] 480 (513))
+  if (rounds.tiles <= 3 * 256 || tokens >= 1280) return true;
+  // six rounds, three of 128 x 256 ([11264, 2048] 768 48 (62))
+  if (tokens >= 704 && rounds.tiles >= 5 * 256 && rounds.tiles <= 6 * 256) return true;
+  // token counts that are no whole 32, which the library pays for (100 by [22016, 4096] 64 (98), [4096, 11008] 37 (52), [11264, 2048] 22 (26), [32000, 2048] 49
+  // (53); 500 41 (47) by [6144, 4096], 98 (99) by [32000, 2048]; 333 by [4096, 4096], four rounds, 32 (24), 900 by [27648, 5120] 312 (292))
+  return tokens % 32 && (tokens <= 256 || (rounds.tiles <= 6000 && (tokens >= 500 || (rounds.tiles > 4 * 256 && rounds.tiles < 3000))));
+}
+
+}  // namespace
+
+// C [M, N] over K, as `ds_narrow_gemm` takes it
 extern "C" int ds_narrow_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along) {
   const Rounds rounds(M, N);
-  if (!a_along) {
-    if (M % 16384 == 0 || (M % 4096 == 0 && N % 8192 == 0 && M * N > (1 << 25))) return 0;
-    if (K > 8192) return 0;
-    if (rounds.tiles <= 768 || K >= 1280 || (K >= 704 && rounds.tiles >= 1280 && rounds.tiles <= 1536)) return 1;
-    return K % 32 && (K <= 256 || (rounds.tiles <= 6000 && (K >= 500 || (rounds.tiles > 1024 && rounds.tiles < 3000))));
-  }
-  if (!b_along) {
-    if (M <= 1024 || M * N > (9 << 20)) return M * N <= (9 << 20);
-    return rounds.count == 1 ? (M <= 2048 ? rounds.tiles >= 88 : rounds.full >= 62 && K <= 16384) : rounds.full >= 88;
-  }
-  if (M >= 192 && rounds.count == 1 && !rounds.wide && rounds.tiles >= 176 && (M > 512 || N * K <= (1 << 26))) return 1;
-  if (M > 384 && rounds.count == 1 && rounds.wide) return rounds.full >= 62 && M <= 2048 && K <= 2048;
-  if (M > 256 && K >= 2048 && (M + 63) / 64 * ((N + 63) / 64) > 256) return 0;
-  if (M > 512 && M <= 2048 && K <= 1024 && N <= 8192 && rounds.full >= 90) return 1;
-  if (M > 1024) return M <= 2048 && N <= 1024 && K <= 1024;
-  if (K >= 4096 && M <= 256 && cut_of(M, N, K, true, true).parts >= (M <= 128 ? 3 : 2)) return 1;
-  if (K % 4096 == 0 && M <= 128 && rounds.tiles >= 200 && rounds.tiles <= 256) return 1;
-  return M * N <= (1LL << (N * K <= (1 << 24) ? 32 : 31)) / K;
+  if (!a_along) return dw_pays(K, M, N, rounds);
+  return b_along ? y_pays(M, N, K, rounds) : dx_pays(M, K, N, rounds);
 }
 
 // Bytes of scratch memory that the product wants (0: none)
@@ -558,14 +585,22 @@ Cut ordered_cut(int64_t M, int64_t N, int64_t K) {
 }
 }  // namespace
 
-// Whether ds_narrow_ordered takes x [M, K] by w [N, K] in operand order, and is the faster way. Not over short K from 4096 rows on (33 rows by [8192,
-// 2048] 11.3, before 10.4), nor 33 to 40 by [8192, 4096], 128 tiles in two parts (18.2 and 18.5, before 16.3 and 17.6), nor where the weights' read is what counts ([16384, 8192] 55, before 49; [32000, 4096] 52.5, 53.5, with 33 rows 51
-// and 50). Up to 32 rows small products (24 by [2048, 2048] 6.0, before 6.9, [3072, 1024] 4.8, 5.4; [4096, 2048] 7.8, 7.3) and those a quarter over
-// one round of single blocks (24 by [5120, 5120] 14.4, 16.5).
+// Whether ds_narrow_ordered takes x [M, K] by w [N, K] in operand order, and is the faster way, us here (with the decode kernels).
 extern "C" int ds_narrow_ordered_ok(int64_t M, int64_t N, int64_t K) {
+  // (beyond, the weights' read is what counts: 48 rows by [16384, 8192] 55 (49), [32000, 4096] 52.5 (51))
   if (M > 48 || N <= 0 || N > 16384 || N % 8 || K <= 0 || K % 64 || N * K > (3 << 25)) return 0;
-  if (M > 32) return (K >= 3072 && (M > 40 || N <= 6144 || N > 8192 || K > 4096)) || N <= 4096;
-  return (M > 20 && K <= 2048 && N * K <= (1 << 22)) || (M > 16 && N > 4096 && N <= 5440 && K >= 4096 && K < 8192);
+  const int64_t mid = (N + 63) / 64, blocks = (N + 15) / 16;  // tiles of 64 columns; blocks as the decode kernels take them
+  if (M > 32) {
+    if (mid <= 64) return 1;       // a part, or a few, of a round of tiles
+    if (K < 3072) return 0;        // short K over more of them: the decode kernels' X is small (33 by [8192, 2048] 11.3 (10.4))
+    // Nearly a round in two short parts, whose sums are a launch: not for 33 to 40 rows, which the decode kernels take in a round of two blocks a
+    // workgroup (33 / 40 by [8192, 4096] 18.2 / 18.5 (16.3 / 17.6))
+    return M > 40 || mid <= 96 || mid > 128 || K > 4096;
+  }
+  // small products (24 by [2048, 2048] 6.0 (6.9), [3072, 1024] 4.8 (5.4); [4096, 2048] 7.8 (7.3))
+  if (M > 20 && K <= 2048 && N * K <= (1 << 22)) return 1;
+  // up to a third over one round of single blocks, which the decode kernels fill with two a workgroup (24 by [5120, 5120] 14.4 (16.5))
+  return M > 16 && blocks > 256 && blocks <= 340 && K >= 4096 && K < 8192;
 }
 
 extern "C" int64_t ds_narrow_ordered_scratch(int64_t M, int64_t N, int64_t K) {

@@ -338,6 +338,8 @@ struct Cut {
 // 14; 48 rows with two / four: [8192, 4096] 19 / 24, [9216, 3072] 28 / 19, [12288, 4096] 35 / 26). Products with more blocks than that
 // holds take the most that there are (24 rows x [32000, 4096] 48 with two, 46 with four), up to 16 token rows two (12 rows 42 and 45).
 // Gated pairs take two or four (12 rows: [11264, 2048] 13.0 and 11.0, [28672, 4096] 41 and 38).
+// Of 33 rows and more without a norm or a gate, what arrives here are widths that are no multiple of 8, gate halves that are no whole blocks, more than
+// 16384 weight rows or 3 2^25 weights, and short K over more than 4096 rows: the others are the narrow products' (`narrow_instead`).
 // Eight blocks for 33 rows and more of 4096 and more: X, a quarter to a half of what a CU reads, is then read half as often. One workgroup
 // has a CU to itself, so their number decides: where four blocks (two a CU with a norm) fill their rounds as well or better, it stays at
 // four. 33 / 48 rows, us with four and with eight. Normed, 129 to 256 workgroups of eight: [18432, 4096] 42 / 47 and 36 / 38, gated [22016, 4096]
@@ -350,12 +352,13 @@ struct Cut {
 // and 49).
 // More than 16 token rows of 4096 and more over few blocks: what a CU can read (30 bytes a nanosecond) bounds one block's workgroup,
 // and of that most is X. Several blocks share the reading, and parts of K keep the workgroups at 256; the parts' sums are a launch of
-// 4 us. 48 rows, us with one block and with this: [4096, 4096] 16.3 and 14.6, [4096, 14336] 45 and 28, [2048, 5632] 20.6 and 13.5; 17
-// rows 10.9 and 11.4, 27 and 24, 12.3 and 10.0. Over 2048 the launch costs what it gives ([2048, 2048] 10.2 and 9.9). Four blocks for
-// 33 rows and more of 8192 ([4096, 14336] 33 with two; 17 rows 24.6 with four, 23.6 with two).
-// The same between 256 and 680 blocks where X is long: four blocks and the parts that fill one round or two. 17 / 32 / 48 rows, us
-// without and with: [5120, 13824] 33 / 41 / 52 and 28 / 31 / 33, [8192, 8192] 27 / 29 / 35 and 28 / 28 / 31, [10240, 8192] 35 / 40 / 45
-// and 34 / 35 / 40; shorter ones stay whole ([7168, 7168] 21 / 24 and 23 / 24).
+// 4 us. 33 / 48 rows, us with one block and with this: [4095, 4096] 13.8 / 16.5 and 13.5 / 15.3, [4095, 14336] 41 / 47 and 29 / 30, [2047, 5632]
+// 16.8 / 20.5 and 12.8 / 13.9; 17 rows x [4096, 4096] 10.9 and 11.4, [4096, 14336] 27 and 24, [2048, 5632] 12.3 and 10.0. Over 2048 the launch costs what it
+// gives ([2048, 2048] 10.2 and 9.9). Four blocks for 33 rows and more of 8192 ([4096, 14336] 33 with two; 17 rows 24.6 with four, 23.6 with two).
+// The same between 256 and 680 blocks where X is long: four blocks and the parts that fill one round or two. Us without and with: 17 / 32 rows,
+// [5120, 13824] 33 / 41 and 28 / 31, [8192, 8192] 27 / 29 and 28 / 28, [10240, 8192] 35 / 40 and 34 / 35; 33 / 48 rows, [5119, 13824] 47 / 54 and
+// 34 / 35, [8191, 8192] 32 / 36 and 31.5 / 33, [10239, 8192] 46 / 51 and 40 / 43, gated [5136, 8192], whose halves are no whole blocks, 33 / 36 and 25 / 28;
+// shorter ones stay whole ([7168, 7168] 21 / 24 and 23 / 24).
 // Up to 16 rows parts pay at the ends alone: where a few blocks leave most CUs idle (16 rows x [1024, 4096] 8.7 and 7.7, 2 rows 6.1 and
 // 6.9, x [1024, 8192] 9.6 and 8.4), and where long ones stand a quarter over one round (16 rows x [10240, 8192] 40 and 35); from 12 rows on
 // also over long K, in two blocks, which halve the reading of X (12 / 16 rows x [2048, 5632] 10.4 / 11.7 and 9.5 / 9.7, [4096, 14336] 23.7 / 26.0 and 22.8 / 23.3,
