@@ -154,6 +154,65 @@ def test_outputs_change_in_place(case):
     _same(a, b, case is not _flash)
 
 
+def _result(f):
+    try:
+        return f()
+    except (RuntimeError, NotImplementedError):
+        return None
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: c.__name__[1:])
+def test_node_under_transforms(case):
+    """Gradients that are differentiated again, batches of gradients, tangents and recomputed segments: what the function gives, or its
+    refusal."""
+    from torch.autograd import forward_ad
+    from torch.utils.checkpoint import checkpoint
+    node, function, inputs = case()
+    first = lambda f, ins: (lambda o: o[0] if isinstance(o, (tuple, list)) else o)(f(*ins))  # noqa: E731
+
+    def again(f):
+        grads = torch.autograd.grad(first(f, inputs).float().pow(2).sum(), inputs, create_graph=True, allow_unused=True)
+        flags = [g is not None and g.requires_grad for g in grads]
+        more = _result(lambda: torch.autograd.grad(sum(g.float().pow(2).sum() for g in grads if g is not None), inputs, allow_unused=True))
+        return flags, [g for g in grads if g is not None], more
+
+    def batched(f):
+        y = first(f, inputs)
+        go = torch.stack([torch.ones_like(y), 2 * torch.ones_like(y)])
+        return _result(lambda: torch.autograd.grad(y, inputs, go, is_grads_batched=True, allow_unused=True))
+
+    def tangent(f):
+        with forward_ad.dual_level():
+            dual = [forward_ad.make_dual(t.detach(), torch.ones_like(t)) for t in inputs]
+            return _result(lambda: [t for t in forward_ad.unpack_dual(first(f, dual)) if t is not None])
+
+    def recomputed(f):
+        y = checkpoint(lambda *a: first(f, a) * 2, *inputs, use_reentrant=False)
+        return y, *torch.autograd.grad(y.float().sum(), inputs, allow_unused=True)
+    exact = case is not _flash
+    (flags, grads, more), (flags2, grads2, more2) = again(node), again(function)
+    assert flags == flags2 and (more is None) == (more2 is None)
+    _same(grads, grads2, exact)
+    _same(more or (), more2 or (), exact)
+    for how in (batched, tangent, recomputed):
+        a, b = how(node), how(function)
+        assert (a is None) == (b is None)
+        _same(a or (), b or (), exact)
+
+
+def test_linear_under_transforms():
+    """The layer as it is called, against torch's linear: the gradient's gradient and a batch of vectors through the Jacobian."""
+    x, w, go = _leaf(96, 128), _leaf(192, 128, seed=1), _rnd(96, 192, seed=2)
+    kept = []
+    for f in (L.linear, torch.nn.functional.linear):
+        (g1, ) = torch.autograd.grad(f(x, w).float().pow(2).sum(), x, create_graph=True)
+        (g2, ) = torch.autograd.grad(g1.float().pow(2).sum(), w)
+        kept.append((g1, g2, *torch.autograd.grad(f(x, w), (x, w), torch.stack([go, 2 * go]), is_grads_batched=True)))
+    assert "Node" in L.linear(x, w).grad_fn.name()
+    for got, want in zip(*kept):   # (bf16 in between: a few roundings of 2^-9 each, of sums whose terms may cancel)
+        torch.testing.assert_close(got.float(), want.float(), rtol=0.03, atol=0.03 * want.float().abs().max().item())
+
+
 @pytest.mark.parametrize("lead", [(96, ), (2, 48), (1, 96)])
 def test_linear_changes_in_place(lead):
     """A linear layer's output of a short batch, changed in place by itself and through views, as torch's may be."""
