@@ -16,6 +16,8 @@
 //  * any: a workgroup per entry and 64 columns; fp32 and widths that are no multiple of 8.
 #include "ds_hip.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int MAXE = 256, FEW = 512;
@@ -389,6 +391,9 @@ __global__ void __launch_bounds__(256, 2) expert_tile_kernel(ExpertArgs a) {
 //    step. Every wait counts what may still be on its way: buffers are arrays apart, and all accesses buffer instructions (hipcc waits
 //    for everything where LDS transfers are global ones), so the compiler's own waits for weights count too. Tail steps issue the last
 //    step's transfers again, so that the counts stand;
+//  * beyond 4 GB of rows (LONG) the transfers take an address of 64 bits a lane instead, as inline asm; the compiler's waits for weights
+//    then count weights alone, and are stricter than they need be. 266240 rows of 8192 among 8 experts of 4096: 14.5 ms (eight waves 15.5, the
+//    tile kernel 18.5). Long loops of less take 0.9 % more that way (32 x 1024 rows above 1725 and 1741, plain 901 and 909);
 //  * rows in units of 64 (MT): a short tile moves and multiplies no others.
 // Workgroups walk groups of 8 column tiles by all row tiles of an expert. Then bound by power: 1.6 GHz, matrix cores busy 77 % of the time in
 // a long loop; without any transfers 1.75 GHz and 83 %. 16 x 16 x 32 products: hipcc moves accumulators about, 1.05 times the time.
@@ -407,6 +412,13 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t from, uint32_t lane
   __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void*)dst, 16, lane_bytes, bytes, 0, 0);
 #endif
 }
+__device__ __forceinline__ void dma16(const char* from, lds_char* dst) {
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "v"(from), "s"(__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)dst))
+               : "memory");
+}
 // All of this wave's LDS accesses and all but its NEWER latest loads are done, then those of all waves.
 template <int NEWER>
 __device__ __forceinline__ void meet() {
@@ -415,7 +427,7 @@ __device__ __forceinline__ void meet() {
   asm volatile("s_barrier" ::: "memory");
 }
 
-template <bool GLU>
+template <bool GLU, bool LONG>
 __global__ void __launch_bounds__(256, 1) expert_big_kernel(ExpertArgs a) {
   // rows of a step each, as arrays apart: the compiler then knows which transfers a read has to wait for
   __shared__ __attribute__((aligned(16))) char b0[TM * 128], b1[TM * 128], b2[TM * 128], b3[TM * 128];
@@ -467,19 +479,24 @@ __global__ void __launch_bounds__(256, 1) expert_big_kernel(ExpertArgs a) {
         for (int r = 0; r < 16; ++r) acc[t][m][r] = 0.f;
     // ---- rows on their way: MT pieces of 8 rows of 128 bytes per wave (16 bytes p of row r: columns 8 (p ^ (r / 2 % 8)) .. + 7)
     const int mine = 8 * MT * wid, entry = a.order[pl.first + min(mine + lane, left - 1)];
-    uint32_t xo[MT];
+    std::conditional_t<LONG, const char*, uint32_t> xo[MT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
       const int r = i * 8 + (lane >> 3);
-      xo[i] = ((uint32_t)__shfl(entry / a.div, r, 64) * K + 8 * ((lane & 7) ^ (((mine + r) >> 1) & 7))) * 2;
+      const int row = __shfl(entry / a.div, r, 64), piece = 8 * ((lane & 7) ^ (((mine + r) >> 1) & 7));
+      if constexpr (LONG) xo[i] = (const char*)a.x + ((int64_t)row * K + piece) * 2;
+      else xo[i] = ((uint32_t)row * K + piece) * 2;
     }
     if (lane < 8 * MT) ents[mine + lane] = entry;
     // those of step kq that part p issues; past the end the last step again, into a buffer that nobody reads
     auto move = [&](int kq, auto b_c, int p, int only) {
 #pragma unroll
       for (int i = p * MT / 4; i < (p + 1) * MT / 4; ++i)
-        if (only < 0 || only == i - p * MT / 4)
-          dma16(xs, xo[i], min(kq, KQ - 1) * 128, buffer(b_c) + 128 * mine + 1024 * i);
+        if (only < 0 || only == i - p * MT / 4) {
+          lds_char* to = buffer(b_c) + 128 * mine + 1024 * i;
+          if constexpr (LONG) dma16(xo[i] + min(kq, KQ - 1) * 128, to);
+          else dma16(xs, xo[i], min(kq, KQ - 1) * 128, to);
+        }
     };
     bf16x8 w[2][4][2], x[2][MT];
     // (in the order of the loop, which waits by it)
@@ -616,7 +633,8 @@ constexpr int BIG_ROWS = 128;
 template <bool GLU>
 int launch_big(const ExpertArgs& a, int per, hipStream_t st) {  // per: columns of a tile
   const int64_t grid = ((int64_t)a.entries / TM + a.E) * ((a.N + per - 1) / per);
-  hipLaunchKernelGGL((expert_big_kernel<GLU>), dim3((unsigned)grid), dim3(256), 0, st, a);
+  if (a.xbytes) hipLaunchKernelGGL((expert_big_kernel<GLU, false>), dim3((unsigned)grid), dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((expert_big_kernel<GLU, true>), dim3((unsigned)grid), dim3(256), 0, st, a);
   DS_CHECK_LAUNCH();
   return 0;
 }
@@ -643,7 +661,7 @@ extern "C" int ds_expert_gemm(const void* x, const void* w, void* y, const int* 
     const int per = gated ? BN / 2 : BN;
     const int64_t grid = ((int64_t)entries / BM + E) * ((N + per - 1) / per);
     if (grid > INT32_MAX) return (int)hipErrorInvalidValue;
-    if (entries >= (int64_t)BIG_ROWS * E && a.xbytes) return gated ? launch_big<true>(a, per, st) : launch_big<false>(a, per, st);
+    if (entries >= (int64_t)BIG_ROWS * E) return gated ? launch_big<true>(a, per, st) : launch_big<false>(a, per, st);
     if (gated) hipLaunchKernelGGL(expert_tile_kernel<true>, dim3((unsigned)grid), dim3(256), 0, st, a);
     else hipLaunchKernelGGL(expert_tile_kernel<false>, dim3((unsigned)grid), dim3(256), 0, st, a);
     DS_CHECK_LAUNCH();

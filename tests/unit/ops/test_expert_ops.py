@@ -308,8 +308,31 @@ def test_gates_of_tiles_are_exact_to_fp32(rows):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("act", ["silu_glu", "none"])
+@pytest.mark.parametrize("K,n,div", [(4160, 516300, 1), (8256, 260160, 1), (8256, 520300, 2)])
+def test_big_tiles_over_long_inputs(K, n, div, act):
+    """More than 4 GB of rows, an odd number of steps, experts of every remainder, rows for one entry and for two: the same bits as over
+    the last rows alone, a short input, in which every entry of the same expert has the same row."""
+    from deepspeedsyclsupport_amd.ops.expert_ops import ACTS, expert_ops, operand_order
+    E, N, tail = 6, 96, 1800
+    g = torch.Generator(device="cuda").manual_seed(n)
+    assert (n - 1) // div * K * 2 > 1 << 32 and tail >= 128 * E
+    w = operand_order((torch.randn(E, (2 if act == "silu_glu" else 1) * N, K, device="cuda", generator=g) * K**-0.5).bfloat16())
+    x = torch.zeros((n - 1) // div + 1, K, device="cuda", dtype=torch.bfloat16)
+    x[-tail // div:] = torch.randn(tail // div, K, device="cuda", generator=g).bfloat16()
+    experts = torch.randint(0, E, (n, ), device="cuda", generator=g).int()
+
+    def run(x, experts):
+        order = torch.argsort(experts, stable=True).int()
+        offs = torch.cat([torch.zeros(1, dtype=torch.long, device="cuda"), torch.bincount(experts, minlength=E).cumsum(0)]).int()
+        return expert_ops().expert_gemm(x, w, experts, offs, order, div, ACTS[act], True, True)
+    y = run(x, experts)
+    assert torch.equal(y[-tail:], run(x[-tail // div:].clone(), experts[-tail:].clone())) and not y[:-tail].any()
+
+
+@pytest.mark.gpu
 def test_big_tiles_leave_long_inputs():
-    """Rows that 32 bits of bytes do not reach go by the tile kernel."""
+    """Rows that 32 bits of bytes do not reach."""
     from deepspeedsyclsupport_amd.ops.expert_ops import expert_ops, operand_order
     N, K, n = 32, 8192, (1 << 18) + 96    # 4 GiB and a little
     w = (torch.randn(1, N, K, device="cuda") * K**-0.5).bfloat16()
