@@ -570,37 +570,43 @@ extern "C" int ds_narrow_gemm(const void* A, const void* B, void* C, int64_t M, 
 namespace {
 // Decode batches of 33 to 48 rows by weights in operand order. Against ds_decode_gemm's kernels (eight waves that load what they multiply) the
 // transfers run three steps ahead without registers, a workgroup's tile has 64 weight rows (there 32, or 64 with a CU to itself) and
-// the parts' sums are as many rows as there are. 64 x 64 in parts up to a workgroup a CU, whole from 129 tiles on, 128 x 128 of long K there;
-// few blocks 32 x 32. us before and now, 48 rows: [1024, 4096] 10.5 / 7.8, [2048, 2048] 9.8 / 6.1, [4096, 2048] 10.1 / 7.6, [4096, 4096] 14.3 / 12.2, [5120,
-// 5120] 22.8 / 15.6, [2048, 5632] 13.0 / 11.6, [4096, 14336] 28.5 / 26.4, [10240, 8192] 39.6 / 37.0, [16384, 4096] 28.2 / 26.9.
+// the parts' sums are as many rows as there are. What a CU reads bounds it, so K goes in parts up to a workgroup a CU, in tiles of 64 x 64 over 64 of
+// them and more, over 33 from K = 4608 on and over 22 from 6144 on (33 rows, us as 32 x 32 in parts up to a workgroup a CU and so: [2304, 7168] 16.6, 12.9,
+// [2112, 4608] 11.9, 10.7, [1536, 14336] 19.5, 15.7, [1344, 14336] with 21 tiles 15.6, 15.3). Beyond 128 tiles, 128 x 128 in parts where a round holds three
+// (33 rows by [9216, 7168] whole as 64 x 64 34.6, so 29.8; [9216, 4096] 21.8, 20.5; [9216, 3072] 16.8, 17.2) and of long K, else 64 x 64 whole; few or
+// short ones 32 x 32. us before and now, weights from memory, 48 rows: [1024, 4096] 10.2 / 8.4, [2048, 2048] 9.7 / 7.2, [4096, 2048] 10.2 / 7.6, [4096, 4096] 14.5 /
+// 12.3, [5120, 5120] 23.0 / 15.9, [2048, 5632] 13.0 / 11.6, [4096, 14336] 28.9 / 26.8, [10240, 8192] 39.8 / 37.9, [16384, 4096] 28.5 / 27.5. Of 2336 products at
+// random (33 to 48 rows, up to 20800 weight rows, K of 512 to 15360; profiles/decode_products_at_random.csv) 2166 are faster by more than 4 %, 2 slower by
+// as much (1.07 and 1.05 times as long); 0.84 of the time in the mean.
 Cut ordered_cut(int64_t M, int64_t N, int64_t K) {
   const int64_t mid = (N + 63) / 64, low = (M + 31) / 32 * ((N + 31) / 32), big = (N + 127) / 128;
-  auto parts = [&](int64_t tiles) { return (int)std::max<int64_t>(std::min<int64_t>(std::min<int64_t>(256 / tiles, K / 1024), 8), 1); };
+  auto parts = [&](int64_t tiles, int64_t least) { return (int)std::max<int64_t>(std::min<int64_t>(std::min<int64_t>(256 / tiles, K / least), 8), 1); };
   Cut c = {32, 32, 1};
-  if (mid > 128) c = K >= 8192 ? Cut{128, 128, parts(big)} : Cut{64, 64, 1};
-  else if (K >= 3072) c = mid >= (K >= 8192 ? 32 : 64) ? Cut{64, 64, parts(mid)} : Cut{32, 32, parts(low)};
+  if (mid > 128) c = K >= 8192 || (K >= 3584 && big <= 85) ? Cut{128, 128, parts(big, 1024)} : Cut{64, 64, 1};
+  else if (mid >= 64 && K >= 3072) c = Cut{64, 64, parts(mid, 1024)};
+  else if ((mid > 32 && K >= 4608) || (mid > 21 && K >= 6144)) c = Cut{64, 64, parts(mid, 768)};
+  else if (K >= 3072) c = Cut{32, 32, parts(low, 1024)};
   if (g_tile) c.tm = c.tn = std::min(g_tile, 128);
   if (g_parts) c.parts = (int)std::min<int64_t>(g_parts, K / 64);
   return c;
 }
 }  // namespace
 
-// Whether ds_narrow_ordered takes x [M, K] by w [N, K] in operand order, and is the faster way, us here (with the decode kernels).
+// Whether ds_narrow_ordered takes x [M, K] by w [N, K] in operand order, and is the faster way, us here (with the decode kernels). Weights from memory.
 extern "C" int ds_narrow_ordered_ok(int64_t M, int64_t N, int64_t K) {
   // (beyond, the weights' read is what counts: 48 rows by [16384, 8192] 55 (49), [32000, 4096] 52.5 (51))
   if (M > 48 || N <= 0 || N > 16384 || N % 8 || K <= 0 || K % 64 || N * K > (3 << 25)) return 0;
-  const int64_t mid = (N + 63) / 64, blocks = (N + 15) / 16;  // tiles of 64 columns; blocks as the decode kernels take them
+  const int64_t mid = (N + 63) / 64, big = (N + 127) / 128, blocks = (N + 15) / 16;  // tiles of 64 and 128 columns; blocks as the decode kernels take them
   if (M > 32) {
     if (mid <= 64) return 1;       // a part, or a few, of a round of tiles
     if (K < 3072) return 0;        // short K over more of them: the decode kernels' X is small (33 by [8192, 2048] 11.3 (10.4))
-    // Nearly a round in two short parts, whose sums are a launch: not for 33 to 40 rows, which the decode kernels take in a round of two blocks a
-    // workgroup (33 / 40 by [8192, 4096] 18.2 / 18.5 (16.3 / 17.6))
-    return M > 40 || mid <= 96 || mid > 128 || K > 4096;
+    // Nearly a round in two short parts, whose sums are a launch, or a round and more of whole tiles: not for 33 to 40 rows (33 by [8192, 4096] 18.2
+    // (16.3), [11920, 7616] 41.6 (39.3), [13136, 4992] 29.7 (28.2))
+    return M > 40 || !((mid > 96 && mid <= 128 && K <= 4096) || (big > 85 && K < 8192));
   }
-  // small products (24 by [2048, 2048] 6.0 (6.9), [3072, 1024] 4.8 (5.4); [4096, 2048] 7.8 (7.3))
-  if (M > 20 && K <= 2048 && N * K <= (1 << 22)) return 1;
-  // up to a third over one round of single blocks, which the decode kernels fill with two a workgroup (24 by [5120, 5120] 14.4 (16.5))
-  return M > 16 && blocks > 256 && blocks <= 340 && K >= 4096 && K < 8192;
+  // Up to a third over one round of single blocks, which the decode kernels fill with two a workgroup (24 / 32 by [5120, 5120] 14.6 / 15.1 (16.6 / 18.1); 20 by [5336, 4096] 13.6 (12.7)). Small
+  // products stay there: 24 by [2048, 2048] 7.4 (6.8), [1024, 1024] 5.5 (5.0), 32 rows 7.7 (7.7), 5.7 (5.5)
+  return M > (K >= 5120 ? 16 : 24) && blocks > 256 && blocks <= 340 && K >= 4096 && K < 8192;
 }
 
 extern "C" int64_t ds_narrow_ordered_scratch(int64_t M, int64_t N, int64_t K) {
