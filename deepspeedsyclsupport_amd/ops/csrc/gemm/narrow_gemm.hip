@@ -379,16 +379,17 @@ struct Cut {
 };
 
 // Rounds that the chip makes of tiles of 128 x 128, or 128 x 256, which take 1.8 times as long (dW of 3000 tokens, us: 256 of the first 25, of the
-// second 44): `wide` where those are the faster ones
+// second 44), over longer K 1.6 times (5 rounds and 3, the medians of 114 products of K from 1024 on: 0.96; 9 and 5 0.92; of K below 1.05): `wide` where those
+// are the faster ones
 struct Rounds {
   int64_t tiles;  // of 128 x 128
   bool wide;
   int full;       // percent of the chosen one's rounds that is work
   int64_t count;  // ... and their number
-  Rounds(int64_t M, int64_t N) {
+  Rounds(int64_t M, int64_t N, int64_t K) {
     tiles = (M + 127) / 128 * ((N + 127) / 128);
     const int64_t half = (M + 127) / 128 * ((N + 255) / 256), a = (tiles + 255) / 256, b = (half + 255) / 256;
-    wide = 9 * b < 5 * a;
+    wide = (K >= 1024 ? 8 : 9) * b < 5 * a;
     count = wide ? b : a;
     full = (int)(100 * (wide ? half : tiles) / (256 * count));
   }
@@ -400,40 +401,50 @@ struct Rounds {
 // 128 x 256 by `Rounds` (us with 128, 256: y 500 by [11264, 2048] 33.4, 28.0; dX 700 by [2048, 5632] 33.0, 27.5; dW 3000 by [11264, 2048] 145, 124; in one
 // round anyhow, y 1000 by [4096, 4096], 34.3, 44.2).
 // From K = 4096 on weights come from memory and a CU's share of the operands bounds: 128 x 128 tiles, in parts of 768 or more, where those make
-// 192 to 256 workgroups (128 by [4096, 14336] 63.9 with 64x1, 34.8 with 128x8; by [6144, 4096] 22.2, 128x5 20.7; but 256 by [4096, 4096] 21.2
-// with 64x1, 128x4 22.4), else 64 x 64 in parts of 1024 or more (128 by [2048, 5632] 18.2 with 32x2, 13.9; by [1024, 8192] 18.4, 13.1).
+// 172 to 256 workgroups (128 by [4096, 14336] 63.9 with 64x1, 34.8 with 128x8; by [6144, 4096] 22.2, 128x5 20.7; 238 by [4096, 5120], weights from memory,
+// 31.0 with 64x1, 128x4 25.4; but 454 by [2048, 4096] 19.0, 128x4 20.8), else 64 x 64 in parts (128 by [2048, 5632] 18.2 with 32x2, 13.9; by [1024, 8192] 18.4,
+// 13.1; 50 by [3072, 5632], from memory, 18.7, 64x4 13.9). Up to 64 rows over shorter K fill half of 128 x 128 (52 by [16384, 2048] 23.9, 64x1 18.9; dX, 57 by
+// [3072, 14336] 30.9, 25.4).
 // One across (dX): those rows come in runs of 64 columns, never 32 (half a cache line). 64 x 64 from 160 tiles on, of long K from 64
 // (256 tokens by [5632, 1024] 32x2 13.0, 64x4 11.8; 512 17.5, 64x2 15.8; by [3072, 1024] 9.5, 10.5), 128 x 128 from 88 (1400 by [8000, 1024], 88, 57 with 64,
 // 49, x2 35; 600 by [1024, 2816], 110, 10.0, 10.5; 300 by [2048, 5632], 132, 19.6, 16.3). Parts of 768 up to a workgroup a CU, of 128 x 128 2560
-// (128 by [3072, 1024] 10.6, x2 9.4, x4 8.9; by [1024, 1024] 5.3, 6.4, 6.9).
+// (128 by [3072, 1024] 10.6, x2 9.4, x4 8.9; by [1024, 1024] 5.3, 6.4, 6.9). Over long K 128 x 128 in parts as above, from 43 tiles on (weights from memory,
+// 128 by [11264, 11008] 118 with 64x1, 128x2 69, library 104; 250 by [5632, 4096] 38.1, 128x4 27.5, 43; by [4096, 4096], a round of 64 x 64, 25.8, 25.8, in cache
+// 18.3, 22.5); both forms from 80 on that 64 x 64 would not do in a round (768 by [3072, 2048] 25.3, 128x2 24.1, by [2048, 2048] 18.0, 19.5; dW, 2705 by [376,
+// 3584] 34.5, 23.4, library 32.2; not 128 of them, 2299 by [2048, 1024] 18.0, 24.0).
 // Both across (dW): 64 x 64, 128 x 128 from 140 of them on (500 / 2000 / 8000 by [1536, 1536], 144, 9.4 / 21.8 / 78, 8.0 / 16.7 / 49; 500 / 2000 by [1024, 2048],
 // 128, 7.3 / 15.9, 7.9 / 15.8).
 Cut cut_of(int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) {
   auto tiles = [&](int t, int u) { return ((M + t - 1) / t) * ((N + u - 1) / u); };
   const bool along = a_along && b_along, across = !a_along && !b_along;
   int tm = 32, tn = along ? 32 : 64;
-  const Rounds rounds(M, N);
-  if (rounds.tiles >= (along ? 126 : across ? 140 : 88)) {
+  const Rounds rounds(M, N, K);
+  const int64_t big = rounds.tiles, mid = tiles(64, 64);
+  if (big >= (along ? 126 : across ? 140 : 88) && !(K < 4096 && M <= 64 && mid <= 256)) {
     tm = 128;
     tn = rounds.wide ? 256 : 128;
-  } else if (along ? tiles(32, 32) > 512 : across || tiles(64, 64) >= (K >= 4096 ? 64 : 160)) tm = tn = 64;
+  } else if (along ? tiles(32, 32) > 512 : across || mid >= (K >= 4096 ? 64 : 160)) tm = tn = 64;
   int64_t parts = 0;
   if (along && K >= 4096) {
-    const int64_t big = tiles(128, 128), mid = tiles(64, 64), cut = std::min<int64_t>(256 / std::max<int64_t>(big, 1), 8);
-    if (cut >= 2 && cut * big >= 192 && K / cut >= 768 && (K >= 8192 || mid <= 224 || mid > 256)) {
+    const int64_t cut = std::min<int64_t>(256 / std::max<int64_t>(big, 1), 8);
+    if (cut >= 2 && cut * big >= 172 && K / cut >= 768 && (K >= 5120 || mid <= 224 || mid > 256)) {
       tm = tn = 128;
       parts = cut;
-    } else if (mid >= (K >= 8192 ? 32 : 64) && mid <= 128) {
+    } else if (mid <= 128 && (mid >= 64 || (mid >= 32 && K >= 8192) || (mid > 32 && K >= 4608))) {
       tm = tn = 64;
-      parts = std::min<int64_t>(std::min<int64_t>(256 / mid, K / 1024), 8);
+      parts = std::min<int64_t>(std::min<int64_t>(256 / mid, K / (mid < 64 ? 768 : 1024)), 8);
     }
+  } else if (!along && ((!across && big >= 43 && big <= 128 && K >= (mid > 256 ? 4096 : 5120)) ||
+                        (big >= 80 && big <= 120 && mid > 256 && K >= (across ? 2048 : 3072)))) {
+    tm = tn = 128;
+    parts = std::min<int64_t>(std::min<int64_t>(256 / big, K / 1024), 8);
   }
   if (g_tile) {
     tm = g_tile;
     tn = g_tile == 32 && !along ? 64 : g_tile;
     if (g_tile == 256) tm = 128;
   }
-  if (!parts || g_tile) parts = std::min<int64_t>(std::min<int64_t>((along && tm < 128 ? 512 : 256) / tiles(tm, tn), K / (along || tm == 128 ? 2560 : 768)), 8);
+  if (parts <= 0 || g_tile) parts = std::min<int64_t>(std::min<int64_t>((along && tm < 128 ? 512 : 256) / tiles(tm, tn), K / (along || tm == 128 ? 2560 : 768)), 8);
   if (g_parts) parts = std::min<int64_t>(g_parts, (K + 63) / 64);
   return {tm, tn, (int)std::max<int64_t>(parts, 1)};
 }
@@ -454,14 +465,15 @@ extern "C" int ds_narrow_gemm_ok(int64_t M, int64_t N, int64_t K, int64_t lda, i
 
 // Whether the kernel is as fast as the library's, for each product of a linear layer of `tokens` rows by a weight [out, in]; us here (there).
 // A cost model was not found that orders the library's side, which jumps with its own choice of tiles. What the lines go by is stated with each:
-// whole rounds of the chip (`Rounds`), which products of its size the library is bad at, and rows that meet in memory channels. On 300 layers at
-// random (33 to 8000 tokens, widths of 256 to 32768, none of which the lines were drawn by) 601 products go here, 580 of them faster by more than 4 %, 4
-// slower by as much (12.6 (12.1), 37.6 (30.1), 46.5 (43.2), 28.6 (27.0)); y / dX / dW of all 300 take 0.86 / 0.73 / 0.61 of the library's time in the mean
-// (profiles/narrow_products_at_random.csv).
+// whole rounds of the chip (`Rounds`), which products of its size the library is bad at, and rows that meet in memory channels. On layers at
+// random, none of which the lines were drawn by, with weights (for dW the input) from memory 617 / 553 / 1074 products y / dX / dW of 1200 layers go here and
+// take 0.73 / 0.68 / 0.68 of the library's time in the mean, 2138 of them faster by more than 4 %, 22 slower by as much, at worst 35 %; out of the caches 769
+// of 400 layers 0.76 / 0.66 / 0.63, 753 faster, 2 slower (profiles/narrow_products_at_random.csv).
 namespace {
 
 // y: a tile's operands come as the library's do; what is gained is its launch, and tiles that fill the chip.
 bool y_pays(int64_t tokens, int64_t out, int64_t in, const Rounds& rounds) {
+  const int64_t mid = (tokens + 63) / 64 * ((out + 63) / 64);
   const bool one = rounds.count == 1;
   // one round of 128 x 128 that is 69 % full (200 / 256 by [11264, 2048] 16.9 / 17.3 (22.4 / 23.7), 1000 by [4096, 4096] 34 (38), 4096 by [1024, 2816]
   // 26.2 (28.3); 175 by [16384, 1024] 14.1 (13.2)); of few tokens over weights up to 2^26 (160 by [16384, 8192] 73 (65))
@@ -469,8 +481,8 @@ bool y_pays(int64_t tokens, int64_t out, int64_t in, const Rounds& rounds) {
   // one round of 128 x 256 over short K (500 by [11264, 2048] 27.4 (31.1), 1400 by [4096, 2048] 27.8 (30.8); 320 by [16384, 2048] 28 (26), 3000 by
   // [2048, 2048] 28.7 (28.3))
   if (tokens > 384 && one && rounds.wide) return rounds.full >= 62 && tokens <= 2048 && in <= 2048;
-  // more than a round of 64 x 64 (700 by [2048, 2048] 15.2 (13.8))
-  if (tokens > 256 && in >= 2048 && (tokens + 63) / 64 * ((out + 63) / 64) > 256) return false;
+  // more than a round of 64 x 64 (700 by [2048, 2048] 15.2 (13.8); 188 by [6544, 2176] 22.4 (17.7), 250 by [5632, 2048] 20.6 (16.4))
+  if (in >= 2048 && (tokens > 256 ? mid > 256 : in < 4096 && mid > 300)) return false;
   // several rounds that are full, over short K (1400 / 2000 by [8000, 1024] 33.2 / 40.6 (34.9 / 42.2))
   if (tokens > 512 && tokens <= 2048 && in <= 1024 && out <= 8192 && rounds.full >= 90) return true;
   if (tokens > 1024) return tokens <= 2048 && out <= 1024 && in <= 1024;  // (1400 by [1024, 1024] 8.9 (10.8))
@@ -487,10 +499,12 @@ bool y_pays(int64_t tokens, int64_t out, int64_t in, const Rounds& rounds) {
 // dX: the library is slow over a weight read across its rows, up to 9 2^20 results.
 bool dx_pays(int64_t tokens, int64_t out, int64_t in, const Rounds& rounds) {
   if (tokens * in > (9 << 20)) return false;
-  // 500 by [2048, 2048] 10.5 (15.1), [11264, 2048] 42 (63), [4096, 4096] 27.5 (34.6); 1024 by [11264, 2048] 54 (79), [12288, 4096] 94 (111)
-  if (tokens <= 1024) return true;
-  // several rounds: 88 % full (2000 by [2048, 5632] 53.5 (55.2); 1032 by [5632, 8192], 75 %, 120 (96))
-  if (rounds.count > 1) return rounds.full >= 88;
+  // several rounds: 88 % full (2000 by [2048, 5632] 53.5 (55.2); 1032 by [5632, 8192], 75 %, 120 (96); 607 by [5632, 14336], 72 %, 138 (99)), or the last
+  // one of a few tiles (700 by [2048, 11008], 516, 48.5 (56.7))
+  if (rounds.count > 1) return rounds.full >= 88 || (tokens <= 1024 && rounds.tiles % 256 <= 16);
+  // 500 by [2048, 2048] 10.5 (15.1), [11264, 2048] 42 (63), [4096, 4096] 27.5 (34.6); 1024 by [11264, 2048] 54 (79), [12288, 4096] 94 (111), but 614 by [32000,
+  // 8192] in wide tiles 406 (305)
+  if (tokens <= 1024) return !rounds.wide || out <= 16384;
   // one: of 88 tiles (1400 / 2000 by [3072, 2048] 23.7 / 29.5 (28.4 / 32.6), [8000, 1024] 35 / 44 (72 / 64)), of many tokens 62 % full (3000 / 4096 by
   // [2048, 2048] 29.6 / 35.5 (30.2 / 36.4), 3000 by [11264, 2048] 125 (130), [32000, 2048] 393 (344))
   return tokens <= 2048 ? rounds.tiles >= 88 : rounds.full >= 62 && out <= 16384;
@@ -515,7 +529,7 @@ bool dw_pays(int64_t tokens, int64_t out, int64_t in, const Rounds& rounds) {
 
 // C [M, N] over K, as `ds_narrow_gemm` takes it
 extern "C" int ds_narrow_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along) {
-  const Rounds rounds(M, N);
+  const Rounds rounds(M, N, K);
   if (!a_along) return dw_pays(K, M, N, rounds);
   return b_along ? y_pays(M, N, K, rounds) : dx_pays(M, K, N, rounds);
 }

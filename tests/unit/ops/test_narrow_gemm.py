@@ -81,6 +81,23 @@ def test_long_inner_dimensions(M, N, K):
 
 
 @GPU
+@pytest.mark.parametrize("form,M,N,K", [("dX", 128, 5376, 5120), ("dX", 120, 5504, 5120), ("dX", 128, 5504, 5056), ("dX", 57, 11008, 5632), ("dX", 250, 8192, 4160),
+                                        ("dX", 250, 8320, 4160), ("dX", 250, 5120, 3072), ("dX", 250, 5120, 3008), ("dX", 250, 7680, 3136), ("dX", 250, 7808, 3136), ("dX", 250, 7808, 4096),
+                                        ("dW", 376, 3584, 2705), ("dW", 1032, 1064, 2047), ("dW", 1032, 1064, 2048), ("dW", 1280, 1544, 2200), ("dW", 1280, 1536, 2200),
+                                        ("y", 52, 16384, 2048), ("y", 65, 16384, 2048), ("y", 52, 16392, 2048), ("y", 50, 2112, 4608), ("y", 50, 2048, 4608),
+                                        ("y", 238, 4096, 5120), ("y", 238, 4096, 5056), ("y", 100, 11008, 4096), ("y", 130, 5504, 8192),
+                                        ("dW", 2432, 6664, 1023), ("dW", 2432, 6664, 1024)])
+def test_cuts(form, M, N, K):
+    """Either side of the lines between tiles and parts; the same bits each time."""
+    ops = hip_ops()
+    a, b = _rnd(M, K, seed=1), _rnd(N, K, seed=2)
+    args = {"y": (a, b, True, True), "dX": (a, b.t().contiguous(), True, False), "dW": (a.t().contiguous(), b.t().contiguous(), False, False)}[form]
+    got = ops.narrow_gemm(*args)
+    _check(got, a, b)
+    assert torch.equal(got, ops.narrow_gemm(*args))
+
+
+@GPU
 @pytest.mark.parametrize("T,O,I", [(1027, 2056, 520), (1027, 520, 2056), (1500, 1608, 1608), (3001, 256, 1032), (8192, 136, 264), (300, 2048, 5632), (2049, 1032, 1024)])
 def test_gradients_of_many_tokens(T, O, I):
     """Tiles in bands of rows, the last one of fewer, over inner dimensions of any length; what the layer takes."""
