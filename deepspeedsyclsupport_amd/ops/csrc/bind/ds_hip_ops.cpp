@@ -560,6 +560,12 @@ Tensor linear_weight_grad(Tensor go, Tensor x) {
   return c.defined() ? c : at::mm(go.t(), x);
 }
 
+// Whether one of these two takes the tiles of 256 columns (else the caller may have copies along the inner dimension for the library's call)
+bool linear_grad_is_wide(Tensor go, Tensor b, bool weight_grad) {
+  int64_t M, N, K, lda, ldb;
+  return unwatched(go, b) && narrow_sizes(go, b, !weight_grad, false, M, N, K, lda, ldb) && ds_wide_gemm_pays(M, N, K, !weight_grad, false);
+}
+
 Tensor transpose16(Tensor x, int64_t pad_to) {
   TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1, "transpose16: 2-D device tensor, unit last stride");
   TORCH_CHECK(x.element_size() == 2, "transpose16: 16-bit dtypes only");
@@ -983,6 +989,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("xent_mean_node", &xent_mean_node);
   m.def("linear_weight_grad", &linear_weight_grad);
   m.def("narrow_gemm_tune", [](int64_t tile, int64_t parts) { ds_narrow_gemm_tune((int)tile, (int)parts); });
+  m.def("wide_gemm_tune", [](int64_t rows) { ds_wide_gemm_tune((int)rows); });
+  m.def("linear_grad_is_wide", &linear_grad_is_wide);
+  m.def("wide_gemm_pays", [](int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) { return ds_wide_gemm_pays(M, N, K, a_along, b_along) != 0; });
   m.def("transpose16", &transpose16, py::arg("x"), py::arg("pad_to") = 0);
   m.def("flash_fwd", &flash_fwd);
   m.def("flash_fwd_sparse", &flash_fwd_sparse, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("scale"),

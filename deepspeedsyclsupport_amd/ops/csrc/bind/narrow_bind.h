@@ -13,6 +13,8 @@ int64_t ds_narrow_gemm_scratch(int64_t, int64_t, int64_t, int, int);
 int ds_narrow_gemm_pays(int64_t, int64_t, int64_t, int, int);
 int ds_narrow_gemm(const void*, const void*, void*, int64_t, int64_t, int64_t, int64_t, int64_t, int, int, void*, hipStream_t);
 void ds_narrow_gemm_tune(int, int);
+int ds_wide_gemm_pays(int64_t, int64_t, int64_t, int, int);
+void ds_wide_gemm_tune(int);
 }
 
 namespace {
@@ -35,19 +37,23 @@ bool unwatched(const Tensor& a, const Tensor& b) {
   return !(at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad())) && unseen({&a, &b});
 }
 
-// A B^T over the inner dimension: a [M, K], or [K, M] if not a_along; b [N, K], or [K, N]. Undefined where the kernel does not take it
-// or (unless asked to take what it can) the library's is faster. sizes: the result's where it is no matrix (a view of one, made in an autograd
-// function, could not be changed in place).
-Tensor narrow_product(const Tensor& a, const Tensor& b, bool a_along, bool b_along, bool any, at::OptionalIntArrayRef sizes = c10::nullopt) {
+// A B^T over the inner dimension: a [M, K], or [K, M] if not a_along; b [N, K], or [K, N]. Whether the kernels take it as it lies.
+bool narrow_sizes(const Tensor& a, const Tensor& b, bool a_along, bool b_along, int64_t& M, int64_t& N, int64_t& K, int64_t& lda, int64_t& ldb) {
   if (!a.is_cuda() || a.device() != b.device() || a.scalar_type() != at::kBFloat16 || b.scalar_type() != at::kBFloat16 || a.dim() != 2 || b.dim() != 2 ||
       a.stride(1) != 1 || b.stride(1) != 1)
-    return Tensor();
-  const int64_t M = a.size(a_along ? 0 : 1), K = a.size(a_along ? 1 : 0), N = b.size(b_along ? 0 : 1);
-  const int64_t lda = a.size(0) > 1 ? a.stride(0) : a.size(1), ldb = b.size(0) > 1 ? b.stride(0) : b.size(1);
-  if (b.size(b_along ? 1 : 0) != K || !ds_narrow_gemm_ok(M, N, K, lda, ldb, a_along, b_along) || (!any && !ds_narrow_gemm_pays(M, N, K, a_along, b_along)))
-    return Tensor();
+    return false;
+  M = a.size(a_along ? 0 : 1), K = a.size(a_along ? 1 : 0), N = b.size(b_along ? 0 : 1);
+  lda = a.size(0) > 1 ? a.stride(0) : a.size(1), ldb = b.size(0) > 1 ? b.stride(0) : b.size(1);
+  return b.size(b_along ? 1 : 0) == K && ds_narrow_gemm_ok(M, N, K, lda, ldb, a_along, b_along) &&
+         !((uintptr_t)a.const_data_ptr() % 16 || (uintptr_t)b.const_data_ptr() % 16);
+}
+
+// The product. Undefined where the kernels do not take it or (unless asked to take what they can) the library's is faster. sizes: the result's where it
+// is no matrix (a view of one, made in an autograd function, could not be changed in place).
+Tensor narrow_product(const Tensor& a, const Tensor& b, bool a_along, bool b_along, bool any, at::OptionalIntArrayRef sizes = c10::nullopt) {
+  int64_t M, N, K, lda, ldb;
+  if (!narrow_sizes(a, b, a_along, b_along, M, N, K, lda, ldb) || (!any && !ds_narrow_gemm_pays(M, N, K, a_along, b_along))) return Tensor();
   const char *pa = (const char*)a.const_data_ptr(), *pb = (const char*)b.const_data_ptr();
-  if ((uintptr_t)pa % 16 || (uintptr_t)pb % 16) return Tensor();
   const c10::DeviceGuard guard(a.device());  // (the stream below is the tensors' device's, whichever is current)
   Tensor c = torch::empty(sizes ? *sizes : at::IntArrayRef{M, N}, a.options());
   const int64_t scratch = ds_narrow_gemm_scratch(M, N, K, a_along, b_along);

@@ -1,0 +1,177 @@
+// bf16 products of a linear layer of many tokens: y = X W^T, dX = dY W and dW = dY^T X, each over the operands as they lie in memory, sums in fp32, one
+// rounding at the end. Tiles of 256, 192 or 128 rows by 256 columns, with the loop of wide_core.h.
+#include "wide_core.h"
+
+#include <algorithm>
+#include <cmath>
+
+namespace {
+using namespace wide;
+
+struct WideArgs {
+  const bf16 *a, *b;  // a: M x K, b: N x K, or with rows along k: K x M, K x N
+  bf16* c;            // [M, N], rows ldc apart
+  int M, N, K, ldc;
+  uint32_t lda, ldb, abytes, bbytes;
+  int band;           // row tiles that are walked together, column by column
+};
+
+template <int AK, int BK, int MI>
+__global__ void __launch_bounds__(256, 1) wide_gemm_kernel(WideArgs a) {
+  typedef Loop<AK, BK, MI> L;
+  constexpr int TM = L::TM, TN = L::TN, NI = L::NI, STORES = MI * NI / 2;
+  __shared__ __attribute__((aligned(16))) char lds[L::LDS];
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int mt = (a.M + TM - 1) / TM, nt = (a.N + TN - 1) / TN, tiles = mt * nt;
+  // an XCD's tiles are neighbours; its workgroups take them in turn
+  const int xcd = blockIdx.x & 7, per = tiles >> 3, more = tiles & 7, stride = ((int)gridDim.x - xcd + 7) >> 3;
+  const int last = per * (xcd + 1) + min(xcd + 1, more);
+  int id = per * xcd + min(xcd, more) + ((int)blockIdx.x >> 3);
+  if (id >= last) return;
+  const int steps = (a.K + 63) / 64;
+  auto place = [&](int t, int& m0, int& n0) {
+    const int strip = t / (a.band * nt), spot = t - strip * a.band * nt, deep = min(a.band, mt - strip * a.band);
+    m0 = __builtin_amdgcn_readfirstlane((strip * a.band + spot % deep) * TM);
+    n0 = __builtin_amdgcn_readfirstlane(spot / deep * TN);
+  };
+  int m0, n0;
+  place(id, m0, n0);
+  L loop;
+  loop.oa.from = L::A::tile(a.a, a.abytes, a.lda, m0);
+  loop.ob.from = L::B::tile(a.b, a.bbytes, a.ldb, n0);
+  loop.begin(lds, a.lda, a.ldb, lane, wid);
+  for (;;) {
+    // the tile that follows, or this one's beginning again, for nobody
+    const bool ends = id + stride >= last;
+    int m2 = m0, n2 = n0;
+    if (!ends) place(id + stride, m2, n2);
+    loop.template tile<STORES>(steps, L::A::tile(a.a, a.abytes, a.lda, m2), L::B::tile(a.b, a.bbytes, a.ldb, n2));
+    // ---- a lane has columns 4 (lane / 16) .. + 3 of blocks n and n + 1: 16-lane rows change places, and it has eight neighbours. What lies past C's
+    // rows or columns lies past the buffer's end: every wave stores as often as the next tile's barrier counts.
+    // Past the caches (y, 6005 by [32000, 2048] 601 -> 556 us, 8192 by [22016, 4096] 998 -> 981): the next tile's second barrier waits for them.
+    const auto c = __builtin_amdgcn_make_buffer_rsrc(a.c + (int64_t)m0 * a.ldc, 0, (int)((uint32_t)(min(TM, a.M - m0) - 1) * a.ldc * 2 + a.N * 2), 0x00020000);
+    const int row = (wid & 1) * 16 * MI + (lane & 15), col = n0 + (wid >> 1) * 16 * NI + 16 * ((lane >> 4) & 1) + 8 * (lane >> 5);
+    each<NI / 2>([&](auto n_c) {
+      constexpr int n = 2 * n_c.value;
+      uint32_t at = (uint32_t)row * a.ldc * 2 + (col + 16 * n < a.N ? 2 * (col + 16 * n) : 0xc0000000u);
+      each<MI>([&](auto m_c) {
+        const f32x4 x = loop.acc[m_c.value][n], y = loop.acc[m_c.value][n + 1];
+        u32x4 o;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+#ifdef __HIP_DEVICE_COMPILE__
+          const auto v = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x[2 * q], x[2 * q + 1]}, bf16x2)),
+                                                          __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{y[2 * q], y[2 * q + 1]}, bf16x2)), false, false);
+          o[q] = v[0];
+          o[2 + q] = v[1];
+#endif
+        }
+        __builtin_amdgcn_raw_buffer_store_b128(o, c, at, 0, 2);  // (nt)
+        at += 32 * a.ldc;
+      });
+    });
+    if (ends) break;
+    id += stride;
+    m0 = m2;
+    n0 = n2;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the surplus transfers)
+}
+
+thread_local int g_rows = 0;  // (a thread's own)
+
+// us of a launch over tiles of so many rows: a round takes a step's clocks, and the chip's power its share for every tile, so a round that is not full costs
+// less than a full one. Drawn by 400 products at random (mean error 4 to 6 %; the rows chosen by it take 0.24 % longer than the best of the three in the mean);
+// tiles of 192 and 128 rows are put 4 % higher than the fit, as they read more and suffer where that comes from memory.
+double time_of(int rows, int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = (M + rows - 1) / rows * ((N + 255) / 256), rounds = (tiles + 255) / 256, steps = (K + 63) / 64;
+  const double step = rows == 256 ? 0.908 : rows == 192 ? 0.742 : 0.531, round = rows == 256 ? 5.9 : rows == 192 ? 4.3 : 2.9,
+               power = rows == 256 ? 0.965 : rows == 192 ? 0.772 : 0.551;
+  return 3 + std::hypot(rounds * (step * steps + round), tiles / 256. * power * steps);
+}
+
+// C in one part, or in two that are cut between rows or columns: tiles of `rows` up to m, n and of `other` beyond
+struct Plan {
+  int rows, other;
+  int64_t m, n;
+  double time;
+};
+
+// Tiles of 256 rows where they fill the chip's rounds, of fewer for what would leave a round half empty
+Plan plan_of(int64_t M, int64_t N, int64_t K) {
+  const int sizes[3] = {256, 192, 128};
+  if (g_rows) return {g_rows, 0, M, N, 0};
+  Plan best = {0, 0, M, N, 0};
+  auto offer = [&](const Plan& p) {
+    if (!best.rows || p.time < best.time) best = p;
+  };
+  for (int rows : sizes) {
+    offer({rows, 0, M, N, time_of(rows, M, N, K)});
+    const int64_t mt = (M + rows - 1) / rows, nt = (N + 255) / 256;
+    for (int64_t k = mt * nt / 256; k > 0 && k >= mt * nt / 256 - 1; --k) {  // the first part's rounds
+      const int64_t m = std::min<int64_t>(256 * k / nt, mt - 1) * rows, n = std::min<int64_t>(256 * k / mt, nt - 1) * 256;
+      for (int other : sizes) {
+        if (m > 0) offer({rows, other, m, N, time_of(rows, m, N, K) + time_of(other, M - m, N, K)});
+        if (n > 0) offer({rows, other, M, n, time_of(rows, M, n, K) + time_of(other, M, N - n, K)});
+      }
+    }
+  }
+  return best;
+}
+
+int launch(WideArgs a, int rows, int a_along, int b_along, hipStream_t st) {
+  const int64_t mt = (a.M + rows - 1) / rows, nt = (a.N + 255) / 256;
+  a.band = (int)std::min<int64_t>(4, mt);
+  const dim3 grid((unsigned)std::min<int64_t>(mt * nt, 256));
+#define GO(AK, BK)                                                                                            \
+  do {                                                                                                        \
+    if (rows == 256) hipLaunchKernelGGL((wide_gemm_kernel<AK, BK, 8>), grid, dim3(256), 0, st, a);            \
+    else if (rows == 192) hipLaunchKernelGGL((wide_gemm_kernel<AK, BK, 6>), grid, dim3(256), 0, st, a);       \
+    else hipLaunchKernelGGL((wide_gemm_kernel<AK, BK, 4>), grid, dim3(256), 0, st, a);                        \
+  } while (0)
+  if (a_along && b_along) GO(ALONG, ALONG);
+  else if (a_along) GO(ALONG, ACROSS);
+  else GO(ACROSS, ACROSS);
+#undef GO
+  DS_CHECK_LAUNCH();
+  return 0;
+}
+
+}  // namespace
+
+// Forces tiles of 256, 192 or 128 rows, in one part, for the calling thread's products; 0: by the rule
+extern "C" void ds_wide_gemm_tune(int rows) { g_rows = rows; }
+
+// Whether the kernel takes a product that ds_narrow_gemm_ok has, and is the fastest way: the estimate comes to a rate that neither the library's call nor the
+// narrow tiles reach on average. 1200 products of 400 layers at random (profiles/wide_products_at_random.csv), time here over the time before, in the
+// mean, by the rate of the estimate in TF/s: y 800 - 1000 0.92, 1000 - 1500 0.86, below 800 1.43; dX 800 - 1000 0.94, 1000 - 1500 0.81, below 1.8; dW 600 -
+// 800 0.90, 800 - 1500 0.82, below 1.4. Rows of 8192 and more that few tokens share come from memory, which the library waits for better (us here (there):
+// y, 640 by [12288, 11008] 179 (158), 467 by [10240, 8192] 78 (71), dX, 697 by [28672, 8192] 344 (301)).
+extern "C" int ds_wide_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along) {
+  // (four steps, which a tile of 128 rows has on their way; offsets within a tile's rows of C, of which a quarter of 32 bits marks none)
+  if (K <= 192 || N >= 1 << 21 || (!a_along && b_along)) return 0;
+  if (g_rows) return 1;
+  if ((a_along ? M : K) < 400 || M * N < 1 << 20 || (a_along && M <= 1152 && K >= 8192)) return 0;
+  return 2e-6 * M * N * K >= plan_of(M, N, K).time * (b_along ? 1000 : a_along ? 950 : 800);
+}
+
+// C [M, N] as ds_narrow_gemm takes it
+extern "C" int ds_wide_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_along, int b_along,
+                            hipStream_t st) {
+  const Plan p = plan_of(M, N, K);
+  const int64_t ar = a_along ? M : K, ac = a_along ? K : M, br = b_along ? N : K, bc = b_along ? K : N;
+  WideArgs a{(const bf16*)A, (const bf16*)B, (bf16*)C, (int)p.m, (int)p.n, (int)K, (int)N, (uint32_t)lda, (uint32_t)ldb,
+             (uint32_t)(((ar - 1) * lda + ac) * 2), (uint32_t)(((br - 1) * ldb + bc) * 2), 0};
+  int rc = launch(a, p.rows, a_along, b_along, st);
+  if (rc || (p.m == M && p.n == N)) return rc;
+  // the second part: rows of A and C from m on, or B's and C's columns from n on
+  const int64_t m = p.m < M ? p.m : 0, n = p.n < N ? p.n : 0, oa = m * (a_along ? lda : 1), ob = n * (b_along ? ldb : 1);
+  a.a += oa;
+  a.b += ob;
+  a.c += m * N + n;
+  a.M = (int)(M - m);
+  a.N = (int)(N - n);
+  a.abytes -= (uint32_t)(oa * 2);
+  a.bbytes -= (uint32_t)(ob * 2);
+  return launch(a, p.other, a_along, b_along, st);
+}

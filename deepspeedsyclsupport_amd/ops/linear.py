@@ -1,13 +1,12 @@
-"""Training linear layer with a K-major weight-gradient GEMM.
+"""Training linear layer.
 
-`dW = dY^T X` contracts over the token dimension. Read straight from the [T, out] / [T, in] activations both GEMM
-operands are MN-major, a layout the library GEMMs run at ~1.0-1.1 PF/s on MI355X for the Llama-7B shapes
-(T = 32768); with K-major operands the same GEMM runs at ~1.4-1.5 PF/s (`profiles/wgrad_gemm_layouts_r2.jsonl`).
-So for long token dimensions the backward first streams dY and X through the HBM-speed transpose kernel
-(`csrc/act/transpose.hip`) and then issues the K-major GEMM. The function also saves the Parameter (not a view of
+The products of many tokens run in tiles of 256 columns over the operands as they lie (`csrc/gemm/wide_gemm.hip`), those of
+few in `csrc/gemm/narrow_gemm.hip`, each where it is the faster way; the rest is the library's. Of what is left to that,
+`dW = dY^T X` and `dX = dY W` read operands across the inner dimension, a layout that the library runs at ~1.0-1.1 PF/s where
+K-major operands reach ~1.4-1.5 (`profiles/wgrad_gemm_layouts_r2.jsonl`): for long token dimensions the operands are first
+streamed through the HBM-speed transpose kernel (`csrc/act/transpose.hip`). The function also saves the Parameter (not a view of
 it), so under ZeRO-3 a released gathered weight is not kept alive by autograd (reference
-`runtime/zero/linear.py:43` LinearFunctionForZeroStage3). Short token dimensions take the products of
-`csrc/gemm/narrow_gemm.hip`.
+`runtime/zero/linear.py:43` LinearFunctionForZeroStage3).
 """
 import os
 
@@ -27,6 +26,11 @@ def _kmajor_ok(go, x):
             and x.dtype == go.dtype and T % 8 == 0 and go.shape[1] % 8 == 0 and x.shape[1] % 8 == 0)
 
 
+def _wide(go2d, other, weight_grad):
+    """Whether dW of [T, out] and [T, in], or dX of [T, out] and [out, in], takes the tiles of 256 columns, which want no copies."""
+    return _narrow(go2d, other) and hip_ops().linear_grad_is_wide(go2d, other, weight_grad)
+
+
 def _rows16(t):
     if t.stride(1) != 1 or t.stride(0) % 8 or t.data_ptr() % 16:
         t = t.contiguous()
@@ -37,6 +41,18 @@ def kmajor_wanted(rows, dtype):
     """Should a producer of a [rows, n] linear operand also write its token-contiguous copy? (same test as the
     weight-gradient GEMM's, so a copy is only made where it will be used)"""
     return _ENABLED and rows >= KMAJOR_MIN_ROWS and rows % 8 == 0 and dtype in (torch.bfloat16, torch.float16)
+
+
+def kmajor_of_gate(rows, dtype, width):
+    """Whether a gated activation of `width` columns should write the copies of its output and of its gradient: not where the weight
+    gradients that they are for take the operands as they lie. (Of the model's width this sees nothing: 0.3 of the layer's, as
+    in Llama's, where 2816 columns get the first copy and 5632 none.)"""
+    if not kmajor_wanted(rows, dtype):
+        return False, False
+    if dtype != torch.bfloat16:
+        return True, True
+    pays, model = hip_ops().wide_gemm_pays, int(0.3 * width)
+    return not pays(model, width, rows, False, False), not pays(2 * width, model, rows, False, False)
 
 
 STATS = {"kmajor_from_producer": 0, "kmajor_transposed": 0}  # how the weight-gradient operands were obtained
@@ -69,6 +85,8 @@ def weight_grad(go2d, x2d, go_kmajor=None, x_kmajor=None):
     LM head's 32760 shifted tokens -> 32768: measured 7.6 ms -> 5.0 ms for that GEMM). `x2d` may be None when the
     forward kept only `x_kmajor`."""
     T = go2d.shape[0]
+    if x2d is not None and x_kmajor is None and T >= KMAJOR_MIN_ROWS and _wide(go2d, x2d, True):
+        return hip_ops().linear_weight_grad(go2d, x2d)
     if x_kmajor is not None or _kmajor_ok(go2d, x2d):
         Tp = -(-T // 256) * 256
         got = _kmajor_of(go2d, go_kmajor, Tp)                                    # [out, Tp]
@@ -85,7 +103,7 @@ def input_grad(go2d, weight):
     """[T, out] . W [out, in] -> dX [T, in]. Read row-major, W is an MN-major B operand; for long token dimensions
     a K-major copy W^T [in, out] (one HBM-speed transpose of the weight, ~0.04 ms for a 7B layer's QKV) turns the
     product into the TN layout of the forward GEMMs."""
-    if _DGRAD_ENABLED and _kmajor_ok(go2d, weight) and weight.dim() == 2 and weight.stride(1) == 1:
+    if _DGRAD_ENABLED and _kmajor_ok(go2d, weight) and weight.dim() == 2 and weight.stride(1) == 1 and not _wide(go2d, weight, False):
         wt = hip_ops().transpose16(_rows16(weight))   # [in, out]
         return torch.mm(go2d, wt.t())
     if _narrow(go2d, weight):

@@ -39,6 +39,7 @@ EXTENSIONS = {
             "act/dropout_kernels.hip",
             "act/transpose.hip",
             "gemm/narrow_gemm.hip",
+            "gemm/wide_gemm.hip",
             "rope/rope_kernels.hip",
             "xent/xent_kernels.hip",
             "attn/decode_attn.hip",
@@ -69,6 +70,7 @@ EXTENSIONS = {
             "gemv/skinny_mfma.hip",
             "gemv/skinny_bf16_sh.hip",
             "gemm/narrow_gemm.hip",
+            "gemm/wide_gemm.hip",
             "ragged/upload.hip",
         ],
         "bindings": ["bind/gemv_bind.cpp"],

@@ -116,9 +116,11 @@ class _GatedActKMajorFn(torch.autograd.Function):
     them to a separate transpose pass (see `ops/linear.py`)."""
 
     @staticmethod
-    def forward(ctx, gu, act):
-        ctx.act = act
+    def forward(ctx, gu, act, of_out, of_grad):
+        ctx.act, ctx.of_grad = act, of_grad
         ctx.save_for_backward(gu)
+        if not of_out:
+            return hip_ops().gated_act_fwd(gu, act), None
         out, out_t = hip_ops().gated_act_fwd_t(gu, act, 256)
         ctx.mark_non_differentiable(out_t)
         return out, out_t
@@ -126,20 +128,23 @@ class _GatedActKMajorFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout, _unused=None):
         (gu, ) = ctx.saved_tensors
+        if not ctx.of_grad:
+            return hip_ops().gated_act_bwd(dout.contiguous(), gu, ctx.act), None, None, None
         dgu, dgu_t = hip_ops().gated_act_bwd_t(dout.contiguous(), gu, ctx.act, 256)
         dgu._ds_kmajor = dgu_t
-        return dgu, None
+        return dgu, None, None, None
 
 
 def gated_activation(gate_up, act="silu"):
     """[.., 2I] = [gate | up] -> act(gate) * up  (SwiGLU for act='silu', GEGLU for 'gelu')."""
     code = ACT_CODES[act]
     if gate_up.is_cuda and (gate_up.shape[-1] // 2) % 8 == 0:
-        from ..linear import kmajor_wanted
+        from ..linear import kmajor_of_gate
         rows = gate_up.numel() // gate_up.shape[-1]
-        if gate_up.requires_grad and torch.is_grad_enabled() and kmajor_wanted(rows, gate_up.dtype):
-            out, out_t = _GatedActKMajorFn.apply(gate_up.contiguous(), code)
-            out._ds_kmajor = out_t
+        if gate_up.requires_grad and torch.is_grad_enabled() and any(copies := kmajor_of_gate(rows, gate_up.dtype, gate_up.shape[-1] // 2)):
+            out, out_t = _GatedActKMajorFn.apply(gate_up.contiguous(), code, *copies)
+            if out_t is not None:
+                out._ds_kmajor = out_t
             return out
         gate_up = gate_up.contiguous()
         out = hip_ops().gated_act_node(gate_up, code) if unseen_from_python(gate_up) else None

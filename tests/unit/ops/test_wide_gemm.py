@@ -1,0 +1,102 @@
+"""Products of many tokens in tiles of 256 columns (`csrc/gemm/wide_gemm.hip`) and the layers that take them."""
+import pytest
+import torch
+
+from deepspeedsyclsupport_amd.ops import linear as L
+from deepspeedsyclsupport_amd.ops.native import hip_ops
+
+GPU = pytest.mark.gpu
+
+
+def _rnd(*shape, seed=0):
+    return torch.randn(*shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(seed)).bfloat16()
+
+
+def _check(got, a, b):
+    """One rounding to bf16 (2^-9 of the value) and sums of K products in fp32, off by less than K 2^-23 of the magnitudes' sum."""
+    a, b = a.double(), b.double()
+    want, size = a @ b.t(), a.abs() @ b.abs().t()
+    assert got.shape == want.shape
+    assert ((got.double() - want).abs() <= want.abs() * 2**-8 + size * a.shape[1] * 2**-23).all()
+
+
+@GPU
+@pytest.mark.parametrize("rows", [256, 192, 128])
+@pytest.mark.parametrize("M,N,K", [(8, 8, 256), (128, 256, 256), (136, 264, 320), (200, 248, 448), (264, 520, 576), (520, 1032, 1088), (4104, 4872, 256)])
+def test_tiles_at_their_edges(M, N, K, rows):
+    """Every form; tiles that rows or columns do not fill; the fewest steps, and more; several tiles a workgroup; operands that are columns of
+    wider matrices; the same bits each time."""
+    ops = hip_ops()
+    a, b = _rnd(M, K, seed=1), _rnd(N, K, seed=2)
+    wide_a, wide_b = _rnd(M, K + 24, seed=3), _rnd(K, N + 16, seed=4)
+    at, bt = a.t().contiguous(), b.t().contiguous()
+    ops.wide_gemm_tune(rows)
+    try:
+        got = ops.narrow_gemm(a, b, True, True)
+        _check(got, a, b)
+        assert torch.equal(got, ops.narrow_gemm(a, b, True, True))
+        _check(ops.narrow_gemm(a, bt, True, False), a, b)
+        _check(ops.narrow_gemm(wide_a[:, 8:8 + K], wide_b[:, 8:8 + N], True, False), wide_a[:, 8:8 + K], wide_b[:, 8:8 + N].t())
+        for k in (K, K - 1, K - 37, 193):   # (an inner dimension of any length)
+            _check(ops.narrow_gemm(at[:k], bt[:k], False, False), a[:, :k], b[:, :k])
+    finally:
+        ops.wide_gemm_tune(0)
+
+
+@GPU
+@pytest.mark.parametrize("T,O,I", [(1500, 8192, 1024), (2048, 5632, 2048), (4096, 3072, 1536), (4200, 2824, 2816), (1156, 11008, 4096), (8200, 2048, 5632), (600, 8192, 4096)])
+def test_products_of_a_layer(T, O, I):
+    """In one part and in two, cut between rows or columns, as the rule has it."""
+    ops = hip_ops()
+    x, w, go = _rnd(T, I, seed=1), _rnd(O, I, seed=2), _rnd(T, O, seed=3)
+    _check(L.plain_linear(x, w), x, w)
+    _check(ops.narrow_gemm(x, w, True, True), x, w)
+    if O % 64 == 0:
+        _check(L.input_grad(go, w), go, w.t())
+        _check(ops.narrow_gemm(go, w, True, False), go, w.t())
+    _check(L.weight_grad(go, x), go.t(), x.t())
+    got = ops.narrow_gemm(go, x, False, False)
+    _check(got, go.t(), x.t())
+    assert torch.equal(got, ops.narrow_gemm(go, x, False, False))
+
+
+@GPU
+def test_values_that_do_not_mix():
+    """Infinities and NaN stay in their rows; nothing from past the end of an operand, or of the inner dimension, comes in."""
+    ops = hip_ops()
+    a, b = _rnd(300, 256), _rnd(280, 256, seed=1)
+    a[3, 5], a[4, 7] = float("inf"), float("nan")
+    big = _rnd(300, 600, seed=2)
+    big[260:] = float("nan")
+    ops.wide_gemm_tune(256)
+    try:
+        y = ops.narrow_gemm(a, b, True, True)
+        keep = [i for i in range(300) if i not in (3, 4)]
+        _check(y[keep], a[keep], b)
+        assert not y[3].isfinite().any() and y[4].isnan().all()
+        _check(ops.narrow_gemm(big[:260, :256], b, True, True), big[:260, :256], b)
+        _check(ops.narrow_gemm(big[:257, :272], big[:257, 272:600], False, False), big[:257, :272].t(), big[:257, 272:600].t())
+    finally:
+        ops.wide_gemm_tune(0)
+
+
+@GPU
+@pytest.mark.parametrize("I,copies", [(704, 2), (2816, 1), (5632, 0)])
+def test_copies_of_gated_activations(I, copies):
+    """Of 8192 tokens on the gate writes the copies along the tokens that the weight gradients around it will read, and only those."""
+    from deepspeedsyclsupport_amd.ops.transformer import functional as DF
+    T, H = 8192, max(256, I * 3 // 8 // 64 * 64)
+    assert sum(L.kmajor_of_gate(T, torch.bfloat16, I)) == copies
+    x, w1, w2 = (_rnd(*s, seed=i).mul_(0.05 if i else 1).requires_grad_() for i, s in enumerate(((T, H), (2 * I, H), (H, I))))
+    before = dict(L.STATS)
+    act = DF.gated_activation(L.linear(x, w1), "silu")
+    y = L.linear(act, w2)
+    go = _rnd(T, H, seed=5)
+    got = torch.autograd.grad(y, (x, w1, w2), go)
+    if copies == 0:
+        assert L.STATS == before
+    xf, w1f, w2f = (t.detach().float().requires_grad_() for t in (x, w1, w2))
+    h = xf @ w1f.t()
+    want = torch.autograd.grad((torch.nn.functional.silu(h[:, :I]) * h[:, I:]) @ w2f.t(), (xf, w1f, w2f), go.float())
+    for g, r in zip(got, want):
+        assert ((g.float() - r).norm() / r.norm()).item() < 1e-2
