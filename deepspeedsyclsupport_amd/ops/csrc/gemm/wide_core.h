@@ -73,6 +73,22 @@ __device__ __forceinline__ void product_and_dma(f32x4& c, bf16x8 a, bf16x8 b, i3
                  : "v"(a), "v"(b), "v"(lane_bytes), "s"(from), "s"(to), "i"(more)
                  : "memory", "scc");
 }
+__device__ __forceinline__ void dma16(i32x4, const char* from, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(from) : "memory");
+}
+template <bool FIRST>
+__device__ __forceinline__ void product_and_dma(f32x4& c, bf16x8 a, bf16x8 b, i32x4, const char* from, uint32_t to, int more) {
+  if constexpr (FIRST)
+    asm volatile("s_add_u32 m0, %4, %5\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, 0\n\tglobal_load_lds_dwordx4 %3, off"
+                 : "=&a"(c)
+                 : "v"(a), "v"(b), "v"(from), "s"(to), "i"(more)
+                 : "memory", "scc");
+  else
+    asm volatile("s_add_u32 m0, %4, %5\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %3, off"
+                 : "+a"(c)
+                 : "v"(a), "v"(b), "v"(from), "s"(to), "i"(more)
+                 : "memory", "scc");
+}
 __device__ __forceinline__ void hold(f32x4& c) { asm volatile("" : "+a"(c)); }
 
 // All of this wave's LDS accesses and all but its NEWER latest transfers and stores are done, then those of all waves.
@@ -84,69 +100,85 @@ __device__ __forceinline__ void meet() {
   asm volatile("s_barrier" ::: "memory");
 }
 
-// How an operand lies: its rows across the inner dimension, or along it
-enum : int { ACROSS = 0, ALONG = 1 };
+// How an operand lies: its rows across the inner dimension; along it; along it in rows that lie anywhere, by 64-bit addresses; in operand order (blocks of
+// 16 rows, of which 64 columns at a time are 2 KB: `preshuffle16` of ops/bf16_gemv.py)
+enum : int { ACROSS = 0, ALONG = 1, FAR = 2, ORDERED = 3 };
 
 // One operand's R rows (or columns) of a step of 64, of which a wave multiplies F blocks of 16: its way into LDS and out of it
 template <int LAY, int R, int F>
 struct Operand {
   static constexpr int BYTES = R * 128, PIECES = R / 32;  // LDS bytes a step, transfers of 1 KB a wave
-  i32x4 from;                  // the tile, from the step of the next transfers on
-  uint32_t src[PIECES], step;  // per lane: bytes from there; bytes from a step to the next
-  uint32_t at[LAY == ALONG ? 2 : F];  // LDS address of the lane's reads in the slot at work: of either half, or of each block
+  static constexpr int BASES = LAY == ACROSS ? F : LAY == ORDERED ? 1 : 2;
+  typedef std::conditional_t<LAY == FAR, const char*, uint32_t> Source;
+  i32x4 from;          // the tile, from the step of the next transfers on
+  Source src[PIECES];  // per lane: bytes from there (FAR: where they are)
+  uint32_t step;       // bytes from a step to the next
+  uint32_t at[BASES];  // LDS address of the lane's reads in the slot at work: of either half, of each block, or of all
 
   static __device__ __forceinline__ i32x4 tile(const bf16* p, uint32_t bytes, uint32_t ld, int r0) {
-    const uint32_t off = LAY == ALONG ? (uint32_t)r0 * ld * 2 : 2u * r0;
+    const uint32_t off = LAY == ACROSS ? 2u * r0 : (uint32_t)r0 * ld * 2;
     return buffer_of((const char*)p + off, bytes - off);
   }
   // A transposed read takes 32 bytes of four rows, and of the four that lie 8 further, at a time: those of rows of 2 R bytes that meet in a bank are apart
   static __device__ __forceinline__ int turn(int r) { return (R % 128 ? ((r >> 1) & 1) << 2 : (r & 3) << 2) ^ (((r >> 3) & 1) << 1); }
-  // r0: first of the wave's rows in the tile
-  __device__ __forceinline__ void init(uint32_t ld, uint32_t slot, int r0, int lane, int wid) {
+  // Row r of a step of rows along the inner dimension: 8 chunks of 16 bytes, chunk c at c ^ (r / 2 % 8). Of the lane's row in piece i
+  static __device__ __forceinline__ int row(int i, int lane, int wid) { return 8 * (wid * PIECES + i) + (lane >> 3); }
+  static __device__ __forceinline__ uint32_t chunk(int i, int lane, int wid) { return 16 * ((lane & 7) ^ ((row(i, lane, wid) >> 1) & 7)); }
+  // Rows ld apart
+  __device__ __forceinline__ void sources(uint32_t ld, int lane, int wid) {
     step = __builtin_amdgcn_readfirstlane(LAY == ALONG ? 128 : 128 * ld);
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
-      const int piece = wid * PIECES + i;
-      if constexpr (LAY == ALONG) {  // 8 rows of 8 chunks of 16 bytes: chunk c of row r at c ^ (r / 2 % 8)
-        const int r = 8 * piece + (lane >> 3);
-        src[i] = (uint32_t)r * ld * 2 + 16 * ((lane & 7) ^ ((r >> 1) & 7));
+      if constexpr (LAY == ALONG) {
+        src[i] = (uint32_t)row(i, lane, wid) * ld * 2 + chunk(i, lane, wid);
       } else {  // R / 8 chunks of each of the step's rows, swizzled by `turn`
-        const int c = piece * 64 + lane, r = c / (R / 8);
+        const int c = (wid * PIECES + i) * 64 + lane, r = c / (R / 8);
         src[i] = (uint32_t)r * ld * 2 + 16 * (c % (R / 8) ^ turn(r));
       }
     }
-    if constexpr (LAY == ALONG) {
-      const int r = r0 + (lane & 15);
-#pragma unroll
-      for (int h = 0; h < 2; ++h) at[h] = slot + r * 128 + 16 * ((4 * h + (lane >> 4)) ^ ((r >> 1) & 7));
-    } else {
+  }
+  // r0: first of the wave's rows in the tile
+  __device__ __forceinline__ void reads(uint32_t slot, int r0, int lane) {
+    if constexpr (LAY == ACROSS) {
       const int k = 8 * (lane >> 4) + ((lane >> 2) & 3);
 #pragma unroll
       for (int f = 0; f < F; ++f) at[f] = slot + k * 2 * R + 16 * ((r0 / 8 + 2 * f + ((lane >> 1) & 1)) ^ turn(k)) + 8 * (lane & 1);
+    } else if constexpr (LAY == ORDERED) {  // chunk 2 q + h of a block's row r at 64 h + 16 q + r
+      at[0] = slot + r0 * 128 + 1024 * ((lane >> 4) & 1) + 256 * (lane >> 5) + 16 * (lane & 15);
+    } else {
+      const int r = r0 + (lane & 15);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) at[h] = slot + r * 128 + 16 * ((4 * h + (lane >> 4)) ^ ((r >> 1) & 7));
     }
   }
-  // The next transfers: a step further, or another tile's first
-  __device__ __forceinline__ void next() {
-    const uint64_t p = ((uint64_t)(uint32_t)from[1] << 32 | (uint32_t)from[0]) + step;
-    from[0] = (int)(uint32_t)p;
-    from[1] = (int)(uint32_t)(p >> 32);
-    if constexpr (LAY == ACROSS) from[2] -= (int)step;  // (rows past the end read as zero)
+  // The next transfers: `by` bytes further, or another tile's first
+  __device__ __forceinline__ void next(uint32_t by) {
+    if constexpr (LAY == FAR) {
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i) src[i] += by;
+    } else {
+      const uint64_t p = ((uint64_t)(uint32_t)from[1] << 32 | (uint32_t)from[0]) + by;
+      from[0] = (int)(uint32_t)p;
+      from[1] = (int)(uint32_t)(p >> 32);
+      if constexpr (LAY == ACROSS) from[2] -= (int)by;  // (rows past the end read as zero)
+    }
   }
   __device__ __forceinline__ void next(bool other, const i32x4& tile) {
-    next();
+    next(step);
 #pragma unroll
     for (int i = 0; i < 3; ++i) from[i] = other ? tile[i] : from[i];
   }
   // Block B of half H; a step's first half lies in a slot `delta` further than what was read last
   template <int H, int B>
   __device__ __forceinline__ bf16x8 read(uint32_t delta) {
-    if constexpr (LAY == ALONG) {
-      if constexpr (H == 0 && B == 0) at[0] += delta;
-      if constexpr (H == 0 && B == 1) at[1] += delta;
+    if constexpr (H == 0 && B < BASES) at[B] += delta;
+    if constexpr (LAY == ORDERED) {
+      const lds_char* p = (const lds_char*)(uintptr_t)at[0];
+      return *reinterpret_cast<const lds_bf16x8*>(p + B * 2048 + H * 512);
+    } else if constexpr (LAY != ACROSS) {
       const lds_char* p = (const lds_char*)(uintptr_t)at[H];
       return *reinterpret_cast<const lds_bf16x8*>(p + B * 2048);
     } else {
-      if constexpr (H == 0) at[B] += delta;
       lds_char* p = (lds_char*)(uintptr_t)at[B];
       s16x8 v;
 #ifdef __HIP_DEVICE_COMPILE__
@@ -159,12 +191,12 @@ struct Operand {
   }
 };
 
-// A's and B's rings, and the loop over one tile's steps after another's
-template <int AK, int BK, int MI>
+// A's and B's rings, and the loop over one tile's steps, after another's (CHAIN) or alone
+template <int AK, int BK, int MI, bool CHAIN>
 struct Loop {
   static constexpr int NI = 8, TM = 32 * MI, TN = 32 * NI;
   // 160 KB: as many steps ahead as there is room for
-  static constexpr int RA = MI == 8 ? 3 : 4, RB = MI == 4 ? 3 : 2;
+  static constexpr int RA = MI == 8 ? 3 : 4, RB = MI == 2 ? 4 : MI == 4 ? 3 : 2;
   typedef Operand<AK, TM, MI> A;
   typedef Operand<BK, TN, NI> B;
   static constexpr int PA = A::PIECES, PB = B::PIECES, LDS = RA * A::BYTES + RB * B::BYTES;
@@ -175,7 +207,7 @@ struct Loop {
   static constexpr int EVERY = (MEET - 1) / (EARLY > LATE ? EARLY : LATE);  // products from a transfer to the next
   // At a step's barrier the next step has to be there: what may be newer than its last piece of B, and of A
   static constexpr int NEWER_B = PA + (RB - 2) * (PA + PB), NEWER_A = (RA - 2) * (PA + PB), NEWER = NEWER_B < NEWER_A ? NEWER_B : NEWER_A;
-  static constexpr int STEPS = RA > RB ? RA : RB;         // the fewest of a tile
+  static constexpr int STEPS = CHAIN ? (RA > RB ? RA : RB) : 1;  // the fewest of a tile
   static_assert(LDS <= 160 * 1024 && EVERY >= 1 && LATE <= PB);
 
   A oa;
@@ -193,21 +225,21 @@ struct Loop {
   __device__ __forceinline__ void move_b(int slot) {
     each<N>([&](auto i) { dma16(ob.from, ob.src[i.value], first_b + slot * B::BYTES + 1024 * i.value); });
   }
-  // Before the first tile; oa.from and ob.from are its beginning
-  __device__ __forceinline__ void begin(char* lds, uint32_t lda, uint32_t ldb, int lane, int wid) {
+  // Before the first tile, of so many steps; from, src and step are the operands'
+  __device__ __forceinline__ void begin(char* lds, int steps, int lane, int wid) {
     const uint32_t base = (uint32_t)(uintptr_t)(lds_char*)lds, bbase = base + RA * A::BYTES;
-    oa.init(lda, base, (wid & 1) * 16 * MI, lane, wid);
-    ob.init(ldb, bbase, (wid >> 1) * 16 * NI, lane, wid);
+    oa.reads(base, (wid & 1) * 16 * MI, lane);
+    ob.reads(bbase, (wid >> 1) * 16 * NI, lane);
     first_a = base + wid * PA * 1024;
     first_b = bbase + wid * PB * 1024;
-    each<(RA > RB ? RA : RB)>([&](auto s) {
-      if constexpr (s.value < RB - 1) { move_b<PB>(s.value); ob.next(); }
+    each<(RA > RB ? RA : RB)>([&](auto s) {  // (past the end of a tile alone its last step again, for nobody)
+      if constexpr (s.value < RB - 1) { move_b<PB>(s.value); ob.next(CHAIN || s.value + 1 < steps ? ob.step : 0); }
       if constexpr (s.value == RB - 1) move_b<LATE>(s.value);
-      if constexpr (s.value < RA - 1) { move_a<PA>(s.value); oa.next(); }
+      if constexpr (s.value < RA - 1) { move_a<PA>(s.value); oa.next(CHAIN || s.value + 1 < steps ? oa.step : 0); }
     });
     da = first_a + (RA - 1) * A::BYTES;
     db = first_b + (RB - 1) * B::BYTES;
-    if constexpr (LATE == PB) { db = first_b; ob.next(); }
+    if constexpr (LATE == PB) { db = first_b; ob.next(CHAIN || RB < steps ? ob.step : 0); }
     ta = tb = 0;
     // (the first two steps: the first barrier counts by what was stored before it, which here is nothing)
     constexpr int AFTER = (RB > 2 ? (RB - 3) * PB + LATE : 0) + (RA - 3) * PA;
@@ -216,6 +248,12 @@ struct Loop {
     each<MI>([&](auto i) { xa[0][i.value] = oa.template read<0, i.value>(0); });
   }
 
+  // The operand's next transfers, which are those of AHEAD steps from here on
+  template <int AHEAD, class O>
+  __device__ __forceinline__ void go(O& o, int left, const i32x4& after) {
+    if constexpr (CHAIN) o.next(left == AHEAD, after);
+    else o.next(left > AHEAD ? o.step : 0);
+  }
   // Half H of a step, `left` steps of the tile left with it. after: where the tile that follows begins. STORES: those since the tile before (its first half).
   template <int H, bool FIRST, int STORES>
   __device__ __forceinline__ void half(int left, const i32x4& after_a, const i32x4& after_b) {
@@ -231,19 +269,19 @@ struct Loop {
         }
       });
       // the slots and addresses of the next transfers, once those of before are out
-      if constexpr (H == 0 && t == ALL - 3) oa.next(left == RA, after_a);
+      if constexpr (H == 0 && t == ALL - 3) go<RA>(oa, left, after_a);
       if constexpr (H == 0 && t == ALL - 2) {
         const uint32_t turned = da == first_a + (RA - 1) * A::BYTES ? first_a : da + A::BYTES;  // slot of step s + RA, as of step s
         da = turned;
         ta = turned == first_a + (RA - 1) * A::BYTES ? -(uint32_t)(RA - 1) * A::BYTES : A::BYTES;
       }
       if constexpr (H == 0 && t == ALL - 1) {
-        if constexpr (LATE < PB) ob.next(left == RB, after_b);
+        if constexpr (LATE < PB) go<RB>(ob, left, after_b);
         const uint32_t turned = LATE < PB ? (db == first_b + (RB - 1) * B::BYTES ? first_b : db + B::BYTES) : db;
         db = turned;
         tb = turned == first_b + (RB - 1) * B::BYTES ? -(uint32_t)(RB - 1) * B::BYTES : B::BYTES;
       }
-      if constexpr (H == 1 && LATE == PB && t == ALL - 3) ob.next(left == RB + 1, after_b);
+      if constexpr (H == 1 && LATE == PB && t == ALL - 3) go<RB + 1>(ob, left, after_b);
       if constexpr (H == 1 && LATE == PB && t == ALL - 2) db += tb;
       __builtin_amdgcn_sched_barrier(0);
       constexpr int m = t / NI, n = m & 1 ? NI - 1 - t % NI : t % NI;

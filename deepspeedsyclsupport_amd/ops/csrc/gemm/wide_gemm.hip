@@ -18,7 +18,7 @@ struct WideArgs {
 
 template <int AK, int BK, int MI>
 __global__ void __launch_bounds__(256, 1) wide_gemm_kernel(WideArgs a) {
-  typedef Loop<AK, BK, MI> L;
+  typedef Loop<AK, BK, MI, true> L;
   constexpr int TM = L::TM, TN = L::TN, NI = L::NI, STORES = MI * NI / 2;
   __shared__ __attribute__((aligned(16))) char lds[L::LDS];
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -39,7 +39,9 @@ __global__ void __launch_bounds__(256, 1) wide_gemm_kernel(WideArgs a) {
   L loop;
   loop.oa.from = L::A::tile(a.a, a.abytes, a.lda, m0);
   loop.ob.from = L::B::tile(a.b, a.bbytes, a.ldb, n0);
-  loop.begin(lds, a.lda, a.ldb, lane, wid);
+  loop.oa.sources(a.lda, lane, wid);
+  loop.ob.sources(a.ldb, lane, wid);
+  loop.begin(lds, steps, lane, wid);
   for (;;) {
     // the tile that follows, or this one's beginning again, for nobody
     const bool ends = id + stride >= last;

@@ -11,10 +11,10 @@
 //    operand order and every wave has rows of its own, so they go from memory to registers in 512-byte runs, one step of 64
 //    ahead; only the entries' rows pass through LDS (swizzled, two buffers). Two workgroups share a CU. Workgroups walk groups
 //    of 4 column tiles by all row tiles of an expert, so that those at work on an XCD at a time share both operands in its L2.
-//  * big tile: a hundred rows per expert or more. 256 entries x 256 weight rows per workgroup of 4 waves, entries' rows through LDS by
-//    DMA (four buffers of 64 columns, 128 KB), weights straight into registers: see expert_big_kernel.
+//  * big tile: a hundred rows per expert or more. 256 entries x 256 weight rows per workgroup of 4 waves, both by DMA through LDS: see expert_big_kernel.
 //  * any: a workgroup per entry and 64 columns; fp32 and widths that are no multiple of 8.
 #include "ds_hip.h"
+#include "../gemm/wide_core.h"
 
 #include <type_traits>
 
@@ -380,205 +380,79 @@ __global__ void __launch_bounds__(256, 2) expert_tile_kernel(ExpertArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------ hundreds of rows per expert
-// What bounds the tile kernel above is traffic into the CU: for each step of 64 columns its two workgroups take 2 x (128 + 256)
-// rows, 48 bytes a clock at the full matrix rate. One tile of 256 x 256 takes 32. Of that tile's step (2048 clocks of the matrix
-// cores) LDS would be busy as long with both operands in it and waves of 64 x 128; so
-//  * four waves, one on a SIMD with all its registers, have 64 weight rows (gated: 32 of either part) by all 256 entries each: no
-//    wave reads another's weights, which go from memory (operand order: 512-byte runs) to registers two steps ahead. LDS carries the
-//    entries' rows alone, 1280 of the 2048 clocks, by DMA three steps ahead into four buffers; swizzled by the source address,
-//    read without bank conflicts a quarter step ahead;
-//  * a step is 64 products of 32 x 32 x 16; one LDS read, at most one transfer and one load of weights go between two of them. One barrier a
-//    step. Every wait counts what may still be on its way: buffers are arrays apart, and all accesses buffer instructions (hipcc waits
-//    for everything where LDS transfers are global ones), so the compiler's own waits for weights count too. Tail steps issue the last
-//    step's transfers again, so that the counts stand;
-//  * beyond 4 GB of rows (LONG) the transfers take an address of 64 bits a lane instead, as inline asm; the compiler's waits for weights
-//    then count weights alone, and are stricter than they need be. 266240 rows of 8192 among 8 experts of 4096: 14.5 ms (eight waves 15.5, the
-//    tile kernel 18.5). Long loops of less take 0.9 % more that way (32 x 1024 rows above 1725 and 1741, plain 901 and 909);
-//  * rows in units of 64 (MT): a short tile moves and multiplies no others.
-// Workgroups walk groups of 8 column tiles by all row tiles of an expert. Then bound by power: 1.6 GHz, matrix cores busy 77 % of the time in
-// a long loop; without any transfers 1.75 GHz and 83 %. 16 x 16 x 32 products: hipcc moves accumulators about, 1.05 times the time.
-// 32 experts, 1024 rows each on average, at random: 3584 gated columns of 4096: 1812 -> 1683 us (all even 1680 -> 1561), 4096 plain columns of
-// 3584: 990 -> 880 us (eight waves, both operands in LDS, a wait for all transfers every step); 256 rows: 655 -> 579; 8 x 128 rows: 115 -> 97.
-// Finding the place in registers is 2 % of it. A gate by the hardware's exponential and reciprocal would be another 3 to 5 % (1617, 1510), but its error
-// grows as |g| 2^-24, past that of expf and a division from |g| = 5 on.
+// A tile of 256 entries by 256 weight rows (gated: 128 of either part, block by block in turn, so that a lane has gate and up of the same columns), with the
+// loop of gemm/wide_core.h: power bounds it there. Rows in units of 64 (MI): a short tile moves and multiplies no others. Workgroups walk groups of 8
+// column tiles by all row tiles of an expert. Beyond 4 GB of rows (LONG) their transfers take an address of 64 bits a lane.
 constexpr int TM = 256, TN = 256;
-typedef __attribute__((address_space(3))) char lds_char;
-typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
-typedef __attribute__((address_space(3))) void lds_void;
-
-// 16 bytes per lane to LDS bytes dst + 16 lane. (The host's pass does not know the size.)
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t from, uint32_t lane_bytes, uint32_t bytes, lds_char* dst) {
-#ifdef __HIP_DEVICE_COMPILE__
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void*)dst, 16, lane_bytes, bytes, 0, 0);
-#endif
-}
-__device__ __forceinline__ void dma16(const char* from, lds_char* dst) {
-  uint32_t keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep)
-               : "v"(from), "s"(__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)dst))
-               : "memory");
-}
-// All of this wave's LDS accesses and all but its NEWER latest loads are done, then those of all waves.
-template <int NEWER>
-__device__ __forceinline__ void meet() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt((NEWER & 15) | 7 << 4 | (NEWER >> 4) << 14);
-  asm volatile("s_barrier" ::: "memory");
-}
 
 template <bool GLU, bool LONG>
 __global__ void __launch_bounds__(256, 1) expert_big_kernel(ExpertArgs a) {
-  // rows of a step each, as arrays apart: the compiler then knows which transfers a read has to wait for
-  __shared__ __attribute__((aligned(16))) char b0[TM * 128], b1[TM * 128], b2[TM * 128], b3[TM * 128];
-  __shared__ int ents[TM];
-  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
-  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  __shared__ __attribute__((aligned(16))) char lds[160 * 1024];
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int N = a.N, K = a.K, KQ = K / 64;
   Place pl;
   if (!place_of<TM, 8>(a, GLU ? TN / 2 : TN, pl)) return;
-  const int e = pl.e, n0 = pl.n0, left = min(TM, pl.left);
-  const auto xs = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, (int)a.xbytes, 0x00020000);
-  // ---- this wave's 2 x 32 weight rows: gate and up of the same columns, or 64 neighbours
-  __amdgpu_buffer_rsrc_t ws[2];
+  const int left = min(TM, pl.left);
+  // MI: 32-entry units
+  auto sweep = [&](auto mi_c) {
+    constexpr int MI = decltype(mi_c)::value;
+    typedef wide::Loop<LONG ? wide::FAR : wide::ALONG, wide::ORDERED, MI, false> L;
+    static_assert(L::LDS <= sizeof(lds));
+    L loop;
+    const int mine = 8 * MI * wid, row = a.order[pl.first + min(mine + lane, left - 1)] / a.div;  // this wave moves 8 MI of the rows
+    wide::each<MI>([&](auto i) {
+      const int r = __shfl(row, 8 * i.value + (lane >> 3), 64);
+      const uint32_t chunk = L::A::chunk(i.value, lane, wid);
+      if constexpr (LONG) loop.oa.src[i.value] = (const char*)a.x + (int64_t)r * K * 2 + chunk;
+      else loop.oa.src[i.value] = (uint32_t)r * K * 2 + chunk;
+    });
+    loop.oa.from = wide::buffer_of(a.x, a.xbytes);
+    loop.oa.step = 128;
+    const int last = N / 16 - 1;
+    wide::each<8>([&](auto i) {  // pieces: halves of blocks of 16 weight rows
+      const int b = (8 * wid + i.value) >> 1, column = pl.n0 / 16 + (GLU ? b >> 1 : b);
+      const int block = min(column, last) + (GLU && (b & 1) ? N / 16 : 0);
+      loop.ob.src[i.value] = (uint32_t)block * KQ * 2048 + 1024 * (i.value & 1) + 16 * lane;
+    });
+    const uint32_t wbytes = (uint32_t)(GLU ? 2 : 1) * N * K * 2;
+    loop.ob.from = wide::buffer_of((const bf16*)a.w + (int64_t)pl.e * (GLU ? 2 : 1) * N * K, wbytes);
+    loop.ob.step = 2048;
+    int entry[MI];  // of the results (asked for here, ahead of the loop: behind it each would wait for the stores before it)
+    const int first = (wid & 1) * 16 * MI + (lane & 15);
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int row = GLU ? min(n0 + 32 * wid, N - 32) + t * N : min(n0 + 64 * wid + 32 * t, N - 32);
-    ws[t] = __builtin_amdgcn_make_buffer_rsrc((bf16*)a.w + ((int64_t)e * (GLU ? 2 : 1) * N + row) * K, 0, 64 * K, 0x00020000);
-  }
-  const uint32_t wo = (uint32_t)(l32 >> 4) * KQ * 2048 + hh * 256 + (l32 & 15) * 16;
-  auto buffer = [&](auto b_c) -> lds_char* {
-    constexpr int b = decltype(b_c)::value & 3;
-    if constexpr (b == 0) return (lds_char*)b0;
-    else if constexpr (b == 1) return (lds_char*)b1;
-    else if constexpr (b == 2) return (lds_char*)b2;
-    else return (lds_char*)b3;
-  };
-  auto weights = [&](int kq, int i, int t) {
-    return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(ws[t], wo + (i >> 1) * 1024 + (i & 1) * 512,
-                                                                            min(kq, KQ - 1) * 2048, 0));
-  };
-  // ---- operand reads: entry 32 m + l32, columns 16 (2 j + hh) + 8 h .. + 7 of step (h, j) = (i / 2, i % 2)
-  uint32_t xa[4];
+    for (int m = 0; m < MI; ++m) entry[m] = a.order[pl.first + min(first + 16 * m, left - 1)];
+    loop.begin(lds, KQ, lane, wid);
+    loop.template tile<0>(KQ, loop.oa.from, loop.ob.from);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the surplus transfers)
+    // ---- lane: entry lane % 16 of a block of 16, columns 4 (lane / 16) .. + 3 of blocks of 16: those of two blocks change places between 16-lane rows
+    constexpr int NB = GLU ? 4 : 8;
+    const int g = lane >> 4, n0 = pl.n0 + (wid >> 1) * 16 * NB + 16 * (g & 1) + 8 * (g >> 1);
+    wide::each<MI>([&](auto m_c) {
+      constexpr int m = m_c.value;
+      const int r = first + 16 * m;
+      bf16* yr = (bf16*)a.y + (int64_t)entry[m] * N;
+      wide::each<NB / 2>([&](auto n_c) {
+        constexpr int n = 2 * n_c.value;
+        auto two = [&](auto b_c, int q) {  // columns 2 q and 2 q + 1 of the lane's four in block b
+          constexpr int b = decltype(b_c)::value;
+          f32x2 v;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int h = i >> 1, j = i & 1;
-    xa[i] = (uint32_t)(l32 * 128 + 16 * ((4 * j + 2 * hh + h) ^ ((l32 >> 1) & 7)));
-  }
-  auto rows = [&](auto b_c, int i, int m) { return *reinterpret_cast<const lds_bf16x8*>(buffer(b_c) + xa[i] + m * 4096); };
-
-  // MT: 32-entry tiles
-  auto sweep = [&](auto mt_c) {
-    constexpr int MT = decltype(mt_c)::value;
-    f32x16 acc[2][MT];
+          for (int i = 0; i < 2; ++i)
+            v[i] = GLU ? silu_mul(loop.acc[m][GLU ? 2 * b : b][2 * q + i], loop.acc[m][GLU ? 2 * b + 1 : b][2 * q + i]) : plain_act(loop.acc[m][b][2 * q + i], a.act);
+          return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+        };
+        u32x4 o;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[t][m][r] = 0.f;
-    // ---- rows on their way: MT pieces of 8 rows of 128 bytes per wave (16 bytes p of row r: columns 8 (p ^ (r / 2 % 8)) .. + 7)
-    const int mine = 8 * MT * wid, entry = a.order[pl.first + min(mine + lane, left - 1)];
-    std::conditional_t<LONG, const char*, uint32_t> xo[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const int r = i * 8 + (lane >> 3);
-      const int row = __shfl(entry / a.div, r, 64), piece = 8 * ((lane & 7) ^ (((mine + r) >> 1) & 7));
-      if constexpr (LONG) xo[i] = (const char*)a.x + ((int64_t)row * K + piece) * 2;
-      else xo[i] = ((uint32_t)row * K + piece) * 2;
-    }
-    if (lane < 8 * MT) ents[mine + lane] = entry;
-    // those of step kq that part p issues; past the end the last step again, into a buffer that nobody reads
-    auto move = [&](int kq, auto b_c, int p, int only) {
-#pragma unroll
-      for (int i = p * MT / 4; i < (p + 1) * MT / 4; ++i)
-        if (only < 0 || only == i - p * MT / 4) {
-          lds_char* to = buffer(b_c) + 128 * mine + 1024 * i;
-          if constexpr (LONG) dma16(xo[i] + min(kq, KQ - 1) * 128, to);
-          else dma16(xs, xo[i], min(kq, KQ - 1) * 128, to);
+        for (int q = 0; q < 2; ++q) {
+#ifdef __HIP_DEVICE_COMPILE__
+          const auto v = __builtin_amdgcn_permlane16_swap(two(Int<n>{}, q), two(Int<n + 1>{}, q), false, false);
+          o[q] = v[0];
+          o[2 + q] = v[1];
+#endif
         }
-    };
-    bf16x8 w[2][4][2], x[2][MT];
-    // (in the order of the loop, which waits by it)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) move(0, Int<0>{}, i, -1);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) move(1, Int<1>{}, i, -1);
-#pragma unroll
-    for (int i = 0; i < 7; ++i) {
-      if (i >= 3) move(2, Int<2>{}, i - 3, -1);
-#pragma unroll
-      for (int t = 0; t < 2; ++t) w[i >> 2][i & 3][t] = weights(i >> 2, i & 3, t);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    meet<2 * MT + 14>();
-#pragma unroll
-    for (int m = 0; m < MT; ++m) x[0][m] = rows(Int<0>{}, 0, m);
-    auto part = [&](int kq, auto s_c, auto i_c) {
-      constexpr int s = decltype(s_c)::value, i = decltype(i_c)::value, ni = (i + 1) & 3;
-      using Next = Int<i == 3 ? s + 1 : s>;
-      if constexpr (i == 3) {  // the next step has come, and nobody reads the one before this any more
-        meet<MT + 14 + 3 * MT / 4>();
-      }
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        x[(i + 1) & 1][m] = rows(Next{}, ni, m);
-#pragma unroll
-        for (int l = 0; l < 4; ++l) {
-          if (l * MT / 4 != m) continue;
-          if (l < 2) move(kq + 3, Int<s + 3>{}, i, l);
-          else if (i == 0) w[(s & 1) ^ 1][3][l - 2] = weights(kq + 1, 3, l - 2);
-          else w[s & 1][i ? i - 1 : 0][l - 2] = weights(kq + 2, i - 1, l - 2);
-        }
-        __builtin_amdgcn_sched_barrier(0x6);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-          acc[t][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[s & 1][i][t], x[i & 1][m], acc[t][m], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0x6);
-      }
-    };
-    auto step = [&](int kq, auto s_c) {
-      part(kq, s_c, Int<0>{});
-      part(kq, s_c, Int<1>{});
-      part(kq, s_c, Int<2>{});
-      part(kq, s_c, Int<3>{});
-    };
-    int kq = 0;
-    for (; kq + 4 <= KQ; kq += 4) {
-      step(kq, Int<0>{});
-      step(kq + 1, Int<1>{});
-      step(kq + 2, Int<2>{});
-      step(kq + 3, Int<3>{});
-    }
-    if (kq < KQ) {
-      step(kq, Int<0>{});
-      if (kq + 1 < KQ) {
-        step(kq + 1, Int<1>{});
-        if (kq + 2 < KQ) step(kq + 2, Int<2>{});
-      }
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    // lane: entry l of a tile, weight rows 8 q + 4 h + 0..3 (found anew: held over the loop they are spilled)
-    const int l = __lane_id() & 31, h = __lane_id() >> 5;
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const int r = 32 * m + l;
-      if (r >= left) continue;
-      bf16* yr = (bf16*)a.y + (int64_t)ents[r] * N;
-#pragma unroll
-      for (int t = 0; t < (GLU ? 1 : 2); ++t) {
-        const int n = n0 + (GLU ? 32 : 64) * wid + 32 * t;
-        if (n >= N) continue;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          bf16x4 o;
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            o[i] = (bf16)(GLU ? silu_mul(acc[0][m][4 * q + i], acc[1][m][4 * q + i]) : plain_act(acc[t][m][4 * q + i], a.act));
-          *reinterpret_cast<bf16x4*>(yr + n + 8 * q + 4 * h) = o;
-        }
-      }
-    }
+        if (r < left && n0 + 16 * n < N) *reinterpret_cast<u32x4*>(yr + n0 + 16 * n) = o;
+      });
+    });
   };
   const int tiles = (left + 63) / 64;
   if (tiles == 4) sweep(Int<8>{});
@@ -661,7 +535,7 @@ extern "C" int ds_expert_gemm(const void* x, const void* w, void* y, const int* 
     const int per = gated ? BN / 2 : BN;
     const int64_t grid = ((int64_t)entries / BM + E) * ((N + per - 1) / per);
     if (grid > INT32_MAX) return (int)hipErrorInvalidValue;
-    if (entries >= (int64_t)BIG_ROWS * E) return gated ? launch_big<true>(a, per, st) : launch_big<false>(a, per, st);
+    if (entries >= (int64_t)BIG_ROWS * E && (int64_t)(gated ? 2 : 1) * N * K * 2 <= UINT32_MAX) return gated ? launch_big<true>(a, per, st) : launch_big<false>(a, per, st);
     if (gated) hipLaunchKernelGGL(expert_tile_kernel<true>, dim3((unsigned)grid), dim3(256), 0, st, a);
     else hipLaunchKernelGGL(expert_tile_kernel<false>, dim3((unsigned)grid), dim3(256), 0, st, a);
     DS_CHECK_LAUNCH();
