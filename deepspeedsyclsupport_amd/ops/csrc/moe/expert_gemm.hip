@@ -381,7 +381,8 @@ __global__ void __launch_bounds__(256, 2) expert_tile_kernel(ExpertArgs a) {
 
 // ------------------------------------------------------------------------------------------------ hundreds of rows per expert
 // A tile of 256 entries by 256 weight rows (gated: 128 of either part, block by block in turn, so that a lane has gate and up of the same columns), with the
-// loop of gemm/wide_core.h: power bounds it there. Rows in units of 64 (MI): a short tile moves and multiplies no others. Workgroups walk groups of 8
+// loop of gemm/wide_core.h: power bounds it there. 32 experts, 1024 rows each on average, at random (all even), us with products of 32 x 32 x 16 and weights
+// straight into registers, and so: 3584 gated columns of 4096 1693 (1583), 1550 (1460); 4096 plain ones of 3584 867 (796), 769 (705). Rows in units of 64 (MI): a short tile moves and multiplies no others. Workgroups walk groups of 8
 // column tiles by all row tiles of an expert. Beyond 4 GB of rows (LONG) their transfers take an address of 64 bits a lane.
 constexpr int TM = 256, TN = 256;
 
@@ -495,13 +496,13 @@ __global__ void __launch_bounds__(256) expert_sum_kernel(const T* __restrict__ y
   }
 }
 
-// Rows per expert on average from which 256-row tiles pay: of 864 products of 128 to 1024 rows (12 sets of 8 to 256 experts, gated and plain, four
-// distributions of the rows) 717 are faster with them by more than 4 %, 91 slower. Their time by that of 128-row tiles, median and worst: shares at
-// random, 128 rows 0.78 and 1.16, 192 rows 0.84 and 0.99, 512 rows 0.82 and 1.24 (a last round of few tiles), 1024 rows 0.81 and 0.97. All even 1.01 and 1.16
-// with 128 rows, which fill the smaller tiles, 0.75 and 0.88 with 160. An eighth of the experts with 83 % of the rows 1.01 and 1.31 with 128, 1.10 and
-// 1.33 with 160, 1.08 and 1.48 with 192, 1.02 and 1.48 with 256, 0.89 and 1.07 with 320, 0.94 and 1.17 with 384: the host knows the
-// average alone. With 96 it goes either way (even shares, gated 32 of 1408 by 2048 1.18, 8 of 3584 by 4096 0.71). A choice on the device, one large tile or two small ones
-// per workgroup, lost more than it saved: two small ones behind one barrier take 1.25 times as long as in two workgroups.
+// Rows per expert on average from which 256-row tiles pay: of 664 products of 128 to 1024 rows (12 sets of 8 to 256 experts, gated and plain, four
+// distributions of the rows; profiles/expert_tiles_by_shares.csv) 560 are faster with them by more than 4 %, 51 slower. Their time by that of 128-row tiles,
+// median and worst: shares at random, 128 rows 0.74 and 0.95, 256 rows 0.85 and 1.10, 512 rows 0.78 and 1.16 (a last round of few tiles), 1024 rows 0.74 and
+// 0.93. All even 0.94 and 1.10 with 128 rows, which fill the smaller tiles, 0.77 and 0.90 with 160. An eighth of the experts with 83 % of the rows 0.94 and 1.21
+// with 128, 1.01 and 1.24 with 160, 1.01 and 1.42 with 192, 0.96 and 1.43 with 256, 0.86 and 1.06 with 384: the host knows the average alone. With 96 it
+// goes either way (even shares 0.99 and 1.17). A choice on the device, one large tile or two small ones per workgroup, lost more than it saved when both kernels
+// had one loop: two small ones behind one barrier took 1.25 times as long as in two workgroups.
 constexpr int BIG_ROWS = 128;
 
 template <bool GLU>
