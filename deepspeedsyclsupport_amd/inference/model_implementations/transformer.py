@@ -493,11 +493,10 @@ class DSInferenceLayer(ProjectionLayer):
     def _mlp(self, x):
         if self.spec.num_experts:
             return self._moe(x)
-        h = self._linear(x, "fc1_w", self.fc1_b)
-        if self.spec.gated_mlp:
-            h = DF.gated_activation(h, self.spec.act)
-        else:
-            h = DF.bias_activation(h, None, self.spec.act)
+        plain = self.spec.gated_mlp and self.fc1_b is None and "fc1_w" not in self.split_w and "fc1_w" not in self.quant
+        h = DF.linear_gated(x, self.fc1_w, self.spec.act) if plain else None
+        if h is None:
+            h = self._act(self._linear(x, "fc1_w", self.fc1_b))
         out = self._linear(h, "fc2_w")
         out = self._allreduce(out)
         if self.fc2_b is not None:

@@ -560,6 +560,21 @@ Tensor linear_weight_grad(Tensor go, Tensor x) {
   return c.defined() ? c : at::mm(go.t(), x);
 }
 
+// silu(x g^T) (x u^T) of x [.., I] and w [2 O, I], g before u: nothing where the product and the activation are launches of their own
+OptT linear_gated(Tensor x, Tensor w) {
+  if (!unwatched(x, w) || x.dim() < 2 || !x.is_contiguous() || w.dim() != 2 || !w.is_contiguous() || x.size(-1) != w.size(1) || w.size(0) % 16 || !x.numel())
+    return c10::nullopt;
+  auto sizes = x.sizes().vec();
+  sizes.back() = w.size(0) / 2;
+  const Tensor rows = x.view({-1, x.size(-1)});
+  int64_t M, N, K, lda, ldb;
+  if (!narrow_sizes(rows, w, true, true, M, N, K, lda, ldb) || !ds_wide_gemm_pays(M, N, K, 1, 1)) return c10::nullopt;
+  const c10::DeviceGuard guard(x.device());
+  Tensor y = torch::empty(sizes, x.options());
+  check(ds_wide_gated(x.const_data_ptr(), w.const_data_ptr(), y.data_ptr(), M, N / 2, K, lda, stream()), "linear_gated");
+  return y;
+}
+
 // Whether one of these two takes the tiles of 256 columns (else the caller may have copies along the inner dimension for the library's call)
 bool linear_grad_is_wide(Tensor go, Tensor b, bool weight_grad) {
   int64_t M, N, K, lda, ldb;
@@ -990,6 +1005,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_weight_grad", &linear_weight_grad);
   m.def("narrow_gemm_tune", [](int64_t tile, int64_t parts) { ds_narrow_gemm_tune((int)tile, (int)parts); });
   m.def("wide_gemm_tune", [](int64_t rows) { ds_wide_gemm_tune((int)rows); });
+  m.def("linear_gated", &linear_gated);
   m.def("linear_grad_is_wide", &linear_grad_is_wide);
   m.def("wide_gemm_pays", [](int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) { return ds_wide_gemm_pays(M, N, K, a_along, b_along) != 0; });
   m.def("transpose16", &transpose16, py::arg("x"), py::arg("pad_to") = 0);

@@ -1,5 +1,6 @@
 // bf16 products of a linear layer of many tokens: y = X W^T, dX = dY W and dW = dY^T X, each over the operands as they lie in memory, sums in fp32, one
-// rounding at the end. Tiles of 256, 192 or 128 rows by 256 columns, with the loop of wide_core.h.
+// rounding at the end. Tiles of 256, 192 or 128 rows by 256 columns, with the loop of wide_core.h. Of y, a gated activation's silu(gate) up as well, of two
+// neighbours' sums in registers: what a prompt's gate and up would be written and read for.
 #include "wide_core.h"
 
 #include <algorithm>
@@ -14,12 +15,14 @@ struct WideArgs {
   int M, N, K, ldc;
   uint32_t lda, ldb, abytes, bbytes;
   int band;           // row tiles that are walked together, column by column
+  int up;             // (gated) rows from the gate's part of b to the other
 };
 
-template <int AK, int BK, int MI>
+// GATE: b is [2 N, K], the gate's rows before the up part's; a tile has 128 of either, in blocks of 16 in turn
+template <int AK, int BK, int MI, bool GATE>
 __global__ void __launch_bounds__(256, 1) wide_gemm_kernel(WideArgs a) {
   typedef Loop<AK, BK, MI, true> L;
-  constexpr int TM = L::TM, TN = L::TN, NI = L::NI, STORES = MI * NI / 2;
+  constexpr int TM = L::TM, NB = GATE ? L::NI / 2 : L::NI, TN = 32 * NB, STORES = MI * NB / 2;  // NB: blocks of 16 columns that a wave writes
   __shared__ __attribute__((aligned(16))) char lds[L::LDS];
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int mt = (a.M + TM - 1) / TM, nt = (a.N + TN - 1) / TN, tiles = mt * nt;
@@ -41,6 +44,11 @@ __global__ void __launch_bounds__(256, 1) wide_gemm_kernel(WideArgs a) {
   loop.ob.from = L::B::tile(a.b, a.bbytes, a.ldb, n0);
   loop.oa.sources(a.lda, lane, wid);
   loop.ob.sources(a.ldb, lane, wid);
+  if constexpr (GATE)
+    each<L::PB>([&](auto i) {
+      const int r = L::B::row(i.value, lane, wid);
+      loop.ob.src[i.value] = (uint32_t)((r >> 5) * 16 + (r & 15) + (r & 16 ? a.up : 0)) * a.ldb * 2 + L::B::chunk(i.value, lane, wid);
+    });
   loop.begin(lds, steps, lane, wid);
   for (;;) {
     // the tile that follows, or this one's beginning again, for nobody
@@ -48,22 +56,32 @@ __global__ void __launch_bounds__(256, 1) wide_gemm_kernel(WideArgs a) {
     int m2 = m0, n2 = n0;
     if (!ends) place(id + stride, m2, n2);
     loop.template tile<STORES>(steps, L::A::tile(a.a, a.abytes, a.lda, m2), L::B::tile(a.b, a.bbytes, a.ldb, n2));
-    // ---- a lane has columns 4 (lane / 16) .. + 3 of blocks n and n + 1: 16-lane rows change places, and it has eight neighbours. What lies past C's
+    // ---- a lane has columns 4 (lane / 16) .. + 3 of every block: 16-lane rows change places, and it has eight neighbours. What lies past C's
     // rows or columns lies past the buffer's end: every wave stores as often as the next tile's barrier counts.
     // Past the caches (y, 6005 by [32000, 2048] 601 -> 556 us, 8192 by [22016, 4096] 998 -> 981): the next tile's second barrier waits for them.
     const auto c = __builtin_amdgcn_make_buffer_rsrc(a.c + (int64_t)m0 * a.ldc, 0, (int)((uint32_t)(min(TM, a.M - m0) - 1) * a.ldc * 2 + a.N * 2), 0x00020000);
-    const int row = (wid & 1) * 16 * MI + (lane & 15), col = n0 + (wid >> 1) * 16 * NI + 16 * ((lane >> 4) & 1) + 8 * (lane >> 5);
-    each<NI / 2>([&](auto n_c) {
+    const int row = (wid & 1) * 16 * MI + (lane & 15), col = n0 + (wid >> 1) * 16 * NB + 16 * ((lane >> 4) & 1) + 8 * (lane >> 5);
+    each<NB / 2>([&](auto n_c) {
       constexpr int n = 2 * n_c.value;
       uint32_t at = (uint32_t)row * a.ldc * 2 + (col + 16 * n < a.N ? 2 * (col + 16 * n) : 0xc0000000u);
       each<MI>([&](auto m_c) {
-        const f32x4 x = loop.acc[m_c.value][n], y = loop.acc[m_c.value][n + 1];
+        auto two = [&](auto b_c, int q) {  // columns 2 q and 2 q + 1 of the lane's four in block b
+          constexpr int b = decltype(b_c)::value, m = decltype(m_c)::value;
+          f32x2 v;
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            if constexpr (GATE) {
+              const float g = loop.acc[m][2 * b][2 * q + i];
+              v[i] = g / (1.f + __expf(-g)) * loop.acc[m][2 * b + 1][2 * q + i];
+            } else v[i] = loop.acc[m][b][2 * q + i];
+          }
+          return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+        };
         u32x4 o;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
 #ifdef __HIP_DEVICE_COMPILE__
-          const auto v = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x[2 * q], x[2 * q + 1]}, bf16x2)),
-                                                          __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{y[2 * q], y[2 * q + 1]}, bf16x2)), false, false);
+          const auto v = __builtin_amdgcn_permlane16_swap(two(Int<n>{}, q), two(Int<n + 1>{}, q), false, false);
           o[q] = v[0];
           o[2 + q] = v[1];
 #endif
@@ -121,19 +139,20 @@ Plan plan_of(int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
-int launch(WideArgs a, int rows, int a_along, int b_along, hipStream_t st) {
-  const int64_t mt = (a.M + rows - 1) / rows, nt = (a.N + 255) / 256;
+int launch(WideArgs a, int rows, int a_along, int b_along, bool gate, hipStream_t st) {
+  const int64_t mt = (a.M + rows - 1) / rows, nt = (a.N + (gate ? 127 : 255)) / (gate ? 128 : 256);
   a.band = (int)std::min<int64_t>(4, mt);
   const dim3 grid((unsigned)std::min<int64_t>(mt * nt, 256));
-#define GO(AK, BK)                                                                                            \
+#define GO(AK, BK, GATE)                                                                                      \
   do {                                                                                                        \
-    if (rows == 256) hipLaunchKernelGGL((wide_gemm_kernel<AK, BK, 8>), grid, dim3(256), 0, st, a);            \
-    else if (rows == 192) hipLaunchKernelGGL((wide_gemm_kernel<AK, BK, 6>), grid, dim3(256), 0, st, a);       \
-    else hipLaunchKernelGGL((wide_gemm_kernel<AK, BK, 4>), grid, dim3(256), 0, st, a);                        \
+    if (rows == 256) hipLaunchKernelGGL((wide_gemm_kernel<AK, BK, 8, GATE>), grid, dim3(256), 0, st, a);      \
+    else if (rows == 192) hipLaunchKernelGGL((wide_gemm_kernel<AK, BK, 6, GATE>), grid, dim3(256), 0, st, a); \
+    else hipLaunchKernelGGL((wide_gemm_kernel<AK, BK, 4, GATE>), grid, dim3(256), 0, st, a);                  \
   } while (0)
-  if (a_along && b_along) GO(ALONG, ALONG);
-  else if (a_along) GO(ALONG, ACROSS);
-  else GO(ACROSS, ACROSS);
+  if (gate) GO(ALONG, ALONG, true);
+  else if (a_along && b_along) GO(ALONG, ALONG, false);
+  else if (a_along) GO(ALONG, ACROSS, false);
+  else GO(ACROSS, ACROSS, false);
 #undef GO
   DS_CHECK_LAUNCH();
   return 0;
@@ -157,23 +176,36 @@ extern "C" int ds_wide_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along, i
   return 2e-6 * M * N * K >= plan_of(M, N, K).time * (b_along ? 1000 : a_along ? 950 : 800);
 }
 
+namespace {
+// gate: N weight rows, half of them the gate's, make N / 2 columns of C
+int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_along, int b_along, bool gate, hipStream_t st) {
+  const Plan p = plan_of(M, N, K);
+  const int64_t ar = a_along ? M : K, ac = a_along ? K : M, br = b_along ? N : K, bc = b_along ? K : N;
+  const int64_t of = gate ? 2 : 1, cols = N / of, cut = p.n < N ? p.n / of : cols;  // C's columns, those of the first part
+  WideArgs a{(const bf16*)A, (const bf16*)B, (bf16*)C, (int)p.m, (int)cut, (int)K, (int)cols, (uint32_t)lda, (uint32_t)ldb,
+             (uint32_t)(((ar - 1) * lda + ac) * 2), (uint32_t)(((br - 1) * ldb + bc) * 2), 0, (int)cols};
+  int rc = launch(a, p.rows, a_along, b_along, gate, st);
+  if (rc || (p.m == M && cut == cols)) return rc;
+  // the second part: rows of A and C from m on, or B's and C's columns from n on
+  const int64_t m = p.m < M ? p.m : 0, n = cut < cols ? cut : 0, oa = m * (a_along ? lda : 1), ob = n * (b_along ? ldb : 1);
+  a.a += oa;
+  a.b += ob;
+  a.c += m * cols + n;
+  a.M = (int)(M - m);
+  a.N = (int)(cols - n);
+  a.abytes -= (uint32_t)(oa * 2);
+  a.bbytes -= (uint32_t)(ob * 2);
+  return launch(a, p.other, a_along, b_along, gate, st);
+}
+}  // namespace
+
 // C [M, N] as ds_narrow_gemm takes it
 extern "C" int ds_wide_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_along, int b_along,
                             hipStream_t st) {
-  const Plan p = plan_of(M, N, K);
-  const int64_t ar = a_along ? M : K, ac = a_along ? K : M, br = b_along ? N : K, bc = b_along ? K : N;
-  WideArgs a{(const bf16*)A, (const bf16*)B, (bf16*)C, (int)p.m, (int)p.n, (int)K, (int)N, (uint32_t)lda, (uint32_t)ldb,
-             (uint32_t)(((ar - 1) * lda + ac) * 2), (uint32_t)(((br - 1) * ldb + bc) * 2), 0};
-  int rc = launch(a, p.rows, a_along, b_along, st);
-  if (rc || (p.m == M && p.n == N)) return rc;
-  // the second part: rows of A and C from m on, or B's and C's columns from n on
-  const int64_t m = p.m < M ? p.m : 0, n = p.n < N ? p.n : 0, oa = m * (a_along ? lda : 1), ob = n * (b_along ? ldb : 1);
-  a.a += oa;
-  a.b += ob;
-  a.c += m * N + n;
-  a.M = (int)(M - m);
-  a.N = (int)(N - n);
-  a.abytes -= (uint32_t)(oa * 2);
-  a.bbytes -= (uint32_t)(ob * 2);
-  return launch(a, p.other, a_along, b_along, st);
+  return run(A, B, C, M, N, K, lda, ldb, a_along, b_along, false, st);
+}
+
+// y [M, N] = silu(x g^T) (x u^T) of w [2 N, K], g before u; rows of x lda apart, of w K. Where ds_narrow_gemm_ok and ds_wide_gemm_pays have the product by w.
+extern "C" int ds_wide_gated(const void* X, const void* W, void* Y, int64_t M, int64_t N, int64_t K, int64_t lda, hipStream_t st) {
+  return run(X, W, Y, M, 2 * N, K, lda, K, 1, 1, true, st);
 }

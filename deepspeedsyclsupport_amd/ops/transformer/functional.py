@@ -153,6 +153,13 @@ def gated_activation(gate_up, act="silu"):
     return reference.ACTS[code](g) * u
 
 
+def linear_gated(x, weight, act="silu"):
+    """`gated_activation` of x weight^T in one launch, without a gradient of its own; None where product and activation are two."""
+    if ACT_CODES[act] != ACT_CODES["silu"] or not x.is_cuda or not weight.is_cuda or not unseen_from_python(x, weight):
+        return None
+    return hip_ops().linear_gated(x, weight)
+
+
 class _BiasActFn(torch.autograd.Function):
 
     @staticmethod

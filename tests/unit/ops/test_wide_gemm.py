@@ -100,3 +100,29 @@ def test_copies_of_gated_activations(I, copies):
     want = torch.autograd.grad((torch.nn.functional.silu(h[:, :I]) * h[:, I:]) @ w2f.t(), (xf, w1f, w2f), go.float())
     for g, r in zip(got, want):
         assert ((g.float() - r).norm() / r.norm()).item() < 1e-2
+
+
+@GPU
+@pytest.mark.parametrize("rows", [256, 192, 128, 0])
+@pytest.mark.parametrize("T,I,K", [(8, 8, 256), (200, 136, 320), (520, 392, 576), (2048, 2816, 1024), (4200, 1416, 256)])
+def test_gated_products(rows, T, I, K):
+    """silu of the first half of the columns times the others: what the two launches make, without the rounding between them."""
+    from deepspeedsyclsupport_amd.ops.transformer import functional as DF
+    x, w = _rnd(T, K, seed=1), _rnd(2 * I, K, seed=2) * 0.1
+    hip_ops().wide_gemm_tune(rows)
+    try:
+        got = DF.linear_gated(x, w)
+        assert (got is None) != hip_ops().wide_gemm_pays(T, 2 * I, K, True, True)
+        if got is None:
+            return
+        assert torch.equal(got, DF.linear_gated(x, w))
+        assert torch.equal(DF.linear_gated(x.view(2, T // 2, K), w), got.view(2, T // 2, I))
+    finally:
+        hip_ops().wide_gemm_tune(0)
+    g, u = (x.double() @ w.double().t()).split(I, -1)
+    size = x.double().abs() @ w.double().abs().t() * K * 2**-23   # (of the sums; the gate's slope is at most 1.1)
+    want = torch.nn.functional.silu(g) * u
+    bound = want.abs() * 2**-8 + 1.1 * size[:, :I] * u.abs() + size[:, I:] * g.abs() + 2**-20
+    assert ((got.double() - want).abs() <= bound).all()
+    with torch.enable_grad():
+        assert DF.linear_gated(x.requires_grad_(), w) is None
