@@ -8,7 +8,7 @@ transformer_block}.py` (fused attention and the fused LayerNorm / GEGLU / bias-a
 Here (diffusers itself is not required; modules are recognised by class name and attributes):
  * every `Attention` / `CrossAttention` module becomes `DSDiffusersAttention`: one fused QKV GEMM for self-attention
    (Q + fused KV GEMMs for cross-attention), the attention itself on the in-tree flash kernels — head dim 32/64 on
-   `csrc/attn/flash_small.hip` (any context length), 128 on `flash_fwd.hip` — and the output projection with its bias
+   `csrc/attn/flash_small.hip` (any context length), 128 on `flash_dense.hip` — and the output projection with its bias
    in the GEMM epilogue; VAE-style 4-D inputs (group norm, residual connection, output rescale) are handled;
  * every `BasicTransformerBlock` with LayerNorms becomes `DSDiffusersTransformerBlock`: LayerNorm kernels with the
    residual adds fused in, GEGLU on the gated-activation kernel (the projection's halves swapped once so the gate

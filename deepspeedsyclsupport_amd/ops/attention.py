@@ -1,8 +1,8 @@
 """Attention dispatch for training and prefill.
 
 On MI355X (bf16, head dim 128, no explicit mask / dropout) both passes run in-tree CDNA4 kernels:
- * forward `csrc/attn/flash_fwd.hip` (MFMA 32x32x16, swapped QK^T with in-register online softmax, transposed-LDS V
-   reads). Its output memory is laid out [B, S, H, D], so the caller's `o.transpose(1, 2).reshape(B, S, H*D)` is free;
+ * forward `csrc/attn/flash_dense.hip` (MFMA 16x16x32, swapped QK^T, exponentials beside the products of the neighbouring
+   halves of tiles). Its output memory is laid out [B, S, H, D], so the caller's `o.transpose(1, 2).reshape(B, S, H*D)` is free;
  * backward `csrc/attn/flash_bwd.hip`: one workgroup per 256 keys of one (batch, kv head) sweeping every query head
    of the GQA group (no repeat_interleave of K/V, no dK/dV reduction), P recomputed from the forward's LSE, dQ by
    f32 atomics. dq/dk/dv come back in the same [B, S, H, D] memory layout.

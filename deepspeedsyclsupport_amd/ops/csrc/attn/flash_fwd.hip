@@ -1,9 +1,6 @@
-// CDNA4 flash-attention forward (training / prefill), bf16, head dim 128.
+// Block-sparse attention forward for heads of 128, bf16, CDNA4 (gfx950). (Dense attention: flash_dense.hip.)
 //
-// Reference counterparts: the fused softmax-context path of `csrc/transformer/inference/csrc/pt_binding.cpp:434-557`,
-// the Triton `_flash_packed_kernel` (`ops/transformer/inference/triton/attention.py:253`) and the prebuilt
-// `flash_attn_by_atoms` of inference v2 (`inference/v2/kernels/ragged_ops/blocked_flash/blocked_flash.cpp:21-100`).
-// This is a gfx950 design, not a translation of any of them:
+// Reference counterpart: the Triton SDD / softmax / DSD kernels of `ops/sparse_attention`. Design:
 //
 //  * one workgroup = 4 waves = 128 query rows (32 per wave); K/V tiles of 64 keys are staged once per workgroup into
 //    LDS (double buffered, 2 x 32 KB) and shared by the 4 waves; 2 workgroups per CU (launch bounds 256 x 2);
@@ -13,22 +10,13 @@
 //    trip for P); V is consumed column-wise with the hardware transposed read `ds_read_b64_tr_b16`;
 //  * K and V share one LDS image (256-B rows, 16-B chunks XOR-swizzled by the row) that is conflict-free both for the
 //    row reads of K (`ds_read_b128`) and the transposed reads of V;
-//  * global->LDS staging is split (issue the next tile's loads before the current tile's MFMAs, write LDS after them),
-//    so HBM latency hides under the MFMA work; one barrier per tile;
-//    What bounds it: a tile's 32 products of a wave take a SIMD 1024 clocks, and the 32 KB that it reads of K and V for its
-//    32 rows take LDS as long, with eight waves of a CU; the exponentials 512 more where nothing else runs, at 1.7 GHz under
-//    this load. (Tried: reads further ahead; the products of the next keys and of the last ones between a tile's
-//    exponentials: the same time; 64 rows per wave, half the reads: one wave per SIMD, 28 spilled registers, 988 us.)
-//    B1 Hq32 Hkv8 S8192 causal 599 -> 589 us, B2 Hq32 S4096 341 -> 335, with the row maximum in short chains and no
-//    arithmetic for a rescale where no maximum moves;
-//  * causal: fully-masked tiles are skipped per wave, heavy query blocks are launched first, and the block->tile map
-//    keeps every (batch, head) on one XCD so its K/V stay in that XCD's L2.
-//  * block-sparse variant (SPARSE=true, reference `ops/sparse_attention` SDD/softmax/DSD Triton kernels): each
-//    workgroup walks only the 64-key tiles listed for its (layout head, 128-row query block) in a host-built plan, and
+//  * the next tile moves to LDS by DMA under the current tile's products; one barrier per tile;
+//  * each workgroup walks only the 64-key tiles listed for its (layout head, 128-row query block) in a host-built plan, and
 //    masks inside a tile by the 32 bits that the plan holds per tile (16 rows x 16 keys each) — compute and K/V traffic
-//    scale with the layout's density, not with S^2. Lists much longer than the average (the global rows of BigBird) are
-//    cut into parts that leave unnormalised rows in a workspace; a second launch merges them.
-//    What the sparse loop must not do is load from global memory: hipcc waits for its own loads with vmcnt(0), which
+//    scale with the layout's density, not with S^2; a wave whose rows see nothing of a tile skips it (the loop of flash_core.h,
+//    whose halves overlap from tile to tile, takes all tiles of all waves). Lists much longer than the average (the global rows
+//    of BigBird) are cut into parts that leave unnormalised rows in a workspace; a second launch merges them.
+//    What the loop must not do is load from global memory: hipcc waits for its own loads with vmcnt(0), which
 //    drains the tile transfer that was just issued, so that every tile paid a full trip to memory. The list and the
 //    masks come through scalar loads (address space 4), the per-key bias by LDS-DMA with its tile.
 //    B2 H8 S16384, BigBird of 64-key blocks with padding: 1572 -> 113 us (1150 tiles per head; uncut, one workgroup
@@ -46,8 +34,8 @@ constexpr int BM = 128;            // query rows per workgroup
 constexpr int BN = 64;             // keys per tile
 constexpr int NTHR = 256;
 constexpr int TILE_BYTES = BN * D * 2;     // 16 KB
-constexpr int LDS_BYTES = 4 * TILE_BYTES + 4 * 32 * 4;  // K0 K1 V0 V1 + per-wave row scratch
-constexpr int LDS_SPARSE = LDS_BYTES + 2 * BN * 4;      // + the per-key bias of two tiles
+constexpr int BIAS_AT = 4 * TILE_BYTES + 4 * 32 * 4;  // K0 K1 V0 V1 + per-wave row scratch
+constexpr int LDS_BYTES = BIAS_AT + 2 * BN * 4;      // + the per-key bias of two tiles
 
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -58,20 +46,10 @@ typedef __attribute__((address_space(3))) char lds_char;
 typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
 typedef __attribute__((address_space(3))) bf16x8_t lds_bf16x8;
 
-// LDS-DMA: every lane fetches 16 bytes from its own global address; they land at lds_base + 16 * lane. Issued from
-// inline asm on purpose: hipcc tracks its own global_load_lds builtins and then waits vmcnt(0) before every LDS read it
-// cannot prove disjoint from the DMA target, draining the prefetch. Out of its sight the DMA is ordered only by the
-// `s_waitcnt vmcnt(0)` + barrier at the end of each tile (see flash_bwd.hip for the same idiom).
-__device__ __forceinline__ void glds16(const void* g, const char* lds_base) {
-  const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_char*)lds_base);
-  uint32_t keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
-               "s_mov_b32 m0, %0"
-               : "=&s"(keep)
-               : "v"(g), "s"(dst)
-               : "memory");
-}
-// same with a wave-uniform 64-bit base (scalar registers) and a 32-bit per-lane byte offset
+// LDS-DMA: every lane fetches 16 bytes at a wave-uniform 64-bit base (scalar registers) plus its own 32-bit byte offset; they
+// land at lds_base + 16 * lane. Issued from inline asm on purpose: hipcc tracks its own global_load_lds builtins and then waits
+// vmcnt(0) before every LDS read it cannot prove disjoint from the DMA target, draining the prefetch. Out of its sight the DMA
+// is ordered only by the `s_waitcnt vmcnt(0)` + barrier at the end of each tile (see flash_bwd.hip for the same idiom).
 __device__ __forceinline__ void glds16_s(const char* base, uint32_t voff, const char* lds_base) {
   const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const lds_char*)lds_base);
   const uint64_t sb = (uint64_t)(uintptr_t)base;
@@ -117,7 +95,7 @@ __device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
   return r;
 }
 
-// block-sparse plan: tiles, masks [lay_heads, nqb, max_tiles] (64-key tile ids; bit 4 r + k of a mask: rows 16r.. of the
+// The plan: tiles, masks [lay_heads, nqb, max_tiles] (64-key tile ids; bit 4 r + k of a mask: rows 16r.. of the
 // query block see keys 16k.. of the tile), work [lay_heads, nwork, 4] = (query block or -1, first entry of its list, number of
 // entries, part slot or -1) longest first, merges [lay_heads, nmerge, 4] = (query block or -1, first slot, slots, 0)
 struct SparseLut {
@@ -140,10 +118,10 @@ typedef __attribute__((address_space(4))) const int const_int;
 __device__ __forceinline__ const_int* uniform_ints(const int* p) { return (const_int*)(uintptr_t)p; }
 
 // ROWB: biases per query row and key (the loop without them keeps its registers)
-template <bool CAUSAL, bool SPARSE, bool ROWB = false>
+template <bool ROWB>
 __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
     const bf16* __restrict__ Q, const bf16* __restrict__ K, const bf16* __restrict__ V, bf16* __restrict__ O,
-    float* __restrict__ LSE, int B, int Hq, int Hk, int S, int Skv, int64_t qsb, int64_t qsh, int64_t qss,
+    float* __restrict__ LSE, int B, int Hq, int Hk, int S, int64_t qsb, int64_t qsh, int64_t qss,
     int64_t ksb, int64_t ksh, int64_t kss, int64_t vsb, int64_t vsh, int64_t vss, int64_t osb, int64_t osh,
     int64_t oss, float c /* softmax scale * log2(e) */, float scale, SparseLut lut) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -151,30 +129,23 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
 
   // ------------------------------------------------------------------ block -> (batch, head, query block)
   const int nqb = (S + BM - 1) / BM;
-  const int nwg = gridDim.x;
-  const int logical = xcd_remap(blockIdx.x, nwg);
   // (batch, head)-major so one head's query blocks share an XCD's L2 (K/V tiles reused across its query blocks);
-  // within a head the heaviest query blocks go first (causal: the longest rows; sparse: the LUT's order by tile
-  // count, so global-attention rows do not start last). Measured: query-block-major heavy-first order loses more
-  // to L2 misses than it gains in tail length (tools/bench_sparse_attn.py).
-  const int per_bh = SPARSE ? lut.nwork : nqb;
-  int bh = logical / per_bh, qbi = logical % per_bh;
-  if (SPARSE && B * Hq % 8 == 0) {  // an XCD takes the longest lists of all its heads first
+  // within a head the plan's order, longest lists first
+  int bh, at_work;
+  if (B * Hq % 8 == 0) {  // an XCD takes the longest lists of all its heads first
     const int per = B * Hq / 8, at = blockIdx.x / 8;
     bh = blockIdx.x % 8 * per + at % per;
-    qbi = at / per;
+    at_work = at / per;
+  } else {
+    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    bh = logical / lut.nwork;
+    at_work = logical % lut.nwork;
   }
   const int b = bh / Hq, hq = bh % Hq, hk = hq / (Hq / Hk);
-  const int lh = SPARSE ? (lut.lay_heads == 1 ? 0 : hq) : 0;
-  int qb = CAUSAL ? nqb - 1 - qbi : qbi, first = 0, count = 0, slot = -1;  // heaviest first
-  if constexpr (SPARSE) {
-    const_int* wk = uniform_ints(lut.work) + ((int64_t)lh * lut.nwork + qbi) * 4;
-    qb = wk[0];
-    first = wk[1];
-    count = wk[2];
-    slot = wk[3];
-    if (qb < 0) return;  // (heads with fewer parts than the others)
-  }
+  const int lh = lut.lay_heads == 1 ? 0 : hq;
+  const_int* wk = uniform_ints(lut.work) + ((int64_t)lh * lut.nwork + at_work) * 4;
+  const int qb = wk[0], first = wk[1], nt = wk[2], slot = wk[3];
+  if (qb < 0) return;  // (heads with fewer parts than the others)
   const int q0 = qb * BM, q0w = q0 + wid * 32;
 
   const bf16* Qp = Q + b * qsb + hq * qsh;
@@ -190,20 +161,11 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
     for (int kk = 0; kk < 8; ++kk) qf[kk] = *reinterpret_cast<const bf16x8_t*>(qrow + 16 * kk);
   }
 
-  int nt = (Skv + BN - 1) / BN;
-  if (CAUSAL) nt = min(nt, (q0 + BM + BN - 1) / BN);
-  const_int* tlist = nullptr;
-  const_int* mlist = nullptr;
-  const float* kbp = nullptr;
-  if constexpr (SPARSE) {
-    nt = count;
-    tlist = uniform_ints(lut.tiles) + ((int64_t)lh * nqb + qb) * lut.max_tiles + first;
-    mlist = uniform_ints(lut.masks) + ((int64_t)lh * nqb + qb) * lut.max_tiles + first;
-    if (lut.kbias != nullptr) kbp = lut.kbias + (int64_t)b * lut.kb_stride;
-  }
-  auto tile_of = [&](int j) { return SPARSE ? tlist[j] : j; };
+  const_int* tlist = uniform_ints(lut.tiles) + ((int64_t)lh * nqb + qb) * lut.max_tiles + first;
+  const_int* mlist = uniform_ints(lut.masks) + ((int64_t)lh * nqb + qb) * lut.max_tiles + first;
+  const float* kbp = lut.kbias != nullptr ? lut.kbias + (int64_t)b * lut.kb_stride : nullptr;
 
-  // LDS: [K0][K1][V0][V1][scratch][SPARSE: bias0 bias1]
+  // LDS: [K0][K1][V0][V1][scratch][bias0 bias1]
   float* scratch = reinterpret_cast<float*>(smem + 4 * TILE_BYTES) + wid * 32;
   const lds_char* s3 = (const lds_char*)smem;  // 32-bit LDS addressing: per-lane base + compile-time displacement
 
@@ -213,31 +175,19 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
   // MFMAs of tile j. Lane L of piece p lands at physical chunk L%16 of row 4p + L/16, so it fetches the logical
   // chunk (L%16) ^ swizzle(row) — the image's XOR swizzle goes on the SOURCE address. The row's low four bits
   // (4w + L/16) do not depend on the piece, so one 32-bit byte offset per lane serves all pieces of all tiles; the
-  // tile / piece part of the address is wave-uniform (scalar base). Only a ragged last tile builds clamped
-  // per-lane addresses.
+  // tile / piece part of the address is wave-uniform (scalar base).
   const int drow = 4 * wid + (lane >> 4);
   const int dch = (lane & 15) ^ (((drow & 3) << 2) | ((drow >> 2) & 3));
   const uint32_t kdma = (uint32_t)((drow * kss + dch * 8) * 2);
   const uint32_t vdma = (uint32_t)((drow * vss + dch * 8) * 2);
   auto dma_tile = [&](int tile, int buf) {
-    if constexpr (SPARSE) {
-      if (kbp != nullptr && wid == 0) glds4(kbp + tile * BN + lane, smem + LDS_BYTES + buf * BN * 4);
-    }
-    if (tile * BN + BN <= Skv) {
-      const char* kb = reinterpret_cast<const char*>(Kp + (int64_t)tile * BN * kss);
-      const char* vb = reinterpret_cast<const char*>(Vp + (int64_t)tile * BN * vss);
+    if (kbp != nullptr && wid == 0) glds4(kbp + tile * BN + lane, smem + BIAS_AT + buf * BN * 4);
+    const char* kb = reinterpret_cast<const char*>(Kp + (int64_t)tile * BN * kss);
+    const char* vb = reinterpret_cast<const char*>(Vp + (int64_t)tile * BN * vss);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        glds16_s(kb + (int64_t)32 * i * kss, kdma, smem + buf * TILE_BYTES + 1024 * (wid + 4 * i));
-        glds16_s(vb + (int64_t)32 * i * vss, vdma, smem + (2 + buf) * TILE_BYTES + 1024 * (wid + 4 * i));
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int key = min(tile * BN + 16 * i + drow, Skv - 1);
-        glds16(Kp + (int64_t)key * kss + dch * 8, smem + buf * TILE_BYTES + 1024 * (wid + 4 * i));
-        glds16(Vp + (int64_t)key * vss + dch * 8, smem + (2 + buf) * TILE_BYTES + 1024 * (wid + 4 * i));
-      }
+    for (int i = 0; i < 4; ++i) {
+      glds16_s(kb + (int64_t)32 * i * kss, kdma, smem + buf * TILE_BYTES + 1024 * (wid + 4 * i));
+      glds16_s(vb + (int64_t)32 * i * vss, vdma, smem + (2 + buf) * TILE_BYTES + 1024 * (wid + 4 * i));
     }
   };
   // every wave: its own DMA pieces have landed (vmcnt) and its LDS reads are done (lgkmcnt), then the barrier
@@ -274,7 +224,7 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
 
   // the Q fragments are the only loads hipcc tracks: retired after the first DMA is on its way and before the loop, so that its
   // own counted waits never have to look past transfers it does not know about
-  if (nt > 0) dma_tile(tile_of(0), 0);  // uniform per workgroup (a sparse row block may have no tiles)
+  if (nt > 0) dma_tile(tlist[0], 0);  // uniform per workgroup (a sparse row block may have no tiles)
 #pragma unroll
   for (int kk = 0; kk < 8; ++kk) asm volatile("" : : "v"(qf[kk]));
   tile_barrier();
@@ -282,12 +232,11 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
   // one tile; `cur` (the LDS buffer) is a compile-time constant so it folds into the displacements
   auto tile_step = [&](int j, auto cur_c) {
     constexpr int cur = decltype(cur_c)::value;
-    if (j + 1 < nt) dma_tile(tile_of(j + 1), cur ^ 1);
-    const int k0 = tile_of(j) * BN;
-    // SPARSE: this wave's 8 bits of the tile's mask
-    const unsigned seen = SPARSE ? ((unsigned)mlist[j] >> (8 * __builtin_amdgcn_readfirstlane(wid))) & 0xffu : 0xffu;
-    const bool active = (!CAUSAL || k0 <= q0w + 31) && seen != 0;
-    if (active) {
+    if (j + 1 < nt) dma_tile(tlist[j + 1], cur ^ 1);
+    const int k0 = tlist[j] * BN;
+    // this wave's 8 bits of the tile's mask
+    const unsigned seen = ((unsigned)mlist[j] >> (8 * __builtin_amdgcn_readfirstlane(wid))) & 0xffu;
+    if (seen != 0) {
       // ---------------- S^T = K . Q^T  (two 32-key halves), K fragments read three MFMAs ahead: left to itself
       // hipcc issued each ds_read right before its MFMA and waited lgkmcnt(0) in between, so every MFMA paid a
       // full LDS round trip. The order is pinned with sched_barrier (VALU and SALU may cross, MFMA / LDS may not).
@@ -328,54 +277,41 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
       bf16x8_t v0f = ldv(0), v1f = ldv(1);
       // ---------------- additive biases (key padding / attention mask / relative position), in raw score units
       // (bias / scale), then the block-sparse mask: 16 x 16 per bit, eight registers of a lane share one
-      if constexpr (SPARSE) {
-        if (kbp != nullptr) {
-          const float inv_scale = 1.f / scale;
-          const float* kbl = reinterpret_cast<const float*>(smem + LDS_BYTES + cur * BN * 4);
-#pragma unroll
-          for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {  // four consecutive keys: registers 4g .. 4g+3
-              const f32x4 bv = *reinterpret_cast<const f32x4*>(kbl + t * 32 + 8 * g + 4 * h);
-#pragma unroll
-              for (int i = 0; i < 4; ++i) s[t][4 * g + i] = fmaf(bv[i], inv_scale, s[t][4 * g + i]);
-            }
-        }
-        if constexpr (ROWB) {
-          const float inv_scale = 1.f / scale;
-          const float* abp = lut.abias ? lut.abias + (int64_t)qrow_lane * lut.ab_stride : nullptr;
-          const float* rpp = lut.rpe ? lut.rpe + (int64_t)hq * lut.rpe_hs + (int64_t)qrow_lane * lut.rpe_rs : nullptr;
-#pragma unroll
-          for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              const int key = k0 + t * 32 + 8 * g + 4 * h;
-              f32x4 bsum = {0.f, 0.f, 0.f, 0.f};
-              if (abp) bsum += *reinterpret_cast<const f32x4*>(abp + key);
-              if (rpp) bsum += *reinterpret_cast<const f32x4*>(rpp + key);
-#pragma unroll
-              for (int i = 0; i < 4; ++i) s[t][4 * g + i] = fmaf(bsum[i], inv_scale, s[t][4 * g + i]);
-            }
-        }
-        if (seen != 0xffu) {
-          const unsigned mine = seen >> (4 * (l32 >> 4));
-#pragma unroll
-          for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-              if (!((mine >> (2 * t + (r >> 3))) & 1u)) s[t][r] = -INFINITY;
-        }
-      }
-      // ---------------- masking (causal diagonal / ragged key tail)
-      const bool need_mask = !SPARSE && ((CAUSAL && k0 + BN - 1 > q0w) || (k0 + BN > Skv));
-      if (need_mask) {
+      if (kbp != nullptr) {
+        const float inv_scale = 1.f / scale;
+        const float* kbl = reinterpret_cast<const float*>(smem + BIAS_AT + cur * BN * 4);
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = k0 + t * 32 + (r & 3) + 8 * (r >> 2) + 4 * h;
-            if (key >= Skv || (CAUSAL && key > qrow_lane)) s[t][r] = -INFINITY;
+          for (int g = 0; g < 4; ++g) {  // four consecutive keys: registers 4g .. 4g+3
+            const f32x4 bv = *reinterpret_cast<const f32x4*>(kbl + t * 32 + 8 * g + 4 * h);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[t][4 * g + i] = fmaf(bv[i], inv_scale, s[t][4 * g + i]);
           }
+      }
+      if constexpr (ROWB) {
+        const float inv_scale = 1.f / scale;
+        const float* abp = lut.abias ? lut.abias + (int64_t)qrow_lane * lut.ab_stride : nullptr;
+        const float* rpp = lut.rpe ? lut.rpe + (int64_t)hq * lut.rpe_hs + (int64_t)qrow_lane * lut.rpe_rs : nullptr;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const int key = k0 + t * 32 + 8 * g + 4 * h;
+            f32x4 bsum = {0.f, 0.f, 0.f, 0.f};
+            if (abp) bsum += *reinterpret_cast<const f32x4*>(abp + key);
+            if (rpp) bsum += *reinterpret_cast<const f32x4*>(rpp + key);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[t][4 * g + i] = fmaf(bsum[i], inv_scale, s[t][4 * g + i]);
+          }
+      }
+      if (seen != 0xffu) {
+        const unsigned mine = seen >> (4 * (l32 >> 4));
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (!((mine >> (2 * t + (r >> 3))) & 1u)) s[t][r] = -INFINITY;
       }
       // ---------------- online softmax (row = this lane's query; partner lane^32 holds the other 32 keys)
       // row max: one v_max3 per register pair (fmaxf on MFMA outputs makes hipcc canonicalise every input first), in four
@@ -458,21 +394,19 @@ __global__ void __launch_bounds__(NTHR, 2) flash_fwd_kernel(
 
   // ------------------------------------------------------------------ epilogue: O / l, LSE
   const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
-  if constexpr (SPARSE) {
-    if (slot >= 0) {  // a part of the list: rows as they are, maximum and sum
-      const int64_t at = (int64_t)(lut.lay_heads == 1 ? bh : b) * lut.nslots + slot;
-      float* po = lut.part_o + at * BM * D;
+  if (slot >= 0) {  // a part of the list: rows as they are, maximum and sum
+    const int64_t at = (int64_t)(lut.lay_heads == 1 ? bh : b) * lut.nslots + slot;
+    float* po = lut.part_o + at * BM * D;
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
+    for (int r = 0; r < 16; ++r)
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-          po[(wid * 32 + (r & 3) + 8 * (r >> 2) + 4 * h) * D + dt * 32 + l32] = o[dt][r];
-      if (lane < 32) {
-        lut.part_ml[at * 2 * BM + wid * 32 + l32] = m_run;
-        lut.part_ml[at * 2 * BM + BM + wid * 32 + l32] = l_tot;
-      }
-      return;
+      for (int dt = 0; dt < 4; ++dt)
+        po[(wid * 32 + (r & 3) + 8 * (r >> 2) + 4 * h) * D + dt * 32 + l32] = o[dt][r];
+    if (lane < 32) {
+      lut.part_ml[at * 2 * BM + wid * 32 + l32] = m_run;
+      lut.part_ml[at * 2 * BM + BM + wid * 32 + l32] = l_tot;
     }
+    return;
   }
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (lane < 32) scratch[lane] = inv;
@@ -542,25 +476,22 @@ __global__ void __launch_bounds__(256) flash_merge_kernel(bf16* __restrict__ O, 
     LSE[((int64_t)b * Hq + hq) * S + q] = l > 0.f ? (m * c + __log2f(l)) * 0.69314718055994531f : INFINITY;
 }
 
-template <bool C, bool SP, bool RB = false>
-int launch(const bf16* q, const bf16* k, const bf16* v, bf16* o, float* lse, int B, int Hq, int Hk, int S, int Skv,
+template <bool ROWB>
+int launch(const bf16* q, const bf16* k, const bf16* v, bf16* o, float* lse, int B, int Hq, int Hk, int S,
            const int64_t* qs, const int64_t* ks, const int64_t* vs, const int64_t* os, float scale, hipStream_t st,
-           const SparseLut& lut = SparseLut{}) {
-  constexpr int LDS = SP ? LDS_SPARSE : LDS_BYTES;
+           const SparseLut& lut) {
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_fwd_kernel<C, SP, RB>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_fwd_kernel<ROWB>),
+                        hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
     attr = true;
   }
-  const int nqb = (S + BM - 1) / BM;
-  const int grid = (SP ? lut.nwork : nqb) * B * Hq;
   const float c = scale * 1.4426950408889634f;
-  hipLaunchKernelGGL((flash_fwd_kernel<C, SP, RB>), dim3(grid), dim3(NTHR), LDS, st, q, k, v, o, lse, B, Hq, Hk, S,
-                     Skv, qs[0], qs[1], qs[2], ks[0], ks[1], ks[2], vs[0], vs[1], vs[2], os[0], os[1], os[2], c, scale,
+  hipLaunchKernelGGL(flash_fwd_kernel<ROWB>, dim3(lut.nwork * B * Hq), dim3(NTHR), LDS_BYTES, st, q, k, v, o, lse, B, Hq, Hk, S,
+                     qs[0], qs[1], qs[2], ks[0], ks[1], ks[2], vs[0], vs[1], vs[2], os[0], os[1], os[2], c, scale,
                      lut);
   DS_CHECK_LAUNCH();
-  if (SP && lut.nmerge > 0) {
+  if (lut.nmerge > 0) {
     hipLaunchKernelGGL(flash_merge_kernel, dim3(lut.nmerge * 4, B * Hq), dim3(256), 0, st, o, lse, lut, Hq, S, os[0], os[1],
                        os[2], c);
     DS_CHECK_LAUNCH();
@@ -569,20 +500,6 @@ int launch(const bf16* q, const bf16* k, const bf16* v, bf16* o, float* lse, int
 }
 
 }  // namespace
-
-// q [B,Hq,S,128], k/v [B,Hk,Skv,128] (bf16, unit last stride, any outer strides), o [B,Hq,S,128] (any outer strides),
-// lse [B,Hq,S] fp32 (optional). strides are (batch, head, seq) in elements. Top-left causal alignment (SDPA's).
-extern "C" int ds_flash_fwd(const void* q, const void* k, const void* v, void* o, float* lse, int B, int Hq, int Hk,
-                            int S, int Skv, const int64_t* qs, const int64_t* ks, const int64_t* vs,
-                            const int64_t* os, float scale, int causal, hipStream_t st) {
-  if (Hk <= 0 || Hq % Hk != 0 || S <= 0 || Skv <= 0) return (int)hipErrorInvalidValue;
-  auto q_ = (const bf16*)q;
-  auto k_ = (const bf16*)k;
-  auto v_ = (const bf16*)v;
-  auto o_ = (bf16*)o;
-  return causal ? launch<true, false>(q_, k_, v_, o_, lse, B, Hq, Hk, S, Skv, qs, ks, vs, os, scale, st)
-                : launch<false, false>(q_, k_, v_, o_, lse, B, Hq, Hk, S, Skv, qs, ks, vs, os, scale, st);
-}
 
 // Block-sparse forward: same tensors as ds_flash_fwd (non-causal; causality, if wanted, is part of the layout) plus
 // the plan described at SparseLut. lay_heads is 1 (shared layout) or Hq. Requires S == Skv, a multiple of 128. The merges'
@@ -604,6 +521,6 @@ extern "C" int ds_flash_fwd_sparse(const void* q, const void* k, const void* v, 
   if (!al(kbias, kb_stride) || !al(abias, ab_stride) || !al(rpe, rpe_rs) || rpe_hs % 4) return (int)hipErrorInvalidValue;
   const SparseLut lut{tiles, masks, work, merges, part_o, part_ml, max_tiles, lay_heads, nwork, nmerge, nslots,
                       kbias, abias, rpe, kb_stride, ab_stride, rpe_hs, rpe_rs};
-  auto run = abias != nullptr || rpe != nullptr ? launch<false, true, true> : launch<false, true>;
-  return run((const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)o, lse, B, Hq, Hk, S, S, qs, ks, vs, os, scale, st, lut);
+  auto run = abias != nullptr || rpe != nullptr ? launch<true> : launch<false>;
+  return run((const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)o, lse, B, Hq, Hk, S, qs, ks, vs, os, scale, st, lut);
 }

@@ -9,7 +9,7 @@
 //    output is rescaled only when the maximum has moved by more than 2^8;
 //  * workgroups go head by head, heaviest query blocks first. Block by block, as the other kernel has it, an XCD got all heads
 //    of a run of neighbouring query blocks: the last XCD did 15 / 8 of the mean work while the first was idle.
-// 1 x 8192 causal, 32 query heads over 8: 1545 -> 664 us (828 TFLOP/s); 4 x 2048, chunks of 2048, two-term weights, sink: 540 ->
+// 1 x 8192 causal, 32 query heads over 8: 1545 -> 587 us (paged_rows.h now: 546); 4 x 2048, chunks of 2048, two-term weights, sink: 540 ->
 // 265 us.
 #pragma once
 #include <type_traits>

@@ -1,6 +1,7 @@
 // Ragged paged flash attention for inference prefill / prompt chunks (SplitFuse): entry points. The kernels are in
-// paged_flash.h (heads of 128) and paged_prefill_core.h (other widths and page sizes).
+// paged_rows.h and paged_flash.h (heads of 128, without and with what the first leaves out) and paged_prefill_core.h (other widths and page sizes).
 #include "paged_flash.h"
+#include "paged_rows.h"
 
 // q / o [T, Hq, D] bf16 (contiguous), caches [blocks, Hk, BS, D] bf16, D in {64, 80, 96, 128, 256}, block_table
 // [nseq, max_blocks] int32, start [nseq], cu_q [nseq + 1], work [nwork, 2] (sequence, 128-row query block) int32,
@@ -14,7 +15,7 @@ extern "C" int ds_paged_prefill(const void* q, const void* kc, const void* vc, v
   PagedArgs a{(const bf16*)q, (const bf16*)kc, (const bf16*)vc, (bf16*)o, block_table, start, cu_q, work, alibi,
               Hq, Hk, BS, max_blocks, window, scale * 1.4426950408889634f, 1.f / scale, D, D, 0, nullptr, nullptr, 0, 0, 0, 0, 0, nullptr, (int64_t)Hq * D,
               (int64_t)Hq * D, nullptr, 0, 0.f, 0.f};
-  if (paged_flash_fits(a)) return launch_flash<PLAIN>(a, nwork, st);
+  if (paged_flash_fits(a)) return paged_rows_fits(a) && paged_rows_pays(a, nwork) ? launch_rows(a, nwork, st) : launch_flash<PLAIN>(a, nwork, st);
   switch (D) {
     case 64: return launch<64, 64, PLAIN>(a, nwork, st);
     case 80: return launch<80, 80, PLAIN>(a, nwork, st);

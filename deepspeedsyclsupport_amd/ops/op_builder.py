@@ -44,6 +44,7 @@ EXTENSIONS = {
             "xent/xent_kernels.hip",
             "attn/decode_attn.hip",
             "attn/flash_fwd.hip",
+            "attn/flash_dense.hip",
             "attn/flash_bwd.hip",
             "attn/sparse_bwd.hip",
             "attn/paged_prefill.hip",

@@ -1,7 +1,7 @@
 """Block-sparse attention on the gfx950 flash kernel (reference: the Triton SDD / softmax / DSD kernels of
 `ops/sparse_attention/{matmul.py:628, softmax.py:224}` driven by `sparse_self_attention.py`).
 
-Forward: `csrc/attn/flash_fwd.hip` in its SPARSE instantiation — every workgroup (one 128-row query block of one
+Forward: `csrc/attn/flash_fwd.hip` — every workgroup (one 128-row query block of one
 head) visits only the 64-key tiles its layout rows touch, listed in a LUT built here once per (layout, sequence
 length), and masks inside a tile by 16 x 16 pieces. Work and K/V traffic therefore scale with the
 layout density. Head dims below 128 are zero-padded to 128 (zeros change neither QK^T nor the kept part of PV).

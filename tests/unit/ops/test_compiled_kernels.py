@@ -129,3 +129,59 @@ def test_sums_keep_their_registers(source, tmp_path):
     """hipcc 7.2 has put a step's addresses into registers of a product's sums here."""
     text = _assembly(source, tmp_path / "kernels.s")
     assert text.count("v_mfma") > 100 and not _overwritten_sums(text)
+
+
+def _agprs(operand):
+    m = re.fullmatch(r"a(\d+)|a\[(\d+):(\d+)\]", operand.strip())
+    if m is None:
+        return set()
+    return {int(m[1])} if m[1] else set(range(int(m[2]), int(m[3]) + 1))
+
+
+def _moved_sums(text, after=16, before=2):
+    """Accumulators that something other than a product reads fewer than `after` wait states behind the product that wrote them, or that a product
+    takes fewer than `before` behind another's write."""
+    found, now, product, other = [], 0, {}, {}
+    for op, operands in _lines(text):
+        if _is_label(op, operands):
+            if not op.startswith(".L"):
+                product, other = {}, {}
+            continue
+        now += 1 + int(operands[0]) if op == "s_nop" else 1
+        if op.startswith("v_mfma"):
+            if any(now - other.get(r, -99) <= before for x in operands[1:] for r in _agprs(x)):
+                found.append((op, operands))
+            product.update({r: now for r in _agprs(operands[0])})
+        elif op.startswith(("v_accvgpr", "scratch_store", "buffer_store", "global_store")):
+            read = operands[1:] if op.startswith("v_accvgpr") else operands
+            if any(now - product.get(r, -99) <= after for x in read for r in _agprs(x)):
+                found.append((op, operands))
+            if op.startswith("v_accvgpr"):
+                if any(now - product.get(r, -99) <= after for r in _agprs(operands[0])):
+                    found.append((op, operands))
+                other.update({r: now for r in _agprs(operands[0])})
+    return found
+
+
+def test_the_scan_finds_a_moved_sum():
+    product, read, write = "v_mfma_f32_16x16x32_bf16 a[0:3], v[8:11], v[12:15], a[0:3]", "v_accvgpr_read_b32 v2, a3", "v_accvgpr_write_b32 a2, v3"
+    assert _moved_sums(f"{product}\n{read}") and _moved_sums(f"{product}\n\ts_nop 7\n{read}") and _moved_sums(f"{write}\n{product}")
+    assert _moved_sums(f"{product}\nv_accvgpr_mov_b32 a9, a0") and _moved_sums(f"{product}\n{write}")
+    assert not _moved_sums(f"{product}\n\ts_nop 15\n\ts_nop 7\n{read}") and not _moved_sums(f"{write}\n\ts_nop 1\n{product}")
+
+
+@pytest.mark.skipif(not op_builder.toolchain_available(), reason="needs hipcc")
+@pytest.mark.parametrize("source,kernel", [("gemm/wide_gemm.hip", "wide_gemm_kernel"), ("moe/expert_gemm.hip", "expert_big_kernel")])
+def test_sums_of_products_in_assembly_stay(source, kernel, tmp_path):
+    """The loop of the wide products has them in inline assembly, whose waits hipcc does not know: it must not move, spill or read a sum near one."""
+    parts = re.split(r"\n(?=_Z\w+:)", _assembly(source, tmp_path / "kernels.s"))
+    text = "\n".join(p.split(".Lfunc_end")[0] for p in parts if kernel in p.split(":")[0])
+    assert text.count("v_mfma_f32_16x16x32_bf16 a[") > 1000 and not _moved_sums(text) and not _early_swaps(text)
+    assert "scratch_" not in text
+
+
+@pytest.mark.skipif(not op_builder.toolchain_available(), reason="needs hipcc")
+@pytest.mark.parametrize("source", ["attn/flash_dense.hip", "attn/paged_prefill.hip"])
+def test_swaps_of_results_wait_for_their_operands(source, tmp_path):
+    text = _assembly(source, tmp_path / "kernels.s")
+    assert "v_permlane16_swap" in text and not _early_swaps(text)
