@@ -27,7 +27,9 @@
 //    tile so hipcc does not hoist ~40 derived addresses into registers (2 waves per SIMD leave 256 per lane);
 //  * causal: waves whose 32 keys lie entirely above a tile skip it, the dQ product stops at the diagonal, workgroups
 //    with the most tiles (low key blocks) start first, and each (batch, kv head)'s key blocks share an XCD (Q / dO
-//    reuse in L2);
+//    reuse in L2). Where they do not all run at once, the first blocks of all heads go first: head by head, the last heads' long sweeps
+//    began when the rest was nearly done (us: 2 x 4096, 32 heads 1118, 1036; 1 x 4096, 20 heads 437, 405; 4 x 8192 heads, all at
+//    once, 341 as it is and 361 round the chip);
 //  * too few sweeps to fill the chip (short sequences of grouped-query models) are cut into parts that leave fp32 dK / dV in a
 //    workspace; a second launch adds them up in a fixed order. B3 Hq16 Hk4 S1000 causal (48 workgroups uncut): 313 -> 103 us.
 // Measured (tools/bench_flash_bwd.py, profiles/flash_bwd_bench_r2_final.jsonl): B8 H32 S4096 D128 causal 4.2-4.3 ms
@@ -152,9 +154,14 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
             l32 = lane & 31;
   const int S = a.S;
   const int nkb = (S + KB - 1) / KB;
-  const int logical = xcd_remap(blockIdx.x, gridDim.x);
   const int per_bh = nkb * a.nsplit;
-  const int bh = logical / per_bh, wi = logical % per_bh;
+  int bh, wi;
+  if (CAUSAL && gridDim.x > 256) by_block(a.B * a.Hk, per_bh, true, bh, wi);
+  else {
+    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    bh = logical / per_bh;
+    wi = logical % per_bh;
+  }
   const int b = bh / a.Hk, hk = bh % a.Hk, rep = a.Hq / a.Hk;
   const int kb = wi / a.nsplit;  // causal: low key blocks (most tiles) first within a head
   const int k0 = kb * KB;

@@ -14,7 +14,7 @@
 //  * a row's reference (the exponent that its weights are taken against) is the maximum of the first 64 keys and moves, to a maximum, only once one is 2^8 past
 //    it, a half's check without an exchange between lanes. What waits for its values then is still weighed against the old one: the result is rescaled
 //    after it.
-// us before (a tile's scores, weights and values one after another, 32 x 32 x 16) and so, causal: 1 x 8192, 32 heads over 8 587, 491; 2 x 4096, 32 heads
+// us before (a tile's scores, weights and values one after another, 32 x 32 x 16) and so, causal, head by head: 1 x 8192, 32 heads over 8 587, 491; 2 x 4096, 32 heads
 // 335, 301; 8 x 512, 16 over 8 25.6, 23.8; without a mask, 1 x 8192 1053, 930.
 #pragma once
 #include "ds_hip.h"
@@ -73,6 +73,37 @@ __device__ __forceinline__ void dma16(const char* from, uint32_t dst) {
 // All transfers and LDS accesses of this wave are done, then those of all waves
 __device__ __forceinline__ void meet() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// 16 columns of 32 rows of a tile, transposed: rows 4 (lane / 16) .. + 3 of either 16, as two blocks of sums have them. at: of rows 0 .. 15
+__device__ __forceinline__ bf16x8 columns(uint32_t at) {
+  lds_char* p = (lds_char*)(uintptr_t)at;
+  s16x8 v;
+#ifdef __HIP_DEVICE_COMPILE__
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p), hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 4096));
+  v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+#endif
+  return __builtin_bit_cast(bf16x8, v);
+}
+// 128 columns of the row that a lane has, 4 (lane / 16) .. + 3 of every 16 in o, times `by`: eight columns a piece
+__device__ __forceinline__ void store_row(const f32x4 (&o)[8], float by, bf16* row, int lane, bool mine) {
+  const int g = lane >> 4;
+  each<4>([&](auto d_c) {
+    constexpr int d = 2 * d_c.value;
+    const f32x4 a = o[d] * by, b = o[d + 1] * by;
+    u32x4 w;
+#ifdef __HIP_DEVICE_COMPILE__
+    // (packed in the compiler's sight, which knows what a swap waits for)
+    auto two = [](float lo, float hi) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2)); };
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const auto v = __builtin_amdgcn_permlane16_swap(two(a[2 * i], a[2 * i + 1]), two(b[2 * i], b[2 * i + 1]), false, false);
+      w[i] = v[0];
+      w[2 + i] = v[1];
+    }
+#endif
+    if (mine) *reinterpret_cast<u32x4*>(row + 16 * d + 16 * (g & 1) + 8 * (g >> 1)) = w;
+  });
+}
+
 // A wave's 32 rows: blocks q of 16, of which a lane has row lane % 16
 struct Rows {
   bf16x8 qf[2][4], kf[4], vf[4];  // queries; operands read ahead
@@ -85,16 +116,8 @@ struct Rows {
   float c;                        // scale log2(e)
 
   __device__ __forceinline__ bf16x8 keys(int kb, int ks) const { return *reinterpret_cast<const lds_bf16x8*>((const lds_char*)(uintptr_t)ka[ks] + kb * 4096); }
-  // 16 columns db of 32 keys: those of a lane's weights, 4 (lane / 16) .. + 3 of either 16
-  __device__ __forceinline__ bf16x8 values(int db, int half) const {
-    lds_char* at = (lds_char*)(uintptr_t)va[db] + half * 8192;
-    s16x8 v;
-#ifdef __HIP_DEVICE_COMPILE__
-    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at), hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 4096));
-    v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-#endif
-    return __builtin_bit_cast(bf16x8, v);
-  }
+  // 16 columns db of 32 keys: those of a lane's weights
+  __device__ __forceinline__ bf16x8 values(int db, int half) const { return columns(va[db] + half * 8192); }
   // The keys' first tile, the values' place before theirs. base: of the LDS, a multiple of 32 KB
   __device__ __forceinline__ void init(uint32_t base, int lane, float scale_log2) {
     const int g = lane >> 4, l16 = lane & 15, r = 4 * g + ((lane >> 2) & 3);
@@ -259,26 +282,8 @@ struct Rows {
     const float v = l[q] + __shfl_xor(l[q], 16, 64);
     return v + __shfl_xor(v, 32, 64);
   }
-  // Block q of the result times `by`, to the row that the lane has: eight columns a piece
-  __device__ __forceinline__ void store(int q, float by, bf16* row, int lane, bool mine) {
-    const int g = lane >> 4;
-    each<4>([&](auto d_c) {
-      constexpr int d = 2 * d_c.value;
-      const f32x4 a = o[q][d] * by, b = o[q][d + 1] * by;
-      u32x4 w;
-#ifdef __HIP_DEVICE_COMPILE__
-      // (packed in the compiler's sight, which knows what a swap waits for)
-      auto two = [](float lo, float hi) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2)); };
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const auto v = __builtin_amdgcn_permlane16_swap(two(a[2 * i], a[2 * i + 1]), two(b[2 * i], b[2 * i + 1]), false, false);
-        w[i] = v[0];
-        w[2 + i] = v[1];
-      }
-#endif
-      if (mine) *reinterpret_cast<u32x4*>(row + 16 * d + 16 * (g & 1) + 8 * (g >> 1)) = w;
-    });
-  }
+  // Block q of the result times `by`, to the row that the lane has
+  __device__ __forceinline__ void store(int q, float by, bf16* row, int lane, bool mine) { store_row(o[q], by, row, lane, mine); }
 };
 
 }  // namespace flash

@@ -7,9 +7,13 @@
 //    tile ahead, and the rest of the address one offset per lane for all tiles. Only a ragged last tile is addressed row by row;
 //  * operand reads from LDS run ahead of their products in a pinned order; probabilities are packed two per instruction; the
 //    output is rescaled only when the maximum has moved by more than 2^8;
-//  * workgroups go head by head, heaviest query blocks first. Block by block, as the other kernel has it, an XCD got all heads
-//    of a run of neighbouring query blocks: the last XCD did 15 / 8 of the mean work while the first was idle.
-// 1 x 8192 causal, 32 query heads over 8: 1545 -> 587 us (paged_rows.h now: 546); 4 x 2048, chunks of 2048, two-term weights, sink: 540 ->
+//  * an XCD has heads of its own and takes the heaviest query blocks of all of them first. (All heads of a run of neighbouring blocks to an
+//    XCD: the last one did 15 / 8 of the mean work while the first was idle. Head by head: the last head's longest rows began when the others
+//    were nearly through.) Heads that do not share out evenly go round the chip only over long contexts, which outweigh the other XCDs' reads of
+//    their keys. us, head by head and so, the sink's form: 1 x 8192, 32 heads over 8 738, 697; 4 x 2048 229, 204; 8 x 660 on average 83, 74;
+//    1 x 1500 54.6, 45.9; 16 over 8 4 x 2048 134, 115; 21 x 230 27.7, 28.1; 20 over 4 1 x 8192 556, 450, but 48 x 160 41.0, 44.3; 12 over 12
+//    1 x 8192 348, 285, but 4 x 2048 99, 103 and 12 x 640 41.4, 45.3.
+// 1 x 8192 causal, 32 query heads over 8: 1545 -> 587 us (paged_rows.h now: 492); 4 x 2048, chunks of 2048, two-term weights, sink: 540 ->
 // 265 us.
 #pragma once
 #include <type_traits>
@@ -64,8 +68,10 @@ __global__ void __launch_bounds__(NTHR, 2) paged_flash_kernel(PagedArgs a, int p
   constexpr bool EXT = MODE == EXT_;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, l32 = lane & 31;
-  const int logical = xcd_remap(blockIdx.x, gridDim.x), per_head = gridDim.x / a.Hq;
-  const int w = per_head - 1 - logical % per_head, hq = logical / per_head, hk = hq / (a.Hq / a.Hk);
+  const int per_head = gridDim.x / a.Hq;
+  int hq, at;
+  by_block(a.Hq, per_head, (int64_t)a.max_blocks * a.BS >= 4096, hq, at);
+  const int w = per_head - 1 - at, hk = hq / (a.Hq / a.Hk);
   const int seq = __builtin_amdgcn_readfirstlane(a.work[2 * w]), qb = __builtin_amdgcn_readfirstlane(a.work[2 * w + 1]);
   const int t0 = __builtin_amdgcn_readfirstlane(a.cu_q[seq]), n = __builtin_amdgcn_readfirstlane(a.cu_q[seq + 1]) - t0;
   const int start = __builtin_amdgcn_readfirstlane(a.start[seq]), Skv = start + n;

@@ -1,10 +1,9 @@
 // Ragged paged attention for heads of 128 that see all keys up to their position (ALiBi or not), with the loop of flash_core.h: the arguments of
 // paged_prefill_core.h. Waves have 32 query rows each: of 4, 2 or 1 heads that share their keys, then as many equal waves, or of the 128 neighbours of a
-// work item. Groups of heads one after another on an XCD, whose L2 keeps their keys, the heaviest rows of a group first.
+// work item. The heaviest rows of all groups of an XCD's heads first (as in paged_flash.h).
 // A page of 16 tokens or more holds 16 rows of a tile at a place of its own. Lanes have the numbers of 16 tiles' pages, asked for eight tiles ahead (a scalar
 // load a tile is waited for with the LDS reads behind it); only a ragged last tile is addressed row by row.
-// 1 x 8192, 32 heads over 8, pages of 64 and of 16, us with the loop of paged_flash.h and this one: 587, 546; 564, 530. (With the places of a tile's rows
-// worked out between its two halves' transfers, for keys and for values, instead of once: 551, 520.)
+// (With the places of a tile's rows worked out between its two halves' transfers, for keys and for values, instead of once, 1 % longer.)
 #pragma once
 #include "flash_core.h"
 #include "paged_prefill_core.h"
@@ -17,7 +16,9 @@ __global__ void __launch_bounds__(256, 2) paged_rows_kernel(PagedArgs a, int hea
   __shared__ __attribute__((aligned(32768))) char lds[flash::LDS];
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, l16 = lane & 15;
   const int rows = WAVES * ROWS / heads;
-  const int logical = xcd_remap(blockIdx.x, gridDim.x), per = gridDim.x / (a.Hq / heads), group = logical / per, rest = logical % per;
+  const int per = gridDim.x / (a.Hq / heads);
+  int group, rest;
+  by_block(a.Hq / heads, per, (int64_t)a.max_blocks * a.BS >= 4096, group, rest);
   const int item = (per - 1 - rest) / heads, part = (per - 1 - rest) % heads;
   const int hq = group * heads + wid % heads, hk = group * heads / (a.Hq / a.Hk);
   const int seq = __builtin_amdgcn_readfirstlane(a.work[2 * item]), q0 = __builtin_amdgcn_readfirstlane(a.work[2 * item + 1]) * ::BM + part * rows;
@@ -132,14 +133,10 @@ __global__ void __launch_bounds__(256, 2) paged_rows_kernel(PagedArgs a, int hea
 
 // Without a window: with one, a row's first tile may hold none of its keys.
 inline bool paged_rows_fits(const PagedArgs& a) { return a.window <= 0; }
-// Its first tile and its last values stand alone: it needs some tiles, two workgroups a CU twice over, and heads that share their keys. us with the loop of
-// paged_flash.h and this one, 32 heads over 8: 8192 tokens as 48 x 160 57, 63; 21 x 384 55.0, 55.6; 18 x 448 71.8, 62.2; 16 x 512 74.4, 62.9; 8 x 1024 109,
-// 92.5; 4 x 2048 178, 149; 2048 tokens as 4 x 512 22.8, 24.0; 2 x 1024 35.6, 36.6; 16 over 8, 8192 tokens as 16 x 512 40.7, 41.1; 10 x 768 48.6, 47.8;
-// 4 x 2048 107, 88.6; 32 over 32 16 x 512 74.9, 77.0; 8 x 1024 109, 112; 4 x 2048 178, 177.
-inline bool paged_rows_pays(const PagedArgs& a, int nwork) {
-  const int share = a.Hq / a.Hk;
-  return share % 2 == 0 && (int64_t)nwork * a.Hq >= 1024 && (int64_t)a.max_blocks * a.BS >= (share % 4 == 0 ? 448 : 768);
-}
+// Its first tile and its last values stand alone: it needs many tiles, and two workgroups a CU twice over. us with the loop of paged_flash.h and this one, 32
+// heads over 8, 16 over 8, 32 over 32: 1 x 8192 537, 506; 290, 277; 546, 522; 4 x 2048 158, 150; 91.6, 88.8; 159, 153; 8 x 1024 95.7, 92.3; 59.2, 60.1;
+// 96.9, 94.2; 16 x 512 62.8, 62.7; 39.7, 41.5; 64.3, 64.4; 48 x 160 52, 59; 29.5, 34.0; 57, 61; 1 x 2048 52.6, 51.3; 45.7, 46.7; 52.3, 50.8.
+inline bool paged_rows_pays(const PagedArgs& a, int nwork) { return (int64_t)nwork * a.Hq >= 1024 && (int64_t)a.max_blocks * a.BS >= 2048; }
 
 int launch_rows(const PagedArgs& a, int nwork, hipStream_t st) {
   const int share = a.Hq / a.Hk, heads = share % 4 == 0 ? 4 : share % 2 == 0 ? 2 : 1;

@@ -146,6 +146,25 @@ __device__ __forceinline__ int xcd_remap(int orig, int nwg) {
   return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + orig / 8;
 }
 
+// Workgroup -> (head, one of its `blocks`), the first blocks of all heads before the second ones. A head stays on one XCD, whose L2 keeps its keys, where the
+// heads share out evenly; else they go round the chip, or, not `round`, head by head.
+__device__ __forceinline__ void by_block(int heads, int blocks, bool round, int& head, int& block) {
+  if (heads % 8 && !round) {
+    const int at = xcd_remap(blockIdx.x, gridDim.x);
+    head = at / blocks;
+    block = at % blocks;
+    return;
+  }
+  int at = blockIdx.x, h = heads, first = 0;
+  if (heads % 8 == 0) {
+    h = heads / 8;
+    first = at % 8 * h;
+    at /= 8;
+  }
+  head = first + at % h;
+  block = at / h;
+}
+
 // Tile of a transposing kernel's workgroup: an XCD's share in columns of 16 tiles, row by row. Single columns of tiles read 128 bytes of each row
 // (us on data that a product has just written, 8192 x 11008 / 8192 x 8192: transpose16 70 / 56, this 64 / 53, with `load_once` 63 / 45; gated_fwd_t
 // 147 / 104, 131 / 96, 120 / 92; gated_bwd_t 266 / 192, 244 / 181, 224 / 179; up to 3000 rows of 5632 the same).
