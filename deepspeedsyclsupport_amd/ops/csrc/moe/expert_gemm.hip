@@ -31,6 +31,26 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.f + expf(-g)) * u; }
+// v = silu(g) u of several elements, to the same 3 2^-23: up to 87, where e^-g and its reciprocal are normal numbers, the exponent is a product in two parts, of
+// which the second corrects v_exp_f32's result, and the quotient is v_rcp_f32's with one residual. 12 instructions for 32. Beyond, which a wave finds for all of its elements, expf and the division as they are.
+template <int N>
+__device__ __forceinline__ void silu_muls(const float (&g)[N], const float (&u)[N], float (&v)[N]) {
+  float most = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; i += 2) most = fmaxf(fmaxf(most, fabsf(g[i])), fabsf(g[i + 1]));
+  if (__any(most > 87.f)) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = silu_mul(g[i], u[i]);
+    return;
+  }
+  constexpr float L = 1.44269502162933349609375f, REST = 1.92596299e-8f;  // log2(e) = L + REST
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float t = -L * g[i], more = fmaf(-REST, g[i], fmaf(-L, g[i], -t));  // -g log2(e) = t + more
+    const float p = __builtin_amdgcn_exp2f(t), d = 1.f + fmaf(p, more * 0.693147180559945309f, p), r = __builtin_amdgcn_rcpf(d), q = g[i] * r;
+    v[i] = fmaf(fmaf(-d, q, g[i]), r, q) * u[i];
+  }
+}
 enum : int { NONE = 0, SILU_GLU = 1, RELU2 = 2 };  // activation codes
 __device__ __forceinline__ float plain_act(float x, int act) {
   if (act != RELU2) return x;
@@ -367,12 +387,24 @@ __global__ void __launch_bounds__(256, 2) expert_tile_kernel(ExpertArgs a) {
     for (int t = 0; t < (GLU ? 1 : 2); ++t) {
       const int n = GLU ? n0 + wid * 32 : n0 + wid * 64 + 32 * t;
       if (n >= N) continue;
+      float v[16];
+      if constexpr (GLU) {
+        float gate[16], up[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          gate[i] = acc[0][m][i];
+          up[i] = acc[1][m][i];
+        }
+        silu_muls(gate, up, v);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = plain_act(acc[t][m][i], a.act);
+      }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         bf16x4 o;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          o[i] = (bf16)(GLU ? silu_mul(acc[0][m][4 * q + i], acc[1][m][4 * q + i]) : plain_act(acc[t][m][4 * q + i], a.act));
+        for (int i = 0; i < 4; ++i) o[i] = (bf16)v[4 * q + i];
         *reinterpret_cast<bf16x4*>(yr + n + 8 * q + 4 * hh) = o;
       }
     }
@@ -382,7 +414,7 @@ __global__ void __launch_bounds__(256, 2) expert_tile_kernel(ExpertArgs a) {
 // ------------------------------------------------------------------------------------------------ hundreds of rows per expert
 // A tile of 256 entries by 256 weight rows (gated: 128 of either part, block by block in turn, so that a lane has gate and up of the same columns), with the
 // loop of gemm/wide_core.h: power bounds it there. 32 experts, 1024 rows each on average, at random (all even), us with products of 32 x 32 x 16 and weights
-// straight into registers, and so: 3584 gated columns of 4096 1693 (1583), 1550 (1460); 4096 plain ones of 3584 867 (796), 769 (705). Rows in units of 64 (MI): a short tile moves and multiplies no others. Workgroups walk groups of 8
+// straight into registers, and so: 3584 gated columns of 4096 1693 (1583), 1550 (1446), with the gates of silu_muls 1496 (1397); 4096 plain ones of 3584 867 (796), 769 (711). Rows in units of 64 (MI): a short tile moves and multiplies no others. Workgroups walk groups of 8
 // column tiles by all row tiles of an expert. Beyond 4 GB of rows (LONG) their transfers take an address of 64 bits a lane.
 constexpr int TM = 256, TN = 256;
 
@@ -432,21 +464,33 @@ __global__ void __launch_bounds__(256, 1) expert_big_kernel(ExpertArgs a) {
       constexpr int m = m_c.value;
       const int r = first + 16 * m;
       bf16* yr = (bf16*)a.y + (int64_t)entry[m] * N;
+      float v[NB][4];  // of a lane's four columns in each block
+      if constexpr (GLU) {
+        float gate[4 * NB], up[4 * NB], of[4 * NB];
+        wide::each<NB>([&](auto b) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            gate[4 * b.value + i] = loop.acc[m][2 * b.value][i];
+            up[4 * b.value + i] = loop.acc[m][2 * b.value + 1][i];
+          }
+        });
+        silu_muls(gate, up, of);
+#pragma unroll
+        for (int i = 0; i < 4 * NB; ++i) v[i / 4][i % 4] = of[i];
+      } else {
+        wide::each<NB>([&](auto b) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[b.value][i] = plain_act(loop.acc[m][b.value][i], a.act);
+        });
+      }
       wide::each<NB / 2>([&](auto n_c) {
         constexpr int n = 2 * n_c.value;
-        auto two = [&](auto b_c, int q) {  // columns 2 q and 2 q + 1 of the lane's four in block b
-          constexpr int b = decltype(b_c)::value;
-          f32x2 v;
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-            v[i] = GLU ? silu_mul(loop.acc[m][GLU ? 2 * b : b][2 * q + i], loop.acc[m][GLU ? 2 * b + 1 : b][2 * q + i]) : plain_act(loop.acc[m][b][2 * q + i], a.act);
-          return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
-        };
+        auto two = [&](int b, int q) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{v[b][2 * q], v[b][2 * q + 1]}, bf16x2)); };
         u32x4 o;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
 #ifdef __HIP_DEVICE_COMPILE__
-          const auto v = __builtin_amdgcn_permlane16_swap(two(Int<n>{}, q), two(Int<n + 1>{}, q), false, false);
+          const auto v = __builtin_amdgcn_permlane16_swap(two(n, q), two(n + 1, q), false, false);
           o[q] = v[0];
           o[2 + q] = v[1];
 #endif

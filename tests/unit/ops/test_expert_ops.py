@@ -308,6 +308,35 @@ def test_gates_of_tiles_are_exact_to_fp32(rows):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [128, 64])
+@pytest.mark.parametrize("ends", [(-87.5, -86.5), (86.5, 87.5), (-89, -87), (-1e4, 1e4)])
+def test_gates_of_tiles_at_the_line_of_their_short_form(rows, ends):
+    """Gates up to 87 in size take a shorter form, a wave's others the long one: the bound of the test above on both sides of the line, and what is
+    not finite as expf and the division have it. (From -88 on e^-g overflows: results below 2^-120 are zero.)"""
+    from deepspeedsyclsupport_amd.ops.expert_ops import ACTS, expert_ops, operand_order
+    E, N, K = 2, 128, 64
+    n, d = rows * E, 3 * 2.0**-23
+    experts = torch.arange(n, dtype=torch.int32, device="cuda") // rows
+    order, offs = torch.arange(n, dtype=torch.int32, device="cuda"), torch.arange(E + 1, dtype=torch.int32, device="cuda") * rows
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    w = torch.zeros(E, 2 * N, K, device="cuda")
+    w[:, :N, 0] = torch.rand(E, N, device="cuda", generator=gen) * (ends[1] - ends[0]) + ends[0]
+    w[1, 3:8, 0] = torch.tensor([math.inf, -math.inf, math.nan, 0.0, 3e38], device="cuda")
+    w[:, N:, 0] = 1 + torch.rand(E, N, device="cuda", generator=gen)
+    w = w.bfloat16()
+    x = torch.zeros(n, K, device="cuda").bfloat16()
+    x[:, 0] = 1
+    y = expert_ops().expert_gemm(x, operand_order(w), experts, offs, order, 1, ACTS["silu_glu"], True, True).double().view(E, rows, N)
+    assert torch.equal(y.nan_to_num(7.0), y[:, :1].expand_as(y).nan_to_num(7.0))
+    y, z = y[:, 0], w[..., 0].double()
+    z = z[:, :N] * torch.sigmoid(z[:, :N]) * z[:, N:]
+    assert y[1, 3] == math.inf and y[1, 4].isnan() and y[1, 5].isnan() and y[1, 6] == 0
+    y[1, 4:6] = z[1, 4:6] = 0
+    low, high = torch.stack([(z * (1 - d)).bfloat16().double(), (z * (1 + d)).bfloat16().double()]).sort(0).values
+    assert (((low <= y) & (y <= high)) | ((z.abs() < 2.0**-120) & ((y == 0) | ((y / z - 1).abs() < 2.0**-8)))).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("act", ["silu_glu", "none"])
 @pytest.mark.parametrize("K,n,div", [(4160, 516300, 1), (8256, 260160, 1), (8256, 520300, 2)])
 def test_big_tiles_over_long_inputs(K, n, div, act):
