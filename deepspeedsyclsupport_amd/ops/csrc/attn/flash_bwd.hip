@@ -31,7 +31,7 @@
 //    began when the rest was nearly done (us: 2 x 4096, 32 heads 1118, 1036; 1 x 4096, 20 heads 437, 405; 4 x 8192 heads, all at
 //    once, 341 as it is and 361 round the chip);
 //  * too few sweeps to fill the chip (short sequences of grouped-query models) are cut into parts that leave fp32 dK / dV in a
-//    workspace; a second launch adds them up in a fixed order. B3 Hq16 Hk4 S1000 causal (48 workgroups uncut): 313 -> 103 us.
+//    workspace; a second launch adds them up in a fixed order. B3 Hq16 Hk4 S1000 causal (48 workgroups uncut): 313 -> 97 us.
 // Measured (tools/bench_flash_bwd.py, profiles/flash_bwd_bench_r2_final.jsonl): B8 H32 S4096 D128 causal 4.2-4.3 ms
 // (before the trims above: 4.58). SQ PMC before them: ~29 % MFMA busy, ~9 VALU per MFMA -- the VALU issue slots, not
 // the matrix pipe, are what the trims above (packed converts, pre-scaled row constants, uniform mask skip) buy back.
@@ -47,6 +47,8 @@
 // splitting long key blocks' query ranges over several workgroups with fp32 dK/dV atomics (4 heads x 32k: 6.7 vs
 // 4.3 ms; +10 SGPR spills and the split bookkeeping slowed every shape).
 #include "ds_hip.h"
+
+#include <algorithm>
 
 namespace {
 
@@ -136,10 +138,19 @@ struct BwdArgs {
   int64_t qsb, qsh, qss, ksb, ksh, kss, vsb, vsh, vss, osb, osh, oss, dksb, dksh, dkss, dvsb, dvsh, dvss;
   float c;      // softmax scale * log2(e)
   float scale;
-  // parts: dense sweeps are cut into nsplit of them (part p of key block kb: slot kb * nsplit + p)
-  int nsplit, nslots;
-  f32x4* part;  // [B * Hk, nslots, 32, 512]
+  int nparts;   // of the sweeps of a head's key blocks: as many as those, or more (see parts_before)
+  f32x4* part;  // [B * Hk, nparts, 32, 512]
 };
+
+// Tiles of the sweeps of a head's first `blocks` key blocks, by query head: ntq each, causal 8 less from block to block. Of n parts of all the sweeps, those
+// before block kb: one each, the others by the sweeps' lengths.
+__host__ __device__ __forceinline__ int64_t sweep_tiles(int blocks, int ntq, bool causal) {
+  return (int64_t)blocks * ntq - (causal ? (int64_t)(KB / QT) * blocks * (blocks - 1) / 2 : 0);
+}
+__device__ __forceinline__ int parts_before(int kb, int blocks, int n, int ntq, bool causal) {
+  const int all = (int)sweep_tiles(blocks, ntq, causal);  // (few blocks and parts, where there are more of those)
+  return kb + ((n - blocks) * (int)sweep_tiles(kb, ntq, causal) + all - 1) / all;
+}
 
 // NW waves per workgroup, each owning KPW = 256 / NW keys (NC = KPW / 32 column tiles of the S / dP accumulators).
 // NW = 4: one wave per SIMD with the whole 512-register file (dK^T/dV^T of 64 keys = 256 accumulator registers),
@@ -154,7 +165,7 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
             l32 = lane & 31;
   const int S = a.S;
   const int nkb = (S + KB - 1) / KB;
-  const int per_bh = nkb * a.nsplit;
+  const int per_bh = a.nparts;
   int bh, wi;
   if (CAUSAL && gridDim.x > 256) by_block(a.B * a.Hk, per_bh, true, bh, wi);
   else {
@@ -163,9 +174,20 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
     wi = logical % per_bh;
   }
   const int b = bh / a.Hk, hk = bh % a.Hk, rep = a.Hq / a.Hk;
-  const int kb = wi / a.nsplit;  // causal: low key blocks (most tiles) first within a head
-  const int k0 = kb * KB;
   const int ntq = (S + QT - 1) / QT;
+  int kb = wi, part = 0, parts = 1;  // causal: low key blocks (most tiles) first within a head
+  if (per_bh > nkb) {
+    auto before = [&](int k) { return parts_before(k, nkb, per_bh, ntq, CAUSAL); };
+    int past = nkb;
+    for (kb = 0; past - kb > 1;) {
+      const int mid = (kb + past) / 2;
+      (before(mid) <= wi ? kb : past) = mid;
+    }
+    const int first = before(kb);
+    part = wi - first;
+    parts = before(kb + 1) - first;
+  }
+  const int k0 = kb * KB;
 
   char* Kimg = smem;
   char* QD = smem + K_BYTES;                      // [NBUF][Q tile | dO tile]
@@ -178,8 +200,8 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
   // ------------------------------------------------------------------ iteration space: (query head, query tile)
   const int t0 = CAUSAL ? k0 / QT : 0;
   const int per_head_dense = ntq - t0;
-  const int all = rep * per_head_dense, part = wi % a.nsplit, it0 = (int)((int64_t)all * part / a.nsplit);
-  const int n_it = (int)((int64_t)all * (part + 1) / a.nsplit) - it0, slot = a.nsplit > 1 ? wi : -1;
+  const int all = rep * per_head_dense, it0 = (int)((int64_t)all * part / parts);
+  const int n_it = (int)((int64_t)all * (part + 1) / parts) - it0, slot = per_bh > nkb ? wi : -1;
   // it -> (query head, query tile)
   auto tile_at = [&](int it, int& hq, int& qt) {
     hq = hk * rep + (it0 + it) / per_head_dense;
@@ -510,7 +532,7 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
   // ------------------------------------------------------------------ epilogue: dK = scale * dK^T^T, dV
   if (slot >= 0) {  // a part of the sweep: the accumulators as they are, 16 bytes per thread and piece
     static_assert(NC == 1 && NTHR == 512, "the parts' layout");
-    f32x4* po = a.part + ((int64_t)bh * a.nslots + slot) * (32 * NTHR) + tid;
+    f32x4* po = a.part + ((int64_t)bh * per_bh + slot) * (32 * NTHR) + tid;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -551,11 +573,12 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
 
 // dK and dV of key blocks whose sweep was cut: the parts' accumulators added up, a block per 32 columns of one of the two (the
 // thread layout is the main kernel's).
-__global__ void __launch_bounds__(512) flash_bwd_merge_kernel(BwdArgs a) {
+__global__ void __launch_bounds__(512) flash_bwd_merge_kernel(BwdArgs a, bool causal) {
   const int bh = blockIdx.y, b = bh / a.Hk, hk = bh % a.Hk, mi = blockIdx.x / 8, dt = blockIdx.x & 3, isv = (blockIdx.x >> 2) & 1;
-  const int kb = mi, slot0 = mi * a.nsplit, n = a.nsplit;
+  const int nkb = (a.S + KB - 1) / KB, ntq = (a.S + QT - 1) / QT, kb = mi;
+  const int slot0 = parts_before(kb, nkb, a.nparts, ntq, causal), n = parts_before(kb + 1, nkb, a.nparts, ntq, causal) - slot0;
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, key = kb * KB + 32 * (tid >> 6) + (lane & 31);
-  const f32x4* src = a.part + ((int64_t)bh * a.nslots + slot0) * (32 * 512) + (16 * isv + 4 * dt) * 512 + tid;
+  const f32x4* src = a.part + ((int64_t)bh * a.nparts + slot0) * (32 * 512) + (16 * isv + 4 * dt) * 512 + tid;
   f32x4 acc[4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) acc[g] = src[g * 512];
@@ -638,10 +661,10 @@ int launch_main(const BwdArgs& a, hipStream_t st) {
     attr = true;
   }
   const int nkb = (a.S + KB - 1) / KB;
-  hipLaunchKernelGGL((flash_bwd_kernel<NW, C>), dim3(a.B * a.Hk * nkb * a.nsplit), dim3(NW * 64), lds_bytes<NW>(), st, a);
+  hipLaunchKernelGGL((flash_bwd_kernel<NW, C>), dim3(a.B * a.Hk * a.nparts), dim3(NW * 64), lds_bytes<NW>(), st, a);
   DS_CHECK_LAUNCH();
-  if (a.nsplit > 1) {
-    hipLaunchKernelGGL(flash_bwd_merge_kernel, dim3(nkb * 8, a.B * a.Hk), dim3(512), 0, st, a);
+  if (a.nparts > nkb) {
+    hipLaunchKernelGGL(flash_bwd_merge_kernel, dim3(nkb * 8, a.B * a.Hk), dim3(512), 0, st, a, C);
     DS_CHECK_LAUNCH();
   }
   return 0;
@@ -652,18 +675,21 @@ int launch_main(const BwdArgs& a, hipStream_t st) {
 // Strides are (batch, head, seq) in elements, unit last stride everywhere, all bf16 rows 16-B aligned.
 // q/o/dout/dq [B,Hq,S,128], k/v/dk/dv [B,Hk,S,128], lse [B,Hq,S] natural-log (flash_fwd's), workspace:
 // delta [2*B*Hq*S] fp32 (the pre kernel's -delta and -LSE/scale rows) and dqacc [B*Hq*S*128] fp32.
-// mode: 0 full, 1 causal (top-left). part: the workspace of the parts, B * Hk * slots * 256 KB, slots = ds_flash_bwd_split(..) * key
-// blocks of 256 (none if the split is 1).
+// mode: 0 full, 1 causal (top-left). part: the workspace of the parts, B * Hk * ds_flash_bwd_parts(..) * 256 KB (none if those are the key blocks of 256).
 
-// Parts per key block of a dense sweep. A workgroup takes a CU for itself, so anything below 256 of them idles the rest;
-// parts shorter than 4 tiles would spend their time on the K image and the accumulators. Measured, us, causal, for parts
+// Parts of the sweeps of a head's key blocks, as many as those where none is cut. A workgroup takes a CU for itself, so anything below 256 of them idles the
+// rest; parts shorter than 4 tiles would spend their time on the K image and the accumulators. Measured, us, causal, every sweep in as many parts, for parts
 // that make at most 1 / 128 / 256 / 512 / 1024 workgroups: B3 Hq16 Hk4 S1000 313 / 179 / 103 / 110 / 145, B1 Hq32 Hk8 S2048
 // 605 / 333 / 208 / 190 / 264, B1 Hq8 Hk2 S4096 1144 / 322 / 195 / 196 / 253; B1 H16 S512 (32 workgroups) with parts of at
-// least 16 / 8 / 4 tiles 55 / 45 / 39.
-extern "C" int ds_flash_bwd_split(int B, int Hq, int Hk, int S) {
-  const int nkb = (S + KB - 1) / KB, tiles = Hq / Hk * ((S + QT - 1) / QT);
-  const int fill = 256 / max(B * Hk * nkb, 1), most = tiles / 4;
-  return max(1, min(fill, most));
+// least 16 / 8 / 4 tiles 55 / 45 / 39. They all run at once, so the longest counts. Shared out by the
+// sweeps' lengths, evenly and so: B3 Hq16 Hk4 S1000 109, 97, B2 Hq16 Hk4 S2048 210, 187, B1 Hq8 Hk2 S4096 198, 163, B1 H12 S2048 109, 87; B1 Hq8 Hk1 S600
+// 47, 49. Half as many more than blocks are enough then: B1 H20 S2048, H5 S8192 uncut 175, 603, 12 parts of 8 blocks and 51 of 32 149, 487; a quarter, H24
+// S2048 178, 184, H7 S8192 619, 651.
+extern "C" int ds_flash_bwd_parts(int B, int Hq, int Hk, int S, int causal) {
+  const int nkb = (S + KB - 1) / KB, ntq = (S + QT - 1) / QT;
+  const int64_t tiles = (int64_t)(Hq / Hk) * sweep_tiles(nkb, ntq, causal);
+  const int64_t n = std::min<int64_t>(256 / std::max(B * Hk, 1), tiles / 4);
+  return n * 2 >= nkb * (causal ? 3 : 4) ? (int)n : nkb;
 }
 
 extern "C" int ds_flash_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout,
@@ -672,8 +698,8 @@ extern "C" int ds_flash_bwd(const void* q, const void* k, const void* v, const v
                             const int64_t* dos, const int64_t* dqs, const int64_t* dks, const int64_t* dvs,
                             float scale, int mode, float* part, hipStream_t st) {
   if (Hk <= 0 || Hq % Hk != 0 || S <= 0 || B <= 0) return (int)hipErrorInvalidValue;
-  const int nsplit = ds_flash_bwd_split(B, Hq, Hk, S);
-  if (nsplit > 1 && part == nullptr) return (int)hipErrorInvalidValue;
+  const int nparts = ds_flash_bwd_parts(B, Hq, Hk, S, mode == 1);
+  if (nparts > (S + KB - 1) / KB && part == nullptr) return (int)hipErrorInvalidValue;
   const int64_t rows = (int64_t)B * Hq * S;
   const int pgrid = (int)((rows + 15) / 16);
   hipLaunchKernelGGL(flash_bwd_pre_kernel, dim3(pgrid), dim3(256), 0, st, (const bf16*)o, (const bf16*)dout, lse,
@@ -691,8 +717,7 @@ extern "C" int ds_flash_bwd(const void* q, const void* k, const void* v, const v
   a.dvsb = dvs[0]; a.dvsh = dvs[1]; a.dvss = dvs[2];
   a.c = scale * 1.4426950408889634f;
   a.scale = scale;
-  a.nsplit = nsplit;
-  a.nslots = nsplit * ((S + KB - 1) / KB);
+  a.nparts = nparts;
   a.part = reinterpret_cast<f32x4*>(part);
   const int rc = mode == 1 ? launch_main<8, true>(a, st) : launch_main<8, false>(a, st);
   if (rc) return rc;

@@ -61,7 +61,7 @@ int ds_flash_fwd_sparse(const void*, const void*, const void*, void*, float*, in
 int ds_sparse_bwd(const void*, const void*, const void*, const void*, const void*, const float*, float*, void*, void*, void*, int, int,
                   int, const int64_t*, float, const int* const*, const int*, float*, const int* const*, const int*, float*, const float*,
                   int64_t, const float*, int64_t, const float*, int64_t, int64_t, hipStream_t);
-int ds_flash_bwd_split(int, int, int, int);
+int ds_flash_bwd_parts(int, int, int, int, int);
 int ds_flash_bwd(const void*, const void*, const void*, const void*, const void*, const float*, float*, float*, void*,
                  void*, void*, int, int, int, int, const int64_t*, const int64_t*, const int64_t*, const int64_t*,
                  const int64_t*, const int64_t*, const int64_t*, const int64_t*, float, int, float*, hipStream_t);
@@ -745,9 +745,9 @@ std::vector<Tensor> flash_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse
   TORCH_CHECK(lse.is_cuda() && lse.scalar_type() == at::kFloat && lse.is_contiguous() && lse.numel() == B * Hq * S,
               "flash_bwd: lse [B,Hq,S] fp32 contiguous");
   TORCH_CHECK(mode == 0 || mode == 1, "flash_bwd: mode");
-  const int nsplit = ds_flash_bwd_split((int)B, (int)Hq, (int)Hk, (int)S);
+  const int64_t nparts = ds_flash_bwd_parts((int)B, (int)Hq, (int)Hk, (int)S, mode == 1);
   Tensor parts;
-  if (nsplit > 1) parts = torch::empty({B * Hk * nsplit * ((S + 255) / 256), 65536}, q.options().dtype(at::kFloat));
+  if (nparts > (S + 255) / 256) parts = torch::empty({B * Hk * nparts, 65536}, q.options().dtype(at::kFloat));
   auto mk = [&](int64_t H) { return torch::empty({B, S, H, 128}, q.options()).transpose(1, 2); };
   auto dq = mk(Hq), dk = mk(Hk), dv = mk(Hk);
   auto delta = torch::empty({2 * B * Hq * S}, q.options().dtype(at::kFloat));  // -delta and -LSE/scale rows
@@ -758,7 +758,7 @@ std::vector<Tensor> flash_bwd(Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse
   check(ds_flash_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dout.data_ptr(), lse.data_ptr<float>(),
                      delta.data_ptr<float>(), dqacc.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
                      (int)B, (int)Hq, (int)Hk, (int)S, qs, ks, vs, os, gs, dqs, dks, dvs, (float)scale, (int)mode,
-                     nsplit > 1 ? parts.data_ptr<float>() : nullptr, stream()),
+                     parts.defined() ? parts.data_ptr<float>() : nullptr, stream()),
         "flash_bwd");
   return {dq, dk, dv};
 }

@@ -123,6 +123,13 @@ def test_flash_more_blocks_than_run_at_once(B, Hq, Hk, S):
     _bwd_case(B, Hq, Hk, S, True, seed=S)
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,Hq,Hk,S", [(1, 20, 20, 2048), (3, 16, 4, 1000), (2, 6, 2, 257), (1, 8, 1, 600), (1, 3, 3, 1793)])
+def test_flash_bwd_parts_of_uneven_sweeps(causal, B, Hq, Hk, S):
+    """Fewer sweeps than workgroups are cut, the long ones into more parts; half as many more parts than sweeps are enough."""
+    _bwd_case(B, Hq, Hk, S, causal, seed=S)
+
+
 def test_flash_bwd_strided():
     _bwd_case(2, 4, 2, 640, True, strided=True)
 
