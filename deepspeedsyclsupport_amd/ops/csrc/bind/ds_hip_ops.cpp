@@ -1004,7 +1004,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("xent_mean_node", &xent_mean_node);
   m.def("linear_weight_grad", &linear_weight_grad);
   m.def("narrow_gemm_tune", [](int64_t tile, int64_t parts) { ds_narrow_gemm_tune((int)tile, (int)parts); });
-  m.def("wide_gemm_tune", [](int64_t rows) { ds_wide_gemm_tune((int)rows); });
+  m.def("wide_gemm_tune", [](int64_t rows, int64_t parts) { ds_wide_gemm_tune((int)rows, (int)parts); }, py::arg("rows"), py::arg("parts") = 0);
   m.def("linear_gated", &linear_gated);
   m.def("linear_grad_is_wide", &linear_grad_is_wide);
   m.def("wide_gemm_pays", [](int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) { return ds_wide_gemm_pays(M, N, K, a_along, b_along) != 0; });

@@ -529,20 +529,24 @@ bool dw_pays(int64_t tokens, int64_t out, int64_t in, const Rounds& rounds) {
 
 // Products of many tokens, in tiles of 256 columns (wide_gemm.hip)
 extern "C" int ds_wide_gemm_pays(int64_t, int64_t, int64_t, int, int);
-extern "C" int ds_wide_gemm(const void*, const void*, void*, int64_t, int64_t, int64_t, int64_t, int64_t, int, int, hipStream_t);
+extern "C" int64_t ds_wide_gemm_scratch(int64_t, int64_t, int64_t);
+extern "C" int ds_wide_gemm(const void*, const void*, void*, int64_t, int64_t, int64_t, int64_t, int64_t, int, int, void*, hipStream_t);
 static bool wide(int64_t M, int64_t N, int64_t K, int a_along, int b_along) { return !g_tile && !g_parts && ds_wide_gemm_pays(M, N, K, a_along, b_along); }
 
-// C [M, N] over K, as `ds_narrow_gemm` takes it
-extern "C" int ds_narrow_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along) {
-  if (wide(M, N, K, a_along, b_along)) return 1;
+// Whether these tiles are faster than the library's product
+extern "C" int ds_narrow_tiles_pay(int64_t M, int64_t N, int64_t K, int a_along, int b_along) {
   const Rounds rounds(M, N, K);
   if (!a_along) return dw_pays(K, M, N, rounds);
   return b_along ? y_pays(M, N, K, rounds) : dx_pays(M, K, N, rounds);
 }
+// C [M, N] over K, as `ds_narrow_gemm` takes it
+extern "C" int ds_narrow_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along) {
+  return wide(M, N, K, a_along, b_along) || ds_narrow_tiles_pay(M, N, K, a_along, b_along);
+}
 
 // Bytes of scratch memory that the product wants (0: none)
 extern "C" int64_t ds_narrow_gemm_scratch(int64_t M, int64_t N, int64_t K, int a_along, int b_along) {
-  if (wide(M, N, K, a_along, b_along)) return 0;
+  if (wide(M, N, K, a_along, b_along)) return ds_wide_gemm_scratch(M, N, K);
   const Cut c = cut_of(M, N, K, a_along, b_along);
   return c.parts > 1 ? c.parts * M * N * 4 : 0;
 }
@@ -552,7 +556,7 @@ extern "C" int64_t ds_narrow_gemm_scratch(int64_t M, int64_t N, int64_t K, int a
 extern "C" int ds_narrow_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_along,
                               int b_along, void* part, hipStream_t st) {
   if (!ds_narrow_gemm_ok(M, N, K, lda, ldb, a_along, b_along)) return (int)hipErrorInvalidValue;
-  if (wide(M, N, K, a_along, b_along)) return ds_wide_gemm(A, B, C, M, N, K, lda, ldb, a_along, b_along, st);
+  if (wide(M, N, K, a_along, b_along)) return ds_wide_gemm(A, B, C, M, N, K, lda, ldb, a_along, b_along, part, st);
   const Cut cut = cut_of(M, N, K, a_along, b_along);
   if (cut.parts == 1) part = nullptr;
   else if (!part) return (int)hipErrorInvalidValue;

@@ -115,8 +115,9 @@ struct Operand {
   uint32_t step;       // bytes from a step to the next
   uint32_t at[BASES];  // LDS address of the lane's reads in the slot at work: of either half, of each block, or of all
 
-  static __device__ __forceinline__ i32x4 tile(const bf16* p, uint32_t bytes, uint32_t ld, int r0) {
-    const uint32_t off = LAY == ACROSS ? 2u * r0 : (uint32_t)r0 * ld * 2;
+  // from row r0, and k0 of the inner dimension on
+  static __device__ __forceinline__ i32x4 tile(const bf16* p, uint32_t bytes, uint32_t ld, int r0, int k0 = 0) {
+    const uint32_t off = LAY == ACROSS ? 2u * r0 + (uint32_t)k0 * ld * 2 : (uint32_t)r0 * ld * 2 + 2u * k0;
     return buffer_of((const char*)p + off, bytes - off);
   }
   // A transposed read takes 32 bytes of four rows, and of the four that lie 8 further, at a time: those of rows of 2 R bytes that meet in a bank are apart

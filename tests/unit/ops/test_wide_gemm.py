@@ -44,6 +44,51 @@ def test_tiles_at_their_edges(M, N, K, rows):
 
 
 @GPU
+@pytest.mark.parametrize("rows", [256, 192, 128])
+@pytest.mark.parametrize("parts", [2, 3, 4])
+@pytest.mark.parametrize("M,N,K", [(8, 8, 512), (136, 264, 576), (264, 520, 1088), (520, 1032, 1344), (1032, 4104, 2048)])
+def test_parts_of_the_inner_dimension(M, N, K, parts, rows):
+    """Every form with K in parts, the last of them shorter: the same bound, the same bits each time."""
+    ops = hip_ops()
+    a, b = _rnd(M, K, seed=1), _rnd(N, K, seed=2)
+    ops.wide_gemm_tune(rows, parts)
+    try:
+        y = ops.narrow_gemm(a, b, True, True)
+        dx = ops.narrow_gemm(a, b.t().contiguous(), True, False)
+        dw = ops.narrow_gemm(a.t().contiguous(), b.t().contiguous(), False, False)
+        for c in (y, dx, dw):
+            _check(c, a, b)
+        k = K - 37   # (where rows lie across it, any length)
+        _check(ops.narrow_gemm(a.t().contiguous()[:k], b.t().contiguous()[:k], False, False), a[:, :k], b[:, :k])
+        assert torch.equal(y, ops.narrow_gemm(a, b, True, True))
+        assert torch.equal(dx, ops.narrow_gemm(a, b.t().contiguous(), True, False))
+    finally:
+        ops.wide_gemm_tune(0)
+
+
+@GPU
+@pytest.mark.parametrize("T,O,I", [(1500, 32000, 1024), (2100, 22016, 512)])
+def test_gradients_of_wide_outputs_take_parts(T, O, I):
+    """By the rule, in a stream of the caller's and in a graph: the sums' memory is the allocator's."""
+    dy, w = _rnd(T, O, seed=3), _rnd(O, I, seed=4)
+    assert hip_ops().wide_gemm_pays(T, I, O, True, False)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        dx = hip_ops().linear_input_grad(dy, w)
+    torch.cuda.current_stream().wait_stream(side)
+    _check(dx, dy, w.t())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        again = hip_ops().linear_input_grad(dy, w)
+    for _ in range(3):
+        again.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(again, dx)
+
+
+@GPU
 @pytest.mark.parametrize("T,O,I", [(1500, 8192, 1024), (2048, 5632, 2048), (4096, 3072, 1536), (4200, 2824, 2816), (1156, 11008, 4096), (8200, 2048, 5632), (600, 8192, 4096)])
 def test_products_of_a_layer(T, O, I):
     """In one part and in two, cut between rows or columns, as the rule has it."""
