@@ -22,7 +22,7 @@ template <bool CAUSAL>
 __global__ void __launch_bounds__(256, 2) flash_dense_kernel(DenseArgs a) {
   __shared__ __attribute__((aligned(32768))) char lds[LDS];
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, l16 = lane & 15;
-  // the heaviest rows of all heads first: head by head, an XCD's last head began its longest rows when the others were nearly through (us, causal: 2 x 4096, 32
+  // the heaviest rows of several heads first (by_block): head by head, an XCD's last head began its longest rows when the others were nearly through (us, causal: 2 x 4096, 32
   // heads 350, 317; 1 x 4096, 20 heads 129, 102; 1 x 2048, 32 heads 62.6, 50.4; 3 x 1000, 16 heads over 4 38.8, 33.5; 5 x 1500, 8 heads 45.3, 39.3; 1 x 8192, 4
   // heads 160, 161)
   const int rows = WAVES * ROWS / a.heads, blocks = (a.S + rows - 1) / rows, groups = a.Hq / a.heads;

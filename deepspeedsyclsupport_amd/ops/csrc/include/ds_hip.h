@@ -146,8 +146,11 @@ __device__ __forceinline__ int xcd_remap(int orig, int nwg) {
   return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + orig / 8;
 }
 
-// Workgroup -> (head, one of its `blocks`), the first blocks of all heads before the second ones. A head stays on one XCD, whose L2 keeps its keys, where the
-// heads share out evenly; else they go round the chip, or, not `round`, head by head.
+// Workgroup -> (head, one of its `blocks`), the first blocks of several heads before the second ones. A head stays on one XCD, whose L2 keeps its keys, where
+// the heads share out evenly; else they go round the chip, or, not `round`, head by head. Four heads an XCD at a time, and the last eight to eleven together: what
+// waits at the end is the last ones' short blocks (dense causal forward, us, one / four / eight / all heads at a time and this: 8 x 4096, 32 heads 1151, 1128,
+// 1146, 1454, 1155, not causal 1942, 1950, 2001, 2971, 2008; 2 x 4096 305, 264, 264, 265, 274; 8 x 512, 16 heads 24.1, 24.6, 20.8, 21.1, 20.5; 5 x 1500, 8 heads
+// 47.0, 47.4, 41.6, 42.0, 40.8; backward 8 x 4096, 32 heads 4001, 3931, 3992, 4300, 3971, 1 x 4096, 20 heads 626, 513, 464, 402, 402).
 __device__ __forceinline__ void by_block(int heads, int blocks, bool round, int& head, int& block) {
   if (heads % 8 && !round) {
     const int at = xcd_remap(blockIdx.x, gridDim.x);
@@ -155,14 +158,18 @@ __device__ __forceinline__ void by_block(int heads, int blocks, bool round, int&
     block = at % blocks;
     return;
   }
-  int at = blockIdx.x, h = heads, first = 0;
+  int at = blockIdx.x, h = heads, first = 0, width = 32;
   if (heads % 8 == 0) {
     h = heads / 8;
     first = at % 8 * h;
     at /= 8;
+    width = 4;
   }
-  head = first + at % h;
-  block = at / h;
+  const int group = min(at / (width * blocks), max(h / width - 2, 0));
+  const int here = group < h / width - 2 ? width : h - group * width;
+  at -= group * width * blocks;
+  head = first + group * width + at % here;
+  block = at / here;
 }
 
 // Tile of a transposing kernel's workgroup: an XCD's share in columns of 16 tiles, row by row. Single columns of tiles read 128 bytes of each row

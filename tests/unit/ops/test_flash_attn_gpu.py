@@ -117,7 +117,8 @@ def test_flash_bwd(causal, B, Hq, Hk, S):
     _bwd_case(B, Hq, Hk, S, causal)
 
 
-@pytest.mark.parametrize("B,Hq,Hk,S", [(1, 48, 48, 1500), (3, 36, 12, 700), (1, 20, 20, 3400), (17, 1, 1, 2060)])
+@pytest.mark.parametrize("B,Hq,Hk,S", [(1, 48, 48, 1500), (3, 36, 12, 700), (1, 20, 20, 3400), (17, 1, 1, 2060),
+                                        (13, 8, 8, 700), (5, 20, 20, 700)])
 def test_flash_more_blocks_than_run_at_once(B, Hq, Hk, S):
     """Long sweeps of all heads go first: on an XCD's own heads, or round the chip."""
     _bwd_case(B, Hq, Hk, S, True, seed=S)
