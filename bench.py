@@ -335,7 +335,7 @@ def main():
                 # timed steps (always with > 1 data-parallel rank; at one rank only with DS_ZERO_FORCE_PARTITION=1)
                 "zero_partitioned": partitioned,
                 "twin_flow_offload_ratio": args.offload_ratio,
-                "attention": "in-tree CDNA4 flash fwd+bwd (csrc/attn/flash_{fwd,bwd}.hip)",
+                "attention": "in-tree CDNA4 flash fwd+bwd (csrc/attn/flash_{dense,bwd}.hip)",
                 "micro_batch_per_gpu": args.micro_batch,
                 "gradient_accumulation_steps": args.gas,
                 "activation_checkpointing": bool(args.ckpt),

@@ -512,7 +512,7 @@ bool dx_pays(int64_t tokens, int64_t out, int64_t in, const Rounds& rounds) {
 
 // dW: both operands lie across the inner dimension, as the library likes least.
 bool dw_pays(int64_t tokens, int64_t out, int64_t in, const Rounds& rounds) {
-  // From 8192 tokens on the layer makes copies along them for the library. Rows that meet in memory channels: 32 KB apart ([16384, 2048] 320 45 (35)), or
+  // From 8192 tokens on the layer makes copies along them for the library, where the wide tiles do not pay. Rows that meet in memory channels: 32 KB apart ([16384, 2048] 320 45 (35)), or
   // 8 and 16 KB ([12288, 8192] 528 158 (149))
   if (tokens > 8192 || out % 16384 == 0 || (out % 4096 == 0 && in % 8192 == 0 && out * in > (1 << 25))) return false;
   // up to three rounds of 128 x 128 (256 / 1024 / 4096 by [2048, 2048] 7.8 / 14.5 / 35.7 (10 / 17.2 / 45.5), [2048, 5632] 17 / 34 / 93 (24 / 41 / 96), 8000 by
