@@ -7,7 +7,7 @@
 //    tile ahead, and the rest of the address one offset per lane for all tiles. Only a ragged last tile is addressed row by row;
 //  * operand reads from LDS run ahead of their products in a pinned order; probabilities are packed two per instruction; the
 //    output is rescaled only when the maximum has moved by more than 2^8;
-//  * an XCD has heads of its own and takes the heaviest query blocks of all of them first. (All heads of a run of neighbouring blocks to an
+//  * an XCD has heads of its own and takes the heaviest query blocks of all of them first (from twelve heads on of four at a time). (All heads of a run of neighbouring blocks to an
 //    XCD: the last one did 15 / 8 of the mean work while the first was idle. Head by head: the last head's longest rows began when the others
 //    were nearly through.) Heads that do not share out evenly go round the chip only over long contexts, which outweigh the other XCDs' reads of
 //    their keys. us, head by head and so, the sink's form: 1 x 8192, 32 heads over 8 738, 697; 4 x 2048 229, 204; 8 x 660 on average 83, 74;
