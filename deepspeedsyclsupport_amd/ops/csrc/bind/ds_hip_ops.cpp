@@ -568,7 +568,7 @@ OptT linear_gated(Tensor x, Tensor w) {
   sizes.back() = w.size(0) / 2;
   const Tensor rows = x.view({-1, x.size(-1)});
   int64_t M, N, K, lda, ldb;
-  if (!narrow_sizes(rows, w, true, true, M, N, K, lda, ldb) || !ds_wide_gemm_pays(M, N, K, 1, 1)) return c10::nullopt;
+  if (!narrow_sizes(rows, w, true, true, M, N, K, lda, ldb) || !ds_wide_gated_pays(M, N / 2, K)) return c10::nullopt;
   const c10::DeviceGuard guard(x.device());
   Tensor y = torch::empty(sizes, x.options());
   check(ds_wide_gated(x.const_data_ptr(), w.const_data_ptr(), y.data_ptr(), M, N / 2, K, lda, stream()), "linear_gated");
@@ -1008,6 +1008,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_gated", &linear_gated);
   m.def("linear_grad_is_wide", &linear_grad_is_wide);
   m.def("wide_gemm_pays", [](int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) { return ds_wide_gemm_pays(M, N, K, a_along, b_along) != 0; });
+  m.def("wide_gated_pays", [](int64_t M, int64_t N, int64_t K) { return ds_wide_gated_pays(M, N, K) != 0; });
   m.def("transpose16", &transpose16, py::arg("x"), py::arg("pad_to") = 0);
   m.def("flash_fwd", &flash_fwd);
   m.def("flash_fwd_sparse", &flash_fwd_sparse, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("scale"),

@@ -249,16 +249,20 @@ extern "C" int ds_narrow_tiles_pay(int64_t, int64_t, int64_t, int, int);
 // Of dX, where K is in parts and the narrow tiles do not take it either, the library has few tiles, too, and a lower line stands, also for results of 2^19 (us there,
 // here: 1821 by [22016, 512] 139, 47; 1452 by [11264, 768] 90, 36; 2306 by [11264, 1024] 95, 58; by a line of 550 1629 by [8192, 1024] 38, 44; beside narrow tiles 1556 by
 // [5632, 2048] 40, 46).
-extern "C" int ds_wide_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along) {
+static int pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along, bool parts_too) {
   // (four steps, which a tile of 128 rows has on their way; offsets within a tile's rows of C, of which a quarter of 32 bits marks none)
   if (K <= 192 || N >= 1 << 21 || (!a_along && b_along)) return 0;
   if (g_rows) return 1;
   if ((a_along ? M : K) < 400 || M * N < 1 << 19 || (a_along && M <= 1152 && K >= 8192)) return 0;
-  const Plan p = plan_of(M, N, K);
+  const Plan p = plan_of(M, N, K, parts_too);
   if (M * N < 1 << 20 && p.parts == 1) return 0;
   const bool alone = p.parts > 1 && a_along && !b_along && !ds_narrow_tiles_pay(M, N, K, a_along, b_along);
   return 2e-6 * M * N * K >= p.time * (alone ? 650 : b_along ? 1000 : a_along ? 950 : 800);
 }
+extern "C" int ds_wide_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along) { return pays(M, N, K, a_along, b_along, true); }
+// The same for ds_wide_gated, whose inner dimension stays whole (us in one launch, and the product in parts and the activation: 3939 tokens by 2 x 512 of 12992
+// 111, 103; 6116 by 2 x 256 of 15360 131, 85; accepted, 4096 by 2 x 1024 of 8192 99, 107, 8192 by 2 x 14336 of 4096 1272, 1401)
+extern "C" int ds_wide_gated_pays(int64_t M, int64_t N, int64_t K) { return pays(M, 2 * N, K, 1, 1, false); }
 
 namespace {
 // gate: N weight rows, half of them the gate's, make N / 2 columns of C
@@ -296,7 +300,7 @@ extern "C" int ds_wide_gemm(const void* A, const void* B, void* C, int64_t M, in
   return run(A, B, C, M, N, K, lda, ldb, a_along, b_along, false, part, st);
 }
 
-// y [M, N] = silu(x g^T) (x u^T) of w [2 N, K], g before u; rows of x lda apart, of w K. Where ds_narrow_gemm_ok and ds_wide_gemm_pays have the product by w.
+// y [M, N] = silu(x g^T) (x u^T) of w [2 N, K], g before u; rows of x lda apart, of w K. Where ds_narrow_gemm_ok has the product by w and ds_wide_gated_pays this.
 extern "C" int ds_wide_gated(const void* X, const void* W, void* Y, int64_t M, int64_t N, int64_t K, int64_t lda, hipStream_t st) {
   return run(X, W, Y, M, 2 * N, K, lda, K, 1, 1, true, nullptr, st);
 }

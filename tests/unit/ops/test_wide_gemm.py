@@ -147,6 +147,15 @@ def test_copies_of_gated_activations(I, copies):
         assert ((g.float() - r).norm() / r.norm()).item() < 1e-2
 
 
+@pytest.mark.parametrize("T,I,K,gated", [(3939, 512, 12992, False), (8105, 256, 10624, False), (6116, 256, 15360, False), (3453, 512, 15488, False),
+                                         (6116, 2048, 15360, True), (8192, 14336, 4096, True), (2392, 4096, 1024, True)])
+def test_rule_of_gated_products(T, I, K, gated):
+    """Gate and up of few columns by a long inner dimension pay in parts of it, which the gated product is never cut into."""
+    ops = hip_ops()
+    assert ops.wide_gemm_pays(T, 2 * I, K, True, True)
+    assert ops.wide_gated_pays(T, I, K) == gated
+
+
 @GPU
 @pytest.mark.parametrize("rows", [256, 192, 128, 0])
 @pytest.mark.parametrize("T,I,K", [(8, 8, 256), (200, 136, 320), (520, 392, 576), (2048, 2816, 1024), (4200, 1416, 256)])
@@ -157,7 +166,7 @@ def test_gated_products(rows, T, I, K):
     hip_ops().wide_gemm_tune(rows)
     try:
         got = DF.linear_gated(x, w)
-        assert (got is None) != hip_ops().wide_gemm_pays(T, 2 * I, K, True, True)
+        assert (got is None) != hip_ops().wide_gated_pays(T, I, K)
         if got is None:
             return
         assert torch.equal(got, DF.linear_gated(x, w))
