@@ -560,16 +560,18 @@ Tensor linear_weight_grad(Tensor go, Tensor x) {
   return c.defined() ? c : at::mm(go.t(), x);
 }
 
-// silu(x g^T) (x u^T) of x [.., I] and w [2 O, I], g before u: nothing where the product and the activation are launches of their own
-OptT linear_gated(Tensor x, Tensor w) {
-  if (!unwatched(x, w) || x.dim() < 2 || !x.is_contiguous() || w.dim() != 2 || !w.is_contiguous() || x.size(-1) != w.size(1) || w.size(0) % 16 || !x.numel())
+// act(x g^T) (x u^T) of x [.., I] and w [2 O, I], g before u: in one launch where that pays, else in two. Nothing for what torch has to see or is to take.
+OptT linear_gated(Tensor x, Tensor w, int64_t act) {
+  const auto type = x.scalar_type();
+  if (!unwatched(x, w) || x.dim() < 2 || !x.is_contiguous() || !x.numel() || w.dim() != 2 || !w.is_contiguous() || !w.numel() || x.size(-1) != w.size(1) ||
+      w.size(0) % 16 || !x.is_cuda() || x.device() != w.device() || type != w.scalar_type() || (type != at::kBFloat16 && type != at::kHalf && type != at::kFloat))
     return c10::nullopt;
+  const c10::DeviceGuard guard(x.device());
+  int64_t M, N, K, lda, ldb;
+  if (act != 0 || !narrow_sizes(x.view({-1, x.size(-1)}), w, true, true, M, N, K, lda, ldb) || !ds_wide_gated_pays(M, N / 2, K))
+    return gated_act_fwd(linear_product(x, w), act);
   auto sizes = x.sizes().vec();
   sizes.back() = w.size(0) / 2;
-  const Tensor rows = x.view({-1, x.size(-1)});
-  int64_t M, N, K, lda, ldb;
-  if (!narrow_sizes(rows, w, true, true, M, N, K, lda, ldb) || !ds_wide_gated_pays(M, N / 2, K)) return c10::nullopt;
-  const c10::DeviceGuard guard(x.device());
   Tensor y = torch::empty(sizes, x.options());
   check(ds_wide_gated(x.const_data_ptr(), w.const_data_ptr(), y.data_ptr(), M, N / 2, K, lda, stream()), "linear_gated");
   return y;

@@ -154,10 +154,11 @@ def gated_activation(gate_up, act="silu"):
 
 
 def linear_gated(x, weight, act="silu"):
-    """`gated_activation` of x weight^T in one launch, without a gradient of its own; None where product and activation are two."""
-    if ACT_CODES[act] != ACT_CODES["silu"] or not x.is_cuda or not weight.is_cuda or not unseen_from_python(x, weight):
+    """`gated_activation` of x weight^T without a gradient of its own, asked for once: in one launch where that is the faster way, else in
+    two. None where torch has to see the two, or has one of them alone."""
+    if not x.is_cuda or not weight.is_cuda or not unseen_from_python(x, weight):
         return None
-    return hip_ops().linear_gated(x, weight)
+    return hip_ops().linear_gated(x, weight, ACT_CODES[act])
 
 
 class _BiasActFn(torch.autograd.Function):
