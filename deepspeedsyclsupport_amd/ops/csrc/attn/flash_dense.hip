@@ -22,12 +22,18 @@ template <bool CAUSAL>
 __global__ void __launch_bounds__(256, 2) flash_dense_kernel(DenseArgs a) {
   __shared__ __attribute__((aligned(32768))) char lds[LDS];
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, l16 = lane & 15;
-  // the heaviest rows of several heads first (by_block): head by head, an XCD's last head began its longest rows when the others were nearly through (us, causal: 2 x 4096, 32
-  // heads 350, 317; 1 x 4096, 20 heads 129, 102; 1 x 2048, 32 heads 62.6, 50.4; 3 x 1000, 16 heads over 4 38.8, 33.5; 5 x 1500, 8 heads 45.3, 39.3; 1 x 8192, 4
-  // heads 160, 161)
+  // causal: the heaviest rows of several heads first (by_block): head by head, an XCD's last head began its longest rows when the others were nearly through (us:
+  // 2 x 4096, 32 heads 350, 317; 1 x 4096, 20 heads 129, 102; 1 x 2048, 32 heads 62.6, 50.4; 3 x 1000, 16 heads over 4 38.8, 33.5; 5 x 1500, 8 heads 45.3, 39.3;
+  // 1 x 8192, 4 heads 160, 161). Else all rows weigh the same, and an XCD reads the keys of one head after another (by_block, and so: 5 x 1500, 20 heads
+  // 133, 125; 1 x 4096, 12, 20 and 28 heads 123, 194, 247, 122, 191, 245; 2 x 4096, 32 heads 522, 508; 8 x 4096 2086, 2030; 8 x 512, 16 heads over 8 24.1, 24.3)
   const int rows = WAVES * ROWS / a.heads, blocks = (a.S + rows - 1) / rows, groups = a.Hq / a.heads;
   int bh, at;
-  by_block(a.B * groups, blocks, true, bh, at);
+  if constexpr (CAUSAL) by_block(a.B * groups, blocks, true, bh, at);
+  else {
+    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    bh = logical / blocks;
+    at = logical % blocks;
+  }
   const int b = bh / groups, hq = bh % groups * a.heads + wid % a.heads, hk = bh % groups * a.heads / (a.Hq / a.Hk);
   const int q0 = (CAUSAL ? blocks - 1 - at : at) * rows, q0w = q0 + wid / a.heads * ROWS;
   const int tiles = (a.Skv + BN - 1) / BN;

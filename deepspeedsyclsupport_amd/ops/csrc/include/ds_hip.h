@@ -149,7 +149,7 @@ __device__ __forceinline__ int xcd_remap(int orig, int nwg) {
 // Workgroup -> (head, one of its `blocks`), the first blocks of several heads before the second ones. A head stays on one XCD, whose L2 keeps its keys, where
 // the heads share out evenly; else they go round the chip, or, not `round`, head by head. Four heads an XCD at a time, and the last eight to eleven together: what
 // waits at the end is the last ones' short blocks (dense causal forward, us, one / four / eight / all heads at a time and this: 8 x 4096, 32 heads 1151, 1128,
-// 1146, 1454, 1155, not causal 1942, 1950, 2001, 2971, 2008; 2 x 4096 305, 264, 264, 265, 274; 8 x 512, 16 heads 24.1, 24.6, 20.8, 21.1, 20.5; 5 x 1500, 8 heads
+// 1146, 1454, 1155, not causal 1942, 1950, 2001, 2971, 2008, hence there head by head; 2 x 4096 305, 264, 264, 265, 274; 8 x 512, 16 heads 24.1, 24.6, 20.8, 21.1, 20.5; 5 x 1500, 8 heads
 // 47.0, 47.4, 41.6, 42.0, 40.8; backward 8 x 4096, 32 heads 4001, 3931, 3992, 4300, 3971, 1 x 4096, 20 heads 626, 513, 464, 402, 402).
 __device__ __forceinline__ void by_block(int heads, int blocks, bool round, int& head, int& block) {
   if (heads % 8 && !round) {

@@ -38,6 +38,20 @@ def test_flash_fwd(causal, B, Hq, Hk, S):
     assert o.transpose(1, 2).is_contiguous()  # memory is [B,S,H,D]
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,Hq,Hk,S", [(5, 20, 20, 300), (1, 12, 12, 1100), (13, 28, 4, 140), (2, 96, 24, 140), (1, 40, 40, 520)])
+def test_flash_fwd_orders(causal, B, Hq, Hk, S):
+    """Every row of every head is somebody's, in either order of the workgroups: heads that share out evenly among the XCDs, and that do not."""
+    from deepspeedsyclsupport_amd.ops.native import hip_ops
+    torch.manual_seed(S)
+    q, k = (torch.randn(B, H, S, 128, device="cuda").bfloat16() for H in (Hq, Hk))
+    v = (torch.rand(B, Hk, S, 128, device="cuda") * 2 - 1).bfloat16()
+    o, lse = hip_ops().flash_fwd(q, k, v, causal, 128**-0.5, True)
+    ro, rlse = ref_attn(q, k, v, causal, 128**-0.5)
+    assert (o.float() - ro).abs().max().item() < 2 * 2**-9 + 1e-4   # (values within 1; weights and result are rounded to bf16 once each)
+    torch.testing.assert_close(lse, rlse, rtol=1e-4, atol=1e-4)
+
+
 @pytest.mark.parametrize("S", [128, 96, 33])
 def test_flash_fwd_peak_at_every_key(S):
     """Each key in turn is one row's only large score: a maximum that misses any of them overflows that row's weights."""
