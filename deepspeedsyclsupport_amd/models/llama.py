@@ -138,7 +138,7 @@ class LlamaMLP(nn.Module):
         self.act = cfg.hidden_act
 
     def forward(self, x):
-        return self.down_proj(DF.gated_activation(self.gate_up_proj(x), self.act))
+        return self.down_proj(DF.gated_activation(self.gate_up_proj(x), self.act, x.shape[-1]))
 
 
 class LlamaDecoderLayer(nn.Module):

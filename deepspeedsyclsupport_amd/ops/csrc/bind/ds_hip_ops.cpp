@@ -1009,7 +1009,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("wide_gemm_tune", [](int64_t rows, int64_t parts) { ds_wide_gemm_tune((int)rows, (int)parts); }, py::arg("rows"), py::arg("parts") = 0);
   m.def("linear_gated", &linear_gated);
   m.def("linear_grad_is_wide", &linear_grad_is_wide);
-  m.def("wide_gemm_pays", [](int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) { return ds_wide_gemm_pays(M, N, K, a_along, b_along) != 0; });
+  m.def("wide_gemm_pays", [](int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) {  // (of whole matrices)
+    return ds_narrow_gemm_ok(M, N, K, a_along ? K : M, b_along ? K : N, a_along, b_along) && ds_wide_gemm_pays(M, N, K, a_along, b_along);
+  });
   m.def("wide_gated_pays", [](int64_t M, int64_t N, int64_t K) { return ds_wide_gated_pays(M, N, K) != 0; });
   m.def("transpose16", &transpose16, py::arg("x"), py::arg("pad_to") = 0);
   m.def("flash_fwd", &flash_fwd);

@@ -43,16 +43,19 @@ def kmajor_wanted(rows, dtype):
     return _ENABLED and rows >= KMAJOR_MIN_ROWS and rows % 8 == 0 and dtype in (torch.bfloat16, torch.float16)
 
 
-def kmajor_of_gate(rows, dtype, width):
-    """Whether a gated activation of `width` columns should write the copies of its output and of its gradient: not where the weight
-    gradients that they are for take the operands as they lie. (Of the model's width this sees nothing: 0.3 of the layer's, as
-    in Llama's, where 2816 columns get the first copy and 5632 none.)"""
+def kmajor_of_gate(rows, dtype, width, around):
+    """Whether a gated activation of `width` columns should write the copies of its output and of its gradient for the layers before and behind
+    it, of `around` inputs and outputs: not where their weight gradients take the operands as they lie. Where `around` is None, neither in
+    bf16: the layers choose then, and make what copies they need (us of a step through both layers, copies from the gate and from the
+    layers: 8192 tokens, 256 by 704 312, 305; 65536, 4096 by 16384, operands of more than 4 GB, 57600, 58300)."""
     if not kmajor_wanted(rows, dtype):
         return False, False
     if dtype != torch.bfloat16:
         return True, True
-    pays, model = hip_ops().wide_gemm_pays, int(0.3 * width)
-    return not pays(model, width, rows, False, False), not pays(2 * width, model, rows, False, False)
+    if around is None:
+        return False, False
+    pays = hip_ops().wide_gemm_pays
+    return not pays(around, width, rows, False, False), not pays(2 * width, around, rows, False, False)
 
 
 STATS = {"kmajor_from_producer": 0, "kmajor_transposed": 0}  # how the weight-gradient operands were obtained

@@ -135,13 +135,14 @@ class _GatedActKMajorFn(torch.autograd.Function):
         return dgu, None, None, None
 
 
-def gated_activation(gate_up, act="silu"):
-    """[.., 2I] = [gate | up] -> act(gate) * up  (SwiGLU for act='silu', GEGLU for 'gelu')."""
+def gated_activation(gate_up, act="silu", around=None):
+    """[.., 2I] = [gate | up] -> act(gate) * up  (SwiGLU for act='silu', GEGLU for 'gelu'). around: the width of the model, that is the inputs
+    of the layer before and the outputs of the one behind, for what they need in training (`kmajor_of_gate`)."""
     code = ACT_CODES[act]
     if gate_up.is_cuda and (gate_up.shape[-1] // 2) % 8 == 0:
         from ..linear import kmajor_of_gate
         rows = gate_up.numel() // gate_up.shape[-1]
-        if gate_up.requires_grad and torch.is_grad_enabled() and any(copies := kmajor_of_gate(rows, gate_up.dtype, gate_up.shape[-1] // 2)):
+        if gate_up.requires_grad and torch.is_grad_enabled() and any(copies := kmajor_of_gate(rows, gate_up.dtype, gate_up.shape[-1] // 2, around)):
             out, out_t = _GatedActKMajorFn.apply(gate_up.contiguous(), code, *copies)
             if out_t is not None:
                 out._ds_kmajor = out_t

@@ -125,16 +125,27 @@ def test_values_that_do_not_mix():
         ops.wide_gemm_tune(0)
 
 
+@pytest.mark.parametrize("T,I,H", [(8192, 704, 256), (8192, 2816, 1024), (8192, 5632, 2048), (8192, 1376, 4096), (8192, 2752, 4096), (8192, 1408, 2048),
+                                   (16384, 1408, 2048), (32768, 1376, 4096), (8192, 2048, 250), (8200, 4096, 4096)])
+def test_copies_of_gated_activations_by_the_layers_around(T, I, H):
+    """A copy is written exactly where the weight gradient that would read it goes to the library: by the widths of that product, a shard's too."""
+    pays = hip_ops().wide_gemm_pays
+    assert L.kmajor_of_gate(T, torch.bfloat16, I, H) == (not pays(H, I, T, False, False), not pays(2 * I, H, T, False, False))
+    assert L.kmajor_of_gate(T, torch.bfloat16, I, None) == L.kmajor_of_gate(8184, torch.bfloat16, I, H) == (False, False)
+    assert L.kmajor_of_gate(T, torch.float16, I, H) == L.kmajor_of_gate(T, torch.float16, I, None) == (True, True)
+    assert not pays(H + 4, I, T, False, False)   # (no whole pieces of rows: nobody's)
+
+
 @GPU
-@pytest.mark.parametrize("I,copies", [(704, 2), (2816, 1), (5632, 0)])
-def test_copies_of_gated_activations(I, copies):
+@pytest.mark.parametrize("H,I,copies", [(256, 704, 2), (1024, 2816, 1), (2112, 5632, 0), (4096, 1376, 0), (2048, 1408, 1)])
+def test_copies_of_gated_activations(H, I, copies):
     """Of 8192 tokens on the gate writes the copies along the tokens that the weight gradients around it will read, and only those."""
     from deepspeedsyclsupport_amd.ops.transformer import functional as DF
-    T, H = 8192, max(256, I * 3 // 8 // 64 * 64)
-    assert sum(L.kmajor_of_gate(T, torch.bfloat16, I)) == copies
+    T = 8192
+    assert sum(L.kmajor_of_gate(T, torch.bfloat16, I, H)) == copies
     x, w1, w2 = (_rnd(*s, seed=i).mul_(0.05 if i else 1).requires_grad_() for i, s in enumerate(((T, H), (2 * I, H), (H, I))))
     before = dict(L.STATS)
-    act = DF.gated_activation(L.linear(x, w1), "silu")
+    act = DF.gated_activation(L.linear(x, w1), "silu", H)
     y = L.linear(act, w2)
     go = _rnd(T, H, seed=5)
     got = torch.autograd.grad(y, (x, w1, w2), go)
