@@ -90,6 +90,8 @@ def weight_grad(go2d, x2d, go_kmajor=None, x_kmajor=None):
     T = go2d.shape[0]
     if x2d is not None and x_kmajor is None and T >= KMAJOR_MIN_ROWS and _wide(go2d, x2d, True):
         return hip_ops().linear_weight_grad(go2d, x2d)
+    if x_kmajor is not None and go2d.shape[1] % 8:   # (outputs that no copy is made of)
+        return go2d.t().mm(x_kmajor[:, :T].t())
     if x_kmajor is not None or _kmajor_ok(go2d, x2d):
         Tp = -(-T // 256) * 256
         got = _kmajor_of(go2d, go_kmajor, Tp)                                    # [out, Tp]

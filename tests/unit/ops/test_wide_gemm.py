@@ -158,6 +158,23 @@ def test_copies_of_gated_activations(H, I, copies):
         assert ((g.float() - r).norm() / r.norm()).item() < 1e-2
 
 
+@GPU
+@pytest.mark.parametrize("around", [True, False])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_copies_for_odd_widths(dtype, around):
+    """A gate's copy reaches a layer whose outputs come in no whole pieces of 16 bytes."""
+    from deepspeedsyclsupport_amd.ops.transformer import functional as DF
+    T, H, I = 8200, 252, 320
+    x, w1, w2 = (_rnd(*s, seed=i).mul_(0.05 if i else 1).to(dtype).requires_grad_() for i, s in enumerate(((T, H), (2 * I, H), (H, I))))
+    go = _rnd(T, H, seed=5).to(dtype)
+    got = torch.autograd.grad(L.linear(DF.gated_activation(L.linear(x, w1), "silu", H if around else None), w2), (x, w1, w2), go)
+    xf, w1f, w2f = (t.detach().float().requires_grad_() for t in (x, w1, w2))
+    h = xf @ w1f.t()
+    want = torch.autograd.grad((torch.nn.functional.silu(h[:, :I]) * h[:, I:]) @ w2f.t(), (xf, w1f, w2f), go.float())
+    for g, r in zip(got, want):
+        assert ((g.float() - r).norm() / r.norm()).item() < 1e-2
+
+
 @pytest.mark.parametrize("T,I,K,gated", [(3939, 512, 12992, False), (8105, 256, 10624, False), (6116, 256, 15360, False), (3453, 512, 15488, False),
                                          (6116, 2048, 15360, True), (8192, 14336, 4096, True), (2392, 4096, 1024, True)])
 def test_rule_of_gated_products(T, I, K, gated):
