@@ -192,6 +192,8 @@ struct Operand {
   }
 };
 
+constexpr int STEPS = 4;  // the fewest of a tile that others follow: its transfers are so far ahead
+
 // A's and B's rings, and the loop over one tile's steps, after another's (CHAIN) or alone
 template <int AK, int BK, int MI, bool CHAIN>
 struct Loop {
@@ -208,8 +210,8 @@ struct Loop {
   static constexpr int EVERY = (MEET - 1) / (EARLY > LATE ? EARLY : LATE);  // products from a transfer to the next
   // At a step's barrier the next step has to be there: what may be newer than its last piece of B, and of A
   static constexpr int NEWER_B = PA + (RB - 2) * (PA + PB), NEWER_A = (RA - 2) * (PA + PB), NEWER = NEWER_B < NEWER_A ? NEWER_B : NEWER_A;
-  static constexpr int STEPS = CHAIN ? (RA > RB ? RA : RB) : 1;  // the fewest of a tile
   static_assert(LDS <= 160 * 1024 && EVERY >= 1 && LATE <= PB);
+  static_assert(!CHAIN || (RA <= STEPS && RB <= STEPS), "a tile's transfers end before they are as far ahead");
 
   A oa;
   B ob;

@@ -165,15 +165,15 @@ struct Plan {
 Plan plan_for(int64_t M, int64_t N, int64_t K, bool parts_too) {
   const int sizes[3] = {256, 192, 128};
   const int steps = (int)((K + 63) / 64);
-  auto cut = [&](int rows, int parts) {  // parts of four steps or more
+  auto cut = [&](int rows, int parts) {
     int deep = (steps + parts - 1) / parts;
-    while (steps % deep && steps % deep < 4) ++deep;
+    while (steps % deep && steps % deep < STEPS) ++deep;
     Plan p{rows, 0, M, N, 0, (steps + deep - 1) / deep, deep};
     const int64_t mt = (M + rows - 1) / rows;
     p.time = time_of(rows, mt * rows * p.parts, N, deep * 64) + 4 + (8 * p.parts + 2) * 1e-6 / 5 * M * N;
     return p;
   };
-  if (g_rows) return cut(g_rows, parts_too ? std::max(1, std::min(g_parts, steps / 4)) : 1);
+  if (g_rows) return cut(g_rows, parts_too ? std::max(1, std::min(g_parts, steps / STEPS)) : 1);
   Plan best = {0, 0, M, N, 0};
   auto offer = [&](const Plan& p) {
     if (!best.rows || p.time < best.time) best = p;
@@ -249,9 +249,10 @@ extern "C" int ds_narrow_tiles_pay(int64_t, int64_t, int64_t, int, int);
 // Of dX, where K is in parts and the narrow tiles do not take it either, the library has few tiles, too, and a lower line stands, also for results of 2^19 (us there,
 // here: 1821 by [22016, 512] 139, 47; 1452 by [11264, 768] 90, 36; 2306 by [11264, 1024] 95, 58; by a line of 550 1629 by [8192, 1024] 38, 44; beside narrow tiles 1556 by
 // [5632, 2048] 40, 46).
+// Steps of a tile; offsets within a tile's rows of C, of which a quarter of 32 bits marks none
+static bool takes(int64_t N, int64_t K, int a_along, int b_along) { return (K + 63) / 64 >= STEPS && N < 1 << 21 && (a_along || !b_along); }
 static int pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along, bool parts_too) {
-  // (four steps, which a tile of 128 rows has on their way; offsets within a tile's rows of C, of which a quarter of 32 bits marks none)
-  if (K <= 192 || N >= 1 << 21 || (!a_along && b_along)) return 0;
+  if (!takes(N, K, a_along, b_along)) return 0;
   if (g_rows) return 1;
   if ((a_along ? M : K) < 400 || M * N < 1 << 19 || (a_along && M <= 1152 && K >= 8192)) return 0;
   const Plan p = plan_of(M, N, K, parts_too);
@@ -267,7 +268,8 @@ extern "C" int ds_wide_gated_pays(int64_t M, int64_t N, int64_t K) { return pays
 namespace {
 // gate: N weight rows, half of them the gate's, make N / 2 columns of C
 int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int a_along, int b_along, bool gate, void* part, hipStream_t st) {
-  Plan p = plan_of(M, N, K, !gate);
+  if (!takes(N, K, a_along, b_along)) return (int)hipErrorInvalidValue;
+  const Plan p = plan_of(M, N, K, !gate);
   if (p.parts > 1 && !part) return (int)hipErrorInvalidValue;
   const int64_t ar = a_along ? M : K, ac = a_along ? K : M, br = b_along ? N : K, bc = b_along ? K : N;
   const int64_t of = gate ? 2 : 1, cols = N / of, cut = p.n < N ? p.n / of : cols;  // C's columns, those of the first part

@@ -175,6 +175,21 @@ def test_copies_for_odd_widths(dtype, around):
         assert ((g.float() - r).norm() / r.norm()).item() < 1e-2
 
 
+def test_products_that_the_loop_cannot_take_are_refused():
+    """At the C entries, before anything is launched: fewer steps than a tile's transfers are ahead, columns past what the stores' offsets mark."""
+    import ctypes
+    from deepspeedsyclsupport_amd.ops import op_builder
+    hip_ops()
+    lib, i64 = ctypes.CDLL(op_builder.so_path("ds_hip_ops")), ctypes.c_int64
+    M, invalid = 512, 1
+    for N, K, a, b in ((512, 192, 1, 1), (512, 64, 1, 0), (512, 100, 0, 0), (1 << 21, 256, 1, 1), (512, 256, 0, 1)):
+        lda, ldb = K if a else M, K if b else N
+        assert lib.ds_wide_gemm(None, None, None, i64(M), i64(N), i64(K), i64(lda), i64(ldb), a, b, None, None) == invalid
+        if a and b:
+            assert lib.ds_wide_gated(None, None, None, i64(M), i64(N // 2), i64(K), i64(lda), None) == invalid
+        assert not hip_ops().wide_gemm_pays(M, N, K, bool(a), bool(b))
+
+
 @pytest.mark.parametrize("T,I,K,gated", [(3939, 512, 12992, False), (8105, 256, 10624, False), (6116, 256, 15360, False), (3453, 512, 15488, False),
                                          (6116, 2048, 15360, True), (8192, 14336, 4096, True), (2392, 4096, 1024, True)])
 def test_rule_of_gated_products(T, I, K, gated):
