@@ -17,28 +17,10 @@
 // us before (a tile's scores, weights and values one after another, 32 x 32 x 16) and so, causal, head by head: 1 x 8192, 32 heads over 8 587, 491; 2 x 4096, 32 heads
 // 335, 301; 8 x 512, 16 over 8 25.6, 23.8; without a mask, 1 x 8192 1053, 930.
 #pragma once
-#include "ds_hip.h"
-
-#include <type_traits>
-#include <utility>
+#include "each.h"
 
 namespace flash {
-
-template <int N>
-using Int = std::integral_constant<int, N>;
-template <class F, int... I>
-__device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, I...>) {
-  (f(Int<I>{}), ...);
-}
-// f(Int<0>{}) .. f(Int<N - 1>{})
-template <int N, class F>
-__device__ __forceinline__ void each(F&& f) {
-  each_of(f, std::make_integer_sequence<int, N>{});
-}
-
-typedef __attribute__((address_space(3))) char lds_char;
-typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+using namespace constants;
 
 constexpr int D = 128, BN = 64, WAVES = 4, ROWS = 32;  // head, keys of a tile, rows of a wave
 constexpr uint32_t TILE = BN * D * 2;                  // 16 KB

@@ -17,29 +17,12 @@
 // 8192 tokens, us here and by the library's call: y by [4096, 11008] 455 / 454 (1624 TF/s), by [12288, 4096] 527 / 524; dX by [4096, 11008] 464 / 524;
 // dW [4096, 11008] 508 / 768, of 688 tiles where 768 would fit.
 #pragma once
-#include "ds_hip.h"
-
-#include <type_traits>
-#include <utility>
+#include "each.h"
 
 namespace wide {
+using namespace constants;
 
-typedef __attribute__((address_space(3))) char lds_char;
-typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 typedef int i32x4 __attribute__((ext_vector_type(4)));
-
-template <int N>
-using Int = std::integral_constant<int, N>;
-template <class F, int... I>
-__device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, I...>) {
-  (f(Int<I>{}), ...);
-}
-// f(Int<0>{}) .. f(Int<N - 1>{}): indexes that are constants, whatever the compiler unrolls
-template <int N, class F>
-__device__ __forceinline__ void each(F&& f) {
-  each_of(f, std::make_integer_sequence<int, N>{});
-}
 
 // A buffer of `bytes` bytes: what lies past its end reads as zero
 __device__ __forceinline__ i32x4 buffer_of(const void* p, uint32_t bytes) {
