@@ -465,10 +465,10 @@ extern "C" int ds_narrow_gemm_ok(int64_t M, int64_t N, int64_t K, int64_t lda, i
 
 // Whether the kernel is as fast as the library's, for each product of a linear layer of `tokens` rows by a weight [out, in]; us here (there).
 // A cost model was not found that orders the library's side, which jumps with its own choice of tiles. What the lines go by is stated with each:
-// whole rounds of the chip (`Rounds`), which products of its size the library is bad at, and rows that meet in memory channels. On layers at
-// random, none of which the lines were drawn by, with weights (for dW the input) from memory 617 / 553 / 1074 products y / dX / dW of 1200 layers go here and
-// take 0.73 / 0.68 / 0.68 of the library's time in the mean, 2138 of them faster by more than 4 %, 22 slower by as much, at worst 35 %; out of the caches 769
-// of 400 layers 0.76 / 0.66 / 0.63, 753 faster, 2 slower (profiles/narrow_products_at_random.csv).
+// whole rounds of the chip (`Rounds`), which products of its size the library is bad at, and rows that meet in memory channels. The wide tiles are asked first
+// (`wide` below). On layers at random, none of which the lines were drawn by, with weights (for dW the input) from memory 613 / 508 / 812 products y / dX / dW of
+// 1200 layers go here and take 0.75 / 0.69 / 0.65 of the library's time in the mean, 1859 of them faster by more than 4 %, 15 slower by as much, at worst 35 %;
+// out of the caches 673 of 400 layers 0.77 / 0.68 / 0.60, 662 faster, none slower (profiles/narrow_products_at_random.csv, without what the wide tiles take).
 namespace {
 
 // y: a tile's operands come as the library's do; what is gained is its launch, and tiles that fill the chip.
