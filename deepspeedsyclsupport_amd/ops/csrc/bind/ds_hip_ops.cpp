@@ -1012,6 +1012,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("wide_gemm_pays", [](int64_t M, int64_t N, int64_t K, bool a_along, bool b_along) {  // (of whole matrices)
     return ds_narrow_gemm_ok(M, N, K, a_along ? K : M, b_along ? K : N, a_along, b_along) && ds_wide_gemm_pays(M, N, K, a_along, b_along);
   });
+  m.def("wide_plan", [](int64_t M, int64_t N, int64_t K, bool gated) {
+    std::array<int64_t, 5> p;
+    ds_wide_plan(M, N, K, gated, p.data());
+    return p;
+  });
   m.def("wide_gated_pays", [](int64_t M, int64_t N, int64_t K) { return ds_wide_gated_pays(M, N, K) != 0; });
   m.def("transpose16", &transpose16, py::arg("x"), py::arg("pad_to") = 0);
   m.def("flash_fwd", &flash_fwd);

@@ -15,6 +15,7 @@ int ds_narrow_gemm(const void*, const void*, void*, int64_t, int64_t, int64_t, i
 void ds_narrow_gemm_tune(int, int);
 int ds_wide_gemm_pays(int64_t, int64_t, int64_t, int, int);
 void ds_wide_gemm_tune(int, int);
+void ds_wide_plan(int64_t, int64_t, int64_t, int, int64_t*);
 int ds_wide_gated_pays(int64_t, int64_t, int64_t);
 int ds_wide_gated(const void*, const void*, void*, int64_t, int64_t, int64_t, int64_t, hipStream_t);
 }

@@ -290,6 +290,13 @@ int run(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, 
 }
 }  // namespace
 
+// How C [M, N] over K (gated: M by N weight rows) goes out: rows of a tile; those of the second part's tiles (0: one part); where that begins, in rows or in
+// columns; parts of K
+extern "C" void ds_wide_plan(int64_t M, int64_t N, int64_t K, int gated, int64_t* to) {
+  const Plan p = plan_of(M, N, K, !gated);
+  to[0] = p.rows, to[1] = p.other, to[2] = p.m, to[3] = p.n, to[4] = p.parts;
+}
+
 // Bytes of scratch memory that the product wants (0: none)
 extern "C" int64_t ds_wide_gemm_scratch(int64_t M, int64_t N, int64_t K) {
   const int parts = plan_of(M, N, K).parts;

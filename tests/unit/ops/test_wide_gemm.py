@@ -20,6 +20,16 @@ def _check(got, a, b):
     assert ((got.double() - want).abs() <= want.abs() * 2**-8 + size * a.shape[1] * 2**-23).all()
 
 
+def _check_gated(got, x, w):
+    """Both sums off by less than `size` and multiplied into each other (the gate's slope is at most 1.1), one rounding to bf16."""
+    I, K = w.shape[0] // 2, w.shape[1]
+    g, u = (x.double() @ w.double().t()).split(I, -1)
+    size = x.double().abs() @ w.double().abs().t() * K * 2**-23
+    want = torch.nn.functional.silu(g) * u
+    bound = want.abs() * 2**-8 + 1.1 * size[:, :I] * u.abs() + size[:, I:] * g.abs() + 2**-20
+    assert ((got.double() - want).abs() <= bound).all()
+
+
 @GPU
 @pytest.mark.parametrize("rows", [256, 192, 128])
 @pytest.mark.parametrize("M,N,K", [(8, 8, 256), (128, 256, 256), (136, 264, 320), (200, 248, 448), (264, 520, 576), (520, 1032, 1088), (4104, 4872, 256)])
@@ -232,10 +242,22 @@ def test_gated_products(rows, T, I, K):
         assert torch.equal(DF.linear_gated(x.view(2, T // 2, K), w), got.view(2, T // 2, I))
     finally:
         hip_ops().wide_gemm_tune(0)
-    g, u = (x.double() @ w.double().t()).split(I, -1)
-    size = x.double().abs() @ w.double().abs().t() * K * 2**-23   # (of the sums; the gate's slope is at most 1.1)
-    want = torch.nn.functional.silu(g) * u
-    bound = want.abs() * 2**-8 + 1.1 * size[:, :I] * u.abs() + size[:, I:] * g.abs() + 2**-20
-    assert ((got.double() - want).abs() <= bound).all()
+    _check_gated(got, x, w)
     with torch.enable_grad():
         assert DF.linear_gated(x.requires_grad_(), w) is None
+
+
+@GPU
+@pytest.mark.parametrize("T,I,K,rows,other,m,n", [
+    (2391, 4096, 1024, 192, 128, 1536, 4096), (5247, 3800, 640, 256, 128, 4352, 3800), (4694, 2912, 768, 256, 192, 2816, 2912),
+    (4189, 3080, 896, 192, 256, 1920, 3080), (4770, 2128, 960, 192, 128, 2880, 2128), (6782, 1400, 1152, 128, 192, 2944, 1400),
+    (6301, 5632, 2048, 256, 128, 6301, 5120), (1970, 6040, 960, 256, 128, 1970, 4096), (2843, 4720, 832, 256, 192, 2843, 2688),
+    (3626, 3672, 896, 192, 256, 3626, 1664), (1914, 5184, 1024, 192, 128, 1914, 3200), (2775, 3312, 1280, 128, 192, 2775, 1408)])
+def test_gated_products_in_two(T, I, K, rows, other, m, n):
+    """Cut between rows, or between columns, which are of either part of the weight."""
+    from deepspeedsyclsupport_amd.ops.transformer import functional as DF
+    assert hip_ops().wide_gated_pays(T, I, K) and hip_ops().wide_plan(T, 2 * I, K, True) == [rows, other, m, 2 * n, 1]
+    x, w = _rnd(T, K, seed=1), _rnd(2 * I, K, seed=2) * 0.1
+    got = DF.linear_gated(x, w)
+    assert torch.equal(got, DF.linear_gated(x, w))
+    _check_gated(got, x, w)
