@@ -52,6 +52,25 @@ def test_flash_fwd_orders(causal, B, Hq, Hk, S):
     torch.testing.assert_close(lse, rlse, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("Hq,Hk", [(3, 3), (4, 2), (8, 2)])
+@pytest.mark.parametrize("S,Skv", [(200, 77), (77, 200), (300, 64), (64, 300), (129, 1), (1, 129), (513, 511), (128, 320), (320, 128)])
+def test_flash_fwd_other_keys(S, Skv, Hq, Hk, causal):
+    """Keys of another length than the queries', a causal row's first ones the same; what lies behind the last one is nobody's."""
+    from deepspeedsyclsupport_amd.ops.attention import attention, flash_supported
+    from deepspeedsyclsupport_amd.ops.native import hip_ops
+    torch.manual_seed(S)
+    q = torch.randn(2, Hq, S, 128, device="cuda").bfloat16()
+    k, v = (torch.full((2, Hk, Skv + 64, 128), float("nan"), device="cuda").bfloat16()[:, :, :Skv] for _ in range(2))
+    k.copy_(torch.randn(k.shape, device="cuda"))
+    v.copy_(torch.rand(v.shape, device="cuda") * 2 - 1)
+    o, lse = hip_ops().flash_fwd(q, k, v, causal, 128**-0.5, True)
+    ro, rlse = ref_attn(q, k, v, causal, 128**-0.5)
+    assert (o.float() - ro).abs().max().item() < 2 * 2**-9 + 1e-4   # (values within 1; weights and result are rounded to bf16 once each)
+    torch.testing.assert_close(lse, rlse, rtol=1e-4, atol=1e-4)
+    assert flash_supported(q, k, v) and torch.equal(attention(q, k, v, causal=causal), o)
+
+
 @pytest.mark.parametrize("S", [128, 96, 33])
 def test_flash_fwd_peak_at_every_key(S):
     """Each key in turn is one row's only large score: a maximum that misses any of them overflows that row's weights."""
