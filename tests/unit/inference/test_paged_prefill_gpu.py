@@ -8,7 +8,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _case(lens, starts, Hq, Hk, BS, alibi, window, seed=0, D=128):
+def _case(lens, starts, Hq, Hk, BS, alibi, window, seed=0, D=128, own_loop=False):
     from deepspeedsyclsupport_amd.inference.model_implementations.transformer import RaggedMeta, alibi_slopes
     from deepspeedsyclsupport_amd.ops.native import hip_ops
     g = torch.Generator(device="cuda").manual_seed(seed)
@@ -24,6 +24,8 @@ def _case(lens, starts, Hq, Hk, BS, alibi, window, seed=0, D=128):
         o += nb
     meta = RaggedMeta.build(starts, lens, blocks, 0, BS, torch.device("cuda"))
     T = sum(lens)
+    if own_loop:  # (many rows of long contexts: paged_rows.h)
+        assert D == 128 and not window and meta.work.shape[0] * Hq >= 1024 and meta.block_tables.shape[1] * BS >= 2048
     q = torch.randn(T, Hq, D, device="cuda", generator=g).bfloat16()
     slopes = alibi_slopes(Hq).cuda() if alibi else None
     scale = 1.0 / math.sqrt(D)
@@ -81,6 +83,17 @@ def test_paged_prefill_alibi_window(window):
 
 def test_paged_prefill_long_prefix():
     _case([256, 17], [3000, 4095], 8, 1, 64, alibi=False, window=0, seed=3)
+
+
+@pytest.mark.parametrize("alibi", [False, True])
+@pytest.mark.parametrize("Hq,Hk,BS,lens,starts", [
+    (32, 8, 64, [4096], [0]),
+    (32, 4, 16, [1200, 37, 2100, 900], [0, 2011, 130, 17]),
+    (16, 8, 32, [3000, 65, 2049, 3100], [0, 4031, 63, 1]),
+    (12, 12, 128, [4130, 90, 7000], [0, 4001, 30]),
+])
+def test_long_prompts(Hq, Hk, BS, lens, starts, alibi):
+    _case(lens, starts, Hq, Hk, BS, alibi, 0, seed=BS, own_loop=True)
 
 
 @pytest.mark.parametrize("D", [64, 80, 96, 256])
