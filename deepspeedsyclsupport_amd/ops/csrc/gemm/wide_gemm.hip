@@ -241,6 +241,9 @@ extern "C" void ds_wide_gemm_tune(int rows, int parts) { g_rows = rows, g_parts 
 // (narrow_gemm.hip)
 extern "C" int ds_narrow_tiles_pay(int64_t, int64_t, int64_t, int, int);
 
+// Steps of a tile; offsets within a tile's rows of C, of which a quarter of 32 bits marks none
+static bool takes(int64_t N, int64_t K, int a_along, int b_along) { return (K + 63) / 64 >= STEPS && N < 1 << 21 && (a_along || !b_along); }
+
 // Whether the kernel takes a product that ds_narrow_gemm_ok has, and is the fastest way: the estimate comes to a rate that neither the library's call nor the
 // narrow tiles reach on average. 1200 products of 400 layers at random (profiles/wide_products_at_random.csv), time here over the time before, in the
 // mean, by the rate of the estimate in TF/s: y 800 - 1000 0.92, 1000 - 1500 0.86, below 800 1.43; dX 800 - 1000 0.94, 1000 - 1500 0.81, below 1.8; dW 600 -
@@ -248,17 +251,22 @@ extern "C" int ds_narrow_tiles_pay(int64_t, int64_t, int64_t, int, int);
 // y, 640 by [12288, 11008] 179 (158), 467 by [10240, 8192] 78 (71), dX, 697 by [28672, 8192] 344 (301)).
 // Of dX, where K is in parts and the narrow tiles do not take it either, the library has few tiles, too, and a lower line stands, also for results of 2^19 (us there,
 // here: 1821 by [22016, 512] 139, 47; 1452 by [11264, 768] 90, 36; 2306 by [11264, 1024] 95, 58; by a line of 550 1629 by [8192, 1024] 38, 44; beside narrow tiles 1556 by
-// [5632, 2048] 40, 46).
-// Steps of a tile; offsets within a tile's rows of C, of which a quarter of 32 bits marks none
-static bool takes(int64_t N, int64_t K, int a_along, int b_along) { return (K + 63) / 64 >= STEPS && N < 1 << 21 && (a_along || !b_along); }
+// [5632, 2048] 40, 46). dW in parts beside narrow tiles, which are one round of those, is no gain (6464 tokens by [2048, 2048] 50, 56; 7848 by [2048, 1920] 58, 64; 6720 by
+// [8192, 488] 57, 56); from 8192 tokens on, where a layer makes copies for the library instead,
+// it takes 0.51 of the time (140 at random: 8512 by [2048, 2048] 100, 68).
 static int pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along, bool parts_too) {
   if (!takes(N, K, a_along, b_along)) return 0;
   if (g_rows) return 1;
   if ((a_along ? M : K) < 400 || M * N < 1 << 19 || (a_along && M <= 1152 && K >= 8192)) return 0;
   const Plan p = plan_of(M, N, K, parts_too);
   if (M * N < 1 << 20 && p.parts == 1) return 0;
-  const bool alone = p.parts > 1 && a_along && !b_along && !ds_narrow_tiles_pay(M, N, K, a_along, b_along);
-  return 2e-6 * M * N * K >= p.time * (alone ? 650 : b_along ? 1000 : a_along ? 950 : 800);
+  int line = b_along ? 1000 : a_along ? 950 : 800;
+  if (p.parts > 1 && !b_along) {
+    const bool narrow = (a_along || K < 8192) && ds_narrow_tiles_pay(M, N, K, a_along, b_along);
+    if (narrow && !a_along) return 0;
+    if (!narrow && a_along) line = 650;
+  }
+  return 2e-6 * M * N * K >= p.time * line;
 }
 extern "C" int ds_wide_gemm_pays(int64_t M, int64_t N, int64_t K, int a_along, int b_along) { return pays(M, N, K, a_along, b_along, true); }
 // The same for ds_wide_gated, whose inner dimension stays whole (us in one launch, and the product in parts and the activation: 3939 tokens by 2 x 512 of 12992

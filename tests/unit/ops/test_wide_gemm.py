@@ -185,6 +185,14 @@ def test_copies_for_odd_widths(dtype, around):
         assert ((g.float() - r).norm() / r.norm()).item() < 1e-2
 
 
+@pytest.mark.parametrize("T,O,I,wide", [(6464, 2048, 2048, False), (6016, 512, 8192, False), (7848, 2048, 1920, False), (7360, 4096, 1016, False),
+                                        (8192, 2048, 2048, True), (8512, 2048, 2048, True), (11008, 1536, 3072, True), (13184, 1536, 3072, True)])
+def test_weight_gradients_in_parts_go_where_the_narrow_tiles_do_not(T, O, I, wide):
+    ops = hip_ops()
+    assert ops.wide_plan(O, I, T, False)[4] > 1
+    assert ops.wide_gemm_pays(O, I, T, False, False) == wide
+
+
 def test_products_that_the_loop_cannot_take_are_refused():
     """At the C entries, before anything is launched: fewer steps than a tile's transfers are ahead, columns past what the stores' offsets mark."""
     import ctypes
