@@ -31,7 +31,7 @@
 //    began when the rest was nearly done (us: 2 x 4096, 32 heads 1118, 1036; 1 x 4096, 20 heads 437, 405; 4 x 8192 heads, all at
 //    once, 341 as it is and 361 round the chip);
 //  * too few sweeps to fill the chip (short sequences of grouped-query models) are cut into parts that leave fp32 dK / dV in a
-//    workspace; a second launch adds them up in a fixed order. B3 Hq16 Hk4 S1000 causal (48 workgroups uncut): 313 -> 97 us.
+//    workspace; a second launch adds them up in a fixed order. B3 Hq16 Hk4 S1000 causal (48 workgroups uncut): 313 -> 93 us.
 // Measured (tools/bench_flash_bwd.py, profiles/flash_bwd_bench_r2_final.jsonl): B8 H32 S4096 D128 causal 4.2-4.3 ms
 // (before the trims above: 4.58). SQ PMC before them: ~29 % MFMA busy, ~9 VALU per MFMA -- the VALU issue slots, not
 // the matrix pipe, are what the trims above (packed converts, pre-scaled row constants, uniform mask skip) buy back.
@@ -138,19 +138,32 @@ struct BwdArgs {
   int64_t qsb, qsh, qss, ksb, ksh, kss, vsb, vsh, vss, osb, osh, oss, dksb, dksh, dkss, dvsb, dvsh, dvss;
   float c;      // softmax scale * log2(e)
   float scale;
-  int nparts;   // of the sweeps of a head's key blocks: as many as those, or more (see parts_before)
-  f32x4* part;  // [B * Hk, nparts, 32, 512]
+  int nparts, deep;  // of the sweeps of a head's key blocks: as many as those, or more, of `deep` tiles at most (see Sweep)
+  f32x4* part;       // [B * Hk, nparts, 32, 512]
 };
 
-// Tiles of the sweeps of a head's first `blocks` key blocks, by query head: ntq each, causal 8 less from block to block. Of n parts of all the sweeps, those
-// before block kb: one each, the others by the sweeps' lengths.
-__host__ __device__ __forceinline__ int64_t sweep_tiles(int blocks, int ntq, bool causal) {
-  return (int64_t)blocks * ntq - (causal ? (int64_t)(KB / QT) * blocks * (blocks - 1) / 2 : 0);
-}
-__device__ __forceinline__ int parts_before(int kb, int blocks, int n, int ntq, bool causal) {
-  const int all = (int)sweep_tiles(blocks, ntq, causal);  // (few blocks and parts, where there are more of those)
-  return kb + ((n - blocks) * (int)sweep_tiles(kb, ntq, causal) + all - 1) / all;
-}
+// Tiles of key block kb's sweep over the query rows, of `rep` query heads
+__host__ __device__ __forceinline__ int sweep_tiles(int kb, int ntq, int rep, bool causal) { return rep * (ntq - (causal ? KB / QT * kb : 0)); }
+// One of a head's sweeps, all of which are cut into parts of `deep` tiles or less: its key block, the slot of its first part, its parts. By its block, or by a
+// slot of it (the other one past any).
+struct Sweep {
+  int kb = 0, first = 0, parts;
+  __device__ __forceinline__ Sweep(int block, int slot, int ntq, int rep, int deep, bool causal) {
+    uint32_t past = sweep_tiles(0, ntq, rep, causal) + deep - 1;
+    parts = past / (uint32_t)deep;
+    if (!causal) {  // (equal ones)
+      kb = min(block, slot / parts);
+      first = kb * parts;
+      return;
+    }
+    while (kb < block && first + parts <= slot) {
+      ++kb;
+      first += parts;
+      past -= rep * (KB / QT);
+      parts = past / (uint32_t)deep;
+    }
+  }
+};
 
 // NW waves per workgroup, each owning KPW = 256 / NW keys (NC = KPW / 32 column tiles of the S / dP accumulators).
 // NW = 4: one wave per SIMD with the whole 512-register file (dK^T/dV^T of 64 keys = 256 accumulator registers),
@@ -177,15 +190,10 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
   const int ntq = (S + QT - 1) / QT;
   int kb = wi, part = 0, parts = 1;  // causal: low key blocks (most tiles) first within a head
   if (per_bh > nkb) {
-    auto before = [&](int k) { return parts_before(k, nkb, per_bh, ntq, CAUSAL); };
-    int past = nkb;
-    for (kb = 0; past - kb > 1;) {
-      const int mid = (kb + past) / 2;
-      (before(mid) <= wi ? kb : past) = mid;
-    }
-    const int first = before(kb);
-    part = wi - first;
-    parts = before(kb + 1) - first;
+    const Sweep sweep(nkb, wi, ntq, rep, a.deep, CAUSAL);
+    kb = sweep.kb;
+    part = wi - sweep.first;
+    parts = sweep.parts;
   }
   const int k0 = kb * KB;
 
@@ -575,8 +583,9 @@ __global__ void __launch_bounds__(NW * 64, 1) flash_bwd_kernel(BwdArgs a) {
 // thread layout is the main kernel's).
 __global__ void __launch_bounds__(512) flash_bwd_merge_kernel(BwdArgs a, bool causal) {
   const int bh = blockIdx.y, b = bh / a.Hk, hk = bh % a.Hk, mi = blockIdx.x / 8, dt = blockIdx.x & 3, isv = (blockIdx.x >> 2) & 1;
-  const int nkb = (a.S + KB - 1) / KB, ntq = (a.S + QT - 1) / QT, kb = mi;
-  const int slot0 = parts_before(kb, nkb, a.nparts, ntq, causal), n = parts_before(kb + 1, nkb, a.nparts, ntq, causal) - slot0;
+  const int ntq = (a.S + QT - 1) / QT, kb = mi;
+  const Sweep sweep(kb, a.nparts, ntq, a.Hq / a.Hk, a.deep, causal);
+  const int slot0 = sweep.first, n = sweep.parts;
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, key = kb * KB + 32 * (tid >> 6) + (lane & 31);
   const f32x4* src = a.part + ((int64_t)bh * a.nparts + slot0) * (32 * 512) + (16 * isv + 4 * dt) * 512 + tid;
   f32x4 acc[4];
@@ -681,16 +690,39 @@ int launch_main(const BwdArgs& a, hipStream_t st) {
 // rest; parts shorter than 4 tiles would spend their time on the K image and the accumulators. Measured, us, causal, every sweep in as many parts, for parts
 // that make at most 1 / 128 / 256 / 512 / 1024 workgroups: B3 Hq16 Hk4 S1000 313 / 179 / 103 / 110 / 145, B1 Hq32 Hk8 S2048
 // 605 / 333 / 208 / 190 / 264, B1 Hq8 Hk2 S4096 1144 / 322 / 195 / 196 / 253; B1 H16 S512 (32 workgroups) with parts of at
-// least 16 / 8 / 4 tiles 55 / 45 / 39. They all run at once, so the longest counts. Shared out by the
-// sweeps' lengths, evenly and so: B3 Hq16 Hk4 S1000 109, 97, B2 Hq16 Hk4 S2048 210, 187, B1 Hq8 Hk2 S4096 198, 163, B1 H12 S2048 109, 87; B1 Hq8 Hk1 S600
-// 47, 49. Half as many more than blocks are enough then: B1 H20 S2048, H5 S8192 uncut 175, 603, 12 parts of 8 blocks and 51 of 32 149, 487; a quarter, H24
-// S2048 178, 184, H7 S8192 619, 651.
-extern "C" int ds_flash_bwd_parts(int B, int Hq, int Hk, int S, int causal) {
-  const int nkb = (S + KB - 1) / KB, ntq = (S + QT - 1) / QT;
-  const int64_t tiles = (int64_t)(Hq / Hk) * sweep_tiles(nkb, ntq, causal);
-  const int64_t n = std::min<int64_t>(256 / std::max(B * Hk, 1), tiles / 4);
-  return n * 2 >= nkb * (causal ? 3 : 4) ? (int)n : nkb;
+// least 16 / 8 / 4 tiles 55 / 45 / 39. They all run at once, so the longest counts, and no sweep is in parts longer than those of the longest one; then the
+// merge, by the parts that one of its workgroups adds up and by all that is written and read. Of times of 88 shapes in 1 to 64 parts of the longest
+// sweep, a tile takes 2.1 us, a merge 2, 0.3 for each part of a sweep and 0.06 for each of all; what these choose takes 1.1 % longer than the best in the mean, at worst 8 %.
+// us, 1.5 parts a block shared out by rounded shares of the length, and so: causal, B1 H8 S5311 (uncut 400) 427, 268; B1 H20 S2048 150, 130; B1 H5 S8192 487, 377; B3 Hq16
+// Hk4 S1000 97, 93; B1 Hq8 Hk1 S1280 69, 58; full, B2 Hq12 Hk3 S4096 788, 687; B1 H6 S4191 237, 217; B1 H32 S768 75, 67.
+namespace {
+constexpr double TILE_US = 2.1, CUT_US = 2, MERGE_US = 0.3, PART_US = 0.06;
+struct Parts {
+  int n, deep;  // of a head's sweeps; tiles of each at most
+};
+Parts parts_for(int B, int Hq, int Hk, int S, bool causal) {
+  const int nkb = (S + KB - 1) / KB, ntq = (S + QT - 1) / QT, rep = Hq / Hk, longest = sweep_tiles(0, ntq, rep, causal);
+  Parts best = {nkb, longest};
+  double least = TILE_US * longest;
+  const int most = 256 / std::max(B * Hk, 1);
+  for (int p = 2; p <= longest / 4 && p <= most; ++p) {
+    const int deep = (longest + p - 1) / p;
+    int n = 0;
+    for (int kb = 0; kb < nkb && n <= most; ++kb) n += (sweep_tiles(kb, ntq, rep, causal) + deep - 1) / deep;
+    if (n > most) break;
+    const double t = TILE_US * deep + CUT_US + MERGE_US * p + PART_US * n * B * Hk;
+    if (t < least) least = t, best = {n, deep};
+  }
+  return best;
 }
+// (a backward asks for it twice, a model's layers for the same)
+Parts parts_of(int B, int Hq, int Hk, int S, bool causal) {
+  thread_local struct { int B = 0, Hq, Hk, S; bool causal; Parts parts; } last;
+  if (last.B != B || last.Hq != Hq || last.Hk != Hk || last.S != S || last.causal != causal) last = {B, Hq, Hk, S, causal, parts_for(B, Hq, Hk, S, causal)};
+  return last.parts;
+}
+}  // namespace
+extern "C" int ds_flash_bwd_parts(int B, int Hq, int Hk, int S, int causal) { return parts_of(B, Hq, Hk, S, causal).n; }
 
 extern "C" int ds_flash_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout,
                             const float* lse, float* delta, float* dqacc, void* dq, void* dk, void* dv, int B, int Hq,
@@ -698,8 +730,8 @@ extern "C" int ds_flash_bwd(const void* q, const void* k, const void* v, const v
                             const int64_t* dos, const int64_t* dqs, const int64_t* dks, const int64_t* dvs,
                             float scale, int mode, float* part, hipStream_t st) {
   if (Hk <= 0 || Hq % Hk != 0 || S <= 0 || B <= 0) return (int)hipErrorInvalidValue;
-  const int nparts = ds_flash_bwd_parts(B, Hq, Hk, S, mode == 1);
-  if (nparts > (S + KB - 1) / KB && part == nullptr) return (int)hipErrorInvalidValue;
+  const Parts parts = parts_of(B, Hq, Hk, S, mode == 1);
+  if (parts.n > (S + KB - 1) / KB && part == nullptr) return (int)hipErrorInvalidValue;
   const int64_t rows = (int64_t)B * Hq * S;
   const int pgrid = (int)((rows + 15) / 16);
   hipLaunchKernelGGL(flash_bwd_pre_kernel, dim3(pgrid), dim3(256), 0, st, (const bf16*)o, (const bf16*)dout, lse,
@@ -717,7 +749,8 @@ extern "C" int ds_flash_bwd(const void* q, const void* k, const void* v, const v
   a.dvsb = dvs[0]; a.dvsh = dvs[1]; a.dvss = dvs[2];
   a.c = scale * 1.4426950408889634f;
   a.scale = scale;
-  a.nparts = nparts;
+  a.nparts = parts.n;
+  a.deep = parts.deep;
   a.part = reinterpret_cast<f32x4*>(part);
   const int rc = mode == 1 ? launch_main<8, true>(a, st) : launch_main<8, false>(a, st);
   if (rc) return rc;

@@ -158,9 +158,10 @@ def test_flash_more_blocks_than_run_at_once(B, Hq, Hk, S):
 
 
 @pytest.mark.parametrize("causal", [True, False])
-@pytest.mark.parametrize("B,Hq,Hk,S", [(1, 20, 20, 2048), (3, 16, 4, 1000), (2, 6, 2, 257), (1, 8, 1, 600), (1, 3, 3, 1793)])
+@pytest.mark.parametrize("B,Hq,Hk,S", [(1, 20, 20, 2048), (3, 16, 4, 1000), (2, 6, 2, 257), (1, 8, 1, 600), (1, 3, 3, 1793), (1, 6, 6, 4191), (1, 8, 1, 1280),
+                                        (1, 8, 8, 5311), (2, 4, 4, 2130), (1, 1, 1, 8000)])
 def test_flash_bwd_parts_of_uneven_sweeps(causal, B, Hq, Hk, S):
-    """Fewer sweeps than workgroups are cut, the long ones into more parts; half as many more parts than sweeps are enough."""
+    """Fewer sweeps than workgroups are cut, none into longer parts than the longest one."""
     _bwd_case(B, Hq, Hk, S, causal, seed=S)
 
 
