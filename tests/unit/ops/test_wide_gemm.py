@@ -141,7 +141,8 @@ def test_copies_of_gated_activations_by_the_layers_around(T, I, H):
     """A copy is written exactly where the weight gradient that would read it goes to the library: by the widths of that product, a shard's too."""
     pays = hip_ops().wide_gemm_pays
     assert L.kmajor_of_gate(T, torch.bfloat16, I, H) == (not pays(H, I, T, False, False), not pays(2 * I, H, T, False, False))
-    assert L.kmajor_of_gate(T, torch.bfloat16, I, None) == L.kmajor_of_gate(8184, torch.bfloat16, I, H) == (False, False)
+    assert L.kmajor_of_gate(T, torch.bfloat16, I, None) == L.kmajor_of_gate(T, torch.bfloat16, I, I)
+    assert L.kmajor_of_gate(8184, torch.bfloat16, I, H) == (False, False)
     assert L.kmajor_of_gate(T, torch.float16, I, H) == L.kmajor_of_gate(T, torch.float16, I, None) == (True, True)
     assert not pays(H + 4, I, T, False, False)   # (no whole pieces of rows: nobody's)
 
