@@ -219,12 +219,14 @@ class PipelineEngine(DeepSpeedEngine):
             loss = out / self.micro_batches
             if opt.dtype == torch.float16:
                 loss = loss.float() * opt.loss_scale
-            loss.backward()
+            with torch.autograd.set_multithreading_enabled(False):  # (as the optimizer's own backward)
+                loss.backward()
         else:
             outs = [out] if torch.is_tensor(out) else list(out)
             grads = self.pipe_buffers["output_tensors"][buffer_id]
             pairs = [(o, g) for o, g in zip(outs, grads) if o.requires_grad]
-            torch.autograd.backward([o for o, _ in pairs], [g for _, g in pairs])
+            with torch.autograd.set_multithreading_enabled(False):
+                torch.autograd.backward([o for o, _ in pairs], [g for _, g in pairs])
         opt.backward_epilogue()
         self.pipe_buffers["outputs"][buffer_id] = None
         self.pipe_buffers["output_tensors"][buffer_id] = None

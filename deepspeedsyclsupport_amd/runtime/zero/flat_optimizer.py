@@ -769,11 +769,15 @@ class FlatZeroOptimizer(ZeROOptimizer):
             self.coordinator.begin_backward()
 
     def backward(self, loss, retain_graph=False):
+        """On the calling thread: from a thread of autograd's own, which waits for nothing but this one, all that both touch goes to and fro
+        between two cores. A step of 128 tokens, 1024 wide, two layers, took 760 - 870 us or 1040 - 1110 by the two cores that a process
+        got, forward and optimizer included; so 760 - 870."""
         self.backward_prologue()
-        if self.dtype == torch.float16:
-            self.loss_scaler.backward(loss.float(), retain_graph=retain_graph)
-        else:
-            loss.backward(retain_graph=retain_graph)
+        with torch.autograd.set_multithreading_enabled(False):
+            if self.dtype == torch.float16:
+                self.loss_scaler.backward(loss.float(), retain_graph=retain_graph)
+            else:
+                loss.backward(retain_graph=retain_graph)
         self.backward_epilogue()
 
     @instrument_w_nvtx
