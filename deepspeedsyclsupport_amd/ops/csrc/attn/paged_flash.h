@@ -13,7 +13,7 @@
 //    their keys. us, head by head and so, the sink's form: 1 x 8192, 32 heads over 8 738, 697; 4 x 2048 229, 204; 8 x 660 on average 83, 74;
 //    1 x 1500 54.6, 45.9; 16 over 8 4 x 2048 134, 115; 21 x 230 27.7, 28.1; 20 over 4 1 x 8192 556, 450, but 48 x 160 41.0, 44.3; 12 over 12
 //    1 x 8192 348, 285, but 4 x 2048 99, 103 and 12 x 640 41.4, 45.3.
-// 1 x 8192 causal, 32 query heads over 8: 1545 -> 587 us (paged_rows.h now: 492); 4 x 2048, chunks of 2048, two-term weights, sink: 540 ->
+// 1 x 8192 causal, 32 query heads over 8: 1545 -> 587 us (paged_rows.h now: 512 back to back, 557 in a pass between other kernels); 4 x 2048, chunks of 2048, two-term weights, sink: 540 ->
 // 265 us.
 #pragma once
 #include <type_traits>
