@@ -139,7 +139,7 @@ struct BwdArgs {
   float c;      // softmax scale * log2(e)
   float scale;
   int nparts, deep;  // of the sweeps of a head's key blocks: as many as those, or more, of `deep` tiles at most (see Sweep)
-  f32x4* part;       // [B * Hk, nparts, 32, 512]
+  f32x4* part;       // [B * Hk, nparts, 32, 512] (with eight bytes more in here hipcc schedules the loop otherwise: full, 2 % longer)
 };
 
 // Tiles of key block kb's sweep over the query rows, of `rep` query heads
